@@ -120,6 +120,9 @@ constexpr int kFillThreads = 1024;  // 256 / 512 threads: 0.49 / 0.38 ms
 __host__ __device__ inline bool sorted_fill_applies(int bins_per_bm, int LP) { return bins_per_bm <= kSortedBins && LP <= kStage; }
 constexpr size_t kSortedFillLds = (size_t)kStage * (16 + 4 + 4) + (size_t)(3 * kSortedBins + 1) * 4;
 
+// this block's part of the total that chunk_of() reads
+__device__ __forceinline__ int *counted_points(const BinWorkspace &ws) { return &ws.queues[(blockIdx.x % kClasses) * kQueueStride + 1]; }
+
 // MODE 0: count.  MODE 1: fill (needs the scanned cursor).
 template <int MODE>
 __global__ __launch_bounds__(256) void bin_points_kernel(
@@ -136,6 +139,7 @@ __global__ __launch_bounds__(256) void bin_points_kernel(
   // The launch is a few thousand workgroups that walk the n_blocks blocks of work (so that it costs next to nothing
   // when the kernel steps aside).  head = block % M: with the round-robin placement of workgroups on the 8 XCDs
   // and a grid that is a multiple of 8, the records of one (batch, head) are written through one XCD's L2.
+  int counted = 0;
   for (int blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
   __syncthreads();                          // the previous block's LDS histogram is no longer in use
   const int m = blk % M, rest = blk / M;
@@ -167,6 +171,7 @@ __global__ __launch_bounds__(256) void bin_points_kernel(
 #pragma unroll
         for (int k = 0; k < kKept; ++k) kept[k] = round == k ? bin : kept[k];
       }
+      ++counted;
       if (use_lds) atomicAdd(&s_hist[bin], 1);
       else if (MODE == 0) atomicAdd(&gcount[bin], 1);
     } else if (MODE == 1) {
@@ -214,6 +219,10 @@ __global__ __launch_bounds__(256) void bin_points_kernel(
     }
   }
   }
+  if (MODE == 0) {
+    counted = wave_inclusive_scan(counted);
+    if (threadIdx.x % kWave == kWave - 1) atomicAdd(counted_points(ws), counted);
+  }
 }
 
 // Count in the same shape as the sorted fill: 1024 threads, kStage points per block, all loads of a thread issued
@@ -248,15 +257,19 @@ __global__ __launch_bounds__(kFillThreads) void bin_count_kernel(
     }
   }
   __syncthreads();
+  int counted = 0;
 #pragma unroll
   for (int r = 0; r < kPer; ++r) {
+    bool inside = false;
     if (lv[r] >= 0) {
       const int l = lv[r];
       const Point2D<float> g = locate_2d<float>(x[r], y[r], p.H[l], p.W[l], p.start[l]);
-      if (g.inside && p.tiles_x[l] > 0) atomicAdd(&s_cnt[bin_of(p, l, g)], 1);
+      inside = g.inside && p.tiles_x[l] > 0;
+      if (inside) atomicAdd(&s_cnt[bin_of(p, l, g)], 1);
     }
+    counted += __syncthreads_count(inside);                      // the last one: all have been counted
   }
-  __syncthreads();
+  if (tid == 0) atomicAdd(counted_points(ws), counted);
   int *gcount = ws.counts + (size_t)bm * nb;
   for (int i = tid; i < nb; i += kFillThreads) {
     const int c = s_cnt[i];
@@ -406,7 +419,7 @@ __device__ __forceinline__ void clear_unstored(const BinWorkspace &ws, const Cle
   const int value_row_bytes = ca.value_row_bytes, dist_row_bytes = ca.dist_row_bytes;
   const int B = ca.B, S = ca.S, M = ca.M, L = ca.L, stores = ca.stores;
   const BinPlan &p = *ws.plan;
-  const int nb = p.bins_per_bm, TY = p.ty, TX = p.tx, ch = p.chunk;
+  const int nb = p.bins_per_bm, TY = p.ty, TX = p.tx, ch = chunk_of(ws, p);
   const size_t rows = (size_t)B * S * M;
   const int lane = threadIdx.x % kWave;
   // every wavefront takes 64 consecutive rows per turn; all its lanes stay in the loop (shuffles)
@@ -424,7 +437,7 @@ __device__ __forceinline__ void clear_unstored(const BinWorkspace &ws, const Cle
           if ((y + 1) % TY != 0 && (x + 1) % TX != 0) {       // the first tile starts at pixel -1
             const int bin = slot_of(b, m, B, M) * nb + p.level_base[l] + ((y + 1) / TY) * p.tiles_x[l] + (x + 1) / TX;
             const int c = ws.counts[bin];
-            clear_mine = !(c > 0 && c <= ch);                 // exactly one work item: it stores this row
+            clear_mine = items_of_bin(c, ch) != 1;            // exactly one work item stores this row
           }
           break;
         }
@@ -434,9 +447,6 @@ __device__ __forceinline__ void clear_unstored(const BinWorkspace &ws, const Cle
     if (grad_dist != nullptr) clear_rows_of_wave(grad_dist, i0, dist_row_bytes, clear_mine, lane);
   }
 }
-
-// work items of a bin with c points (most bins fit one item, which saves the division)
-__device__ __forceinline__ int items_of_bin(int c, int ch) { return c <= ch ? (c > 0 ? 1 : 0) : (c + ch - 1) / ch; }
 
 // The first `scan_blocks` blocks scan, 1024 bins each (in turns if there are more bins than that).  A block needs no
 // word from the blocks before it: it adds up the counts of all bins before its own (a few dozen loads per thread for
@@ -449,7 +459,7 @@ __global__ __launch_bounds__(1024, 8) void bin_scan_kernel(BinWorkspace ws, Clea
     return;
   }
   __shared__ int s_pts[16], s_chk[16], s_bp[16], s_bc[16];
-  const int n = ws.plan->total_bins, ch = ws.plan->chunk, per_class = ws.plan->bins_per_class;
+  const int n = ws.plan->total_bins, ch = chunk_of(ws, *ws.plan), per_class = ws.plan->bins_per_class;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   for (int base = (int)blockIdx.x * 1024; base < n; base += scan_blocks * 1024) {
     // points and work items of the bins before this block's: every thread its share, summed over the wavefront
@@ -477,8 +487,12 @@ __global__ __launch_bounds__(1024, 8) void bin_scan_kernel(BinWorkspace ws, Clea
     if (i < n) {
       if (i % per_class == 0) ws.plan->class_start[i / per_class] = run_c;
       ws.cursor[i] = run_p;
-      for (int t = 0; t < k; ++t)
-        ws.items[run_c + t] = make_int4(i, run_p + t * ch, min(ch, c - t * ch), k);
+      if (k == 1) ws.items[run_c] = make_int4(i, run_p, c, 1);
+      for (int t = 0, begin = 0; k > 1 && t < k; ++t) {
+        const int end = share_begin(c, k, t + 1);
+        ws.items[run_c + t] = make_int4(i, run_p + begin, end - begin, k);
+        begin = end;
+      }
       if (i == n - 1) {
         ws.plan->total_chunks = run_c + k;
         ws.plan->class_start[kClasses] = run_c + k;
@@ -1139,10 +1153,6 @@ static int max_bins_per_bm(int S, int L, int ty, int tx) {
 }
 
 constexpr int kMinChunk = 64;        // smallest accepted points-per-item
-// Points of a bin per work item.  A bin that fits one item is flushed with stores instead of atomic adds, so
-// large items pay; the queues are served from their ends so that the heavy bins of the coarse levels do not
-// come last.  Measured at the BEVFormer-base shape: 1024 -> 2.01 ms, 2048 -> 1.87, 4096 -> 1.83, 8192 -> 1.92.
-constexpr int kDefaultChunk = 4096;
 // only the fused entry point sets dist_heads
 static bool shared_dist(const BwdArgs &a) { return a.dist_heads == 1 && a.M > 1; }
 
@@ -1246,25 +1256,23 @@ static size_t tile_lds_bytes(int kind, int ty, int tx, int C, int D, int pp) {
 //   * tiles above 8x16 pixels lose (the rows phase needs several rounds); passes of 64 points lose to 128 and 256;
 //   * an 8x8 tile at pp 128 beats a 4x8 tile at pp 256 (128 bins: 0.68 against 0.74 ms for 2.56 M points) unless
 //     most tiles take several passes (`dense`: the dense BEV workload, 41 points per pixel, 7.0 against 8.9 ms).
-static TileConfig pick_tile_config(int kind, int C, int D, int tile_hint, int block_hint, int pass_hint, bool dense,
+static TileConfig pick_tile_config(int kind, int C, int D, int elem, int tile_hint, int block_hint, int pass_hint, bool dense,
                                    bool cells_wanted) {
   TileConfig c;
   c.cells = false;
-  if (cells_wanted && kind != 2 && (block_hint == 0 || block_hint == 512) && (pass_hint == 0 || pass_hint == 256)) {
-    // The cell-owned kernel (rows of 32 channels): the largest tile of at most 64 pixels whose depth tile leaves
-    // room for two workgroups per CU, else for one.
-    static const int order[][2] = {{8, 8}, {6, 8}, {4, 8}, {4, 4}, {2, 4}, {2, 2}, {1, 1}};
-    const int hy = tile_hint / 100, hx = tile_hint % 100;
-    // two workgroups per CU: half of the 160 KB less the kernel's static LDS (a depth tile of 112 bins on 8x8 pixels
-    // just fits; 128 bins would fit on 8x7 pixels, which is no faster than 6x8 on the dense workload: 5.66 against 5.65 ms)
+  if (cells_wanted && kind != 2 && C <= 64 && (block_hint == 0 || block_hint == cell_kernel_block(C)) &&
+      (pass_hint == 0 || pass_hint == cell_kernel_pass(C))) {
+    // The cell-owned kernel: the tallest tile whose depth tile leaves room for two workgroups per CU (half of the 160 KB
+    // less the kernel's static LDS: 8x8 pixels up to 112 bins, 7x8 with 128), else for one.
+    const int hy = tile_hint / 100, hx = tile_hint % 100, Dk = kind == 1 ? 0 : D;
     for (size_t budget : {cell_kernel_half_cu_lds(), (size_t)150 * 1024}) {
-      for (auto &t : order) {
-        const int ty = tile_hint > 0 ? hy : t[0], tx = tile_hint > 0 ? hx : t[1];
-        const int Dk = kind == 1 ? 0 : D;
-        if (cell_kernel_applies(C, Dk, ty, tx, kind == 0) && cell_kernel_lds_bytes(ty, tx, Dk) <= budget) {
-          c.cells = true; c.block = 512; c.pp = 256; c.ty = ty; c.tx = tx; c.lds = cell_kernel_lds_bytes(ty, tx, Dk);
+      for (int ty = tile_hint > 0 ? hy : cell_max_ty(C); ty >= 1; --ty) {
+        if (cell_kernel_applies(C, ty, tile_hint > 0 ? hx : kCellTX) && cell_kernel_lds_bytes(ty, C, Dk, elem) <= budget) {
+          c.cells = true; c.block = cell_kernel_block(C); c.pp = cell_kernel_pass(C); c.ty = ty; c.tx = kCellTX;
+          c.lds = cell_kernel_lds_bytes(ty, C, Dk, elem);
           return c;
         }
+        if (tile_hint > 0) break;
       }
     }
   }
@@ -1304,10 +1312,12 @@ static TileConfig pick_tile_config(int kind, int C, int D, int tile_hint, int bl
 }
 
 static int bwd_kind(const BwdArgs &a) { return a.dist != nullptr ? 0 : 1; }
-static TileConfig tile_config_of(const BwdArgs &a, int kind) {
+static TileConfig tile_config_of(const BwdArgs &a, int kind, int dtype) {
   const double per_pixel = (double)a.Q * a.L * a.P / (a.S > 0 ? a.S : 1);      // sampling points per pixel of a (batch, head)
   // a caller that names the channels per lane asks for the row-owned kernel, whose tiling that is
-  return pick_tile_config(kind, a.C, a.D, a.tile_hint, a.block_hint, a.pass_hint, per_pixel >= 16.0, a.vec_hint == 0);
+  // (its per-point gradients are buffer-addressed per batch element: below 2^31 bytes of 16 per point)
+  const bool cells = a.vec_hint == 0 && (size_t)a.Q * a.M * a.L * a.P * 16 < (size_t)kNoRow;
+  return pick_tile_config(kind, a.C, a.D, dtype == DFA3D_F32 ? 4 : 2, a.tile_hint, a.block_hint, a.pass_hint, per_pixel >= 16.0, cells);
 }
 
 static size_t workspace_bytes_for(const BwdArgs &a, int kind, int dtype) {
@@ -1315,7 +1325,7 @@ static size_t workspace_bytes_for(const BwdArgs &a, int kind, int dtype) {
   if ((size_t)a.B * a.Q * a.M * a.L * a.P >= (1ull << 31)) return 0;          // point indices and segment offsets are 32-bit
   if (kind != 2 && (size_t)a.Q * a.M * a.C * 4 >= (size_t)kMaxSliceBytes) return 0;   // grad_out rows are buffer-addressed per batch element
   if (a.grad_bf16 && (kind != 0 || ((a.C | a.D) & 3) != 0)) return 0;          // bfloat16 gradients: whole 8-byte groups
-  const TileConfig c = tile_config_of(a, kind);
+  const TileConfig c = tile_config_of(a, kind, dtype);
   if (c.lds > 150 * 1024) return 0;                                            // rows too long for LDS tiles
   return bin_layout(a, c.ty, c.tx).total;
 }
@@ -1401,8 +1411,9 @@ static hipError_t launch_tile_typed(const BwdArgs &a, const BinWorkspace &ws, co
                                     hipStream_t stream) {
   if (c.cells) {
     const int dtype = sizeof(T) == 4 ? DFA3D_F32 : DFA3D_BF16;
-    if (hipError_t e = allow_lds(cell_kernel_symbol(dtype, a.dist != nullptr), c.lds)) return e;
-    return launch_cell_kernel(a, dtype, ws, c.lds, tile_grid(c.lds, c.block), gd_heads, stream);
+    if (hipError_t e = allow_lds(cell_kernel_symbol(dtype, a.C, a.dist != nullptr), c.lds)) return e;
+    // two workgroups per CU at most (its registers): a workgroup that had to wait for a place would sit on dealt items
+    return launch_cell_kernel(a, dtype, ws, c.lds, tile_grid(c.lds < 80 * 1024 ? 80 * 1024 : c.lds, c.block), gd_heads, stream);
   }
   // Eight channels per lane when the tile has more rows than four-channel row groups (a 9x9 tile against 64
   // groups of 8 lanes): 128 groups of 4 lanes then cover it in one round with fewer instructions per corner
@@ -1436,10 +1447,13 @@ static BinWorkspace carve_workspace(void *workspace, const BinLayout &lay) {
 
 // plan, count, scan, fill.  `a` supplies dimensions, shapes, locations and the per-point gradient
 // buffers that receive zeros for points the operator skips.
-static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, int ty, int tx, float *gd_heads, hipStream_t stream) {
+static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, const TileConfig &cfg, float *gd_heads, hipStream_t stream) {
+  // gradients stored in bfloat16 are rounded at every atomic add: their bins are split no more than they have to be
+  const int chunk = a.chunk_hint > 0 ? a.chunk_hint : a.grad_bf16 ? kMaxChunk : 0;
+  const int ty = cfg.ty, tx = cfg.tx;
   const int mb = max_bins_per_bm(a.S, a.L, ty, tx);
   hipLaunchKernelGGL(plan_and_clear_kernel, dim3(64), dim3(256), 0, stream, ws, a.shapes, a.shape_stride, a.level_start,
-                     a.L, a.S, (a.dist != nullptr || a.C == 0) ? a.D : 0, a.B, a.M, ty, tx, a.chunk_hint > 0 ? a.chunk_hint : kDefaultChunk, mb);
+                     a.L, a.S, (a.dist != nullptr || a.C == 0) ? a.D : 0, a.B, a.M, ty, tx, chunk, mb);
   const int q_blocks = (a.Q + kBinQueries - 1) / kBinQueries;
   const long long blocks = (long long)a.B * a.M * q_blocks;
   if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
@@ -1469,7 +1483,7 @@ static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, int ty, 
     if (gd_heads != nullptr) { ca.grad_dist = reinterpret_cast<char *>(gd_heads); ca.dist_row_bytes = a.D * 4; }
     else if (a.dist != nullptr) { ca.grad_dist = static_cast<char *>(a.grad_dist); ca.dist_row_bytes = a.D * ge; }
     ca.B = a.B; ca.S = a.S; ca.M = a.M; ca.L = a.L;
-    ca.stores = ((a.C | (a.dist != nullptr ? a.D : 0)) & 3) == 0 ? 1 : 0;        // the tile kernel's own condition
+    ca.stores = (cfg.cells || ((a.C | (a.dist != nullptr ? a.D : 0)) & 3) == 0) ? 1 : 0;        // the tile kernel's own condition
     const size_t rows = (size_t)a.B * a.S * a.M;
     clear_blocks = (unsigned)((rows + 1023) / 1024 < 4096 ? (rows + 1023) / 1024 : 4096);
   }
@@ -1506,7 +1520,7 @@ hipError_t launch_backward_binned(const BwdArgs &a, int dtype, void *workspace, 
     // or the direct kernels (which clear everything) take the call
     if ((((uintptr_t)a.grad_value | (uintptr_t)a.grad_dist) & 15) != 0) return hipErrorNotSupported;
   }
-  const TileConfig cfg = tile_config_of(a, kind);
+  const TileConfig cfg = tile_config_of(a, kind, dtype);
   const BinLayout lay = bin_layout(a, cfg.ty, cfg.tx);
   const BinWorkspace ws = carve_workspace(workspace, lay);
   float *gd_heads = shared_dist(a) ? reinterpret_cast<float *>(static_cast<char *>(workspace) + lay.gd_heads) : nullptr;
@@ -1516,7 +1530,7 @@ hipError_t launch_backward_binned(const BwdArgs &a, int dtype, void *workspace, 
   constexpr int stage = 0;
 #endif
   if (stage == 0 || stage == 1) {
-    if (hipError_t e = run_binning(a, ws, cfg.ty, cfg.tx, gd_heads, stream)) return e;
+    if (hipError_t e = run_binning(a, ws, cfg, gd_heads, stream)) return e;
   }
   if (a.event_binned != nullptr) {
     if (hipError_t e = hipEventRecord((hipEvent_t)a.event_binned, stream)) return e;
@@ -1553,9 +1567,9 @@ hipError_t launch_depth_score_backward_binned(const DepthScoreBwdArgs &d, int dt
   const size_t need = workspace_bytes_for(a, 2, dtype);
   if (need == 0 || workspace == nullptr || workspace_bytes < need || ((uintptr_t)workspace & 255) != 0)
     return hipErrorNotSupported;
-  const TileConfig cfg = tile_config_of(a, 2);
+  const TileConfig cfg = tile_config_of(a, 2, dtype);
   const BinWorkspace ws = carve_workspace(workspace, bin_layout(a, cfg.ty, cfg.tx));
-  if (hipError_t e = run_binning(a, ws, cfg.ty, cfg.tx, nullptr, stream)) return e;
+  if (hipError_t e = run_binning(a, ws, cfg, nullptr, stream)) return e;
   if (event_binned != nullptr) {
     if (hipError_t e = hipEventRecord((hipEvent_t)event_binned, stream)) return e;
   }

@@ -1,44 +1,42 @@
-// Tile kernel of the binned backward for rows of 32 channels: cell-owned lane groups and two kinds of wavefronts.
+// Tile kernel of the binned backward for rows of up to 64 channels: cell-owned lane groups and two kinds of wavefronts.
 //
 // The bins, work items and queues are those of dfa3d_backward_binned.hip; only the work inside a tile differs.
-// A tile of TY x TX pixels (at most 64) is seen as its "cells": the points whose base pixel (upper left of the
-// four pixels around the location) is that pixel.  All points of a cell touch the same four value rows, so
-//   * a group of 4 lanes (8 channels each) owns a cell for the whole work item: the four value rows and the four
-//     accumulators of weight * grad_out live in its registers, every point's grad_out row is read from LDS
-//     once, the four dot products and the four weighted sums are formed from it, and nothing is added to an LDS
-//     tile during the passes (the accumulators of the cells are put together once, when the item ends);
-//   * a pass sorts its 256 points by cell: one integer LDS atomic per point.
+// A tile of TY x 8 pixels is seen as its "cells": the points whose base pixel (upper left of the four pixels around
+// the location) is that pixel.  All points of a cell touch the same four value rows, so
+//   * a group of LPR lanes (VEC channels each) owns a cell for the whole work item: the four value rows and the four
+//     accumulators of weight * grad_out live in its registers, every point's grad_out row is read from LDS once, the
+//     four dot products and the four weighted sums are formed from it, and nothing is added to an LDS tile during the
+//     passes.  The weighted sums are outer products (4 corners x channels, one point deep) of 4-lane blocks: one
+//     v_mfma_f32_4x4x1 per channel of a lane does what four FMAs per lane would, on the matrix pipe;
+//   * a pass sorts its points (256, or 128 with long rows) by cell: one integer LDS atomic per point.
 // (Base pixels run from -1, for a location within half a pixel of the map's upper or left edge, to H - 1 / W - 1;
 // the tiles are laid over that range, so a cell's upper or left pixels may lie outside the map like its lower or
 // right ones: such corners carry weight zero, their value rows read as zero and their sums are never written.)
 //
-// The 8 wavefronts of a workgroup have two roles.  "Walkers" (wavefronts 0-3, 16 cells each) stage the grad_out
-// rows of a pass in LDS and walk the cells' lists; "pointers" (wavefronts 4-7, one point of the pass per thread)
-// do everything that is per point: geometry, depth taps, corner weights, the sort, and afterwards the point's
-// gradients and its grad_dist taps into the LDS depth tile.  The two roles meet at two barriers per pass and
-// otherwise overlap: while the walkers walk pass i the pointers prepare pass i + 1, while the walkers stage pass
-// i + 1 the pointers finish pass i.
-//   phase X(t):  walkers: walk(t-1)                 pointers: late taps of pass t-2, then prepare(t)
-//   phase Y(t):  walkers: stage(t)                  pointers: place(t) (scan + sorted records), finish(t-1)
-// grad_dist taps go to the LDS tile as in the row-owned kernel: the first tap at an address in a pass adds with a
-// plain read-modify-write, later ones use the LDS float atomic one phase later; who is first is decided by an
-// integer atomic on a bitmap with one bit per tile address.
+// The 8 wavefronts of a workgroup have two roles.  "Walkers" (wavefronts 0-3, one or two tile rows of 8 cells each)
+// walk the cells' lists; "pointers" (wavefronts 4-7, one point of the pass per thread) do everything that is per point:
+// geometry, depth taps, corner weights, the sort, bringing its grad_out row to LDS, and afterwards the point's gradients
+// and its grad_dist taps into the LDS depth tile.  The roles meet at two barriers per turn and
+// otherwise overlap.  Turns follow one another without a gap, whatever item their passes belong to (pass t: one of
+// the item's passes), so that an item of a single pass costs a single turn:
+//   phase X(t):  walkers: walk(t-1)        pointers: scores and corner weights of t, prepare(t+1)
+//   phase Y(t):  walkers: flush            pointers: stage(t), place(t) (scan + sorted slots), finish(t-1)
+// and where pass t-1 was its item's last:
+//   Y(t):    walkers ask for the value rows of the item of pass t and put the old item's corner sums together in
+//            registers (neighbouring cells are neighbouring lane groups); sums that cross into the next wavefront's rows
+//            go through a few rows of LDS and out in X(t+1)
+//   X(t+1):  everybody flushes the depth tile, before the first finish of the next item in Y(t+1)
+// grad_dist taps go to the LDS tile by compare-and-swap on the word's bits: the LDS float atomic retires 0.33 lanes per
+// clock and CU, read + compare-and-swap 2.9 (and a tap is complete when its phase ends, which the flush relies on).
 //
 // Semantics are those of bwd_attention_kernel (dfa3d_backward.hip holds the formulas and the reference lines).
 #include "dfa3d_binned.h"
 
 namespace dfa3d {
 
-constexpr int kCellBlock = 512;       // threads: wavefronts 0-3 walk, 4-7 own the points
-constexpr int kCellPass = 256;        // points per pass: one per pointer thread
-constexpr int kCellC = 32;            // channels: 4 lanes of 8
-constexpr int kCellMax = 64;          // cells per tile: 4 walker wavefronts of 16 groups
-#ifndef DFA3D_CELL_GPITCH
-#define DFA3D_CELL_GPITCH 32
-#endif
-constexpr int kGPitch = DFA3D_CELL_GPITCH;       // words between staged grad_out rows
-// the row of zeros behind the staged rows must also lie behind the accumulators that take their place when an item ends
-static_assert(kCellMax * 4 * kCellC <= kCellPass * kGPitch, "accumulators would overwrite the row of zeros");
+typedef unsigned int u32x3 __attribute__((ext_vector_type(3)));
+
+constexpr int kWalkers = 256;         // threads of the walker wavefronts 0-3; the wavefronts after them own the points
 
 #ifdef DFA3D_TILE_TIMING
 // thread 0 (a walker) clocks slots 0-7, thread 256 (a pointer) slots 8-15
@@ -51,28 +49,52 @@ static_assert(kCellMax * 4 * kCellC <= kCellPass * kGPitch, "accumulators would 
 #define CT_FLUSH() do { } while (0)
 #endif
 
+// Lane groups by row length: LPR lanes of VEC channels per row, 64 / LPR cells per wavefront; points per pass, one per
+// pointer thread (256 staged rows of 64 channels would leave room for one workgroup per CU only).
+struct CellShape { int vec, lpr, pass; };
+__host__ __device__ constexpr int cell_pass(int lpr) { return lpr == 4 ? 256 : 128; }
+__host__ __device__ inline CellShape cell_shape(int C) {
+  return C <= 16 ? CellShape{4, 4, cell_pass(4)} : C <= 32 ? CellShape{8, 4, cell_pass(4)} : CellShape{8, 8, cell_pass(8)};
+}
+// the most tile rows of 8 cells that four walker wavefronts own
+int cell_max_ty(int C) { return 4 * (kWave / cell_shape(C).lpr) / kCellTX; }
+
+// The rim of a tile of (ty + 1) x 9 pixels, numbered: row 0, row ty, then the first and last pixel of the rows between.
+__host__ __device__ inline int rim_pixels(int ty) { return 2 * (kCellTX + 1) + 2 * (ty - 1); }
+__device__ __forceinline__ int rim_index(int row, int col, int ty) {
+  return row == 0 ? col : row == ty ? kCellTX + 1 + col : 2 * (kCellTX + 1) + 2 * (row - 1) + (col == 0 ? 0 : 1);
+}
+__device__ __forceinline__ void rim_decode(int i, int ty, int &row, int &col) {
+  const int s = i - 2 * (kCellTX + 1);
+  row = s >= 0 ? 1 + (s >> 1) : i <= kCellTX ? 0 : ty;
+  col = s >= 0 ? ((s & 1) ? kCellTX : 0) : i <= kCellTX ? i : i - (kCellTX + 1);
+}
+
 struct CellLds {      // offsets (in 4-byte words) into the dynamic LDS block
-  int gd, bits, gstage, sw, sslot, dots, cnt, offs, goff, total;
+  int gd, gstage, dots, sslot, cnt, offs, goff, cross, rim, total;
 };
-__host__ __device__ inline CellLds cell_lds_layout(int ty, int tx, int D) {
+__host__ __device__ inline CellLds cell_lds_layout(int ty, int row, int cells, int pass, int D, int elem) {
   CellLds o;
-  const int R = (ty + 1) * (tx + 1);
+  const int R = (ty + 1) * (kCellTX + 1);
   o.gd = 0;
-  o.bits = (o.gd + R * D + 3) & ~3;
-  o.gstage = (o.bits + (R * D + 31) / 32 + 3) & ~3;          // 16-byte aligned rows
-  // kCellPass staged rows and a row of zeros; when the item ends the same words hold the cells' accumulators
-  const int stage_words = (kCellPass + 1) * kGPitch, acc_words = kCellMax * 4 * kCellC;
-  o.sw = o.gstage + (stage_words > acc_words ? stage_words : acc_words);
-  o.sslot = o.sw + kCellPass * 4;
-  o.dots = o.sslot + kCellPass / 2;                          // 16-bit point slots
-  o.cnt = o.dots + kCellPass * 4;
-  o.offs = o.cnt + 2 * kCellMax;
-  o.goff = o.offs + kCellMax + 1;
-  o.total = o.goff + kCellPass;
+  o.gstage = (o.gd + R * D + 3) & ~3;                        // 16-byte aligned rows
+  o.dots = o.gstage + (pass + 1) * row * elem / 4;           // the staged rows, as they lie in memory, and a row of zeros
+  o.sslot = o.dots + (pass + 1) * 4;                    // corner weights, then dot products; four zeros at the end
+  o.cnt = o.sslot + (pass + 2) / 2;                     // 16-bit point slots; the one at the end names the row of zeros
+  o.offs = o.cnt + 3 * cells;
+  o.goff = o.offs + cells + 1;
+  o.cross = (o.goff + 2 * pass + 3) & ~3;                   // sums that cross into the next wavefront's tile rows
+  o.rim = o.cross + 3 * (kCellTX + 1) * row;                 // sums of the tile's rim pixels, on their way out
+  o.total = o.rim + rim_pixels(ty) * row;
   return o;
 }
 
-size_t cell_kernel_lds_bytes(int ty, int tx, int D) { return (size_t)cell_lds_layout(ty, tx, D).total * 4; }
+int cell_kernel_pass(int C) { return cell_shape(C).pass; }
+int cell_kernel_block(int C) { return kWalkers + cell_shape(C).pass; }
+size_t cell_kernel_lds_bytes(int ty, int C, int D, int elem) {
+  const CellShape s = cell_shape(C);
+  return (size_t)cell_lds_layout(ty, s.vec * s.lpr, 4 * kWave / s.lpr, s.pass, D, elem).total * 4;
+}
 
 // what a pointer thread keeps of its point between the phases
 struct PointState {
@@ -82,13 +104,11 @@ struct PointState {
   unsigned bits;              // bit k: corner k inside the map; 4: depth inside; 5, 6: lower, upper tap exists; 7: live;
                               // 8-13: the point's cell; 16-31: lower depth bin + 1
 };
-// the taps of a finished point that found their address taken: added atomically one phase later
-struct LateTaps {
-  float gs[4], hd, ld;        // gradient at each corner's score; weights of the lower and the upper bin
-  unsigned pack;              // bit j: tap j (corner j / 2, lower / upper bin) is still to be added; 8-13: cell; 16-31: lower bin + 1
-};
 // Queue state of the thread that fetches the work items: the item taken now was popped two items ago and its two
-// records asked for one item ago, so neither the queue atomic nor the loads are waited for.
+// records asked for one item ago, so neither the queue atomic nor the loads are waited for.  A workgroup's first
+// kDealt items are dealt, not popped (its number among the workgroups of its class says which), so that a workgroup
+// starts after one round trip to memory instead of one for each item it looks ahead.
+constexpr int kDealt = 4;
 struct CellFetch {
   int classes_done, w_next;
   int4 rec, geo;
@@ -96,23 +116,36 @@ struct CellFetch {
     rec = w >= 0 ? ws.items[w] : make_int4(-1, 0, 0, 0);
     geo = w >= 0 ? ws.geom[w] : make_int4(0, 0, 0, 0);
   }
-  __device__ __forceinline__ void start(const BinWorkspace &ws, const BinPlan &p, int home) {
-    classes_done = 0;
-    const int w = pop_item(ws, p, home, classes_done);
-    load(ws, w);
-    w_next = w >= 0 ? pop_item(ws, p, home, classes_done) : -1;
+  __device__ __forceinline__ int pop(const BinWorkspace &ws, const BinPlan &p) {
+    return pop_item(ws, p, blockIdx.x % kClasses, classes_done, kDealt);
   }
-  __device__ __forceinline__ void advance(const BinWorkspace &ws, const BinPlan &p, int home, int4 *r, int4 *g) {
+  __device__ __forceinline__ void start(const BinWorkspace &ws, const BinPlan &p, int4 (&r)[kDealt - 1], int4 (&g)[kDealt - 1]) {
+    const int c = blockIdx.x % kClasses, lo = p.class_start[c], hi = p.class_start[c + 1], n_wg = workgroups_of_class(c);
+    int w[kDealt];
+    classes_done = 0;
+    for (int k = 0; k < kDealt; ++k) w[k] = hi - 1 - ((int)blockIdx.x / kClasses + k * n_wg);
+    for (int k = 0; k < kDealt; ++k)
+      if (w[k] < lo) w[k] = pop(ws, p);                     // the class has no more: another one's
+    for (int k = 0; k < kDealt - 1; ++k) {
+      load(ws, w[k]);
+      r[k] = rec; g[k] = geo;
+    }
+    load(ws, w[kDealt - 1]);
+    w_next = w[kDealt - 1] >= 0 ? pop(ws, p) : -1;
+  }
+  __device__ __forceinline__ void advance(const BinWorkspace &ws, const BinPlan &p, int4 *r, int4 *g) {
     *r = rec; *g = geo;
     load(ws, w_next);
-    w_next = w_next >= 0 ? pop_item(ws, p, home, classes_done) : -1;
+    w_next = w_next >= 0 ? pop(ws, p) : -1;
   }
 };
 // a work item, decoded
 struct ItemGeom { int bin, seg, n_item, chunks, b, m, H, W, Dd, start, y0, x0; };
-// what the kernel declares as static LDS (level tables, the fetching thread's state, three item records): the dynamic
+constexpr int kItemSlots = 8;      // a power of two; in use: the item before (finish, flush), this one and the next three
+__device__ __forceinline__ int slot_of_item(int it) { return it & (kItemSlots - 1); }
+// what the kernel declares as static LDS (level tables, the fetching thread's state, item records): the dynamic
 // block of each of two workgroups on a CU may be half of the CU's 160 KB less this
-constexpr size_t kCellStaticLds = 4 * DFA3D_MAX_LEVELS * sizeof(int) + sizeof(CellFetch) + 3 * sizeof(ItemGeom);
+constexpr size_t kCellStaticLds = 4 * DFA3D_MAX_LEVELS * sizeof(int) + sizeof(CellFetch) + kItemSlots * sizeof(ItemGeom);
 size_t cell_kernel_half_cu_lds() { return 80 * 1024 - kCellStaticLds; }
 // an item record read from LDS is the same in every lane: keep it in scalar registers
 __device__ __forceinline__ ItemGeom uniform(const ItemGeom &g) {
@@ -126,7 +159,7 @@ __device__ __forceinline__ ItemGeom uniform(const ItemGeom &g) {
   return u;
 }
 
-// Four partial sums per lane (one per corner) over the four lanes of a group: lane c gets the whole sum of corner c.
+// Four partial sums per lane (one per corner) over the four lanes of a quad: lane c gets the whole sum of corner c.
 // Two exchange steps in which every lane passes on the two (then one) partial sums its partner collects.
 __device__ __forceinline__ float quad_corner_sum(float d0, float d1, float d2, float d3, bool odd, bool upper) {
   const float keep_a = odd ? d1 : d0, send_a = odd ? d0 : d1, keep_b = odd ? d3 : d2, send_b = odd ? d2 : d3;
@@ -136,124 +169,264 @@ __device__ __forceinline__ float quad_corner_sum(float d0, float d1, float d2, f
   return keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(send), 0x4E, 0xF, 0xF, true));               // quad_perm [2,3,0,1]
 }
 
+// The channels of one lane of a row of C elements, in NG groups of four.  Rows of 4-byte elements: group g covers
+// channels 4 (LPR g + cl) .. + 3, so that the lanes of a row read whole 64-byte pieces together; 2-byte elements: VEC
+// consecutive channels.  A group beyond C reads as zero and is never written.
+template <typename T, int VEC, int LPR> struct LaneChannels {
+  static constexpr int NG = VEC / 4;
+  int first[NG];            // first channel of each group
+  uint32_t off[NG];         // its byte offset inside a row, kNoChan beyond the last channel
+  bool c8;
+  __device__ __forceinline__ LaneChannels(int cl, int C) : c8((C & 7) == 0) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      first[g] = sizeof(T) == 4 ? 4 * (LPR * g + cl) : VEC * cl + 4 * g;
+      off[g] = first[g] < C ? (uint32_t)(first[g] * (int)sizeof(T)) : kNoChan;
+    }
+  }
+  // the lane's elements as they lie in memory
+  struct Raw { uint32_t w[VEC * (int)sizeof(T) / 4]; };
+  __device__ __forceinline__ void load(rsrc_t r, uint32_t row, Raw &o) const {
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r, row + off[g], 0, 0);
+        o.w[4 * g] = t.x; o.w[4 * g + 1] = t.y; o.w[4 * g + 2] = t.z; o.w[4 * g + 3] = t.w;
+      }
+    } else {
+      if (VEC == 8 && c8) {                                  // uniform
+        const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r, row + off[0], 0, 0);
+        o.w[0] = t.x; o.w[1] = t.y;
+        if constexpr (VEC == 8) { o.w[2] = t.z; o.w[3] = t.w; }
+      } else {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+          const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(r, row + off[g], 0, 0);
+          o.w[2 * g] = t.x; o.w[2 * g + 1] = t.y;
+        }
+      }
+    }
+  }
+  static __device__ __forceinline__ void to_float(const Raw &r, float (&v)[VEC]) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      if constexpr (sizeof(T) == 4) v[i] = __uint_as_float(r.w[i]);
+      else v[i] = __uint_as_float((i & 1) ? r.w[i / 2] & 0xFFFF0000u : r.w[i / 2] << 16);
+    }
+  }
+  // the same lane's place in a row staged in LDS
+  __device__ __forceinline__ void put(T *row, const Raw &r) const {
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if constexpr (sizeof(T) == 4) *reinterpret_cast<uint4 *>(row + first[g]) = make_uint4(r.w[4 * g], r.w[4 * g + 1], r.w[4 * g + 2], r.w[4 * g + 3]);
+      else *reinterpret_cast<uint2 *>(row + first[g]) = make_uint2(r.w[2 * g], r.w[2 * g + 1]);
+    }
+  }
+  __device__ __forceinline__ void get(const T *row, Raw &r) const {
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const uint4 t = *reinterpret_cast<const uint4 *>(row + first[g]);
+        r.w[4 * g] = t.x; r.w[4 * g + 1] = t.y; r.w[4 * g + 2] = t.z; r.w[4 * g + 3] = t.w;
+      }
+    } else if constexpr (VEC == 8) {
+      const uint4 t = *reinterpret_cast<const uint4 *>(row + first[0]);
+      r.w[0] = t.x; r.w[1] = t.y; r.w[2] = t.z; r.w[3] = t.w;
+    } else {
+      const uint2 t = *reinterpret_cast<const uint2 *>(row + first[0]);
+      r.w[0] = t.x; r.w[1] = t.y;
+    }
+  }
+};
+
+// The two taps (bins db, db + 1) of each of a point's four corners, asked for one phase before they are looked at.
+template <typename T> struct TapsInFlight {
+  u32x2 t[4];
+  // off: byte offset of bin db of each corner's distribution, kNoRow where there is nothing to fetch
+  __device__ __forceinline__ void ask(rsrc_t r, const uint32_t (&off)[4], int D) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if constexpr (sizeof(T) == 4) {
+        t[k] = __builtin_amdgcn_raw_buffer_load_b64(r, off[k], 0, 0);
+      } else if ((D & 1) == 0) {                             // uniform: see BufPair<__hip_bfloat16>::ld_word_aligned
+        t[k] = __builtin_amdgcn_raw_buffer_load_b64(r, off[k] == kNoRow ? kNoRow : (off[k] & ~3u), 0, 0);
+      } else {
+        t[k].x = __builtin_amdgcn_raw_buffer_load_b16(r, off[k], 0, 0);
+        t[k].y = __builtin_amdgcn_raw_buffer_load_b16(r, off[k] == kNoRow ? kNoRow : off[k] + 2, 0, 0);
+      }
+    }
+  }
+  __device__ __forceinline__ void get(int k, int db, int D, float &x, float &y) const {
+    if constexpr (sizeof(T) == 4) {
+      x = __uint_as_float(t[k].x); y = __uint_as_float(t[k].y);
+    } else if ((D & 1) == 0) {                               // rows start on words: the pair's place depends on the bin alone
+      const uint32_t lo = t[k].x, hi = t[k].y;
+      x = (db & 1) ? __uint_as_float(lo & 0xFFFF0000u) : __uint_as_float(lo << 16);
+      y = (db & 1) ? __uint_as_float(hi << 16) : __uint_as_float(lo & 0xFFFF0000u);
+    } else {
+      x = bf16_bits_to_float(t[k].x); y = bf16_bits_to_float(t[k].y);
+    }
+  }
+};
+
+// 16 bytes per lane from a buffer to consecutive LDS addresses (`lds`: the wavefront's first byte).  Written out because
+// behind the builtin the compiler waits for the data before the next LDS read of any kind; here wait_for_loads() /
+// wait_for_all_but_two() do, when the phase ends.  (The compiler does not count these loads: where it waits for an older
+// one, it waits for more than it has to, never for less.)
+__device__ __forceinline__ void load_to_lds16(rsrc_t r, const void *lds, uint32_t off) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)lds);
+  uint32_t kept;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
+               : "=&s"(kept) : "s"(at), "v"(off), "s"(r) : "memory");
+#endif
+}
+__device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }           // vmcnt(0)
+__device__ __forceinline__ void wait_for_all_but_two() { __builtin_amdgcn_s_waitcnt(0x0F72); }     // vmcnt(2)
+
 // FUSED: both stages (depth scores recomputed from dist, grad_dist and the z gradient produced).
 // !FUSED: stage 2 alone: scores read from score_in, their gradient written to grad_score_out, no depth tile
 // (the launcher passes D = 0), grad_loc has gl_stride components of which x, y are written.
-template <typename T, bool FUSED>
-__global__ __launch_bounds__(kCellBlock, 4) void cell_backward_kernel(
+template <typename T, int VEC, int LPR, bool FUSED>
+__global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_kernel(
     BinWorkspace ws, const T *__restrict__ value, const T *__restrict__ dist, const T *__restrict__ score_in,
     const T *__restrict__ grad_out, const T *__restrict__ grad_score_in,
     void *__restrict__ grad_value, void *__restrict__ grad_dist, float *__restrict__ grad_loc, int gl_stride,
     float *__restrict__ grad_attn, float *__restrict__ grad_score_out, const float *__restrict__ grad_wu, int Md,
-    int Mg, int B, int S, int M, int D, int L, int Q, int P, int grad16 DFA3D_DIAG_PARAM) {
+    int Mg, int B, int S, int M, int C, int D, int L, int Q, int P, FastDiv div_lp, int grad16 DFA3D_DIAG_PARAM) {
   // grad16: bit 0 = grad_value is bfloat16, bit 1 = grad_dist is bfloat16 (else float)
   // Md: heads stored in dist (M, or 1 = shared by all heads); Mg: heads of the grad_dist buffer written here
-  constexpr int C = kCellC, PP = kCellPass, VEC = 8, LPR = 4;
+  constexpr int PP = cell_pass(LPR), BLOCK = kWalkers + PP, TX = kCellTX, TW = TX + 1, ROW = VEC * LPR;
+  constexpr int GPW = kWave / LPR, CELLS = 4 * GPW, ROWS = GPW / TX;      // cells and tile rows per walker wavefront
+  typedef float f4 __attribute__((ext_vector_type(4)));
   extern __shared__ __align__(16) float smem[];
   __shared__ int s_lv[4][DFA3D_MAX_LEVELS];              // the plan's level tables: H, W, Dd, first key
   __shared__ CellFetch s_fetch;                           // the fetching thread's queue state, between its turns
-  __shared__ ItemGeom s_geom[3];                         // the item before, this one and the next, decoded by the thread that fetches them
+  __shared__ ItemGeom s_geom[kItemSlots];                // items, decoded by the thread that fetches them
 
   const BinPlan &p = *ws.plan;
-  const int nb = p.bins_per_bm;
-  if (nb == 0) return;
-  const int TY = p.ty, TX = p.tx, TW = TX + 1, R = (TY + 1) * TW, n_cells = TY * TX;
-  const CellLds lay = cell_lds_layout(TY, TX, D);
+  if (p.bins_per_bm == 0) return;
+  const int TY = p.ty, R = (TY + 1) * TW;
+  const CellLds lay = cell_lds_layout(TY, ROW, CELLS, PP, D, (int)sizeof(T));
   const int tid = threadIdx.x, lane = tid % kWave;
   // The role is decided by a scalar, so that the compiler branches on it uniformly: a wavefront must never run
   // through the other role's code with all lanes switched off, because barriers count wavefronts, not lanes.
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const bool walker = wave < 4;
-  const int pslot = tid - PP;                              // pointers: the point slot of this thread
-  float *gd = smem + lay.gd, *gstage = smem + lay.gstage, *dots = smem + lay.dots;
-  uint32_t *bitmap = reinterpret_cast<uint32_t *>(smem + lay.bits);
-  float4 *s_w = reinterpret_cast<float4 *>(smem + lay.sw);
+  T *gstage = reinterpret_cast<T *>(smem + lay.gstage);
+  float *gd = smem + lay.gd, *dots = smem + lay.dots, *cross = smem + lay.cross, *rim = smem + lay.rim;
   uint16_t *s_slot = reinterpret_cast<uint16_t *>(smem + lay.sslot);
   int *cnt = reinterpret_cast<int *>(smem + lay.cnt), *offs = reinterpret_cast<int *>(smem + lay.offs);
   uint32_t *goff = reinterpret_cast<uint32_t *>(smem + lay.goff);
-  const int cl = lane % LPR;
-  const int cell = wave * (kWave / LPR) + lane / LPR;      // walkers: the cell of this lane group
-  const int LP = L * P;
-  const int n_bit_words = (R * D + 31) / 32;
   const bool gv16 = (grad16 & 1) != 0, gd16 = (grad16 & 2) != 0;          // uniform
 
-  for (int i = tid; i < lay.gstage; i += kCellBlock) smem[i] = 0;                   // depth tile and bitmap
-  for (int i = tid; i < 2 * kCellMax; i += kCellBlock) cnt[i] = 0;
+  for (int i = tid; i < lay.gstage; i += BLOCK) smem[i] = 0;                   // depth tile
+  for (int i = tid; i < 3 * CELLS; i += BLOCK) cnt[i] = 0;
+  for (int i = tid; i < ROW * (int)sizeof(T) / 4; i += BLOCK) smem[lay.gstage + PP * ROW * (int)sizeof(T) / 4 + i] = 0;   // what a group without a point reads
+  if (tid < 4) dots[PP * 4 + tid] = 0;
+  if (tid == 0) s_slot[PP] = (uint16_t)PP;
   if (tid < DFA3D_MAX_LEVELS) {      // decoding an item then costs no dependent loads from device memory
     s_lv[0][tid] = p.H[tid]; s_lv[1][tid] = p.W[tid]; s_lv[2][tid] = p.Dd[tid]; s_lv[3][tid] = p.start[tid];
   }
   __syncthreads();
   CT_DECL
 
-  // four consecutive elements at element index `e` of a batch slice of a gradient: stored, or added atomically
-  auto put4 = [&](char *base, rsrc_t r, bool is16, uint32_t e, const float4 &val, bool store, bool every) {
-    if (!is16) {
-      float *fb = reinterpret_cast<float *>(base);
-      if (store) {
-        *reinterpret_cast<float4 *>(fb + e) = val;                              // zeros too: full lines
-      } else {
-        if (every || val.x != 0) scatter_add(r, fb, e * 4, val.x);
-        if (every || val.y != 0) scatter_add(r, fb, e * 4 + 4, val.y);
-        if (every || val.z != 0) scatter_add(r, fb, e * 4 + 8, val.z);
-        if (every || val.w != 0) scatter_add(r, fb, e * 4 + 12, val.w);
+  // Gradient rows leave in two ways: stored, or added atomically.  The L2 executes about 20 G (instruction, 64-byte piece)
+  // pairs of float atomics per second on the whole part, whatever the number of floats in a pair: added rows go out
+  // one float (bfloat16: one pair) per lane on consecutive addresses, 16 to a pair (four floats per lane took four times
+  // the pairs: this kernel's flushes alone were worth 1 ms at the BEVFormer-base shape).
+
+  // The depth tile of the item in slot `which` goes out and is left zeroed, by `threads` threads of which this one is
+  // number `first`, in the phase in which nobody adds to the tile.  A tile row (one pixel) takes 2^sh threads; no
+  // divisions.  Pixels 1..TY-1 x 1..7 belong to no neighbour's halo: when the item held all the points of its bin they are
+  // stored, the others are added.
+  auto flush_gd = [&](int which, int first, int threads) {
+    const ItemGeom q = uniform(s_geom[which]);
+    const int mg = Mg == 1 ? 0 : q.m;
+    char *gdist_b = static_cast<char *>(grad_dist) + (size_t)q.b * S * Mg * D * (gd16 ? 2 : 4);
+    float *gdist_f = reinterpret_cast<float *>(gdist_b);
+    const rsrc_t gdist_r = make_rsrc(gdist_b, (size_t)S * Mg * D * sizeof(float));
+    const bool sole_d = q.chunks == 1 && Mg == M;       // a gradient shared by the heads collects from all of them
+    const bool d4 = (D & 3) == 0;
+    auto lanes_log2 = [](int n) { return n > 32 ? 6 : n > 16 ? 5 : n > 8 ? 4 : n > 4 ? 3 : 2; };
+    if (sole_d) {
+      const int n = d4 ? D >> 2 : D, sh = lanes_log2(n), inner = (TY - 1) * (TX - 1);
+      for (int i = first >> sh; i < inner; i += threads >> sh) {
+        const int ry = i / (TX - 1) + 1, rx = i % (TX - 1) + 1, r = ry * TW + rx;
+        const int y = q.y0 + ry, x = q.x0 + rx;
+        const bool out = y < q.H && x < q.W && !DFA3D_DIAG(diag, 4);
+        const uint32_t e0 = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D);
+        for (int c = first & ((1 << sh) - 1); c < n; c += 1 << sh) {
+          if (d4) {
+            float4 *at = reinterpret_cast<float4 *>(gd + r * D) + c;
+            const float4 val = *at;
+            *at = make_float4(0, 0, 0, 0);
+            if (out) {
+              if (gd16) *reinterpret_cast<uint2 *>(gdist_b + (size_t)(e0 + 4 * c) * 2) = make_uint2(pack_bf16x2(val.x, val.y), pack_bf16x2(val.z, val.w));
+              else *reinterpret_cast<float4 *>(gdist_f + e0 + 4 * c) = val;
+            }
+          } else {                                        // float gradients only (the launcher sees to it)
+            const float val = gd[r * D + c];
+            gd[r * D + c] = 0;
+            if (out) gdist_f[e0 + c] = val;
+          }
+        }
       }
-    } else {
-      char *dst = base + (size_t)e * 2;
-      if (store) {
-        *reinterpret_cast<uint2 *>(dst) = make_uint2(pack_bf16x2(val.x, val.y), pack_bf16x2(val.z, val.w));
+    }
+    const int n = gd16 ? D >> 1 : D, sh = lanes_log2(n);
+    const int rows = sole_d ? rim_pixels(TY) : R;
+    for (int i = first >> sh; i < rows; i += threads >> sh) {
+      int ry, rx;
+      if (sole_d) {
+        rim_decode(i, TY, ry, rx);
       } else {
-        if (val.x != 0 || val.y != 0) atomic_add_bf16x2(dst, val.x, val.y);
-        if (val.z != 0 || val.w != 0) atomic_add_bf16x2(dst + 4, val.z, val.w);
+        ry = i / TW; rx = i % TW;
+      }
+      const int r = ry * TW + rx, y = q.y0 + ry, x = q.x0 + rx;
+      const bool out = in_map(y, x, q.H, q.W) && !DFA3D_DIAG(diag, 4);
+      const uint32_t e0 = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D);
+      for (int c = first & ((1 << sh) - 1); c < n; c += 1 << sh) {
+        if (gd16) {
+          float2 *at = reinterpret_cast<float2 *>(gd + r * D) + c;
+          const float2 val = *at;
+          if (val.x != 0 || val.y != 0) {
+            *at = make_float2(0, 0);
+            if (out) atomic_add_bf16x2(gdist_b + (size_t)(e0 + 2 * c) * 2, val.x, val.y);
+          }
+        } else {
+          const float val = gd[r * D + c];
+          if (val != 0) {
+            gd[r * D + c] = 0;
+            if (out) scatter_add(gdist_r, gdist_f, (e0 + c) * 4, val);
+          }
+        }
       }
     }
   };
 
-  // The depth tile of the item in slot `which` goes out and is left zeroed: threads first, first + step, ... of the
-  // float4 groups (both roles share the work in the one phase in which nobody adds to the tile).
-  auto flush_gd = [&](int which, int first, int step) {
-const ItemGeom q = uniform(s_geom[which]);
-    const int mg = Mg == 1 ? 0 : q.m;
-    char *gdist_b = static_cast<char *>(grad_dist) + (size_t)q.b * S * Mg * D * (gd16 ? 2 : 4);
-    const rsrc_t gdist_r = make_rsrc(gdist_b, (size_t)S * Mg * D * sizeof(float));
-    const bool sole_d = q.chunks == 1 && Mg == M;       // a gradient shared by the heads collects from all of them
-    const int d4n = D >> 2;
-    for (int i0 = first; i0 < R * d4n; i0 += step) {
-      int i = i0;
-      asm volatile("" : "+v"(i));                 // not to be worked out ahead of the loop and kept in registers
-      const int r = i / d4n, d = (i - r * d4n) << 2;
-      float4 val = *reinterpret_cast<float4 *>(gd + r * D + d);
-      const bool nz = val.x != 0 || val.y != 0 || val.z != 0 || val.w != 0;
-      if (nz) *reinterpret_cast<float4 *>(gd + r * D + d) = make_float4(0, 0, 0, 0);
-      const int ry = r / TW, rx = r - ry * TW;
-      const int y = q.y0 + ry, x = q.x0 + rx;
-      if (in_map(y, x, q.H, q.W) && !DFA3D_DIAG(diag, 4)) {
-        const uint32_t e = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D + d);
-        const bool store = sole_d && ry >= 1 && ry < TY && rx >= 1 && rx < TX;
-        if (store || nz) put4(gdist_b, gdist_r, gd16, e, val, store, false);
-      }
-    }
-  };
-  // Work items follow one another without a pause.  An item of n passes takes n + 1 turns of two phases (X, Y: one
-  // barrier after each); what is left of it when its last turn ends is dealt with beside the first turns of the item
-  // after it: its accumulators (handed over in LDS in its last phase Y) go out in phase X of turn 0, the late taps of
-  // its last pass come in that same phase, and its depth tile goes out in phase X of turn 1, before the new item's
-  // first finish touches the tile.  When the queues are drained one more item of zero passes does the same for the
-  // last real one.
-  //   X(t)  walkers: t = 0: value rows of the item, accumulators of the item before; else walk pass t - 1
-  //         pointers: late taps of the pass finished last; prepare pass t; t = 1: depth tile of the item before
-  //   Y(t)  walkers: stage pass t, or (t = n) hand over the accumulators
-  //         pointers: place pass t; finish pass t - 1; ask for the records of the next pass
-  // The two roles run the same sequence of items, turns and barriers, each in a loop of its own: what a role keeps in
-  // registers from turn to turn then never competes with the other role's registers.
+  // Both roles run the same sequence of turns and barriers, each in a loop of its own: what a role keeps in registers
+  // from turn to turn then never competes with the other role's registers.
+  //   pass t: points [base, base + PP) of item `it` (g, valid); pass t - 1: item it1 (valid1, last1: its item's last
+  //   pass); last2, it2: the same of pass t - 2
   if (walker) {
     // =========================== walkers ===========================
-    float v[4][VEC], acc[4][VEC];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) { v[k][i] = 0; acc[k][i] = 0; }
-    }
-    const uint32_t chan_off = (uint32_t)(cl * VEC * sizeof(T));
+    // What a lane owns, worked out anew in every block that needs it (from a copy of the lane number that the compiler
+    // does not see through): kept from turn to turn it would cost the registers that the value rows and sums need.
+    struct Owner {
+      int lane, cl, group, crow, ccol;                       // lane of the wavefront, of its group; the group's cell
+      LaneChannels<T, VEC, LPR> ch;
+      __device__ __forceinline__ Owner(unsigned lane, int wave, int C)
+          : lane(lane), cl(lane % LPR), group(lane / LPR), crow(wave * ROWS + lane / LPR / TX), ccol(lane / LPR % TX), ch(lane % LPR, C) {}
+      // x of the lane `back` lanes before this one
+      __device__ __forceinline__ float from_before(float x, int back) const {
+        return __int_as_float(__builtin_amdgcn_ds_bpermute((lane - back) << 2, __float_as_int(x)));
+      }
+    };
+    auto owner = [&]() {
+      unsigned l = lane;
+      asm volatile("" : "+v"(l));
+      return Owner(l, wave, C);
+    };
     auto decode = [&](const int4 &item, const int4 &geo) {
       ItemGeom g;
       g.bin = item.x; g.seg = item.y; g.n_item = item.z; g.chunks = item.w;
@@ -265,375 +438,533 @@ const ItemGeom q = uniform(s_geom[which]);
     };
     if (tid == 0) {
       CellFetch fetch;
-      int4 rec, geo;
-      fetch.start(ws, p, blockIdx.x % kClasses);
-      fetch.advance(ws, p, blockIdx.x % kClasses, &rec, &geo);
-      s_geom[0] = decode(rec, geo);
+      int4 rec[kDealt - 1], geo[kDealt - 1];
+      fetch.start(ws, p, rec, geo);
+      for (int k = 0; k < kDealt - 1; ++k) s_geom[k] = decode(rec[k], geo[k]);
       s_fetch = fetch;
     }
     __syncthreads();                                        // the first item's record is there
-    for (int it = 0;; ++it) {
-      const ItemGeom g = uniform(s_geom[it % 3]);
-      const bool have_prev = it > 0, done = g.bin < 0;
-      if (done && !have_prev) break;
-      const int n_pass = done ? 0 : (g.n_item + PP - 1) / PP;
-      CT_MARK(0);
-      // The record of the item after this one, first of all: here the walkers hold nothing in registers (the
-      // accumulators were handed over, the value rows are about to be replaced), and nobody reads the slot before
-      // this item's last phase Y.
-      if (tid == 0 && !done) {
-        CellFetch fetch = s_fetch;
-        int4 rec, geo;
-        fetch.advance(ws, p, blockIdx.x % kClasses, &rec, &geo);
-        s_geom[(it + 1) % 3] = decode(rec, geo);
-        s_fetch = fetch;
+
+    auto put_lds = [&](const Owner &o, float *row, const float (&val)[VEC]) {
+#pragma unroll
+      for (int gi = 0; gi < VEC / 4; ++gi)
+        *reinterpret_cast<float4 *>(row + o.ch.first[gi]) = make_float4(val[4 * gi], val[4 * gi + 1], val[4 * gi + 2], val[4 * gi + 3]);
+    };
+    // The sums of tile pixel (crow, ccol) of item q are complete in u.  Pixels 1..TY-1 x 1..7 belong to no neighbour's
+    // halo: when the item held all the points of its bin they are stored (grad_value is zero on entry, or the binning
+    // launches cleared what is added to), else added.  Rim pixels go to their place in LDS, to be added by put_rim.
+    auto put_pixel = [&](const Owner &o, const ItemGeom &q, const float (&u)[VEC], bool active) {
+      const int y = q.y0 + o.crow, x = q.x0 + o.ccol;
+      if (active && (o.crow == 0 || o.ccol == 0)) put_lds(o, rim + rim_index(o.crow, o.ccol, TY) * ROW, u);
+      if (active && o.crow > 0 && o.ccol > 0 && y < q.H && x < q.W && !DFA3D_DIAG(diag, 4)) {
+        char *gvalue_b = static_cast<char *>(grad_value) + (size_t)q.b * S * M * C * (gv16 ? 2 : 4);
+        float *gvalue_f = reinterpret_cast<float *>(gvalue_b);
+        const rsrc_t gvalue_r = make_rsrc(gvalue_b, (size_t)S * M * C * sizeof(float));
+        const uint32_t e = (uint32_t)(((q.start + y * q.W + x) * M + q.m) * C);
+#pragma unroll
+        for (int gi = 0; gi < VEC / 4; ++gi) {
+          const uint32_t at = e + o.ch.first[gi];
+          const float4 f = make_float4(u[4 * gi], u[4 * gi + 1], u[4 * gi + 2], u[4 * gi + 3]);
+          if (o.ch.first[gi] < C) {
+            if (q.chunks == 1) {                            // uniform
+              if (gv16) *reinterpret_cast<uint2 *>(gvalue_b + (size_t)at * 2) = make_uint2(pack_bf16x2(f.x, f.y), pack_bf16x2(f.z, f.w));
+              else *reinterpret_cast<float4 *>(gvalue_f + at) = f;
+            } else if (gv16) {
+              atomic_add_bf16x2(gvalue_b + (size_t)at * 2, f.x, f.y);
+              atomic_add_bf16x2(gvalue_b + (size_t)at * 2 + 4, f.z, f.w);
+            } else {
+              scatter_add(gvalue_r, gvalue_f, at * 4, f.x); scatter_add(gvalue_r, gvalue_f, at * 4 + 4, f.y);
+              scatter_add(gvalue_r, gvalue_f, at * 4 + 8, f.z); scatter_add(gvalue_r, gvalue_f, at * 4 + 12, f.w);
+            }
+          }
+        }
       }
-      const rsrc_t value_r = make_rsrc(value + (size_t)g.b * S * M * C, (size_t)S * M * C * sizeof(T));
+    };
+    // Rim pixels [first, first + n) of item q, whose sums this wavefront left in LDS.
+    auto put_rim = [&](const ItemGeom &q, int first, int n) {
+      char *gvalue_b = static_cast<char *>(grad_value) + (size_t)q.b * S * M * C * (gv16 ? 2 : 4);
+      float *gvalue_f = reinterpret_cast<float *>(gvalue_b);
+      const rsrc_t gvalue_r = make_rsrc(gvalue_b, (size_t)S * M * C * sizeof(float));
+      const int per = gv16 ? ROW / 2 : ROW;                 // lanes per pixel: a float, or a pair of bfloat16
+      for (int i = lane; i < n * per; i += kWave) {
+        const int k = first + i / per, c = (i % per) * (gv16 ? 2 : 1);
+        int ry, rx;
+        rim_decode(k, TY, ry, rx);
+        const int y = q.y0 + ry, x = q.x0 + rx;
+        const float *from = rim + k * ROW + c;
+        const float f0 = from[0], f1 = gv16 ? from[1] : 0.f;
+        if (c < C && in_map(y, x, q.H, q.W) && (f0 != 0 || f1 != 0) && !DFA3D_DIAG(diag, 4)) {
+          const uint32_t e = (uint32_t)(((q.start + y * q.W + x) * M + q.m) * C + c);
+          if (gv16) atomic_add_bf16x2(gvalue_b + (size_t)e * 2, f0, f1);
+          else scatter_add(gvalue_r, gvalue_f, e * 4, f0);
+        }
+      }
+    };
+
+    int turn = 0, it = 0;                                    // of phase X; the item being walked
+    ItemGeom g = uniform(s_geom[0]);
+    constexpr int kRows = PP / 4, IN_FLIGHT = kRows / GPW < 4 ? kRows / GPW : 4;   // rows per walker wavefront; loads asked for at once
+
+    // Always true, which the compiler cannot know: keeps the walk in a block of its own.  Scheduled together with what
+    // surrounds it, it spills registers, and every reload waits for all of the wavefront's memory accesses.
+    auto apart = []() {
+      int yes = 1;
+      asm volatile("" : "+s"(yes));
+      return yes != 0;
+    };
+    // phase X: the counters of the pass sorted in the phase Y before this turn's
+    auto clear_counts = [&]() {
+      unsigned i = tid;
+      asm volatile("" : "+v"(i));
+      if (i < (unsigned)CELLS) cnt[(turn + 2) % 3 * CELLS + i] = 0;
+    };
+    // phase Y: the grad_out rows of the pass, where they cannot go straight from memory to LDS (then the pointers see to it)
+    auto stage = [&]() {
+      if (C == ROW) return;                                  // uniform
+      const Owner o = owner();
       const rsrc_t go_r = make_rsrc(grad_out + (size_t)g.b * Q * M * C, (size_t)Q * M * C * sizeof(T));
-      for (int turn = 0; turn <= n_pass; ++turn) {          // uniform over the workgroup
-        // ---------------- phase X ----------------
-        for (int i = tid; i < n_bit_words; i += PP) bitmap[i] = 0;                 // last used in the phase Y before
-        if (turn >= 1 && tid < kCellMax) cnt[((turn - 1) & 1) * kCellMax + tid] = 0;   // the sort of pass turn - 1 is over
-        if (turn == 0) {
-          // the four value rows of this group's cell (zero outside the map, or when the cell is not part of the
-          // tile), asked for first: they arrive while the accumulators of the item before go out
-          {
-            const int cy = cell / TX, cx = cell - cy * TX;
+      const uint32_t *offs_of = goff + (turn & 1) * PP + wave * kRows;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const int y = g.y0 + cy + (k >= 2 ? 1 : 0), x = g.x0 + cx + ((k == 1 || k == 2) ? 1 : 0);
-              const bool ok = !done && cell < n_cells && in_map(y, x, g.H, g.W) && !DFA3D_DIAG(diag, 8);
-              RowVec<T, float, VEC>::ld(value_r, (ok ? (uint32_t)(((g.start + y * g.W + x) * M + g.m) * C * (int)sizeof(T)) : kNoRow) + chan_off, v[k]);
+      for (int j0 = 0; j0 < kRows / GPW; j0 += IN_FLIGHT) {
+        typename LaneChannels<T, VEC, LPR>::Raw gg[IN_FLIGHT];
+#pragma unroll
+        for (int j = 0; j < IN_FLIGHT; ++j) o.ch.load(go_r, offs_of[(j0 + j) * GPW + o.group], gg[j]);
+#pragma unroll
+        for (int j = 0; j < IN_FLIGHT; ++j) o.ch.put(gstage + (wave * kRows + (j0 + j) * GPW + o.group) * ROW, gg[j]);
+      }
+    };
+    // phase X: walk the lists of the staged pass, one point per step and group; the next step's row and weights and the
+    // slot after that are asked for while this step's sums are formed, so that no LDS round trip is waited for with
+    // nothing to do.  A group whose list has ended goes on with the row of zeros and weight zero (the matrix
+    // instructions ignore the execution mask).
+    auto walk = [&](const float (&v)[4][VEC], f4 (&acc)[VEC]) {
+      const Owner o = owner();
+      const int corner = o.cl & 3, cell = o.crow * TX + o.ccol;
+      const bool cell_ok = o.crow < TY;
+      const int beg = cell_ok ? offs[cell] : 0, n = cell_ok ? offs[cell + 1] - beg : 0;
+      int s0 = s_slot[n > 0 ? beg : PP], s1 = s_slot[n > 1 ? beg + 1 : PP];
+      typedef typename LaneChannels<T, VEC, LPR>::Raw Raw;
+      Raw r0;
+      o.ch.get(gstage + s0 * ROW, r0);
+      float w0 = dots[s0 * 4 + corner];
+      for (int t = 0; __any(t < n); ++t) {
+        const int s2 = s_slot[t + 2 < n ? beg + t + 2 : PP];
+        Raw r1;
+        o.ch.get(gstage + s1 * ROW, r1);
+        const float w1 = dots[s1 * 4 + corner];
+        float d[4], g0[VEC];
+        LaneChannels<T, VEC, LPR>::to_float(r0, g0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          d[k] = v[k][0] * g0[0];
+#pragma unroll
+          for (int i = 1; i < VEC; ++i) d[k] += v[k][i] * g0[i];
+        }
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) acc[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(w0, g0[i], acc[i], 0, 0, 0);
+        float dot = quad_corner_sum(d[0], d[1], d[2], d[3], (o.cl & 1) != 0, (o.cl & 2) != 0);      // lane c: corner c
+        if (LPR == 8) dot += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(dot), 0x104, 0xF, 0xF, true));   // row_shl:4
+        if (t < n && o.cl < 4) dots[s0 * 4 + corner] = dot;
+        s0 = s1; s1 = s2; w0 = w1; r0 = r1;
+      }
+    };
+
+    if (g.bin >= 0) {
+      CT_MARK(0);
+      lds_barrier();                                         // X(0): nothing to walk yet
+      bool have_prev = false;
+      f4 acc[VEC];                                           // acc[channel][corner] of the item before, then of this one
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) acc[i] = (f4){0, 0, 0, 0};
+      for (;;) {                                             // items: from the phase Y of one's first pass to the next one's
+        const bool done = g.bin < 0;
+        const int r0 = wave * ROWS;                          // this wavefront's first tile row
+        float u[VEC];                                        // sums of this group's pixel, on their way out
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) u[i] = 0;
+        CT_MARK(0);
+        // The record of the item three on, first of all: what thread 0 waits for was asked for an item ago.
+        if (tid == 0 && !done) {
+          CellFetch fetch = s_fetch;
+          int4 rec, geo;
+          fetch.advance(ws, p, &rec, &geo);
+          s_geom[slot_of_item(it + 3)] = decode(rec, geo);
+          s_fetch = fetch;
+        }
+        if (have_prev) {
+          // The item before is over.  Tile pixel (r, c) collects corner 0 of cell (r, c), corner 1 of (r, c - 1), corner 2
+          // of (r - 1, c - 1) and corner 3 of (r - 1, c): the cell to the left is the lane group to the left, the row
+          // above the lower half of this wavefront, or the wavefront before it.
+          const Owner o = owner();
+          float dn[VEC], ux[VEC], dx[VEC];                   // for the row below; the same of the ninth pixel (last cell)
+#pragma unroll
+          for (int i = 0; i < VEC; ++i) {
+            const float l1 = o.from_before(acc[i][1], LPR), l2 = o.from_before(acc[i][2], LPR);
+            u[i] = acc[i][0] + (o.ccol > 0 ? l1 : 0.f);
+            dn[i] = acc[i][3] + (o.ccol > 0 ? l2 : 0.f);
+            ux[i] = acc[i][1];
+            dx[i] = acc[i][2];
+            if (ROWS == 2) {
+              const float up = o.from_before(dn[i], kWave / 2), upx = o.from_before(dx[i], kWave / 2);
+              if (o.group >= TX) { u[i] += up; ux[i] += upx; }
             }
           }
-          if (have_prev) {
-            // Pixel (ry, rx) of the tile collects corner 0 of cell (ry, rx), corner 1 of (ry, rx - 1), corner 2 of
-            // (ry - 1, rx - 1) and corner 3 of (ry - 1, rx), four floats per lane.  Pixels 1..TY-1 x 1..TX-1 belong to
-            // no neighbour's halo; when the item held all the points of its bin nobody else adds to them, so they are
-            // stored instead of added atomically (grad_value is zero on entry, or the binning launches cleared what is
-            // added to).
-            const ItemGeom q = uniform(s_geom[(it + 2) % 3]);
-            char *gvalue_b = static_cast<char *>(grad_value) + (size_t)q.b * S * M * C * (gv16 ? 2 : 4);
-            const rsrc_t gvalue_r = make_rsrc(gvalue_b, (size_t)S * M * C * sizeof(float));
-            constexpr int c4n = C >> 2;
-            for (int i0 = tid; i0 < R * c4n; i0 += PP) {
-              int i = i0;
-              asm volatile("" : "+v"(i));             // not to be worked out ahead of the loop and kept in registers
-              const int r = i / c4n, c = (i - r * c4n) << 2;
-              const int ry = r / TW, rx = r - ry * TW;
-              float4 val = make_float4(0, 0, 0, 0);
-#pragma unroll
-              for (int k = 0; k < 4; ++k) {
-                const int cy = ry - (k >= 2 ? 1 : 0), cx = rx - ((k == 1 || k == 2) ? 1 : 0);
-                if (cy >= 0 && cy < TY && cx >= 0 && cx < TX) {
-                  const float4 t = *reinterpret_cast<const float4 *>(gstage + ((cy * TX + cx) * 4 + k) * C + c);
-                  val.x += t.x; val.y += t.y; val.z += t.z; val.w += t.w;
-                }
-              }
-              const bool nz = val.x != 0 || val.y != 0 || val.z != 0 || val.w != 0;
-              const int y = q.y0 + ry, x = q.x0 + rx;
-              if (in_map(y, x, q.H, q.W) && !DFA3D_DIAG(diag, 4)) {
-                const uint32_t e = (uint32_t)(((q.start + y * q.W + x) * M + q.m) * C + c);
-                const bool store = q.chunks == 1 && ry >= 1 && ry < TY && rx >= 1 && rx < TX;
-                if (store || nz) put4(gvalue_b, gvalue_r, gv16, e, val, store, true);
-              }
+          if (o.crow < TY) {
+            if (o.ccol == TX - 1) put_lds(o, rim + rim_index(o.crow, TX, TY) * ROW, ux);
+            if (o.crow + 1 == TY) {
+              put_lds(o, rim + rim_index(TY, o.ccol, TY) * ROW, dn);
+              if (o.ccol == TX - 1) put_lds(o, rim + rim_index(TY, TX, TY) * ROW, dx);
+            } else if (o.group >= (ROWS - 1) * TX) {         // for the wavefront below
+              put_lds(o, cross + (wave * TW + o.ccol) * ROW, dn);
+              if (o.ccol == TX - 1) put_lds(o, cross + (wave * TW + TX) * ROW, dx);
             }
           }
+          if (ROWS == 2) put_pixel(o, uniform(s_geom[slot_of_item(it - 1)]), u, o.crow < TY && o.group >= TX);   // the second row is complete
+        }
+        CT_MARK(3);
+        typename LaneChannels<T, VEC, LPR>::Raw vr[4];
+        {
+          // the four value rows of this group's cell (zero outside the map, when the cell is not part of the tile, or when
+          // there is no item)
+          const Owner o = owner();
+          const rsrc_t value_r = make_rsrc(value + (size_t)g.b * S * M * C, (size_t)S * M * C * sizeof(T));
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) acc[k][i] = 0;
+            const int y = g.y0 + o.crow + (k >= 2 ? 1 : 0), x = g.x0 + o.ccol + ((k == 1 || k == 2) ? 1 : 0);
+            const bool ok = !done && o.crow < TY && in_map(y, x, g.H, g.W) && !DFA3D_DIAG(diag, 8);
+            o.ch.load(value_r, ok ? (uint32_t)(((g.start + y * g.W + x) * M + g.m) * C * (int)sizeof(T)) : kNoRow, vr[k]);
           }
-        } else if (!DFA3D_DIAG(diag, 16)) {
-          // walk the lists of pass turn - 1
-          const int beg = cell < n_cells ? offs[cell] : 0, end = cell < n_cells ? offs[cell + 1] : 0;
-          if (beg < end) {                                  // lanes leave the loop as their cell's list ends
-            // One point per step; the next step's grad_out row is asked for while this step's sums are formed, so
-            // that no LDS round trip is waited for with nothing to do.
-            const float *g_lane = gstage + cl * VEC;
-            int s_cur = s_slot[beg];
-            float g_cur[VEC];
-            lds_ld<VEC>(g_lane + s_cur * kGPitch, g_cur);
-            for (int t = beg; t < end; ++t) {
-              const int s_nxt = s_slot[t + 1 < end ? t + 1 : t];
-              const float4 w_cur = s_w[t];
-              float d[4];
+        }
+        if (!done) {
+          stage();
+        }
+        CT_MARK(6);
+        lds_barrier();
+        CT_MARK(4);
+        // ---------------- phase X of the first pass ----------------
+        ++turn;
+        clear_counts();
+        if (have_prev && r0 < TY) {                          // uniform
+          // The first tile row of this wavefront collects what the wavefront before it left for it; then the rim goes out.
+          const ItemGeom q = uniform(s_geom[slot_of_item(it - 1)]);
+          const Owner o = owner();
+          const bool mine = o.crow < TY && o.group < TX;
+          if (wave > 0 && mine) {
+            const float *from = cross + ((wave - 1) * TW + o.ccol) * ROW;
 #pragma unroll
-              for (int k = 0; k < 4; ++k) {
-                d[k] = 0;
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) d[k] += v[k][i] * g_cur[i];
+            for (int gi = 0; gi < VEC / 4; ++gi) {
+              const float4 a = *reinterpret_cast<const float4 *>(from + o.ch.first[gi]);
+              u[4 * gi] += a.x; u[4 * gi + 1] += a.y; u[4 * gi + 2] += a.z; u[4 * gi + 3] += a.w;
+              if (o.ccol == TX - 1) {
+                float4 *at = reinterpret_cast<float4 *>(rim + rim_index(o.crow, TX, TY) * ROW + o.ch.first[gi]);
+                const float4 b = *reinterpret_cast<const float4 *>(from + ROW + o.ch.first[gi]), c = *at;
+                *at = make_float4(c.x + b.x, c.y + b.y, c.z + b.z, c.w + b.w);
               }
-              float g_nxt[VEC];
-              lds_ld<VEC>(g_lane + s_nxt * kGPitch, g_nxt);
-              const float wk[4] = {w_cur.x, w_cur.y, w_cur.z, w_cur.w};
-#pragma unroll
-              for (int k = 0; k < 4; ++k) {
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) acc[k][i] += wk[k] * g_cur[i];
-              }
-              dots[s_cur * 4 + cl] = quad_corner_sum(d[0], d[1], d[2], d[3], (cl & 1) != 0, (cl & 2) != 0);   // lane c reports corner c
-              s_cur = s_nxt;
-#pragma unroll
-              for (int i = 0; i < VEC; ++i) g_cur[i] = g_nxt[i];
             }
           }
+          put_pixel(o, q, u, mine);
+          wave_lds_handover();
+          const int ra = max(r0, 1), n_side = min(r0 + ROWS, TY) - ra;
+          if (wave == 0) put_rim(q, 0, TW);
+          if (n_side > 0) put_rim(q, rim_index(ra, 0, TY), 2 * n_side);
+          if (r0 + ROWS >= TY) put_rim(q, TW, TW);
         }
-        if (turn == 1) {
-          // the depth tile of the item before: complete since the late taps of turn 0, not touched again before this
-          // item's first finish in phase Y of this turn
-          if (FUSED && have_prev) flush_gd((it + 2) % 3, tid, kCellBlock);
-        }
+        if (done) break;
+        float v[4][VEC];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) LaneChannels<T, VEC, LPR>::to_float(vr[k], v[k]);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) acc[i] = (f4){0, 0, 0, 0};
+        CT_MARK(5);
+        if (apart() && !DFA3D_DIAG(diag, 16)) walk(v, acc);
         CT_MARK(1);
         lds_barrier();
         CT_MARK(2);
-        // ---------------- phase Y ----------------
-        if (turn < n_pass) {
-          // stage the grad_out rows of pass turn
-          constexpr int RPI = kWave / LPR, kRows = PP / 4;      // rows per load instruction, rows per walker wavefront
-#pragma unroll
-          for (int j = 0; j < kRows; j += RPI) {
-            const int slot = wave * kRows + j + lane / LPR;
-            float gg[VEC];
-            if (DFA3D_DIAG(diag, 256)) { for (int i = 0; i < VEC; ++i) gg[i] = 1.f; } else   // cost of the grad_out loads
-            RowVec<T, float, VEC>::ld(go_r, goff[slot] + chan_off, gg);
-            LdsVec<VEC>::st(gstage + slot * kGPitch + cl * VEC, gg);
-          }
-        } else if (done) {
-          if (FUSED && have_prev) flush_gd((it + 2) % 3, tid, PP);   // the last item's depth tile: nothing follows
-        } else {
-          // the item's last walk is over: the cells' accumulators go where the staged rows were
-          if (cell < n_cells) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) LdsVec<VEC>::st(gstage + (cell * 4 + k) * C + cl * VEC, acc[k]);
-          }
+        for (int base = PP; base < g.n_item; base += PP) {   // the item's further passes
+          stage();
+          CT_MARK(6);
+          lds_barrier();
+          CT_MARK(4);
+          ++turn;
+          clear_counts();
+          if (apart() && !DFA3D_DIAG(diag, 16)) walk(v, acc);
+          CT_MARK(1);
+          lds_barrier();
+          CT_MARK(2);
         }
-        CT_MARK(3);
-        lds_barrier();
-        CT_MARK(4);
+        have_prev = true;
+        ++it;
+        g = uniform(s_geom[slot_of_item(it)]);
       }
-      if (done) break;
     }
   } else {
     // =========================== pointers ===========================
-    PointState cur, nxt;
-    LateTaps late;
-    uint32_t pre_gp = 0;                                    // index and record of the point this thread prepares next
-    float4 pre_rec = make_float4(0, 0, 0, 0);
-    cur.bits = 0; nxt.bits = 0; late.pack = 0; late.hd = late.ld = 0;
+    // What a point needs from memory is asked for ahead of time: its record two turns, its depth taps one phase before
+    // they are used.  Loads and stores that are always issued (inactive lanes with offsets beyond the buffer) let the
+    // waits be counted: a wait for a load does not have to include the stores issued after it.
+    const int pslot = tid - kWalkers;                        // the point slot of this thread
+    PointState cur, nxt;                                     // of pass t - 1 and of pass t
+    TapsInFlight<T> taps;                                    // of the pass prepared last
+    u32x4 given = {0, 0, 0, 0};                              // (stage 2 alone) its given scores
+    int rank = 0;                                            // place of its point among the points of its cell
+    cur.bits = 0; nxt.bits = 0;
     cur.gp = nxt.gp = 0; cur.a = nxt.a = 0; cur.lh = cur.lw = cur.ld = nxt.lh = nxt.lw = nxt.ld = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) { cur.sc[k] = cur.hl[k] = nxt.sc[k] = nxt.hl[k] = 0; late.gs[k] = 0; }
-    __syncthreads();                                        // the first item's record is there
-    {
-      const ItemGeom g0 = uniform(s_geom[0]);
-      if (g0.bin >= 0 && pslot < g0.n_item) {
-        pre_gp = ws.entries[g0.seg + pslot];
-        pre_rec = ws.recs[g0.seg + pslot];
+    for (int k = 0; k < 4; ++k) { cur.sc[k] = cur.hl[k] = nxt.sc[k] = nxt.hl[k] = 0; taps.t[k] = (u32x2){0, 0}; }
+    const uint32_t slice = (uint32_t)Q * (uint32_t)M * (uint32_t)(L * P);             // points of a batch element
+    __syncthreads();                                        // the first items' records are there
+
+    ItemGeom g = uniform(s_geom[0]);                         // pass A (the one prepared last): points [base, base + PP) of item `it`
+    int it = 0, base = 0;
+    int rec_it = 0, rec_base = 0, rec_bin = g.bin, rec_seg = g.seg, rec_n = g.n_item;      // the pass whose records were asked for last
+    uint32_t pre_gp = 0;
+    float4 pre_rec = make_float4(0, 0, 0, 0);
+    auto ask_records = [&]() {
+      const int at = rec_bin >= 0 ? rec_seg + rec_base + min(pslot, rec_n - rec_base - 1) : 0;
+      pre_gp = ws.entries[at];
+      pre_rec = ws.recs[at];
+    };
+    auto next_records = [&]() {
+      if (rec_bin >= 0) {
+        rec_base += PP;
+        if (rec_base >= rec_n) {
+          ++rec_it;
+          rec_base = 0;
+          const ItemGeom &q = s_geom[slot_of_item(rec_it)];
+          rec_bin = __builtin_amdgcn_readfirstlane(q.bin); rec_seg = __builtin_amdgcn_readfirstlane(q.seg);
+          rec_n = __builtin_amdgcn_readfirstlane(q.n_item);
+        }
       }
-    }
-    for (int it = 0;; ++it) {
-      const ItemGeom g = uniform(s_geom[it % 3]);
-      const bool have_prev = it > 0, done = g.bin < 0;
-      if (done && !have_prev) break;
-      const int n_pass = done ? 0 : (g.n_item + PP - 1) / PP;
+    };
+    // geometry of this thread's point of pass A, its place in the sort, its grad_out row for the walkers; its taps are asked for
+    auto prepare = [&](int pass) {
+      const bool live = g.bin >= 0 && pslot < g.n_item - base;
+      const uint32_t gp = live ? pre_gp : 0u;
+      const float4 rec = pre_rec;
+      const uint32_t unit = div_lp.div(gp);
+      goff[(pass & 1) * PP + pslot] = live ? (unit - (uint32_t)g.b * (uint32_t)Q * (uint32_t)M) * (uint32_t)(C * (int)sizeof(T)) : kNoRow;
+      const Point2D<float> pg = locate_2d<float>(rec.x, rec.y, g.H, g.W, g.start);
+      const bool in = live && pg.inside;
+      DepthTap<float> tap;
+      tap.inside = tap.lo_ok = tap.hi_ok = false; tap.d0 = 0; tap.ld = tap.hd = 0;
+      unsigned on_bits = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) on_bits |= (in && pg.key[k] >= 0) ? 1u << k : 0u;
+      if (FUSED) {
+        tap = locate_depth<float>(rec.z, g.Dd);
+        const int md = Md == 1 ? 0 : g.m, db = min(max(tap.d0, 0), max(D - 2, 0));
+        const rsrc_t dist_r = make_rsrc(dist + (size_t)g.b * S * Md * D, (size_t)S * Md * D * sizeof(T));
+        uint32_t off[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          off[k] = ((on_bits >> k & 1) && tap.inside && !DFA3D_DIAG(diag, 32)) ? (uint32_t)(((pg.key[k] * Md + md) * D + db) * (int)sizeof(T)) : kNoRow;
+        taps.ask(dist_r, off, D);
+      } else if (score_in != nullptr) {                      // uniform
+        const T *si = score_in + (size_t)gp * 4;
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) given[k] = __float_as_uint(si[k]);
+        } else {
+          const uint16_t *sh = reinterpret_cast<const uint16_t *>(si);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) given[k] = (uint32_t)sh[k] << 16;
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) given[k] = __float_as_uint(1.f);
+      }
+      // the cell: the base pixel within the tile (the binning put the point into this tile by it)
+      const int cy = min(max(pg.h0 - g.y0, 0), TY - 1), cx = min(max(pg.w0 - g.x0, 0), TX - 1), cell = cy * TX + cx;
+      if (in) rank = atomicAdd(cnt + pass % 3 * CELLS + cell, 1);
+      nxt.gp = gp; nxt.a = rec.w; nxt.lh = pg.lh; nxt.lw = pg.lw; nxt.ld = tap.ld;
+      nxt.bits = on_bits | (tap.inside ? 16u : 0u) | (tap.lo_ok ? 32u : 0u) | (tap.hi_ok ? 64u : 0u) | (in ? 128u : 0u) |
+                 ((unsigned)(in ? cell : 0) << 8) | ((unsigned)(tap.d0 + 1) << 16);
+    };
+    ask_records();
+    prepare(0);
+    next_records();
+    ask_records();
+
+    int it1 = 0, it2 = 0;
+    bool valid1 = false, last1 = false, last2 = false;
+    for (int turn = 0;; ++turn) {                            // uniform over the workgroup
+      const bool valid = g.bin >= 0, last = valid && base + PP >= g.n_item;
+      const int it_now = it, b_now = g.b;
       CT_MARK(0);
-      const int md = Md == 1 ? 0 : g.m;
-      const rsrc_t dist_r = make_rsrc(FUSED ? dist + (size_t)g.b * S * Md * D : nullptr, FUSED ? (size_t)S * Md * D * sizeof(T) : 0);
-      const rsrc_t go_r = make_rsrc(grad_out + (size_t)g.b * Q * M * C, (size_t)Q * M * C * sizeof(T));
-      for (int turn = 0; turn <= n_pass; ++turn) {          // uniform over the workgroup
-        // ---------------- phase X: late taps of the pass finished last, then prepare pass turn ----------------
-        if (FUSED && (late.pack & 0xFFu)) {
-          const int lcell = (late.pack >> 8) & 63, lcy = lcell / TX, lcx = lcell - lcy * TX, ld0 = (int)(late.pack >> 16) - 1;
+      // ---------------- phase X: scores and corner weights of pass t, prepare pass t + 1 ----------------
+      float4 pw = make_float4(0, 0, 0, 0);                  // corner weights of this thread's point
+      if (valid) {
+        const float hh = 1 - nxt.lh, hw = 1 - nxt.lw;
+        const int d0 = (int)(nxt.bits >> 16) - 1, db = min(max(d0, 0), max(D - 2, 0));
+        const bool lo_ok = (nxt.bits & 32u) != 0, hi_ok = (nxt.bits & 64u) != 0;
+        const float hd = (nxt.bits & 16u) != 0 ? 1 - nxt.ld : 0.f;
+        float wk[4];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            if (late.pack >> j & 1) {
-              const int k = j >> 1, row = (lcy + (k >= 2 ? 1 : 0)) * TW + lcx + ((k == 1 || k == 2) ? 1 : 0);
-              atomicAdd(gd + row * D + ld0 + (j & 1), ((j & 1) ? late.ld : late.hd) * late.gs[k]);
-            }
+        for (int k = 0; k < 4; ++k) {
+          if (FUSED) {
+            float x, y;
+            taps.get(k, db, D, x, y);
+            const float lo = (lo_ok && d0 == db) ? x : (lo_ok && d0 == db + 1) ? y : 0.f;
+            const float hi = (hi_ok && d0 + 1 == db) ? x : (hi_ok && d0 == db) ? y : 0.f;
+            nxt.sc[k] = depth_lerp(lo, hi, hd, nxt.ld);
+            nxt.hl[k] = hi - lo;
+          } else {
+            nxt.sc[k] = __uint_as_float(given[k]);
           }
-          late.pack = 0;
+          const float bk = k == 0 ? hh * hw : k == 1 ? hh * nxt.lw : k == 2 ? nxt.lh * nxt.lw : nxt.lh * hw;
+          wk[k] = (nxt.bits >> k & 1) ? bk * nxt.sc[k] * nxt.a : 0.f;
         }
-        CT_MARK(1);
-        float4 pw = make_float4(0, 0, 0, 0);               // corner weights of this thread's point
-        int my_cell = -1, my_rank = 0;
-        if (turn < n_pass) {
-          const int base = turn * PP;
-          const bool live = pslot < g.n_item - base;
-          Point2D<float> pg;
-          DepthTap<float> tap;
-          size_t gp = 0;
-          float a = 0, wk[4] = {0, 0, 0, 0};
-          unsigned on_bits = 0;
+        pw = make_float4(wk[0], wk[1], wk[2], wk[3]);
+      }
+      const PointState now = nxt;                            // of pass t
+      const int rank_now = rank;
+      base += PP;
+      if (last) { ++it; base = 0; g = uniform(s_geom[slot_of_item(it)]); }
+      nxt.bits = 0;
+      if (g.bin >= 0) prepare(turn + 1);
+      next_records();
+      ask_records();
+      CT_MARK(1);
+      if (FUSED && last2) flush_gd(slot_of_item(it2), pslot, PP);
+      if (!valid && !valid1) break;
+      CT_MARK(2);
+      lds_barrier();
+      CT_MARK(3);
+      // ---------------- phase Y: place pass t, finish pass t - 1 ----------------
+      const bool straight = valid && C == ROW;               // uniform
+      if (straight) {
+        // The grad_out rows of pass t: whole rows go straight into LDS, 16 bytes per lane, without a register in between,
+        // and arrive while this phase's other work is done.
+        constexpr int RL = ROW * (int)sizeof(T) / 16, RPI = kWave / RL;        // lanes per row, rows per instruction
+        const rsrc_t go_r = make_rsrc(grad_out + (size_t)b_now * Q * M * C, (size_t)Q * M * C * sizeof(T));
+        const int row0 = (wave - kWalkers / kWave) * kWave;
+        unsigned l = lane;
+        asm volatile("" : "+v"(l));                          // (not worth registers from turn to turn)
+        uint32_t row[kWave / RPI];
 #pragma unroll
-          for (int k = 0; k < 4; ++k) { nxt.sc[k] = 0; nxt.hl[k] = 0; pg.key[k] = -1; }
-          pg.inside = false; pg.lh = pg.lw = pg.hh = pg.hw = 0; pg.h0 = pg.w0 = 0;
-          tap.inside = tap.lo_ok = tap.hi_ok = false; tap.d0 = 0; tap.ld = tap.hd = 0;
-          uint32_t my_goff = kNoRow, touch = 0;
-          if (live) {
-            gp = pre_gp;                                     // asked for one phase ago
-            const float4 rec = pre_rec;
-            const size_t unit = gp / LP;
-            a = rec.w;
-            my_goff = (uint32_t)((unit - (size_t)g.b * Q * M) * C * sizeof(T));
-            // ask for the point's grad_out row now, so that the walkers' staging loads of the next phase find it in the L2
-            touch = __builtin_amdgcn_raw_buffer_load_b32(go_r, my_goff, 0, 0);
-            pg = locate_2d<float>(rec.x, rec.y, g.H, g.W, g.start);
-            if (FUSED) {
-              tap = locate_depth<float>(rec.z, g.Dd);
-              if (DFA3D_DIAG(diag, 32)) { for (int k = 0; k < 4; ++k) { nxt.sc[k] = 0.5f; nxt.hl[k] = 0.1f; } } else   // cost of the depth taps
-              {
-                float lo[4], hi[4];
-                corner_scores<T, float, true>(dist_r, pg.key, tap, md, Md, D, nxt.sc, lo, hi);
+        for (int j = 0; j < kWave / RPI; ++j) row[j] = goff[(turn & 1) * PP + row0 + j * RPI + l / RL];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) nxt.hl[k] = hi[k] - lo[k];
-              }
-            } else {
-              const T *si = score_in + gp * 4;
+        for (int j = 0; j < kWave / RPI; ++j) load_to_lds16(go_r, gstage + (row0 + j * RPI) * ROW, row[j] + 16 * (l % RL));
+      }
+      const float4 d4 = *reinterpret_cast<const float4 *>(dots + pslot * 4);       // of pass t - 1, before its place is taken
+      if (valid) {
+        // exclusive prefix of the cell counters; every pointer wavefront computes it and writes the same numbers,
+        // so it can go on with its own copy without waiting for the others
+        const int c = lane < CELLS ? cnt[turn % 3 * CELLS + lane] : 0;
+        const int inc = wave_inclusive_scan(c);
+        if (lane < CELLS) offs[lane] = inc - c;
+        if (lane == kWave - 1) offs[CELLS] = inc;
+        *reinterpret_cast<float4 *>(dots + pslot * 4) = pw;
+        if (now.bits & 128u) s_slot[offs[(now.bits >> 8) & 63] + rank_now] = (uint16_t)pslot;
+      }
+      CT_MARK(4);
+      if (valid1 && !DFA3D_DIAG(diag, 512)) {                // (development builds: cost of phase C)
+        const ItemGeom &q = s_geom[slot_of_item(it1)];
+        const int gH = __builtin_amdgcn_readfirstlane(q.H), gW = __builtin_amdgcn_readfirstlane(q.W), gDd = __builtin_amdgcn_readfirstlane(q.Dd);
+        const int gb = __builtin_amdgcn_readfirstlane(q.b);
+        const bool live = (cur.bits & 128u) != 0;
+        Point2D<float> pg;
+        DepthTap<float> tap;
+        pg.lh = cur.lh; pg.lw = cur.lw; pg.hh = 1 - cur.lh; pg.hw = 1 - cur.lw;
+        tap.inside = (cur.bits & 16u) != 0; tap.lo_ok = (cur.bits & 32u) != 0; tap.hi_ok = (cur.bits & 64u) != 0;
+        tap.d0 = (int)(cur.bits >> 16) - 1; tap.ld = cur.ld; tap.hd = tap.inside ? 1 - cur.ld : 0.f;
+        const unsigned on_bits = cur.bits & 15u;
+        const int ccell = (cur.bits >> 8) & 63, ccy = ccell / TX, ccx = ccell % TX;
+        const float a = cur.a;
+        const float dc[4] = {d4.x, d4.y, d4.z, d4.w};
+        float gs[4], sk[4], ga = 0;
 #pragma unroll
-              for (int k = 0; k < 4; ++k) nxt.sc[k] = score_in != nullptr ? Elem<T>::ld(si + k) : 1.f;
-            }
+        for (int k = 0; k < 4; ++k) {
+          const bool on = on_bits >> k & 1;
+          const float bk = pg.bil(k);
+          gs[k] = on ? bk * a * dc[k] : 0.f;
+          sk[k] = on ? cur.sc[k] * dc[k] : 0.f;
+          ga += bk * sk[k];
+        }
+        const float gx = (float)gW * a * (pg.hh * (sk[1] - sk[0]) + pg.lh * (sk[2] - sk[3]));
+        const float gy = (float)gH * a * (pg.hw * (sk[3] - sk[0]) + pg.lw * (sk[2] - sk[1]));
+        // where the point's gradients go, relative to its batch element
+        const uint32_t at = live ? cur.gp - (uint32_t)gb * slice : 0u;
+        const rsrc_t gl_r = make_rsrc(grad_loc + (size_t)gb * slice * gl_stride, (size_t)slice * gl_stride * 4);
+        const rsrc_t ga_r = make_rsrc(grad_attn + (size_t)gb * slice, (size_t)slice * 4);
+        const uint32_t gl_off = live ? at * (uint32_t)(gl_stride * 4) : kNoRow, ga_off = live ? at * 4 : kNoRow;
+        if (FUSED) {
+          if (grad_score_in != nullptr) {
+            const T *gi = grad_score_in + (size_t)cur.gp * 4;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              if (pg.key[k] >= 0) {
-                on_bits |= 1u << k;
-                wk[k] = pg.bil(k) * nxt.sc[k] * a;
-              }
-            }
-            if (pg.inside) {
-              // the cell: the base pixel within the tile (the binning put the point into this tile by it)
-              const int cy = min(max(pg.h0 - g.y0, 0), TY - 1), cx = min(max(pg.w0 - g.x0, 0), TX - 1);
-              my_cell = cy * TX + cx;
-              my_rank = atomicAdd(cnt + (turn & 1) * kCellMax + my_cell, 1);
-            }
+            for (int k = 0; k < 4; ++k) gs[k] += Elem<T>::ld(gi + k);
           }
-          if (touch == 0x7FC12345u) my_goff = kNoRow;      // never (a NaN payload no gradient carries): keeps the load alive
-          goff[pslot] = my_goff;
-          pw = make_float4(wk[0], wk[1], wk[2], wk[3]);
-          nxt.gp = (uint32_t)gp; nxt.a = a; nxt.lh = pg.lh; nxt.lw = pg.lw; nxt.ld = tap.ld;
-          nxt.bits = on_bits | (tap.inside ? 16u : 0u) | (tap.lo_ok ? 32u : 0u) | (tap.hi_ok ? 64u : 0u) |
-                     ((live && my_cell >= 0) ? 128u : 0u) | ((unsigned)max(my_cell, 0) << 8) | ((unsigned)(tap.d0 + 1) << 16);
-        }
-        if (FUSED && have_prev && turn == 1) flush_gd((it + 2) % 3, tid, kCellBlock);     // the walkers take the other half
-        CT_MARK(2);
-        lds_barrier();
-        CT_MARK(3);
-        // ---------------- phase Y: place pass turn, finish pass turn - 1 ----------------
-        if (turn < n_pass) {
-          // exclusive prefix of the cell counters; every pointer wavefront computes it and writes the same numbers,
-          // so it can go on with its own copy without waiting for the others
-          const int c = cnt[(turn & 1) * kCellMax + lane];
-          const int inc = wave_inclusive_scan(c);
-          offs[lane] = inc - c;
-          if (lane == kWave - 1) offs[kCellMax] = inc;
-          if (my_cell >= 0) {
-            const int pos = offs[my_cell] + my_rank;
-            s_slot[pos] = (uint16_t)pslot;
-            s_w[pos] = pw;
+          if (grad_wu != nullptr) {       // weight_update = sum over points of attn * mean corner score
+            const float gw = grad_wu[div_lp.div(cur.gp)] * 0.25f;
+            ga += gw * (cur.sc[0] + cur.sc[1] + cur.sc[2] + cur.sc[3]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) gs[k] += gw * a;
           }
-        }
-        CT_MARK(4);
-        if (turn >= 1 && (cur.bits & 128u) && !DFA3D_DIAG(diag, 512)) {       // (development builds: cost of phase C)
-          Point2D<float> pg;
-          DepthTap<float> tap;
-          pg.lh = cur.lh; pg.lw = cur.lw; pg.hh = 1 - cur.lh; pg.hw = 1 - cur.lw;
-          tap.inside = (cur.bits & 16u) != 0; tap.lo_ok = (cur.bits & 32u) != 0; tap.hi_ok = (cur.bits & 64u) != 0;
-          tap.d0 = (int)(cur.bits >> 16) - 1; tap.ld = cur.ld; tap.hd = tap.inside ? 1 - cur.ld : 0.f;
-          const unsigned on_bits = cur.bits & 15u;
-          const int ccell = (cur.bits >> 8) & 63, ccy = ccell / TX, ccx = ccell - ccy * TX;
-          const float a = cur.a;
-          const size_t gp = cur.gp;
-          const float4 d4 = *reinterpret_cast<const float4 *>(dots + pslot * 4);
-          const float dc[4] = {d4.x, d4.y, d4.z, d4.w};
-          float gs[4], sk[4], ga = 0;
+          float gz = 0;
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            const bool on = on_bits >> k & 1;
-            const float bk = pg.bil(k);
-            gs[k] = on ? bk * a * dc[k] : 0.f;
-            sk[k] = on ? cur.sc[k] * dc[k] : 0.f;
-            ga += bk * sk[k];
+            if (!tap.inside) gs[k] = 0.f;              // (a corner outside the map has none already)
+            gz += gs[k] * cur.hl[k];
           }
-          const float gx = (float)g.W * a * (pg.hh * (sk[1] - sk[0]) + pg.lh * (sk[2] - sk[3]));
-          const float gy = (float)g.H * a * (pg.hw * (sk[3] - sk[0]) + pg.lw * (sk[2] - sk[1]));
-          float *gl = grad_loc + gp * gl_stride;
-          if (!FUSED) { gl[0] = gx; gl[1] = gy; }
-          if (FUSED) {
-            if (grad_score_in != nullptr) {
-              const T *gi = grad_score_in + gp * 4;
-#pragma unroll
-              for (int k = 0; k < 4; ++k) gs[k] += Elem<T>::ld(gi + k);
-            }
-            if (grad_wu != nullptr) {       // weight_update = sum over points of attn * mean corner score
-              const float gw = grad_wu[gp / LP] * 0.25f;
-              ga += gw * (cur.sc[0] + cur.sc[1] + cur.sc[2] + cur.sc[3]);
-#pragma unroll
-              for (int k = 0; k < 4; ++k) gs[k] += gw * a;
-            }
-            float gz = 0;
-            unsigned want = 0;                          // bit j: tap j exists
-            int at4[4];                                 // tile address of each corner's lower tap
+          const u32x3 g3 = {__float_as_uint(gx), __float_as_uint(gy), __float_as_uint(gz * (float)gDd)};
+          __builtin_amdgcn_raw_buffer_store_b96(g3, gl_r, gl_off, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ga), ga_r, ga_off, 0, 0);
+          // The taps: read, add, compare-and-swap, all eight in flight together; a tap that met another one tries again
+          // with what it found, and after a few rounds (many points on one pixel and depth) the float atomic ends it.  A tap
+          // that does not exist adds zero to a word nearby: the four pixels always lie in the tile, the bins are clamped.
+          if (live && !DFA3D_DIAG(diag, 2)) {
+            uint32_t *gdw = reinterpret_cast<uint32_t *>(gd);
+            const int row0 = (ccy * TW + ccx) * D, lo_at = max(tap.d0, 0), hi_at = min(tap.d0 + 1, D - 1);
+            const float w_lo = tap.lo_ok ? tap.hd : 0.f, w_hi = tap.hi_ok ? tap.ld : 0.f;
+            int at[8];
+            float tv[8];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-              const bool corner_in = (on_bits >> k & 1) && tap.inside;     // a corner inside the map lies inside the tile
-              if (!corner_in) gs[k] = 0.f;
-              const bool taps = corner_in && gs[k] != 0 && !DFA3D_DIAG(diag, 2);
-              at4[k] = ((ccy + (k >= 2 ? 1 : 0)) * TW + ccx + ((k == 1 || k == 2) ? 1 : 0)) * D + tap.d0;
-              if (taps && tap.lo_ok) want |= 1u << (2 * k);
-              if (taps && tap.hi_ok) want |= 2u << (2 * k);
-              gz += gs[k] * cur.hl[k];
-              late.gs[k] = gs[k];
+              const int row = row0 + (k == 0 ? 0 : k == 1 ? D : k == 2 ? (TW + 1) * D : TW * D);
+              at[2 * k] = row + lo_at; at[2 * k + 1] = row + hi_at;
+              tv[2 * k] = tap.lo_ok ? w_lo * gs[k] : 0.f; tv[2 * k + 1] = tap.hi_ok ? w_hi * gs[k] : 0.f;
             }
-            late.hd = tap.hd; late.ld = tap.ld;
-            gl[0] = gx; gl[1] = gy; gl[2] = gz * (float)g.Dd;      // one 12-byte store
-            grad_attn[gp] = ga;                       // all stores before the tile updates: they complete slowly
-            // Who is first at a tile address in this pass: the bit of the address in the bitmap, set with an integer
-            // atomic.  The first adds at once with a plain read-modify-write (nobody else touches the address before
-            // the next barrier); the others add atomically in the next phase.
-            unsigned first = 0;
+            uint32_t old[8], got[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              if (want >> j & 1) {
-                const int at = at4[j >> 1] + (j & 1);
-                const uint32_t bit = 1u << (at & 31);
-                if (DFA3D_DIAG(diag, 1024) || (atomicOr(&bitmap[at >> 5], bit) & bit)) {} else first |= 1u << j;
+            for (int j = 0; j < 8; ++j) old[j] = gdw[at[j]];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) got[j] = atomicCAS(gdw + at[j], old[j], __float_as_uint(__uint_as_float(old[j]) + tv[j]));
+            unsigned again = 0;                         // bit j: tap j is still to be added
+#pragma unroll
+            for (int j = 0; j < 8; ++j) again |= got[j] != old[j] ? 1u << j : 0u;
+            for (int round = 0; again != 0 && round < 4; ++round) {
+#pragma unroll
+              for (int j = 0; j < 8; ++j) {
+                old[j] = got[j];
+                if (again >> j & 1) got[j] = atomicCAS(gdw + at[j], old[j], __float_as_uint(__uint_as_float(old[j]) + tv[j]));
               }
-            }
-            float cur8[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) cur8[j] = (first >> j & 1) ? gd[at4[j >> 1] + (j & 1)] : 0.f;
+              for (int j = 0; j < 8; ++j) again &= got[j] == old[j] ? ~(1u << j) : ~0u;
+            }
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-              if (first >> j & 1) gd[at4[j >> 1] + (j & 1)] = cur8[j] + ((j & 1) ? tap.ld : tap.hd) * gs[j >> 1];
-            late.pack = (want & ~first) | (cur.bits & 0xFFFF3F00u);
-          } else if (grad_score_out != nullptr) {
-            float *go4 = grad_score_out + gp * 4;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) go4[k] = gs[k];
-            grad_attn[gp] = ga;
-          } else {
-            grad_attn[gp] = ga;
+              if (again >> j & 1) atomicAdd(gd + at[j], tv[j]);
+          }
+        } else {
+          const u32x2 g2 = {__float_as_uint(gx), __float_as_uint(gy)};
+          __builtin_amdgcn_raw_buffer_store_b64(g2, gl_r, gl_off, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ga), ga_r, ga_off, 0, 0);
+          if (grad_score_out != nullptr) {                   // uniform
+            const rsrc_t gs_r = make_rsrc(grad_score_out + (size_t)gb * slice * 4, (size_t)slice * 16);
+            const u32x4 g4 = {__float_as_uint(gs[0]), __float_as_uint(gs[1]), __float_as_uint(gs[2]), __float_as_uint(gs[3])};
+            __builtin_amdgcn_raw_buffer_store_b128(g4, gs_r, live ? at * 16 : kNoRow, 0, 0);
           }
         }
-        // the records of the next pass's points (of this item, or of the first pass of the item after it, whose record
-        // was written in phase X of turn 1): they arrive while the workgroup waits at the barrier
-        if (!done) {
-          const bool last = turn >= n_pass;
-          const ItemGeom ng = uniform(s_geom[(it + 1) % 3]);
-          const int next_seg = last ? ng.seg : g.seg, next_base = last ? 0 : (turn + 1) * PP;
-          const int next_n = last ? (ng.bin >= 0 ? ng.n_item : 0) : g.n_item;
-          if ((!last || turn >= 1) && pslot < next_n - next_base) {
-            pre_gp = ws.entries[next_seg + next_base + pslot];
-            pre_rec = ws.recs[next_seg + next_base + pslot];
-          }
-        }
-        cur = nxt;
-        nxt.bits = 0;
-        CT_MARK(5);
-        lds_barrier();
-        CT_MARK(6);
       }
-      if (done) break;
+      // The staged rows must have come (the barrier orders LDS accesses only), the two stores after them need not have.
+      if (straight) {
+        if (valid1 && !DFA3D_DIAG(diag, 512)) wait_for_all_but_two(); else wait_for_loads();
+      }
+      cur = now;
+      CT_MARK(5);
+      lds_barrier();
+      CT_MARK(6);
+      it2 = it1; last2 = last1; it1 = it_now; valid1 = valid; last1 = last;
     }
   }
   CT_FLUSH();
@@ -642,45 +973,61 @@ const ItemGeom q = uniform(s_geom[which]);
 // ---------------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------------
-// The kernel takes rows of 32 channels on tiles of at most 64 pixels whose rows and depth rows are whole
-// 16-byte groups; everything else stays with the row-owned tile kernel.
-bool cell_kernel_applies(int C, int D, int ty, int tx, bool fused) {
-  return C == kCellC && ty * tx <= kCellMax && ty >= 1 && tx >= 1 && (!fused || (D & 3) == 0);
-}
+// The kernel takes rows of up to 64 channels, whole groups of four, on tiles 8 pixels wide of at most as many rows as
+// its walkers own.  The row-owned tile kernel keeps the rest.
+bool cell_kernel_applies(int C, int ty, int tx) { return C <= 64 && (C & 3) == 0 && tx == kCellTX && ty >= 1 && ty <= cell_max_ty(C); }
 
-template <typename T>
-static hipError_t launch_cell_typed(const BwdArgs &a, const BinWorkspace &ws, size_t lds, int grid, float *gd_heads,
-                                    hipStream_t stream) {
+template <typename T, int VEC, int LPR>
+static hipError_t launch_cell_cfg(const BwdArgs &a, const BinWorkspace &ws, size_t lds, int grid, float *gd_heads,
+                                  hipStream_t stream) {
+  const FastDiv div_lp((uint32_t)(a.L * a.P));
   if (a.dist != nullptr) {
-    hipLaunchKernelGGL((cell_backward_kernel<T, true>), dim3(grid), dim3(kCellBlock), lds, stream, ws, (const T *)a.value,
+    hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, true>), dim3(grid), dim3(kWalkers + cell_pass(LPR)), lds, stream, ws, (const T *)a.value,
                        (const T *)a.dist, (const T *)nullptr, (const T *)a.grad_out, (const T *)a.grad_score_in,
                        a.grad_value, gd_heads != nullptr ? (void *)gd_heads : a.grad_dist, (float *)a.grad_loc,
                        a.grad_loc_stride, (float *)a.grad_attn, (float *)nullptr, (const float *)a.grad_weight_update,
                        a.dist_heads == 1 ? 1 : a.M, (a.dist_heads == 1 && gd_heads == nullptr) ? 1 : a.M, a.B, a.S, a.M,
-                       a.D, a.L, a.Q, a.P, (a.grad_bf16 ? 1 : 0) | ((a.grad_bf16 && gd_heads == nullptr) ? 2 : 0)
+                       a.C, a.D, a.L, a.Q, a.P, div_lp, (a.grad_bf16 ? 1 : 0) | ((a.grad_bf16 && gd_heads == nullptr) ? 2 : 0)
                        DFA3D_DIAG_ARG(a));
   } else {
-    hipLaunchKernelGGL((cell_backward_kernel<T, false>), dim3(grid), dim3(kCellBlock), lds, stream, ws, (const T *)a.value,
+    hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, false>), dim3(grid), dim3(kWalkers + cell_pass(LPR)), lds, stream, ws, (const T *)a.value,
                        (const T *)nullptr, (const T *)a.score_in, (const T *)a.grad_out, (const T *)nullptr,
                        a.grad_value, (void *)nullptr, (float *)a.grad_loc, a.grad_loc_stride, (float *)a.grad_attn,
-                       (float *)a.grad_score_out, (const float *)nullptr, a.M, a.M, a.B, a.S, a.M, 0, a.L, a.Q, a.P, 0
-                       DFA3D_DIAG_ARG(a));
+                       (float *)a.grad_score_out, (const float *)nullptr, a.M, a.M, a.B, a.S, a.M, a.C, 0, a.L, a.Q, a.P,
+                       div_lp, 0 DFA3D_DIAG_ARG(a));
   }
   return hipGetLastError();
 }
 
-const void *cell_kernel_symbol(int dtype, bool fused) {
-  if (dtype == DFA3D_F32)
-    return fused ? reinterpret_cast<const void *>(cell_backward_kernel<float, true>)
-                 : reinterpret_cast<const void *>(cell_backward_kernel<float, false>);
-  return fused ? reinterpret_cast<const void *>(cell_backward_kernel<__hip_bfloat16, true>)
-               : reinterpret_cast<const void *>(cell_backward_kernel<__hip_bfloat16, false>);
+template <typename T, int VEC, int LPR> static const void *symbol_of(bool fused) {
+  return fused ? reinterpret_cast<const void *>(cell_backward_kernel<T, VEC, LPR, true>)
+               : reinterpret_cast<const void *>(cell_backward_kernel<T, VEC, LPR, false>);
+}
+
+#define DFA3D_CELL_DISPATCH(dtype, C, CALL)                                  \
+  do {                                                                       \
+    const CellShape s = cell_shape(C);                                       \
+    if (dtype == DFA3D_F32) {                                                \
+      if (s.lpr == 8) return CALL(float, 8, 8);                              \
+      if (s.vec == 8) return CALL(float, 8, 4);                              \
+      return CALL(float, 4, 4);                                              \
+    }                                                                        \
+    if (s.lpr == 8) return CALL(__hip_bfloat16, 8, 8);                       \
+    if (s.vec == 8) return CALL(__hip_bfloat16, 8, 4);                       \
+    return CALL(__hip_bfloat16, 4, 4);                                       \
+  } while (0)
+
+const void *cell_kernel_symbol(int dtype, int C, bool fused) {
+#define DFA3D_CELL_SYMBOL(T, V, R) (symbol_of<T, V, R>(fused))
+  DFA3D_CELL_DISPATCH(dtype, C, DFA3D_CELL_SYMBOL);
+#undef DFA3D_CELL_SYMBOL
 }
 
 hipError_t launch_cell_kernel(const BwdArgs &a, int dtype, const BinWorkspace &ws, size_t lds, int grid, float *gd_heads,
                               hipStream_t stream) {
-  return dtype == DFA3D_F32 ? launch_cell_typed<float>(a, ws, lds, grid, gd_heads, stream)
-                            : launch_cell_typed<__hip_bfloat16>(a, ws, lds, grid, gd_heads, stream);
+#define DFA3D_CELL_LAUNCH(T, V, R) (launch_cell_cfg<T, V, R>(a, ws, lds, grid, gd_heads, stream))
+  DFA3D_CELL_DISPATCH(dtype, a.C, DFA3D_CELL_LAUNCH);
+#undef DFA3D_CELL_LAUNCH
 }
 
 }  // namespace dfa3d

@@ -22,7 +22,7 @@ struct BinPlan {
   int bins_per_class;  // total_bins / kClasses
   int class_start[kClasses + 1];   // first work item of each head class (written by the scan)
   int ty, tx;          // tile edge in pixels
-  int chunk;           // points of a bin handled by one work item
+  int chunk;           // points of a bin per work item that the caller asked for, 0: chunk_of() decides
   int total_chunks;    // work items (written by the scan)
 };
 
@@ -41,6 +41,17 @@ __device__ __forceinline__ void slot_decode(int slot, int B, int M, int &b, int 
   m = (hm % G) * kClasses + hm / G;
 }
 
+// Division of n < 2^31 by a number the host knows: multiply by ceil(2^(32 + shift) / d) - 2^32, add, shift.
+struct FastDiv {
+  uint32_t mul, shift;
+  explicit FastDiv(uint32_t d) {
+    shift = 0;
+    while ((1ull << shift) < d) ++shift;
+    mul = (uint32_t)((((1ull << shift) - d) << 32) / d + 1);
+  }
+  __device__ __forceinline__ uint32_t div(uint32_t n) const { return (__umulhi(mul, n) + n) >> shift; }
+};
+
 // pixel (y, x) lies inside an H x W map (a tile's first row and column may be pixel -1)
 __device__ __forceinline__ bool in_map(int y, int x, int H, int W) { return (unsigned)y < (unsigned)H && (unsigned)x < (unsigned)W; }
 
@@ -55,7 +66,7 @@ __device__ __forceinline__ void lds_barrier() {
 
 struct BinWorkspace {      // device pointers into the caller's workspace
   BinPlan *plan;
-  int *queues;             // kClasses counters, kQueueStride ints apart
+  int *queues;             // kClasses counters, kQueueStride ints apart; beside each, a part of the number of points counted
   int *counts;             // points per bin
   int *cursor;             // begin of each bin's segment after the scan, end after the fill
   int4 *items;             // work items: (bin, begin of its points, number of points, work items of the bin)
@@ -76,6 +87,23 @@ __device__ __forceinline__ int wave_inclusive_scan(int x) {
   return x;
 }
 
+// Points of a bin per work item.  Small items balance the workgroups, but the items of one bin add to its gradients
+// with atomics, which the memory takes at one 64-byte piece per 50 ps (a split bin of 96 channels and depth bins:
+// 20 ns per item), where a bin of one item stores them.  So: about 4096 items if that leaves large ones, else down to
+// 1024 items, none under 256 points.  0.34 M points in 240 bins: 88 us with 4096 points per item, 44 with these; 0.58 M
+// of plain attention: 230 and 60; 15.4 M: no difference.
+constexpr int kMaxChunk = 4096;
+__device__ __forceinline__ int chunk_of(const BinWorkspace &ws, const BinPlan &p) {
+  if (p.chunk > 0) return p.chunk;
+  int n = 0;
+  for (int c = 0; c < kClasses; ++c) n += ws.queues[c * kQueueStride + 1];
+  return min(max(max(n >> 12, min(n >> 10, 1280)), 256), kMaxChunk);
+}
+// Work items of a bin with c points, of equal shares (most bins have one, which saves the division); item t of k starts
+// at point share_begin(c, k, t) of the bin.
+__device__ __forceinline__ int items_of_bin(int c, int ch) { return c <= ch ? (c > 0 ? 1 : 0) : (c + ch - 1) / ch; }
+__device__ __forceinline__ int share_begin(int c, int k, int t) { const int q = c / k; return t * q + min(t, c - q * k); }
+
 // Optional phase timing of the tile kernel (development builds only, -DDFA3D_TILE_TIMING): thread 0
 // of every workgroup accumulates shader-clock ticks per phase and adds them to 64-bit counters that
 // live in the padding behind the queue counter.
@@ -89,12 +117,16 @@ __device__ __forceinline__ int wave_inclusive_scan(int x) {
 #define TT_FLUSH() do { } while (0)
 #endif
 
+// Workgroups of this launch whose home is class c.
+__device__ __forceinline__ int workgroups_of_class(int c) { return ((int)gridDim.x - c + kClasses - 1) / kClasses; }
+
 // Thread 0 of a tile workgroup: next work item, from the queue of the workgroup's own class first and
-// from the other classes once that is empty; -1 when every queue is drained.
-__device__ __forceinline__ int pop_item(const BinWorkspace &ws, const BinPlan &p, int home, int &classes_done) {
+// from the other classes once that is empty; -1 when every queue is drained.  `dealt`: items per workgroup of the class
+// that are not taken from the queue.
+__device__ __forceinline__ int pop_item(const BinWorkspace &ws, const BinPlan &p, int home, int &classes_done, int dealt = 0) {
   while (classes_done < kClasses) {
     const int c = (home + classes_done) % kClasses;
-    const int lo = p.class_start[c], hi = p.class_start[c + 1];
+    const int lo = p.class_start[c], hi = p.class_start[c + 1] - dealt * workgroups_of_class(c);
     if (lo < hi) {
       // from the end: the bins of the coarsest level, which hold the most points, come last in a (batch, head)
       // and should not be what the kernel's last workgroups are left with
@@ -185,11 +217,15 @@ template <> struct LdsVec<8> {
 };
 template <int VEC> __device__ __forceinline__ void lds_ld(const float *p, float (&v)[VEC]) { LdsVec<VEC>::ld(p, v); }
 
-// The cell-owned tile kernel (dfa3d_backward_cells.hip): rows of 32 channels, tiles of at most 64 pixels.
-bool cell_kernel_applies(int C, int D, int ty, int tx, bool fused);
-size_t cell_kernel_lds_bytes(int ty, int tx, int D);
+// The cell-owned tile kernel (dfa3d_backward_cells.hip): rows of up to 64 channels, tiles 8 pixels wide.
+constexpr int kCellTX = 8;
+int cell_max_ty(int C);                // the most tile rows its walkers own
+bool cell_kernel_applies(int C, int ty, int tx);
+int cell_kernel_pass(int C);           // points per pass
+int cell_kernel_block(int C);          // threads per workgroup
+size_t cell_kernel_lds_bytes(int ty, int C, int D, int elem);
 size_t cell_kernel_half_cu_lds();      // the most dynamic LDS with which two of its workgroups fit a CU
-const void *cell_kernel_symbol(int dtype, bool fused);
+const void *cell_kernel_symbol(int dtype, int C, bool fused);
 hipError_t launch_cell_kernel(const BwdArgs &a, int dtype, const BinWorkspace &ws, size_t lds, int grid, float *gd_heads,
                               hipStream_t stream);
 

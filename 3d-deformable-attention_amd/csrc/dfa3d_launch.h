@@ -80,7 +80,7 @@ struct BwdArgs {
 #endif
   int tile_hint;                     // binned path: tile edge as ty * 100 + tx (0 = automatic)
   int block_hint;                    // binned path: threads per tile workgroup (0 = 512)
-  int chunk_hint;                    // binned path: points of a bin per work item (0 = 4096)
+  int chunk_hint;                    // binned path: points of a bin per work item (0: by the number of points)
   int pass_hint;                     // binned path: points per pass, 64, 128 or 256 (0 = automatic)
   void *event_binned;                // hipEvent_t recorded between the binning kernels and the tile kernel, or nullptr
 };

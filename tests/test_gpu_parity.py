@@ -512,6 +512,29 @@ def _gpu_two_stage(inp, dev, sliced):
     return out.detach().cpu(), score.detach().cpu(), gv.cpu(), gd.cpu(), gl.cpu(), ga.cpu()
 
 
+@pytest.mark.parametrize("C,D,levels", [(4, 1, ((9, 8), (3, 2))), (16, 59, ((33, 17), (8, 7))), (20, 41, ((24, 41), (7, 9))),
+                                        (24, 64, ((16, 16),)), (32, 112, ((23, 40), (12, 20))), (32, 128, ((30, 9),)),
+                                        (40, 33, ((15, 25), (1, 1))), (64, 16, ((40, 31), (20, 16)))],
+                         ids=lambda v: str(v) if isinstance(v, int) else "")
+def test_cell_kernel_row_lengths_bins_and_tile_edges(oracle, C, D, levels):
+    """Enough points for the tile kernels, on every lane grouping of the cell-owned kernel: rows shorter than their lane
+    group, bins that are no multiple of four, tiles of fewer pixel rows (many bins), maps of one tile and of one pixel,
+    several work items per tile; one stage, and stage two alone."""
+    dev = _dev()
+    t = tiny_case(seed=C + D, B=2, M=4, C=C, D=D, Q=2600, P=4, levels=levels, dtype=torch.float32)
+    inp = _as_inputs(t)
+    want = _oracle_one_stage(oracle, inp)
+    from dfa3D import _lib
+    for chunk in (0, 256):
+        with _lib.launch_options(chunk=chunk):
+            got = _gpu_one_stage(inp, dev)
+            two = _gpu_two_stage(inp, dev, sliced=False)
+        for g in (got, two):
+            for i in (0, 1, 4, 5):
+                torch.testing.assert_close(g[i], want[i], **(F32_FWD if i < 2 else F32_BWD))
+            _assert_sums_within_term_count_bound(oracle, inp, g[2], g[3])
+
+
 @pytest.mark.parametrize("binned", [1, 0], ids=["tiles", "atomics"])
 @pytest.mark.parametrize("sliced", [True, False], ids=["sliced", "wide"])
 def test_fp32_two_stage_workloads_match_checker(oracle, binned, sliced):
