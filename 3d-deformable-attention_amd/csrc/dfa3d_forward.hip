@@ -12,37 +12,57 @@
 
 namespace dfa3d {
 
-// Phase B of the forward pass: acc += sum over tasks [t_begin, t_end) of w * row, the wavefront
-// covering 64/LPR rows per step with LPR lanes of VEC channels per row.  `chan_off` is the lane's
-// byte offset inside a row (kNoChan for a lane beyond the last channel).
-template <typename T, typename A, int VEC, int LPR>
-__device__ __forceinline__ void gather_rows(rsrc_t value_r, const Task<A> *tasks, int t_begin, int t_end, int row_slot,
+// How the wavefronts share the units: `upw` units of L * P points each, a power of two so that the row slots of phase B
+// can be dealt to them evenly; `chunks` rounds of 64 points where one unit has more.
+struct FwdShape { int LP, upw, chunks; };
+__host__ __device__ inline FwdShape fwd_shape(int L, int P, int upw) {
+  return FwdShape{L * P, upw, upw > 1 ? 1 : (L * P + kWave - 1) / kWave};
+}
+constexpr int kMaxUnitsPerWave = 16;
+constexpr int kTaskPad = 2;            // tasks left free after each unit's, so that the units start on different LDS banks
+
+// Phase B of the forward pass: acc += sum of w * row over the tasks first, first + step, ... below n of one unit.  LPR lanes
+// of VEC channels take a row; the wavefront's 64/LPR row slots may work on the same unit (step > 1) or on units of
+// their own.  Eight rows per lane are in flight, whatever the length of the list: a unit of 8 points has 32 tasks, and
+// walking it one row at a time waited for memory once per row.  A batch is summed in two chains and added to acc as a
+// whole, which keeps the longest chain of additions of a unit at about what a tree over the row slots has.
+// `chan_off` is the lane's byte offset inside a row (kNoChan for a lane beyond the last channel).
+template <typename T, typename A, int VEC>
+__device__ __forceinline__ void gather_rows(rsrc_t value_r, const Task<A> *tasks, int first, int step, int n,
                                             uint32_t chan_off, A (&acc)[VEC]) {
-  constexpr int RPI = kWave / LPR;
-  constexpr int U = 8;
-  int t0 = t_begin;
-  for (; t0 + RPI * U <= t_end; t0 += RPI * U) {
+  constexpr int U = 8, UT = 4;
+  int t = 0;                                             // uniform
+  for (; t + step * U <= n; t += step * U) {
     Task<A> e[U];
 #pragma unroll
-    for (int j = 0; j < U; ++j) e[j] = tasks[t0 + j * RPI + row_slot];
+    for (int j = 0; j < U; ++j) e[j] = tasks[t + j * step + first];
     A v[U][VEC];
 #pragma unroll
     for (int j = 0; j < U; ++j) RowVec<T, A, VEC>::ld(value_r, e[j].off + chan_off, v[j]);
 #pragma unroll
-    for (int j = 0; j < U; ++j) {
+    for (int i = 0; i < VEC; ++i) {
+      A s0 = e[0].w * v[0][i], s1 = e[1].w * v[1][i];
+#pragma unroll
+      for (int j = 2; j < U; j += 2) { s0 += e[j].w * v[j][i]; s1 += e[j + 1].w * v[j + 1][i]; }
+      acc[i] += s0 + s1;
+    }
+  }
+  for (; t < n; t += step * UT) {
+    Task<A> e[UT];
+#pragma unroll
+    for (int j = 0; j < UT; ++j) {
+      const int at = t + j * step + first;
+      e[j] = tasks[min(at, n - 1)];
+      if (at >= n) { e[j].off = kNoRow; e[j].w = 0; }
+    }
+    A v[UT][VEC];
+#pragma unroll
+    for (int j = 0; j < UT; ++j) RowVec<T, A, VEC>::ld(value_r, e[j].off + chan_off, v[j]);
+#pragma unroll
+    for (int j = 0; j < UT; ++j) {
 #pragma unroll
       for (int i = 0; i < VEC; ++i) acc[i] += e[j].w * v[j][i];
     }
-  }
-  for (; t0 < t_end; t0 += RPI) {
-    const int t = t0 + row_slot;
-    const Task<A> e = tasks[min(t, kWave * 4 - 1)];
-    const bool in = t < t_end;
-    A v[VEC];
-    RowVec<T, A, VEC>::ld(value_r, (in ? e.off : kNoRow) + chan_off, v);
-    const A w = in ? e.w : (A)0;
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) acc[i] += w * v[i];
   }
 }
 
@@ -50,6 +70,14 @@ __device__ __forceinline__ void gather_rows(rsrc_t value_r, const Task<A> *tasks
 // Fused / stage-2 forward.
 // grid: M * B * ceil(Q / queries_per_block) blocks; block id % M = head, so that with the
 // round-robin placement of workgroups on the 8 XCDs each XCD's L2 serves one head (M = 8).
+//
+// Bound by the rate at which a CU's front end turns gathered lines around, and by the L2 misses of the finest level, once
+// enough rows are in flight.  In phase B the row slots are dealt to the wavefront's units (8 units of 8 points: one slot
+// each), so that lists of any length keep eight rows per lane in flight and a unit's sum crosses lanes only where
+// it has several slots.  Before, the whole wavefront walked one unit after the other, and short units one row at a time:
+//   6 x 10000 queries, 4 levels from 116 x 200, points around the query   664 -> 617 us
+//   6 x 4000 queries, one level of 8 points (training step)               261 -> 239 us
+//   2 x 40000 queries, plain attention, 4 points (training step)          461 -> 427 us
 // ---------------------------------------------------------------------------------------
 template <typename T, typename A, int VEC, int LPR, bool FUSED>
 __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
@@ -57,10 +85,10 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
     const int64_t *__restrict__ level_start, const A *__restrict__ loc, int loc_stride,
     const A *__restrict__ attn, const T *__restrict__ score_in, T *__restrict__ out, T *__restrict__ score_out,
     A *__restrict__ weight_update, const T *__restrict__ packed_arg, int Md, int B, int S, int M, int C, int D, int L,
-    int Q, int P, int iters, int q_blocks) {
+    int Q, int P, int upw, int iters, int q_blocks) {
   // packed: the head-shared distribution as dfa3d_pack_dist lays it out (D >= 2), or nullptr
   __shared__ LevelTable tab;
-  __shared__ Task<A> s_tasks[kWavesPerBlock][kWave * 4];
+  __shared__ __align__(16) Task<A> s_tasks[kWavesPerBlock][kWave * 4 + kMaxUnitsPerWave * kTaskPad];
 
   load_level_table(tab, shapes, shape_stride, level_start, L, S, FUSED ? D : 0);
   if (FUSED && packed_arg != nullptr) load_cell_starts(tab, L);      // uniform
@@ -69,7 +97,7 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
   // come from dist itself.
   const T *packed = (FUSED && packed_arg != nullptr && tab.cell[L] <= packed_cell_capacity(S, L)) ? packed_arg : nullptr;
 
-  const WaveShape ws = wave_shape(L, P);
+  const FwdShape ws = fwd_shape(L, P, upw);
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int m = blockIdx.x % M;
   const int rest = blockIdx.x / M;
@@ -77,6 +105,10 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
   const int row_slot = lane / LPR, cl = lane % LPR;
   const int passes = (C + VEC * LPR - 1) / (VEC * LPR);
   Task<A> *tasks = s_tasks[wave];
+  // phase B: `par` units at a time, `spu` row slots each
+  constexpr int RPI = kWave / LPR;
+  const int par = min(ws.upw, RPI), spu = RPI / par;
+  const int unit_tasks = ws.LP * 4 + kTaskPad;              // where the next unit's tasks start (upw > 1)
 
   const rsrc_t value_r = make_rsrc(value + (size_t)b * S * M * C, (size_t)S * M * C * sizeof(T));
   const rsrc_t dist_r = make_rsrc(FUSED ? dist + (size_t)b * S * Md * D : nullptr,
@@ -178,43 +210,30 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
           }
         }
         wave_lds_handover();     // previous phase B has consumed the task list
+        if (ws.upw == 1 || ul < ws.upw) {
+          Task<A> *to = tasks + (ws.upw == 1 ? lane * 4 : ul * unit_tasks + lp * 4);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) tasks[lane * 4 + k] = t4[k];
+          for (int k = 0; k < 4; ++k) to[k] = t4[k];
+        }
         wave_lds_handover();
 
         // ---------------- phase B: lanes over channels ----------------
-        if (ws.upw == 1) {
-          const int n_pts = min(kWave, ws.LP - chunk * kWave);
-          gather_rows<T, A, VEC, LPR>(value_r, tasks, 0, n_pts * 4, row_slot, chan_off, acc);
-        } else {
-          // several whole units in this chunk: finish each one here
-          for (int u = 0; u < ws.upw; ++u) {
-            if (q0 + u >= Q) break;
-            A au[VEC];
+        for (int u0 = 0; u0 < ws.upw; u0 += par) {              // (one round where a unit takes several chunks)
+          const int u = u0 + row_slot / spu;
+          const int n = (ws.upw == 1 ? min(kWave, ws.LP - chunk * kWave) : ws.LP) * 4;
+          gather_rows<T, A, VEC>(value_r, tasks + u * (ws.upw == 1 ? 0 : unit_tasks), row_slot % spu, spu, n, chan_off, acc);
+          if (chunk == ws.chunks - 1) {
+            for (int off = LPR; off < spu * LPR; off <<= 1) {
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) au[i] = 0;
-            gather_rows<T, A, VEC, LPR>(value_r, tasks, u * ws.LP * 4, (u + 1) * ws.LP * 4, row_slot, chan_off, au);
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) {
-#pragma unroll
-              for (int off = LPR; off < kWave; off <<= 1) au[i] += __shfl_xor(au[i], off, kWave);
+              for (int i = 0; i < VEC; ++i) acc[i] += __shfl_xor(acc[i], off, kWave);
             }
-            if (row_slot == 0 && chan_ok) {
+            if (row_slot % spu == 0 && chan_ok && q0 + u < Q) {
               const size_t unit = ((size_t)b * Q + (q0 + u)) * M + m;
-              RowVec<T, A, VEC>::st(out + unit * C + chan, au);
+              RowVec<T, A, VEC>::st(out + unit * C + chan, acc);
             }
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) acc[i] = 0;
           }
-        }
-      }
-      if (ws.upw == 1) {
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) {
-#pragma unroll
-          for (int off = LPR; off < kWave; off <<= 1) acc[i] += __shfl_xor(acc[i], off, kWave);
-        }
-        if (row_slot == 0 && chan_ok) {
-          const size_t unit = ((size_t)b * Q + q0) * M + m;
-          RowVec<T, A, VEC>::st(out + unit * C + chan, acc);
         }
       }
     }
@@ -314,7 +333,14 @@ hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int6
 // ---------------------------------------------------------------------------------------
 template <typename T, typename A, int VEC, int LPR>
 static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
-  const WaveShape ws = wave_shape(a.L, a.P);
+  // Units per wavefront: as many as its 64 lanes have points for.  A call with few units is spread over more wavefronts
+  // instead, down to one unit each, while that leaves fewer than kFewWaves of them (four per CU): its time is the
+  // length of one wavefront's chain of loads, which is proportional to the units.
+  constexpr long long kFewWaves = 1024;
+  int upw = 1;
+  while (upw < kMaxUnitsPerWave && 2 * upw * a.L * a.P <= kWave) upw *= 2;
+  while (upw > 1 && (long long)a.M * a.B * ((a.Q + upw - 1) / upw) < kFewWaves) upw /= 2;
+  const FwdShape ws = fwd_shape(a.L, a.P, upw);
   const int q_per_iter = kWavesPerBlock * ws.upw;
   const int iters = a.iters > 0 ? a.iters : 1;
   const int q_blocks = (a.Q + q_per_iter * iters - 1) / (q_per_iter * iters);
@@ -325,12 +351,12 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
                        (const T *)a.value, (const T *)a.dist, a.shapes, a.shape_stride, a.level_start,
                        (const A *)a.loc, a.loc_stride, (const A *)a.attn, (const T *)nullptr, (T *)a.out,
                        (T *)a.score_out, (A *)a.weight_update, (const T *)a.packed_dist, a.dist_heads == 1 ? 1 : a.M, a.B,
-                       a.S, a.M, a.C, a.D, a.L, a.Q, a.P, iters, q_blocks);
+                       a.S, a.M, a.C, a.D, a.L, a.Q, a.P, upw, iters, q_blocks);
   } else {
     hipLaunchKernelGGL((fwd_attention_kernel<T, A, VEC, LPR, false>), dim3((unsigned)blocks), dim3(kBlock), 0, stream,
                        (const T *)a.value, (const T *)nullptr, a.shapes, a.shape_stride, a.level_start,
                        (const A *)a.loc, a.loc_stride, (const A *)a.attn, (const T *)a.score_in, (T *)a.out,
-                       (T *)nullptr, (A *)nullptr, (const T *)nullptr, a.M, a.B, a.S, a.M, a.C, a.D, a.L, a.Q, a.P, iters,
+                       (T *)nullptr, (A *)nullptr, (const T *)nullptr, a.M, a.B, a.S, a.M, a.C, a.D, a.L, a.Q, a.P, upw, iters,
                        q_blocks);
   }
   return hipGetLastError();
@@ -338,10 +364,10 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
 
 template <typename T, typename A>
 static hipError_t launch_fwd_typed(const FwdArgs &a, hipStream_t stream) {
-  const RowTiling rt = pick_row_tiling(a.C, (int)sizeof(T), a.vec_hint);
+  const RowTiling rt = pick_gather_tiling(a.C, (int)sizeof(T), a.vec_hint);
 #define DFA3D_CASE(V, R) \
   if (rt.vec == V && rt.lpr == R) return launch_fwd_cfg<T, A, V, R>(a, stream);
-  DFA3D_ROW_TILINGS(DFA3D_CASE)
+  DFA3D_GATHER_TILINGS(DFA3D_CASE)
 #undef DFA3D_CASE
   return hipErrorInvalidValue;
 }
