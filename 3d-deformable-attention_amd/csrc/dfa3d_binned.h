@@ -24,6 +24,7 @@ struct BinPlan {
   int ty, tx;          // tile edge in pixels
   int chunk;           // points of a bin per work item that the caller asked for, 0: chunk_of() decides
   int total_chunks;    // work items (written by the scan)
+  int disjoint;        // no key belongs to two levels
 };
 
 // Bins are numbered slot * bins_per_bm + tile, where the slot of (batch b, head m) puts the heads with the
@@ -216,6 +217,44 @@ template <> struct LdsVec<8> {
   }
 };
 template <int VEC> __device__ __forceinline__ void lds_ld(const float *p, float (&v)[VEC]) { LdsVec<VEC>::ld(p, v); }
+
+// The eight depth taps of a point added to an LDS tile of floats: read, add, compare-and-swap, all eight in flight
+// together; a tap that met another one tries again with what it found, and after a few rounds (many points on one pixel
+// and depth) the float atomic ends it.  The LDS float atomic alone retires 0.33 lanes per clock and CU, this 2.9.
+__device__ __forceinline__ void lds_add_taps(float *tile, const int (&at)[8], const float (&tv)[8]) {
+  uint32_t *words = reinterpret_cast<uint32_t *>(tile);
+  uint32_t old[8], got[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) old[j] = words[at[j]];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) got[j] = atomicCAS(words + at[j], old[j], __float_as_uint(__uint_as_float(old[j]) + tv[j]));
+  unsigned again = 0;                         // bit j: tap j is still to be added
+#pragma unroll
+  for (int j = 0; j < 8; ++j) again |= got[j] != old[j] ? 1u << j : 0u;
+  for (int round = 0; again != 0 && round < 4; ++round) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      old[j] = got[j];
+      if (again >> j & 1) got[j] = atomicCAS(words + at[j], old[j], __float_as_uint(__uint_as_float(old[j]) + tv[j]));
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) again &= got[j] == old[j] ? ~(1u << j) : ~0u;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    if (again >> j & 1) atomicAdd(tile + at[j], tv[j]);
+}
+
+// The rim of a tile of (ty + 1) x (tx + 1) pixels, numbered: row 0, row ty, then the first and last pixel of the rows between.
+__host__ __device__ inline int rim_pixels(int ty, int tx) { return 2 * (tx + 1) + 2 * (ty - 1); }
+__device__ __forceinline__ int rim_index(int row, int col, int ty, int tx) {
+  return row == 0 ? col : row == ty ? tx + 1 + col : 2 * (tx + 1) + 2 * (row - 1) + (col == 0 ? 0 : 1);
+}
+__device__ __forceinline__ void rim_decode(int i, int ty, int tx, int &row, int &col) {
+  const int s = i - 2 * (tx + 1);
+  row = s >= 0 ? 1 + (s >> 1) : i <= tx ? 0 : ty;
+  col = s >= 0 ? ((s & 1) ? tx : 0) : i <= tx ? i : i - (tx + 1);
+}
 
 // The cell-owned tile kernel (dfa3d_backward_cells.hip): rows of up to 64 channels, tiles 8 pixels wide.
 constexpr int kCellTX = 8;

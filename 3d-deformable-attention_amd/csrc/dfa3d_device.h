@@ -69,6 +69,7 @@ template <> struct Elem<__hip_bfloat16> {
 // ---------------------------------------------------------------------------------------
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x3 __attribute__((ext_vector_type(3)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kNoRow = 0x80000000u;    // offset of a task with nothing to gather
