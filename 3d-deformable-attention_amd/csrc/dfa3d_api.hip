@@ -448,4 +448,28 @@ int dfa3d_rebatch_combine(const void *src, const int32_t *pos, const void *scale
                                                   (hipStream_t)stream), fn);
 }
 
+static int check_linear(const char *fn, long long N, int O, int K) {
+  if (N <= 0 || O <= 0 || K <= 0) return fail(DFA3D_EINVAL, "%s: dimensions must be positive (N=%lld O=%d K=%d)", fn, N, O, K);
+  if ((O & 1) || (K & 1)) return fail(DFA3D_EINVAL, "%s: O and K must be even (O=%d K=%d)", fn, O, K);
+  if (O > 16384 || K > 16384 || N > (1LL << 31))
+    return fail(DFA3D_ERANGE, "%s: at most 2^31 rows of 16384 columns (N=%lld O=%d K=%d)", fn, N, O, K);
+  return 0;
+}
+
+size_t dfa3d_linear_grad_workspace_bytes(long long N, int O, int K) {
+  if (check_linear("dfa3d_linear_grad_workspace_bytes", N, O, K)) return 0;
+  return dfa3d::linear_grad_workspace_bytes(N, O, K);
+}
+
+int dfa3d_linear_grad(const float *x, const float *grad_out, float *grad_weight, float *grad_bias, void *workspace,
+                      size_t workspace_bytes, long long N, int O, int K, void *stream) {
+  const char *fn = "dfa3d_linear_grad";
+  if (int rc = check_linear(fn, N, O, K)) return rc;
+  REQUIRE_PTR(fn, x); REQUIRE_PTR(fn, grad_out); REQUIRE_PTR(fn, grad_weight); REQUIRE_PTR(fn, workspace);
+  if (workspace_bytes < dfa3d::linear_grad_workspace_bytes(N, O, K) || ((uintptr_t)workspace & 15) != 0)
+    return fail(DFA3D_EINVAL, "%s: workspace too small or not on a 16-byte boundary", fn);
+  return hip_result(dfa3d::launch_linear_grad(x, grad_out, grad_weight, grad_bias, (float *)workspace, N, O, K,
+                                              (hipStream_t)stream), fn);
+}
+
 }  // extern "C"

@@ -142,4 +142,9 @@ hipError_t launch_rebatch_gather(const void *src, long long cam_stride, long lon
 hipError_t launch_rebatch_combine(const void *src, const int *pos, const void *scale, void *dst, int bs, int cams,
                                   int max_len, int Nq, int E, int dtype, hipStream_t stream);
 
+// Weight and bias gradients of a linear layer (dfa3d_linear.hip); O and K even.
+size_t linear_grad_workspace_bytes(long long N, int O, int K);
+hipError_t launch_linear_grad(const float *x, const float *g, float *grad_weight, float *grad_bias, float *workspace,
+                              long long N, int O, int K, hipStream_t stream);
+
 }  // namespace dfa3d

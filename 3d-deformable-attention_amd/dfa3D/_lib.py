@@ -42,6 +42,7 @@ SIGNATURES = {
     "dfa3d_fused_backward_static": [_P] * 13 + _DIMS8 + [_I, _I, _O, _P],
     "dfa3d_rebatch_gather": [_P, ctypes.c_longlong, ctypes.c_longlong, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "dfa3d_rebatch_combine": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
+    "dfa3d_linear_grad": [_P] * 5 + [ctypes.c_size_t, ctypes.c_longlong, _I, _I, _P],
     "dfa3d_abi_version": [],
 }
 
@@ -69,6 +70,8 @@ def lib():
             fn.restype = ctypes.c_size_t
         handle.dfa3d_packed_dist_bytes.argtypes = [_I] * 5
         handle.dfa3d_packed_dist_bytes.restype = ctypes.c_size_t
+        handle.dfa3d_linear_grad_workspace_bytes.argtypes = [ctypes.c_longlong, _I, _I]
+        handle.dfa3d_linear_grad_workspace_bytes.restype = ctypes.c_size_t
         handle.dfa3d_static_scratch_bytes.argtypes = []
         handle.dfa3d_static_scratch_bytes.restype = ctypes.c_size_t
         handle.dfa3d_last_error.argtypes = []

@@ -18,6 +18,7 @@ from torch import nn
 
 from ..functional import (MultiScale3DDeformableAttnFunction_fp32,
                           MultiScale3DDeformableAttnWeightUpdateFunction_fp32)
+from .projection import Projection
 
 __all__ = ["MSDeformableAttention3D_DFA3D"]
 
@@ -47,10 +48,10 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         self.num_levels = num_levels
         self.num_heads = num_heads
         self.num_points = num_points
-        self.sampling_offsets = nn.Linear(embed_dims, num_heads * num_levels * num_points * 2)
-        self.attention_weights = nn.Linear(embed_dims, num_heads * num_levels * num_points)
-        self.value_proj = nn.Linear(embed_dims, embed_dims)
-        self.sampling_offsets_depth = nn.Linear(embed_dims, num_heads * num_levels * num_points)
+        self.sampling_offsets = Projection(embed_dims, num_heads * num_levels * num_points * 2)
+        self.attention_weights = Projection(embed_dims, num_heads * num_levels * num_points)
+        self.value_proj = Projection(embed_dims, embed_dims)
+        self.sampling_offsets_depth = Projection(embed_dims, num_heads * num_levels * num_points)
         self.init_weights()
         self.init_smpl_off_weights()
 

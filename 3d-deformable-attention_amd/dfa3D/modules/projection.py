@@ -1,0 +1,74 @@
+"""The linear layers around the operator: ``nn.Linear`` with the weight and bias gradients formed by the library's own
+kernel (csrc/dfa3d_linear.hip) where that applies.  A cross-attention layer projects 10^5 rows (the pixels of six cameras, or
+the queries re-batched per camera) with weights of 256 x 256: the gradient of such a weight is a product with a tiny
+result and a very long inner dimension."""
+import torch
+import torch.nn.functional as F
+from torch import nn
+from torch.autograd import Function
+
+from .. import _lib
+
+__all__ = ["Projection"]
+
+# Fewer rows than this: the library product is as fast and there is one launch less.
+_MIN_ROWS = 4096
+
+
+def _weight_gradients(x, grad, want_bias):
+    """grad_weight (O, K) and grad_bias (O) or None, of contiguous float32 rows x (N, K) and grad (N, O)."""
+    N, K = x.shape
+    O = grad.shape[1]
+    grad_weight = torch.empty(O, K, dtype=torch.float32, device=x.device)
+    grad_bias = torch.empty(O, dtype=torch.float32, device=x.device) if want_bias else None
+    lib = _lib.lib()
+    nbytes = lib.dfa3d_linear_grad_workspace_bytes(N, O, K)
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    with torch.cuda.device(x.device):
+        rc = lib.dfa3d_linear_grad(_lib.ptr(x), _lib.ptr(grad), _lib.ptr(grad_weight), _lib.ptr(grad_bias),
+                                   _lib.ptr(workspace), nbytes, N, O, K, _lib.stream_of(x))
+    _lib.check(rc, "dfa3d_linear_grad")
+    return grad_weight, grad_bias
+
+
+class _ProjectionFunction(Function):
+    """``F.linear(x, weight, bias)`` with a bias; differentiable any number of times (a backward that is itself recorded
+    is made of torch operations)."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias):
+        ctx.save_for_backward(x, weight)
+        return F.linear(x, weight, bias)
+
+    @staticmethod
+    def backward(ctx, grad):
+        x, weight = ctx.saved_tensors
+        want_x, want_weight, want_bias = ctx.needs_input_grad
+        grad_x = grad.matmul(weight) if want_x else None
+        rows, grad_rows = x.reshape(-1, x.shape[-1]), grad.reshape(-1, grad.shape[-1])
+        if torch.is_grad_enabled() or not want_weight or grad.dtype != torch.float32:
+            return grad_x, grad_rows.t().mm(rows) if want_weight else None, grad_rows.sum(0) if want_bias else None
+        return (grad_x, *_weight_gradients(rows.contiguous(), grad_rows.contiguous(), want_bias))
+
+
+def _applies(x, weight, bias):
+    """The plain case: float32 rows on the GPU in ordinary reverse-mode training.  Autocast, functorch transforms,
+    forward-mode derivatives, tracing and compilation see the torch operation itself."""
+    return (bias is not None and x.is_cuda and x.dtype == weight.dtype == bias.dtype == torch.float32
+            and torch.is_grad_enabled() and weight.requires_grad and x.dim() >= 2
+            and weight.shape[0] % 2 == 0 and weight.shape[1] % 2 == 0 and max(weight.shape) <= 16384
+            and _MIN_ROWS <= x.numel() // max(x.shape[-1], 1) <= 2 ** 31
+            and type(x) in (torch.Tensor, nn.Parameter) and type(weight) is nn.Parameter and type(bias) is nn.Parameter
+            and x.device == weight.device == bias.device
+            and not torch.is_autocast_enabled() and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0)
+
+
+class Projection(nn.Linear):
+    """``nn.Linear``: same parameters, same results."""
+
+    def forward(self, input):
+        if _applies(input, self.weight, self.bias):
+            return _ProjectionFunction.apply(input, self.weight, self.bias)
+        return F.linear(input, self.weight, self.bias)

@@ -9,6 +9,7 @@ from torch import nn
 
 from ..rebatch import RebatchCombineFunction, RebatchGatherFunction, camera_index, rebatch_gather
 from .ms_deform_attn_3d import MSDeformableAttention3D_DFA3D
+from .projection import Projection
 
 __all__ = ["SpatialCrossAttention_DFA3D"]
 
@@ -39,7 +40,7 @@ class SpatialCrossAttention_DFA3D(nn.Module):
         self.deformable_attention = deformable_attention
         self.embed_dims = embed_dims
         self.num_cams = num_cams
-        self.output_proj = nn.Linear(embed_dims, embed_dims)
+        self.output_proj = Projection(embed_dims, embed_dims)
         self.batch_first = batch_first
         self.bev_h = bev_h
         self.bev_w = bev_w

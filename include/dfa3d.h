@@ -231,6 +231,14 @@ int dfa3d_rebatch_gather(const void *src, long long cam_stride, long long batch_
 int dfa3d_rebatch_combine(const void *src, const int32_t *pos, const void *scale, void *dst, int bs, int cams,
                           int max_len, int Nq, int E, int dtype, void *stream);
 
+/* Weight and bias gradients of a linear layer y = x weight^T + bias in float32: grad_weight (O, K) = grad_out^T x,
+ * grad_bias (O) = column sums of grad_out, or not formed when it is NULL; x (N, K) and grad_out (N, O) row-major, O and K
+ * even, every element of the results written, no atomics (the same result every time).  `workspace`: 16-byte aligned
+ * device memory of the size the other function gives. */
+size_t dfa3d_linear_grad_workspace_bytes(long long N, int O, int K);
+int dfa3d_linear_grad(const float *x, const float *grad_out, float *grad_weight, float *grad_bias, void *workspace,
+                      size_t workspace_bytes, long long N, int O, int K, void *stream);
+
 /* Message for the last non-zero return on the calling thread ("" if none). */
 const char *dfa3d_last_error(void);
 
