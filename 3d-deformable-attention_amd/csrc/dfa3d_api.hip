@@ -448,6 +448,37 @@ int dfa3d_rebatch_combine(const void *src, const int32_t *pos, const void *scale
                                                   (hipStream_t)stream), fn);
 }
 
+static int check_cameras(const char *fn, int cams, int bs, int Nq, int Z) {
+  if (cams <= 0 || bs <= 0 || Nq <= 0 || Z <= 0)
+    return fail(DFA3D_EINVAL, "%s: dimensions must be positive (cams=%d bs=%d Nq=%d Z=%d)", fn, cams, bs, Nq, Z);
+  if (cams > 65535) return fail(DFA3D_ERANGE, "%s: at most 65535 cameras", fn);
+  if (Nq > (1 << 30)) return fail(DFA3D_ERANGE, "%s: at most 2^30 queries", fn);
+  return 0;
+}
+
+int dfa3d_camera_hits(const uint8_t *mask, uint8_t *hit, float *scale, int cams, int bs, int Nq, int Z, void *stream) {
+  const char *fn = "dfa3d_camera_hits";
+  if (int rc = check_cameras(fn, cams, bs, Nq, Z)) return rc;
+  REQUIRE_PTR(fn, mask); REQUIRE_PTR(fn, hit); REQUIRE_PTR(fn, scale);
+  return hip_result(dfa3d::launch_camera_hits(mask, hit, scale, cams, bs, Nq, Z, (hipStream_t)stream), fn);
+}
+
+int dfa3d_camera_count(const uint8_t *hit, int32_t *totals, int cams, int Nq, void *stream) {
+  const char *fn = "dfa3d_camera_count";
+  if (int rc = check_cameras(fn, cams, 1, Nq, 1)) return rc;
+  REQUIRE_PTR(fn, hit); REQUIRE_PTR(fn, totals);
+  return hip_result(dfa3d::launch_camera_count(hit, totals, cams, Nq, (hipStream_t)stream), fn);
+}
+
+int dfa3d_camera_index(const uint8_t *hit, const int32_t *totals, int32_t *index, int32_t *pos, int cams, int Nq, int max_len,
+                       void *stream) {
+  const char *fn = "dfa3d_camera_index";
+  if (int rc = check_cameras(fn, cams, 1, Nq, 1)) return rc;
+  if (max_len <= 0 || max_len > Nq) return fail(DFA3D_EINVAL, "%s: max_len must be in [1, Nq]", fn);
+  REQUIRE_PTR(fn, hit); REQUIRE_PTR(fn, totals); REQUIRE_PTR(fn, index); REQUIRE_PTR(fn, pos);
+  return hip_result(dfa3d::launch_camera_index(hit, totals, index, pos, cams, Nq, max_len, (hipStream_t)stream), fn);
+}
+
 static int check_linear(const char *fn, long long N, int O, int K) {
   if (N <= 0 || O <= 0 || K <= 0) return fail(DFA3D_EINVAL, "%s: dimensions must be positive (N=%lld O=%d K=%d)", fn, N, O, K);
   if ((O & 1) || (K & 1)) return fail(DFA3D_EINVAL, "%s: O and K must be even (O=%d K=%d)", fn, O, K);

@@ -142,6 +142,11 @@ hipError_t launch_rebatch_gather(const void *src, long long cam_stride, long lon
 hipError_t launch_rebatch_combine(const void *src, const int *pos, const void *scale, void *dst, int bs, int cams,
                                   int max_len, int Nq, int E, int dtype, hipStream_t stream);
 
+hipError_t launch_camera_hits(const uint8_t *mask, uint8_t *hit, float *scale, int cams, int bs, int Nq, int Z, hipStream_t stream);
+hipError_t launch_camera_count(const uint8_t *hit, int *totals, int cams, int Nq, hipStream_t stream);
+hipError_t launch_camera_index(const uint8_t *hit, const int *totals, int *index, int *pos, int cams, int Nq, int max_len,
+                               hipStream_t stream);
+
 // Weight and bias gradients of a linear layer (dfa3d_linear.hip); O and K even.
 size_t linear_grad_workspace_bytes(long long N, int O, int K);
 hipError_t launch_linear_grad(const float *x, const float *g, float *grad_weight, float *grad_bias, float *workspace,

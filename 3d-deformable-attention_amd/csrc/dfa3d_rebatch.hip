@@ -12,6 +12,10 @@
 //   rebatch_combine_kernel  dst[j, q, :] = scale[j, q] * sum over cameras i with pos[i, q] >= 0 of
 //                           src[j, i, pos[i, q], :]; also the backward of the gather
 //
+//   camera_hits_kernel      which cameras see a query, and one over how many do
+//   camera_count_kernel, camera_index_kernel   the queries of each camera in ascending order, and the inverse
+//                           (:704-707 is a nonzero call per camera)
+//
 // index (cams, max_len) lists the queries of each camera, pos (cams, Nq) is its inverse
 // (position of query q in camera i's list, or -1).  Rows are E contiguous elements; a lane moves
 // 16 bytes when the row length allows it.  Pure streaming: bound by HBM bandwidth.
@@ -167,6 +171,96 @@ hipError_t launch_rebatch_combine(const void *src, const int *pos, const void *s
   if (dtype == DFA3D_F32) return combine_typed<float>(src, pos, scale, dst, bs, cams, max_len, Nq, E, aligned, stream);
   if (dtype == DFA3D_F64) return combine_typed<double>(src, pos, scale, dst, bs, cams, max_len, Nq, E, aligned, stream);
   return hipErrorInvalidValue;
+}
+
+// ---------------------------------------------------------------------------------------
+// From the mask of the anchors to index and pos.  All of it is a few hundred kilobytes: what it costs is launches and
+// dependent passes, of which plain tensor operations take about twenty (a running sum along 40 000 queries alone
+// 93 us: one workgroup per camera walks them); these are three launches, with the one copy of the camera totals to the
+// host, which has to size the batch, between the second and the third.
+// ---------------------------------------------------------------------------------------
+constexpr int kIndexBlock = 1024;
+
+// mask (cams, bs, Nq, Z) bytes: hit[i, q] = any anchor of query q of the first batch element falls into camera i;
+// scale[j, q] = 1 / max(number of cameras with any anchor of query q of batch element j, 1)
+__global__ __launch_bounds__(256) void camera_hits_kernel(const uint8_t *__restrict__ mask, uint8_t *__restrict__ hit,
+                                                          float *__restrict__ scale, int cams, int bs, int Nq, int Z) {
+  const long long n = (long long)bs * Nq;
+  for (long long t = (long long)blockIdx.x * 256 + threadIdx.x; t < n; t += (long long)gridDim.x * 256) {
+    int seen = 0;
+    for (int i = 0; i < cams; ++i) {
+      const uint8_t *p = mask + ((long long)i * n + t) * Z;
+      int any = 0;
+      if (Z == 4 && ((uintptr_t)mask & 3) == 0) {            // uniform
+        any = *reinterpret_cast<const uint32_t *>(p) != 0;
+      } else {
+        for (int z = 0; z < Z; ++z) any |= p[z] != 0;
+      }
+      seen += any;
+      if (t < Nq) hit[(long long)i * Nq + t] = (uint8_t)any;
+    }
+    scale[t] = 1.0f / (float)max(seen, 1);
+  }
+}
+
+// the block's sum of a number per thread, in every thread
+__device__ __forceinline__ int block_sum(int x, int *s_part) {
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = x;
+  __syncthreads();
+  int sum = 0;
+  for (int w = 0; w < kIndexBlock / 64; ++w) sum += s_part[w];
+  return sum;
+}
+
+__global__ __launch_bounds__(kIndexBlock) void camera_count_kernel(const uint8_t *__restrict__ hit, int *__restrict__ totals, int Nq) {
+  __shared__ int s_part[kIndexBlock / 64];
+  const uint8_t *mine = hit + (long long)blockIdx.x * Nq;
+  int n = 0;
+  for (int q = threadIdx.x; q < Nq; q += kIndexBlock) n += mine[q] != 0;
+  n = block_sum(n, s_part);
+  if (threadIdx.x == 0) totals[blockIdx.x] = n;
+}
+
+// A block ranks kIndexBlock queries of one camera; it counts the hits before them itself instead of waiting for the
+// blocks that rank those.  pos is written whole, index from 0 to max_len: ranks, then the padding.
+__global__ __launch_bounds__(kIndexBlock) void camera_index_kernel(const uint8_t *__restrict__ hit, const int *__restrict__ totals,
+                                                                   int *__restrict__ index, int *__restrict__ pos, int Nq, int max_len) {
+  __shared__ int s_part[kIndexBlock / 64];
+  const int cam = blockIdx.y, first = blockIdx.x * kIndexBlock, q = first + threadIdx.x;
+  const uint8_t *mine = hit + (long long)cam * Nq;
+  int *index_row = index + (long long)cam * max_len;
+  int before = 0;
+  for (int k = threadIdx.x; k < first; k += kIndexBlock) before += mine[k] != 0;
+  before = block_sum(before, s_part);
+  const bool on = q < Nq && mine[q] != 0;
+  const unsigned long long lanes = __ballot(on);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __syncthreads();
+  if (lane == 0) s_part[wave] = __popcll(lanes);
+  __syncthreads();
+  int rank = before + __popcll(lanes & ((1ull << lane) - 1));
+  for (int w = 0; w < wave; ++w) rank += s_part[w];
+  if (q < Nq) pos[(long long)cam * Nq + q] = on ? rank : -1;
+  if (on && rank < max_len) index_row[rank] = q;
+  if (q < max_len && q >= totals[cam]) index_row[q] = -1;     // max_len <= max(Nq, 1): the blocks cover it
+}
+
+hipError_t launch_camera_hits(const uint8_t *mask, uint8_t *hit, float *scale, int cams, int bs, int Nq, int Z, hipStream_t stream) {
+  hipLaunchKernelGGL(camera_hits_kernel, dim3(rebatch_grid((long long)bs * Nq)), dim3(256), 0, stream, mask, hit, scale, cams,
+                     bs, Nq, Z);
+  return hipGetLastError();
+}
+hipError_t launch_camera_count(const uint8_t *hit, int *totals, int cams, int Nq, hipStream_t stream) {
+  hipLaunchKernelGGL(camera_count_kernel, dim3(cams), dim3(kIndexBlock), 0, stream, hit, totals, Nq);
+  return hipGetLastError();
+}
+hipError_t launch_camera_index(const uint8_t *hit, const int *totals, int *index, int *pos, int cams, int Nq, int max_len,
+                               hipStream_t stream) {
+  hipLaunchKernelGGL(camera_index_kernel, dim3((Nq + kIndexBlock - 1) / kIndexBlock, cams), dim3(kIndexBlock), 0, stream, hit,
+                     totals, index, pos, Nq, max_len);
+  return hipGetLastError();
 }
 
 }  // namespace dfa3d

@@ -42,6 +42,9 @@ SIGNATURES = {
     "dfa3d_fused_backward_static": [_P] * 13 + _DIMS8 + [_I, _I, _O, _P],
     "dfa3d_rebatch_gather": [_P, ctypes.c_longlong, ctypes.c_longlong, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "dfa3d_rebatch_combine": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
+    "dfa3d_camera_hits": [_P] * 3 + [_I] * 4 + [_P],
+    "dfa3d_camera_count": [_P, _P, _I, _I, _P],
+    "dfa3d_camera_index": [_P] * 4 + [_I] * 3 + [_P],
     "dfa3d_linear_grad": [_P] * 5 + [ctypes.c_size_t, ctypes.c_longlong, _I, _I, _P],
     "dfa3d_abi_version": [],
 }

@@ -7,7 +7,7 @@ re-batching (python loops over batch x cameras in the reference, :716-722 and :7
 import torch
 from torch import nn
 
-from ..rebatch import RebatchCombineFunction, RebatchGatherFunction, camera_index, rebatch_gather
+from ..rebatch import RebatchCombineFunction, RebatchGatherFunction, camera_hits, camera_index, rebatch_gather
 from .ms_deform_attn_3d import MSDeformableAttention3D_DFA3D
 from .projection import Projection
 
@@ -74,7 +74,7 @@ class SpatialCrossAttention_DFA3D(nn.Module):
         Z = reference_points_cam.size(3)
         cams = self.num_cams
 
-        hit = bev_mask[:, 0].sum(-1) > 0                                         # (cams, Nq)
+        hit, scale = camera_hits(bev_mask)                                       # (cams, Nq), (bs, Nq)
         index, pos, max_len = camera_index(hit)
         queries_rebatch = RebatchGatherFunction.apply(query, index, pos)         # (bs, cams, max_len, E)
         ref = reference_points_cam.to(query.dtype).reshape(cams, bs, num_query, Z * 3).contiguous()
@@ -99,8 +99,6 @@ class SpatialCrossAttention_DFA3D(nn.Module):
             empty = table[index.clamp(min=0).long()] * valid[..., None, None].to(table.dtype)   # (cams, L, heads, E)
             queries = queries + ((1 - update_weight) * empty[None]).mean(dim=-2)
 
-        count = (bev_mask.sum(-1) > 0).permute(1, 2, 0).sum(-1)                  # (bs, Nq) cameras seeing each query
-        scale = (1.0 / torch.clamp(count, min=1.0)).to(queries.dtype).contiguous()
-        slots = RebatchCombineFunction.apply(queries, index, pos, scale)         # (bs, Nq, E)
+        slots = RebatchCombineFunction.apply(queries, index, pos, scale.to(queries.dtype).contiguous())     # (bs, Nq, E)
         slots = self.output_proj(slots)
         return self.dropout(slots) + inp_residual

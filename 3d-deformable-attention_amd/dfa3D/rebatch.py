@@ -9,7 +9,7 @@ from torch.autograd.function import once_differentiable
 
 from . import _lib
 
-__all__ = ["camera_index", "rebatch_gather", "rebatch_combine", "RebatchGatherFunction", "RebatchCombineFunction"]
+__all__ = ["camera_hits", "camera_index", "rebatch_gather", "rebatch_combine", "RebatchGatherFunction", "RebatchCombineFunction"]
 
 
 def camera_index(hit):
@@ -19,6 +19,8 @@ def camera_index(hit):
     device once, like the reference's ``nonzero`` calls (spatial_cross_attention.py:704-707)."""
     cams, Nq = hit.shape
     hit = hit.bool()
+    if hit.is_cuda and 0 < cams <= 65535 and 0 < Nq <= 2 ** 30:
+        return _camera_index_on_gpu(hit.contiguous())
     rank = hit.cumsum(1, dtype=torch.int32) - 1                      # position among the camera's queries
     pos = torch.where(hit, rank, torch.full_like(rank, -1)).contiguous()
     max_len = int(hit.sum(1).max().item()) if hit.numel() else 0
@@ -26,6 +28,37 @@ def camera_index(hit):
     cam, q = hit.nonzero(as_tuple=True)
     index[cam, rank[cam, q].long()] = q.to(torch.int32)
     return index, pos, max_len
+
+
+def _camera_index_on_gpu(hit):
+    cams, Nq = hit.shape
+    dev, lib = hit.device, _lib.lib()
+    totals = torch.empty(cams, dtype=torch.int32, device=dev)
+    pos = torch.empty(cams, Nq, dtype=torch.int32, device=dev)
+    with torch.cuda.device(dev):
+        _lib.check(lib.dfa3d_camera_count(_lib.ptr(hit), _lib.ptr(totals), cams, Nq, _lib.stream_of(hit)), "dfa3d_camera_count")
+        max_len = max(totals.tolist())                              # waits for the device
+        index = torch.empty(cams, max(max_len, 1), dtype=torch.int32, device=dev)
+        _lib.check(lib.dfa3d_camera_index(_lib.ptr(hit), _lib.ptr(totals), _lib.ptr(index), _lib.ptr(pos), cams, Nq,
+                                          max(max_len, 1), _lib.stream_of(hit)), "dfa3d_camera_index")
+    return index, pos, max_len
+
+
+def camera_hits(bev_mask):
+    """``bev_mask`` (cams, bs, Nq, Z): ``hit`` (cams, Nq) bool, the queries of the first batch element with any anchor in a
+    camera, and ``scale`` (bs, Nq) float32, one over the number of cameras with any anchor of a query (at least 1)."""
+    cams, bs, Nq, Z = bev_mask.shape
+    if bev_mask.is_cuda and bev_mask.dtype == torch.bool and bev_mask.numel() and cams <= 65535 and Nq <= 2 ** 30:
+        mask = bev_mask.contiguous()
+        hit = torch.empty(cams, Nq, dtype=torch.bool, device=mask.device)
+        scale = torch.empty(bs, Nq, dtype=torch.float32, device=mask.device)
+        with torch.cuda.device(mask.device):
+            rc = _lib.lib().dfa3d_camera_hits(_lib.ptr(mask), _lib.ptr(hit), _lib.ptr(scale), cams, bs, Nq, Z,
+                                              _lib.stream_of(mask))
+        _lib.check(rc, "dfa3d_camera_hits")
+        return hit, scale
+    seen = bev_mask.sum(-1) > 0                                              # (cams, bs, Nq)
+    return seen[:, 0], 1.0 / torch.clamp(seen.permute(1, 2, 0).sum(-1), min=1.0)
 
 
 def _check(t, name, dtype=None):

@@ -231,6 +231,18 @@ int dfa3d_rebatch_gather(const void *src, long long cam_stride, long long batch_
 int dfa3d_rebatch_combine(const void *src, const int32_t *pos, const void *scale, void *dst, int bs, int cams,
                           int max_len, int Nq, int E, int dtype, void *stream);
 
+/* From the mask of a re-batching to its lists.  mask (cams, bs, Nq, Z) bytes, non-zero = anchor z of query q of batch
+ * element j falls into camera i.
+ * hits:  hit[i,q] = any anchor of query q of the FIRST batch element; scale[j,q] = 1 / max(cameras that see query q of
+ *        batch element j, 1).
+ * count: totals[i] = number of queries camera i hits.
+ * index: index (cams, max_len) lists the queries of each camera in ascending order, padded with -1, and pos (cams, Nq) is
+ *        its inverse (-1: not seen); 1 <= max_len <= Nq, the largest of totals (or 1). */
+int dfa3d_camera_hits(const uint8_t *mask, uint8_t *hit, float *scale, int cams, int bs, int Nq, int Z, void *stream);
+int dfa3d_camera_count(const uint8_t *hit, int32_t *totals, int cams, int Nq, void *stream);
+int dfa3d_camera_index(const uint8_t *hit, const int32_t *totals, int32_t *index, int32_t *pos, int cams, int Nq, int max_len,
+                       void *stream);
+
 /* Weight and bias gradients of a linear layer y = x weight^T + bias in float32: grad_weight (O, K) = grad_out^T x,
  * grad_bias (O) = column sums of grad_out, or not formed when it is NULL; x (N, K) and grad_out (N, O) row-major, O and K
  * even, every element of the results written, no atomics (the same result every time).  `workspace`: 16-byte aligned
