@@ -24,7 +24,7 @@ MEASURE_LIB = os.path.join(ROOT, "libdfa3d_measure.so")
 EXPERIMENT_LIB = os.path.join(ROOT, "libdfa3d_hip_experiment.so")
 EXPERIMENT_FLAGS = ["-DDFA3D_EXPERIMENT", "-DDFA3D_TILE_TIMING"]
 SOURCES = ["dfa3d_forward.hip", "dfa3d_backward.hip", "dfa3d_backward_binned.hip", "dfa3d_backward_cells.hip",
-           "dfa3d_rebatch.hip", "dfa3d_linear.hip",
+           "dfa3d_rebatch.hip", "dfa3d_linear.hip", "dfa3d_locations.hip",
            "dfa3d_api.hip"]
 HEADERS = ["dfa3d_device.h", "dfa3d_launch.h", "dfa3d_binned.h", os.path.join("..", "..", "include", "dfa3d.h")]
 FLAGS = [

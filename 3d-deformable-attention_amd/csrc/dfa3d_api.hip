@@ -479,6 +479,30 @@ int dfa3d_camera_index(const uint8_t *hit, const int32_t *totals, int32_t *index
   return hip_result(dfa3d::launch_camera_index(hit, totals, index, pos, cams, Nq, max_len, (hipStream_t)stream), fn);
 }
 
+static int check_locations(const char *fn, long long rows, int M, int L, int P, int Z) {
+  if (rows <= 0 || M <= 0 || L <= 0 || P <= 0 || Z <= 0)
+    return fail(DFA3D_EINVAL, "%s: dimensions must be positive (rows=%lld M=%d L=%d P=%d Z=%d)", fn, rows, M, L, P, Z);
+  if (rows > (1LL << 31) || (long long)M * L * P > (1 << 30))
+    return fail(DFA3D_ERANGE, "%s: at most 2^31 rows of 2^30 points", fn);
+  return 0;
+}
+
+int dfa3d_locations(const float *uv, const float *dz, const float *ref, const int64_t *shapes3, float *loc, long long rows, int M,
+                    int L, int P, int Z, void *stream) {
+  const char *fn = "dfa3d_locations";
+  if (int rc = check_locations(fn, rows, M, L, P, Z)) return rc;
+  REQUIRE_PTR(fn, uv); REQUIRE_PTR(fn, dz); REQUIRE_PTR(fn, ref); REQUIRE_PTR(fn, shapes3); REQUIRE_PTR(fn, loc);
+  return hip_result(dfa3d::launch_locations(uv, dz, ref, shapes3, loc, rows, M, L, P, Z, (hipStream_t)stream), fn);
+}
+
+int dfa3d_locations_grad(const float *grad_loc, const int64_t *shapes3, float *grad_uv, float *grad_dz, long long rows, int M, int L,
+                         int P, void *stream) {
+  const char *fn = "dfa3d_locations_grad";
+  if (int rc = check_locations(fn, rows, M, L, P, 1)) return rc;
+  REQUIRE_PTR(fn, grad_loc); REQUIRE_PTR(fn, shapes3); REQUIRE_PTR(fn, grad_uv); REQUIRE_PTR(fn, grad_dz);
+  return hip_result(dfa3d::launch_locations_grad(grad_loc, shapes3, grad_uv, grad_dz, rows, M, L, P, (hipStream_t)stream), fn);
+}
+
 static int check_linear(const char *fn, long long N, int O, int K) {
   if (N <= 0 || O <= 0 || K <= 0) return fail(DFA3D_EINVAL, "%s: dimensions must be positive (N=%lld O=%d K=%d)", fn, N, O, K);
   if ((O & 1) || (K & 1)) return fail(DFA3D_EINVAL, "%s: O and K must be even (O=%d K=%d)", fn, O, K);

@@ -147,6 +147,12 @@ hipError_t launch_camera_count(const uint8_t *hit, int *totals, int cams, int Nq
 hipError_t launch_camera_index(const uint8_t *hit, const int *totals, int *index, int *pos, int cams, int Nq, int max_len,
                                hipStream_t stream);
 
+// Sampling locations of a layer and their gradients (dfa3d_locations.hip).
+hipError_t launch_locations(const float *uv, const float *dz, const float *ref, const int64_t *shapes3, float *loc, long long rows,
+                            int M, int L, int P, int Z, hipStream_t stream);
+hipError_t launch_locations_grad(const float *grad_loc, const int64_t *shapes3, float *grad_uv, float *grad_dz, long long rows,
+                                 int M, int L, int P, hipStream_t stream);
+
 // Weight and bias gradients of a linear layer (dfa3d_linear.hip); O and K even.
 size_t linear_grad_workspace_bytes(long long N, int O, int K);
 hipError_t launch_linear_grad(const float *x, const float *g, float *grad_weight, float *grad_bias, float *workspace,

@@ -15,12 +15,46 @@ import warnings
 
 import torch
 from torch import nn
+from torch.autograd import Function
 
 from ..functional import (MultiScale3DDeformableAttnFunction_fp32,
                           MultiScale3DDeformableAttnWeightUpdateFunction_fp32)
-from .projection import Projection
+from .. import _lib
+from .projection import Projection, ordinary
 
 __all__ = ["MSDeformableAttention3D_DFA3D"]
+
+
+class _LocationsFunction(Function):
+    """uv (bs, Q, M, L, P, 2), dz (bs, Q, M, L, P, 1), reference points (bs, Q, Z, 3) and shapes (L, 3) to sampling locations
+    in one kernel; differentiable in uv and dz, any number of times."""
+
+    @staticmethod
+    def forward(ctx, uv, dz, reference_points, shapes3):
+        ctx.save_for_backward(shapes3)
+        bs, Q, M, L, P, _ = uv.shape
+        loc = torch.empty(bs, Q, M, L, P, 3, dtype=torch.float32, device=uv.device)
+        if loc.numel():
+            with torch.cuda.device(uv.device):
+                rc = _lib.lib().dfa3d_locations(_lib.ptr(uv), _lib.ptr(dz), _lib.ptr(reference_points), _lib.ptr(shapes3),
+                                                _lib.ptr(loc), bs * Q, M, L, P, reference_points.shape[2], _lib.stream_of(uv))
+            _lib.check(rc, "dfa3d_locations")
+        return loc
+
+    @staticmethod
+    def backward(ctx, grad):
+        shapes3, = ctx.saved_tensors
+        if torch.is_grad_enabled() or grad.dtype != torch.float32 or not grad.is_cuda or grad.numel() == 0:
+            scaled = grad / shapes3[:, [1, 0, 2]].to(grad.dtype)[None, None, None, :, None, :]
+            return scaled[..., :2], scaled[..., 2:], None, None
+        grad = grad.contiguous()
+        bs, Q, M, L, P, _ = grad.shape
+        grad_uv, grad_dz = grad.new_empty(bs, Q, M, L, P, 2), grad.new_empty(bs, Q, M, L, P, 1)
+        with torch.cuda.device(grad.device):
+            rc = _lib.lib().dfa3d_locations_grad(_lib.ptr(grad), _lib.ptr(shapes3), _lib.ptr(grad_uv), _lib.ptr(grad_dz), bs * Q,
+                                                 M, L, P, _lib.stream_of(grad))
+        _lib.check(rc, "dfa3d_locations_grad")
+        return grad_uv, grad_dz, None, None
 
 
 class MSDeformableAttention3D_DFA3D(nn.Module):
@@ -110,6 +144,11 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
             raise ValueError(f"num_points ({P}) must be a multiple of the number of Z anchors ({Z})")
         uv = self.sampling_offsets(query).view(bs, Q, M, L, P, 2)
         dz = self.sampling_offsets_depth(query).view(bs, Q, M, L, P, 1)
+        if (ordinary(uv, dz, reference_points) and uv.is_contiguous() and dz.is_contiguous()
+                and reference_points.is_contiguous() and not reference_points.requires_grad
+                and reference_points.shape[:2] == (bs, Q) and spatial_shapes_3D.device == uv.device
+                and spatial_shapes_3D.dtype == torch.int64 and spatial_shapes_3D.shape == (L, 3)):
+            return _LocationsFunction.apply(uv, dz, reference_points, spatial_shapes_3D.contiguous())
         normalizer = spatial_shapes_3D[:, [1, 0, 2]].to(query.dtype)              # (W, H, D) per level
         offsets = torch.cat([uv, dz], dim=-1) / normalizer[None, None, None, :, None, :]
         anchors = reference_points[:, :, None, None, None, :, :]                   # (bs, Q, 1, 1, 1, Z, 3)

@@ -11,6 +11,16 @@ from .. import _lib
 
 __all__ = ["Projection"]
 
+
+def ordinary(*tensors):
+    """Plain float32 tensors on one GPU, outside autocast, functorch transforms, forward-mode derivatives, tracing and
+    compilation: what this package's kernels may stand in for torch operations on."""
+    return (all(type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.dtype == torch.float32
+                and t.device == tensors[0].device for t in tensors)
+            and not torch.is_autocast_enabled() and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0)
+
 # Fewer rows than this: the library product is as fast and there is one launch less.
 _MIN_ROWS = 4096
 
@@ -52,17 +62,10 @@ class _ProjectionFunction(Function):
 
 
 def _applies(x, weight, bias):
-    """The plain case: float32 rows on the GPU in ordinary reverse-mode training.  Autocast, functorch transforms,
-    forward-mode derivatives, tracing and compilation see the torch operation itself."""
-    return (bias is not None and x.is_cuda and x.dtype == weight.dtype == bias.dtype == torch.float32
-            and torch.is_grad_enabled() and weight.requires_grad and x.dim() >= 2
+    """Float32 rows on the GPU in ordinary reverse-mode training."""
+    return (bias is not None and torch.is_grad_enabled() and weight.requires_grad and x.dim() >= 2
             and weight.shape[0] % 2 == 0 and weight.shape[1] % 2 == 0 and max(weight.shape) <= 16384
-            and _MIN_ROWS <= x.numel() // max(x.shape[-1], 1) <= 2 ** 31
-            and type(x) in (torch.Tensor, nn.Parameter) and type(weight) is nn.Parameter and type(bias) is nn.Parameter
-            and x.device == weight.device == bias.device
-            and not torch.is_autocast_enabled() and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0)
+            and _MIN_ROWS <= x.numel() // max(x.shape[-1], 1) <= 2 ** 31 and ordinary(x, weight, bias))
 
 
 class Projection(nn.Linear):

@@ -243,6 +243,14 @@ int dfa3d_camera_count(const uint8_t *hit, int32_t *totals, int cams, int Nq, vo
 int dfa3d_camera_index(const uint8_t *hit, const int32_t *totals, int32_t *index, int32_t *pos, int cams, int Nq, int max_len,
                        void *stream);
 
+/* Sampling locations of a cross-attention layer in float32: loc (rows, M, L, P, 3) = (uv / (W, H), dz / D) of the level plus
+ * ref[row, p % Z], with uv (rows, M, L, P, 2), dz (rows, M, L, P), ref (rows, Z, 3) and shapes3 (L, 3) = (H, W, D) on the
+ * device; and the gradients of uv and dz from grad_loc.  Every element written. */
+int dfa3d_locations(const float *uv, const float *dz, const float *ref, const int64_t *shapes3, float *loc, long long rows, int M,
+                    int L, int P, int Z, void *stream);
+int dfa3d_locations_grad(const float *grad_loc, const int64_t *shapes3, float *grad_uv, float *grad_dz, long long rows, int M, int L,
+                         int P, void *stream);
+
 /* Weight and bias gradients of a linear layer y = x weight^T + bias in float32: grad_weight (O, K) = grad_out^T x,
  * grad_bias (O) = column sums of grad_out, or not formed when it is NULL; x (N, K) and grad_out (N, O) row-major, O and K
  * even, every element of the results written, no atomics (the same result every time).  `workspace`: 16-byte aligned
