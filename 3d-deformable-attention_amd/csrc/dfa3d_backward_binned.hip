@@ -50,39 +50,48 @@ __global__ __launch_bounds__(256) void plan_and_clear_kernel(
     BinWorkspace ws, const int64_t *__restrict__ shapes, int shape_stride, const int64_t *__restrict__ level_start, int L,
     int S, int D,
     int B, int M, int ty, int tx, int chunk, int max_bins_per_bm) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    BinPlan p;
-    int base = 0;
-    for (int l = 0; l < DFA3D_MAX_LEVELS; ++l) {
+  if (blockIdx.x == 0) {      // a lane per level, a lane per pair of levels: one after the other they took most of the launch
+    static_assert(DFA3D_MAX_LEVELS * DFA3D_MAX_LEVELS == 256, "one thread per pair of levels");
+    __shared__ BinPlan p;
+    __shared__ int s_tiles[DFA3D_MAX_LEVELS];
+    const int t = threadIdx.x;
+    if (t < DFA3D_MAX_LEVELS) {
       int64_t H = 0, W = 0, Dd = 0, st = 0;
       bool ok = false;
-      if (l < L) {
-        H = shapes[l * shape_stride]; W = shapes[l * shape_stride + 1];
-        Dd = (shape_stride > 2 && D > 0) ? shapes[l * shape_stride + 2] : 1; st = level_start[l];
+      if (t < L) {
+        H = shapes[t * shape_stride]; W = shapes[t * shape_stride + 1];
+        Dd = (shape_stride > 2 && D > 0) ? shapes[t * shape_stride + 2] : 1; st = level_start[t];
         ok = H > 0 && W > 0 && st >= 0 && H <= S && W <= S && st + H * W <= (int64_t)S && Dd > 0 &&
              (D <= 0 || Dd <= D);
       }
-      p.H[l] = ok ? (int)H : 0; p.W[l] = ok ? (int)W : 0; p.Dd[l] = ok ? (int)Dd : 0; p.start[l] = ok ? (int)st : 0;
+      p.H[t] = ok ? (int)H : 0; p.W[t] = ok ? (int)W : 0; p.Dd[t] = ok ? (int)Dd : 0; p.start[t] = ok ? (int)st : 0;
       // tiles are laid over the base pixels of the points, which run from -1 (a location within half a pixel of
       // the map's upper / left edge) to H - 1 / W - 1: the first tile starts at pixel -1
       const int nx = ok ? ((int)W + tx) / tx : 0, ny = ok ? ((int)H + ty) / ty : 0;
-      p.tiles_x[l] = nx;
-      p.level_base[l] = base;
-      base += nx * ny;
+      p.tiles_x[t] = nx;
+      s_tiles[t] = nx * ny;
     }
-    // the host sized the counters from an upper bound of the tile count; never exceed it
-    if (base > max_bins_per_bm) base = 0;
-    p.bins_per_bm = base;
-    p.total_bins = base * slot_count(B, M);
-    p.bins_per_class = base * head_groups(M) * B;
-    for (int c = 0; c <= kClasses; ++c) p.class_start[c] = 0;
-    p.ty = ty; p.tx = tx;
-    p.chunk = chunk; p.total_chunks = 0;
-    p.disjoint = 1;
-    for (int l = 1; l < L; ++l)
-      for (int k = 0; k < l; ++k)
-        if (p.start[l] < p.start[k] + p.H[k] * p.W[k] && p.start[k] < p.start[l] + p.H[l] * p.W[l]) p.disjoint = 0;
-    *ws.plan = p;
+    if (t <= kClasses) p.class_start[t] = 0;
+    if (t == 0) p.disjoint = 1;
+    __syncthreads();
+    const int l = t / DFA3D_MAX_LEVELS, k = t % DFA3D_MAX_LEVELS;
+    if (k < l && l < L && p.start[l] < p.start[k] + p.H[k] * p.W[k] && p.start[k] < p.start[l] + p.H[l] * p.W[l]) p.disjoint = 0;
+    if (t == 0) {
+      int base = 0;
+      for (int i = 0; i < DFA3D_MAX_LEVELS; ++i) {
+        p.level_base[i] = base;
+        base += s_tiles[i];
+      }
+      // the host sized the counters from an upper bound of the tile count; never exceed it
+      if (base > max_bins_per_bm) base = 0;
+      p.bins_per_bm = base;
+      p.total_bins = base * slot_count(B, M);
+      p.bins_per_class = base * head_groups(M) * B;
+      p.ty = ty; p.tx = tx;
+      p.chunk = chunk; p.total_chunks = 0;
+    }
+    __syncthreads();
+    for (int i = t; i < (int)(sizeof(BinPlan) / 4); i += 256) reinterpret_cast<int *>(ws.plan)[i] = reinterpret_cast<const int *>(&p)[i];
   }
   const size_t n = (size_t)max_bins_per_bm * slot_count(B, M);
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
@@ -229,12 +238,34 @@ __global__ __launch_bounds__(256) void bin_points_kernel(
   }
 }
 
+// What the count and the sorted fill divide by, per point: points of a unit and of a level, tile edges.
+struct BinDivs { FastDiv lp, p, ty, tx; };
+// The plan's tables in LDS: a block of these two kernels lives a few microseconds, most of it waiting, and the bin of a point
+// otherwise takes a chain of three reads of device memory after its location has come, and four divisions by numbers
+// the compiler does not know.  15.36 M points: count 89 -> 52 us (184 MB read, 3.5 TB/s), fill 195 -> 153 us (553 MB moved,
+// 3.6 TB/s, where a copy reaches 4.7).
+struct BinTable {
+  int H[DFA3D_MAX_LEVELS], W[DFA3D_MAX_LEVELS], base[DFA3D_MAX_LEVELS], tiles_x[DFA3D_MAX_LEVELS];
+  __device__ __forceinline__ void load(const BinPlan &p) {     // the caller's barrier
+    const int l = threadIdx.x;
+    if (l < DFA3D_MAX_LEVELS) { H[l] = p.H[l]; W[l] = p.W[l]; base[l] = p.level_base[l]; tiles_x[l] = p.tiles_x[l]; }
+  }
+  // bin of a location on level l, or -1 when the operator skips it (see bin_of)
+  __device__ __forceinline__ int bin(int l, float x, float y, const BinDivs &d) const {
+    const Point2D<float> g = locate_2d<float>(x, y, H[l], W[l], 0);
+    const int across = tiles_x[l];
+    if (!g.inside || across <= 0) return -1;
+    return base[l] + (int)d.ty.div(g.h0 + 1) * across + (int)d.tx.div(g.w0 + 1);
+  }
+};
+
 // Count in the same shape as the sorted fill: 1024 threads, kStage points per block, all loads of a thread issued
 // before its first LDS atomic.
 __global__ __launch_bounds__(kFillThreads) void bin_count_kernel(
     BinWorkspace ws, const float *__restrict__ loc, int loc_stride, int B, int M, int L, int Q, int P, int nq_block,
-    int q_blocks) {
-  __shared__ int s_cnt[kSortedBins];
+    int q_blocks, BinDivs divs) {
+  __shared__ int s_cnt[kSortedBins], s_inside;
+  __shared__ BinTable tab;
   const BinPlan &p = *ws.plan;
   const int nb = p.bins_per_bm;
   const int LP = L * P;
@@ -246,7 +277,6 @@ __global__ __launch_bounds__(kFillThreads) void bin_count_kernel(
   const int q0 = qb * nq_block, nq = min(nq_block, Q - q0);      // any split of the queries gives the same counts
   const int npts = nq * LP;
   constexpr int kPer = kStage / kFillThreads;
-  for (int i = tid; i < nb; i += kFillThreads) s_cnt[i] = 0;
   float x[kPer], y[kPer];
   int lv[kPer];
 #pragma unroll
@@ -254,26 +284,26 @@ __global__ __launch_bounds__(kFillThreads) void bin_count_kernel(
     const int i = tid + kFillThreads * r;
     lv[r] = -1; x[r] = y[r] = 0;
     if (i < npts) {
-      const int qi = i / LP, lp = i - qi * LP;
+      const int qi = divs.lp.div(i), lp = i - qi * LP;
       const size_t gp = ((size_t)(b * (size_t)Q + q0 + qi) * M + m) * LP + lp;
       x[r] = loc[gp * loc_stride]; y[r] = loc[gp * loc_stride + 1];
-      lv[r] = lp / P;
+      lv[r] = divs.p.div(lp);
     }
   }
+  for (int i = tid; i < nb; i += kFillThreads) s_cnt[i] = 0;
+  if (tid == 0) s_inside = 0;
+  tab.load(p);
   __syncthreads();
-  int counted = 0;
+  int counted = 0;                                               // of this wavefront
 #pragma unroll
   for (int r = 0; r < kPer; ++r) {
-    bool inside = false;
-    if (lv[r] >= 0) {
-      const int l = lv[r];
-      const Point2D<float> g = locate_2d<float>(x[r], y[r], p.H[l], p.W[l], p.start[l]);
-      inside = g.inside && p.tiles_x[l] > 0;
-      if (inside) atomicAdd(&s_cnt[bin_of(p, l, g)], 1);
-    }
-    counted += __syncthreads_count(inside);                      // the last one: all have been counted
+    const int bin = lv[r] >= 0 ? tab.bin(lv[r], x[r], y[r], divs) : -1;
+    if (bin >= 0) atomicAdd(&s_cnt[bin], 1);
+    counted += __popcll(__ballot(bin >= 0));
   }
-  if (tid == 0) atomicAdd(counted_points(ws), counted);
+  if (tid % kWave == 0) atomicAdd(&s_inside, counted);
+  __syncthreads();
+  if (tid == 0) atomicAdd(counted_points(ws), s_inside);
   int *gcount = ws.counts + (size_t)bm * nb;
   for (int i = tid; i < nb; i += kFillThreads) {
     const int c = s_cnt[i];
@@ -284,8 +314,9 @@ __global__ __launch_bounds__(kFillThreads) void bin_count_kernel(
 __global__ __launch_bounds__(kFillThreads) void bin_fill_sorted_kernel(
     BinWorkspace ws, const float *__restrict__ loc, int loc_stride, const float *__restrict__ attn,
     float *__restrict__ grad_loc, int gl_stride, float *__restrict__ grad_attn, float *__restrict__ grad_score,
-    int B, int M, int L, int Q, int P, int q_blocks) {
+    int B, int M, int L, int Q, int P, int q_blocks, BinDivs divs) {
   extern __shared__ __align__(16) unsigned char s_raw[];        // kSortedFillLds bytes
+  __shared__ BinTable tab;
   uint4 *s_rec = reinterpret_cast<uint4 *>(s_raw);               // staged records, grouped by bin
   uint32_t *s_gp = reinterpret_cast<uint32_t *>(s_rec + kStage);
   int *s_dst = reinterpret_cast<int *>(s_gp + kStage);
@@ -297,7 +328,6 @@ __global__ __launch_bounds__(kFillThreads) void bin_fill_sorted_kernel(
   const int nb = p.bins_per_bm;
   const int LP = L * P;
   if (nb == 0 || !sorted_fill_applies(nb, LP)) return;
-  decode_items(ws, B, M, L, blockIdx.x, gridDim.x);
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int m = blockIdx.x % M, rest = blockIdx.x / M;          // head = block % M, as in bin_points_kernel
   const int qb = rest % q_blocks, b = rest / q_blocks;
@@ -312,8 +342,6 @@ __global__ __launch_bounds__(kFillThreads) void bin_fill_sorted_kernel(
   int *gcursor = ws.cursor + (size_t)bm * nb;
   constexpr int kPer = kStage / kFillThreads;                             // points per thread
 
-  for (int i = tid; i < nb; i += kFillThreads) s_cnt[i] = 0;
-  __syncthreads();
   // 1. every point: its bin and its rank among this block's points of that bin
   int bin[kPer], rank[kPer];
   uint4 rec[kPer];
@@ -321,26 +349,35 @@ __global__ __launch_bounds__(kFillThreads) void bin_fill_sorted_kernel(
 #pragma unroll
   for (int r = 0; r < kPer; ++r) {
     const int i = tid + kFillThreads * r;
-    bin[r] = -1; rank[r] = 0;
+    bin[r] = -1; rank[r] = 0; gpi[r] = 0;
+    rec[r] = make_uint4(0, 0, 0, 0);
     if (i < npts) {
-      const int qi = i / LP, lp = i - qi * LP, l = lp / P;
+      const int qi = divs.lp.div(i), lp = i - qi * LP;
       const size_t gp = ((size_t)(b * (size_t)Q + qb + (size_t)qi * q_blocks) * M + m) * LP + lp;
-      const float x = loc[gp * loc_stride], y = loc[gp * loc_stride + 1];
-      const Point2D<float> g = locate_2d<float>(x, y, p.H[l], p.W[l], p.start[l]);
-      if (g.inside && p.tiles_x[l] > 0) {
-        bin[r] = bin_of(p, l, g);
-        rank[r] = atomicAdd(&s_cnt[bin[r]], 1);
-        rec[r] = make_uint4(__float_as_uint(x), __float_as_uint(y),
-                            loc_stride > 2 ? __float_as_uint(loc[gp * loc_stride + 2]) : 0u,
-                            attn != nullptr ? __float_as_uint(attn[gp]) : 0u);
-        gpi[r] = (uint32_t)gp;
-      } else {
-        // skipped by the operator: all its gradients are zero, and no tile will visit it
-        for (int c = 0; c < gl_stride; ++c) grad_loc[gp * gl_stride + c] = 0;
-        if (grad_attn != nullptr) grad_attn[gp] = 0;
-        if (grad_score != nullptr) {
-          for (int k = 0; k < 4; ++k) grad_score[gp * 4 + k] = 0;
-        }
+      const float *at = loc + gp * loc_stride;
+      rec[r] = make_uint4(__float_as_uint(at[0]), __float_as_uint(at[1]), loc_stride > 2 ? __float_as_uint(at[2]) : 0u,
+                          attn != nullptr ? __float_as_uint(attn[gp]) : 0u);
+      gpi[r] = (uint32_t)gp;
+      bin[r] = divs.p.div(lp);                                     // the level, for now
+    }
+  }
+  for (int i = tid; i < nb; i += kFillThreads) s_cnt[i] = 0;
+  tab.load(p);
+  decode_items(ws, B, M, L, blockIdx.x, gridDim.x);
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    if (bin[r] < 0) continue;
+    bin[r] = tab.bin(bin[r], __uint_as_float(rec[r].x), __uint_as_float(rec[r].y), divs);
+    if (bin[r] >= 0) {
+      rank[r] = atomicAdd(&s_cnt[bin[r]], 1);
+    } else {
+      // skipped by the operator: all its gradients are zero, and no tile will visit it
+      const size_t gp = gpi[r];
+      for (int c = 0; c < gl_stride; ++c) grad_loc[gp * gl_stride + c] = 0;
+      if (grad_attn != nullptr) grad_attn[gp] = 0;
+      if (grad_score != nullptr) {
+        for (int k = 0; k < 4; ++k) grad_score[gp * 4 + k] = 0;
       }
     }
   }
@@ -1526,17 +1563,22 @@ static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, const Ti
   if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
   const int hist_cap = mb < kHistCap ? mb : kHistCap;
   const unsigned grid = blocks < 2048 ? (unsigned)blocks : 2048u;
-  hipLaunchKernelGGL(bin_points_kernel<0>, dim3(grid), dim3(256), (size_t)hist_cap * 4, stream, ws,
+  const int LP = a.L * a.P;
+  // Of the two forms of counting and filling the plan kernel's result decides between, and the other steps aside; a map
+  // so small that it cannot have too many bins for the sorted form spares the two launches that would (4.5 us each).
+  const bool sorted_surely = LP <= kStage && mb <= kSortedBins;
+  if (!sorted_surely)
+    hipLaunchKernelGGL(bin_points_kernel<0>, dim3(grid), dim3(256), (size_t)hist_cap * 4, stream, ws,
                      (const float *)a.loc, a.loc_stride, (const float *)a.attn, (float *)a.grad_loc, a.grad_loc_stride,
                      (float *)a.grad_attn, (float *)a.grad_score_out, a.B, a.M, a.L, a.Q, a.P, q_blocks, (int)blocks, hist_cap DFA3D_DIAG_ARG(a));
-  const int LP = a.L * a.P;
   const int nq_block = LP <= kStage ? kStage / LP : 1;
   const int q_blocks2 = (a.Q + nq_block - 1) / nq_block;
   const long long blocks2 = (long long)a.B * a.M * q_blocks2;
   if (blocks2 > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
+  const BinDivs divs{FastDiv((uint32_t)LP), FastDiv((uint32_t)a.P), FastDiv((uint32_t)ty), FastDiv((uint32_t)tx)};
   if (LP <= kStage)                         // steps aside if there turn out to be too many bins, as the one above does if not
     hipLaunchKernelGGL(bin_count_kernel, dim3((unsigned)blocks2), dim3(kFillThreads), 0, stream, ws, (const float *)a.loc,
-                       a.loc_stride, a.B, a.M, a.L, a.Q, a.P, nq_block, q_blocks2);
+                       a.loc_stride, a.B, a.M, a.L, a.Q, a.P, nq_block, q_blocks2, divs);
   // What further blocks of the scan's launch clear meanwhile: for a caller that did not zero them (options.clear),
   // the rows of grad_value / grad_dist that the tile kernel adds to rather than stores; and always, for a
   // distribution shared by the heads, those rows of the per-head grad_dist in the workspace (the head sum then
@@ -1562,9 +1604,10 @@ static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, const Ti
     if (hipError_t e = allow_lds(bin_fill_sorted_kernel, kSortedFillLds)) return e;
     hipLaunchKernelGGL(bin_fill_sorted_kernel, dim3((unsigned)blocks2), dim3(kFillThreads), kSortedFillLds, stream, ws, (const float *)a.loc,
                        a.loc_stride, (const float *)a.attn, (float *)a.grad_loc, a.grad_loc_stride, (float *)a.grad_attn,
-                       (float *)a.grad_score_out, a.B, a.M, a.L, a.Q, a.P, q_blocks2);
+                       (float *)a.grad_score_out, a.B, a.M, a.L, a.Q, a.P, q_blocks2, divs);
   }
-  hipLaunchKernelGGL(bin_points_kernel<1>, dim3(grid), dim3(256), (size_t)hist_cap * 8, stream, ws,
+  if (!sorted_surely)
+    hipLaunchKernelGGL(bin_points_kernel<1>, dim3(grid), dim3(256), (size_t)hist_cap * 8, stream, ws,
                      (const float *)a.loc, a.loc_stride, (const float *)a.attn, (float *)a.grad_loc, a.grad_loc_stride,
                      (float *)a.grad_attn, (float *)a.grad_score_out, a.B, a.M, a.L, a.Q, a.P, q_blocks, (int)blocks, hist_cap DFA3D_DIAG_ARG(a));
   return hipGetLastError();
