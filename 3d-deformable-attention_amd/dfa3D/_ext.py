@@ -58,7 +58,7 @@ def _aux_dtype(storage):
 
 
 def _expect(t, name, shape=None, dtype=None):
-    if shape is not None and tuple(t.shape) != tuple(shape):
+    if shape is not None and t.shape != tuple(shape):
         raise RuntimeError(f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
     if dtype is not None and t.dtype != dtype:
         raise RuntimeError(f"{name} has dtype {t.dtype}, expected {dtype}")
@@ -96,7 +96,7 @@ def ms_depth_score_sample_forward(value, value_spatial_shapes, value_level_start
     score = torch.empty(B, Q, M, L, P, 4, dtype=value.dtype, device=dev)
     if score.numel() == 0:
         return score
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib().dfa3d_ms_depth_score_sample_forward(
             _lib.ptr(value), _lib.ptr(value_spatial_shapes), _lib.ptr(value_level_start_index),
             _lib.ptr(sampling_locations), _lib.ptr(score), B, S, M, D, L, Q, P, code,
@@ -129,7 +129,7 @@ def ms_depth_score_sample_backward(value, value_spatial_shapes, value_level_star
     code = _lib.dtype_code(value)
     ws_bytes = _lib.lib().dfa3d_ms_depth_score_sample_backward_workspace_bytes(B, S, M, D, L, Q, P, code, _lib.options())
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib().dfa3d_ms_depth_score_sample_backward(
             _lib.ptr(value), _lib.ptr(value_spatial_shapes), _lib.ptr(value_level_start_index),
             _lib.ptr(sampling_locations), _lib.ptr(grad_output), _lib.ptr(grad_value), _lib.ptr(grad_sampling_loc),
@@ -171,7 +171,7 @@ def wms_deform_attn_forward(value, value_spatial_shapes, value_level_start_index
     out = torch.empty(B, Q, M * C, dtype=value.dtype, device=dev)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib().dfa3d_wms_deform_attn_forward(
             _lib.ptr(value), _lib.ptr(value_spatial_shapes), sw, _lib.ptr(value_level_start_index),
             _lib.ptr(sampling_locations), lw, _lib.ptr(attention_weights), _lib.ptr(depth_scores), _lib.ptr(out),
@@ -226,7 +226,7 @@ def wms_deform_attn_backward_into(value, value_spatial_shapes, value_level_start
     with (_lib.launch_options(clear=1) if clear else contextlib.nullcontext()):
         ws_bytes = _lib.lib().dfa3d_wms_deform_attn_backward_workspace_bytes(B, S, M, C, L, Q, P, code, _lib.options())
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = _lib.lib().dfa3d_wms_deform_attn_backward(
                 _lib.ptr(value), _lib.ptr(value_spatial_shapes), sw, _lib.ptr(value_level_start_index),
                 _lib.ptr(sampling_locations), lw, _lib.ptr(attention_weights), _lib.ptr(depth_scores),
@@ -252,7 +252,7 @@ def ms_deform_attn_forward(value, value_spatial_shapes, value_level_start_index,
     out = torch.empty(B, Q, M * C, dtype=value.dtype, device=dev)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib().dfa3d_wms_deform_attn_forward(
             _lib.ptr(value), _lib.ptr(value_spatial_shapes), sw, _lib.ptr(value_level_start_index),
             _lib.ptr(sampling_locations), lw, _lib.ptr(attention_weights), None, _lib.ptr(out),
@@ -290,7 +290,7 @@ def ms_deform_attn_backward(value, value_spatial_shapes, value_level_start_index
     with (_lib.launch_options(clear=1) if clear else contextlib.nullcontext()):
         ws_bytes = _lib.lib().dfa3d_wms_deform_attn_backward_workspace_bytes(B, S, M, C, L, Q, P, code, _lib.options())
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = _lib.lib().dfa3d_wms_deform_attn_backward(
                 _lib.ptr(value), _lib.ptr(value_spatial_shapes), sw, _lib.ptr(value_level_start_index),
                 _lib.ptr(sampling_locations), lw, _lib.ptr(attention_weights), None, _lib.ptr(grad_output),
@@ -335,7 +335,7 @@ def pack_shared_dist(value_dpt_dist, value_spatial_shapes, value_level_start_ind
     if n == 0:
         return None
     packed = torch.empty(n, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib().dfa3d_pack_dist(_lib.ptr(value_dpt_dist), _lib.ptr(value_spatial_shapes),
                                         _lib.ptr(value_level_start_index), _lib.ptr(packed), n, B, S, D, L, code,
                                         _lib.stream_of(value_dpt_dist))
@@ -370,7 +370,7 @@ def dfa3d_fused_forward(value, value_dpt_dist, value_spatial_shapes, value_level
     wu = torch.empty(B, Q, M, 1, dtype=_aux_dtype(value.dtype), device=dev) if need_weight_update else None
     if out.numel() == 0:
         return (out, score, wu) if need_weight_update else (out, score)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib().dfa3d_fused_forward(
             _lib.ptr(value), _lib.ptr(value_dpt_dist), _lib.ptr(value_spatial_shapes),
             _lib.ptr(value_level_start_index), _lib.ptr(sampling_locations), _lib.ptr(attention_weights),
@@ -444,7 +444,7 @@ def dfa3d_fused_backward(value, value_dpt_dist, value_spatial_shapes, value_leve
         ws_bytes = _lib.lib().dfa3d_fused_backward_workspace_bytes(B, S, M, C, D, L, Q, P, value_dpt_dist.shape[2],
                                                                     code, _lib.options())
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = _lib.lib().dfa3d_fused_backward(
                 _lib.ptr(value), _lib.ptr(value_dpt_dist), _lib.ptr(value_spatial_shapes),
                 _lib.ptr(value_level_start_index), _lib.ptr(sampling_locations), _lib.ptr(attention_weights),

@@ -159,8 +159,18 @@ def dtype_code(t):
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    """Address of a tensor's data for a pointer argument, None for NULL."""
+    return t.data_ptr() if t is not None else None
 
 
 def stream_of(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    """The current stream of a tensor's GPU (the handle alone: a Stream object costs as much as a launch)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+_HERE_ALREADY = contextlib.nullcontext()
+
+
+def on_device(dev):
+    """Context in which ``dev`` is the current GPU; nothing to enter or leave when it is that already."""
+    return _HERE_ALREADY if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)

@@ -35,7 +35,7 @@ class _LocationsFunction(Function):
         bs, Q, M, L, P, _ = uv.shape
         loc = torch.empty(bs, Q, M, L, P, 3, dtype=torch.float32, device=uv.device)
         if loc.numel():
-            with torch.cuda.device(uv.device):
+            with _lib.on_device(uv.device):
                 rc = _lib.lib().dfa3d_locations(_lib.ptr(uv), _lib.ptr(dz), _lib.ptr(reference_points), _lib.ptr(shapes3),
                                                 _lib.ptr(loc), bs * Q, M, L, P, reference_points.shape[2], _lib.stream_of(uv))
             _lib.check(rc, "dfa3d_locations")
@@ -50,7 +50,7 @@ class _LocationsFunction(Function):
         grad = grad.contiguous()
         bs, Q, M, L, P, _ = grad.shape
         grad_uv, grad_dz = grad.new_empty(bs, Q, M, L, P, 2), grad.new_empty(bs, Q, M, L, P, 1)
-        with torch.cuda.device(grad.device):
+        with _lib.on_device(grad.device):
             rc = _lib.lib().dfa3d_locations_grad(_lib.ptr(grad), _lib.ptr(shapes3), _lib.ptr(grad_uv), _lib.ptr(grad_dz), bs * Q,
                                                  M, L, P, _lib.stream_of(grad))
         _lib.check(rc, "dfa3d_locations_grad")

@@ -34,7 +34,7 @@ def _weight_gradients(x, grad, want_bias):
     lib = _lib.lib()
     nbytes = lib.dfa3d_linear_grad_workspace_bytes(N, O, K)
     workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = lib.dfa3d_linear_grad(_lib.ptr(x), _lib.ptr(grad), _lib.ptr(grad_weight), _lib.ptr(grad_bias),
                                    _lib.ptr(workspace), nbytes, N, O, K, _lib.stream_of(x))
     _lib.check(rc, "dfa3d_linear_grad")

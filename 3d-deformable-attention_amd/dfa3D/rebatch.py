@@ -35,7 +35,7 @@ def _camera_index_on_gpu(hit):
     dev, lib = hit.device, _lib.lib()
     totals = torch.empty(cams, dtype=torch.int32, device=dev)
     pos = torch.empty(cams, Nq, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(lib.dfa3d_camera_count(_lib.ptr(hit), _lib.ptr(totals), cams, Nq, _lib.stream_of(hit)), "dfa3d_camera_count")
         max_len = max(totals.tolist())                              # waits for the device
         index = torch.empty(cams, max(max_len, 1), dtype=torch.int32, device=dev)
@@ -52,7 +52,7 @@ def camera_hits(bev_mask):
         mask = bev_mask.contiguous()
         hit = torch.empty(cams, Nq, dtype=torch.bool, device=mask.device)
         scale = torch.empty(bs, Nq, dtype=torch.float32, device=mask.device)
-        with torch.cuda.device(mask.device):
+        with _lib.on_device(mask.device):
             rc = _lib.lib().dfa3d_camera_hits(_lib.ptr(mask), _lib.ptr(hit), _lib.ptr(scale), cams, bs, Nq, Z,
                                               _lib.stream_of(mask))
         _lib.check(rc, "dfa3d_camera_hits")
@@ -93,7 +93,7 @@ def rebatch_gather(src, index, scale=None, per_camera=False):
     dst = torch.empty(bs, cams, max_len, E, dtype=src.dtype, device=src.device)
     if dst.numel() == 0:
         return dst
-    with torch.cuda.device(src.device):
+    with _lib.on_device(src.device):
         rc = _lib.lib().dfa3d_rebatch_gather(_lib.ptr(src), cam_stride, batch_stride, _lib.ptr(index), _lib.ptr(scale),
                                              _lib.ptr(dst), bs, cams, max_len, Nq, E, _lib.dtype_code(src),
                                              _lib.stream_of(src))
@@ -119,7 +119,7 @@ def rebatch_combine(src, pos, scale=None):
         return dst
     if src.numel() == 0:
         return dst.zero_()
-    with torch.cuda.device(src.device):
+    with _lib.on_device(src.device):
         rc = _lib.lib().dfa3d_rebatch_combine(_lib.ptr(src), _lib.ptr(pos), _lib.ptr(scale), _lib.ptr(dst), bs, cams,
                                               max_len, Nq, E, _lib.dtype_code(src), _lib.stream_of(src))
     _lib.check(rc, "dfa3d_rebatch_combine")
