@@ -20,7 +20,7 @@ from torch.autograd import Function
 from ..functional import (MultiScale3DDeformableAttnFunction_fp32,
                           MultiScale3DDeformableAttnWeightUpdateFunction_fp32)
 from .. import _lib
-from .projection import Projection, ordinary
+from .projection import Projection, ordinary, plain_gradient
 
 __all__ = ["MSDeformableAttention3D_DFA3D"]
 
@@ -44,7 +44,7 @@ class _LocationsFunction(Function):
     @staticmethod
     def backward(ctx, grad):
         shapes3, = ctx.saved_tensors
-        if torch.is_grad_enabled() or grad.dtype != torch.float32 or not grad.is_cuda or grad.numel() == 0:
+        if not plain_gradient(grad) or grad.numel() == 0:
             scaled = grad / shapes3[:, [1, 0, 2]].to(grad.dtype)[None, None, None, :, None, :]
             return scaled[..., :2], scaled[..., 2:], None, None
         grad = grad.contiguous()

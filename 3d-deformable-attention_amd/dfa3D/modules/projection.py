@@ -41,6 +41,12 @@ def _weight_gradients(x, grad, want_bias):
     return grad_weight, grad_bias
 
 
+def plain_gradient(grad):
+    """A gradient that a kernel may read: float32 on the GPU, not recorded and not a batch of gradients (is_grads_batched)."""
+    return (not torch.is_grad_enabled() and grad.is_cuda and grad.dtype == torch.float32
+            and not torch._C._functorch.is_batchedtensor(grad) and not torch._C._functorch.is_legacy_batchedtensor(grad))
+
+
 class _ProjectionFunction(Function):
     """``F.linear(x, weight, bias)`` with a bias; differentiable any number of times (a backward that is itself recorded
     is made of torch operations)."""
@@ -56,7 +62,7 @@ class _ProjectionFunction(Function):
         want_x, want_weight, want_bias = ctx.needs_input_grad
         grad_x = grad.matmul(weight) if want_x else None
         rows, grad_rows = x.reshape(-1, x.shape[-1]), grad.reshape(-1, grad.shape[-1])
-        if torch.is_grad_enabled() or not want_weight or grad.dtype != torch.float32:
+        if not want_weight or not plain_gradient(grad):
             return grad_x, grad_rows.t().mm(rows) if want_weight else None, grad_rows.sum(0) if want_bias else None
         return (grad_x, *_weight_gradients(rows.contiguous(), grad_rows.contiguous(), want_bias))
 

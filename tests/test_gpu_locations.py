@@ -37,6 +37,10 @@ def test_locations_and_gradients(bs, Q, M, L, P, Z):
     first = torch.autograd.grad((got ** 3).sum(), [query], create_graph=True)[0]
     if Q:
         assert torch.autograd.grad(first.sum(), [query])[0].abs().max() > 0
+        many = torch.randn(2, *got.shape, device=dev)
+        batch, = torch.autograd.grad(mod.sampling_locations(query, ref, shapes), [mod.sampling_offsets_depth.bias], many, is_grads_batched=True)
+        plain, = torch.autograd.grad(_plain(mod, query, ref, shapes), [mod.sampling_offsets_depth.bias], many, is_grads_batched=True)
+        torch.testing.assert_close(batch, plain, rtol=1e-4, atol=1e-4)
     wanting = ref.clone().requires_grad_()
     moved = mod.sampling_locations(query, wanting, shapes)
     assert torch.equal(moved, want) and torch.autograd.grad(moved.sum(), [wanting])[0].shape == ref.shape

@@ -55,6 +55,9 @@ def test_calls_that_keep_the_librarys_operation():
     rw, = torch.autograd.grad(ref(x, layer.weight, layer.bias).square().sum(), [layer.weight], create_graph=True)
     want, = torch.autograd.grad(rw.square().sum(), [x])
     torch.testing.assert_close(second, want, rtol=1e-3, atol=1e-3 * want.abs().max().item())
+    gs = torch.randn(3, 4200, 64, device=dev)
+    batched, = torch.autograd.grad(layer(x), [layer.weight], gs, is_grads_batched=True)
+    torch.testing.assert_close(batched, gs.transpose(1, 2) @ x.detach(), rtol=1e-3, atol=1e-2)
     per = torch.func.vmap(lambda t: layer(t))(x.detach().view(1, 4200, 64))
     torch.testing.assert_close(per[0], layer(x.detach()))
     out, tangent = torch.func.jvp(lambda t: layer(t), (x.detach(),), (torch.ones_like(x),))
