@@ -128,8 +128,31 @@ size_t dfa3d_ms_depth_score_sample_backward_workspace_bytes(int B, int S, int M,
   dfa3d_launch_options o;
   if (check_dims(fn, B, S, M, D, L, Q, P, dtype) || check_opts(fn, opts, &o)) return 0;
   if (o.direct) return 0;
-  dfa3d::DepthScoreBwdArgs a{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, B, S, M, D, L, Q, P};
+  dfa3d::DepthScoreBwdArgs a{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, B, S, M, D, L, Q, P, 0};
   return dfa3d::binned_depth_score_backward_workspace_bytes(a, dtype, o.tile);
+}
+
+static int depth_score_backward(const char *fn, bool clear, const void *dist, const int64_t *shapes3, const int64_t *level_start,
+                                const void *loc3, const void *grad_score, void *grad_dist, void *grad_loc3, void *workspace,
+                                size_t workspace_bytes, int B, int S, int M, int D, int L, int Q, int P, int dtype,
+                                const dfa3d_launch_options *opts, void *stream) {
+  dfa3d_launch_options o;
+  if (int rc = check_dims(fn, B, S, M, D, L, Q, P, dtype)) return rc;
+  if (int rc = check_opts(fn, opts, &o)) return rc;
+  REQUIRE_PTR(fn, dist); REQUIRE_PTR(fn, shapes3); REQUIRE_PTR(fn, level_start); REQUIRE_PTR(fn, loc3);
+  REQUIRE_PTR(fn, grad_score); REQUIRE_PTR(fn, grad_dist); REQUIRE_PTR(fn, grad_loc3);
+  dfa3d::DepthScoreBwdArgs a{dist, shapes3, level_start, loc3, grad_score, grad_dist, grad_loc3, B, S, M, D, L, Q, P, clear ? 1 : 0};
+  if (workspace != nullptr && !o.direct) {
+    const hipError_t e = dfa3d::launch_depth_score_backward_binned(a, dtype, workspace, workspace_bytes, o.tile, o.chunk,
+                                                                   o.event_binned, (hipStream_t)stream);
+    if (e != hipErrorNotSupported) return hip_result(e, fn);
+  }
+  if (clear) {
+    const size_t bytes = (size_t)B * S * M * D * (dtype == DFA3D_F64 ? 8 : 4);
+    const hipError_t e = dfa3d::launch_zero_fill(grad_dist, bytes, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_result(e, fn);
+  }
+  return hip_result(dfa3d::launch_depth_score_backward(a, dtype, (hipStream_t)stream), fn);
 }
 
 int dfa3d_ms_depth_score_sample_backward(const void *dist, const int64_t *shapes3, const int64_t *level_start,
@@ -137,19 +160,17 @@ int dfa3d_ms_depth_score_sample_backward(const void *dist, const int64_t *shapes
                                          void *workspace, size_t workspace_bytes,
                                          int B, int S, int M, int D, int L, int Q, int P, int dtype,
                                          const dfa3d_launch_options *opts, void *stream) {
-  const char *fn = "dfa3d_ms_depth_score_sample_backward";
-  dfa3d_launch_options o;
-  if (int rc = check_dims(fn, B, S, M, D, L, Q, P, dtype)) return rc;
-  if (int rc = check_opts(fn, opts, &o)) return rc;
-  REQUIRE_PTR(fn, dist); REQUIRE_PTR(fn, shapes3); REQUIRE_PTR(fn, level_start); REQUIRE_PTR(fn, loc3);
-  REQUIRE_PTR(fn, grad_score); REQUIRE_PTR(fn, grad_dist); REQUIRE_PTR(fn, grad_loc3);
-  dfa3d::DepthScoreBwdArgs a{dist, shapes3, level_start, loc3, grad_score, grad_dist, grad_loc3, B, S, M, D, L, Q, P};
-  if (workspace != nullptr && !o.direct) {
-    const hipError_t e = dfa3d::launch_depth_score_backward_binned(a, dtype, workspace, workspace_bytes, o.tile, o.chunk,
-                                                                   o.event_binned, (hipStream_t)stream);
-    if (e != hipErrorNotSupported) return hip_result(e, fn);
-  }
-  return hip_result(dfa3d::launch_depth_score_backward(a, dtype, (hipStream_t)stream), fn);
+  return depth_score_backward("dfa3d_ms_depth_score_sample_backward", false, dist, shapes3, level_start, loc3, grad_score, grad_dist,
+                              grad_loc3, workspace, workspace_bytes, B, S, M, D, L, Q, P, dtype, opts, stream);
+}
+
+int dfa3d_ms_depth_score_sample_backward_into(const void *dist, const int64_t *shapes3, const int64_t *level_start,
+                                              const void *loc3, const void *grad_score, void *grad_dist, void *grad_loc3,
+                                              void *workspace, size_t workspace_bytes,
+                                              int B, int S, int M, int D, int L, int Q, int P, int dtype,
+                                              const dfa3d_launch_options *opts, void *stream) {
+  return depth_score_backward("dfa3d_ms_depth_score_sample_backward_into", true, dist, shapes3, level_start, loc3, grad_score,
+                              grad_dist, grad_loc3, workspace, workspace_bytes, B, S, M, D, L, Q, P, dtype, opts, stream);
 }
 
 int dfa3d_wms_deform_attn_forward(const void *value, const int64_t *shapes, int shape_stride,

@@ -454,6 +454,7 @@ __device__ __forceinline__ void clear_rows_of_wave(char *base, size_t first_row,
 struct ClearArgs {
   char *grad_value, *grad_dist;     // either may be nullptr: not that one
   int value_row_bytes, dist_row_bytes, B, S, M, L, stores;
+  int only_disjoint;                // the tile kernel stores nothing where levels share keys
 };
 __device__ __forceinline__ void clear_unstored(const BinWorkspace &ws, const ClearArgs &ca, unsigned block, unsigned n_blocks) {
   char *grad_value = ca.grad_value, *grad_dist = ca.grad_dist;
@@ -467,7 +468,7 @@ __device__ __forceinline__ void clear_unstored(const BinWorkspace &ws, const Cle
   for (size_t i0 = ((size_t)block * blockDim.x + threadIdx.x) - lane; i0 < rows; i0 += (size_t)n_blocks * blockDim.x) {
     const size_t i = i0 + lane;
     bool clear_mine = i < rows;
-    if (clear_mine && stores && nb > 0) {
+    if (clear_mine && stores && nb > 0 && !(ca.only_disjoint && p.disjoint == 0)) {
       const int m = (int)(i % M);
       const size_t bs = i / M;
       const int s = (int)(bs % S), b = (int)(bs / S);
@@ -1076,11 +1077,12 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
 // What bounds it is the random access of each point (its score gradient, its z gradient, four pairs of bins) and the
 // tile's way out, so the kernel keeps both going at once: four workgroups per CU, no barrier between the points of
 // an item (taps go to LDS by compare-and-swap, so nobody waits for anybody), the next round's records asked for one
-// round ahead and the next item's before the tile is flushed.  A pixel that only this item can touch (no neighbour's
-// halo, all the points of its bin, levels that share no keys) is read, added to and stored 16 bytes per lane; the
-// others are added atomically, one float per lane on consecutive addresses.
-// 6 x 9502 queries, 4 levels from 116 x 200, 8 points, 112 bins (14.6 M points): 1.19 -> 1.03 ms against a kernel that took
-// a ticket per tap and met at three barriers per 256 points.
+// round ahead and the next item's before the tile is flushed.  For a caller whose buffer may hold anything, a pixel that
+// only this item can touch (no neighbour's halo, all the points of its bin, levels that share no keys) is stored 16
+// bytes per lane; everything else is added atomically, one float per lane on consecutive addresses.
+// 6 x 9502 queries, 4 levels from 116 x 200, 8 points, 112 bins (14.6 M points): 1.19 ms with a ticket per tap and
+// three barriers per 256 points, 1.01 ms now; with parts cut out, the z gradients' scattered stores are 0.27 of it, the
+// tiles' way out 0.2, the taps 0.10, the score gradients' gathers 0.09.
 // ---------------------------------------------------------------------------------------
 constexpr int kDepthBlock = 256;
 // The fetching thread's state: the queue is asked for an item's number when another item is begun, the answer is looked
@@ -1109,7 +1111,8 @@ struct DepthFetch {
 template <typename T>
 __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
     BinWorkspace ws, const T *__restrict__ dist, const T *__restrict__ grad_score, float *__restrict__ grad_dist,
-    float *__restrict__ grad_loc3, int B, int S, int M, int D, int L, int Q, int P) {
+    float *__restrict__ grad_loc3, int B, int S, int M, int D, int L, int Q, int P, int stores) {
+  // stores: the binning launches cleared what is added to here and nothing else (clear_unstored), else everything is added
   extern __shared__ __align__(16) float smem[];
   __shared__ int4 s_item[2], s_geo[2];
   __shared__ int s_lv[4][DFA3D_MAX_LEVELS];              // H, W, Dd, first key
@@ -1122,7 +1125,7 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
   if (tid < DFA3D_MAX_LEVELS) {
     s_lv[0][tid] = p.H[tid]; s_lv[1][tid] = p.W[tid]; s_lv[2][tid] = p.Dd[tid]; s_lv[3][tid] = p.start[tid];
   }
-  const bool may_store = p.disjoint != 0 && (D & 3) == 0;
+  const bool may_store = stores != 0 && p.disjoint != 0;
   const int home = blockIdx.x % kClasses;
   DepthFetch fetch;
   if (tid == 0) {
@@ -1198,30 +1201,16 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
     const bool sole = chunks == 1 && may_store;
     auto lanes_log2 = [](int n) { return n > 32 ? 6 : n > 16 ? 5 : n > 8 ? 4 : n > 4 ? 3 : 2; };
     if (sole) {
-      const int n = D >> 2, sh = lanes_log2(n), inner = (TY - 1) * (TX - 1), step = kDepthBlock >> sh;
-      for (int c = tid & ((1 << sh) - 1); c < n; c += 1 << sh) {
-        for (int i0 = tid >> sh; i0 < inner; i0 += 4 * step) {      // four pixels' sums asked for together
-          uint32_t off[4];
-          int at[4];
-          u32x4 o[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int i = i0 + j * step, ry = i / (TX - 1) + 1, rx = i % (TX - 1) + 1, y = y0 + ry, x = x0 + rx;
-            const bool in = i < inner;
-            at[j] = in ? (ry * TW + rx) * D + 4 * c : -1;
-            off[j] = in && y < H && x < W ? (uint32_t)((((start + y * W + x) * M + m) * D + 4 * c) * 4) : kNoRow;
-            o[j] = __builtin_amdgcn_raw_buffer_load_b128(gdist_r, off[j], 0, 0);
-          }
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            if (at[j] < 0) continue;
-            float4 *from = reinterpret_cast<float4 *>(gd + at[j]);
-            const float4 v = *from;
-            *from = make_float4(0, 0, 0, 0);
-            const u32x4 sum = {__float_as_uint(__uint_as_float(o[j].x) + v.x), __float_as_uint(__uint_as_float(o[j].y) + v.y),
-                               __float_as_uint(__uint_as_float(o[j].z) + v.z), __float_as_uint(__uint_as_float(o[j].w) + v.w)};
-            __builtin_amdgcn_raw_buffer_store_b128(sum, gdist_r, off[j], 0, 0);
-          }
+      const int n = D >> 2, sh = lanes_log2(n), inner = (TY - 1) * (TX - 1);
+      for (int i = tid >> sh; i < inner; i += kDepthBlock >> sh) {
+        const int ry = i / (TX - 1) + 1, rx = i % (TX - 1) + 1, y = y0 + ry, x = x0 + rx;
+        const uint32_t e0 = (uint32_t)((((start + y * W + x) * M + m) * D) * 4);
+        for (int c = tid & ((1 << sh) - 1); c < n; c += 1 << sh) {
+          float4 *from = reinterpret_cast<float4 *>(gd + (ry * TW + rx) * D) + c;
+          const float4 v = *from;
+          *from = make_float4(0, 0, 0, 0);
+          const u32x4 o = {__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
+          __builtin_amdgcn_raw_buffer_store_b128(o, gdist_r, y < H && x < W ? e0 + 16 * c : kNoRow, 0, 0);
         }
       }
     }
@@ -1587,12 +1576,13 @@ static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, const Ti
   unsigned clear_blocks = 0;
   if (a.clear_grads || gd_heads != nullptr) {            // launch_backward_binned has checked that this applies
     const int ge = a.grad_bf16 ? 2 : 4;
-    ca.grad_value = a.clear_grads ? static_cast<char *>(a.grad_value) : nullptr;
+    ca.grad_value = a.clear_grads && a.C > 0 ? static_cast<char *>(a.grad_value) : nullptr;
     ca.value_row_bytes = a.C * ge;
     if (gd_heads != nullptr) { ca.grad_dist = reinterpret_cast<char *>(gd_heads); ca.dist_row_bytes = a.D * 4; }
-    else if (a.dist != nullptr) { ca.grad_dist = static_cast<char *>(a.grad_dist); ca.dist_row_bytes = a.D * ge; }
+    else if (a.dist != nullptr || a.C == 0) { ca.grad_dist = static_cast<char *>(a.grad_dist); ca.dist_row_bytes = a.D * ge; }
     ca.B = a.B; ca.S = a.S; ca.M = a.M; ca.L = a.L;
-    ca.stores = (cfg.cells || ((a.C | (a.dist != nullptr ? a.D : 0)) & 3) == 0) ? 1 : 0;        // the tile kernel's own condition
+    ca.only_disjoint = a.C == 0 ? 1 : 0;                     // stage 1 alone
+    ca.stores = (cfg.cells || ((a.C | (a.dist != nullptr || a.C == 0 ? a.D : 0)) & 3) == 0) ? 1 : 0;        // the tile kernel's own condition
     const size_t rows = (size_t)a.B * a.S * a.M;
     clear_blocks = (unsigned)((rows + 1023) / 1024 < 4096 ? (rows + 1023) / 1024 : 4096);
   }
@@ -1625,7 +1615,6 @@ hipError_t launch_backward_binned(const BwdArgs &a, int dtype, void *workspace, 
   if (need == 0 || workspace == nullptr || workspace_bytes < need || ((uintptr_t)workspace & 255) != 0)
     return hipErrorNotSupported;
   if (a.clear_grads) {
-    if (kind == 2) return hipErrorInvalidValue;            // the depth-only tile kernel stores nothing
     // clear_unstored writes 16-byte groups where a row is made of them: buffers on 16-byte boundaries,
     // or the direct kernels (which clear everything) take the call
     if ((((uintptr_t)a.grad_value | (uintptr_t)a.grad_dist) & 15) != 0) return hipErrorNotSupported;
@@ -1674,6 +1663,9 @@ hipError_t launch_depth_score_backward_binned(const DepthScoreBwdArgs &d, int dt
   a.shapes = d.shapes3; a.shape_stride = 3; a.level_start = d.level_start; a.loc = d.loc3; a.loc_stride = 3;
   a.attn = nullptr; a.grad_loc = d.grad_loc3; a.grad_loc_stride = 3; a.grad_attn = nullptr; a.grad_score_out = nullptr;
   a.tile_hint = tile_hint; a.chunk_hint = chunk_hint;
+  a.grad_dist = d.grad_dist; a.clear_grads = d.clear;
+  if (d.clear && ((uintptr_t)d.grad_dist & 15) != 0) return hipErrorNotSupported;      // as in launch_backward_binned
+  const int stores = d.clear && (d.D & 3) == 0 ? 1 : 0;
   const size_t need = workspace_bytes_for(a, 2, dtype);
   if (need == 0 || workspace == nullptr || workspace_bytes < need || ((uintptr_t)workspace & 255) != 0)
     return hipErrorNotSupported;
@@ -1690,11 +1682,11 @@ hipError_t launch_depth_score_backward_binned(const DepthScoreBwdArgs &d, int dt
   if (dtype == DFA3D_F32) {
     hipLaunchKernelGGL(tile_depth_backward_kernel<float>, dim3(grid), dim3(cfg.block), cfg.lds, stream, ws,
                        (const float *)d.dist, (const float *)d.grad_score, (float *)d.grad_dist, (float *)d.grad_loc3,
-                       d.B, d.S, d.M, d.D, d.L, d.Q, d.P);
+                       d.B, d.S, d.M, d.D, d.L, d.Q, d.P, stores);
   } else {
     hipLaunchKernelGGL(tile_depth_backward_kernel<__hip_bfloat16>, dim3(grid), dim3(cfg.block), cfg.lds, stream, ws,
                        (const __hip_bfloat16 *)d.dist, (const __hip_bfloat16 *)d.grad_score, (float *)d.grad_dist,
-                       (float *)d.grad_loc3, d.B, d.S, d.M, d.D, d.L, d.Q, d.P);
+                       (float *)d.grad_loc3, d.B, d.S, d.M, d.D, d.L, d.Q, d.P, stores);
   }
   return hipGetLastError();
 }

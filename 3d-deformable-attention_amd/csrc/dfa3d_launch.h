@@ -111,6 +111,7 @@ struct DepthScoreBwdArgs {
   const void *dist; const int64_t *shapes3, *level_start; const void *loc3, *grad_score;
   void *grad_dist, *grad_loc3;
   int B, S, M, D, L, Q, P;
+  int clear;                         // grad_dist holds anything on entry (binned kernels; the caller clears for the direct ones)
 };
 
 hipError_t launch_forward(const FwdArgs &a, int dtype, hipStream_t stream);

@@ -109,6 +109,14 @@ def ms_depth_score_sample_backward(value, value_spatial_shapes, value_level_star
                                    grad_output, grad_value, grad_sampling_loc, im2col_step):
     """Accumulates into ``grad_value`` (pre-zeroed by the caller) and overwrites ``grad_sampling_loc``
     (x and y components are zero: the scores do not depend on x, y inside a pixel cell)."""
+    ms_depth_score_sample_backward_into(value, value_spatial_shapes, value_level_start_index, sampling_locations, grad_output,
+                                        grad_value, grad_sampling_loc, im2col_step, clear=False)
+
+
+def ms_depth_score_sample_backward_into(value, value_spatial_shapes, value_level_start_index, sampling_locations,
+                                        grad_output, grad_value, grad_sampling_loc, im2col_step, clear=False):
+    """``ms_depth_score_sample_backward`` with one more choice: ``clear=True`` takes a ``grad_value`` that holds anything
+    (``torch.empty``); it then holds the gradient on return."""
     _contig(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
             sampling_loc=sampling_locations, grad_output=grad_output, grad_value=grad_value,
             grad_sampling_loc=grad_sampling_loc)
@@ -125,12 +133,15 @@ def ms_depth_score_sample_backward(value, value_spatial_shapes, value_level_star
     _expect(grad_sampling_loc, "grad_sampling_loc", shape=sampling_locations.shape, dtype=aux)
     _step(B, im2col_step)
     if grad_output.numel() == 0:
+        if clear:
+            grad_value.zero_()
         return
     code = _lib.dtype_code(value)
     ws_bytes = _lib.lib().dfa3d_ms_depth_score_sample_backward_workspace_bytes(B, S, M, D, L, Q, P, code, _lib.options())
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
     with _lib.on_device(dev):
-        rc = _lib.lib().dfa3d_ms_depth_score_sample_backward(
+        rc = (_lib.lib().dfa3d_ms_depth_score_sample_backward_into if clear else
+              _lib.lib().dfa3d_ms_depth_score_sample_backward)(
             _lib.ptr(value), _lib.ptr(value_spatial_shapes), _lib.ptr(value_level_start_index),
             _lib.ptr(sampling_locations), _lib.ptr(grad_output), _lib.ptr(grad_value), _lib.ptr(grad_sampling_loc),
             _lib.ptr(workspace), ws_bytes, B, S, M, D, L, Q, P, code, _lib.options(), _lib.stream_of(value))

@@ -33,6 +33,7 @@ _O = ctypes.POINTER(LaunchOptions)
 SIGNATURES = {
     "dfa3d_ms_depth_score_sample_forward": [_P] * 5 + _DIMS7 + [_I, _O, _P],
     "dfa3d_ms_depth_score_sample_backward": [_P] * 8 + [ctypes.c_size_t] + _DIMS7 + [_I, _O, _P],
+    "dfa3d_ms_depth_score_sample_backward_into": [_P] * 8 + [ctypes.c_size_t] + _DIMS7 + [_I, _O, _P],
     "dfa3d_wms_deform_attn_forward": [_P, _P, _I, _P, _P, _I, _P, _P, _P] + _DIMS7 + [_I, _O, _P],
     "dfa3d_wms_deform_attn_backward": [_P, _P, _I, _P, _P, _I, _P, _P, _P, _P, _P, _I, _P, _P, _P, ctypes.c_size_t]
     + _DIMS7 + [_I, _O, _P],

@@ -98,11 +98,11 @@ class MultiScaleDepthScoreSampleFunction(Function):
     @_with_forward_options
     def backward(ctx, grad_output):
         value, value_spatial_shapes, value_level_start_index, sampling_locations = ctx.saved_tensors
-        grad_value = torch.zeros(value.shape, dtype=_aux(value), device=value.device)
+        grad_value = torch.empty(value.shape, dtype=_aux(value), device=value.device)      # cleared by the call (clear=True)
         grad_sampling_loc = torch.empty_like(sampling_locations)
-        _ext.ms_depth_score_sample_backward(
+        _ext.ms_depth_score_sample_backward_into(
             value, value_spatial_shapes, value_level_start_index, sampling_locations,
-            _grad_in(grad_output, value.dtype), grad_value, grad_sampling_loc, im2col_step=ctx.im2col_step)
+            _grad_in(grad_output, value.dtype), grad_value, grad_sampling_loc, im2col_step=ctx.im2col_step, clear=True)
         return grad_value.to(value.dtype), None, None, grad_sampling_loc, None
 
 

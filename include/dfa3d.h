@@ -95,6 +95,13 @@ int dfa3d_ms_depth_score_sample_backward(
     void *grad_dist, void *grad_loc3,
     void *workspace, size_t workspace_bytes,
     int B, int S, int M, int D, int L, int Q, int P, int dtype, const dfa3d_launch_options *opts, void *stream);
+/* The same for a `grad_dist` that may hold anything on entry: the call clears what it adds to and stores the rest. */
+int dfa3d_ms_depth_score_sample_backward_into(
+    const void *dist, const int64_t *shapes3, const int64_t *level_start, const void *loc3,
+    const void *grad_score,
+    void *grad_dist, void *grad_loc3,
+    void *workspace, size_t workspace_bytes,
+    int B, int S, int M, int D, int L, int Q, int P, int dtype, const dfa3d_launch_options *opts, void *stream);
 size_t dfa3d_ms_depth_score_sample_backward_workspace_bytes(int B, int S, int M, int D, int L, int Q, int P,
                                                             int dtype, const dfa3d_launch_options *opts);
 

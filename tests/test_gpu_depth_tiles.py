@@ -39,3 +39,10 @@ def test_stage_one_backward(oracle, D, levels, Q, chunk, where, overlap, dtype):
     tol = F32_BWD if where is None else dict(rtol=1e-4, atol=2.0 ** -24 * 16 * Q * len(levels))
     torch.testing.assert_close((gd.cpu() - held).double(), want, **tol)
     torch.testing.assert_close(gl.cpu().double(), want_gl, rtol=1e-4, atol=1e-3)     # z gradient: differences of bins, times D
+    # a buffer that may hold anything
+    for direct in (0, 1):
+        fresh = torch.full(dist.shape, float("nan"), device=dev)
+        with _lib.launch_options(direct=direct, **({"chunk": chunk} if chunk else {})):
+            _ext.ms_depth_score_sample_backward_into(dist.to(dev), sh.to(dev), lsi.to(dev), loc.to(dev), go.to(dev), fresh, gl, 64,
+                                                     clear=True)
+        torch.testing.assert_close(fresh.cpu().double(), want, **tol)
