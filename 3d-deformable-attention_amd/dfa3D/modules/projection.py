@@ -15,11 +15,12 @@ __all__ = ["Projection"]
 def ordinary(*tensors):
     """Plain float32 tensors on one GPU, outside autocast, functorch transforms, forward-mode derivatives, tracing and
     compilation: what this package's kernels may stand in for torch operations on."""
-    return (all(type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.dtype == torch.float32
-                and t.device == tensors[0].device for t in tensors)
-            and not torch.is_autocast_enabled() and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+    return (not torch.compiler.is_compiling() and not torch.jit.is_tracing() and not torch.is_autocast_enabled()
+            and all(type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.dtype == torch.float32
+                    and t.device == tensors[0].device for t in tensors)
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0)
+
 
 # Fewer rows than this: the library product is as fast and there is one launch less.
 _MIN_ROWS = 4096
@@ -69,7 +70,8 @@ class _ProjectionFunction(Function):
 
 def _applies(x, weight, bias):
     """Float32 rows on the GPU in ordinary reverse-mode training."""
-    return (bias is not None and torch.is_grad_enabled() and weight.requires_grad and x.dim() >= 2
+    return (not torch.compiler.is_compiling() and bias is not None and torch.is_grad_enabled() and weight.requires_grad
+            and x.dim() >= 2
             and weight.shape[0] % 2 == 0 and weight.shape[1] % 2 == 0 and max(weight.shape) <= 16384
             and _MIN_ROWS <= x.numel() // max(x.shape[-1], 1) <= 2 ** 31 and ordinary(x, weight, bias))
 
