@@ -449,15 +449,28 @@ static int check_rebatch(const char *fn, int bs, int cams, int max_len, int Nq, 
   return 0;
 }
 
-int dfa3d_rebatch_gather(const void *src, long long cam_stride, long long batch_stride, const int32_t *index,
-                         const void *scale, void *dst, int bs, int cams, int max_len, int Nq, int E, int dtype,
-                         void *stream) {
-  const char *fn = "dfa3d_rebatch_gather";
+static int rebatch_gather(const char *fn, const void *src, long long cam_stride, long long batch_stride, const int32_t *index,
+                          const void *scale, void *dst, int bs, int cams, int max_len, int Nq, int E, int dtype, double pad,
+                          void *stream) {
   if (int rc = check_rebatch(fn, bs, cams, max_len, Nq, E, dtype)) return rc;
   if (cam_stride < 0 || batch_stride < 0) return fail(DFA3D_EINVAL, "%s: strides must not be negative", fn);
   REQUIRE_PTR(fn, src); REQUIRE_PTR(fn, index); REQUIRE_PTR(fn, dst);
   return hip_result(dfa3d::launch_rebatch_gather(src, cam_stride, batch_stride, index, scale, dst, bs, cams, max_len,
-                                                 Nq, E, dtype, (hipStream_t)stream), fn);
+                                                 Nq, E, dtype, pad, (hipStream_t)stream), fn);
+}
+
+int dfa3d_rebatch_gather(const void *src, long long cam_stride, long long batch_stride, const int32_t *index,
+                         const void *scale, void *dst, int bs, int cams, int max_len, int Nq, int E, int dtype,
+                         void *stream) {
+  return rebatch_gather("dfa3d_rebatch_gather", src, cam_stride, batch_stride, index, scale, dst, bs, cams, max_len, Nq, E, dtype,
+                        0.0, stream);
+}
+
+int dfa3d_rebatch_gather_padded(const void *src, long long cam_stride, long long batch_stride, const int32_t *index,
+                                const void *scale, void *dst, int bs, int cams, int max_len, int Nq, int E, int dtype,
+                                double pad, void *stream) {
+  return rebatch_gather("dfa3d_rebatch_gather_padded", src, cam_stride, batch_stride, index, scale, dst, bs, cams, max_len, Nq, E,
+                        dtype, pad, stream);
 }
 
 int dfa3d_rebatch_combine(const void *src, const int32_t *pos, const void *scale, void *dst, int bs, int cams,

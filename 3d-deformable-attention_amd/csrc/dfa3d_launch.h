@@ -139,7 +139,7 @@ size_t tile_timer_offset();
 // Camera re-batching (dfa3d_rebatch.hip); strides in elements.
 hipError_t launch_rebatch_gather(const void *src, long long cam_stride, long long batch_stride, const int *index,
                                  const void *scale, void *dst, int bs, int cams, int max_len, int Nq, int E,
-                                 int dtype, hipStream_t stream);
+                                 int dtype, double pad, hipStream_t stream);
 hipError_t launch_rebatch_combine(const void *src, const int *pos, const void *scale, void *dst, int bs, int cams,
                                   int max_len, int Nq, int E, int dtype, hipStream_t stream);
 

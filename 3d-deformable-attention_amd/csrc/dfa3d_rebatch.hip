@@ -8,7 +8,7 @@
 // :741-748).  Here each direction is one kernel, and neither uses atomics:
 //
 //   rebatch_gather_kernel   dst[j, i, k, :] = scale[j, q] * src[i, j, q, :]   with q = index[i, k]
-//                           (zeros where index[i, k] < 0); also the backward of the combine
+//                           (`pad`, usually zero, where index[i, k] < 0); also the backward of the combine
 //   rebatch_combine_kernel  dst[j, q, :] = scale[j, q] * sum over cameras i with pos[i, q] >= 0 of
 //                           src[j, i, pos[i, q], :]; also the backward of the gather
 //
@@ -56,7 +56,7 @@ __device__ __forceinline__ void store_pack(T *p, const Pack<T, VEC> &r) {
 template <typename T, int VEC>
 __global__ __launch_bounds__(kRebatchBlock) void rebatch_gather_kernel(
     const T *__restrict__ src, long long cam_stride, long long batch_stride, const int *__restrict__ index,
-    const T *__restrict__ scale, T *__restrict__ dst, int bs, int cams, int max_len, int Nq, int E) {
+    const T *__restrict__ scale, T *__restrict__ dst, int bs, int cams, int max_len, int Nq, int E, T pad) {
   const int per_row = E / VEC;
   const long long total = (long long)bs * cams * max_len * per_row;
   for (long long t = (long long)blockIdx.x * kRebatchBlock + threadIdx.x; t < total;
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kRebatchBlock) void rebatch_gather_kernel(
     const int q = index[(long long)i * max_len + k];
     Pack<T, VEC> r;
 #pragma unroll
-    for (int c = 0; c < VEC; ++c) r.v[c] = 0;
+    for (int c = 0; c < VEC; ++c) r.v[c] = pad;
     if (q >= 0 && q < Nq) {
       r = load_pack<T, VEC>(src + i * cam_stride + j * batch_stride + (long long)q * E + e);
       if (scale != nullptr) {
@@ -124,17 +124,17 @@ static unsigned rebatch_grid(long long threads) {
 template <typename T>
 static hipError_t gather_typed(const void *src, long long cam_stride, long long batch_stride, const int *index,
                                const void *scale, void *dst, int bs, int cams, int max_len, int Nq, int E,
-                               bool aligned, hipStream_t stream) {
+                               double pad, bool aligned, hipStream_t stream) {
   constexpr int W = 16 / (int)sizeof(T);
   const long long rows = (long long)bs * cams * max_len;
   if (aligned && E % W == 0 && cam_stride % W == 0 && batch_stride % W == 0) {
     hipLaunchKernelGGL((rebatch_gather_kernel<T, W>), dim3(rebatch_grid(rows * (E / W))), dim3(kRebatchBlock), 0, stream,
                        (const T *)src, cam_stride, batch_stride, index, (const T *)scale, (T *)dst, bs, cams, max_len,
-                       Nq, E);
+                       Nq, E, (T)pad);
   } else {
     hipLaunchKernelGGL((rebatch_gather_kernel<T, 1>), dim3(rebatch_grid(rows * E)), dim3(kRebatchBlock), 0, stream,
                        (const T *)src, cam_stride, batch_stride, index, (const T *)scale, (T *)dst, bs, cams, max_len,
-                       Nq, E);
+                       Nq, E, (T)pad);
   }
   return hipGetLastError();
 }
@@ -156,12 +156,12 @@ static hipError_t combine_typed(const void *src, const int *pos, const void *sca
 
 hipError_t launch_rebatch_gather(const void *src, long long cam_stride, long long batch_stride, const int *index,
                                  const void *scale, void *dst, int bs, int cams, int max_len, int Nq, int E,
-                                 int dtype, hipStream_t stream) {
+                                 int dtype, double pad, hipStream_t stream) {
   const bool aligned = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
   if (dtype == DFA3D_F32)
-    return gather_typed<float>(src, cam_stride, batch_stride, index, scale, dst, bs, cams, max_len, Nq, E, aligned, stream);
+    return gather_typed<float>(src, cam_stride, batch_stride, index, scale, dst, bs, cams, max_len, Nq, E, pad, aligned, stream);
   if (dtype == DFA3D_F64)
-    return gather_typed<double>(src, cam_stride, batch_stride, index, scale, dst, bs, cams, max_len, Nq, E, aligned, stream);
+    return gather_typed<double>(src, cam_stride, batch_stride, index, scale, dst, bs, cams, max_len, Nq, E, pad, aligned, stream);
   return hipErrorInvalidValue;
 }
 

@@ -42,6 +42,8 @@ SIGNATURES = {
     "dfa3d_fused_backward": [_P] * 14 + [ctypes.c_size_t] + _DIMS8 + [_I, _I, _O, _P],
     "dfa3d_fused_backward_static": [_P] * 13 + _DIMS8 + [_I, _I, _O, _P],
     "dfa3d_rebatch_gather": [_P, ctypes.c_longlong, ctypes.c_longlong, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
+    "dfa3d_rebatch_gather_padded": [_P, ctypes.c_longlong, ctypes.c_longlong, _P, _P, _P, _I, _I, _I, _I, _I, _I,
+                                    ctypes.c_double, _P],
     "dfa3d_rebatch_combine": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "dfa3d_camera_hits": [_P] * 3 + [_I] * 4 + [_P],
     "dfa3d_camera_count": [_P, _P, _I, _I, _P],

@@ -70,9 +70,9 @@ def _check(t, name, dtype=None):
         raise RuntimeError(f"{name} has dtype {t.dtype}, expected {dtype}")
 
 
-def rebatch_gather(src, index, scale=None, per_camera=False):
+def rebatch_gather(src, index, scale=None, per_camera=False, pad=0.0):
     """``src`` (bs, Nq, E), or (cams, bs, Nq, E) with ``per_camera`` -> (bs, cams, max_len, E):
-    row [j, i, k] = scale[j, q] * src[(i,) j, q] with q = index[i, k], zeros where index is -1."""
+    row [j, i, k] = scale[j, q] * src[(i,) j, q] with q = index[i, k], ``pad`` where index is -1."""
     _check(src, "src")
     _check(index, "index", torch.int32)
     cams, max_len = index.shape
@@ -94,9 +94,9 @@ def rebatch_gather(src, index, scale=None, per_camera=False):
     if dst.numel() == 0:
         return dst
     with _lib.on_device(src.device):
-        rc = _lib.lib().dfa3d_rebatch_gather(_lib.ptr(src), cam_stride, batch_stride, _lib.ptr(index), _lib.ptr(scale),
-                                             _lib.ptr(dst), bs, cams, max_len, Nq, E, _lib.dtype_code(src),
-                                             _lib.stream_of(src))
+        rc = _lib.lib().dfa3d_rebatch_gather_padded(_lib.ptr(src), cam_stride, batch_stride, _lib.ptr(index), _lib.ptr(scale),
+                                                    _lib.ptr(dst), bs, cams, max_len, Nq, E, _lib.dtype_code(src), pad,
+                                                    _lib.stream_of(src))
     _lib.check(rc, "dfa3d_rebatch_gather")
     return dst
 

@@ -62,7 +62,7 @@ typedef struct dfa3d_launch_options {
   int tile;     /* binned backward: tile edge in pixels as ty*100+tx, 0 = automatic */
   int block;    /* binned backward: threads per tile workgroup, 256 or 0/512 */
   int pass;     /* binned backward: points a tile workgroup takes per pass, 64, 128 or 256; 0 = automatic */
-  int chunk;    /* binned backward: points of one tile handled by one work item, 0 = 4096 */
+  int chunk;    /* binned backward: points of one tile handled by one work item; 0 = by the number of points, 256 to 4096 */
   int clear;    /* dfa3d_fused_backward, dfa3d_fused_backward_static and dfa3d_wms_deform_attn_backward only (0
                  * elsewhere): non-zero = grad_value (and grad_dist) may hold anything on entry, the call clears what
                  * its kernels add to instead of storing (a quarter of the buffers with the tile kernel, all of
@@ -235,6 +235,10 @@ size_t dfa3d_static_scratch_bytes(void);
 int dfa3d_rebatch_gather(const void *src, long long cam_stride, long long batch_stride, const int32_t *index,
                          const void *scale, void *dst, int bs, int cams, int max_len, int Nq, int E, int dtype,
                          void *stream);
+/* The gather with another value than zero in the padding. */
+int dfa3d_rebatch_gather_padded(const void *src, long long cam_stride, long long batch_stride, const int32_t *index,
+                                const void *scale, void *dst, int bs, int cams, int max_len, int Nq, int E, int dtype,
+                                double pad, void *stream);
 int dfa3d_rebatch_combine(const void *src, const int32_t *pos, const void *scale, void *dst, int bs, int cams,
                           int max_len, int Nq, int E, int dtype, void *stream);
 

@@ -26,3 +26,40 @@ def test_hits_scale_and_lists(cams, bs, Nq, Z, share):
     assert max_len == want_len and torch.equal(index.cpu(), want_index) and torch.equal(pos.cpu(), want_pos)
     counted = camera_hits(mask.cuda().long())             # numbers instead of truth values: as before
     assert torch.equal(counted[0], hit) and torch.equal(counted[1], scale)
+
+
+@pytest.mark.parametrize("E", [12, 7])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["fp32", "fp64"])
+def test_gather_pads_with_what_it_is_told(E, dtype):
+    from dfa3D.rebatch import rebatch_gather
+    index = torch.tensor([[0, 3, 4, -1], [2, -1, -1, -1]], dtype=torch.int32, device="cuda")
+    src = torch.randn(2, 3, 5, E, dtype=dtype, device="cuda")
+    zeros, far = rebatch_gather(src, index, per_camera=True), rebatch_gather(src, index, per_camera=True, pad=-64.0)
+    on = (index >= 0)[None, :, :, None].expand_as(zeros)
+    assert torch.equal(zeros[on], far[on]) and (zeros[~on] == 0).all() and (far[~on] == -64).all()
+
+
+def test_layer_does_not_depend_on_the_padding(monkeypatch):
+    """Results and gradients with the padded queries' samples outside the map and on its first pixels."""
+    from dfa3D.modules import SpatialCrossAttention_DFA3D, spatial_cross_attention
+    torch.manual_seed(0)
+    dev, cams, bs, Nq, E, maps = "cuda", 3, 2, 300, 64, [(9, 14), (5, 7)]
+    keys = sum(h * w for h, w in maps)
+    layer = SpatialCrossAttention_DFA3D(embed_dims=E, num_cams=cams, bev_h=15, bev_w=20, dropout=0.0, num_head=4, use_empty=True,
+                                        deformable_attention=dict(embed_dims=E, num_heads=4, num_levels=2, num_points=4)).to(dev)
+    for p in layer.parameters():
+        torch.nn.init.normal_(p, std=0.1)
+    query = torch.randn(bs, Nq, E, device=dev, requires_grad=True)
+    feats = torch.randn(cams, keys, bs, E, device=dev, requires_grad=True)
+    dist = torch.rand(cams, keys, bs, 8, device=dev).softmax(-1).requires_grad_()
+    mask = torch.rand(cams, bs, Nq, 4, device=dev) < torch.tensor([0.05, 0.3, 0.6], device=dev).view(3, 1, 1, 1)
+    args = dict(spatial_shapes=torch.tensor(maps, device=dev), level_start_index=torch.tensor([0, 126], device=dev),
+                reference_points_cam=torch.rand(cams, bs, Nq, 4, 3, device=dev), bev_mask=mask, value_dpt_dist=dist)
+    leaves = [query, feats, dist] + list(layer.parameters())
+    got = []
+    for pad in (-64.0, 0.0):
+        monkeypatch.setattr(spatial_cross_attention, "_OUTSIDE", pad)
+        out = layer(query, feats, feats, **args)
+        got.append([out.detach()] + list(torch.autograd.grad(out.square().sum(), leaves)))
+    for a, b in zip(*got):
+        torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4 * b.abs().max().item())
