@@ -12,8 +12,8 @@
 
 namespace dfa3d {
 
-// How the wavefronts share the units: `upw` units of L * P points each, a power of two so that the row slots of phase B
-// can be dealt to them evenly; `chunks` rounds of 64 points where one unit has more.
+// How the wavefronts share the units: `upw` units of L * P points each, a power of two, or three times one, so that the
+// row slots of phase B can be dealt to them evenly; `chunks` rounds of 64 points where one unit has more.
 struct FwdShape { int LP, upw, chunks; };
 __host__ __device__ inline FwdShape fwd_shape(int L, int P, int upw) {
   return FwdShape{L * P, upw, upw > 1 ? 1 : (L * P + kWave - 1) / kWave};
@@ -47,17 +47,21 @@ __device__ __forceinline__ void gather_rows(rsrc_t value_r, const Task<A> *tasks
       acc[i] += s0 + s1;
     }
   }
-  for (; t < n; t += step * UT) {
+  for (; t < n; t += step * UT) {                       // the rest: no load is issued that no slot has a row for
     Task<A> e[UT];
-#pragma unroll
-    for (int j = 0; j < UT; ++j) {
-      const int at = t + j * step + first;
-      e[j] = tasks[min(at, n - 1)];
-      if (at >= n) { e[j].off = kNoRow; e[j].w = 0; }
-    }
     A v[UT][VEC];
 #pragma unroll
-    for (int j = 0; j < UT; ++j) RowVec<T, A, VEC>::ld(value_r, e[j].off + chan_off, v[j]);
+    for (int j = 0; j < UT; ++j) {
+      e[j].off = kNoRow; e[j].w = 0;
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) v[j][i] = 0;
+      if (t + j * step < n) {                            // uniform
+        const int at = t + j * step + first;
+        e[j] = tasks[min(at, n - 1)];
+        if (at >= n) { e[j].off = kNoRow; e[j].w = 0; }
+        RowVec<T, A, VEC>::ld(value_r, e[j].off + chan_off, v[j]);
+      }
+    }
 #pragma unroll
     for (int j = 0; j < UT; ++j) {
 #pragma unroll
@@ -107,7 +111,7 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
   Task<A> *tasks = s_tasks[wave];
   // phase B: `par` units at a time, `spu` row slots each
   constexpr int RPI = kWave / LPR;
-  const int par = min(ws.upw, RPI), spu = RPI / par;
+  const int par = min(ws.upw & -ws.upw, RPI), spu = RPI / par;
   const int unit_tasks = ws.LP * 4 + kTaskPad;              // where the next unit's tasks start (upw > 1)
 
   const rsrc_t value_r = make_rsrc(value + (size_t)b * S * M * C, (size_t)S * M * C * sizeof(T));
@@ -218,7 +222,7 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
         wave_lds_handover();
 
         // ---------------- phase B: lanes over channels ----------------
-        for (int u0 = 0; u0 < ws.upw; u0 += par) {              // (one round where a unit takes several chunks)
+        for (int u0 = 0; u0 < ws.upw; u0 += par) {              // one round, or three (one where a unit takes several chunks)
           const int u = u0 + row_slot / spu;
           const int n = (ws.upw == 1 ? min(kWave, ws.LP - chunk * kWave) : ws.LP) * 4;
           gather_rows<T, A, VEC>(value_r, tasks + u * (ws.upw == 1 ? 0 : unit_tasks), row_slot % spu, spu, n, chan_off, acc);
@@ -339,6 +343,7 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   constexpr long long kFewWaves = 1024;
   int upw = 1;
   while (upw < kMaxUnitsPerWave && 2 * upw * a.L * a.P <= kWave) upw *= 2;
+  if (upw > 1 && upw < kMaxUnitsPerWave && upw / 2 * 3 * a.L * a.P <= kWave) upw = upw / 2 * 3;    // 20 points: 60 lanes, not 40
   while (upw > 1 && (long long)a.M * a.B * ((a.Q + upw - 1) / upw) < kFewWaves) upw /= 2;
   const FwdShape ws = fwd_shape(a.L, a.P, upw);
   const int q_per_iter = kWavesPerBlock * ws.upw;

@@ -14,7 +14,7 @@ LEVELS = ((9, 13), (5, 7), (3, 4), (2, 2))
 
 @pytest.mark.parametrize("L,P,C,Q", [
     (1, 1, 32, 3001), (1, 2, 16, 1500), (1, 3, 20, 1111), (1, 4, 32, 2049), (1, 4, 3, 7), (1, 5, 24, 901), (1, 8, 32, 640),
-    (2, 5, 36, 513), (2, 6, 5, 333), (3, 5, 20, 257), (2, 8, 64, 300), (3, 7, 40, 129), (4, 8, 32, 260), (4, 8, 32, 3),
+    (2, 5, 36, 513), (2, 6, 5, 333), (3, 5, 20, 257), (2, 8, 64, 300), (4, 5, 32, 700), (1, 9, 32, 900), (2, 5, 16, 1301), (1, 10, 130, 77), (3, 7, 40, 129), (4, 8, 32, 260), (4, 8, 32, 3),
     (3, 11, 12, 65), (4, 16, 28, 33), (4, 17, 100, 31), (4, 33, 32, 9), (1, 4, 260, 40), (2, 4, 1, 90), (2, 4, 66, 50)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16], ids=["fp32", "fp64", "bf16"])
 def test_units_and_row_slots(oracle, L, P, C, Q, dtype):
