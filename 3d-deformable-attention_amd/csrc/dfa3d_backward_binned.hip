@@ -429,9 +429,10 @@ __global__ __launch_bounds__(kFillThreads) void bin_fill_sorted_kernel(
 
 // What the tile kernel adds to instead of storing, cleared for a caller that did not zero grad_value / grad_dist
 // (options.clear).  The tile kernel stores the rows of the pixels that lie inside a tile (not on its first row or
-// column, which are the halo of its upper and left neighbours) when that tile's points fit one work item and the
-// rows are whole 16-byte groups; every other row of the two tensors only ever receives atomic adds, or nothing:
-// pixels on tile rims, pixels of tiles without points or with several work items, keys outside every level.
+// column, which are the halo of its upper and left neighbours) when that tile's points fit one work item, no key belongs
+// to two levels and the kernel stores rows of that length (ClearArgs::stores); every other row of the two tensors only
+// ever receives atomic adds, or nothing: pixels on tile rims, pixels of tiles without points or with several work items,
+// keys outside every level.
 // A lane decides for one (batch, key, head) row; the wavefront then clears its 64 consecutive rows together, 16 bytes
 // per lane on consecutive addresses (the heads of a key share their fate, so whole lines go out).
 __device__ __forceinline__ void clear_rows_of_wave(char *base, size_t first_row, int row_bytes, bool clear_mine, int lane) {
@@ -453,8 +454,8 @@ __device__ __forceinline__ void clear_rows_of_wave(char *base, size_t first_row,
 
 struct ClearArgs {
   char *grad_value, *grad_dist;     // either may be nullptr: not that one
-  int value_row_bytes, dist_row_bytes, B, S, M, L, stores;
-  int only_disjoint;                // the tile kernel stores nothing where levels share keys
+  int value_row_bytes, dist_row_bytes, B, S, M, L;
+  int stores;                       // the tile kernel stores what its item alone writes (else it adds everything)
 };
 __device__ __forceinline__ void clear_unstored(const BinWorkspace &ws, const ClearArgs &ca, unsigned block, unsigned n_blocks) {
   char *grad_value = ca.grad_value, *grad_dist = ca.grad_dist;
@@ -468,7 +469,7 @@ __device__ __forceinline__ void clear_unstored(const BinWorkspace &ws, const Cle
   for (size_t i0 = ((size_t)block * blockDim.x + threadIdx.x) - lane; i0 < rows; i0 += (size_t)n_blocks * blockDim.x) {
     const size_t i = i0 + lane;
     bool clear_mine = i < rows;
-    if (clear_mine && stores && nb > 0 && !(ca.only_disjoint && p.disjoint == 0)) {
+    if (clear_mine && stores && nb > 0 && p.disjoint != 0) {
       const int m = (int)(i % M);
       const size_t bs = i / M;
       const int s = (int)(bs % S), b = (int)(bs / S);
@@ -495,6 +496,9 @@ __device__ __forceinline__ void clear_unstored(const BinWorkspace &ws, const Cle
 // tens of thousands of bins), which is cheaper than one workgroup walking all bins and writing every work item from
 // one CU.  Further blocks, if any, clear the gradient rows that need it meanwhile (both kinds only read the counts);
 // the kernel is held to 64 registers so that two such workgroups fit a CU.
+// An item's last word says whether it alone writes the pixels inside its tile, which the tile kernels then store: it holds
+// all the points of its bin, and no key belongs to two levels (a level table may give one map to several levels; their
+// tiles then meet on the same rows, and all of them add).
 __global__ __launch_bounds__(1024, 8) void bin_scan_kernel(BinWorkspace ws, ClearArgs ca, int scan_blocks) {
   if ((int)blockIdx.x >= scan_blocks) {
     clear_unstored(ws, ca, blockIdx.x - scan_blocks, gridDim.x - scan_blocks);
@@ -502,6 +506,7 @@ __global__ __launch_bounds__(1024, 8) void bin_scan_kernel(BinWorkspace ws, Clea
   }
   __shared__ int s_pts[16], s_chk[16], s_bp[16], s_bc[16];
   const int n = ws.plan->total_bins, ch = chunk_of(ws, *ws.plan), per_class = ws.plan->bins_per_class;
+  const int sole = ws.plan->disjoint;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   for (int base = (int)blockIdx.x * 1024; base < n; base += scan_blocks * 1024) {
     // points and work items of the bins before this block's: every thread its share, summed over the wavefront
@@ -529,10 +534,10 @@ __global__ __launch_bounds__(1024, 8) void bin_scan_kernel(BinWorkspace ws, Clea
     if (i < n) {
       if (i % per_class == 0) ws.plan->class_start[i / per_class] = run_c;
       ws.cursor[i] = run_p;
-      if (k == 1) ws.items[run_c] = make_int4(i, run_p, c, 1);
+      if (k == 1) ws.items[run_c] = make_int4(i, run_p, c, sole);
       for (int t = 0, begin = 0; k > 1 && t < k; ++t) {
         const int end = share_begin(c, k, t + 1);
-        ws.items[run_c + t] = make_int4(i, run_p + begin, end - begin, k);
+        ws.items[run_c + t] = make_int4(i, run_p + begin, end - begin, 0);
         begin = end;
       }
       if (i == n - 1) {
@@ -558,8 +563,8 @@ __global__ __launch_bounds__(1024, 8) void bin_scan_kernel(BinWorkspace ws, Clea
 //   phase C  thread = point: per-point gradients from the four dots; the 8 grad_dist taps of a point go
 //            to the LDS tile (first taker of an address: plain update, later ones: atomics)
 // After the item's last pass the tile is flushed to memory once: stores for the inner rows of an item that
-// holds all the points of its bin, atomic adds for the rest (the chunks of one bin overlap, and so do the
-// rims of neighbouring bins).
+// writes its tile alone, atomic adds for the rest (the chunks of one bin overlap, the rims of neighbouring bins do, and
+// so do the tiles of levels that share keys).
 // ---------------------------------------------------------------------------------------
 
 
@@ -633,7 +638,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
     if (tid == 0) fetch.advance(ws, p, blockIdx.x % kClasses, &s_item);
     TILE_BARRIER();
     const int4 item = s_item;
-    const int bin = item.x, seg = item.y, n_item = item.z, chunks_here = item.w;
+    const int bin = item.x, seg = item.y, n_item = item.z;
     if (bin < 0) break;                                   // queues drained: every wave leaves
     TT_MARK(0);
     const int bm = bin / nb, local = bin - bm * nb;
@@ -983,10 +988,10 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
     char *gdist_b = FUSED ? static_cast<char *>(grad_dist) + (size_t)b * S * Mg * D * (gd16 ? 2 : 4) : nullptr;
     const rsrc_t gvalue_r = make_rsrc(gvalue_b, (size_t)S * M * C * sizeof(float));
     const rsrc_t gdist_r = make_rsrc(gdist_b, FUSED ? (size_t)S * Mg * D * sizeof(float) : 0);
-    // Rows 1..TY-1 x 1..TX-1 of the tile belong to no neighbour's halo; when this item holds all the
-    // points of its bin nobody else adds to them, so they are stored instead of added atomically
-    // (grad_value and grad_dist are zero on entry).
-    const bool sole = chunks_here == 1;
+    // Rows 1..TY-1 x 1..TX-1 of the tile belong to no neighbour's halo; when this item writes its tile alone
+    // nobody else adds to them, so they are stored instead of added atomically (grad_value and grad_dist are
+    // zero on entry).
+    const bool sole = item.w != 0;
     const bool sole_d = sole && Mg == M;                 // a gradient shared by the heads collects from all of them
     // four consecutive elements at element index `e` of a batch slice: stored, or added atomically
     auto put4 = [&](char *base, rsrc_t r, bool is16, uint32_t e, const float4 &val, bool store, bool every) {
@@ -1125,7 +1130,6 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
   if (tid < DFA3D_MAX_LEVELS) {
     s_lv[0][tid] = p.H[tid]; s_lv[1][tid] = p.W[tid]; s_lv[2][tid] = p.Dd[tid]; s_lv[3][tid] = p.start[tid];
   }
-  const bool may_store = stores != 0 && p.disjoint != 0;
   const int home = blockIdx.x % kClasses;
   DepthFetch fetch;
   if (tid == 0) {
@@ -1145,7 +1149,8 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
   if (s_item[0].x >= 0) ask_record(s_item[0].y, s_item[0].z, tid);
   for (int which = 0;; which ^= 1) {
     const int bin = __builtin_amdgcn_readfirstlane(s_item[which].x), seg = __builtin_amdgcn_readfirstlane(s_item[which].y);
-    const int n_item = __builtin_amdgcn_readfirstlane(s_item[which].z), chunks = __builtin_amdgcn_readfirstlane(s_item[which].w);
+    const int n_item = __builtin_amdgcn_readfirstlane(s_item[which].z);
+    const bool sole = stores != 0 && __builtin_amdgcn_readfirstlane(s_item[which].w) != 0;
     if (bin < 0) break;                                   // queues drained: every wave leaves
     if (tid == 0) {
       s_item[which ^ 1] = fetch.rec; s_geo[which ^ 1] = fetch.geo;
@@ -1198,7 +1203,6 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
 
     float *gdist_b = grad_dist + (size_t)b * S * M * D;
     const rsrc_t gdist_r = make_rsrc(gdist_b, (size_t)S * M * D * sizeof(float));
-    const bool sole = chunks == 1 && may_store;
     auto lanes_log2 = [](int n) { return n > 32 ? 6 : n > 16 ? 5 : n > 8 ? 4 : n > 4 ? 3 : 2; };
     if (sole) {
       const int n = D >> 2, sh = lanes_log2(n), inner = (TY - 1) * (TX - 1);
@@ -1581,7 +1585,6 @@ static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, const Ti
     if (gd_heads != nullptr) { ca.grad_dist = reinterpret_cast<char *>(gd_heads); ca.dist_row_bytes = a.D * 4; }
     else if (a.dist != nullptr || a.C == 0) { ca.grad_dist = static_cast<char *>(a.grad_dist); ca.dist_row_bytes = a.D * ge; }
     ca.B = a.B; ca.S = a.S; ca.M = a.M; ca.L = a.L;
-    ca.only_disjoint = a.C == 0 ? 1 : 0;                     // stage 1 alone
     ca.stores = (cfg.cells || ((a.C | (a.dist != nullptr || a.C == 0 ? a.D : 0)) & 3) == 0) ? 1 : 0;        // the tile kernel's own condition
     const size_t rows = (size_t)a.B * a.S * a.M;
     clear_blocks = (unsigned)((rows + 1023) / 1024 < 4096 ? (rows + 1023) / 1024 : 4096);

@@ -140,7 +140,7 @@ struct CellFetch {
   }
 };
 // a work item, decoded
-struct ItemGeom { int bin, seg, n_item, chunks, b, m, H, W, Dd, start, y0, x0; };
+struct ItemGeom { int bin, seg, n_item, sole, b, m, H, W, Dd, start, y0, x0; };      // sole: see bin_scan_kernel
 constexpr int kItemSlots = 8;      // a power of two; in use: the item before (finish, flush), this one and the next three
 __device__ __forceinline__ int slot_of_item(int it) { return it & (kItemSlots - 1); }
 // what the kernel declares as static LDS (level tables, the fetching thread's state, item records): the dynamic
@@ -151,7 +151,7 @@ size_t cell_kernel_half_cu_lds() { return 80 * 1024 - kCellStaticLds; }
 __device__ __forceinline__ ItemGeom uniform(const ItemGeom &g) {
   ItemGeom u;
   u.bin = __builtin_amdgcn_readfirstlane(g.bin); u.seg = __builtin_amdgcn_readfirstlane(g.seg);
-  u.n_item = __builtin_amdgcn_readfirstlane(g.n_item); u.chunks = __builtin_amdgcn_readfirstlane(g.chunks);
+  u.n_item = __builtin_amdgcn_readfirstlane(g.n_item); u.sole = __builtin_amdgcn_readfirstlane(g.sole);
   u.b = __builtin_amdgcn_readfirstlane(g.b); u.m = __builtin_amdgcn_readfirstlane(g.m);
   u.H = __builtin_amdgcn_readfirstlane(g.H); u.W = __builtin_amdgcn_readfirstlane(g.W);
   u.Dd = __builtin_amdgcn_readfirstlane(g.Dd); u.start = __builtin_amdgcn_readfirstlane(g.start);
@@ -338,15 +338,15 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 
   // The depth tile of the item in slot `which` goes out and is left zeroed, by `threads` threads of which this one is
   // number `first`, in the phase in which nobody adds to the tile.  A tile row (one pixel) takes 2^sh threads; no
-  // divisions.  Pixels 1..TY-1 x 1..7 belong to no neighbour's halo: when the item held all the points of its bin they are
-  // stored, the others are added.
+  // divisions.  Pixels 1..TY-1 x 1..7 belong to no neighbour's halo: when the item writes its tile alone they are stored,
+  // the others are added.
   auto flush_gd = [&](int which, int first, int threads) {
     const ItemGeom q = uniform(s_geom[which]);
     const int mg = Mg == 1 ? 0 : q.m;
     char *gdist_b = static_cast<char *>(grad_dist) + (size_t)q.b * S * Mg * D * (gd16 ? 2 : 4);
     float *gdist_f = reinterpret_cast<float *>(gdist_b);
     const rsrc_t gdist_r = make_rsrc(gdist_b, (size_t)S * Mg * D * sizeof(float));
-    const bool sole_d = q.chunks == 1 && Mg == M;       // a gradient shared by the heads collects from all of them
+    const bool sole_d = q.sole != 0 && Mg == M;       // a gradient shared by the heads collects from all of them
     const bool d4 = (D & 3) == 0;
     auto lanes_log2 = [](int n) { return n > 32 ? 6 : n > 16 ? 5 : n > 8 ? 4 : n > 4 ? 3 : 2; };
     if (sole_d) {
@@ -429,7 +429,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     };
     auto decode = [&](const int4 &item, const int4 &geo) {
       ItemGeom g;
-      g.bin = item.x; g.seg = item.y; g.n_item = item.z; g.chunks = item.w;
+      g.bin = item.x; g.seg = item.y; g.n_item = item.z; g.sole = item.w;
       g.b = geo.x & 0xFFFF; g.m = geo.x >> 16;
       const int l = geo.y;
       g.H = s_lv[0][l]; g.W = s_lv[1][l]; g.Dd = s_lv[2][l]; g.start = s_lv[3][l];
@@ -451,8 +451,8 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         *reinterpret_cast<float4 *>(row + o.ch.first[gi]) = make_float4(val[4 * gi], val[4 * gi + 1], val[4 * gi + 2], val[4 * gi + 3]);
     };
     // The sums of tile pixel (crow, ccol) of item q are complete in u.  Pixels 1..TY-1 x 1..7 belong to no neighbour's
-    // halo: when the item held all the points of its bin they are stored (grad_value is zero on entry, or the binning
-    // launches cleared what is added to), else added.  Rim pixels go to their place in LDS, to be added by put_rim.
+    // halo: when the item writes its tile alone they are stored (grad_value is zero on entry, or the binning launches
+    // cleared what is added to), else added.  Rim pixels go to their place in LDS, to be added by put_rim.
     auto put_pixel = [&](const Owner &o, const ItemGeom &q, const float (&u)[VEC], bool active) {
       const int y = q.y0 + o.crow, x = q.x0 + o.ccol;
       if (active && (o.crow == 0 || o.ccol == 0)) put_lds(o, rim + rim_index(o.crow, o.ccol, TY) * ROW, u);
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           const uint32_t at = e + o.ch.first[gi];
           const float4 f = make_float4(u[4 * gi], u[4 * gi + 1], u[4 * gi + 2], u[4 * gi + 3]);
           if (o.ch.first[gi] < C) {
-            if (q.chunks == 1) {                            // uniform
+            if (q.sole != 0) {                              // uniform
               if (gv16) *reinterpret_cast<uint2 *>(gvalue_b + (size_t)at * 2) = make_uint2(pack_bf16x2(f.x, f.y), pack_bf16x2(f.z, f.w));
               else *reinterpret_cast<float4 *>(gvalue_f + at) = f;
             } else if (gv16) {

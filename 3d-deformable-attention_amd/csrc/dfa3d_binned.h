@@ -70,7 +70,7 @@ struct BinWorkspace {      // device pointers into the caller's workspace
   int *queues;             // kClasses counters, kQueueStride ints apart; beside each, a part of the number of points counted
   int *counts;             // points per bin
   int *cursor;             // begin of each bin's segment after the scan, end after the fill
-  int4 *items;             // work items: (bin, begin of its points, number of points, work items of the bin)
+  int4 *items;             // work items: (bin, begin of its points, number of points, 1 = writes its tile alone: see bin_scan_kernel)
   int4 *geom;              // the items' bins decoded: (batch | head << 16, level, pixel row, pixel column of the tile's row 0)
   uint32_t *entries;       // point indices grouped by bin
   float4 *recs;            // (x, y, z, attention weight) of the same points, same order
