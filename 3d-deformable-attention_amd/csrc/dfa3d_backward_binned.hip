@@ -119,7 +119,7 @@ __device__ __forceinline__ void decode_items(const BinWorkspace &ws, int B, int 
     slot_decode(bm, B, M, b, m);
     while (l + 1 < L && local >= p.level_base[l + 1]) ++l;
     const int tile = local - p.level_base[l];
-    ws.geom[w] = make_int4(b | (m << 16), l, (tile / p.tiles_x[l]) * p.ty - 1, (tile % p.tiles_x[l]) * p.tx - 1);
+    ws.geom[w] = make_int4(b, head_level(m, l), (tile / p.tiles_x[l]) * p.ty - 1, (tile % p.tiles_x[l]) * p.tx - 1);
   }
 }
 
@@ -1156,9 +1156,9 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
       s_item[which ^ 1] = fetch.rec; s_geo[which ^ 1] = fetch.geo;
       fetch.ask(ws, home);
     }
-    const int bm = __builtin_amdgcn_readfirstlane(s_geo[which].x), l = __builtin_amdgcn_readfirstlane(s_geo[which].y);
+    const int b = __builtin_amdgcn_readfirstlane(s_geo[which].x), ml = __builtin_amdgcn_readfirstlane(s_geo[which].y);
     const int y0 = __builtin_amdgcn_readfirstlane(s_geo[which].z), x0 = __builtin_amdgcn_readfirstlane(s_geo[which].w);
-    const int b = bm & 0xFFFF, m = bm >> 16;
+    const int m = head_of(ml), l = level_of(ml);
     const int H = __builtin_amdgcn_readfirstlane(s_lv[0][l]), W = __builtin_amdgcn_readfirstlane(s_lv[1][l]);
     const int Dd = __builtin_amdgcn_readfirstlane(s_lv[2][l]), start = __builtin_amdgcn_readfirstlane(s_lv[3][l]);
     const rsrc_t dist_r = make_rsrc(dist + (size_t)b * S * M * D, (size_t)S * M * D * sizeof(T));
@@ -1424,6 +1424,7 @@ static size_t workspace_bytes_for(const BwdArgs &a, int kind, int dtype) {
   if (a.grad_bf16 && (kind != 0 || ((a.C | a.D) & 3) != 0)) return 0;          // bfloat16 gradients: whole 8-byte groups
   const TileConfig c = tile_config_of(a, kind, dtype);
   if (c.lds > 150 * 1024) return 0;                                            // rows too long for LDS tiles
+  if ((size_t)max_bins_per_bm(a.S, a.L, c.ty, c.tx) * slot_count(1, a.M) * a.B >= (1ull << 31)) return 0;      // so are bin numbers
   return bin_layout(a, c.ty, c.tx).total;
 }
 

@@ -430,8 +430,8 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     auto decode = [&](const int4 &item, const int4 &geo) {
       ItemGeom g;
       g.bin = item.x; g.seg = item.y; g.n_item = item.z; g.sole = item.w;
-      g.b = geo.x & 0xFFFF; g.m = geo.x >> 16;
-      const int l = geo.y;
+      g.b = geo.x; g.m = head_of(geo.y);
+      const int l = level_of(geo.y);
       g.H = s_lv[0][l]; g.W = s_lv[1][l]; g.Dd = s_lv[2][l]; g.start = s_lv[3][l];
       g.y0 = geo.z; g.x0 = geo.w;                            // pixel of the tile's row 0
       return g;

@@ -71,10 +71,16 @@ struct BinWorkspace {      // device pointers into the caller's workspace
   int *counts;             // points per bin
   int *cursor;             // begin of each bin's segment after the scan, end after the fill
   int4 *items;             // work items: (bin, begin of its points, number of points, 1 = writes its tile alone: see bin_scan_kernel)
-  int4 *geom;              // the items' bins decoded: (batch | head << 16, level, pixel row, pixel column of the tile's row 0)
+  int4 *geom;              // the items' bins decoded: (batch, head_level(), pixel row, pixel column of the tile's row 0)
   uint32_t *entries;       // point indices grouped by bin
   float4 *recs;            // (x, y, z, attention weight) of the same points, same order
 };
+
+// Head and level of an item in one word (a batch element's slice below 2^30 bytes leaves room for them); the batch has one
+// of its own.
+__device__ __forceinline__ int head_level(int m, int l) { return m * DFA3D_MAX_LEVELS + l; }
+__device__ __forceinline__ int head_of(int word) { return word / DFA3D_MAX_LEVELS; }
+__device__ __forceinline__ int level_of(int word) { return word % DFA3D_MAX_LEVELS; }
 
 // Inclusive prefix sum over the 64 lanes with DPP moves: shifts by 1, 2, 4, 8 inside rows of 16 lanes, then
 // lane 15 of a row to the next row, then lane 31 to the upper half.

@@ -257,3 +257,13 @@ def test_launch_options_follow_a_function_into_its_backward():
         cls = getattr(functional, name)
         base = cls.__mro__[1] if name.endswith(("_fp16", "_fp32")) else cls
         assert hasattr(base.backward.__wrapped__, "__wrapped__"), name     # once_differentiable(_with_forward_options(backward))
+
+
+def test_tile_backward_is_not_offered_beyond_its_index_range():
+    """Bin numbers are 32-bit and padded to eight heads: a batch that would need more takes the direct kernels."""
+    from dfa3D import _lib
+    L = _lib.lib()
+    dims = lambda B, M: (B, 4, M, 4, 4, 1, 1, 1, M, _lib.DFA3D_F32, None)
+    assert L.dfa3d_fused_backward_workspace_bytes(*dims(65539, 2)) > 0
+    assert L.dfa3d_fused_backward_workspace_bytes(*dims(200_000_000, 1)) == 0
+    assert L.dfa3d_fused_backward_workspace_bytes(*dims(1, 16_000_000)) > 0      # all heads that a slice of 2^30 bytes holds
