@@ -82,7 +82,7 @@ __global__ __launch_bounds__(256) void plan_and_clear_kernel(
         p.level_base[i] = base;
         base += s_tiles[i];
       }
-      // the host sized the counters from an upper bound of the tile count; never exceed it
+      // the host sized the counters for levels that share no keys: no bins (backward_without_bins) for more tiles than that
       if (base > max_bins_per_bm) base = 0;
       p.bins_per_bm = base;
       p.total_bins = base * slot_count(B, M);
@@ -136,6 +136,14 @@ constexpr size_t kSortedFillLds = (size_t)kStage * (16 + 4 + 4) + (size_t)(3 * k
 // this block's part of the total that chunk_of() reads
 __device__ __forceinline__ int *counted_points(const BinWorkspace &ws) { return &ws.queues[(blockIdx.x % kClasses) * kQueueStride + 1]; }
 
+// a fill launch's share of the records when there are no bins
+__device__ __forceinline__ void fill_in_point_order(const BinWorkspace &ws, const float *loc, int loc_stride, const float *attn, size_t n) {
+  for (size_t gp = (size_t)blockIdx.x * blockDim.x + threadIdx.x; gp < n; gp += (size_t)gridDim.x * blockDim.x) {
+    const float *at = loc + gp * loc_stride;
+    ws.recs[gp] = make_float4(at[0], at[1], loc_stride > 2 ? at[2] : 0.f, attn != nullptr ? attn[gp] : 0.f);
+  }
+}
+
 // MODE 0: count.  MODE 1: fill (needs the scanned cursor).
 template <int MODE>
 __global__ __launch_bounds__(256) void bin_points_kernel(
@@ -145,8 +153,11 @@ __global__ __launch_bounds__(256) void bin_points_kernel(
   extern __shared__ int s_hist[];          // [0, nb): counts, then for MODE 1 [nb, 2 nb): segment bases
   const BinPlan &p = *ws.plan;
   const int nb = p.bins_per_bm;
-  if (nb == 0) return;
   if (sorted_fill_applies(nb, L * P)) return;                   // bin_count_kernel / bin_fill_sorted_kernel do it
+  if (nb == 0) {
+    if (MODE == 1) fill_in_point_order(ws, loc, loc_stride, attn, (size_t)B * Q * M * L * P);
+    return;
+  }
   const bool use_lds = nb <= hist_cap;
   if (MODE == 1) decode_items(ws, B, M, L, blockIdx.x, gridDim.x);
   // The launch is a few thousand workgroups that walk the n_blocks blocks of work (so that it costs next to nothing
@@ -327,7 +338,11 @@ __global__ __launch_bounds__(kFillThreads) void bin_fill_sorted_kernel(
   const BinPlan &p = *ws.plan;
   const int nb = p.bins_per_bm;
   const int LP = L * P;
-  if (nb == 0 || !sorted_fill_applies(nb, LP)) return;
+  if (!sorted_fill_applies(nb, LP)) return;
+  if (nb == 0) {
+    fill_in_point_order(ws, loc, loc_stride, attn, (size_t)B * Q * M * LP);
+    return;
+  }
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int m = blockIdx.x % M, rest = blockIdx.x / M;          // head = block % M, as in bin_points_kernel
   const int qb = rest % q_blocks, b = rest / q_blocks;
@@ -608,7 +623,11 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
 
   const BinPlan &p = *ws.plan;
   const int nb = p.bins_per_bm;
-  if (nb == 0) return;
+  if (nb == 0) {
+    backward_without_bins<T, FUSED>(ws, value, dist, score_in, grad_out, grad_score_in, grad_value, grad_dist, grad_loc, gl_stride,
+                                    grad_attn, grad_score_out, grad_wu, Md, Mg, B, S, M, C, D, L, Q, P, grad16);
+    return;
+  }
   const int TY = p.ty, TX = p.tx, TW = TX + 1, R = (TY + 1) * TW;
   const TileLds lay = tile_lds_layout(TY, TX, C, D, PP);
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
@@ -1122,7 +1141,11 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
   __shared__ int4 s_item[2], s_geo[2];
   __shared__ int s_lv[4][DFA3D_MAX_LEVELS];              // H, W, Dd, first key
   const BinPlan &p = *ws.plan;
-  if (p.bins_per_bm == 0) return;
+  if (p.bins_per_bm == 0) {
+    backward_without_bins<T, true>(ws, nullptr, dist, nullptr, nullptr, grad_score, nullptr, grad_dist, grad_loc3, 3, nullptr,
+                                   nullptr, nullptr, M, M, B, S, M, 0, D, L, Q, P, 0);
+    return;
+  }
   const int TY = p.ty, TX = p.tx, TW = TX + 1, R = (TY + 1) * TW;
   const int tid = threadIdx.x;
   float *gd = smem;

@@ -17,7 +17,7 @@ constexpr int kHistCap = 8192;      // bins of one (batch, head) that fit the LD
 struct BinPlan {
   int H[DFA3D_MAX_LEVELS], W[DFA3D_MAX_LEVELS], Dd[DFA3D_MAX_LEVELS], start[DFA3D_MAX_LEVELS];
   int tiles_x[DFA3D_MAX_LEVELS], level_base[DFA3D_MAX_LEVELS];
-  int bins_per_bm;     // tiles over all levels of one (batch, head)
+  int bins_per_bm;     // tiles over all levels of one (batch, head); 0: see backward_without_bins
   int total_bins;      // slots * bins_per_bm
   int bins_per_class;  // total_bins / kClasses
   int class_start[kClasses + 1];   // first work item of each head class (written by the scan)
@@ -73,7 +73,7 @@ struct BinWorkspace {      // device pointers into the caller's workspace
   int4 *items;             // work items: (bin, begin of its points, number of points, 1 = writes its tile alone: see bin_scan_kernel)
   int4 *geom;              // the items' bins decoded: (batch, head_level(), pixel row, pixel column of the tile's row 0)
   uint32_t *entries;       // point indices grouped by bin
-  float4 *recs;            // (x, y, z, attention weight) of the same points, same order
+  float4 *recs;            // (x, y, z, attention weight) of the same points, same order; without bins: in point order
 };
 
 // Head and level of an item in one word (a batch element's slice below 2^30 bytes leaves room for them); the batch has one
@@ -260,6 +260,76 @@ __device__ __forceinline__ void rim_decode(int i, int ty, int tx, int &row, int 
   const int s = i - 2 * (tx + 1);
   row = s >= 0 ? 1 + (s >> 1) : i <= tx ? 0 : ty;
   col = s >= 0 ? ((s & 1) ? tx : 0) : i <= tx ? i : i - (tx + 1);
+}
+
+// What the tile kernels do when the plan has no bins: no level of the table is usable (every point is then skipped), or the
+// levels have more tiles than the host sized the counters for, which takes many levels that share keys.  Every thread takes
+// points of its own and adds to device memory; rare enough that only being right counts.  value == nullptr: stage 1 alone
+// (grad_score_in is the scores' gradient); !FUSED: stage 2 alone.
+template <typename T, bool FUSED>
+__device__ __forceinline__ void backward_without_bins(
+    const BinWorkspace &ws, const T *value, const T *dist, const T *score_in, const T *grad_out, const T *grad_score_in,
+    void *grad_value, void *grad_dist, float *grad_loc, int gl_stride, float *grad_attn, float *grad_score_out,
+    const float *grad_wu, int Md, int Mg, int B, int S, int M, int C, int D, int L, int Q, int P, int grad16) {
+  const BinPlan &p = *ws.plan;
+  const uint32_t LP = (uint32_t)L * P, n = (uint32_t)B * Q * M * LP;             // below 2^31
+  auto add = [](void *base, bool is16, size_t e, float x) {      // a bfloat16 element: in its pair, the other one gets zero
+    if (is16) atomic_add_bf16x2(static_cast<char *>(base) + (e & ~(size_t)1) * 2, (e & 1) ? 0.f : x, (e & 1) ? x : 0.f);
+    else atomicAdd(static_cast<float *>(base) + e, x);
+  };
+  for (uint32_t gp = blockIdx.x * blockDim.x + threadIdx.x; gp < n; gp += gridDim.x * blockDim.x) {
+    const float4 rec = ws.recs[gp];
+    const uint32_t unit = gp / LP;
+    const int l = (int)((gp - unit * LP) / P), m = (int)(unit % M), b = (int)(unit / M / Q), md = Md == 1 ? 0 : m, mg = Mg == 1 ? 0 : m;
+    const Point2D<float> g = locate_2d<float>(rec.x, rec.y, p.H[l], p.W[l], p.start[l]);
+    const DepthTap<float> tap = locate_depth<float>(rec.z, p.Dd[l]);
+    const float a = g.inside ? rec.w : 0.f;
+    float sc[4], lo[4] = {0, 0, 0, 0}, hi[4] = {0, 0, 0, 0}, s[4], gs[4], ga = 0;
+    if (FUSED) {
+      corner_scores<T, float>(make_rsrc(dist + (size_t)b * S * Md * D, (size_t)S * Md * D * sizeof(T)), g.key, tap, md, Md, D, sc, lo, hi);
+    } else {
+      for (int k = 0; k < 4; ++k) sc[k] = score_in != nullptr ? Elem<T>::ld(score_in + (size_t)gp * 4 + k) : 1.f;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool on = g.key[k] >= 0;
+      const float bk = g.bil(k), w = bk * sc[k] * a;
+      float dot = 0;
+      if (on && value != nullptr) {
+        const size_t row = (((size_t)b * S + g.key[k]) * M + m) * C;
+        for (int c = 0; c < C; ++c) {
+          const float go = Elem<T>::ld(grad_out + (size_t)unit * C + c);
+          dot += Elem<T>::ld(value + row + c) * go;
+          if (w != 0) add(grad_value, (grad16 & 1) != 0, row + c, w * go);
+        }
+      }
+      s[k] = on ? sc[k] * dot : 0.f;
+      gs[k] = on ? bk * a * dot : 0.f;
+      ga += bk * s[k];
+    }
+    float *gl = grad_loc + (size_t)gp * gl_stride;
+    gl[0] = (float)p.W[l] * a * (g.hh * (s[1] - s[0]) + g.lh * (s[2] - s[3]));
+    gl[1] = (float)p.H[l] * a * (g.hw * (s[3] - s[0]) + g.lw * (s[2] - s[1]));
+    if (FUSED) {
+      const float gw = grad_wu != nullptr ? grad_wu[unit] * 0.25f : 0.f;
+      float gz = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (g.key[k] < 0) continue;
+        ga += gw * sc[k];
+        gs[k] += gw * a + (grad_score_in != nullptr ? Elem<T>::ld(grad_score_in + (size_t)gp * 4 + k) : 0.f);
+        if (!tap.inside) continue;
+        const size_t row = (((size_t)b * S + g.key[k]) * Mg + mg) * D + tap.d0;
+        if (tap.lo_ok) add(grad_dist, (grad16 & 2) != 0, row, tap.hd * gs[k]);
+        if (tap.hi_ok) add(grad_dist, (grad16 & 2) != 0, row + 1, tap.ld * gs[k]);
+        gz += gs[k] * (hi[k] - lo[k]);
+      }
+      gl[2] = gz * (float)p.Dd[l];
+    } else if (grad_score_out != nullptr) {
+      for (int k = 0; k < 4; ++k) grad_score_out[(size_t)gp * 4 + k] = gs[k];
+    }
+    if (grad_attn != nullptr) grad_attn[gp] = ga;
+  }
 }
 
 // The cell-owned tile kernel (dfa3d_backward_cells.hip): rows of up to 64 channels, tiles 8 pixels wide.
