@@ -46,9 +46,11 @@ def _camera_index_on_gpu(hit):
 
 def camera_hits(bev_mask):
     """``bev_mask`` (cams, bs, Nq, Z): ``hit`` (cams, Nq) bool, the queries of the first batch element with any anchor in a
-    camera, and ``scale`` (bs, Nq) float32, one over the number of cameras with any anchor of a query (at least 1)."""
+    camera, and ``scale`` (bs, Nq) of the default dtype, one over the number of cameras with any anchor of a query (at
+    least 1)."""
     cams, bs, Nq, Z = bev_mask.shape
-    if bev_mask.is_cuda and bev_mask.dtype == torch.bool and bev_mask.numel() and cams <= 65535 and Nq <= 2 ** 30:
+    if (bev_mask.is_cuda and bev_mask.dtype == torch.bool and bev_mask.numel() and cams <= 65535 and Nq <= 2 ** 30
+            and torch.get_default_dtype() == torch.float32):           # what the kernel writes
         mask = bev_mask.contiguous()
         hit = torch.empty(cams, Nq, dtype=torch.bool, device=mask.device)
         scale = torch.empty(bs, Nq, dtype=torch.float32, device=mask.device)

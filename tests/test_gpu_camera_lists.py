@@ -63,3 +63,18 @@ def test_layer_does_not_depend_on_the_padding(monkeypatch):
         got.append([out.detach()] + list(torch.autograd.grad(out.square().sum(), leaves)))
     for a, b in zip(*got):
         torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4 * b.abs().max().item())
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.bfloat16], ids=["fp64", "fp32", "bf16"])
+def test_scale_has_the_default_dtype(dtype):
+    """A program in double precision averages with 1/3 in double precision."""
+    from dfa3D.rebatch import camera_hits
+    mask = torch.rand(5, 1, 700, 4, generator=torch.Generator().manual_seed(1)) < 0.3
+    held = torch.get_default_dtype()
+    torch.set_default_dtype(dtype)
+    try:
+        hit, scale = camera_hits(mask.cuda())
+        want_hit, want_scale = camera_hits(mask)
+    finally:
+        torch.set_default_dtype(held)
+    assert scale.dtype == dtype and torch.equal(hit.cpu(), want_hit) and torch.equal(scale.cpu(), want_scale)
