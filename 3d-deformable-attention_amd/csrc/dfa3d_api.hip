@@ -427,7 +427,7 @@ int dfa3d_fused_backward_static(const void *value, const void *dist, const int64
                                     grad_weight_update, grad_value, grad_dist, grad_loc3, grad_attn, B, S, M, C,
                                     D, L, Q, P, dist_heads, o);
   a.grad_bf16 = g16;
-  const size_t need = o.direct ? 0 : dfa3d::binned_backward_workspace_bytes(a, 0, dtype);
+  const size_t need = o.direct ? 0 : dfa3d::binned_backward_least_workspace_bytes(a, 0, dtype);
   if (need > DFA3D_STATIC_SCRATCH_BYTES)
     return fail(DFA3D_ERANGE, "%s: these dimensions need %zu bytes of scratch, the static buffer holds %zu; use "
                 "dfa3d_fused_backward with a workspace", fn, need, (size_t)DFA3D_STATIC_SCRATCH_BYTES);

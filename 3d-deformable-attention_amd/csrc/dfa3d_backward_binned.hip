@@ -1330,8 +1330,18 @@ __global__ __launch_bounds__(256) void head_sum_kernel(const float *__restrict__
     }
   }
 }
-struct BinLayout { size_t plan, queues, counts, cursor, items, geom, entries, recs, gd_heads, total; };
-static BinLayout bin_layout(const BwdArgs &a, int ty, int tx) {
+// bfloat16 gradients from float sums: everything rounded once, after the tile kernel
+__global__ __launch_bounds__(256) void round_rows_kernel(const float4 *__restrict__ value_sums, uint2 *__restrict__ grad_value, size_t nv4,
+                                                         const float4 *__restrict__ dist_sums, uint2 *__restrict__ grad_dist, size_t nd4) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < nv4 + nd4; i += (size_t)gridDim.x * 256) {
+    const float4 f = i < nv4 ? value_sums[i] : dist_sums[i - nv4];
+    *(i < nv4 ? grad_value + i : grad_dist + (i - nv4)) = make_uint2(pack_bf16x2(f.x, f.y), pack_bf16x2(f.z, f.w));
+  }
+}
+
+// gd_heads: grad_dist per head (shared_dist); value_sums, dist_sums: see sums_in_float; without them the workspace ends at `least`
+struct BinLayout { size_t plan, queues, counts, cursor, items, geom, entries, recs, gd_heads, value_sums, dist_sums, least, total; };
+static BinLayout bin_layout(const BwdArgs &a, int ty, int tx, bool float_sums) {
   BinLayout o;
   const size_t nbins = (size_t)max_bins_per_bm(a.S, a.L, ty, tx) * slot_count(a.B, a.M);
   const size_t npts = (size_t)a.B * a.Q * a.M * a.L * a.P;
@@ -1349,7 +1359,12 @@ static BinLayout bin_layout(const BwdArgs &a, int ty, int tx) {
   // summed over the heads afterwards; eight XCDs adding atomically into one shared tile cost twice as much
   o.gd_heads = up(o.recs + npts * sizeof(float4));
   const size_t per_head = shared_dist(a) ? (size_t)a.B * a.S * a.M * a.D * sizeof(float) : 0;
-  o.total = up(o.gd_heads + per_head);
+  o.least = o.total = up(o.gd_heads + per_head);
+  o.value_sums = o.dist_sums = o.total;
+  if (float_sums) {
+    o.dist_sums = up(o.value_sums + (size_t)a.B * a.S * a.M * a.C * sizeof(float));
+    o.total = up(o.dist_sums + (shared_dist(a) ? 0 : (size_t)a.B * a.S * a.M * a.D * sizeof(float)));
+  }
   return o;
 }
 
@@ -1440,7 +1455,23 @@ static TileConfig tile_config_of(const BwdArgs &a, int kind, int dtype) {
   return pick_tile_config(kind, a.C, a.D, dtype == DFA3D_F32 ? 4 : 2, a.tile_hint, a.block_hint, a.pass_hint, per_pixel >= 16.0, cells);
 }
 
-static size_t workspace_bytes_for(const BwdArgs &a, int kind, int dtype) {
+// Whether bfloat16 gradients are summed in float in the workspace and rounded once at the end.  A bfloat16 buffer rounds at
+// every add to a pixel that several tiles share, so the share of such pixels decides the error, and the cell-owned kernel's
+// tiles are smaller than what LDS allows where its walkers own fewer rows (over 32 channels: 4 x 8 pixels, 34 % of them on
+// the rim) or where rows and bins are short (8 x 8: 23 %; 8 x 16: 18 %).  There the sums are formed in float.  2 x 20000
+// queries, 8 heads, 60 x 100 map, relative error of grad_value against float: 64 channels, 16 bins 1.97e-3 with 4 x 8
+// tiles and bfloat16 adds, 1.86e-3 with the row-owned kernel's 8 x 8, 1.66e-3 this way (a single rounding); backward
+// 231 / 354 / 248 us.  16 channels, 16 bins: 1.87e-3, 1.82e-3, 1.66e-3; 134 / 242 / 137 us.
+// Rows of 32 channels stay on 8 x 8 tiles and bfloat16 adds: what LDS allows (from 40 bins on), or the models' own error.
+static bool sums_in_float(const BwdArgs &a, int kind, int dtype, const TileConfig &c) {
+  if (!a.grad_bf16 || kind != 0 || !c.cells || a.tile_hint != 0 || a.C == 32) return false;
+  BwdArgs rows = a;
+  rows.vec_hint = 1;                                                           // asks for the row-owned kernel's tile
+  const TileConfig r = tile_config_of(rows, kind, dtype);
+  return r.ty * r.tx >= 2 * c.ty * c.tx;
+}
+
+static size_t workspace_bytes_for(const BwdArgs &a, int kind, int dtype, bool least = false) {
   if (dtype == DFA3D_F64) return 0;
   if ((size_t)a.B * a.Q * a.M * a.L * a.P >= (1ull << 31)) return 0;          // point indices and segment offsets are 32-bit
   if (kind != 2 && (size_t)a.Q * a.M * a.C * 4 >= (size_t)kMaxSliceBytes) return 0;   // grad_out rows are buffer-addressed per batch element
@@ -1448,11 +1479,13 @@ static size_t workspace_bytes_for(const BwdArgs &a, int kind, int dtype) {
   const TileConfig c = tile_config_of(a, kind, dtype);
   if (c.lds > 150 * 1024) return 0;                                            // rows too long for LDS tiles
   if ((size_t)max_bins_per_bm(a.S, a.L, c.ty, c.tx) * slot_count(1, a.M) * a.B >= (1ull << 31)) return 0;      // so are bin numbers
-  return bin_layout(a, c.ty, c.tx).total;
+  const BinLayout lay = bin_layout(a, c.ty, c.tx, sums_in_float(a, kind, dtype, c));
+  return least ? lay.least : lay.total;
 }
 
 // kind as in tile_lds_bytes; `a.dist != nullptr` is not consulted here, so dimension-only queries work
 size_t binned_backward_workspace_bytes(const BwdArgs &a, int kind, int dtype) { return workspace_bytes_for(a, kind, dtype); }
+size_t binned_backward_least_workspace_bytes(const BwdArgs &a, int kind, int dtype) { return workspace_bytes_for(a, kind, dtype, true); }
 
 // Per-device facts and per-kernel attributes are looked up once and remembered (a launch then costs no
 // runtime queries).
@@ -1633,22 +1666,31 @@ static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, const Ti
 // Binned backward of both stages (a.dist given) or of stage 2 alone (a.dist == nullptr, a.score_in /
 // a.grad_score_out given).  Returns hipErrorNotSupported when the binned path does not apply and the
 // caller should use launch_backward instead.
-hipError_t launch_backward_binned(const BwdArgs &a, int dtype, void *workspace, size_t workspace_bytes,
+hipError_t launch_backward_binned(const BwdArgs &args, int dtype, void *workspace, size_t workspace_bytes,
                                   hipStream_t stream) {
+  BwdArgs a = args;
   const int kind = bwd_kind(a);
   if (dtype == DFA3D_F64) return hipErrorNotSupported;
   if (kind == 0 && (a.loc_stride != 3 || a.grad_loc_stride != 3 || a.shape_stride != 3)) return hipErrorNotSupported;
-  const size_t need = workspace_bytes_for(a, kind, dtype);
+  const size_t need = workspace_bytes_for(a, kind, dtype, true);
   if (need == 0 || workspace == nullptr || workspace_bytes < need || ((uintptr_t)workspace & 255) != 0)
     return hipErrorNotSupported;
+  if (a.grad_bf16 && dtype != DFA3D_BF16) return hipErrorInvalidValue;
   if (a.clear_grads) {
     // clear_unstored writes 16-byte groups where a row is made of them: buffers on 16-byte boundaries,
     // or the direct kernels (which clear everything) take the call
     if ((((uintptr_t)a.grad_value | (uintptr_t)a.grad_dist) & 15) != 0) return hipErrorNotSupported;
   }
   const TileConfig cfg = tile_config_of(a, kind, dtype);
-  const BinLayout lay = bin_layout(a, cfg.ty, cfg.tx);
+  BinLayout lay = bin_layout(a, cfg.ty, cfg.tx, sums_in_float(a, kind, dtype, cfg));
+  if (lay.total > workspace_bytes) lay = bin_layout(a, cfg.ty, cfg.tx, false);      // no room for them
   const BinWorkspace ws = carve_workspace(workspace, lay);
+  const bool float_sums = lay.total > lay.least;
+  if (float_sums) {            // the kernels below see float gradients, which hold anything on entry
+    a.grad_bf16 = 0; a.clear_grads = 1;
+    a.grad_value = static_cast<char *>(workspace) + lay.value_sums;
+    if (!shared_dist(a)) a.grad_dist = static_cast<char *>(workspace) + lay.dist_sums;
+  }
   float *gd_heads = shared_dist(a) ? reinterpret_cast<float *>(static_cast<char *>(workspace) + lay.gd_heads) : nullptr;
 #ifdef DFA3D_EXPERIMENT
   const int stage = a.stage;                     // development builds: 1 = binning launches only, 2 = tile kernel only
@@ -1665,12 +1707,17 @@ hipError_t launch_backward_binned(const BwdArgs &a, int dtype, void *workspace, 
   if (gd_heads != nullptr && stage == 2)
     hipLaunchKernelGGL(fill_zero_kernel, dim3(2048), dim3(256), 0, stream, reinterpret_cast<float4 *>(gd_heads),
                        ((size_t)a.B * a.S * a.M * a.D + 3) / 4);
-  if (a.grad_bf16 && dtype != DFA3D_BF16) return hipErrorInvalidValue;
   const hipError_t e = dtype == DFA3D_F32 ? launch_tile_typed<float>(a, ws, cfg, gd_heads, stream)
                                           : launch_tile_typed<__hip_bfloat16>(a, ws, cfg, gd_heads, stream);
-  if (e != hipSuccess || gd_heads == nullptr) return e;
-  hipLaunchKernelGGL(head_sum_kernel, dim3(2048), dim3(256), 0, stream, gd_heads, a.grad_dist,
-                     (size_t)a.B * a.S, a.M, a.D, a.grad_bf16 ? 1 : 0);
+  if (e != hipSuccess) return e;
+  if (gd_heads != nullptr)
+    hipLaunchKernelGGL(head_sum_kernel, dim3(2048), dim3(256), 0, stream, gd_heads, args.grad_dist,
+                       (size_t)a.B * a.S, a.M, a.D, args.grad_bf16 ? 1 : 0);
+  if (float_sums) {
+    const size_t rows = (size_t)a.B * a.S * a.M;
+    hipLaunchKernelGGL(round_rows_kernel, dim3(2048), dim3(256), 0, stream, (const float4 *)a.grad_value, (uint2 *)args.grad_value,
+                       rows * a.C / 4, (const float4 *)a.grad_dist, (uint2 *)args.grad_dist, gd_heads != nullptr ? 0 : rows * a.D / 4);
+  }
   return hipGetLastError();
 }
 
@@ -1697,7 +1744,7 @@ hipError_t launch_depth_score_backward_binned(const DepthScoreBwdArgs &d, int dt
   if (need == 0 || workspace == nullptr || workspace_bytes < need || ((uintptr_t)workspace & 255) != 0)
     return hipErrorNotSupported;
   const TileConfig cfg = tile_config_of(a, 2, dtype);
-  const BinWorkspace ws = carve_workspace(workspace, bin_layout(a, cfg.ty, cfg.tx));
+  const BinWorkspace ws = carve_workspace(workspace, bin_layout(a, cfg.ty, cfg.tx, false));
   if (hipError_t e = run_binning(a, ws, cfg, nullptr, stream)) return e;
   if (event_binned != nullptr) {
     if (hipError_t e = hipEventRecord((hipEvent_t)event_binned, stream)) return e;

@@ -123,6 +123,8 @@ hipError_t launch_depth_score_backward(const DepthScoreBwdArgs &a, int dtype, hi
 // Binned (LDS-accumulating) backward kernels; hipErrorNotSupported = use the direct launcher instead.
 // kind 0: both stages, 1: stage 2 alone, 2: stage 1 alone.
 size_t binned_backward_workspace_bytes(const BwdArgs &a, int kind, int dtype);
+// the least that launch_backward_binned takes: without room for bfloat16 gradients' sums in float
+size_t binned_backward_least_workspace_bytes(const BwdArgs &a, int kind, int dtype);
 hipError_t launch_backward_binned(const BwdArgs &a, int dtype, void *workspace, size_t workspace_bytes,
                                   hipStream_t stream);
 // Zero fill by a kernel (no memset node: callers may capture the stream in a graph); bytes a multiple of 4.
