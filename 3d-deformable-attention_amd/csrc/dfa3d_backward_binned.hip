@@ -623,7 +623,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
 
   const BinPlan &p = *ws.plan;
   const int nb = p.bins_per_bm;
-  if (nb == 0) {
+  if (__builtin_expect(nb == 0, 0)) {
     backward_without_bins<T, FUSED>(ws, value, dist, score_in, grad_out, grad_score_in, grad_value, grad_dist, grad_loc, gl_stride,
                                     grad_attn, grad_score_out, grad_wu, Md, Mg, B, S, M, C, D, L, Q, P, grad16);
     return;
@@ -1141,7 +1141,7 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
   __shared__ int4 s_item[2], s_geo[2];
   __shared__ int s_lv[4][DFA3D_MAX_LEVELS];              // H, W, Dd, first key
   const BinPlan &p = *ws.plan;
-  if (p.bins_per_bm == 0) {
+  if (__builtin_expect(p.bins_per_bm == 0, 0)) {
     backward_without_bins<T, true>(ws, nullptr, dist, nullptr, nullptr, grad_score, nullptr, grad_dist, grad_loc3, 3, nullptr,
                                    nullptr, nullptr, M, M, B, S, M, 0, D, L, Q, P, 0);
     return;

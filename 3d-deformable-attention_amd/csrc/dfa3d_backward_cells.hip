@@ -305,7 +305,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
   __shared__ ItemGeom s_geom[kItemSlots];                // items, decoded by the thread that fetches them
 
   const BinPlan &p = *ws.plan;
-  if (p.bins_per_bm == 0) {
+  if (__builtin_expect(p.bins_per_bm == 0, 0)) {
     backward_without_bins<T, FUSED>(ws, value, dist, score_in, grad_out, grad_score_in, grad_value, grad_dist, grad_loc, gl_stride,
                                     grad_attn, grad_score_out, grad_wu, Md, Mg, B, S, M, C, D, L, Q, P, grad16);
     return;
