@@ -54,7 +54,9 @@ class _ProjectionFunction(Function):
 
     @staticmethod
     def forward(ctx, x, weight, bias):
-        ctx.save_for_backward(x, weight)
+        # each operand only where the other one's gradient needs it, as F.linear keeps them: the other may be changed in place
+        want_x, want_weight, _ = ctx.needs_input_grad
+        ctx.save_for_backward(x if want_weight else None, weight if want_x else None)
         return F.linear(x, weight, bias)
 
     @staticmethod
@@ -62,9 +64,12 @@ class _ProjectionFunction(Function):
         x, weight = ctx.saved_tensors
         want_x, want_weight, want_bias = ctx.needs_input_grad
         grad_x = grad.matmul(weight) if want_x else None
-        rows, grad_rows = x.reshape(-1, x.shape[-1]), grad.reshape(-1, grad.shape[-1])
-        if not want_weight or not plain_gradient(grad):
-            return grad_x, grad_rows.t().mm(rows) if want_weight else None, grad_rows.sum(0) if want_bias else None
+        grad_rows = grad.reshape(-1, grad.shape[-1])
+        if not want_weight:
+            return grad_x, None, grad_rows.sum(0) if want_bias else None
+        rows = x.reshape(-1, x.shape[-1])
+        if not plain_gradient(grad):
+            return grad_x, grad_rows.t().mm(rows), grad_rows.sum(0) if want_bias else None
         return (grad_x, *_weight_gradients(rows.contiguous(), grad_rows.contiguous(), want_bias))
 
 

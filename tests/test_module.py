@@ -152,3 +152,23 @@ def test_module_with_a_distribution_packed_once_for_several_calls():
     g1, = torch.autograd.grad(out1, q, go, retain_graph=True)
     g2, = torch.autograd.grad(out2, q, go)
     torch.testing.assert_close(g1, g2, rtol=1e-5, atol=1e-6)
+
+
+def test_projection_function_keeps_what_its_gradients_need():
+    """As F.linear: the weight may change in place before a backward that does not ask for the input's gradient, and the
+    input before one that does not ask for the weight's."""
+    from dfa3D.modules.projection import _ProjectionFunction
+    x, w, b = torch.randn(6, 4), torch.randn(2, 4, requires_grad=True), torch.randn(2, requires_grad=True)
+    out = _ProjectionFunction.apply(x, w, b)
+    with torch.no_grad():
+        w.mul_(2)
+    gw, gb = torch.autograd.grad(out.sum(), [w, b])
+    torch.testing.assert_close(gw, x.sum(0).expand(2, 4))
+    torch.testing.assert_close(gb, torch.full((2,), 6.0))
+    x, w = torch.randn(6, 4, requires_grad=True), torch.randn(2, 4)
+    y = x * 1
+    out = _ProjectionFunction.apply(y, w, b)
+    with torch.no_grad():
+        y.mul_(2)
+    gx, = torch.autograd.grad(out.sum(), [x])
+    torch.testing.assert_close(gx, w.sum(0).expand(6, 4))
