@@ -26,6 +26,16 @@ def ordinary(*tensors):
 _MIN_ROWS = 4096
 
 
+def _widths_apply(O, K):
+    """Where the kernel takes the gradient of an O x K weight: even widths of up to 2048 whose product is at most 2^20.  The
+    library's product is slow where the result has few tiles, and has caught up at about 64 tiles of 128 x 128.  Times as
+    fast as the library's product and column sum, 4096 / 20000 / 100000 rows: 256 x 512 1.5 / 4.5 / 4.1, 256 x 2048 1.2 /
+    1.8 / 1.3, 512 x 1024 1.2 / 1.0 / 1.0, 1024 x 1024 1.05 / 0.95 / 1.1; beyond, 1024 x 2048 0.89 / 0.87 / 0.87, 2048 x 2048
+    0.84 / 0.87 / 0.85, 64 x 4096 1.1 / 0.9 / 0.8.  The rule also bounds the workspace, 512 to 1024 tiles of 64 KB (2048 x
+    2048 would take 134 MB, 16384 x 16384 8.6 GB)."""
+    return O % 2 == 0 and K % 2 == 0 and max(O, K) <= 2048 and O * K <= 2 ** 20
+
+
 def _weight_gradients(x, grad, want_bias):
     """grad_weight (O, K) and grad_bias (O) or None, of contiguous float32 rows x (N, K) and grad (N, O)."""
     N, K = x.shape
@@ -76,8 +86,7 @@ class _ProjectionFunction(Function):
 def _applies(x, weight, bias):
     """Float32 rows on the GPU in ordinary reverse-mode training."""
     return (not torch.compiler.is_compiling() and bias is not None and torch.is_grad_enabled() and weight.requires_grad
-            and x.dim() >= 2
-            and weight.shape[0] % 2 == 0 and weight.shape[1] % 2 == 0 and max(weight.shape) <= 16384
+            and x.dim() >= 2 and _widths_apply(*weight.shape)
             and _MIN_ROWS <= x.numel() // max(x.shape[-1], 1) <= 2 ** 31 and ordinary(x, weight, bias))
 
 

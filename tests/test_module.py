@@ -172,3 +172,18 @@ def test_projection_function_keeps_what_its_gradients_need():
         y.mul_(2)
     gx, = torch.autograd.grad(out.sum(), [x])
     torch.testing.assert_close(gx, w.sum(0).expand(6, 4))
+
+
+def test_projection_workspace_stays_small():
+    """Wherever the rule hands a weight gradient to the kernel: 512 tiles of 64 KB over at most 64 tiles of the result, the
+    parts rounded up to a multiple of eight (at most 512 tiles more), and the bias."""
+    from dfa3D import _lib
+    from dfa3D.modules.projection import _widths_apply
+    taken = 0
+    for O in (2, 64, 130, 256, 640, 1024, 1360, 2048, 2050, 4096, 16384):
+        for K in (2, 64, 256, 512, 1024, 2048, 4096, 16384):
+            if _widths_apply(O, K):
+                taken += 1
+                for rows in (4096, 48000, 184950, 500000):
+                    assert _lib.lib().dfa3d_linear_grad_workspace_bytes(rows, O, K) <= 65 << 20, (rows, O, K)
+    assert taken >= 30 and not _widths_apply(2048, 2048) and not _widths_apply(3, 4)
