@@ -64,7 +64,12 @@ class SpatialCrossAttention_DFA3D(nn.Module):
         ``reference_points_cam`` (cams, bs, Nq, Z, 3) normalised image coordinates and depth of the Z anchors of
         every BEV query in every camera; ``bev_mask`` (cams, bs, Nq, Z) which of them fall inside the image.
         Returns (bs, Nq, E).  As in the reference, the queries of a camera are those whose mask is set for the
-        first batch element (:704-706), while the averaging counts cameras per batch element (:745-748)."""
+        first batch element (:704-706), while the averaging counts cameras per batch element (:745-748).
+
+        The attention module sees a batch in which the shorter cameras' lists are padded; nothing is read back from those
+        rows.  Their queries are zero as in the reference; their reference points are zero in the reference and -64 here
+        when the module is ``MSDeformableAttention3D_DFA3D`` itself (zero for any other class), so its samples of them lie
+        outside the map, and a forward hook on it sees other inputs and outputs in those rows than in the reference."""
         if key is None:
             key = query
         if value is None:
