@@ -520,33 +520,36 @@ def cpu_baseline(w, budget_s):
                       f"OpenMP over units (forward) and over the {sample.B} batch elements (backward)"}
 
 
-# What the development build can cut out of the backward's kernels (dfa3d_experiment_set("diag", bits)), and the
-# phases thread 0 of every tile workgroup clocks (-DDFA3D_TILE_TIMING).
-PHASE_CUTS = ((0, "nothing (the kernel as shipped, with the phase clocks compiled in)"),
-              (16, "the walk of the cells' lists / the task loop of the rows phase (dot products, weighted sums)"),
-              (512, "the per-point gradients and grad_dist taps (phase C / finish)"),
-              (2, "the grad_dist taps alone"),
-              (4, "the flush's device writes"),
-              (1, "the LDS tile updates of the rows phase (row-owned kernel only)"),
-              (256, "the grad_out row loads"),
-              (32, "the depth taps of phase A / prepare"),
-              (8, "the value row loads"),
-              (1024, "tickets (every grad_dist tap an LDS float atomic)"))
-# row-owned kernel (tile_backward_kernel): thread 0's clock, ten slots
+# What the development build can cut out of the tile kernels (dfa3d_experiment_set("diag", bits)): bits, what the
+# cell-owned kernel (cell_backward_kernel) and the row-owned one (tile_backward_kernel) then leave out, None = no such part.
+PHASE_CUTS = ((16, "the walk of the cells' lists (dot products, weighted sums)", "the task loop of the rows phase"),
+              (512, "the per-point gradients and grad_dist taps (finish)", "the per-point gradients and grad_dist taps (phase C)"),
+              (2, "the grad_dist taps alone", "the grad_dist taps alone"),
+              (4, "the device writes of both flushes", "the flush's device writes"),
+              (1, None, "the LDS tile updates of the rows phase"),
+              (256, None, "the grad_out row loads"),
+              (32, "the depth taps' loads (prepare)", "the depth taps of phase A"),
+              (8, "the value row loads", "the value row loads"),
+              (1024, None, "tickets (every grad_dist tap an LDS float atomic)"))
+# The phases that are clocked (-DDFA3D_TILE_TIMING), by slot.  Row-owned kernel: thread 0's clock, ten slots.
 PHASE_CLOCKS_ROWS = ("item fetch", "barrier after phases A and C", "rank + staging", "scan + placement", "rows",
                      "phases A and C", "flush", "tail", "-", "-")
-# cell-owned kernel (cell_backward_kernel): thread 0 (a walker) fills slots 0-7, thread 256 (a pointer) slots 8-15
-PHASE_CLOCKS_CELLS = ("walker: item fetch", "walker: walk (phase X)", "walker: wait at the barrier after X",
-                      "walker: stage grad_out rows / hand over accumulators (phase Y)", "walker: wait at the barrier after Y",
-                      "-", "-", "walker: flush",
-                      "pointer: item fetch", "pointer: late grad_dist taps (phase X)", "pointer: prepare (phase X)",
-                      "pointer: wait at the barrier after X", "pointer: place (phase Y)", "pointer: finish (phase Y)",
-                      "pointer: wait at the barrier after Y", "pointer: flush")
+# cell-owned kernel: thread 0 (a walker) fills slots 0-7, thread 256 (a pointer) slots 8-15
+PHASE_CLOCKS_CELLS = ("walker: set-up, the next item's record", "walker: walk (phase X)", "walker: wait at the barrier after X",
+                      "walker: item record fetched, the old item's sums put together (phase Y)",
+                      "walker: wait at the barrier after Y",
+                      "walker: the old item's sums and rim go out, value rows awaited (phase X)",
+                      "walker: value rows asked for, short grad_out rows staged (phase Y)", "-",
+                      "pointer: set-up, turn's bookkeeping", "pointer: scores, corner weights, next pass prepared (phase X)",
+                      "pointer: depth tile goes out (phase X)", "pointer: wait at the barrier after X",
+                      "pointer: grad_out rows asked for, points placed (phase Y)",
+                      "pointer: gradients and grad_dist taps, grad_out rows awaited (phase Y)",
+                      "pointer: wait at the barrier after Y", "-")
 
 
 def phase_costs(a):
-    """Text table: tile kernel duration with each part cut out (the difference to the first row is what that part
-    costs where it stands), and the share of thread 0's clock each phase takes."""
+    """Text table: tile kernel duration with each part cut out (the difference to the whole kernel is what that part
+    costs where it stands), and the share of its clock that a thread of each role spends in each phase."""
     import torch
     from dfa3D import _lib
     _lib.LIB_PATH = os.path.join(ROOT, "libdfa3d_hip_experiment.so")
@@ -608,17 +611,8 @@ def phase_costs(a):
     print(f"# python bench.py --phase-costs --workload {a.workload}" + "".join(f" --option {t}" for t in a.option))
     print(f"# development build (-DDFA3D_EXPERIMENT -DDFA3D_TILE_TIMING) of the kernel sources with digest {sources_digest()[:16]}")
     print(f"# {torch.cuda.get_device_name(0)}; {w.points} points; medians of {a.kernel_reps} launches; a cut changes results, "
-          "its row says what the kernel takes WITHOUT that part")
-    print(f"{'cut out':72s} {'binning ms':>10s} {'tile ms':>9s} {'saves ms':>9s}")
-    base_tile = None
-    for bits, label in PHASE_CUTS:
-        L_.dfa3d_experiment_set(b"diag", bits)
-        b_ms, t_ms = timed(a.kernel_reps)
-        base_tile = t_ms if base_tile is None else base_tile
-        print(f"{label:72s} {b_ms:10.4f} {t_ms:9.4f} {base_tile - t_ms:9.4f}", flush=True)
-    L_.dfa3d_experiment_set(b"diag", 0)
-    gv.zero_()
-    gd.zero_()
+          "its row says what the kernel takes WITHOUT that part, and whole just before and after")
+    call()                                       # once for the clocks, which say which of the kernels the workload takes
     ws.zero_()
     call()
     torch.cuda.synchronize()
@@ -626,6 +620,20 @@ def phase_costs(a):
     ticks = ws[off:off + 128].view(torch.int64).cpu().tolist()
     cells = any(ticks[10:])                      # only the cell-owned kernel clocks more than ten slots
     names = PHASE_CLOCKS_CELLS if cells else PHASE_CLOCKS_ROWS
+    print(f"{'cut out':72s} {'binning ms':>10s} {'tile ms':>9s} {'whole ms':>9s} {'saves ms':>9s}")
+    timed(a.kernel_reps)
+    b_ms, before = timed(a.kernel_reps)
+    print(f"{'nothing (the kernel as shipped, with the phase clocks compiled in)':72s} {b_ms:10.4f} {before:9.4f}", flush=True)
+    for bits, *labels in PHASE_CUTS:
+        label = labels[0 if cells else 1]
+        if label is None:
+            continue
+        L_.dfa3d_experiment_set(b"diag", bits)
+        b_ms, t_ms = timed(a.kernel_reps)
+        L_.dfa3d_experiment_set(b"diag", 0)
+        _, after = timed(a.kernel_reps)          # the whole kernel before and after each cut: the clock drifts
+        whole, before = (before + after) / 2, after
+        print(f"{label:72s} {b_ms:10.4f} {t_ms:9.4f} {whole:9.4f} {whole - t_ms:9.4f}", flush=True)
     print("\nshare of a thread's clock per phase, summed over the workgroups of one launch"
           + (" (walkers: wavefronts 0-3, pointers: wavefronts 4-7; each role's shares add up to 100 %)" if cells else ""))
     for lo, hi in ((0, 8), (8, 16)) if cells else ((0, 10),):
