@@ -20,12 +20,13 @@
 // otherwise overlap.  Turns follow one another without a gap, whatever item their passes belong to (pass t: one of
 // the item's passes), so that an item of a single pass costs a single turn:
 //   phase X(t):  walkers: walk(t-1)        pointers: scores and corner weights of t, prepare(t+1)
-//   phase Y(t):  walkers: flush            pointers: stage(t), place(t) (scan + sorted slots), finish(t-1)
+//   phase Y(t):  walkers: next to nothing  pointers: stage(t), place(t) (scan + sorted slots), finish(t-1)
 // and where pass t-1 was its item's last:
-//   Y(t):    walkers ask for the value rows of the item of pass t and put the old item's corner sums together in
-//            registers (neighbouring cells are neighbouring lane groups); sums that cross into the next wavefront's rows
-//            go through a few rows of LDS and out in X(t+1)
-//   X(t+1):  everybody flushes the depth tile, before the first finish of the next item in Y(t+1)
+//   Y(t):    walkers put the old item's corner sums together in registers (neighbouring cells are neighbouring lane groups;
+//            sums that cross into the next wavefront's rows, and the rim's, go through a few rows of LDS) and ask for the
+//            value rows of the item of pass t
+//   X(t+1):  walkers send the old item's last rows and its rim before they walk; pointers write the depth tile out and leave
+//            it zeroed, before the first finish of the next item in Y(t+1)
 // grad_dist taps go to the LDS tile by compare-and-swap on the word's bits: the LDS float atomic retires 0.33 lanes per
 // clock and CU, read + compare-and-swap 2.9 (and a tap is complete when its phase ends, which the flush relies on).
 //
@@ -33,8 +34,6 @@
 #include "dfa3d_binned.h"
 
 namespace dfa3d {
-
-typedef unsigned int u32x3 __attribute__((ext_vector_type(3)));
 
 constexpr int kWalkers = 256;         // threads of the walker wavefronts 0-3; the wavefronts after them own the points
 
@@ -59,17 +58,6 @@ __host__ __device__ inline CellShape cell_shape(int C) {
 // the most tile rows of 8 cells that four walker wavefronts own
 int cell_max_ty(int C) { return 4 * (kWave / cell_shape(C).lpr) / kCellTX; }
 
-// The rim of a tile of (ty + 1) x 9 pixels, numbered: row 0, row ty, then the first and last pixel of the rows between.
-__host__ __device__ inline int rim_pixels(int ty) { return 2 * (kCellTX + 1) + 2 * (ty - 1); }
-__device__ __forceinline__ int rim_index(int row, int col, int ty) {
-  return row == 0 ? col : row == ty ? kCellTX + 1 + col : 2 * (kCellTX + 1) + 2 * (row - 1) + (col == 0 ? 0 : 1);
-}
-__device__ __forceinline__ void rim_decode(int i, int ty, int &row, int &col) {
-  const int s = i - 2 * (kCellTX + 1);
-  row = s >= 0 ? 1 + (s >> 1) : i <= kCellTX ? 0 : ty;
-  col = s >= 0 ? ((s & 1) ? kCellTX : 0) : i <= kCellTX ? i : i - (kCellTX + 1);
-}
-
 struct CellLds {      // offsets (in 4-byte words) into the dynamic LDS block
   int gd, gstage, dots, sslot, cnt, offs, goff, cross, rim, total;
 };
@@ -85,7 +73,7 @@ __host__ __device__ inline CellLds cell_lds_layout(int ty, int row, int cells, i
   o.goff = o.offs + cells + 1;
   o.cross = (o.goff + 2 * pass + 3) & ~3;                   // sums that cross into the next wavefront's tile rows
   o.rim = o.cross + 3 * (kCellTX + 1) * row;                 // sums of the tile's rim pixels, on their way out
-  o.total = o.rim + rim_pixels(ty) * row;
+  o.total = o.rim + rim_pixels(ty, kCellTX) * row;
   return o;
 }
 
@@ -378,11 +366,11 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       }
     }
     const int n = gd16 ? D >> 1 : D, sh = lanes_log2(n);
-    const int rows = sole_d ? rim_pixels(TY) : R;
+    const int rows = sole_d ? rim_pixels(TY, TX) : R;
     for (int i = first >> sh; i < rows; i += threads >> sh) {
       int ry, rx;
       if (sole_d) {
-        rim_decode(i, TY, ry, rx);
+        rim_decode(i, TY, TX, ry, rx);
       } else {
         ry = i / TW; rx = i % TW;
       }
@@ -459,7 +447,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     // cleared what is added to), else added.  Rim pixels go to their place in LDS, to be added by put_rim.
     auto put_pixel = [&](const Owner &o, const ItemGeom &q, const float (&u)[VEC], bool active) {
       const int y = q.y0 + o.crow, x = q.x0 + o.ccol;
-      if (active && (o.crow == 0 || o.ccol == 0)) put_lds(o, rim + rim_index(o.crow, o.ccol, TY) * ROW, u);
+      if (active && (o.crow == 0 || o.ccol == 0)) put_lds(o, rim + rim_index(o.crow, o.ccol, TY, TX) * ROW, u);
       if (active && o.crow > 0 && o.ccol > 0 && y < q.H && x < q.W && !DFA3D_DIAG(diag, 4)) {
         char *gvalue_b = static_cast<char *>(grad_value) + (size_t)q.b * S * M * C * (gv16 ? 2 : 4);
         float *gvalue_f = reinterpret_cast<float *>(gvalue_b);
@@ -493,7 +481,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       for (int i = lane; i < n * per; i += kWave) {
         const int k = first + i / per, c = (i % per) * (gv16 ? 2 : 1);
         int ry, rx;
-        rim_decode(k, TY, ry, rx);
+        rim_decode(k, TY, TX, ry, rx);
         const int y = q.y0 + ry, x = q.x0 + rx;
         const float *from = rim + k * ROW + c;
         const float f0 = from[0], f1 = gv16 ? from[1] : 0.f;
@@ -614,10 +602,10 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
             }
           }
           if (o.crow < TY) {
-            if (o.ccol == TX - 1) put_lds(o, rim + rim_index(o.crow, TX, TY) * ROW, ux);
+            if (o.ccol == TX - 1) put_lds(o, rim + rim_index(o.crow, TX, TY, TX) * ROW, ux);
             if (o.crow + 1 == TY) {
-              put_lds(o, rim + rim_index(TY, o.ccol, TY) * ROW, dn);
-              if (o.ccol == TX - 1) put_lds(o, rim + rim_index(TY, TX, TY) * ROW, dx);
+              put_lds(o, rim + rim_index(TY, o.ccol, TY, TX) * ROW, dn);
+              if (o.ccol == TX - 1) put_lds(o, rim + rim_index(TY, TX, TY, TX) * ROW, dx);
             } else if (o.group >= (ROWS - 1) * TX) {         // for the wavefront below
               put_lds(o, cross + (wave * TW + o.ccol) * ROW, dn);
               if (o.ccol == TX - 1) put_lds(o, cross + (wave * TW + TX) * ROW, dx);
@@ -660,7 +648,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
               const float4 a = *reinterpret_cast<const float4 *>(from + o.ch.first[gi]);
               u[4 * gi] += a.x; u[4 * gi + 1] += a.y; u[4 * gi + 2] += a.z; u[4 * gi + 3] += a.w;
               if (o.ccol == TX - 1) {
-                float4 *at = reinterpret_cast<float4 *>(rim + rim_index(o.crow, TX, TY) * ROW + o.ch.first[gi]);
+                float4 *at = reinterpret_cast<float4 *>(rim + rim_index(o.crow, TX, TY, TX) * ROW + o.ch.first[gi]);
                 const float4 b = *reinterpret_cast<const float4 *>(from + ROW + o.ch.first[gi]), c = *at;
                 *at = make_float4(c.x + b.x, c.y + b.y, c.z + b.z, c.w + b.w);
               }
@@ -670,7 +658,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           wave_lds_handover();
           const int ra = max(r0, 1), n_side = min(r0 + ROWS, TY) - ra;
           if (wave == 0) put_rim(q, 0, TW);
-          if (n_side > 0) put_rim(q, rim_index(ra, 0, TY), 2 * n_side);
+          if (n_side > 0) put_rim(q, rim_index(ra, 0, TY, TX), 2 * n_side);
           if (r0 + ROWS >= TY) put_rim(q, TW, TW);
         }
         if (done) break;

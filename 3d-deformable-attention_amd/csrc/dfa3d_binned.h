@@ -42,7 +42,8 @@ __device__ __forceinline__ void slot_decode(int slot, int B, int M, int &b, int 
   m = (hm % G) * kClasses + hm / G;
 }
 
-// Division of n < 2^31 by a number the host knows: multiply by ceil(2^(32 + shift) / d) - 2^32, add, shift.
+// Division of n < 2^31 by a number the host knows: multiply by ceil(2^(32 + shift) / d) - 2^32, add, shift (T. Granlund and
+// P. Montgomery, Division by invariant integers using multiplication, 1994).
 struct FastDiv {
   uint32_t mul, shift;
   explicit FastDiv(uint32_t d) {
@@ -97,14 +98,18 @@ __device__ __forceinline__ int wave_inclusive_scan(int x) {
 // Points of a bin per work item.  Small items balance the workgroups, but the items of one bin add to its gradients
 // with atomics, which the memory takes at one 64-byte piece per 50 ps (a split bin of 96 channels and depth bins:
 // 20 ns per item), where a bin of one item stores them.  So: about 4096 items if that leaves large ones, else down to
-// 1024 items, none under 256 points.  0.34 M points in 240 bins: 88 us with 4096 points per item, 44 with these; 0.58 M
-// of plain attention: 230 and 60; 15.4 M: no difference.
-constexpr int kMaxChunk = 4096;
+// 1024 items of up to kMidChunk points, none under 256 points.  0.34 M points in 240 bins: 88 us with 4096 points per item,
+// 44 with these; 0.58 M of plain attention: 230 and 60; 15.4 M: no difference.  kMidChunk, which decides from 1.3 to 5.2 M
+// points, is five passes, in the middle of a flat range: the training step on two levels from 60 x 100, 3 x 10000
+// queries (3.8 M points), takes 635 / 590 / 600 / 622 / 730 us with 512 / 1024 / 1280 / 2048 / 4096 points per item at
+// clustered locations and 621 / 537 / 533 / 530 / 548 at uniform ones, on one level of 29 x 50 at coherent ones (2.6 M)
+// 384 / 333 / 350 / 325 / 335.
+constexpr int kMaxChunk = 4096, kMidChunk = 1280;
 __device__ __forceinline__ int chunk_of(const BinWorkspace &ws, const BinPlan &p) {
   if (p.chunk > 0) return p.chunk;
   int n = 0;
   for (int c = 0; c < kClasses; ++c) n += ws.queues[c * kQueueStride + 1];
-  return min(max(max(n >> 12, min(n >> 10, 1280)), 256), kMaxChunk);
+  return min(max(max(n >> 12, min(n >> 10, kMidChunk)), 256), kMaxChunk);
 }
 // Work items of a bin with c points, of equal shares (most bins have one, which saves the division); item t of k starts
 // at point share_begin(c, k, t) of the bin.
