@@ -11,7 +11,7 @@
  * of the calling thread.
  *
  * Tensor layouts (all contiguous, row-major), with
- *   B batch, S = sum_l H_l*W_l keys, M heads, C channels per head, D depth bins,
+ *   B batch, S keys (sum_l H_l*W_l, fewer where levels share some), M heads, C channels per head, D depth bins,
  *   L levels, Q queries, P points per level:
  *     value        (B,S,M,C)            dist        (B,S,M,D)
  *     shapes       (L,shape_stride) int64, row = (H, W[, Dd]); shape_stride is 2 or 3
@@ -29,7 +29,8 @@
  *                 grad_dist are bfloat16 as well (what an autograd caller has to return for bfloat16 inputs):
  *                 sums are formed in float in LDS and rounded once when a tile is written; the rows that
  *                 several tiles share are added with the hardware's packed bfloat16 atomic, which rounds the
- *                 stored sum at each of the few adds.  Offered on the binned kernels only
+ *                 stored sum at each of the few adds; where tiles are small and most rows shared, the sums are
+ *                 float in the workspace and rounded once.  Offered on the binned kernels only
  *                 (dfa3d_fused_backward_workspace_bytes(..., DFA3D_BF16G, ...) > 0: C and D multiples of 4)
  *
  * The four *_forward / *_backward pairs replace the reference's four native entry
@@ -194,7 +195,8 @@ int dfa3d_fused_backward(
 /* Scratch bytes dfa3d_fused_backward wants for these dimensions; 0 when the binned path does not
  * apply (DFA3D_F64, rows too long for LDS tiles, more than 2^31 points, invalid dimensions).  With
  * dist_heads = 1 this includes B*S*M*D floats: grad_dist is formed per head and summed over the heads
- * by a last kernel. */
+ * by a last kernel.  With DFA3D_BF16G it may include the float sums of both gradients; the bytes for
+ * DFA3D_BF16 are enough then too, with more roundings on the rows that tiles share. */
 size_t dfa3d_fused_backward_workspace_bytes(int B, int S, int M, int C, int D, int L, int Q, int P, int dist_heads,
                                             int dtype, const dfa3d_launch_options *opts);
 
@@ -203,7 +205,7 @@ size_t dfa3d_fused_backward_workspace_bytes(int B, int S, int M, int C, int D, i
  * results as dfa3d_fused_backward, without the workspace: the scratch memory of the binned kernels is a static
  * array of DFA3D_STATIC_SCRATCH_BYTES inside the library's code object, which every GPU the library runs on
  * holds until the process ends.  The call allocates and frees nothing.  Dimensions whose
- * dfa3d_fused_backward_workspace_bytes exceeds that size are rejected with DFA3D_ERANGE (at the BEVFormer-small
+ * dfa3d_fused_backward_workspace_bytes (DFA3D_BF16G: what DFA3D_BF16 takes) exceeds that size are rejected with DFA3D_ERANGE (at the BEVFormer-small
  * shape, 1.5 M sampling points, the kernels want 29.8 MiB); dimensions the binned path does not apply to
  * (workspace size 0, e.g. DFA3D_F64) run on the direct kernels, which need no scratch.
  * Every call on one GPU uses that GPU's one array: calls that overlap in time on the same GPU (two streams, two
