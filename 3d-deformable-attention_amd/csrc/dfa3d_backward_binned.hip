@@ -4,10 +4,10 @@
 // Why: device-memory atomics retire at roughly 10^10 cache-line requests per second on this part,
 // and the straightforward backward (bwd_attention_kernel) needs 4 row updates of grad_value and 8
 // scalar updates of grad_dist per sampling point.  So the points are first binned by the image tile they
-// fall in, and one workgroup per tile accumulates that tile of grad_value and grad_dist in LDS and writes it
-// out once: grad_value rows without any atomics (a lane group owns each tile row), grad_dist taps with
-// plain LDS updates handed out by integer tickets (LDS floating-point atomics only for the few taps that
-// meet another one of the same pass at their address).
+// fall in, and one workgroup per tile accumulates that tile of grad_value and grad_dist in registers and LDS and
+// writes it out once: grad_value without any atomics (a lane group owns a cell, or a tile row), grad_dist taps with
+// plain LDS updates made exclusive by integer operations (compare-and-swap, or tickets; LDS floating-point atomics
+// only for the few taps that meet others at their address).
 //
 //   plan_and_clear_kernel       validates the level table, lays out the tiles (bins), clears counters
 //   bin_count_kernel            points per bin (LDS histogram per block, one atomic per touched bin)
@@ -18,13 +18,15 @@
 //                               gradients for points the operator skips
 //   bin_points_kernel<0>, <1>   count and fill for shapes the two above do not take (more than 2048 tiles per
 //                               (batch, head), more than 2048 points per unit): every record straight to its slot
-//   tile_backward_kernel        persistent workgroups pull work items from per-XCD queues; per item: LDS
-//                               tiles of (TY+1) x (TX+1) pixels (one-pixel halo to the right/bottom, so
-//                               all four corners of a point of this bin land in the tile), the phases
-//                               described above the kernel, then one flush of the tile.  FUSED=false:
-//                               stage 2 alone
+//   cell_backward_kernel        persistent workgroups pull work items from per-XCD queues: rows of up to 64
+//                               channels in whole groups of four (dfa3d_backward_cells.hip)
+//   tile_backward_kernel        the same for all other rows; per item: LDS tiles of (TY+1) x (TX+1) pixels
+//                               (one-pixel halo to the right/bottom, so all four corners of a point of this
+//                               bin land in the tile), the phases described above the kernel, then one
+//                               flush of the tile.  FUSED=false (of both): stage 2 alone
 //   tile_depth_backward_kernel  stage 1 alone on the same bins
-//   fill_zero / head_sum        a distribution shared by the heads: grad_dist per head, then summed
+//   head_sum_kernel             a distribution shared by the heads: grad_dist per head, then summed
+//   round_rows_kernel           bfloat16 gradients whose sums were formed in float (sums_in_float)
 //
 // A point belongs to the tile that holds its base pixel (h0, w0) = floor of its pixel coordinates, -1 <= h0 < H,
 // -1 <= w0 < W; the tiles are laid over that range, so the first tile of a level starts at pixel -1.
