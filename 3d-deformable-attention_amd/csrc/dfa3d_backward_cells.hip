@@ -272,18 +272,42 @@ __device__ __forceinline__ void load_to_lds16(rsrc_t r, const void *lds, uint32_
 __device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }           // vmcnt(0)
 __device__ __forceinline__ void wait_for_all_but_two() { __builtin_amdgcn_s_waitcnt(0x0F72); }     // vmcnt(2)
 
+// The kernel's arguments.  They are read from the constant segment anew in every phase (args()): there are more of them, and
+// of the numbers that follow from them, than scalar registers.  Passed one by one they were kept from turn to turn, at the
+// cost of 98 others (float, 32 channels; 105 with bfloat16) that went to lanes of vector registers and came back one
+// instruction each.  Base shape, 15.4 M points: 1194 -> 1184 us, bfloat16 1160 -> 1100 us.
+template <typename T> struct CellArgs {
+  BinWorkspace ws;
+  const T *value, *dist, *score_in, *grad_out, *grad_score_in;
+  void *grad_value, *grad_dist;
+  float *grad_loc, *grad_attn, *grad_score_out;
+  const float *grad_wu;
+  int gl_stride;
+  int Md, Mg;                 // heads stored in dist (M, or 1 = shared by all heads); heads of the grad_dist buffer written here
+  int B, S, M, C, D, L, Q, P;
+  FastDiv div_lp;
+  int grad16;                 // bit 0 = grad_value is bfloat16, bit 1 = grad_dist is bfloat16 (else float)
+#ifdef DFA3D_EXPERIMENT
+  int diag;
+#endif
+};
+#ifdef __HIP_DEVICE_COMPILE__
+template <typename T> using CellArgsPtr = const __attribute__((address_space(4))) CellArgs<T> *;
+template <typename T> __device__ __forceinline__ CellArgsPtr<T> args() {
+  auto a = (CellArgsPtr<T>)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return a;
+}
+#else
+template <typename T> using CellArgsPtr = const CellArgs<T> *;
+template <typename T> __device__ CellArgsPtr<T> args();
+#endif
+
 // FUSED: both stages (depth scores recomputed from dist, grad_dist and the z gradient produced).
 // !FUSED: stage 2 alone: scores read from score_in, their gradient written to grad_score_out, no depth tile
 // (the launcher passes D = 0), grad_loc has gl_stride components of which x, y are written.
 template <typename T, int VEC, int LPR, bool FUSED>
-__global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_kernel(
-    BinWorkspace ws, const T *__restrict__ value, const T *__restrict__ dist, const T *__restrict__ score_in,
-    const T *__restrict__ grad_out, const T *__restrict__ grad_score_in,
-    void *__restrict__ grad_value, void *__restrict__ grad_dist, float *__restrict__ grad_loc, int gl_stride,
-    float *__restrict__ grad_attn, float *__restrict__ grad_score_out, const float *__restrict__ grad_wu, int Md,
-    int Mg, int B, int S, int M, int C, int D, int L, int Q, int P, FastDiv div_lp, int grad16 DFA3D_DIAG_PARAM) {
-  // grad16: bit 0 = grad_value is bfloat16, bit 1 = grad_dist is bfloat16 (else float)
-  // Md: heads stored in dist (M, or 1 = shared by all heads); Mg: heads of the grad_dist buffer written here
+__global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_kernel(CellArgs<T>) {
   constexpr int PP = cell_pass(LPR), BLOCK = kWalkers + PP, TX = kCellTX, TW = TX + 1, ROW = VEC * LPR;
   constexpr int GPW = kWave / LPR, CELLS = 4 * GPW, ROWS = GPW / TX;      // cells and tile rows per walker wavefront
   typedef float f4 __attribute__((ext_vector_type(4)));
@@ -292,14 +316,17 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
   __shared__ CellFetch s_fetch;                           // the fetching thread's queue state, between its turns
   __shared__ ItemGeom s_geom[kItemSlots];                // items, decoded by the thread that fetches them
 
+  const auto a0 = args<T>();
+  const BinWorkspace ws = a0->ws;
   const BinPlan &p = *ws.plan;
   if (__builtin_expect(p.bins_per_bm == 0, 0)) {
-    backward_without_bins<T, FUSED>(ws, value, dist, score_in, grad_out, grad_score_in, grad_value, grad_dist, grad_loc, gl_stride,
-                                    grad_attn, grad_score_out, grad_wu, Md, Mg, B, S, M, C, D, L, Q, P, grad16);
+    backward_without_bins<T, FUSED>(ws, a0->value, a0->dist, a0->score_in, a0->grad_out, a0->grad_score_in, a0->grad_value, a0->grad_dist,
+                                    a0->grad_loc, a0->gl_stride, a0->grad_attn, a0->grad_score_out, a0->grad_wu, a0->Md, a0->Mg,
+                                    a0->B, a0->S, a0->M, a0->C, a0->D, a0->L, a0->Q, a0->P, a0->grad16);
     return;
   }
   const int TY = p.ty, R = (TY + 1) * TW;
-  const CellLds lay = cell_lds_layout(TY, ROW, CELLS, PP, D, (int)sizeof(T));
+  const CellLds lay = cell_lds_layout(TY, ROW, CELLS, PP, a0->D, (int)sizeof(T));
   const int tid = threadIdx.x, lane = tid % kWave;
   // The role is decided by a scalar, so that the compiler branches on it uniformly: a wavefront must never run
   // through the other role's code with all lanes switched off, because barriers count wavefronts, not lanes.
@@ -310,7 +337,6 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
   uint16_t *s_slot = reinterpret_cast<uint16_t *>(smem + lay.sslot);
   int *cnt = reinterpret_cast<int *>(smem + lay.cnt), *offs = reinterpret_cast<int *>(smem + lay.offs);
   uint32_t *goff = reinterpret_cast<uint32_t *>(smem + lay.goff);
-  const bool gv16 = (grad16 & 1) != 0, gd16 = (grad16 & 2) != 0;          // uniform
 
   for (int i = tid; i < lay.gstage; i += BLOCK) smem[i] = 0;                   // depth tile
   for (int i = tid; i < 3 * CELLS; i += BLOCK) cnt[i] = 0;
@@ -333,6 +359,10 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
   // divisions.  Pixels 1..TY-1 x 1..7 belong to no neighbour's halo: when the item writes its tile alone they are stored,
   // the others are added.
   auto flush_gd = [&](int which, int first, int threads) {
+    const auto a = args<T>();
+    const int D = a->D, S = a->S, M = a->M, Mg = a->Mg;
+    void *grad_dist = a->grad_dist;
+    const bool gd16 = (a->grad16 & 2) != 0;                // uniform
     const ItemGeom q = uniform(s_geom[which]);
     const int mg = Mg == 1 ? 0 : q.m;
     char *gdist_b = static_cast<char *>(grad_dist) + (size_t)q.b * S * Mg * D * (gd16 ? 2 : 4);
@@ -346,7 +376,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       for (int i = first >> sh; i < inner; i += threads >> sh) {
         const int ry = i / (TX - 1) + 1, rx = i % (TX - 1) + 1, r = ry * TW + rx;
         const int y = q.y0 + ry, x = q.x0 + rx;
-        const bool out = y < q.H && x < q.W && !DFA3D_DIAG(diag, 4);
+        const bool out = y < q.H && x < q.W && !DFA3D_DIAG(args<T>()->diag, 4);
         const uint32_t e0 = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D);
         for (int c = first & ((1 << sh) - 1); c < n; c += 1 << sh) {
           if (d4) {
@@ -375,7 +405,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         ry = i / TW; rx = i % TW;
       }
       const int r = ry * TW + rx, y = q.y0 + ry, x = q.x0 + rx;
-      const bool out = in_map(y, x, q.H, q.W) && !DFA3D_DIAG(diag, 4);
+      const bool out = in_map(y, x, q.H, q.W) && !DFA3D_DIAG(args<T>()->diag, 4);
       const uint32_t e0 = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D);
       for (int c = first & ((1 << sh) - 1); c < n; c += 1 << sh) {
         if (gd16) {
@@ -417,7 +447,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     auto owner = [&]() {
       unsigned l = lane;
       asm volatile("" : "+v"(l));
-      return Owner(l, wave, C);
+      return Owner(l, wave, args<T>()->C);
     };
     auto decode = [&](const int4 &item, const int4 &geo) {
       ItemGeom g;
@@ -446,9 +476,13 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     // halo: when the item writes its tile alone they are stored (grad_value is zero on entry, or the binning launches
     // cleared what is added to), else added.  Rim pixels go to their place in LDS, to be added by put_rim.
     auto put_pixel = [&](const Owner &o, const ItemGeom &q, const float (&u)[VEC], bool active) {
+      const auto a = args<T>();
+      const int S = a->S, M = a->M, C = a->C;
+      const bool gv16 = (a->grad16 & 1) != 0;               // uniform
+      void *grad_value = a->grad_value;
       const int y = q.y0 + o.crow, x = q.x0 + o.ccol;
       if (active && (o.crow == 0 || o.ccol == 0)) put_lds(o, rim + rim_index(o.crow, o.ccol, TY, TX) * ROW, u);
-      if (active && o.crow > 0 && o.ccol > 0 && y < q.H && x < q.W && !DFA3D_DIAG(diag, 4)) {
+      if (active && o.crow > 0 && o.ccol > 0 && y < q.H && x < q.W && !DFA3D_DIAG(args<T>()->diag, 4)) {
         char *gvalue_b = static_cast<char *>(grad_value) + (size_t)q.b * S * M * C * (gv16 ? 2 : 4);
         float *gvalue_f = reinterpret_cast<float *>(gvalue_b);
         const rsrc_t gvalue_r = make_rsrc(gvalue_b, (size_t)S * M * C * sizeof(float));
@@ -474,6 +508,10 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     };
     // Rim pixels [first, first + n) of item q, whose sums this wavefront left in LDS.
     auto put_rim = [&](const ItemGeom &q, int first, int n) {
+      const auto a = args<T>();
+      const int S = a->S, M = a->M, C = a->C;
+      const bool gv16 = (a->grad16 & 1) != 0;               // uniform
+      void *grad_value = a->grad_value;
       char *gvalue_b = static_cast<char *>(grad_value) + (size_t)q.b * S * M * C * (gv16 ? 2 : 4);
       float *gvalue_f = reinterpret_cast<float *>(gvalue_b);
       const rsrc_t gvalue_r = make_rsrc(gvalue_b, (size_t)S * M * C * sizeof(float));
@@ -485,7 +523,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         const int y = q.y0 + ry, x = q.x0 + rx;
         const float *from = rim + k * ROW + c;
         const float f0 = from[0], f1 = gv16 ? from[1] : 0.f;
-        if (c < C && in_map(y, x, q.H, q.W) && (f0 != 0 || f1 != 0) && !DFA3D_DIAG(diag, 4)) {
+        if (c < C && in_map(y, x, q.H, q.W) && (f0 != 0 || f1 != 0) && !DFA3D_DIAG(args<T>()->diag, 4)) {
           const uint32_t e = (uint32_t)(((q.start + y * q.W + x) * M + q.m) * C + c);
           if (gv16) atomic_add_bf16x2(gvalue_b + (size_t)e * 2, f0, f1);
           else scatter_add(gvalue_r, gvalue_f, e * 4, f0);
@@ -512,6 +550,9 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     };
     // phase Y: the grad_out rows of the pass, where they cannot go straight from memory to LDS (then the pointers see to it)
     auto stage = [&]() {
+      const auto a = args<T>();
+      const int Q = a->Q, M = a->M, C = a->C;
+      const T *grad_out = a->grad_out;
       if (C == ROW) return;                                  // uniform
       const Owner o = owner();
       const rsrc_t go_r = make_rsrc(grad_out + (size_t)g.b * Q * M * C, (size_t)Q * M * C * sizeof(T));
@@ -579,7 +620,8 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         if (tid == 0 && !done) {
           CellFetch fetch = s_fetch;
           int4 rec, geo;
-          fetch.advance(ws, p, &rec, &geo);
+          const BinWorkspace w = args<T>()->ws;
+          fetch.advance(w, *w.plan, &rec, &geo);
           s_geom[slot_of_item(it + 3)] = decode(rec, geo);
           s_fetch = fetch;
         }
@@ -618,12 +660,15 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         {
           // the four value rows of this group's cell (zero outside the map, when the cell is not part of the tile, or when
           // there is no item)
+          const auto a = args<T>();
+          const int S = a->S, M = a->M, C = a->C;
+          const T *value = a->value;
           const Owner o = owner();
           const rsrc_t value_r = make_rsrc(value + (size_t)g.b * S * M * C, (size_t)S * M * C * sizeof(T));
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
             const int y = g.y0 + o.crow + (k >= 2 ? 1 : 0), x = g.x0 + o.ccol + ((k == 1 || k == 2) ? 1 : 0);
-            const bool ok = !done && o.crow < TY && in_map(y, x, g.H, g.W) && !DFA3D_DIAG(diag, 8);
+            const bool ok = !done && o.crow < TY && in_map(y, x, g.H, g.W) && !DFA3D_DIAG(args<T>()->diag, 8);
             o.ch.load(value_r, ok ? (uint32_t)(((g.start + y * g.W + x) * M + g.m) * C * (int)sizeof(T)) : kNoRow, vr[k]);
           }
         }
@@ -668,7 +713,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = (f4){0, 0, 0, 0};
         CT_MARK(5);
-        if (apart() && !DFA3D_DIAG(diag, 16)) walk(v, acc);
+        if (apart() && !DFA3D_DIAG(args<T>()->diag, 16)) walk(v, acc);
         CT_MARK(1);
         lds_barrier();
         CT_MARK(2);
@@ -679,7 +724,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           CT_MARK(4);
           ++turn;
           clear_counts();
-          if (apart() && !DFA3D_DIAG(diag, 16)) walk(v, acc);
+          if (apart() && !DFA3D_DIAG(args<T>()->diag, 16)) walk(v, acc);
           CT_MARK(1);
           lds_barrier();
           CT_MARK(2);
@@ -703,7 +748,6 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     cur.gp = nxt.gp = 0; cur.a = nxt.a = 0; cur.lh = cur.lw = cur.ld = nxt.lh = nxt.lw = nxt.ld = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) { cur.sc[k] = cur.hl[k] = nxt.sc[k] = nxt.hl[k] = 0; taps.t[k] = (u32x2){0, 0}; }
-    const uint32_t slice = (uint32_t)Q * (uint32_t)M * (uint32_t)(L * P);             // points of a batch element
     __syncthreads();                                        // the first items' records are there
 
     ItemGeom g = uniform(s_geom[0]);                         // pass A (the one prepared last): points [base, base + PP) of item `it`
@@ -713,8 +757,9 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     float4 pre_rec = make_float4(0, 0, 0, 0);
     auto ask_records = [&]() {
       const int at = rec_bin >= 0 ? rec_seg + rec_base + min(pslot, rec_n - rec_base - 1) : 0;
-      pre_gp = ws.entries[at];
-      pre_rec = ws.recs[at];
+      const auto a = args<T>();
+      pre_gp = a->ws.entries[at];
+      pre_rec = a->ws.recs[at];
     };
     auto next_records = [&]() {
       if (rec_bin >= 0) {
@@ -730,6 +775,10 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     };
     // geometry of this thread's point of pass A, its place in the sort, its grad_out row for the walkers; its taps are asked for
     auto prepare = [&](int pass) {
+      const auto ar = args<T>();
+      const int D = ar->D, S = ar->S, M = ar->M, Md = ar->Md, Q = ar->Q, C = ar->C;
+      const T *dist = ar->dist, *score_in = ar->score_in;
+      const FastDiv div_lp = ar->div_lp;
       const bool live = g.bin >= 0 && pslot < g.n_item - base;
       const uint32_t gp = live ? pre_gp : 0u;
       const float4 rec = pre_rec;
@@ -749,7 +798,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         uint32_t off[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          off[k] = ((on_bits >> k & 1) && tap.inside && !DFA3D_DIAG(diag, 32)) ? (uint32_t)(((pg.key[k] * Md + md) * D + db) * (int)sizeof(T)) : kNoRow;
+          off[k] = ((on_bits >> k & 1) && tap.inside && !DFA3D_DIAG(args<T>()->diag, 32)) ? (uint32_t)(((pg.key[k] * Md + md) * D + db) * (int)sizeof(T)) : kNoRow;
         taps.ask(dist_r, off, D);
       } else if (score_in != nullptr) {                      // uniform
         const T *si = score_in + (size_t)gp * 4;
@@ -786,6 +835,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       // ---------------- phase X: scores and corner weights of pass t, prepare pass t + 1 ----------------
       float4 pw = make_float4(0, 0, 0, 0);                  // corner weights of this thread's point
       if (valid) {
+        const int D = args<T>()->D;
         const float hh = 1 - nxt.lh, hw = 1 - nxt.lw;
         const int d0 = (int)(nxt.bits >> 16) - 1, db = min(max(d0, 0), max(D - 2, 0));
         const bool lo_ok = (nxt.bits & 32u) != 0, hi_ok = (nxt.bits & 64u) != 0;
@@ -823,6 +873,12 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       lds_barrier();
       CT_MARK(3);
       // ---------------- phase Y: place pass t, finish pass t - 1 ----------------
+      const auto ar = args<T>();
+      const int C = ar->C, D = ar->D, Q = ar->Q, M = ar->M, gl_stride = ar->gl_stride;
+      const T *grad_out = ar->grad_out, *grad_score_in = ar->grad_score_in;
+      float *grad_loc = ar->grad_loc, *grad_attn = ar->grad_attn, *grad_score_out = ar->grad_score_out;
+      const float *grad_wu = ar->grad_wu;
+      const uint32_t slice = (uint32_t)Q * (uint32_t)M * (uint32_t)(ar->L * ar->P);             // points of a batch element
       const bool straight = valid && C == ROW;               // uniform
       if (straight) {
         // The grad_out rows of pass t: whole rows go straight into LDS, 16 bytes per lane, without a register in between,
@@ -850,7 +906,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         if (now.bits & 128u) s_slot[offs[(now.bits >> 8) & 63] + rank_now] = (uint16_t)pslot;
       }
       CT_MARK(4);
-      if (valid1 && !DFA3D_DIAG(diag, 512)) {                // (development builds: cost of phase C)
+      if (valid1 && !DFA3D_DIAG(args<T>()->diag, 512)) {                // (development builds: cost of phase C)
         const ItemGeom &q = s_geom[slot_of_item(it1)];
         const int gH = __builtin_amdgcn_readfirstlane(q.H), gW = __builtin_amdgcn_readfirstlane(q.W), gDd = __builtin_amdgcn_readfirstlane(q.Dd);
         const int gb = __builtin_amdgcn_readfirstlane(q.b);
@@ -887,7 +943,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
             for (int k = 0; k < 4; ++k) gs[k] += Elem<T>::ld(gi + k);
           }
           if (grad_wu != nullptr) {       // weight_update = sum over points of attn * mean corner score
-            const float gw = grad_wu[div_lp.div(cur.gp)] * 0.25f;
+            const float gw = grad_wu[ar->div_lp.div(cur.gp)] * 0.25f;
             ga += gw * (cur.sc[0] + cur.sc[1] + cur.sc[2] + cur.sc[3]);
 #pragma unroll
             for (int k = 0; k < 4; ++k) gs[k] += gw * a;
@@ -904,7 +960,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           // The taps: read, add, compare-and-swap, all eight in flight together; a tap that met another one tries again
           // with what it found, and after a few rounds (many points on one pixel and depth) the float atomic ends it.  A tap
           // that does not exist adds zero to a word nearby: the four pixels always lie in the tile, the bins are clamped.
-          if (live && !DFA3D_DIAG(diag, 2)) {
+          if (live && !DFA3D_DIAG(args<T>()->diag, 2)) {
             uint32_t *gdw = reinterpret_cast<uint32_t *>(gd);
             const int row0 = (ccy * TW + ccx) * D, lo_at = max(tap.d0, 0), hi_at = min(tap.d0 + 1, D - 1);
             const float w_lo = tap.lo_ok ? tap.hd : 0.f, w_hi = tap.hi_ok ? tap.ld : 0.f;
@@ -950,7 +1006,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       }
       // The staged rows must have come (the barrier orders LDS accesses only), the two stores after them need not have.
       if (straight) {
-        if (valid1 && !DFA3D_DIAG(diag, 512)) wait_for_all_but_two(); else wait_for_loads();
+        if (valid1 && !DFA3D_DIAG(args<T>()->diag, 512)) wait_for_all_but_two(); else wait_for_loads();
       }
       cur = now;
       CT_MARK(5);
@@ -972,22 +1028,18 @@ bool cell_kernel_applies(int C, int ty, int tx) { return C <= 64 && (C & 3) == 0
 template <typename T, int VEC, int LPR>
 static hipError_t launch_cell_cfg(const BwdArgs &a, const BinWorkspace &ws, size_t lds, int grid, float *gd_heads,
                                   hipStream_t stream) {
-  const FastDiv div_lp((uint32_t)(a.L * a.P));
-  if (a.dist != nullptr) {
-    hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, true>), dim3(grid), dim3(kWalkers + cell_pass(LPR)), lds, stream, ws, (const T *)a.value,
-                       (const T *)a.dist, (const T *)nullptr, (const T *)a.grad_out, (const T *)a.grad_score_in,
-                       a.grad_value, gd_heads != nullptr ? (void *)gd_heads : a.grad_dist, (float *)a.grad_loc,
-                       a.grad_loc_stride, (float *)a.grad_attn, (float *)nullptr, (const float *)a.grad_weight_update,
-                       a.dist_heads == 1 ? 1 : a.M, (a.dist_heads == 1 && gd_heads == nullptr) ? 1 : a.M, a.B, a.S, a.M,
-                       a.C, a.D, a.L, a.Q, a.P, div_lp, (a.grad_bf16 ? 1 : 0) | ((a.grad_bf16 && gd_heads == nullptr) ? 2 : 0)
-                       DFA3D_DIAG_ARG(a));
-  } else {
-    hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, false>), dim3(grid), dim3(kWalkers + cell_pass(LPR)), lds, stream, ws, (const T *)a.value,
-                       (const T *)nullptr, (const T *)a.score_in, (const T *)a.grad_out, (const T *)nullptr,
-                       a.grad_value, (void *)nullptr, (float *)a.grad_loc, a.grad_loc_stride, (float *)a.grad_attn,
-                       (float *)a.grad_score_out, (const float *)nullptr, a.M, a.M, a.B, a.S, a.M, a.C, 0, a.L, a.Q, a.P,
-                       div_lp, 0 DFA3D_DIAG_ARG(a));
-  }
+  const bool fused = a.dist != nullptr, one = a.dist_heads == 1;
+  const CellArgs<T> c = {ws, (const T *)a.value, (const T *)a.dist, fused ? nullptr : (const T *)a.score_in, (const T *)a.grad_out,
+                         fused ? (const T *)a.grad_score_in : nullptr, a.grad_value, gd_heads != nullptr ? (void *)gd_heads : a.grad_dist,
+                         (float *)a.grad_loc, (float *)a.grad_attn, fused ? nullptr : (float *)a.grad_score_out,
+                         fused ? (const float *)a.grad_weight_update : nullptr, a.grad_loc_stride,
+                         fused && one ? 1 : a.M, fused && one && gd_heads == nullptr ? 1 : a.M,
+                         a.B, a.S, a.M, a.C, fused ? a.D : 0, a.L, a.Q, a.P, FastDiv((uint32_t)(a.L * a.P)),
+                         !fused ? 0 : (a.grad_bf16 ? 1 : 0) | (a.grad_bf16 && gd_heads == nullptr ? 2 : 0)
+                         DFA3D_DIAG_ARG(a)};
+  const dim3 block(kWalkers + cell_pass(LPR));
+  if (fused) hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, true>), dim3(grid), block, lds, stream, c);
+  else hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, false>), dim3(grid), block, lds, stream, c);
   return hipGetLastError();
 }
 
