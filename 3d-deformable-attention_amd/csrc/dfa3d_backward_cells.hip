@@ -957,11 +957,9 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           const u32x3 g3 = {__float_as_uint(gx), __float_as_uint(gy), __float_as_uint(gz * (float)gDd)};
           __builtin_amdgcn_raw_buffer_store_b96(g3, gl_r, gl_off, 0, 0);
           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ga), ga_r, ga_off, 0, 0);
-          // The taps: read, add, compare-and-swap, all eight in flight together; a tap that met another one tries again
-          // with what it found, and after a few rounds (many points on one pixel and depth) the float atomic ends it.  A tap
-          // that does not exist adds zero to a word nearby: the four pixels always lie in the tile, the bins are clamped.
+          // The taps.  One that does not exist adds zero to a word nearby: the four pixels always lie in the tile, the bins
+          // are clamped.
           if (live && !DFA3D_DIAG(args<T>()->diag, 2)) {
-            uint32_t *gdw = reinterpret_cast<uint32_t *>(gd);
             const int row0 = (ccy * TW + ccx) * D, lo_at = max(tap.d0, 0), hi_at = min(tap.d0 + 1, D - 1);
             const float w_lo = tap.lo_ok ? tap.hd : 0.f, w_hi = tap.hi_ok ? tap.ld : 0.f;
             int at[8];
@@ -972,26 +970,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
               at[2 * k] = row + lo_at; at[2 * k + 1] = row + hi_at;
               tv[2 * k] = tap.lo_ok ? w_lo * gs[k] : 0.f; tv[2 * k + 1] = tap.hi_ok ? w_hi * gs[k] : 0.f;
             }
-            uint32_t old[8], got[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) old[j] = gdw[at[j]];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) got[j] = atomicCAS(gdw + at[j], old[j], __float_as_uint(__uint_as_float(old[j]) + tv[j]));
-            unsigned again = 0;                         // bit j: tap j is still to be added
-#pragma unroll
-            for (int j = 0; j < 8; ++j) again |= got[j] != old[j] ? 1u << j : 0u;
-            for (int round = 0; again != 0 && round < 4; ++round) {
-#pragma unroll
-              for (int j = 0; j < 8; ++j) {
-                old[j] = got[j];
-                if (again >> j & 1) got[j] = atomicCAS(gdw + at[j], old[j], __float_as_uint(__uint_as_float(old[j]) + tv[j]));
-              }
-#pragma unroll
-              for (int j = 0; j < 8; ++j) again &= got[j] == old[j] ? ~(1u << j) : ~0u;
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-              if (again >> j & 1) atomicAdd(gd + at[j], tv[j]);
+            lds_add_taps(gd, at, tv);
           }
         } else {
           const u32x2 g2 = {__float_as_uint(gx), __float_as_uint(gy)};

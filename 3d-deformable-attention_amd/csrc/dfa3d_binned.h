@@ -232,6 +232,9 @@ template <int VEC> __device__ __forceinline__ void lds_ld(const float *p, float 
 // The eight depth taps of a point added to an LDS tile of floats: read, add, compare-and-swap, all eight in flight
 // together; a tap that met another one tries again with what it found, and after a few rounds (many points on one pixel
 // and depth) the float atomic ends it.  The LDS float atomic alone retires 0.33 lanes per clock and CU, this 2.9.
+// A further round swaps at all eight words again, so that all are in flight together: where a tap is done, a value that was
+// found there is replaced by itself.  With a branch around each of them the round waited for one after the other: tile
+// kernel 1185 -> 1153 us at the base shape, 4366 -> 4251 us dense, 117.3 -> 112.6 us small.
 __device__ __forceinline__ void lds_add_taps(float *tile, const int (&at)[8], const float (&tv)[8]) {
   uint32_t *words = reinterpret_cast<uint32_t *>(tile);
   uint32_t old[8], got[8];
@@ -246,7 +249,7 @@ __device__ __forceinline__ void lds_add_taps(float *tile, const int (&at)[8], co
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       old[j] = got[j];
-      if (again >> j & 1) got[j] = atomicCAS(words + at[j], old[j], __float_as_uint(__uint_as_float(old[j]) + tv[j]));
+      got[j] = atomicCAS(words + at[j], old[j], (again >> j & 1) ? __float_as_uint(__uint_as_float(old[j]) + tv[j]) : old[j]);
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) again &= got[j] == old[j] ? ~(1u << j) : ~0u;
