@@ -31,6 +31,8 @@
 // clock and CU, read + compare-and-swap 2.9 (and a tap is complete when its phase ends, which the flush relies on).
 //
 // Semantics are those of bwd_attention_kernel (dfa3d_backward.hip holds the formulas and the reference lines).
+#include <type_traits>
+
 #include "dfa3d_binned.h"
 
 namespace dfa3d {
@@ -157,6 +159,17 @@ __device__ __forceinline__ float quad_corner_sum(float d0, float d1, float d2, f
   return keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(send), 0x4E, 0xF, 0xF, true));               // quad_perm [2,3,0,1]
 }
 
+// Where the 16-byte piece `piece` of staged row `row` lies, in bytes.  Of 2-byte elements the pieces of a row lie in an order that
+// depends on the row, so that the same piece of eight neighbouring rows falls on different banks: a lane that takes a whole row
+// (WholeRow) reads them one after the other, as its neighbours do with theirs.
+template <typename T, int ROWB> __device__ __forceinline__ int piece_at(int row, int piece) {
+  if constexpr (sizeof(T) == 2) {
+    constexpr int N = ROWB / 16, SH = ROWB >= 128 ? 0 : ROWB == 64 ? 1 : 2;
+    piece ^= (row >> SH) & (N - 1);
+  }
+  return row * ROWB + 16 * piece;
+}
+
 // The channels of one lane of a row of C elements, in NG groups of four.  Rows of 4-byte elements: group g covers
 // channels 4 (LPR g + cl) .. + 3, so that the lanes of a row read whole 64-byte pieces together; 2-byte elements: VEC
 // consecutive channels.  A group beyond C reads as zero and is never written.
@@ -203,29 +216,95 @@ template <typename T, int VEC, int LPR> struct LaneChannels {
     }
   }
   // the same lane's place in a row staged in LDS
-  __device__ __forceinline__ void put(T *row, const Raw &r) const {
+  static constexpr int ROWB = VEC * LPR * (int)sizeof(T);
+  __device__ __forceinline__ void put(unsigned char *rows, int row, int cl, const Raw &r) const {
+    if constexpr (sizeof(T) == 4) {
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      if constexpr (sizeof(T) == 4) *reinterpret_cast<uint4 *>(row + first[g]) = make_uint4(r.w[4 * g], r.w[4 * g + 1], r.w[4 * g + 2], r.w[4 * g + 3]);
-      else *reinterpret_cast<uint2 *>(row + first[g]) = make_uint2(r.w[2 * g], r.w[2 * g + 1]);
+      for (int g = 0; g < NG; ++g)
+        *reinterpret_cast<uint4 *>(rows + piece_at<T, ROWB>(row, LPR * g + cl)) = make_uint4(r.w[4 * g], r.w[4 * g + 1], r.w[4 * g + 2], r.w[4 * g + 3]);
+    } else if constexpr (VEC == 8) {
+      *reinterpret_cast<uint4 *>(rows + piece_at<T, ROWB>(row, cl)) = make_uint4(r.w[0], r.w[1], r.w[2], r.w[3]);
+    } else {
+      *reinterpret_cast<uint2 *>(rows + piece_at<T, ROWB>(row, cl >> 1) + 8 * (cl & 1)) = make_uint2(r.w[0], r.w[1]);
     }
   }
-  __device__ __forceinline__ void get(const T *row, Raw &r) const {
+  __device__ __forceinline__ void get(const unsigned char *rows, int row, int cl, Raw &r) const {
     if constexpr (sizeof(T) == 4) {
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
-        const uint4 t = *reinterpret_cast<const uint4 *>(row + first[g]);
+        const uint4 t = *reinterpret_cast<const uint4 *>(rows + piece_at<T, ROWB>(row, LPR * g + cl));
         r.w[4 * g] = t.x; r.w[4 * g + 1] = t.y; r.w[4 * g + 2] = t.z; r.w[4 * g + 3] = t.w;
       }
     } else if constexpr (VEC == 8) {
-      const uint4 t = *reinterpret_cast<const uint4 *>(row + first[0]);
+      const uint4 t = *reinterpret_cast<const uint4 *>(rows + piece_at<T, ROWB>(row, cl));
       r.w[0] = t.x; r.w[1] = t.y; r.w[2] = t.z; r.w[3] = t.w;
     } else {
-      const uint2 t = *reinterpret_cast<const uint2 *>(row + first[0]);
+      const uint2 t = *reinterpret_cast<const uint2 *>(rows + piece_at<T, ROWB>(row, cl >> 1) + 8 * (cl & 1));
       r.w[0] = t.x; r.w[1] = t.y;
     }
   }
 };
+
+// The other way to hold rows, of 2-byte elements: each lane of four takes all that the four hold of one row (with eight lanes to
+// a row: of their half of it), in the order of the four lanes' Raw words.
+template <typename T, int VEC, int LPR> struct WholeRow {
+  static constexpr int W = VEC * 2, ROWB = VEC * LPR * 2;      // words; bytes of a row
+  uint32_t w[W];
+  __device__ __forceinline__ void get(const unsigned char *rows, int row, int half) {
+#pragma unroll
+    for (int i = 0; i < W / 4; ++i) {
+      const uint4 t = *reinterpret_cast<const uint4 *>(rows + piece_at<T, ROWB>(row, 4 * half + i));
+      w[4 * i] = t.x; w[4 * i + 1] = t.y; w[4 * i + 2] = t.z; w[4 * i + 3] = t.w;
+    }
+  }
+};
+// x[k] of lane b of four becomes x[b] of lane k
+__device__ __forceinline__ void quad_transpose(uint32_t (&x)[4], bool odd, bool upper) {
+#pragma unroll
+  for (int k = 0; k < 4; k += 2) {
+    const uint32_t got = __builtin_amdgcn_mov_dpp(odd ? x[k] : x[k + 1], 0xB1, 0xF, 0xF, true);      // quad_perm [1,0,3,2]
+    x[k] = odd ? got : x[k];
+    x[k + 1] = odd ? x[k + 1] : got;
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const uint32_t got = __builtin_amdgcn_mov_dpp(upper ? x[k] : x[k + 2], 0x4E, 0xF, 0xF, true);    // quad_perm [2,3,0,1]
+    x[k] = upper ? got : x[k];
+    x[k + 2] = upper ? x[k + 2] : got;
+  }
+}
+// the four corners' rows, as the lanes of a group hold them, to one corner's row per lane
+template <typename T, int VEC, int LPR>
+__device__ __forceinline__ void whole_rows(const typename LaneChannels<T, VEC, LPR>::Raw (&r)[4], int cl, WholeRow<T, VEC, LPR> &o) {
+#pragma unroll
+  for (int e = 0; e < VEC / 2; ++e) {
+    uint32_t x[4] = {r[0].w[e], r[1].w[e], r[2].w[e], r[3].w[e]};
+    quad_transpose(x, (cl & 1) != 0, (cl & 2) != 0);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) o.w[VEC / 2 * b + e] = x[b];
+  }
+}
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// Dot products of the four corners' rows (a corner per lane of four) with four points' rows (a point per lane): lane j gets those
+// of point j.  Products of bfloat16 numbers are exact in float; up to four chains of sums, added in pairs.
+template <typename T, int VEC, int LPR>
+__device__ __forceinline__ f4 corner_dots(const WholeRow<T, VEC, LPR> &v, const WholeRow<T, VEC, LPR> &g) {
+  constexpr int W = WholeRow<T, VEC, LPR>::W;
+  f4 half[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    f4 d[2] = {(f4){0, 0, 0, 0}, (f4){0, 0, 0, 0}};
+#pragma unroll
+    for (int i = 0; i < W / 4; ++i) {
+      const int k = h * (W / 2) + 2 * i;
+      const u32x2 a = {v.w[k], v.w[k + 1]}, b = {g.w[k], g.w[k + 1]};
+      d[i & 1] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), d[i & 1], 0, 0, 0);
+    }
+    half[h] = d[0] + d[1];
+  }
+  return half[0] + half[1];
+}
 
 // The two taps (bins db, db + 1) of each of a point's four corners, asked for one phase before they are looked at.
 template <typename T> struct TapsInFlight {
@@ -310,7 +389,6 @@ template <typename T, int VEC, int LPR, bool FUSED>
 __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_kernel(CellArgs<T>) {
   constexpr int PP = cell_pass(LPR), BLOCK = kWalkers + PP, TX = kCellTX, TW = TX + 1, ROW = VEC * LPR;
   constexpr int GPW = kWave / LPR, CELLS = 4 * GPW, ROWS = GPW / TX;      // cells and tile rows per walker wavefront
-  typedef float f4 __attribute__((ext_vector_type(4)));
   extern __shared__ __align__(16) float smem[];
   __shared__ int s_lv[4][DFA3D_MAX_LEVELS];              // the plan's level tables: H, W, Dd, first key
   __shared__ CellFetch s_fetch;                           // the fetching thread's queue state, between its turns
@@ -332,7 +410,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
   // through the other role's code with all lanes switched off, because barriers count wavefronts, not lanes.
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const bool walker = wave < 4;
-  T *gstage = reinterpret_cast<T *>(smem + lay.gstage);
+  unsigned char *gstage = reinterpret_cast<unsigned char *>(smem + lay.gstage);
   float *gd = smem + lay.gd, *dots = smem + lay.dots, *cross = smem + lay.cross, *rim = smem + lay.rim;
   uint16_t *s_slot = reinterpret_cast<uint16_t *>(smem + lay.sslot);
   int *cnt = reinterpret_cast<int *>(smem + lay.cnt), *offs = reinterpret_cast<int *>(smem + lay.offs);
@@ -563,14 +641,64 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 #pragma unroll
         for (int j = 0; j < IN_FLIGHT; ++j) o.ch.load(go_r, offs_of[(j0 + j) * GPW + o.group], gg[j]);
 #pragma unroll
-        for (int j = 0; j < IN_FLIGHT; ++j) o.ch.put(gstage + (wave * kRows + (j0 + j) * GPW + o.group) * ROW, gg[j]);
+        for (int j = 0; j < IN_FLIGHT; ++j) o.ch.put(gstage, wave * kRows + (j0 + j) * GPW + o.group, o.cl, gg[j]);
       }
     };
-    // phase X: walk the lists of the staged pass, one point per step and group; the next step's row and weights and the
-    // slot after that are asked for while this step's sums are formed, so that no LDS round trip is waited for with
-    // nothing to do.  A group whose list has ended goes on with the row of zeros and weight zero (the matrix
-    // instructions ignore the execution mask).
-    auto walk = [&](const float (&v)[4][VEC], f4 (&acc)[VEC]) {
+    // phase X: walk the lists of the staged pass.  A group whose list has ended goes on with the row of zeros and weight zero
+    // (the matrix instructions ignore the execution mask).
+    // 2-byte elements: four points per step and group.  Each lane of four takes the row of one of them for the dots, which are
+    // products of matrices then (v_mfma_f32_4x4x4, four channels deep), and all four take all of them for the sums.
+    // The step takes a third of the vector instructions that four steps of one point do, for two and a half times the reads
+    // from LDS: base shape 1061 -> 1040 us.  With 4-byte elements, where a matrix instruction is one channel deep and a row twice
+    // as long, it lost: plain attention 209 -> 227 us, base shape 1194 -> 1277.
+    auto walk_fours = [&](const WholeRow<T, VEC, LPR> &v, f4 (&acc)[VEC]) {
+      const Owner o = owner();
+      const int corner = o.cl & 3, cell = o.crow * TX + o.ccol;
+      const bool cell_ok = o.crow < TY;
+      const int beg = cell_ok ? offs[cell] : 0, n = cell_ok ? offs[cell + 1] - beg : 0;
+      int mine = s_slot[corner < n ? beg + corner : PP];
+      for (int t = 0; __any(t < n); t += 4) {
+        WholeRow<T, VEC, LPR> g;
+        g.get(gstage, mine, o.cl >> 2);
+        int s[4];
+        float w[4];
+        s[0] = __builtin_amdgcn_mov_dpp(mine, 0x00, 0xF, 0xF, true);      // quad_perm [k,k,k,k]
+        s[1] = __builtin_amdgcn_mov_dpp(mine, 0x55, 0xF, 0xF, true);
+        s[2] = __builtin_amdgcn_mov_dpp(mine, 0xAA, 0xF, 0xF, true);
+        s[3] = __builtin_amdgcn_mov_dpp(mine, 0xFF, 0xF, 0xF, true);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = dots[s[k] * 4 + corner];
+        const int ahead = s_slot[t + 4 + corner < n ? beg + t + 4 + corner : PP];
+        f4 d = corner_dots<T, VEC, LPR>(v, g);
+        __builtin_amdgcn_sched_barrier(0);                  // (the whole rows' registers are free)
+        typedef typename LaneChannels<T, VEC, LPR>::Raw Raw;
+        if (LPR == 8) {                                     // the other half of the channels
+#pragma unroll
+          for (int k = 0; k < 4; ++k) d[k] += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(d[k]), 0x104, 0xF, 0xF, true));   // row_shl:4
+        }
+#pragma unroll
+        for (int k0 = 0; k0 < 4; k0 += 2) {
+          Raw r[2];
+#pragma unroll
+          for (int k = 0; k < 2; ++k) o.ch.get(gstage, s[k0 + k], o.cl, r[k]);
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            float gk[VEC];
+            LaneChannels<T, VEC, LPR>::to_float(r[k], gk);
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) acc[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(w[k0 + k], gk[i], acc[i], 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        wave_lds_handover();                                // the weights have been read: the dots take their place
+        if (t + corner < n && o.cl < 4) *reinterpret_cast<float4 *>(dots + mine * 4) = make_float4(d[0], d[1], d[2], d[3]);
+        mine = ahead;
+      }
+    };
+
+    // 4-byte elements: one point per step and group; the next step's row and weights and the slot after that are asked for while
+    // this step's sums are formed, so that no LDS round trip is waited for with nothing to do.
+    auto walk_ones = [&](const float (&v)[4][VEC], f4 (&acc)[VEC]) {
       const Owner o = owner();
       const int corner = o.cl & 3, cell = o.crow * TX + o.ccol;
       const bool cell_ok = o.crow < TY;
@@ -578,12 +706,12 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       int s0 = s_slot[n > 0 ? beg : PP], s1 = s_slot[n > 1 ? beg + 1 : PP];
       typedef typename LaneChannels<T, VEC, LPR>::Raw Raw;
       Raw r0;
-      o.ch.get(gstage + s0 * ROW, r0);
+      o.ch.get(gstage, s0, o.cl, r0);
       float w0 = dots[s0 * 4 + corner];
       for (int t = 0; __any(t < n); ++t) {
         const int s2 = s_slot[t + 2 < n ? beg + t + 2 : PP];
         Raw r1;
-        o.ch.get(gstage + s1 * ROW, r1);
+        o.ch.get(gstage, s1, o.cl, r1);
         const float w1 = dots[s1 * 4 + corner];
         float d[4], g0[VEC];
         LaneChannels<T, VEC, LPR>::to_float(r0, g0);
@@ -600,6 +728,11 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         if (t < n && o.cl < 4) dots[s0 * 4 + corner] = dot;
         s0 = s1; s1 = s2; w0 = w1; r0 = r1;
       }
+    };
+
+    auto walk = [&](const auto &v, f4 (&acc)[VEC]) {
+      if constexpr (sizeof(T) == 4) walk_ones(v, acc);
+      else walk_fours(v, acc);
     };
 
     if (g.bin >= 0) {
@@ -707,9 +840,13 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           if (r0 + ROWS >= TY) put_rim(q, TW, TW);
         }
         if (done) break;
-        float v[4][VEC];
+        typename std::conditional<sizeof(T) == 4, float[4][VEC], WholeRow<T, VEC, LPR>>::type v;      // the four value rows
+        if constexpr (sizeof(T) == 4) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) LaneChannels<T, VEC, LPR>::to_float(vr[k], v[k]);
+          for (int k = 0; k < 4; ++k) LaneChannels<T, VEC, LPR>::to_float(vr[k], v[k]);
+        } else {
+          whole_rows<T, VEC, LPR>(vr, owner().cl, v);
+        }
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = (f4){0, 0, 0, 0};
         CT_MARK(5);
@@ -892,7 +1029,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 #pragma unroll
         for (int j = 0; j < kWave / RPI; ++j) row[j] = goff[(turn & 1) * PP + row0 + j * RPI + l / RL];
 #pragma unroll
-        for (int j = 0; j < kWave / RPI; ++j) load_to_lds16(go_r, gstage + (row0 + j * RPI) * ROW, row[j] + 16 * (l % RL));
+        for (int j = 0; j < kWave / RPI; ++j) load_to_lds16(go_r, gstage + (row0 + j * RPI) * RL * 16, row[j] + piece_at<T, RL * 16>(j * RPI + l / RL, l % RL) % (RL * 16));
       }
       const float4 d4 = *reinterpret_cast<const float4 *>(dots + pslot * 4);       // of pass t - 1, before its place is taken
       if (valid) {
