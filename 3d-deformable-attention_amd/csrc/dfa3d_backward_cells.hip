@@ -15,12 +15,12 @@
 //
 // The 8 wavefronts of a workgroup have two roles.  "Walkers" (wavefronts 0-3, one or two tile rows of 8 cells each)
 // walk the cells' lists; "pointers" (wavefronts 4-7, one point of the pass per thread) do everything that is per point:
-// geometry, depth taps, corner weights, the sort, bringing its grad_out row to LDS, and afterwards the point's gradients
+// geometry, depth taps, corner weights, the sort, and afterwards the point's gradients
 // and its grad_dist taps into the LDS depth tile.  The roles meet at two barriers per turn and
 // otherwise overlap.  Turns follow one another without a gap, whatever item their passes belong to (pass t: one of
 // the item's passes), so that an item of a single pass costs a single turn:
 //   phase X(t):  walkers: walk(t-1)        pointers: scores and corner weights of t, prepare(t+1)
-//   phase Y(t):  walkers: next to nothing  pointers: stage(t), place(t) (scan + sorted slots), finish(t-1)
+//   phase Y(t):  walkers: stage(t)         pointers: place(t) (scan + sorted slots), finish(t-1)
 // and where pass t-1 was its item's last:
 //   Y(t):    walkers put the old item's corner sums together in registers (neighbouring cells are neighbouring lane groups;
 //            sums that cross into the next wavefront's rows, and the rim's, go through a few rows of LDS) and ask for the
@@ -337,8 +337,8 @@ template <typename T> struct TapsInFlight {
 };
 
 // 16 bytes per lane from a buffer to consecutive LDS addresses (`lds`: the wavefront's first byte).  Written out because
-// behind the builtin the compiler waits for the data before the next LDS read of any kind; here wait_for_loads() /
-// wait_for_all_but_two() do, when the phase ends.  (The compiler does not count these loads: where it waits for an older
+// behind the builtin the compiler waits for the data before the next LDS read of any kind; here
+// wait_for_loads() does, when the phase ends.  (The compiler does not count these loads: where it waits for an older
 // one, it waits for more than it has to, never for less.)
 __device__ __forceinline__ void load_to_lds16(rsrc_t r, const void *lds, uint32_t off) {
 #ifdef __HIP_DEVICE_COMPILE__
@@ -349,7 +349,6 @@ __device__ __forceinline__ void load_to_lds16(rsrc_t r, const void *lds, uint32_
 #endif
 }
 __device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }           // vmcnt(0)
-__device__ __forceinline__ void wait_for_all_but_two() { __builtin_amdgcn_s_waitcnt(0x0F72); }     // vmcnt(2)
 
 // The kernel's arguments.  They are read from the constant segment anew in every phase (args()): there are more of them, and
 // of the numbers that follow from them, than scalar registers.  Passed one by one they were kept from turn to turn, at the
@@ -626,12 +625,32 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       asm volatile("" : "+v"(i));
       if (i < (unsigned)CELLS) cnt[(turn + 2) % 3 * CELLS + i] = 0;
     };
-    // phase Y: the grad_out rows of the pass, where they cannot go straight from memory to LDS (then the pointers see to it)
+    // phase Y: the grad_out rows of the pass come to LDS; they must be there before the phase ends (wait_for_loads()).  Whole rows
+    // go straight there, 16 bytes per lane, without a register in between.  (The pointers, whose work in phase Y is the
+    // longer one, brought them before: tile kernel 1158 -> 1121 us at the base shape, bfloat16 1045 -> 1022, dense 4245 -> 4160,
+    // small 111 -> 106.)
     auto stage = [&]() {
       const auto a = args<T>();
       const int Q = a->Q, M = a->M, C = a->C;
       const T *grad_out = a->grad_out;
-      if (C == ROW) return;                                  // uniform
+      if (C == ROW) {                                        // uniform
+        constexpr int RL = ROW * (int)sizeof(T) / 16, RPI = kWave / RL, N = kRows / RPI, NB = N < 4 ? N : 4;      // lanes per row, rows per instruction
+        const rsrc_t go_r = make_rsrc(grad_out + (size_t)g.b * Q * M * C, (size_t)Q * M * C * sizeof(T));
+        const int row0 = wave * kRows;
+        unsigned l = lane;
+        asm volatile("" : "+v"(l));                          // (not worth registers from turn to turn)
+#pragma unroll
+        for (int j0 = 0; j0 < N; j0 += NB) {
+          uint32_t row[NB];
+#pragma unroll
+          for (int j = 0; j < NB; ++j) row[j] = goff[(turn & 1) * PP + row0 + (j0 + j) * RPI + l / RL];
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+            load_to_lds16(go_r, gstage + (row0 + (j0 + j) * RPI) * RL * 16, row[j] + piece_at<T, RL * 16>((j0 + j) * RPI + l / RL, l % RL) % (RL * 16));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        return;
+      }
       const Owner o = owner();
       const rsrc_t go_r = make_rsrc(grad_out + (size_t)g.b * Q * M * C, (size_t)Q * M * C * sizeof(T));
       const uint32_t *offs_of = goff + (turn & 1) * PP + wave * kRows;
@@ -789,6 +808,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           if (ROWS == 2) put_pixel(o, uniform(s_geom[slot_of_item(it - 1)]), u, o.crow < TY && o.group >= TX);   // the second row is complete
         }
         CT_MARK(3);
+        if (!done) stage();
         typename LaneChannels<T, VEC, LPR>::Raw vr[4];
         {
           // the four value rows of this group's cell (zero outside the map, when the cell is not part of the tile, or when
@@ -805,9 +825,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
             o.ch.load(value_r, ok ? (uint32_t)(((g.start + y * g.W + x) * M + g.m) * C * (int)sizeof(T)) : kNoRow, vr[k]);
           }
         }
-        if (!done) {
-          stage();
-        }
+        wait_for_loads();
         CT_MARK(6);
         lds_barrier();
         CT_MARK(4);
@@ -856,6 +874,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         CT_MARK(2);
         for (int base = PP; base < g.n_item; base += PP) {   // the item's further passes
           stage();
+          wait_for_loads();
           CT_MARK(6);
           lds_barrier();
           CT_MARK(4);
@@ -967,7 +986,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     bool valid1 = false, last1 = false, last2 = false;
     for (int turn = 0;; ++turn) {                            // uniform over the workgroup
       const bool valid = g.bin >= 0, last = valid && base + PP >= g.n_item;
-      const int it_now = it, b_now = g.b;
+      const int it_now = it;
       CT_MARK(0);
       // ---------------- phase X: scores and corner weights of pass t, prepare pass t + 1 ----------------
       float4 pw = make_float4(0, 0, 0, 0);                  // corner weights of this thread's point
@@ -1011,26 +1030,11 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       CT_MARK(3);
       // ---------------- phase Y: place pass t, finish pass t - 1 ----------------
       const auto ar = args<T>();
-      const int C = ar->C, D = ar->D, Q = ar->Q, M = ar->M, gl_stride = ar->gl_stride;
-      const T *grad_out = ar->grad_out, *grad_score_in = ar->grad_score_in;
+      const int D = ar->D, gl_stride = ar->gl_stride;
+      const T *grad_score_in = ar->grad_score_in;
       float *grad_loc = ar->grad_loc, *grad_attn = ar->grad_attn, *grad_score_out = ar->grad_score_out;
       const float *grad_wu = ar->grad_wu;
-      const uint32_t slice = (uint32_t)Q * (uint32_t)M * (uint32_t)(ar->L * ar->P);             // points of a batch element
-      const bool straight = valid && C == ROW;               // uniform
-      if (straight) {
-        // The grad_out rows of pass t: whole rows go straight into LDS, 16 bytes per lane, without a register in between,
-        // and arrive while this phase's other work is done.
-        constexpr int RL = ROW * (int)sizeof(T) / 16, RPI = kWave / RL;        // lanes per row, rows per instruction
-        const rsrc_t go_r = make_rsrc(grad_out + (size_t)b_now * Q * M * C, (size_t)Q * M * C * sizeof(T));
-        const int row0 = (wave - kWalkers / kWave) * kWave;
-        unsigned l = lane;
-        asm volatile("" : "+v"(l));                          // (not worth registers from turn to turn)
-        uint32_t row[kWave / RPI];
-#pragma unroll
-        for (int j = 0; j < kWave / RPI; ++j) row[j] = goff[(turn & 1) * PP + row0 + j * RPI + l / RL];
-#pragma unroll
-        for (int j = 0; j < kWave / RPI; ++j) load_to_lds16(go_r, gstage + (row0 + j * RPI) * RL * 16, row[j] + piece_at<T, RL * 16>(j * RPI + l / RL, l % RL) % (RL * 16));
-      }
+      const uint32_t slice = (uint32_t)ar->Q * (uint32_t)ar->M * (uint32_t)(ar->L * ar->P);      // points of a batch element
       const float4 d4 = *reinterpret_cast<const float4 *>(dots + pslot * 4);       // of pass t - 1, before its place is taken
       if (valid) {
         // exclusive prefix of the cell counters; every pointer wavefront computes it and writes the same numbers,
@@ -1119,10 +1123,6 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
             __builtin_amdgcn_raw_buffer_store_b128(g4, gs_r, live ? at * 16 : kNoRow, 0, 0);
           }
         }
-      }
-      // The staged rows must have come (the barrier orders LDS accesses only), the two stores after them need not have.
-      if (straight) {
-        if (valid1 && !DFA3D_DIAG(args<T>()->diag, 512)) wait_for_all_but_two(); else wait_for_loads();
       }
       cur = now;
       CT_MARK(5);
