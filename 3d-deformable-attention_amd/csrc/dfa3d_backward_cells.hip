@@ -354,6 +354,8 @@ __device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x
 // of the numbers that follow from them, than scalar registers.  Passed one by one they were kept from turn to turn, at the
 // cost of 98 others (float, 32 channels; 105 with bfloat16) that went to lanes of vector registers and came back one
 // instruction each.  Base shape, 15.4 M points: 1194 -> 1184 us, bfloat16 1160 -> 1100 us.
+// FRESH: read again at each use.  Stage 2 alone has fewer of them and keeps its 8 to 14 that do not fit (two-stage shape, 14.6 M
+// points: 1037 us against 1040 read anew, 2.6 M points of plain attention 214 against 217).
 template <typename T> struct CellArgs {
   BinWorkspace ws;
   const T *value, *dist, *score_in, *grad_out, *grad_score_in;
@@ -371,14 +373,14 @@ template <typename T> struct CellArgs {
 };
 #ifdef __HIP_DEVICE_COMPILE__
 template <typename T> using CellArgsPtr = const __attribute__((address_space(4))) CellArgs<T> *;
-template <typename T> __device__ __forceinline__ CellArgsPtr<T> args() {
+template <typename T, bool FRESH> __device__ __forceinline__ CellArgsPtr<T> args() {
   auto a = (CellArgsPtr<T>)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(a));
+  if (FRESH) asm volatile("" : "+s"(a));
   return a;
 }
 #else
 template <typename T> using CellArgsPtr = const CellArgs<T> *;
-template <typename T> __device__ CellArgsPtr<T> args();
+template <typename T, bool FRESH> __device__ CellArgsPtr<T> args();
 #endif
 
 // FUSED: both stages (depth scores recomputed from dist, grad_dist and the z gradient produced).
@@ -393,7 +395,8 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
   __shared__ CellFetch s_fetch;                           // the fetching thread's queue state, between its turns
   __shared__ ItemGeom s_geom[kItemSlots];                // items, decoded by the thread that fetches them
 
-  const auto a0 = args<T>();
+  const auto arg = []() { return args<T, FUSED>(); };
+  const auto a0 = arg();
   const BinWorkspace ws = a0->ws;
   const BinPlan &p = *ws.plan;
   if (__builtin_expect(p.bins_per_bm == 0, 0)) {
@@ -436,7 +439,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
   // divisions.  Pixels 1..TY-1 x 1..7 belong to no neighbour's halo: when the item writes its tile alone they are stored,
   // the others are added.
   auto flush_gd = [&](int which, int first, int threads) {
-    const auto a = args<T>();
+    const auto a = arg();
     const int D = a->D, S = a->S, M = a->M, Mg = a->Mg;
     void *grad_dist = a->grad_dist;
     const bool gd16 = (a->grad16 & 2) != 0;                // uniform
@@ -453,7 +456,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       for (int i = first >> sh; i < inner; i += threads >> sh) {
         const int ry = i / (TX - 1) + 1, rx = i % (TX - 1) + 1, r = ry * TW + rx;
         const int y = q.y0 + ry, x = q.x0 + rx;
-        const bool out = y < q.H && x < q.W && !DFA3D_DIAG(args<T>()->diag, 4);
+        const bool out = y < q.H && x < q.W && !DFA3D_DIAG(arg()->diag, 4);
         const uint32_t e0 = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D);
         for (int c = first & ((1 << sh) - 1); c < n; c += 1 << sh) {
           if (d4) {
@@ -482,7 +485,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         ry = i / TW; rx = i % TW;
       }
       const int r = ry * TW + rx, y = q.y0 + ry, x = q.x0 + rx;
-      const bool out = in_map(y, x, q.H, q.W) && !DFA3D_DIAG(args<T>()->diag, 4);
+      const bool out = in_map(y, x, q.H, q.W) && !DFA3D_DIAG(arg()->diag, 4);
       const uint32_t e0 = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D);
       for (int c = first & ((1 << sh) - 1); c < n; c += 1 << sh) {
         if (gd16) {
@@ -524,7 +527,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     auto owner = [&]() {
       unsigned l = lane;
       asm volatile("" : "+v"(l));
-      return Owner(l, wave, args<T>()->C);
+      return Owner(l, wave, arg()->C);
     };
     auto decode = [&](const int4 &item, const int4 &geo) {
       ItemGeom g;
@@ -553,13 +556,13 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     // halo: when the item writes its tile alone they are stored (grad_value is zero on entry, or the binning launches
     // cleared what is added to), else added.  Rim pixels go to their place in LDS, to be added by put_rim.
     auto put_pixel = [&](const Owner &o, const ItemGeom &q, const float (&u)[VEC], bool active) {
-      const auto a = args<T>();
+      const auto a = arg();
       const int S = a->S, M = a->M, C = a->C;
       const bool gv16 = (a->grad16 & 1) != 0;               // uniform
       void *grad_value = a->grad_value;
       const int y = q.y0 + o.crow, x = q.x0 + o.ccol;
       if (active && (o.crow == 0 || o.ccol == 0)) put_lds(o, rim + rim_index(o.crow, o.ccol, TY, TX) * ROW, u);
-      if (active && o.crow > 0 && o.ccol > 0 && y < q.H && x < q.W && !DFA3D_DIAG(args<T>()->diag, 4)) {
+      if (active && o.crow > 0 && o.ccol > 0 && y < q.H && x < q.W && !DFA3D_DIAG(arg()->diag, 4)) {
         char *gvalue_b = static_cast<char *>(grad_value) + (size_t)q.b * S * M * C * (gv16 ? 2 : 4);
         float *gvalue_f = reinterpret_cast<float *>(gvalue_b);
         const rsrc_t gvalue_r = make_rsrc(gvalue_b, (size_t)S * M * C * sizeof(float));
@@ -585,7 +588,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     };
     // Rim pixels [first, first + n) of item q, whose sums this wavefront left in LDS.
     auto put_rim = [&](const ItemGeom &q, int first, int n) {
-      const auto a = args<T>();
+      const auto a = arg();
       const int S = a->S, M = a->M, C = a->C;
       const bool gv16 = (a->grad16 & 1) != 0;               // uniform
       void *grad_value = a->grad_value;
@@ -600,7 +603,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         const int y = q.y0 + ry, x = q.x0 + rx;
         const float *from = rim + k * ROW + c;
         const float f0 = from[0], f1 = gv16 ? from[1] : 0.f;
-        if (c < C && in_map(y, x, q.H, q.W) && (f0 != 0 || f1 != 0) && !DFA3D_DIAG(args<T>()->diag, 4)) {
+        if (c < C && in_map(y, x, q.H, q.W) && (f0 != 0 || f1 != 0) && !DFA3D_DIAG(arg()->diag, 4)) {
           const uint32_t e = (uint32_t)(((q.start + y * q.W + x) * M + q.m) * C + c);
           if (gv16) atomic_add_bf16x2(gvalue_b + (size_t)e * 2, f0, f1);
           else scatter_add(gvalue_r, gvalue_f, e * 4, f0);
@@ -630,7 +633,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     // longer one, brought them before: tile kernel 1158 -> 1121 us at the base shape, bfloat16 1045 -> 1022, dense 4245 -> 4160,
     // small 111 -> 106.)
     auto stage = [&]() {
-      const auto a = args<T>();
+      const auto a = arg();
       const int Q = a->Q, M = a->M, C = a->C;
       const T *grad_out = a->grad_out;
       if (C == ROW) {                                        // uniform
@@ -772,7 +775,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         if (tid == 0 && !done) {
           CellFetch fetch = s_fetch;
           int4 rec, geo;
-          const BinWorkspace w = args<T>()->ws;
+          const BinWorkspace w = arg()->ws;
           fetch.advance(w, *w.plan, &rec, &geo);
           s_geom[slot_of_item(it + 3)] = decode(rec, geo);
           s_fetch = fetch;
@@ -813,7 +816,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         {
           // the four value rows of this group's cell (zero outside the map, when the cell is not part of the tile, or when
           // there is no item)
-          const auto a = args<T>();
+          const auto a = arg();
           const int S = a->S, M = a->M, C = a->C;
           const T *value = a->value;
           const Owner o = owner();
@@ -821,7 +824,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
             const int y = g.y0 + o.crow + (k >= 2 ? 1 : 0), x = g.x0 + o.ccol + ((k == 1 || k == 2) ? 1 : 0);
-            const bool ok = !done && o.crow < TY && in_map(y, x, g.H, g.W) && !DFA3D_DIAG(args<T>()->diag, 8);
+            const bool ok = !done && o.crow < TY && in_map(y, x, g.H, g.W) && !DFA3D_DIAG(arg()->diag, 8);
             o.ch.load(value_r, ok ? (uint32_t)(((g.start + y * g.W + x) * M + g.m) * C * (int)sizeof(T)) : kNoRow, vr[k]);
           }
         }
@@ -868,7 +871,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = (f4){0, 0, 0, 0};
         CT_MARK(5);
-        if (apart() && !DFA3D_DIAG(args<T>()->diag, 16)) walk(v, acc);
+        if (apart() && !DFA3D_DIAG(arg()->diag, 16)) walk(v, acc);
         CT_MARK(1);
         lds_barrier();
         CT_MARK(2);
@@ -880,7 +883,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           CT_MARK(4);
           ++turn;
           clear_counts();
-          if (apart() && !DFA3D_DIAG(args<T>()->diag, 16)) walk(v, acc);
+          if (apart() && !DFA3D_DIAG(arg()->diag, 16)) walk(v, acc);
           CT_MARK(1);
           lds_barrier();
           CT_MARK(2);
@@ -913,7 +916,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     float4 pre_rec = make_float4(0, 0, 0, 0);
     auto ask_records = [&]() {
       const int at = rec_bin >= 0 ? rec_seg + rec_base + min(pslot, rec_n - rec_base - 1) : 0;
-      const auto a = args<T>();
+      const auto a = arg();
       pre_gp = a->ws.entries[at];
       pre_rec = a->ws.recs[at];
     };
@@ -931,7 +934,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     };
     // geometry of this thread's point of pass A, its place in the sort, its grad_out row for the walkers; its taps are asked for
     auto prepare = [&](int pass) {
-      const auto ar = args<T>();
+      const auto ar = arg();
       const int D = ar->D, S = ar->S, M = ar->M, Md = ar->Md, Q = ar->Q, C = ar->C;
       const T *dist = ar->dist, *score_in = ar->score_in;
       const FastDiv div_lp = ar->div_lp;
@@ -954,7 +957,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         uint32_t off[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          off[k] = ((on_bits >> k & 1) && tap.inside && !DFA3D_DIAG(args<T>()->diag, 32)) ? (uint32_t)(((pg.key[k] * Md + md) * D + db) * (int)sizeof(T)) : kNoRow;
+          off[k] = ((on_bits >> k & 1) && tap.inside && !DFA3D_DIAG(arg()->diag, 32)) ? (uint32_t)(((pg.key[k] * Md + md) * D + db) * (int)sizeof(T)) : kNoRow;
         taps.ask(dist_r, off, D);
       } else if (score_in != nullptr) {                      // uniform
         const T *si = score_in + (size_t)gp * 4;
@@ -991,7 +994,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       // ---------------- phase X: scores and corner weights of pass t, prepare pass t + 1 ----------------
       float4 pw = make_float4(0, 0, 0, 0);                  // corner weights of this thread's point
       if (valid) {
-        const int D = args<T>()->D;
+        const int D = arg()->D;
         const float hh = 1 - nxt.lh, hw = 1 - nxt.lw;
         const int d0 = (int)(nxt.bits >> 16) - 1, db = min(max(d0, 0), max(D - 2, 0));
         const bool lo_ok = (nxt.bits & 32u) != 0, hi_ok = (nxt.bits & 64u) != 0;
@@ -1029,7 +1032,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       lds_barrier();
       CT_MARK(3);
       // ---------------- phase Y: place pass t, finish pass t - 1 ----------------
-      const auto ar = args<T>();
+      const auto ar = arg();
       const int D = ar->D, gl_stride = ar->gl_stride;
       const T *grad_score_in = ar->grad_score_in;
       float *grad_loc = ar->grad_loc, *grad_attn = ar->grad_attn, *grad_score_out = ar->grad_score_out;
@@ -1047,7 +1050,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         if (now.bits & 128u) s_slot[offs[(now.bits >> 8) & 63] + rank_now] = (uint16_t)pslot;
       }
       CT_MARK(4);
-      if (valid1 && !DFA3D_DIAG(args<T>()->diag, 512)) {                // (development builds: cost of phase C)
+      if (valid1 && !DFA3D_DIAG(arg()->diag, 512)) {                // (development builds: cost of phase C)
         const ItemGeom &q = s_geom[slot_of_item(it1)];
         const int gH = __builtin_amdgcn_readfirstlane(q.H), gW = __builtin_amdgcn_readfirstlane(q.W), gDd = __builtin_amdgcn_readfirstlane(q.Dd);
         const int gb = __builtin_amdgcn_readfirstlane(q.b);
@@ -1100,7 +1103,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ga), ga_r, ga_off, 0, 0);
           // The taps.  One that does not exist adds zero to a word nearby: the four pixels always lie in the tile, the bins
           // are clamped.
-          if (live && !DFA3D_DIAG(args<T>()->diag, 2)) {
+          if (live && !DFA3D_DIAG(arg()->diag, 2)) {
             const int row0 = (ccy * TW + ccx) * D, lo_at = max(tap.d0, 0), hi_at = min(tap.d0 + 1, D - 1);
             const float w_lo = tap.lo_ok ? tap.hd : 0.f, w_hi = tap.hi_ok ? tap.ld : 0.f;
             int at[8];
