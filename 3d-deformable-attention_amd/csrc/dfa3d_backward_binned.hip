@@ -450,61 +450,73 @@ __global__ __launch_bounds__(kFillThreads) void bin_fill_sorted_kernel(
 // to two levels and the kernel stores rows of that length (ClearArgs::stores); every other row of the two tensors only
 // ever receives atomic adds, or nothing: pixels on tile rims, pixels of tiles without points or with several work items,
 // keys outside every level.
-// A lane decides for one (batch, key, head) row; the wavefront then clears its 64 consecutive rows together, 16 bytes
-// per lane on consecutive addresses (the heads of a key share their fate, so whole lines go out).
-__device__ __forceinline__ void clear_rows_of_wave(char *base, size_t first_row, int row_bytes, bool clear_mine, int lane) {
-  char *dst = base + first_row * row_bytes;
-  if ((row_bytes & 15) == 0) {
-    const int n16 = row_bytes >> 4;
-    for (int c = lane; c < kWave * n16; c += kWave) {
-      const int r = c / n16;
-      if (__shfl((int)clear_mine, r, kWave)) *reinterpret_cast<uint4 *>(dst + (size_t)c * 16) = make_uint4(0, 0, 0, 0);
-    }
-  } else {
-    const int n4 = row_bytes >> 2;
-    for (int c = lane; c < kWave * n4; c += kWave) {
-      const int r = c / n4;
-      if (__shfl((int)clear_mine, r, kWave)) *reinterpret_cast<uint32_t *>(dst + (size_t)c * 4) = 0;
+// A lane decides for one (batch, key, head) row; the wavefront then clears its rows together, 16 bytes per lane on
+// consecutive addresses (the heads of a key share their fate, so whole lines go out).  Every division but that by the
+// map's width is by a number the host knows (FastDiv; a batch element has fewer than 2^28 rows): with the compiler's, in 64 bits
+// for the row and one per 16 bytes cleared, the vector units were what bound the launch.  The launch with the scan: base shape (1.48 M
+// rows of 128 and 256 bytes, 0.13 GB cleared) 40 -> 25 us; 3 levels from 37 x 67, 59 k rows of 80 and 236 bytes, 17 -> 7 us.
+struct ClearRows {                  // one tensor's rows
+  char *base;                       // nullptr: not this one
+  int row_bytes, pieces;            // a row in pieces of 16 bytes, or of 4 where rows are not made of those
+  FastDiv div_pieces;
+  ClearRows(void *at, int bytes) : base(static_cast<char *>(at)), row_bytes(bytes), pieces((bytes & 15) ? bytes >> 2 : bytes >> 4), div_pieces((uint32_t)(pieces > 0 ? pieces : 1)) {}
+  __device__ __forceinline__ void clear(size_t first_row, int rows, uint64_t which, int lane) const {
+    char *dst = base + first_row * row_bytes;
+    const bool wide = (row_bytes & 15) == 0;                 // uniform
+#pragma unroll 1
+    for (int c = lane; c < rows * pieces; c += kWave) {
+      if (!(which >> div_pieces.div(c) & 1)) continue;
+      if (wide) *reinterpret_cast<uint4 *>(dst + (size_t)c * 16) = make_uint4(0, 0, 0, 0);
+      else *reinterpret_cast<uint32_t *>(dst + (size_t)c * 4) = 0;
     }
   }
-}
-
+};
 struct ClearArgs {
-  char *grad_value, *grad_dist;     // either may be nullptr: not that one
-  int value_row_bytes, dist_row_bytes, B, S, M, L;
+  ClearRows value, dist;
+  int B, M, L;
   int stores;                       // the tile kernel stores what its item alone writes (else it adds everything)
+  int rows_of_b, rows_of_wave;      // rows of a batch element (S M); rows a wavefront takes at a time: 64, or 16 where that leaves CUs idle
+  FastDiv div_waves, div_m, div_ty, div_tx;      // by a batch element's turns of a wavefront; heads; tile edges
 };
 __device__ __forceinline__ void clear_unstored(const BinWorkspace &ws, const ClearArgs &ca, unsigned block, unsigned n_blocks) {
-  char *grad_value = ca.grad_value, *grad_dist = ca.grad_dist;
-  const int value_row_bytes = ca.value_row_bytes, dist_row_bytes = ca.dist_row_bytes;
-  const int B = ca.B, S = ca.S, M = ca.M, L = ca.L, stores = ca.stores;
+  __shared__ int4 s_level[DFA3D_MAX_LEVELS];                 // first key, keys, width, tiles across
+  __shared__ int s_base[DFA3D_MAX_LEVELS];
   const BinPlan &p = *ws.plan;
+  if (threadIdx.x < DFA3D_MAX_LEVELS) {
+    const int l = threadIdx.x;
+    s_level[l] = make_int4(p.start[l], p.H[l] * p.W[l], p.W[l], p.tiles_x[l]);
+    s_base[l] = p.level_base[l];
+  }
+  __syncthreads();
   const int nb = p.bins_per_bm, TY = p.ty, TX = p.tx, ch = chunk_of(ws, p);
-  const size_t rows = (size_t)B * S * M;
+  const bool decide = ca.stores != 0 && nb > 0 && p.disjoint != 0;
   const int lane = threadIdx.x % kWave;
-  // every wavefront takes 64 consecutive rows per turn; all its lanes stay in the loop (shuffles)
-  for (size_t i0 = ((size_t)block * blockDim.x + threadIdx.x) - lane; i0 < rows; i0 += (size_t)n_blocks * blockDim.x) {
-    const size_t i = i0 + lane;
-    bool clear_mine = i < rows;
-    if (clear_mine && stores && nb > 0 && p.disjoint != 0) {
-      const int m = (int)(i % M);
-      const size_t bs = i / M;
-      const int s = (int)(bs % S), b = (int)(bs / S);
-      for (int l = 0; l < L; ++l) {
-        const int local = s - p.start[l];
-        if (p.H[l] > 0 && local >= 0 && local < p.H[l] * p.W[l]) {
-          const int y = local / p.W[l], x = local - y * p.W[l];
-          if ((y + 1) % TY != 0 && (x + 1) % TX != 0) {       // the first tile starts at pixel -1
-            const int bin = slot_of(b, m, B, M) * nb + p.level_base[l] + ((y + 1) / TY) * p.tiles_x[l] + (x + 1) / TX;
-            const int c = ws.counts[bin];
-            clear_mine = items_of_bin(c, ch) != 1;            // exactly one work item stores this row
+  const unsigned waves_of_b = (unsigned)((ca.rows_of_b + ca.rows_of_wave - 1) / ca.rows_of_wave);
+  const unsigned step = n_blocks * (blockDim.x / kWave), n = waves_of_b * (unsigned)ca.B;
+  for (unsigned w = block * (blockDim.x / kWave) + threadIdx.x / kWave; w < n; w += step) {
+    const unsigned b = ca.div_waves.div(w);
+    const int first = (int)(w - b * waves_of_b) * ca.rows_of_wave, i = first + lane;
+    bool mine = lane < ca.rows_of_wave && i < ca.rows_of_b;
+    if (mine && decide) {
+      const int s = (int)ca.div_m.div(i), m = i - s * ca.M;
+      for (int l = 0; l < ca.L; ++l) {
+        const int4 lv = s_level[l];
+        const int local = s - lv.x;
+        if (local >= 0 && local < lv.y) {
+          const int y = (int)((unsigned)local / (unsigned)lv.z), x = local - y * lv.z;
+          const int ty = (int)ca.div_ty.div(y + 1), tx = (int)ca.div_tx.div(x + 1);      // the first tile starts at pixel -1
+          if (ty * TY != y + 1 && tx * TX != x + 1) {
+            const int c = ws.counts[slot_of((int)b, m, ca.B, ca.M) * nb + s_base[l] + ty * lv.w + tx];
+            mine = items_of_bin(c, ch) != 1;                // exactly one work item stores this row
           }
           break;
         }
       }
     }
-    if (grad_value != nullptr) clear_rows_of_wave(grad_value, i0, value_row_bytes, clear_mine, lane);
-    if (grad_dist != nullptr) clear_rows_of_wave(grad_dist, i0, dist_row_bytes, clear_mine, lane);
+    const uint64_t which = __ballot(mine);
+    const size_t row = (size_t)b * ca.rows_of_b + first;
+    if (ca.value.base != nullptr) ca.value.clear(row, ca.rows_of_wave, which, lane);
+    if (ca.dist.base != nullptr) ca.dist.clear(row, ca.rows_of_wave, which, lane);
   }
 }
 
@@ -528,11 +540,12 @@ __global__ __launch_bounds__(1024, 8) void bin_scan_kernel(BinWorkspace ws, Clea
   for (int base = (int)blockIdx.x * 1024; base < n; base += scan_blocks * 1024) {
     // points and work items of the bins before this block's: every thread its share, summed over the wavefront
     int bp = 0, bc = 0;
+    const int4 *quads = reinterpret_cast<const int4 *>(ws.counts);      // base is a multiple of 1024
 #pragma unroll 4
-    for (int i = threadIdx.x; i < base; i += 1024) {
-      const int c = ws.counts[i];
-      bp += c;
-      bc += items_of_bin(c, ch);
+    for (int i = threadIdx.x; i < base / 4; i += 1024) {
+      const int4 c = quads[i];
+      bp += c.x + c.y + c.z + c.w;
+      bc += items_of_bin(c.x, ch) + items_of_bin(c.y, ch) + items_of_bin(c.z, ch) + items_of_bin(c.w, ch);
     }
     bp = __builtin_amdgcn_readlane(wave_inclusive_scan(bp), kWave - 1);
     bc = __builtin_amdgcn_readlane(wave_inclusive_scan(bc), kWave - 1);
@@ -544,6 +557,7 @@ __global__ __launch_bounds__(1024, 8) void bin_scan_kernel(BinWorkspace ws, Clea
     if (lane == 0) { s_bp[wave] = bp; s_bc[wave] = bc; }
     __syncthreads();
     int run_p = ip - c, run_c = ic - k;
+#pragma unroll 4
     for (int w = 0; w < 16; ++w) {
       run_p += s_bp[w] + (w < wave ? s_pts[w] : 0);
       run_c += s_bc[w] + (w < wave ? s_chk[w] : 0);
@@ -1637,18 +1651,21 @@ static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, const Ti
   // the rows of grad_value / grad_dist that the tile kernel adds to rather than stores; and always, for a
   // distribution shared by the heads, those rows of the per-head grad_dist in the workspace (the head sum then
   // writes all of the caller's grad_dist).
-  ClearArgs ca{};
+  const int ge = a.grad_bf16 ? 2 : 4;
+  const bool writes_dist = a.dist != nullptr || a.C == 0;
+  const size_t rows_of_b = (size_t)a.S * a.M, rows = rows_of_b * a.B;
+  // 64 rows a turn are four wavefronts per SIMD from 2^18 rows on; fewer would leave CUs idle (59 k rows: 12.1 us against 7.4 in turns of 16)
+  const int rows_of_wave = rows >= (size_t)256 * 1024 ? kWave : 16;
+  const ClearRows value_rows(a.clear_grads && a.C > 0 ? a.grad_value : nullptr, a.C * ge);
+  const ClearRows dist_rows = gd_heads != nullptr ? ClearRows(gd_heads, a.D * 4) : ClearRows(a.clear_grads && writes_dist ? a.grad_dist : nullptr, a.D * ge);
+  const ClearArgs ca = {value_rows, dist_rows, a.B, a.M, a.L,
+                        cfg.cells || ((a.C | (writes_dist ? a.D : 0)) & 3) == 0 ? 1 : 0,        // the tile kernel's own condition
+                        (int)rows_of_b, rows_of_wave, FastDiv((uint32_t)((rows_of_b + rows_of_wave - 1) / rows_of_wave)),
+                        FastDiv((uint32_t)a.M), FastDiv((uint32_t)ty), FastDiv((uint32_t)tx)};
   unsigned clear_blocks = 0;
   if (a.clear_grads || gd_heads != nullptr) {            // launch_backward_binned has checked that this applies
-    const int ge = a.grad_bf16 ? 2 : 4;
-    ca.grad_value = a.clear_grads && a.C > 0 ? static_cast<char *>(a.grad_value) : nullptr;
-    ca.value_row_bytes = a.C * ge;
-    if (gd_heads != nullptr) { ca.grad_dist = reinterpret_cast<char *>(gd_heads); ca.dist_row_bytes = a.D * 4; }
-    else if (a.dist != nullptr || a.C == 0) { ca.grad_dist = static_cast<char *>(a.grad_dist); ca.dist_row_bytes = a.D * ge; }
-    ca.B = a.B; ca.S = a.S; ca.M = a.M; ca.L = a.L;
-    ca.stores = (cfg.cells || ((a.C | (a.dist != nullptr || a.C == 0 ? a.D : 0)) & 3) == 0) ? 1 : 0;        // the tile kernel's own condition
-    const size_t rows = (size_t)a.B * a.S * a.M;
-    clear_blocks = (unsigned)((rows + 1023) / 1024 < 4096 ? (rows + 1023) / 1024 : 4096);
+    const size_t turns = (rows_of_b + rows_of_wave - 1) / rows_of_wave * a.B, per_block = 1024 / kWave;
+    clear_blocks = (unsigned)((turns + per_block - 1) / per_block < 4096 ? (turns + per_block - 1) / per_block : 4096);
   }
   // scanning blocks for the most bins there can be (the plan kernel knows how many there are), 64 at most
   const size_t max_bins = (size_t)mb * slot_count(a.B, a.M);
