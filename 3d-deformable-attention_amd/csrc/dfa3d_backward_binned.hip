@@ -16,8 +16,8 @@
 //   bin_fill_sorted_kernel      writes each point's index and record into its bin's segment, a block's points
 //                               sorted by bin in LDS first so that runs of records leave together; zero
 //                               gradients for points the operator skips
-//   bin_points_kernel<0>, <1>   count and fill for shapes the two above do not take (more than 2048 tiles per
-//                               (batch, head), more than 2048 points per unit): every record straight to its slot
+//                               (both turn to bin_points_in_order for more than 2048 tiles per (batch, head) or
+//                               more than 2048 points per unit: every record straight to its slot)
 //   cell_backward_kernel        persistent workgroups pull work items from per-XCD queues: rows of up to 64
 //                               channels in whole groups of four (dfa3d_backward_cells.hip)
 //   tile_backward_kernel        the same for all other rows; per item: LDS tiles of (TY+1) x (TX+1) pixels
@@ -125,10 +125,11 @@ __device__ __forceinline__ void decode_items(const BinWorkspace &ws, int B, int 
   }
 }
 
-// The fill comes in two forms.  bin_fill_sorted_kernel (few enough bins and points per unit): a block sorts its
-// kStage points by bin in LDS and writes each bin's run of records to consecutive addresses, so a wavefront's
-// store touches a handful of lines instead of 64.  bin_points_kernel<1>: every point's record goes straight to
-// its slot.
+// Count and fill come in two forms, of which the plan's number of bins decides.  The sorted one (few enough bins and points per
+// unit): a block sorts its kStage points by bin in LDS and writes each bin's run of records to consecutive addresses, so a
+// wavefront's store touches a handful of lines instead of 64.  bin_points_in_order: every point's record goes straight to
+// its slot.  Both live in one launch each of count and fill: as launches of their own that stepped aside the others took
+// 4.6 us each (2 x 40000 queries of plain attention: 418 -> XXX us a training step).
 constexpr int kSortedBins = 2048;   // bins of one (batch, head) the sorted fill holds counters for
 constexpr int kStage = 2048;        // points a block of the sorted fill stages (1024: 0.39 ms, 4096: 0.36 ms against 0.32 ms)
 constexpr int kFillThreads = 1024;  // 256 / 512 threads: 0.49 / 0.38 ms
@@ -146,25 +147,25 @@ __device__ __forceinline__ void fill_in_point_order(const BinWorkspace &ws, cons
   }
 }
 
-// MODE 0: count.  MODE 1: fill (needs the scanned cursor).
+// MODE 0: count.  MODE 1: fill (needs the scanned cursor).  For 1 to hist_cap bins s_hist holds [0, nb): counts, then for
+// MODE 1 [nb, 2 nb): segment bases.
 template <int MODE>
-__global__ __launch_bounds__(256) void bin_points_kernel(
-    BinWorkspace ws, const float *__restrict__ loc, int loc_stride, const float *__restrict__ attn,
+__device__ __forceinline__ void bin_points_in_order(
+    const BinWorkspace &ws, const float *__restrict__ loc, int loc_stride, const float *__restrict__ attn,
     float *__restrict__ grad_loc, int gl_stride, float *__restrict__ grad_attn, float *__restrict__ grad_score,
-    int B, int M, int L, int Q, int P, int q_blocks, int n_blocks, int hist_cap DFA3D_DIAG_PARAM) {
-  extern __shared__ int s_hist[];          // [0, nb): counts, then for MODE 1 [nb, 2 nb): segment bases
+    int B, int M, int L, int Q, int P, int hist_cap, int *s_hist) {
   const BinPlan &p = *ws.plan;
   const int nb = p.bins_per_bm;
-  if (sorted_fill_applies(nb, L * P)) return;                   // bin_count_kernel / bin_fill_sorted_kernel do it
   if (nb == 0) {
     if (MODE == 1) fill_in_point_order(ws, loc, loc_stride, attn, (size_t)B * Q * M * L * P);
     return;
   }
   const bool use_lds = nb <= hist_cap;
   if (MODE == 1) decode_items(ws, B, M, L, blockIdx.x, gridDim.x);
-  // The launch is a few thousand workgroups that walk the n_blocks blocks of work (so that it costs next to nothing
-  // when the kernel steps aside).  head = block % M: with the round-robin placement of workgroups on the 8 XCDs
-  // and a grid that is a multiple of 8, the records of one (batch, head) are written through one XCD's L2.
+  // Blocks of work: a thread a point, kBinQueries queries at least.  head = block % M: with the round-robin placement of
+  // workgroups on the 8 XCDs and a grid that is a multiple of 8, the records of one (batch, head) are written through one
+  // XCD's L2.
+  const int q_block = max(kBinQueries, kFillThreads / (L * P)), q_blocks = (Q + q_block - 1) / q_block, n_blocks = B * M * q_blocks;
   int counted = 0;
   for (int blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
   __syncthreads();                          // the previous block's LDS histogram is no longer in use
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(256) void bin_points_kernel(
   const int qb = rest % q_blocks, b = rest / q_blocks;
   const int bm = slot_of(b, m, B, M);
   const int LP = L * P;
-  const int q0 = qb * kBinQueries, nq = min(kBinQueries, Q - q0);
+  const int q0 = qb * q_block, nq = min(q_block, Q - q0);
   const int npts = nq * LP;
   int *gcount = ws.counts + (size_t)bm * nb;
   int *gcursor = ws.cursor + (size_t)bm * nb;
@@ -237,10 +238,9 @@ __global__ __launch_bounds__(256) void bin_points_kernel(
       }
       if (bin >= 0) {
         const int slot = use_lds ? s_hist[nb + bin] + atomicAdd(&s_hist[bin], 1) : atomicAdd(&gcursor[bin], 1);
-        if (!DFA3D_DIAG(diag, 128)) ws.entries[slot] = (uint32_t)gp;
-        if (!DFA3D_DIAG(diag, 64))
-          ws.recs[slot] = make_float4(loc[gp * loc_stride], loc[gp * loc_stride + 1],
-                                      loc_stride > 2 ? loc[gp * loc_stride + 2] : 0.f, attn != nullptr ? attn[gp] : 0.f);
+        ws.entries[slot] = (uint32_t)gp;
+        ws.recs[slot] = make_float4(loc[gp * loc_stride], loc[gp * loc_stride + 1],
+                                    loc_stride > 2 ? loc[gp * loc_stride + 2] : 0.f, attn != nullptr ? attn[gp] : 0.f);
       }
     }
   }
@@ -274,15 +274,20 @@ struct BinTable {
 
 // Count in the same shape as the sorted fill: 1024 threads, kStage points per block, all loads of a thread issued
 // before its first LDS atomic.
-__global__ __launch_bounds__(kFillThreads) void bin_count_kernel(
+__global__ __launch_bounds__(kFillThreads, 8) void bin_count_kernel(
     BinWorkspace ws, const float *__restrict__ loc, int loc_stride, int B, int M, int L, int Q, int P, int nq_block,
-    int q_blocks, BinDivs divs) {
+    int q_blocks, int hist_cap, BinDivs divs) {
   __shared__ int s_cnt[kSortedBins], s_inside;
   __shared__ BinTable tab;
+  extern __shared__ int s_hist[];                                // hist_cap counters, where the host cannot rule them out
   const BinPlan &p = *ws.plan;
   const int nb = p.bins_per_bm;
   const int LP = L * P;
-  if (nb == 0 || !sorted_fill_applies(nb, LP)) return;
+  if (nb == 0) return;
+  if (!sorted_fill_applies(nb, LP)) {
+    bin_points_in_order<0>(ws, loc, loc_stride, nullptr, nullptr, 0, nullptr, nullptr, B, M, L, Q, P, hist_cap, s_hist);
+    return;
+  }
   const int tid = threadIdx.x;
   const int m = blockIdx.x % M, rest = blockIdx.x / M;
   const int qb = rest % q_blocks, b = rest / q_blocks;
@@ -324,10 +329,10 @@ __global__ __launch_bounds__(kFillThreads) void bin_count_kernel(
   }
 }
 
-__global__ __launch_bounds__(kFillThreads) void bin_fill_sorted_kernel(
+__global__ __launch_bounds__(kFillThreads, 8) void bin_fill_sorted_kernel(
     BinWorkspace ws, const float *__restrict__ loc, int loc_stride, const float *__restrict__ attn,
     float *__restrict__ grad_loc, int gl_stride, float *__restrict__ grad_attn, float *__restrict__ grad_score,
-    int B, int M, int L, int Q, int P, int q_blocks, BinDivs divs) {
+    int B, int M, int L, int Q, int P, int q_blocks, int hist_cap, BinDivs divs) {
   extern __shared__ __align__(16) unsigned char s_raw[];        // kSortedFillLds bytes
   __shared__ BinTable tab;
   uint4 *s_rec = reinterpret_cast<uint4 *>(s_raw);               // staged records, grouped by bin
@@ -340,13 +345,12 @@ __global__ __launch_bounds__(kFillThreads) void bin_fill_sorted_kernel(
   const BinPlan &p = *ws.plan;
   const int nb = p.bins_per_bm;
   const int LP = L * P;
-  if (!sorted_fill_applies(nb, LP)) return;
-  if (nb == 0) {
-    fill_in_point_order(ws, loc, loc_stride, attn, (size_t)B * Q * M * LP);
+  if (nb == 0 || !sorted_fill_applies(nb, LP)) {
+    bin_points_in_order<1>(ws, loc, loc_stride, attn, grad_loc, gl_stride, grad_attn, grad_score, B, M, L, Q, P, hist_cap, reinterpret_cast<int *>(s_raw));
     return;
   }
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int m = blockIdx.x % M, rest = blockIdx.x / M;          // head = block % M, as in bin_points_kernel
+  const int m = blockIdx.x % M, rest = blockIdx.x / M;          // head = block % M, as in bin_points_in_order
   const int qb = rest % q_blocks, b = rest / q_blocks;
   const int bm = slot_of(b, m, B, M);
   // A block takes every q_blocks-th query, not a run of consecutive ones.  Consecutive queries of a model look at
@@ -1626,27 +1630,18 @@ static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, const Ti
   const int mb = max_bins_per_bm(a.S, a.L, ty, tx);
   hipLaunchKernelGGL(plan_and_clear_kernel, dim3(64), dim3(256), 0, stream, ws, a.shapes, a.shape_stride, a.level_start,
                      a.L, a.S, (a.dist != nullptr || a.C == 0) ? a.D : 0, a.B, a.M, ty, tx, chunk, mb);
-  const int q_blocks = (a.Q + kBinQueries - 1) / kBinQueries;
+  const int LP = a.L * a.P;
+  const bool sorted_maybe = LP <= kStage, sorted_surely = sorted_maybe && mb <= kSortedBins;
+  const int nq_block = sorted_maybe ? kStage / LP : 1;           // (bin_points_in_order makes its own of it)
+  const int q_blocks = (a.Q + nq_block - 1) / nq_block;
   const long long blocks = (long long)a.B * a.M * q_blocks;
   if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
-  const int hist_cap = mb < kHistCap ? mb : kHistCap;
-  const unsigned grid = blocks < 2048 ? (unsigned)blocks : 2048u;
-  const int LP = a.L * a.P;
-  // Of the two forms of counting and filling the plan kernel's result decides between, and the other steps aside; a map
-  // so small that it cannot have too many bins for the sorted form spares the two launches that would (4.5 us each).
-  const bool sorted_surely = LP <= kStage && mb <= kSortedBins;
-  if (!sorted_surely)
-    hipLaunchKernelGGL(bin_points_kernel<0>, dim3(grid), dim3(256), (size_t)hist_cap * 4, stream, ws,
-                     (const float *)a.loc, a.loc_stride, (const float *)a.attn, (float *)a.grad_loc, a.grad_loc_stride,
-                     (float *)a.grad_attn, (float *)a.grad_score_out, a.B, a.M, a.L, a.Q, a.P, q_blocks, (int)blocks, hist_cap DFA3D_DIAG_ARG(a));
-  const int nq_block = LP <= kStage ? kStage / LP : 1;
-  const int q_blocks2 = (a.Q + nq_block - 1) / nq_block;
-  const long long blocks2 = (long long)a.B * a.M * q_blocks2;
-  if (blocks2 > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
+  const unsigned grid = sorted_maybe || blocks < 2048 ? (unsigned)blocks : 2048u;
+  const int hist_cap = sorted_surely ? 0 : mb < kHistCap ? mb : kHistCap;
+  static_assert((size_t)kHistCap * 8 <= kSortedFillLds, "bin_points_in_order's counters lie in the sorted fill's LDS");
   const BinDivs divs{FastDiv((uint32_t)LP), FastDiv((uint32_t)a.P), FastDiv((uint32_t)ty), FastDiv((uint32_t)tx)};
-  if (LP <= kStage)                         // steps aside if there turn out to be too many bins, as the one above does if not
-    hipLaunchKernelGGL(bin_count_kernel, dim3((unsigned)blocks2), dim3(kFillThreads), 0, stream, ws, (const float *)a.loc,
-                       a.loc_stride, a.B, a.M, a.L, a.Q, a.P, nq_block, q_blocks2, divs);
+  hipLaunchKernelGGL(bin_count_kernel, dim3(grid), dim3(kFillThreads), (size_t)hist_cap * 4, stream, ws, (const float *)a.loc,
+                     a.loc_stride, a.B, a.M, a.L, a.Q, a.P, nq_block, q_blocks, hist_cap, divs);
   // What further blocks of the scan's launch clear meanwhile: for a caller that did not zero them (options.clear),
   // the rows of grad_value / grad_dist that the tile kernel adds to rather than stores; and always, for a
   // distribution shared by the heads, those rows of the per-head grad_dist in the workspace (the head sum then
@@ -1671,16 +1666,10 @@ static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, const Ti
   const size_t max_bins = (size_t)mb * slot_count(a.B, a.M);
   const unsigned scan_blocks = (max_bins + 1023) / 1024 < 64 ? (unsigned)((max_bins + 1023) / 1024) : 64u;
   hipLaunchKernelGGL(bin_scan_kernel, dim3(scan_blocks + clear_blocks), dim3(1024), 0, stream, ws, ca, (int)scan_blocks);
-  if (LP <= kStage) {
-    if (hipError_t e = allow_lds(bin_fill_sorted_kernel, kSortedFillLds)) return e;
-    hipLaunchKernelGGL(bin_fill_sorted_kernel, dim3((unsigned)blocks2), dim3(kFillThreads), kSortedFillLds, stream, ws, (const float *)a.loc,
-                       a.loc_stride, (const float *)a.attn, (float *)a.grad_loc, a.grad_loc_stride, (float *)a.grad_attn,
-                       (float *)a.grad_score_out, a.B, a.M, a.L, a.Q, a.P, q_blocks2, divs);
-  }
-  if (!sorted_surely)
-    hipLaunchKernelGGL(bin_points_kernel<1>, dim3(grid), dim3(256), (size_t)hist_cap * 8, stream, ws,
-                     (const float *)a.loc, a.loc_stride, (const float *)a.attn, (float *)a.grad_loc, a.grad_loc_stride,
-                     (float *)a.grad_attn, (float *)a.grad_score_out, a.B, a.M, a.L, a.Q, a.P, q_blocks, (int)blocks, hist_cap DFA3D_DIAG_ARG(a));
+  if (hipError_t e = allow_lds(bin_fill_sorted_kernel, kSortedFillLds)) return e;
+  hipLaunchKernelGGL(bin_fill_sorted_kernel, dim3(grid), dim3(kFillThreads), kSortedFillLds, stream, ws, (const float *)a.loc,
+                     a.loc_stride, (const float *)a.attn, (float *)a.grad_loc, a.grad_loc_stride, (float *)a.grad_attn,
+                     (float *)a.grad_score_out, a.B, a.M, a.L, a.Q, a.P, q_blocks, hist_cap, divs);
   return hipGetLastError();
 }
 

@@ -11,7 +11,7 @@ namespace dfa3d {
 constexpr int kClasses = 8;         // work queues: one per XCD (workgroup id % 8 with round-robin placement)
 constexpr int kQueueStride = 16;    // ints between queue counters: one 64-byte line each
 constexpr int kQueueInts = kClasses * kQueueStride + 32;   // + room for the optional phase timers
-constexpr int kBinQueries = 32;     // bin_points_kernel: queries of one (batch, head) per block step (16, 64, 128 time worse)
+constexpr int kBinQueries = 32;     // bin_points_in_order: queries of one (batch, head) per block step, at least
 constexpr int kHistCap = 8192;      // bins of one (batch, head) that fit the LDS histogram
 
 struct BinPlan {
