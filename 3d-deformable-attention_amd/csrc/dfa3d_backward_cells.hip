@@ -354,7 +354,7 @@ __device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x
 // of the numbers that follow from them, than scalar registers.  Passed one by one they were kept from turn to turn, at the
 // cost of 98 others (float, 32 channels; 105 with bfloat16) that went to lanes of vector registers and came back one
 // instruction each.  Base shape, 15.4 M points: 1194 -> 1184 us, bfloat16 1160 -> 1100 us.
-// FRESH: read again at each use.  Stage 2 alone has fewer of them and keeps its 8 to 14 that do not fit (two-stage shape, 14.6 M
+// FRESH: read again at each use.  Stage 2 alone has fewer of them, of which 8 to 16 do not fit, and keeps them (two-stage shape, 14.6 M
 // points: 1037 us against 1040 read anew, 2.6 M points of plain attention 214 against 217).
 template <typename T> struct CellArgs {
   BinWorkspace ws;
@@ -524,10 +524,10 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         return __int_as_float(__builtin_amdgcn_ds_bpermute((lane - back) << 2, __float_as_int(x)));
       }
     };
-    auto owner = [&]() {
+    auto owner = [&](auto a) {
       unsigned l = lane;
       asm volatile("" : "+v"(l));
-      return Owner(l, wave, arg()->C);
+      return Owner(l, wave, a->C);
     };
     auto decode = [&](const int4 &item, const int4 &geo) {
       ItemGeom g;
@@ -555,8 +555,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     // The sums of tile pixel (crow, ccol) of item q are complete in u.  Pixels 1..TY-1 x 1..7 belong to no neighbour's
     // halo: when the item writes its tile alone they are stored (grad_value is zero on entry, or the binning launches
     // cleared what is added to), else added.  Rim pixels go to their place in LDS, to be added by put_rim.
-    auto put_pixel = [&](const Owner &o, const ItemGeom &q, const float (&u)[VEC], bool active) {
-      const auto a = arg();
+    auto put_pixel = [&](auto a, const Owner &o, const ItemGeom &q, const float (&u)[VEC], bool active) {
       const int S = a->S, M = a->M, C = a->C;
       const bool gv16 = (a->grad16 & 1) != 0;               // uniform
       void *grad_value = a->grad_value;
@@ -587,8 +586,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       }
     };
     // Rim pixels [first, first + n) of item q, whose sums this wavefront left in LDS.
-    auto put_rim = [&](const ItemGeom &q, int first, int n) {
-      const auto a = arg();
+    auto put_rim = [&](auto a, const ItemGeom &q, int first, int n) {
       const int S = a->S, M = a->M, C = a->C;
       const bool gv16 = (a->grad16 & 1) != 0;               // uniform
       void *grad_value = a->grad_value;
@@ -632,29 +630,33 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     // go straight there, 16 bytes per lane, without a register in between.  (The pointers, whose work in phase Y is the
     // longer one, brought them before: tile kernel 1158 -> 1121 us at the base shape, bfloat16 1045 -> 1022, dense 4245 -> 4160,
     // small 111 -> 106.)
-    auto stage = [&]() {
+    auto stage = [&](int n) {
       const auto a = arg();
       const int Q = a->Q, M = a->M, C = a->C;
       const T *grad_out = a->grad_out;
       if (C == ROW) {                                        // uniform
-        constexpr int RL = ROW * (int)sizeof(T) / 16, RPI = kWave / RL, N = kRows / RPI, NB = N < 4 ? N : 4;      // lanes per row, rows per instruction
+        // Instructions take turns over the wavefronts and stop where the pass's points do: an item of a few dozen points
+        // asks for its rows in one or two of each (6 x 2000 queries, four levels from 116 x 200, 32 points a query: tile kernel
+        // 535 -> 526 us).
+        constexpr int RL = ROW * (int)sizeof(T) / 16, RPI = kWave / RL, N = kRows / RPI, NB = N < 2 ? N : 2;      // lanes per row, rows per instruction
         const rsrc_t go_r = make_rsrc(grad_out + (size_t)g.b * Q * M * C, (size_t)Q * M * C * sizeof(T));
-        const int row0 = wave * kRows;
         unsigned l = lane;
         asm volatile("" : "+v"(l));                          // (not worth registers from turn to turn)
+        const int r0 = wave * RPI, at = r0 + (int)(l / RL);
 #pragma unroll
         for (int j0 = 0; j0 < N; j0 += NB) {
+          if (j0 > 0 && r0 + j0 * 4 * RPI >= n) break;       // uniform
           uint32_t row[NB];
 #pragma unroll
-          for (int j = 0; j < NB; ++j) row[j] = goff[(turn & 1) * PP + row0 + (j0 + j) * RPI + l / RL];
+          for (int j = 0; j < NB; ++j) row[j] = goff[(turn & 1) * PP + (j0 + j) * 4 * RPI + at];
 #pragma unroll
           for (int j = 0; j < NB; ++j)
-            load_to_lds16(go_r, gstage + (row0 + (j0 + j) * RPI) * RL * 16, row[j] + piece_at<T, RL * 16>((j0 + j) * RPI + l / RL, l % RL) % (RL * 16));
+            load_to_lds16(go_r, gstage + (r0 + (j0 + j) * 4 * RPI) * RL * 16, row[j] + piece_at<T, RL * 16>((j0 + j) * 4 * RPI + at, l % RL) % (RL * 16));
           __builtin_amdgcn_sched_barrier(0);
         }
         return;
       }
-      const Owner o = owner();
+      const Owner o = owner(arg());
       const rsrc_t go_r = make_rsrc(grad_out + (size_t)g.b * Q * M * C, (size_t)Q * M * C * sizeof(T));
       const uint32_t *offs_of = goff + (turn & 1) * PP + wave * kRows;
 #pragma unroll
@@ -674,7 +676,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     // from LDS: base shape 1061 -> 1040 us.  With 4-byte elements, where a matrix instruction is one channel deep and a row twice
     // as long, it lost: plain attention 209 -> 227 us, base shape 1194 -> 1277.
     auto walk_fours = [&](const WholeRow<T, VEC, LPR> &v, f4 (&acc)[VEC]) {
-      const Owner o = owner();
+      const Owner o = owner(arg());
       const int corner = o.cl & 3, cell = o.crow * TX + o.ccol;
       const bool cell_ok = o.crow < TY;
       const int beg = cell_ok ? offs[cell] : 0, n = cell_ok ? offs[cell + 1] - beg : 0;
@@ -721,7 +723,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     // 4-byte elements: one point per step and group; the next step's row and weights and the slot after that are asked for while
     // this step's sums are formed, so that no LDS round trip is waited for with nothing to do.
     auto walk_ones = [&](const float (&v)[4][VEC], f4 (&acc)[VEC]) {
-      const Owner o = owner();
+      const Owner o = owner(arg());
       const int corner = o.cl & 3, cell = o.crow * TX + o.ccol;
       const bool cell_ok = o.crow < TY;
       const int beg = cell_ok ? offs[cell] : 0, n = cell_ok ? offs[cell + 1] - beg : 0;
@@ -771,11 +773,12 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 #pragma unroll
         for (int i = 0; i < VEC; ++i) u[i] = 0;
         CT_MARK(0);
+        const auto now = arg();                              // read once for all of the change of items (C = 64, 1.28 M points on 400 x 400: 583 -> 574 us)
         // The record of the item three on, first of all: what thread 0 waits for was asked for an item ago.
         if (tid == 0 && !done) {
           CellFetch fetch = s_fetch;
           int4 rec, geo;
-          const BinWorkspace w = arg()->ws;
+          const BinWorkspace w = now->ws;
           fetch.advance(w, *w.plan, &rec, &geo);
           s_geom[slot_of_item(it + 3)] = decode(rec, geo);
           s_fetch = fetch;
@@ -784,7 +787,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           // The item before is over.  Tile pixel (r, c) collects corner 0 of cell (r, c), corner 1 of (r, c - 1), corner 2
           // of (r - 1, c - 1) and corner 3 of (r - 1, c): the cell to the left is the lane group to the left, the row
           // above the lower half of this wavefront, or the wavefront before it.
-          const Owner o = owner();
+          const Owner o = owner(now);
           float dn[VEC], ux[VEC], dx[VEC];                   // for the row below; the same of the ninth pixel (last cell)
 #pragma unroll
           for (int i = 0; i < VEC; ++i) {
@@ -808,18 +811,17 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
               if (o.ccol == TX - 1) put_lds(o, cross + (wave * TW + TX) * ROW, dx);
             }
           }
-          if (ROWS == 2) put_pixel(o, uniform(s_geom[slot_of_item(it - 1)]), u, o.crow < TY && o.group >= TX);   // the second row is complete
+          if (ROWS == 2) put_pixel(now, o, uniform(s_geom[slot_of_item(it - 1)]), u, o.crow < TY && o.group >= TX);   // the second row is complete
         }
         CT_MARK(3);
-        if (!done) stage();
+        if (!done) stage(g.n_item);
         typename LaneChannels<T, VEC, LPR>::Raw vr[4];
         {
           // the four value rows of this group's cell (zero outside the map, when the cell is not part of the tile, or when
           // there is no item)
-          const auto a = arg();
-          const int S = a->S, M = a->M, C = a->C;
-          const T *value = a->value;
-          const Owner o = owner();
+          const int S = now->S, M = now->M, C = now->C;
+          const T *value = now->value;
+          const Owner o = owner(now);
           const rsrc_t value_r = make_rsrc(value + (size_t)g.b * S * M * C, (size_t)S * M * C * sizeof(T));
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
@@ -838,7 +840,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         if (have_prev && r0 < TY) {                          // uniform
           // The first tile row of this wavefront collects what the wavefront before it left for it; then the rim goes out.
           const ItemGeom q = uniform(s_geom[slot_of_item(it - 1)]);
-          const Owner o = owner();
+          const Owner o = owner(now);
           const bool mine = o.crow < TY && o.group < TX;
           if (wave > 0 && mine) {
             const float *from = cross + ((wave - 1) * TW + o.ccol) * ROW;
@@ -853,12 +855,12 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
               }
             }
           }
-          put_pixel(o, q, u, mine);
+          put_pixel(now, o, q, u, mine);
           wave_lds_handover();
           const int ra = max(r0, 1), n_side = min(r0 + ROWS, TY) - ra;
-          if (wave == 0) put_rim(q, 0, TW);
-          if (n_side > 0) put_rim(q, rim_index(ra, 0, TY, TX), 2 * n_side);
-          if (r0 + ROWS >= TY) put_rim(q, TW, TW);
+          if (wave == 0) put_rim(now, q, 0, TW);
+          if (n_side > 0) put_rim(now, q, rim_index(ra, 0, TY, TX), 2 * n_side);
+          if (r0 + ROWS >= TY) put_rim(now, q, TW, TW);
         }
         if (done) break;
         typename std::conditional<sizeof(T) == 4, float[4][VEC], WholeRow<T, VEC, LPR>>::type v;      // the four value rows
@@ -866,7 +868,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 #pragma unroll
           for (int k = 0; k < 4; ++k) LaneChannels<T, VEC, LPR>::to_float(vr[k], v[k]);
         } else {
-          whole_rows<T, VEC, LPR>(vr, owner().cl, v);
+          whole_rows<T, VEC, LPR>(vr, owner(now).cl, v);
         }
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = (f4){0, 0, 0, 0};
@@ -876,7 +878,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         lds_barrier();
         CT_MARK(2);
         for (int base = PP; base < g.n_item; base += PP) {   // the item's further passes
-          stage();
+          stage(g.n_item - base);
           wait_for_loads();
           CT_MARK(6);
           lds_barrier();
