@@ -32,8 +32,10 @@
 // -1 <= w0 < W; the tiles are laid over that range, so the first tile of a level starts at pixel -1.
 // Semantics are those of bwd_attention_kernel (see dfa3d_backward.hip for the formulas and the
 // reference lines they restate).
+#include <algorithm>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "dfa3d_binned.h"
@@ -129,7 +131,7 @@ __device__ __forceinline__ void decode_items(const BinWorkspace &ws, int B, int 
 // unit): a block sorts its kStage points by bin in LDS and writes each bin's run of records to consecutive addresses, so a
 // wavefront's store touches a handful of lines instead of 64.  bin_points_in_order: every point's record goes straight to
 // its slot.  Both live in one launch each of count and fill: as launches of their own that stepped aside the others took
-// 4.6 us each (2 x 40000 queries of plain attention: 418 -> XXX us a training step).
+// 4.6 us each (2 x 40000 queries of plain attention: 9 of 418 us a training step).
 constexpr int kSortedBins = 2048;   // bins of one (batch, head) the sorted fill holds counters for
 constexpr int kStage = 2048;        // points a block of the sorted fill stages (1024: 0.39 ms, 4096: 0.36 ms against 0.32 ms)
 constexpr int kFillThreads = 1024;  // 256 / 512 threads: 0.49 / 0.38 ms
@@ -253,10 +255,11 @@ __device__ __forceinline__ void bin_points_in_order(
 
 // What the count and the sorted fill divide by, per point: points of a unit and of a level, tile edges.
 struct BinDivs { FastDiv lp, p, ty, tx; };
-// The plan's tables in LDS: a block of these two kernels lives a few microseconds, most of it waiting, and the bin of a point
-// otherwise takes a chain of three reads of device memory after its location has come, and four divisions by numbers
-// the compiler does not know.  15.36 M points: count 89 -> 52 us (184 MB read, 3.5 TB/s), fill 195 -> 153 us (553 MB moved,
-// 3.6 TB/s, where a copy reaches 4.7).
+// The plan's tables in LDS: the bin of a point otherwise takes a chain of three reads of device memory after its location has
+// come, and four divisions by numbers the compiler does not know.  15.36 M points: count 89 -> 52 us, fill 195 -> 153 us.
+// Both kernels then had a block per turn, which waited for its points, then for its reservations.  As many blocks as the
+// chip holds, with the next turn's points on their way while they work on one: count 52 -> 36 us (184 MB read, 5.1 TB/s), fill
+// 153 -> 144 us (553 MB moved, 3.8 TB/s, where a copy reaches 4.7); 61 M clustered points count 281 -> 134 us, fill 595 -> 584.
 struct BinTable {
   int H[DFA3D_MAX_LEVELS], W[DFA3D_MAX_LEVELS], base[DFA3D_MAX_LEVELS], tiles_x[DFA3D_MAX_LEVELS];
   __device__ __forceinline__ void load(const BinPlan &p) {     // the caller's barrier
@@ -272,11 +275,13 @@ struct BinTable {
   }
 };
 
-// Count in the same shape as the sorted fill: 1024 threads, kStage points per block, all loads of a thread issued
-// before its first LDS atomic.
+// Count: turns of kStage points, as many blocks per (batch, head) as the chip holds, each with one set of counters for all its
+// turns: an atomic per bin that it touched.  (Tried: runs of consecutive turns per block, 39 us and slow where the locations
+// come from memory; counters for all heads and turns of consecutive points, 41 us, and too many blocks that meet on the
+// counters of a batch element, 5 -> 10 us for 0.3 M points.)
 __global__ __launch_bounds__(kFillThreads, 8) void bin_count_kernel(
-    BinWorkspace ws, const float *__restrict__ loc, int loc_stride, int B, int M, int L, int Q, int P, int nq_block,
-    int q_blocks, int hist_cap, BinDivs divs) {
+    BinWorkspace ws, const float *__restrict__ loc, int loc_stride, int B, int M, int L, int Q, int P, int q_turn,
+    int parts, int hist_cap, BinDivs divs) {
   __shared__ int s_cnt[kSortedBins], s_inside;
   __shared__ BinTable tab;
   extern __shared__ int s_hist[];                                // hist_cap counters, where the host cannot rule them out
@@ -290,39 +295,51 @@ __global__ __launch_bounds__(kFillThreads, 8) void bin_count_kernel(
   }
   const int tid = threadIdx.x;
   const int m = blockIdx.x % M, rest = blockIdx.x / M;
-  const int qb = rest % q_blocks, b = rest / q_blocks;
-  const int bm = slot_of(b, m, B, M);
-  const int q0 = qb * nq_block, nq = min(nq_block, Q - q0);      // any split of the queries gives the same counts
-  const int npts = nq * LP;
+  const int part = rest % parts, b = rest / parts;
   constexpr int kPer = kStage / kFillThreads;
-  float x[kPer], y[kPer];
-  int lv[kPer];
+  // a thread's points keep their place within the unit from turn to turn
+  int qi[kPer], lp[kPer], lv[kPer];
 #pragma unroll
   for (int r = 0; r < kPer; ++r) {
     const int i = tid + kFillThreads * r;
-    lv[r] = -1; x[r] = y[r] = 0;
-    if (i < npts) {
-      const int qi = divs.lp.div(i), lp = i - qi * LP;
-      const size_t gp = ((size_t)(b * (size_t)Q + q0 + qi) * M + m) * LP + lp;
-      x[r] = loc[gp * loc_stride]; y[r] = loc[gp * loc_stride + 1];
-      lv[r] = divs.p.div(lp);
-    }
+    qi[r] = divs.lp.div(i); lp[r] = i - qi[r] * LP; lv[r] = divs.p.div(lp[r]);
   }
+  float x[kPer], y[kPer];
+  auto ask = [&](int q0) {                                       // always asked for, so that the waits can be counted
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      const int q = min(q0 + qi[r], Q - 1);
+      const float *at = loc + (((size_t)b * Q + q) * M + m) * LP * loc_stride + (size_t)lp[r] * loc_stride;
+      x[r] = at[0]; y[r] = at[1];
+    }
+  };
+  ask(part * q_turn);
   for (int i = tid; i < nb; i += kFillThreads) s_cnt[i] = 0;
   if (tid == 0) s_inside = 0;
   tab.load(p);
   __syncthreads();
   int counted = 0;                                               // of this wavefront
+  auto tally = [&](int q0, const float (&tx)[kPer], const float (&ty)[kPer]) {
 #pragma unroll
-  for (int r = 0; r < kPer; ++r) {
-    const int bin = lv[r] >= 0 ? tab.bin(lv[r], x[r], y[r], divs) : -1;
-    if (bin >= 0) atomicAdd(&s_cnt[bin], 1);
-    counted += __popcll(__ballot(bin >= 0));
+    for (int r = 0; r < kPer; ++r) {
+      const int bin = qi[r] < q_turn && q0 + qi[r] < Q ? tab.bin(lv[r], tx[r], ty[r], divs) : -1;
+      if (bin >= 0) atomicAdd(&s_cnt[bin], 1);
+      counted += __popcll(__ballot(bin >= 0));
+    }
+  };
+  int q0 = part * q_turn;
+  for (; q0 + parts * q_turn < Q; q0 += parts * q_turn) {
+    float tx[kPer], ty[kPer];
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) { tx[r] = x[r]; ty[r] = y[r]; }
+    ask(q0 + parts * q_turn);
+    tally(q0, tx, ty);
   }
+  tally(q0, x, y);
   if (tid % kWave == 0) atomicAdd(&s_inside, counted);
   __syncthreads();
   if (tid == 0) atomicAdd(counted_points(ws), s_inside);
-  int *gcount = ws.counts + (size_t)bm * nb;
+  int *gcount = ws.counts + (size_t)slot_of(b, m, B, M) * nb;
   for (int i = tid; i < nb; i += kFillThreads) {
     const int c = s_cnt[i];
     if (c > 0) atomicAdd(&gcount[i], c);
@@ -350,102 +367,130 @@ __global__ __launch_bounds__(kFillThreads, 8) void bin_fill_sorted_kernel(
     return;
   }
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int m = blockIdx.x % M, rest = blockIdx.x / M;          // head = block % M, as in bin_points_in_order
-  const int qb = rest % q_blocks, b = rest / q_blocks;
-  const int bm = slot_of(b, m, B, M);
-  // A block takes every q_blocks-th query, not a run of consecutive ones.  Consecutive queries of a model look at
+  constexpr int kPer = kStage / kFillThreads;                             // points per thread
+  // A turn takes every q_blocks-th query, not a run of consecutive ones.  Consecutive queries of a model look at
   // neighbouring places (BEV pillars in raster order), so a run of them would put a compact patch of points into a
   // bin, the tile kernel's passes (consecutive points of a bin) would each hit a few tile rows only, and its rows
   // phase, which takes as long as the longest row's list, would slow down (measured: 1.74 -> 2.25 ms).  Spread
-  // over the whole query range a block's points cover each bin's area evenly, whatever the order of the queries.
-  const int nq = (Q - qb + q_blocks - 1) / q_blocks;             // <= kStage / LP, of which q_blocks is the ceiling quotient
-  const int npts = nq * LP;                                      // <= kStage
-  int *gcursor = ws.cursor + (size_t)bm * nb;
-  constexpr int kPer = kStage / kFillThreads;                             // points per thread
-
-  // 1. every point: its bin and its rank among this block's points of that bin
-  int bin[kPer], rank[kPer];
-  uint4 rec[kPer];
-  uint32_t gpi[kPer];
+  // over the whole query range a turn's points cover each bin's area evenly, whatever the order of the queries.
+  int qi[kPer], level[kPer];                                       // a thread's points keep their place within the turn
+  uint32_t from[kPer];
 #pragma unroll
   for (int r = 0; r < kPer; ++r) {
     const int i = tid + kFillThreads * r;
-    bin[r] = -1; rank[r] = 0; gpi[r] = 0;
-    rec[r] = make_uint4(0, 0, 0, 0);
-    if (i < npts) {
-      const int qi = divs.lp.div(i), lp = i - qi * LP;
-      const size_t gp = ((size_t)(b * (size_t)Q + qb + (size_t)qi * q_blocks) * M + m) * LP + lp;
-      const float *at = loc + gp * loc_stride;
-      rec[r] = make_uint4(__float_as_uint(at[0]), __float_as_uint(at[1]), loc_stride > 2 ? __float_as_uint(at[2]) : 0u,
-                          attn != nullptr ? __float_as_uint(attn[gp]) : 0u);
-      gpi[r] = (uint32_t)gp;
-      bin[r] = divs.p.div(lp);                                     // the level, for now
-    }
+    qi[r] = (int)divs.lp.div(i) * q_blocks;
+    const int lp = i - (int)divs.lp.div(i) * LP;
+    level[r] = divs.p.div(lp);
+    from[r] = (uint32_t)qi[r] * (uint32_t)M * (uint32_t)LP + (uint32_t)lp;
   }
+  struct Turn { int b, m, qb; };
+  auto turn_of = [&](unsigned blk) {                                  // head = block % M, as in bin_points_in_order
+    Turn t;
+    t.m = blk % M;
+    const unsigned rest = blk / M;
+    t.qb = rest % q_blocks; t.b = rest / q_blocks;
+    return t;
+  };
+  uint4 rec[kPer];
+  uint32_t gpi[kPer];
+  bool live[kPer];
+  auto ask = [&](const Turn &t) {                                // always asked for, so that the waits can be counted
+    const uint32_t first = (uint32_t)(((size_t)t.b * Q + t.qb) * M + t.m) * LP;
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      live[r] = t.qb + qi[r] < Q;
+      gpi[r] = live[r] ? first + from[r] : first;
+      const float *at = loc + (size_t)gpi[r] * loc_stride;
+      rec[r] = make_uint4(__float_as_uint(at[0]), __float_as_uint(at[1]), loc_stride > 2 ? __float_as_uint(at[2]) : 0u,
+                          attn != nullptr ? __float_as_uint(attn[gpi[r]]) : 0u);
+    }
+  };
+  const unsigned n_turns = (unsigned)(B * M * q_blocks);
+  if (blockIdx.x < n_turns) ask(turn_of(blockIdx.x));
   for (int i = tid; i < nb; i += kFillThreads) s_cnt[i] = 0;
   tab.load(p);
   decode_items(ws, B, M, L, blockIdx.x, gridDim.x);
   __syncthreads();
+  auto turn = [&](unsigned blk, auto more) {                     // more: another one follows
+    const Turn t = turn_of(blk);
+    int *gcursor = ws.cursor + (size_t)slot_of(t.b, t.m, B, M) * nb;
+    // 1. every point: its bin and its rank among this turn's points of that bin
+    int bin[kPer], rank[kPer];
+    uint4 mine[kPer];
+    uint32_t gp[kPer];
 #pragma unroll
-  for (int r = 0; r < kPer; ++r) {
-    if (bin[r] < 0) continue;
-    bin[r] = tab.bin(bin[r], __uint_as_float(rec[r].x), __uint_as_float(rec[r].y), divs);
-    if (bin[r] >= 0) {
-      rank[r] = atomicAdd(&s_cnt[bin[r]], 1);
-    } else {
-      // skipped by the operator: all its gradients are zero, and no tile will visit it
-      const size_t gp = gpi[r];
-      for (int c = 0; c < gl_stride; ++c) grad_loc[gp * gl_stride + c] = 0;
-      if (grad_attn != nullptr) grad_attn[gp] = 0;
-      if (grad_score != nullptr) {
-        for (int k = 0; k < 4; ++k) grad_score[gp * 4 + k] = 0;
+    for (int r = 0; r < kPer; ++r) {
+      mine[r] = rec[r]; gp[r] = gpi[r];
+      bin[r] = -1; rank[r] = 0;
+      if (!live[r]) continue;
+      bin[r] = tab.bin(level[r], __uint_as_float(mine[r].x), __uint_as_float(mine[r].y), divs);
+      if (bin[r] >= 0) {
+        rank[r] = atomicAdd(&s_cnt[bin[r]], 1);
+      } else {
+        // skipped by the operator: all its gradients are zero, and no tile will visit it
+        const size_t at = gp[r];
+        for (int c = 0; c < gl_stride; ++c) grad_loc[at * gl_stride + c] = 0;
+        if (grad_attn != nullptr) grad_attn[at] = 0;
+        if (grad_score != nullptr) {
+          for (int k = 0; k < 4; ++k) grad_score[at * 4 + k] = 0;
+        }
       }
     }
-  }
-  __syncthreads();
-  // 2. runs: reserve this block's run in every touched bin's segment; staged order = bins in order (exclusive scan)
-  {
-    constexpr int kBinsPer = kSortedBins / kFillThreads;                  // consecutive bins per thread
-    int c[kBinsPer], sum = 0;
+    lds_barrier();
+    // 2. runs: reserve this turn's run in every touched bin's segment; staged order = bins in order (exclusive scan).
+    // The next turn's points are asked for behind the reservations, and have come when this turn's are written out.
+    {
+      constexpr int kBinsPer = kSortedBins / kFillThreads;                  // consecutive bins per thread
+      int c[kBinsPer], base[kBinsPer], sum = 0;
 #pragma unroll
-    for (int j = 0; j < kBinsPer; ++j) {
-      const int i = tid * kBinsPer + j;
-      c[j] = i < nb ? s_cnt[i] : 0;
-      sum += c[j];
-      if (c[j] > 0) s_base[i] = atomicAdd(&gcursor[i], c[j]);
-    }
-    const int inc = wave_inclusive_scan(sum);
-    if (lane == kWave - 1) s_wave[wave] = inc;
-    __syncthreads();
-    int run = inc - sum;
-    for (int w = 0; w < wave; ++w) run += s_wave[w];
+      for (int j = 0; j < kBinsPer; ++j) {
+        const int i = tid * kBinsPer + j;
+        c[j] = i < nb ? s_cnt[i] : 0;
+        s_cnt[i] = 0;
+        sum += c[j];
+        base[j] = 0;
+        if (c[j] > 0) base[j] = atomicAdd(&gcursor[i], c[j]);
+      }
+      if constexpr (decltype(more)::value) ask(turn_of(blk + gridDim.x));
+      const int inc = wave_inclusive_scan(sum);
+      if (lane == kWave - 1) s_wave[wave] = inc;
+      lds_barrier();
+      int run = inc - sum;
+      for (int w = 0; w < wave; ++w) run += s_wave[w];
 #pragma unroll
-    for (int j = 0; j < kBinsPer; ++j) {
-      const int i = tid * kBinsPer + j;
-      if (i < nb) s_lofs[i] = run;
-      run += c[j];
+      for (int j = 0; j < kBinsPer; ++j) {
+        const int i = tid * kBinsPer + j;
+        s_lofs[i] = run;
+        s_base[i] = base[j];
+        run += c[j];
+      }
+      if (tid == kFillThreads - 1) s_lofs[kSortedBins] = run;                   // number of staged points
     }
-    if (tid == kFillThreads - 1) s_lofs[kSortedBins] = run;                   // number of staged points
-  }
-  __syncthreads();
-  // 3. stage
+    lds_barrier();
+    // 3. stage
 #pragma unroll
-  for (int r = 0; r < kPer; ++r) {
-    if (bin[r] >= 0) {
-      const int pos = s_lofs[bin[r]] + rank[r];
-      s_rec[pos] = rec[r];
-      s_gp[pos] = gpi[r];
-      s_dst[pos] = s_base[bin[r]] + rank[r];
+    for (int r = 0; r < kPer; ++r) {
+      if (bin[r] >= 0) {
+        const int pos = s_lofs[bin[r]] + rank[r];
+        s_rec[pos] = mine[r];
+        s_gp[pos] = gp[r];
+        s_dst[pos] = s_base[bin[r]] + rank[r];
+      }
     }
-  }
-  __syncthreads();
-  // 4. write out: consecutive staged slots of one bin go to consecutive addresses
-  const int total = s_lofs[kSortedBins];
-  for (int i = tid; i < total; i += kFillThreads) {
-    const int dst = s_dst[i];
-    ws.recs[dst] = *reinterpret_cast<const float4 *>(&s_rec[i]);
-    ws.entries[dst] = s_gp[i];
-  }
+#pragma unroll
+    for (int r = 0; r < kPer && decltype(more)::value; ++r) asm volatile("" : "+v"(rec[r].x), "+v"(rec[r].y), "+v"(rec[r].z), "+v"(rec[r].w));      // waits for them here: behind the stores it would wait for those too
+    lds_barrier();
+    // 4. write out: consecutive staged slots of one bin go to consecutive addresses
+    const int total = s_lofs[kSortedBins];
+    for (int i = tid; i < total; i += kFillThreads) {
+      const int dst = s_dst[i];
+      ws.recs[dst] = *reinterpret_cast<const float4 *>(&s_rec[i]);
+      ws.entries[dst] = s_gp[i];
+    }
+  };
+  unsigned blk = blockIdx.x;
+  for (; blk + gridDim.x < n_turns; blk += gridDim.x) turn(blk, std::true_type());
+  if (blk < n_turns) turn(blk, std::false_type());
 }
 
 // What the tile kernel adds to instead of storing, cleared for a caller that did not zero grad_value / grad_dist
@@ -1632,16 +1677,20 @@ static hipError_t run_binning(const BwdArgs &a, const BinWorkspace &ws, const Ti
                      a.L, a.S, (a.dist != nullptr || a.C == 0) ? a.D : 0, a.B, a.M, ty, tx, chunk, mb);
   const int LP = a.L * a.P;
   const bool sorted_maybe = LP <= kStage, sorted_surely = sorted_maybe && mb <= kSortedBins;
-  const int nq_block = sorted_maybe ? kStage / LP : 1;           // (bin_points_in_order makes its own of it)
-  const int q_blocks = (a.Q + nq_block - 1) / nq_block;
+  const int q_turn = sorted_maybe ? kStage / LP : 1;             // (bin_points_in_order makes its own of it)
+  const int q_blocks = (a.Q + q_turn - 1) / q_turn;
   const long long blocks = (long long)a.B * a.M * q_blocks;
   if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
-  const unsigned grid = sorted_maybe || blocks < 2048 ? (unsigned)blocks : 2048u;
+  const int held = tile_grid(kSortedFillLds, kFillThreads);       // blocks of kFillThreads that the chip holds
+  const unsigned grid = blocks < held ? (unsigned)blocks : (unsigned)held;
   const int hist_cap = sorted_surely ? 0 : mb < kHistCap ? mb : kHistCap;
   static_assert((size_t)kHistCap * 8 <= kSortedFillLds, "bin_points_in_order's counters lie in the sorted fill's LDS");
   const BinDivs divs{FastDiv((uint32_t)LP), FastDiv((uint32_t)a.P), FastDiv((uint32_t)ty), FastDiv((uint32_t)tx)};
-  hipLaunchKernelGGL(bin_count_kernel, dim3(grid), dim3(kFillThreads), (size_t)hist_cap * 4, stream, ws, (const float *)a.loc,
-                     a.loc_stride, a.B, a.M, a.L, a.Q, a.P, nq_block, q_blocks, hist_cap, divs);
+  // blocks of the count per (batch, head): what the chip holds, all with as many turns
+  const int parts_held = std::max(1, held / std::min(held, a.B * a.M)), turns = (q_blocks + parts_held - 1) / parts_held;
+  const int parts = (q_blocks + turns - 1) / turns;
+  hipLaunchKernelGGL(bin_count_kernel, dim3((unsigned)(a.B * a.M * parts)), dim3(kFillThreads), (size_t)hist_cap * 4, stream, ws,
+                     (const float *)a.loc, a.loc_stride, a.B, a.M, a.L, a.Q, a.P, q_turn, parts, hist_cap, divs);
   // What further blocks of the scan's launch clear meanwhile: for a caller that did not zero them (options.clear),
   // the rows of grad_value / grad_dist that the tile kernel adds to rather than stores; and always, for a
   // distribution shared by the heads, those rows of the per-head grad_dist in the workspace (the head sum then
