@@ -136,7 +136,7 @@ constexpr int kSortedBins = 2048;   // bins of one (batch, head) the sorted fill
 constexpr int kStage = 2048;        // points a block of the sorted fill stages (1024: 0.39 ms, 4096: 0.36 ms against 0.32 ms)
 constexpr int kFillThreads = 1024;  // 256 / 512 threads: 0.49 / 0.38 ms
 __host__ __device__ inline bool sorted_fill_applies(int bins_per_bm, int LP) { return bins_per_bm <= kSortedBins && LP <= kStage; }
-constexpr size_t kSortedFillLds = (size_t)kStage * (16 + 4 + 4) + (size_t)(3 * kSortedBins + 1) * 4;
+constexpr size_t kSortedFillLds = (size_t)kStage * (16 + 4 + 2) + (size_t)(3 * kSortedBins + 1) * 4;
 
 // this block's part of the total that chunk_of() reads
 __device__ __forceinline__ int *counted_points(const BinWorkspace &ws) { return &ws.queues[(blockIdx.x % kClasses) * kQueueStride + 1]; }
@@ -259,7 +259,8 @@ struct BinDivs { FastDiv lp, p, ty, tx; };
 // come, and four divisions by numbers the compiler does not know.  15.36 M points: count 89 -> 52 us, fill 195 -> 153 us.
 // Both kernels then had a block per turn, which waited for its points, then for its reservations.  As many blocks as the
 // chip holds, with the next turn's points on their way while they work on one: count 52 -> 36 us (184 MB read, 5.1 TB/s), fill
-// 153 -> 144 us (553 MB moved, 3.8 TB/s, where a copy reaches 4.7); 61 M clustered points count 281 -> 134 us, fill 595 -> 584.
+// 153 -> 144 us, and 141 since it waits for its reservations only when it has staged the points (553 MB moved, 3.9 TB/s, where a
+// copy reaches 4.7); 61 M clustered points count 281 -> 134 us, fill 595 -> 575.
 struct BinTable {
   int H[DFA3D_MAX_LEVELS], W[DFA3D_MAX_LEVELS], base[DFA3D_MAX_LEVELS], tiles_x[DFA3D_MAX_LEVELS];
   __device__ __forceinline__ void load(const BinPlan &p) {     // the caller's barrier
@@ -354,10 +355,10 @@ __global__ __launch_bounds__(kFillThreads, 8) void bin_fill_sorted_kernel(
   __shared__ BinTable tab;
   uint4 *s_rec = reinterpret_cast<uint4 *>(s_raw);               // staged records, grouped by bin
   uint32_t *s_gp = reinterpret_cast<uint32_t *>(s_rec + kStage);
-  int *s_dst = reinterpret_cast<int *>(s_gp + kStage);
-  int *s_cnt = s_dst + kStage;                                   // points of this block per bin
+  uint16_t *s_bin = reinterpret_cast<uint16_t *>(s_gp + kStage);
+  int *s_cnt = reinterpret_cast<int *>(s_bin + kStage);                                   // points of this block per bin
   int *s_lofs = s_cnt + kSortedBins;                             // first staged slot of each bin; [kSortedBins]: total
-  int *s_base = s_lofs + kSortedBins + 1;                        // first slot of this block's run in the bin's segment
+  int *s_shift = s_lofs + kSortedBins + 1;                       // from a staged slot to the record's place, by bin
   __shared__ int s_wave[kFillThreads / kWave];
   const BinPlan &p = *ws.plan;
   const int nb = p.bins_per_bm;
@@ -392,17 +393,15 @@ __global__ __launch_bounds__(kFillThreads, 8) void bin_fill_sorted_kernel(
     return t;
   };
   uint4 rec[kPer];
-  uint32_t gpi[kPer];
-  bool live[kPer];
+  auto first_of = [&](const Turn &t) { return (uint32_t)(((size_t)t.b * Q + t.qb) * M + t.m) * LP; };
   auto ask = [&](const Turn &t) {                                // always asked for, so that the waits can be counted
-    const uint32_t first = (uint32_t)(((size_t)t.b * Q + t.qb) * M + t.m) * LP;
+    const uint32_t first = first_of(t);
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-      live[r] = t.qb + qi[r] < Q;
-      gpi[r] = live[r] ? first + from[r] : first;
-      const float *at = loc + (size_t)gpi[r] * loc_stride;
+      const uint32_t gp = t.qb + qi[r] < Q ? first + from[r] : first;
+      const float *at = loc + (size_t)gp * loc_stride;
       rec[r] = make_uint4(__float_as_uint(at[0]), __float_as_uint(at[1]), loc_stride > 2 ? __float_as_uint(at[2]) : 0u,
-                          attn != nullptr ? __float_as_uint(attn[gpi[r]]) : 0u);
+                          attn != nullptr ? __float_as_uint(attn[gp]) : 0u);
     }
   };
   const unsigned n_turns = (unsigned)(B * M * q_blocks);
@@ -417,18 +416,17 @@ __global__ __launch_bounds__(kFillThreads, 8) void bin_fill_sorted_kernel(
     // 1. every point: its bin and its rank among this turn's points of that bin
     int bin[kPer], rank[kPer];
     uint4 mine[kPer];
-    uint32_t gp[kPer];
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-      mine[r] = rec[r]; gp[r] = gpi[r];
+      mine[r] = rec[r];
       bin[r] = -1; rank[r] = 0;
-      if (!live[r]) continue;
+      if (t.qb + qi[r] >= Q) continue;
       bin[r] = tab.bin(level[r], __uint_as_float(mine[r].x), __uint_as_float(mine[r].y), divs);
       if (bin[r] >= 0) {
         rank[r] = atomicAdd(&s_cnt[bin[r]], 1);
       } else {
         // skipped by the operator: all its gradients are zero, and no tile will visit it
-        const size_t at = gp[r];
+        const size_t at = first_of(t) + from[r];
         for (int c = 0; c < gl_stride; ++c) grad_loc[at * gl_stride + c] = 0;
         if (grad_attn != nullptr) grad_attn[at] = 0;
         if (grad_score != nullptr) {
@@ -437,11 +435,12 @@ __global__ __launch_bounds__(kFillThreads, 8) void bin_fill_sorted_kernel(
       }
     }
     lds_barrier();
+    int base[kSortedBins / kFillThreads];
     // 2. runs: reserve this turn's run in every touched bin's segment; staged order = bins in order (exclusive scan).
     // The next turn's points are asked for behind the reservations, and have come when this turn's are written out.
     {
       constexpr int kBinsPer = kSortedBins / kFillThreads;                  // consecutive bins per thread
-      int c[kBinsPer], base[kBinsPer], sum = 0;
+      int c[kBinsPer], sum = 0;
 #pragma unroll
       for (int j = 0; j < kBinsPer; ++j) {
         const int i = tid * kBinsPer + j;
@@ -461,7 +460,6 @@ __global__ __launch_bounds__(kFillThreads, 8) void bin_fill_sorted_kernel(
       for (int j = 0; j < kBinsPer; ++j) {
         const int i = tid * kBinsPer + j;
         s_lofs[i] = run;
-        s_base[i] = base[j];
         run += c[j];
       }
       if (tid == kFillThreads - 1) s_lofs[kSortedBins] = run;                   // number of staged points
@@ -473,9 +471,15 @@ __global__ __launch_bounds__(kFillThreads, 8) void bin_fill_sorted_kernel(
       if (bin[r] >= 0) {
         const int pos = s_lofs[bin[r]] + rank[r];
         s_rec[pos] = mine[r];
-        s_gp[pos] = gp[r];
-        s_dst[pos] = s_base[bin[r]] + rank[r];
+        s_gp[pos] = first_of(t) + from[r];
+        s_bin[pos] = (uint16_t)bin[r];
       }
+    }
+    // the reservations are only now waited for
+#pragma unroll
+    for (int j = 0; j < kSortedBins / kFillThreads; ++j) {
+      const int i = tid * (kSortedBins / kFillThreads) + j;
+      s_shift[i] = base[j] - s_lofs[i];
     }
 #pragma unroll
     for (int r = 0; r < kPer && decltype(more)::value; ++r) asm volatile("" : "+v"(rec[r].x), "+v"(rec[r].y), "+v"(rec[r].z), "+v"(rec[r].w));      // waits for them here: behind the stores it would wait for those too
@@ -483,7 +487,7 @@ __global__ __launch_bounds__(kFillThreads, 8) void bin_fill_sorted_kernel(
     // 4. write out: consecutive staged slots of one bin go to consecutive addresses
     const int total = s_lofs[kSortedBins];
     for (int i = tid; i < total; i += kFillThreads) {
-      const int dst = s_dst[i];
+      const int dst = s_shift[s_bin[i]] + i;
       ws.recs[dst] = *reinterpret_cast<const float4 *>(&s_rec[i]);
       ws.entries[dst] = s_gp[i];
     }
