@@ -1168,16 +1168,16 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
 // each point is given; grad_dist is accumulated in an LDS tile, the z gradient written per point.
 //
 // What bounds it is the random access of each point (its score gradient, its z gradient, four pairs of bins) and the
-// tile's way out, so the kernel keeps both going at once: four workgroups per CU, no barrier between the points of
-// an item (taps go to LDS by compare-and-swap, so nobody waits for anybody), the next round's records asked for one
-// round ahead and the next item's before the tile is flushed.  For a caller whose buffer may hold anything, a pixel that
+// tile's way out, so the kernel keeps both going at once: no barrier between the points of an item (taps go to LDS by
+// compare-and-swap, so nobody waits for anybody), the next round's records asked for one round ahead and the next item's
+// before the tile is flushed.  The bins come from the caches as long as few tiles are worked on at a time: 16 wavefronts per CU
+// either way, one workgroup of 1024 threads beats four of 256 where tiles have the points for it (BLOCK: tile_config_of).  For a caller whose buffer may hold anything, a pixel that
 // only this item can touch (no neighbour's halo, all the points of its bin, levels that share no keys) is stored 16
 // bytes per lane; everything else is added atomically, one float per lane on consecutive addresses.
 // 6 x 9502 queries, 4 levels from 116 x 200, 8 points, 112 bins (14.6 M points): 1.19 ms with a ticket per tap and
-// three barriers per 256 points, 1.01 ms now; with parts cut out, the z gradients' scattered stores are 0.27 of it, the
+// three barriers per 256 points, 1.01 ms without them and 0.85 ms with 1024 threads per tile; with parts cut out of the 1.01, the z gradients' scattered stores are 0.27 of it, the
 // tiles' way out 0.2, the taps 0.10, the score gradients' gathers 0.09.
 // ---------------------------------------------------------------------------------------
-constexpr int kDepthBlock = 256;
 // The fetching thread's state: the queue is asked for an item's number when another item is begun, the answer is looked
 // at when that one's points are done, and the records asked for then are handed over with the next item.
 struct DepthFetch {
@@ -1201,8 +1201,8 @@ struct DepthFetch {
     load(ws, w >= 0 ? w : pop_item(ws, p, home, classes_done));
   }
 };
-template <typename T>
-__global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
+template <typename T, int BLOCK>
+__global__ __launch_bounds__(BLOCK, 4) void tile_depth_backward_kernel(
     BinWorkspace ws, const T *__restrict__ dist, const T *__restrict__ grad_score, float *__restrict__ grad_dist,
     float *__restrict__ grad_loc3, int B, int S, int M, int D, int L, int Q, int P, int stores) {
   // stores: the binning launches cleared what is added to here and nothing else (clear_unstored), else everything is added
@@ -1218,7 +1218,7 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
   const int TY = p.ty, TX = p.tx, TW = TX + 1, R = (TY + 1) * TW;
   const int tid = threadIdx.x;
   float *gd = smem;
-  for (int i = tid; i < R * D; i += kDepthBlock) gd[i] = 0;
+  for (int i = tid; i < R * D; i += BLOCK) gd[i] = 0;
   if (tid < DFA3D_MAX_LEVELS) {
     s_lv[0][tid] = p.H[tid]; s_lv[1][tid] = p.W[tid]; s_lv[2][tid] = p.Dd[tid]; s_lv[3][tid] = p.start[tid];
   }
@@ -1255,11 +1255,11 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
     const int Dd = __builtin_amdgcn_readfirstlane(s_lv[2][l]), start = __builtin_amdgcn_readfirstlane(s_lv[3][l]);
     const rsrc_t dist_r = make_rsrc(dist + (size_t)b * S * M * D, (size_t)S * M * D * sizeof(T));
 
-    for (int base = 0; base < n_item; base += kDepthBlock) {       // uniform over the workgroup
+    for (int base = 0; base < n_item; base += BLOCK) {       // uniform over the workgroup
       const bool live = base + tid < n_item;
       const uint32_t gp = next_gp;
       const float4 rec = next_rec;
-      if (base + kDepthBlock < n_item) ask_record(seg, n_item, base + kDepthBlock + tid);
+      if (base + BLOCK < n_item) ask_record(seg, n_item, base + BLOCK + tid);
       if (live) {
         const T *gi = grad_score + (size_t)gp * 4;
         float g4[4];
@@ -1298,7 +1298,7 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
     auto lanes_log2 = [](int n) { return n > 32 ? 6 : n > 16 ? 5 : n > 8 ? 4 : n > 4 ? 3 : 2; };
     if (sole) {
       const int n = D >> 2, sh = lanes_log2(n), inner = (TY - 1) * (TX - 1);
-      for (int i = tid >> sh; i < inner; i += kDepthBlock >> sh) {
+      for (int i = tid >> sh; i < inner; i += BLOCK >> sh) {
         const int ry = i / (TX - 1) + 1, rx = i % (TX - 1) + 1, y = y0 + ry, x = x0 + rx;
         const uint32_t e0 = (uint32_t)((((start + y * W + x) * M + m) * D) * 4);
         for (int c = tid & ((1 << sh) - 1); c < n; c += 1 << sh) {
@@ -1311,7 +1311,7 @@ __global__ __launch_bounds__(kDepthBlock, 4) void tile_depth_backward_kernel(
       }
     }
     const int sh = lanes_log2(D), rows = sole ? rim_pixels(TY, TX) : R;
-    for (int i = tid >> sh; i < rows; i += kDepthBlock >> sh) {
+    for (int i = tid >> sh; i < rows; i += BLOCK >> sh) {
       int ry, rx;
       if (sole) {
         rim_decode(i, TY, TX, ry, rx);
@@ -1461,7 +1461,7 @@ static size_t tile_lds_bytes(int kind, int ty, int tx, int C, int D, int pp) {
 //   * an 8x8 tile at pp 128 beats a 4x8 tile at pp 256 (128 bins: 0.68 against 0.74 ms for 2.56 M points) unless
 //     most tiles take several passes (`dense`: the dense BEV workload, 41 points per pixel, 7.0 against 8.9 ms).
 static TileConfig pick_tile_config(int kind, int C, int D, int elem, int tile_hint, int block_hint, int pass_hint, bool dense,
-                                   bool cells_wanted) {
+                                   bool cells_wanted, int depth_block, bool depth_small) {
   TileConfig c;
   c.cells = false;
   if (cells_wanted && kind != 2 && C <= 64 && (block_hint == 0 || block_hint == cell_kernel_block(C)) &&
@@ -1480,10 +1480,10 @@ static TileConfig pick_tile_config(int kind, int C, int D, int elem, int tile_hi
       }
     }
   }
-  c.block = kind == 2 ? 256 : (block_hint == 256 ? 256 : 512);
+  c.block = kind == 2 ? depth_block : (block_hint == 256 ? 256 : 512);
   const int pp_max = kind == 2 ? c.block : c.block / 2;      // the fused tile kernel wants two halves of pp threads
   auto clamp_pp = [&](int pp) { return pp > pp_max ? pp_max : pp; };
-  const size_t two_per_cu = kind == 2 ? 40 * 1024 : 79 * 1024, one_per_cu = 150 * 1024;
+  const size_t two_per_cu = kind == 2 && depth_block == 256 ? 40 * 1024 : 79 * 1024, one_per_cu = 150 * 1024;
   const int hy = tile_hint / 100, hx = tile_hint % 100;
   const bool tile_given = tile_hint > 0 && hy >= 1 && hx >= 1 && hy <= 64 && hx <= 64;
   const bool pass_given = pass_hint == 64 || pass_hint == 128 || pass_hint == 256;
@@ -1499,6 +1499,7 @@ static TileConfig pick_tile_config(int kind, int C, int D, int elem, int tile_hi
   static const Pref dense_order[] = {{8, 16, 256}, {8, 8, 256}, {4, 8, 256}, {4, 4, 256}, {8, 8, 128}, {4, 8, 128},
                                      {4, 4, 128}, {8, 8, 64}, {4, 8, 64}, {4, 4, 64}};
   const Pref *order = dense ? dense_order : sparse_order;
+  if (kind == 2 && depth_small && !tile_given && fits(8, 8, 256, two_per_cu)) return done(8, 8, 256);
   for (size_t budget : {two_per_cu, one_per_cu}) {
     for (int i = 0; i < 10; ++i) {
       const int ty = tile_given ? hy : order[i].ty, tx = tile_given ? hx : order[i].tx;
@@ -1521,7 +1522,17 @@ static TileConfig tile_config_of(const BwdArgs &a, int kind, int dtype) {
   // a caller that names the channels per lane asks for the row-owned kernel, whose tiling that is
   // (its per-point gradients are buffer-addressed per batch element: below 2^31 bytes of 16 per point)
   const bool cells = a.vec_hint == 0 && (size_t)a.Q * a.M * a.L * a.P * 16 < (size_t)kNoRow;
-  return pick_tile_config(kind, a.C, a.D, dtype == DFA3D_F32 ? 4 : 2, a.tile_hint, a.block_hint, a.pass_hint, per_pixel >= 16.0, cells);
+  // Stage 1 alone: threads per tile by the points it can expect, and 8 x 8 tiles instead of 8 x 16 where those would give
+  // a CU only a few.  The call, four levels from 116 x 200 unless said, 256 / 512 / 1024 threads:
+  //   6 x 9502 queries, 32 points each (10 per pixel), 112 bins 1224 / 1154 / 1065 us, 64 bins 1109 / 950 / 872, 16 bins 930 / 750 / 717
+  //   6 x 4000 queries, 16 points (2 per pixel), 64 bins 387 / 367 / 404; 6 x 2000 281 / 284 / 336
+  //   4 x 1000 queries, 16 points (0.5 per pixel), 48 bins 161 / 174 / 212
+  //   8 x 8 for 8 x 16 tiles, 1024 threads: 6 x 4000 queries, 8 points, 23 x 40, 112 bins (345 tiles) 144 -> 122; 2 x 9502 queries,
+  //   32 points, 4 heads, 80 bins (1927 tiles) 230 -> 222; 6 x 9502 queries, 112 bins (11559 tiles) 1065 -> 1097
+  const int depth_block = per_pixel < 0.75 ? 256 : per_pixel < 3.0 ? 512 : 1024;
+  const bool depth_small = depth_block == 1024 && (double)a.S * a.B * a.M / 128 < 4096;
+  return pick_tile_config(kind, a.C, a.D, dtype == DFA3D_F32 ? 4 : 2, a.tile_hint, a.block_hint, a.pass_hint, per_pixel >= 16.0, cells,
+                          depth_block, depth_small);
 }
 
 // Whether bfloat16 gradients are summed in float in the workspace and rounded once at the end.  A bfloat16 buffer rounds at
@@ -1791,6 +1802,19 @@ size_t binned_depth_score_backward_workspace_bytes(const DepthScoreBwdArgs &d, i
   return workspace_bytes_for(a, 2, dtype);
 }
 
+template <typename T>
+static hipError_t launch_depth_tiles(const DepthScoreBwdArgs &d, const BinWorkspace &ws, const TileConfig &cfg, int stores, hipStream_t stream) {
+  auto launch = [&](auto kern) -> hipError_t {
+    if (hipError_t e = allow_lds(kern, cfg.lds)) return e;
+    hipLaunchKernelGGL(kern, dim3(tile_grid(cfg.lds, cfg.block)), dim3(cfg.block), cfg.lds, stream, ws, (const T *)d.dist, (const T *)d.grad_score,
+                       (float *)d.grad_dist, (float *)d.grad_loc3, d.B, d.S, d.M, d.D, d.L, d.Q, d.P, stores);
+    return hipGetLastError();
+  };
+  if (cfg.block == 1024) return launch(tile_depth_backward_kernel<T, 1024>);
+  if (cfg.block == 512) return launch(tile_depth_backward_kernel<T, 512>);
+  return launch(tile_depth_backward_kernel<T, 256>);
+}
+
 hipError_t launch_depth_score_backward_binned(const DepthScoreBwdArgs &d, int dtype, void *workspace,
                                               size_t workspace_bytes, int tile_hint, int chunk_hint,
                                               void *event_binned, hipStream_t stream) {
@@ -1812,20 +1836,7 @@ hipError_t launch_depth_score_backward_binned(const DepthScoreBwdArgs &d, int dt
   if (event_binned != nullptr) {
     if (hipError_t e = hipEventRecord((hipEvent_t)event_binned, stream)) return e;
   }
-  const int grid = tile_grid(cfg.lds, cfg.block);
-  if (hipError_t e = dtype == DFA3D_F32 ? allow_lds(tile_depth_backward_kernel<float>, cfg.lds)
-                                        : allow_lds(tile_depth_backward_kernel<__hip_bfloat16>, cfg.lds))
-    return e;
-  if (dtype == DFA3D_F32) {
-    hipLaunchKernelGGL(tile_depth_backward_kernel<float>, dim3(grid), dim3(cfg.block), cfg.lds, stream, ws,
-                       (const float *)d.dist, (const float *)d.grad_score, (float *)d.grad_dist, (float *)d.grad_loc3,
-                       d.B, d.S, d.M, d.D, d.L, d.Q, d.P, stores);
-  } else {
-    hipLaunchKernelGGL(tile_depth_backward_kernel<__hip_bfloat16>, dim3(grid), dim3(cfg.block), cfg.lds, stream, ws,
-                       (const __hip_bfloat16 *)d.dist, (const __hip_bfloat16 *)d.grad_score, (float *)d.grad_dist,
-                       (float *)d.grad_loc3, d.B, d.S, d.M, d.D, d.L, d.Q, d.P, stores);
-  }
-  return hipGetLastError();
+  return dtype == DFA3D_F32 ? launch_depth_tiles<float>(d, ws, cfg, stores, stream) : launch_depth_tiles<__hip_bfloat16>(d, ws, cfg, stores, stream);
 }
 
 }  // namespace dfa3d
