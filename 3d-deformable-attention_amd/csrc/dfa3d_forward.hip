@@ -7,6 +7,8 @@
 //                                           (wms_deform_attn_cuda_kernel.cuh:240-303)
 //   depth_score_kernel                      stage 1 alone
 //                                           (ms_depth_score_sample_cuda_kernel.cuh:94-148)
+#include <type_traits>
+
 #include "dfa3d_device.h"
 #include "dfa3d_launch.h"
 
@@ -245,37 +247,69 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
-// Stage 1 alone: one lane per sampling point.  Block id -> (head, batch, block of kDsQueries
-// queries) with head = block % M, as in the attention kernels: the distributions one XCD's L2
-// sees are those of one head.
+// Stage 1 alone: one lane per sampling point.  Block id -> (head, block of queries, group of levels, batch) with head =
+// block % M, as in the attention kernels: the distributions one XCD's L2 sees are those of one head.
+//
+// Bound by the gathers, a cache line for each of a point's four pairs of bins.  So a group is one level: what an XCD reads at a time
+// is then one head's distributions of one level, which the L2 holds but for the finest, where all levels together (13.8 MB
+// with 112 bins) pushed one another out.  And a lane takes four points at a time, sixteen gathers in flight, where a block has
+// them; it has where the launch would be more than 4096 blocks of 1024 points.  6 x 9502 queries, four levels from
+// 116 x 200, 8 points (14.6 M points), 112 bins 536 -> 496 us level by level, 470 with four points at a time; 64 bins 514 / 440 /
+// 403, 16 bins 439 / 372 / 331, bfloat16 446 / 432 / 402.  Below four points per level a level's locations and scores
+// are less than half a line each: all levels together (2 points: 53 against 55 us for 1.3 M points).
 // ---------------------------------------------------------------------------------------
-constexpr int kDsQueries = 32;
+struct DepthScoreShape { int levels, points; };          // levels per group, points per block at most
+__host__ __device__ inline DepthScoreShape depth_score_shape(int B, int M, int L, int Q, int P) {
+  return DepthScoreShape{P >= 4 ? 1 : L, (long long)B * M * L * Q * P > 4096LL * 1024 ? 1024 : 256};
+}
+__host__ __device__ inline int depth_score_queries(const DepthScoreShape &s, int P) { return s.points > s.levels * P ? s.points / (s.levels * P) : 1; }
 template <typename T, typename A>
 __global__ __launch_bounds__(kBlock) void depth_score_kernel(
     const T *__restrict__ dist, const int64_t *__restrict__ shapes3, const int64_t *__restrict__ level_start,
     const A *__restrict__ loc3, T *__restrict__ score, int B, int S, int M, int D, int L, int Q, int P) {
   __shared__ LevelTable tab;
   load_level_table(tab, shapes3, 3, level_start, L, S, D);
-  const int LP = L * P;
+  const DepthScoreShape shape = depth_score_shape(B, M, L, Q, P);
+  const int queries = depth_score_queries(shape, P), q_blocks = (Q + queries - 1) / queries, groups = L / shape.levels;
   const int m = blockIdx.x % M;
-  const int rest = blockIdx.x / M;
-  const int q_blocks = (Q + kDsQueries - 1) / kDsQueries;
-  const int qb = rest % q_blocks, b = rest / q_blocks;
-  const int q0 = qb * kDsQueries, nq = min(kDsQueries, Q - q0);
+  int rest = blockIdx.x / M;
+  const int q0 = rest % q_blocks * queries;
+  rest /= q_blocks;
+  const int l0 = rest % groups * shape.levels, b = rest / groups;
+  const int per_query = shape.levels * P, n = min(queries, Q - q0) * per_query;
   const rsrc_t dist_r = make_rsrc(dist + (size_t)b * S * M * D, (size_t)S * M * D * sizeof(T));
-  for (int i = threadIdx.x; i < nq * LP; i += kBlock) {
-    const int ql = i / LP, lp = i - ql * LP;
-    const size_t gp = (((size_t)b * Q + q0 + ql) * M + m) * LP + lp;
-    const int l = lp / P;
-    const A *pl = loc3 + gp * 3;
-    const Point2D<A> g = locate_2d<A>(pl[0], pl[1], tab.H[l], tab.W[l], tab.start[l]);
-    const DepthTap<A> tap = locate_depth<A>(pl[2], tab.Dd[l]);
-    A sc[4], lo[4], hi[4];
-    corner_scores<T, A>(dist_r, g.key, tap, m, M, D, sc, lo, hi);
-    T *so = score + gp * 4;
+  // points i, i + kBlock, ... N of them
+  auto points = [&](int i, auto count) {
+    constexpr int N = decltype(count)::value;
+    A x[N], y[N], z[N];
+    size_t gp[N];
+    int l[N];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) Elem<T>::st(so + k, sc[k]);
-  }
+    for (int r = 0; r < N; ++r) {
+      const int ql = (i + r * kBlock) / per_query, lp = i + r * kBlock - ql * per_query;
+      l[r] = shape.levels == 1 ? l0 : lp / P;
+      gp[r] = (((size_t)b * Q + q0 + ql) * M + m) * ((size_t)L * P) + l0 * P + lp;
+      const A *pl = loc3 + gp[r] * 3;
+      x[r] = pl[0]; y[r] = pl[1]; z[r] = pl[2];
+    }
+    A sc[N][4];
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      const Point2D<A> g = locate_2d<A>(x[r], y[r], tab.H[l[r]], tab.W[l[r]], tab.start[l[r]]);
+      const DepthTap<A> tap = locate_depth<A>(z[r], tab.Dd[l[r]]);
+      A lo[4], hi[4];
+      corner_scores<T, A>(dist_r, g.key, tap, m, M, D, sc[r], lo, hi);
+    }
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      T *so = score + gp[r] * 4;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) Elem<T>::st(so + k, sc[r][k]);
+    }
+  };
+  int i = threadIdx.x;
+  for (; i - (int)threadIdx.x + 4 * kBlock <= n; i += 4 * kBlock) points(i, std::integral_constant<int, 4>());      // uniform
+  for (; i < n; i += kBlock) points(i, std::integral_constant<int, 1>());
 }
 
 // ---------------------------------------------------------------------------------------
@@ -388,7 +422,9 @@ hipError_t launch_forward(const FwdArgs &a, int dtype, hipStream_t stream) {
 
 template <typename T, typename A>
 static hipError_t launch_ds_typed(const DepthScoreArgs &a, hipStream_t stream) {
-  const long long blocks = (long long)a.M * a.B * ((a.Q + kDsQueries - 1) / kDsQueries);
+  const DepthScoreShape shape = depth_score_shape(a.B, a.M, a.L, a.Q, a.P);
+  const int queries = depth_score_queries(shape, a.P);
+  const long long blocks = (long long)a.M * a.B * (a.L / shape.levels) * ((a.Q + queries - 1) / queries);
   if (blocks <= 0 || blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
   hipLaunchKernelGGL((depth_score_kernel<T, A>), dim3((unsigned)blocks), dim3(kBlock), 0, stream, (const T *)a.dist,
                      a.shapes3, a.level_start, (const A *)a.loc3, (T *)a.score, a.B, a.S, a.M, a.D, a.L, a.Q, a.P);
