@@ -45,6 +45,21 @@ def _on_gpu(**tensors):
     return dev
 
 
+def _contig_on_gpu(**tensors):
+    """``_contig`` and ``_on_gpu`` in one pass; they say what is wrong where something is.  With ``_fused_dims`` this is
+    what a small call spends on checks (2 x 100 queries on 16 x 16 maps, forward: 19.6 -> 17.3 us)."""
+    at = -1
+    for t in tensors.values():
+        if not t.is_contiguous() or not t.is_cuda or t.get_device() != at:
+            if at >= 0 or not t.is_contiguous() or not t.is_cuda:
+                break
+            at = t.get_device()
+    else:
+        return t.device
+    _contig(**tensors)
+    return _on_gpu(**tensors)
+
+
 def _step(batch, im2col_step):
     step = min(batch, int(im2col_step))
     if step <= 0 or batch % step != 0:
@@ -81,10 +96,8 @@ def _geometry(shapes, lsi, loc, width, name):
 def ms_depth_score_sample_forward(value, value_spatial_shapes, value_level_start_index,
                                   sampling_locations, im2col_step):
     """value = depth distributions (bs, num_keys, num_heads, D) -> (bs, Q, heads, L, P, 4)."""
-    _contig(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
-            sampling_loc=sampling_locations)
-    dev = _on_gpu(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
-                  sampling_loc=sampling_locations)
+    dev = _contig_on_gpu(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
+                         sampling_loc=sampling_locations)
     if value.dim() != 4:
         raise RuntimeError(f"value must be (bs, num_keys, num_heads, D), got {tuple(value.shape)}")
     B, S, M, D = value.shape
@@ -117,12 +130,9 @@ def ms_depth_score_sample_backward_into(value, value_spatial_shapes, value_level
                                         grad_output, grad_value, grad_sampling_loc, im2col_step, clear=False):
     """``ms_depth_score_sample_backward`` with one more choice: ``clear=True`` takes a ``grad_value`` that holds anything
     (``torch.empty``); it then holds the gradient on return."""
-    _contig(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
-            sampling_loc=sampling_locations, grad_output=grad_output, grad_value=grad_value,
-            grad_sampling_loc=grad_sampling_loc)
-    dev = _on_gpu(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
-                  sampling_loc=sampling_locations, grad_output=grad_output, grad_value=grad_value,
-                  grad_sampling_loc=grad_sampling_loc)
+    dev = _contig_on_gpu(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
+                         sampling_loc=sampling_locations, grad_output=grad_output, grad_value=grad_value,
+                         grad_sampling_loc=grad_sampling_loc)
     B, S, M, D = value.shape
     L = _geometry(value_spatial_shapes, value_level_start_index, sampling_locations, 3, "ms_depth_score_sample_backward")
     _, Q, _, _, P, _ = sampling_locations.shape
@@ -172,10 +182,8 @@ def _wms_dims(value, shapes, lsi, loc, attn, score, name):
 def wms_deform_attn_forward(value, value_spatial_shapes, value_level_start_index, sampling_locations,
                             attention_weights, depth_scores, im2col_step):
     """Depth-weighted multi-scale deformable attention -> (bs, num_queries, heads*channels)."""
-    _contig(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
-            sampling_loc=sampling_locations, attn_weight=attention_weights, depth_score=depth_scores)
-    dev = _on_gpu(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
-                  sampling_loc=sampling_locations, attn_weight=attention_weights, depth_score=depth_scores)
+    dev = _contig_on_gpu(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
+                         sampling_loc=sampling_locations, attn_weight=attention_weights, depth_score=depth_scores)
     B, S, M, C, L, Q, P, sw, lw = _wms_dims(value, value_spatial_shapes, value_level_start_index, sampling_locations,
                                             attention_weights, depth_scores, "wms_deform_attn_forward")
     _step(B, im2col_step)
@@ -207,14 +215,10 @@ def wms_deform_attn_backward_into(value, value_spatial_shapes, value_level_start
                                   grad_attn_weight, grad_depth_score, im2col_step, clear=False):
     """``wms_deform_attn_backward`` with one more choice: ``clear=True`` takes a ``grad_value`` that holds anything
     (``torch.empty``) and clears what the kernels add to rather than store (see ``dfa3d_fused_backward``)."""
-    _contig(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
-            sampling_loc=sampling_locations, attn_weight=attention_weights, depth_score=depth_scores,
-            grad_output=grad_output, grad_value=grad_value, grad_sampling_loc=grad_sampling_loc,
-            grad_attn_weight=grad_attn_weight, grad_depth_score=grad_depth_score)
-    dev = _on_gpu(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
-                  sampling_loc=sampling_locations, attn_weight=attention_weights, depth_score=depth_scores,
-                  grad_output=grad_output, grad_value=grad_value, grad_sampling_loc=grad_sampling_loc,
-                  grad_attn_weight=grad_attn_weight, grad_depth_score=grad_depth_score)
+    dev = _contig_on_gpu(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
+                         sampling_loc=sampling_locations, attn_weight=attention_weights, depth_score=depth_scores,
+                         grad_output=grad_output, grad_value=grad_value, grad_sampling_loc=grad_sampling_loc,
+                         grad_attn_weight=grad_attn_weight, grad_depth_score=grad_depth_score)
     B, S, M, C, L, Q, P, sw, lw = _wms_dims(value, value_spatial_shapes, value_level_start_index, sampling_locations,
                                             attention_weights, depth_scores, "wms_deform_attn_backward")
     aux = _aux_dtype(value.dtype)
@@ -255,8 +259,7 @@ def ms_deform_attn_forward(value, value_spatial_shapes, value_level_start_index,
     Runs the stage-2 kernel without a score tensor."""
     named = dict(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
                  sampling_loc=sampling_locations, attn_weight=attention_weights)
-    _contig(**named)
-    dev = _on_gpu(**named)
+    dev = _contig_on_gpu(**named)
     B, S, M, C, L, Q, P, sw, lw = _wms_dims(value, value_spatial_shapes, value_level_start_index, sampling_locations,
                                             attention_weights, None, "ms_deform_attn_forward")
     _step(B, im2col_step)
@@ -281,8 +284,7 @@ def ms_deform_attn_backward(value, value_spatial_shapes, value_level_start_index
     named = dict(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
                  sampling_loc=sampling_locations, attn_weight=attention_weights, grad_output=grad_output,
                  grad_value=grad_value, grad_sampling_loc=grad_sampling_loc, grad_attn_weight=grad_attn_weight)
-    _contig(**named)
-    dev = _on_gpu(**named)
+    dev = _contig_on_gpu(**named)
     B, S, M, C, L, Q, P, sw, lw = _wms_dims(value, value_spatial_shapes, value_level_start_index, sampling_locations,
                                             attention_weights, None, "ms_deform_attn_backward")
     aux = _aux_dtype(value.dtype)
@@ -311,6 +313,15 @@ def ms_deform_attn_backward(value, value_spatial_shapes, value_level_start_index
 
 
 def _fused_dims(value, dist, shapes3, lsi, loc3, attn, name):
+    vs, ds, ls, dtype = value.shape, dist.shape, loc3.shape, value.dtype
+    if len(vs) == 4 and len(ds) == 4 and len(ls) == 6:           # all is well, as a rule: what follows says what is not
+        B, S, M, C = vs
+        _, Q, _, L, P, _ = ls
+        D, aux = ds[3], _aux_dtype(dtype)
+        if ls == (B, Q, M, L, P, 3) and attn.shape == (B, Q, M, L, P) and (ds == (B, S, M, D) or ds == (B, S, 1, D)) and \
+                shapes3.shape == (L, 3) and lsi.shape == (L,) and dist.dtype == dtype and loc3.dtype == aux and \
+                attn.dtype == aux and shapes3.dtype == torch.int64 and lsi.dtype == torch.int64:
+            return B, S, M, C, D, L, Q, P
     if value.dim() != 4 or dist.dim() != 4 or value.shape[:2] != dist.shape[:2] or \
             dist.shape[2] not in (1, value.shape[2]):
         raise RuntimeError(f"{name}: value (bs, keys, heads, C) and value_dpt_dist (bs, keys, heads or 1, D) must "
@@ -331,10 +342,8 @@ def pack_shared_dist(value_dpt_dist, value_spatial_shapes, value_level_start_ind
     around every base pixel side by side, per bin): pass the result as ``packed_dist`` to ``dfa3d_fused_forward``.
     Returns None where the library does not offer it (D < 2, float64).  Worth keeping: every forward on the same
     distribution (DFA3D-BEVFormer runs six encoder layers on one) can use the same packed tensor."""
-    _contig(value_dpt_dist=value_dpt_dist, spatial_shapes=value_spatial_shapes,
-            level_start_index=value_level_start_index)
-    dev = _on_gpu(value_dpt_dist=value_dpt_dist, spatial_shapes=value_spatial_shapes,
-                  level_start_index=value_level_start_index)
+    dev = _contig_on_gpu(value_dpt_dist=value_dpt_dist, spatial_shapes=value_spatial_shapes,
+                         level_start_index=value_level_start_index)
     if value_dpt_dist.dim() != 4 or value_dpt_dist.shape[2] != 1:
         raise RuntimeError(f"value_dpt_dist must be (bs, keys, 1, D), got {tuple(value_dpt_dist.shape)}")
     if value_dpt_dist.dtype == torch.float64:
@@ -361,11 +370,9 @@ def dfa3d_fused_forward(value, value_dpt_dist, value_spatial_shapes, value_level
     with ``need_weight_update`` a third result, weight_update (bs, Q, heads, 1) = sum over levels and points of
     attention weight * mean corner score.  ``value_dpt_dist`` is (bs, keys, heads, D), or (bs, keys, 1, D) for one
     distribution shared by all heads; for the latter ``packed_dist`` may be what ``pack_shared_dist`` returned for it."""
-    _contig(value=value, value_dpt_dist=value_dpt_dist, spatial_shapes=value_spatial_shapes,
-            level_start_index=value_level_start_index, sampling_loc=sampling_locations, attn_weight=attention_weights)
-    dev = _on_gpu(value=value, value_dpt_dist=value_dpt_dist, spatial_shapes=value_spatial_shapes,
-                  level_start_index=value_level_start_index, sampling_loc=sampling_locations,
-                  attn_weight=attention_weights)
+    dev = _contig_on_gpu(value=value, value_dpt_dist=value_dpt_dist, spatial_shapes=value_spatial_shapes,
+                         level_start_index=value_level_start_index, sampling_loc=sampling_locations,
+                         attn_weight=attention_weights)
     B, S, M, C, D, L, Q, P = _fused_dims(value, value_dpt_dist, value_spatial_shapes, value_level_start_index,
                                          sampling_locations, attention_weights, "dfa3d_fused_forward")
     _step(B, im2col_step)
@@ -383,9 +390,9 @@ def dfa3d_fused_forward(value, value_dpt_dist, value_spatial_shapes, value_level
         return (out, score, wu) if need_weight_update else (out, score)
     with _lib.on_device(dev):
         rc = _lib.lib().dfa3d_fused_forward(
-            _lib.ptr(value), _lib.ptr(value_dpt_dist), _lib.ptr(value_spatial_shapes),
-            _lib.ptr(value_level_start_index), _lib.ptr(sampling_locations), _lib.ptr(attention_weights),
-            _lib.ptr(out), _lib.ptr(score), _lib.ptr(wu), _lib.ptr(packed_dist), B, S, M, C, D, L, Q, P,
+            value.data_ptr(), value_dpt_dist.data_ptr(), value_spatial_shapes.data_ptr(),
+            value_level_start_index.data_ptr(), sampling_locations.data_ptr(), attention_weights.data_ptr(),
+            out.data_ptr(), _lib.ptr(score), _lib.ptr(wu), _lib.ptr(packed_dist), B, S, M, C, D, L, Q, P,
             value_dpt_dist.shape[2],
             _lib.dtype_code(value), _lib.options(), _lib.stream_of(value))
     _lib.check(rc, "dfa3d_fused_forward")
@@ -424,8 +431,7 @@ def dfa3d_fused_backward(value, value_dpt_dist, value_spatial_shapes, value_leve
         named["grad_depth_score"] = grad_depth_score
     if grad_weight_update is not None:
         named["grad_weight_update"] = grad_weight_update
-    _contig(**named)
-    dev = _on_gpu(**named)
+    dev = _contig_on_gpu(**named)
     B, S, M, C, D, L, Q, P = _fused_dims(value, value_dpt_dist, value_spatial_shapes, value_level_start_index,
                                          sampling_locations, attention_weights, "dfa3d_fused_backward")
     aux = _aux_dtype(value.dtype)

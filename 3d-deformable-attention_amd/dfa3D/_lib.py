@@ -176,4 +176,4 @@ _HERE_ALREADY = contextlib.nullcontext()
 
 def on_device(dev):
     """Context in which ``dev`` is the current GPU; nothing to enter or leave when it is that already."""
-    return _HERE_ALREADY if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+    return _HERE_ALREADY if torch._C._cuda_getDevice() == dev.index else torch.cuda.device(dev)
