@@ -574,8 +574,8 @@ __device__ __forceinline__ void clear_unstored(const BinWorkspace &ws, const Cle
 }
 
 // The first `scan_blocks` blocks scan, 1024 bins each (in turns if there are more bins than that).  A block needs no
-// word from the blocks before it: it adds up the counts of all bins before its own (a few dozen loads per thread for
-// tens of thousands of bins), which is cheaper than one workgroup walking all bins and writing every work item from
+// word from the blocks before it: it adds up the counts of all bins before its own (16 bytes a load, a few loads per
+// thread for tens of thousands of bins), which is cheaper than one workgroup walking all bins and writing every work item from
 // one CU.  Further blocks, if any, clear the gradient rows that need it meanwhile (both kinds only read the counts);
 // the kernel is held to 64 registers so that two such workgroups fit a CU.
 // An item's last word says whether it alone writes the pixels inside its tile, which the tile kernels then store: it holds
@@ -1170,13 +1170,14 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
 // What bounds it is the random access of each point (its score gradient, its z gradient, four pairs of bins) and the
 // tile's way out, so the kernel keeps both going at once: no barrier between the points of an item (taps go to LDS by
 // compare-and-swap, so nobody waits for anybody), the next round's records asked for one round ahead and the next item's
-// before the tile is flushed.  The bins come from the caches as long as few tiles are worked on at a time: 16 wavefronts per CU
-// either way, one workgroup of 1024 threads beats four of 256 where tiles have the points for it (BLOCK: tile_config_of).  For a caller whose buffer may hold anything, a pixel that
-// only this item can touch (no neighbour's halo, all the points of its bin, levels that share no keys) is stored 16
-// bytes per lane; everything else is added atomically, one float per lane on consecutive addresses.
-// 6 x 9502 queries, 4 levels from 116 x 200, 8 points, 112 bins (14.6 M points): 1.19 ms with a ticket per tap and
-// three barriers per 256 points, 1.01 ms without them and 0.85 ms with 1024 threads per tile; with parts cut out of the 1.01, the z gradients' scattered stores are 0.27 of it, the
-// tiles' way out 0.2, the taps 0.10, the score gradients' gathers 0.09.
+// before the tile is flushed.  The bins come from the caches as long as few tiles are worked on at a time: with 16
+// wavefronts per CU either way, one workgroup of 1024 threads beats four of 256 where tiles have the points for it (BLOCK:
+// tile_config_of).  For a caller whose buffer may hold anything, a pixel that only this item can touch (no neighbour's halo, all
+// the points of its bin, levels that share no keys) is stored 16 bytes per lane; everything else is added atomically, one
+// float per lane on consecutive addresses.
+// 6 x 9502 queries, 4 levels from 116 x 200, 8 points, 112 bins (14.6 M points): 1.19 ms with a ticket per tap and three
+// barriers per 256 points, 1.01 ms without them, 0.85 ms with 1024 threads per tile.  With parts cut out of the 1.01 ms form, the z
+// gradients' scattered stores were 0.27 of it, the tiles' way out 0.2, the taps 0.10, the score gradients' gathers 0.09.
 // ---------------------------------------------------------------------------------------
 // The fetching thread's state: the queue is asked for an item's number when another item is begun, the answer is looked
 // at when that one's points are done, and the records asked for then are handed over with the next item.

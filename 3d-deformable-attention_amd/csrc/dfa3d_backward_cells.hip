@@ -7,7 +7,8 @@
 //     accumulators of weight * grad_out live in its registers, every point's grad_out row is read from LDS once, the
 //     four dot products and the four weighted sums are formed from it, and nothing is added to an LDS tile during the
 //     passes.  The weighted sums are outer products (4 corners x channels, one point deep) of 4-lane blocks: one
-//     v_mfma_f32_4x4x1 per channel of a lane does what four FMAs per lane would, on the matrix pipe;
+//     v_mfma_f32_4x4x1 per channel of a lane does what four FMAs per lane would, on the matrix pipe; with 2-byte
+//     elements the dot products are matrix instructions too, four points at a time (walk_fours);
 //   * a pass sorts its points (256, or 128 with long rows) by cell: one integer LDS atomic per point.
 // (Base pixels run from -1, for a location within half a pixel of the map's upper or left edge, to H - 1 / W - 1;
 // the tiles are laid over that range, so a cell's upper or left pixels may lie outside the map like its lower or
@@ -15,9 +16,8 @@
 //
 // The 8 wavefronts of a workgroup have two roles.  "Walkers" (wavefronts 0-3, one or two tile rows of 8 cells each)
 // walk the cells' lists; "pointers" (wavefronts 4-7, one point of the pass per thread) do everything that is per point:
-// geometry, depth taps, corner weights, the sort, and afterwards the point's gradients
-// and its grad_dist taps into the LDS depth tile.  The roles meet at two barriers per turn and
-// otherwise overlap.  Turns follow one another without a gap, whatever item their passes belong to (pass t: one of
+// geometry, depth taps, corner weights, the sort, and afterwards the point's gradients and its grad_dist taps into the
+// LDS depth tile.  The roles meet at two barriers per turn and otherwise overlap.  Turns follow one another without a gap, whatever item their passes belong to (pass t: one of
 // the item's passes), so that an item of a single pass costs a single turn:
 //   phase X(t):  walkers: walk(t-1)        pointers: scores and corner weights of t, prepare(t+1)
 //   phase Y(t):  walkers: stage(t)         pointers: place(t) (scan + sorted slots), finish(t-1)
@@ -337,8 +337,8 @@ template <typename T> struct TapsInFlight {
 };
 
 // 16 bytes per lane from a buffer to consecutive LDS addresses (`lds`: the wavefront's first byte).  Written out because
-// behind the builtin the compiler waits for the data before the next LDS read of any kind; here
-// wait_for_loads() does, when the phase ends.  (The compiler does not count these loads: where it waits for an older
+// behind the builtin the compiler waits for the data before the next LDS read of any kind; here wait_for_loads() does,
+// when the phase ends.  (The compiler does not count these loads: where it waits for an older
 // one, it waits for more than it has to, never for less.)
 __device__ __forceinline__ void load_to_lds16(rsrc_t r, const void *lds, uint32_t off) {
 #ifdef __HIP_DEVICE_COMPILE__

@@ -538,12 +538,12 @@ PHASE_CLOCKS_ROWS = ("item fetch", "barrier after phases A and C", "rank + stagi
 PHASE_CLOCKS_CELLS = ("walker: set-up, the next item's record", "walker: walk (phase X)", "walker: wait at the barrier after X",
                       "walker: item record fetched, the old item's sums put together (phase Y)",
                       "walker: wait at the barrier after Y",
-                      "walker: the old item's sums and rim go out, value rows awaited (phase X)",
-                      "walker: value rows asked for, short grad_out rows staged (phase Y)", "-",
+                      "walker: the old item's sums and rim go out (phase X)",
+                      "walker: grad_out rows and value rows asked for and awaited (phase Y)", "-",
                       "pointer: set-up, turn's bookkeeping", "pointer: scores, corner weights, next pass prepared (phase X)",
                       "pointer: depth tile goes out (phase X)", "pointer: wait at the barrier after X",
-                      "pointer: grad_out rows asked for, points placed (phase Y)",
-                      "pointer: gradients and grad_dist taps, grad_out rows awaited (phase Y)",
+                      "pointer: points placed (phase Y)",
+                      "pointer: gradients and grad_dist taps (phase Y)",
                       "pointer: wait at the barrier after Y", "-")
 
 
@@ -816,7 +816,7 @@ def run(a, torch, _ext, _lib, L_, F1, WORKLOADS, make_inputs, user_options):
         bin_ms, tile_ms = sum(bin_t) / len(bin_t), sum(tile_t) / len(tile_t)
         kernels["backward_tile"] = entry("tile kernel of the binned backward (all gradients, one launch)", tile_ms, min(tile_t), bwd_bytes,
                                          "backward_tile")
-        kernels["backward_binning"] = {"kernel": "plan_and_clear + bin_count + bin_scan (whose further blocks clear gradient rows) + bin_fill_sorted (+ their plain forms, which step aside)",
+        kernels["backward_binning"] = {"kernel": "plan_and_clear + bin_count + bin_scan (whose further blocks clear gradient rows) + bin_fill_sorted",
                                        "avg_ms": round(bin_ms, 4), "min_ms": round(min(bin_t), 4)}
         dom = "backward_tile" if tile_ms >= fwd_ms else "forward"
     else:
