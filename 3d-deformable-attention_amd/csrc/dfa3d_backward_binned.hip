@@ -1178,7 +1178,10 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
 // 6 x 9502 queries, 4 levels from 116 x 200, 8 points, 112 bins (14.6 M points): 1.19 ms with a ticket per tap and three
 // barriers per 256 points, 1.01 ms without them, 0.85 ms with 1024 threads per tile.  With parts cut out of the 1.01 ms form, the z
 // gradients' scattered stores were 0.27 of it, the tiles' way out 0.2, the taps 0.10, the score gradients' gathers 0.09.
+// The stored pixels leave the L2 first (non-temporal: nobody reads them again, and the z gradients' lines need the room to fill
+// up): the call 1061 -> 1039 us, 1030 with the z gradients stored behind the taps; 2 x 1000 queries on the same maps 144 -> 128.
 // ---------------------------------------------------------------------------------------
+constexpr int kNonTemporal = 2;       // cache policy of a buffer store on gfx950: the NT bit
 // The fetching thread's state: the queue is asked for an item's number when another item is begun, the answer is looked
 // at when that one's points are done, and the records asked for then are handed over with the next item.
 struct DepthFetch {
@@ -1284,9 +1287,9 @@ __global__ __launch_bounds__(BLOCK, 4) void tile_depth_backward_kernel(
           tv[2 * k + 1] = on && tap.hi_ok ? tap.ld * g4[k] : 0.f;
           gz += on ? g4[k] * (hi[k] - lo[k]) : 0.f;
         }
+        lds_add_taps(gd, at, tv);
         float *gl = grad_loc3 + (size_t)gp * 3;
         gl[0] = 0; gl[1] = 0; gl[2] = gz * (float)Dd;
-        lds_add_taps(gd, at, tv);
       }
     }
     if (tid == 0) fetch.answer(ws, p, home);
@@ -1307,7 +1310,7 @@ __global__ __launch_bounds__(BLOCK, 4) void tile_depth_backward_kernel(
           const float4 v = *from;
           *from = make_float4(0, 0, 0, 0);
           const u32x4 o = {__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
-          __builtin_amdgcn_raw_buffer_store_b128(o, gdist_r, y < H && x < W ? e0 + 16 * c : kNoRow, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b128(o, gdist_r, y < H && x < W ? e0 + 16 * c : kNoRow, 0, kNonTemporal);
         }
       }
     }
