@@ -255,7 +255,8 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
 // with 112 bins) pushed one another out.  And a lane takes four points at a time, sixteen gathers in flight, where a block has
 // them; it has where the launch would be more than 4096 blocks of 1024 points.  6 x 9502 queries, four levels from
 // 116 x 200, 8 points (14.6 M points), 112 bins 536 -> 496 us level by level, 470 with four points at a time; 64 bins 514 / 440 /
-// 403, 16 bins 439 / 372 / 331, bfloat16 446 / 432 / 402.  Below four points per level a level's locations and scores
+// 403, 16 bins 439 / 372 / 331, bfloat16 446 / 432 / 402.  As it stands, with
+// non-temporal stores of the scores: 468, 407, 272 and bfloat16 404.  Below four points per level a level's locations and scores
 // are less than half a line each: all levels together (2 points: 53 against 55 us for 1.3 M points).
 // ---------------------------------------------------------------------------------------
 struct DepthScoreShape { int levels, points; };          // levels per group, points per block at most
@@ -303,8 +304,17 @@ __global__ __launch_bounds__(kBlock) void depth_score_kernel(
 #pragma unroll
     for (int r = 0; r < N; ++r) {
       T *so = score + gp[r] * 4;
+      // non-temporal: the scores leave the L2 to the distributions
+      if constexpr (std::is_same<T, float>::value) {
+        typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+        __builtin_nontemporal_store((f4){sc[r][0], sc[r][1], sc[r][2], sc[r][3]}, reinterpret_cast<f4 *>(so));
+      } else if constexpr (std::is_same<T, __hip_bfloat16>::value) {
+        typedef uint32_t u2 __attribute__((ext_vector_type(2), aligned(2)));
+        __builtin_nontemporal_store((u2){pack_bf16x2(sc[r][0], sc[r][1]), pack_bf16x2(sc[r][2], sc[r][3])}, reinterpret_cast<u2 *>(so));
+      } else {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) Elem<T>::st(so + k, sc[r][k]);
+        for (int k = 0; k < 4; ++k) Elem<T>::st(so + k, sc[r][k]);
+      }
     }
   };
   int i = threadIdx.x;
