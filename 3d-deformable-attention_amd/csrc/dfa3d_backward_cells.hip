@@ -162,7 +162,7 @@ __device__ __forceinline__ float quad_corner_sum(float d0, float d1, float d2, f
 // Where the 16-byte piece `piece` of staged row `row` lies, in bytes.  Of 2-byte elements the pieces of a row lie in an order that
 // depends on the row, so that the same piece of eight neighbouring rows falls on different banks: a lane that takes a whole row
 // (WholeRow) reads them one after the other, as its neighbours do with theirs.
-template <typename T, int ROWB> __device__ __forceinline__ int piece_at(int row, int piece) {
+template <typename T, int ROWB> __device__ __forceinline__ constexpr int piece_at(int row, int piece) {
   if constexpr (sizeof(T) == 2) {
     constexpr int N = ROWB / 16, SH = ROWB >= 128 ? 0 : ROWB == 64 ? 1 : 2;
     piece ^= (row >> SH) & (N - 1);
@@ -420,7 +420,9 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 
   for (int i = tid; i < lay.gstage; i += BLOCK) smem[i] = 0;                   // depth tile
   for (int i = tid; i < 3 * CELLS; i += BLOCK) cnt[i] = 0;
-  for (int i = tid; i < ROW * (int)sizeof(T) / 4; i += BLOCK) smem[lay.gstage + PP * ROW * (int)sizeof(T) / 4 + i] = 0;   // what a group without a point reads
+  // What a group without a point reads; and rows shorter than their lane group once whole, as nothing need be written beyond their
+  // channels.
+  for (int i = tid + (a0->C == ROW ? PP * ROW * (int)sizeof(T) / 4 : 0); i < (PP + 1) * ROW * (int)sizeof(T) / 4; i += BLOCK) smem[lay.gstage + i] = 0;
   if (tid < 4) dots[PP * 4 + tid] = 0;
   if (tid == 0) s_slot[PP] = (uint16_t)PP;
   if (tid < DFA3D_MAX_LEVELS) {      // decoding an item then costs no dependent loads from device memory
@@ -626,37 +628,48 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       asm volatile("" : "+v"(i));
       if (i < (unsigned)CELLS) cnt[(turn + 2) % 3 * CELLS + i] = 0;
     };
-    // phase Y: the grad_out rows of the pass come to LDS; they must be there before the phase ends (wait_for_loads()).  Whole rows
-    // go straight there, 16 bytes per lane, without a register in between.  (The pointers, whose work in phase Y is the
-    // longer one, brought them before: tile kernel 1158 -> 1121 us at the base shape, bfloat16 1045 -> 1022, dense 4245 -> 4160,
-    // small 111 -> 106.)
-    auto stage = [&](int n) {
+    // phase Y: the grad_out rows of the pass come to LDS; they must be there before the phase ends (wait_for_loads()).  (The
+    // pointers, whose work in phase Y is the longer one, brought them before: tile kernel 1158 -> 1121 us at the base shape,
+    // bfloat16 1045 -> 1022, dense 4245 -> 4160, small 111 -> 106.)
+    // Rows of whole 16-byte pieces go straight there, a piece per lane, without a register in between.  Where a row is shorter than
+    // its lane group, a lane beyond its channels asks beyond the buffer.  (Brought by registers, whose wait came before the value rows
+    // were asked for, rows of 40 channels took 737 us in bfloat16, 714 in float, and straight 706 and 685: tile kernel, 4 x 4000 queries,
+    // four levels from 116 x 200, 32 points a query; on a sparse map, 400 x 400 with 8000 queries of 4 points, 554 -> 514 and 514 -> 471,
+    // 20 channels in float 277 -> 258.)
+    const bool straight = sizeof(T) == 4 || (arg()->C & 7) == 0;         // uniform
+    auto stage_straight = [&](int n) {
       const auto a = arg();
       const int Q = a->Q, M = a->M, C = a->C;
       const T *grad_out = a->grad_out;
-      if (C == ROW) {                                        // uniform
-        // Instructions take turns over the wavefronts and stop where the pass's points do: an item of a few dozen points
-        // asks for its rows in one or two of each (6 x 2000 queries, four levels from 116 x 200, 32 points a query: tile kernel
-        // 535 -> 526 us).
-        constexpr int RL = ROW * (int)sizeof(T) / 16, RPI = kWave / RL, N = kRows / RPI, NB = N < 2 ? N : 2;      // lanes per row, rows per instruction
-        const rsrc_t go_r = make_rsrc(grad_out + (size_t)g.b * Q * M * C, (size_t)Q * M * C * sizeof(T));
-        unsigned l = lane;
-        asm volatile("" : "+v"(l));                          // (not worth registers from turn to turn)
-        const int r0 = wave * RPI, at = r0 + (int)(l / RL);
+      // Instructions take turns over the wavefronts and stop where the pass's points do: an item of a few dozen points
+      // asks for its rows in one or two of each (6 x 2000 queries, four levels from 116 x 200, 32 points a query: tile kernel
+      // 535 -> 526 us).
+      constexpr int RL = ROW * (int)sizeof(T) / 16, RPI = kWave / RL, N = kRows / RPI, NB = N < 2 ? N : 2;      // lanes per row, rows per instruction
+      const rsrc_t go_r = make_rsrc(grad_out + (size_t)g.b * Q * M * C, (size_t)Q * M * C * sizeof(T));
+      unsigned l = lane;
+      asm volatile("" : "+v"(l));                            // (not worth registers from turn to turn)
+      const int r0 = wave * RPI, at = r0 + (int)(l / RL);
+      // this lane's piece, the same in every instruction: the order of a row's pieces repeats within the rows of one
+      static_assert(piece_at<T, RL * 16>(4 * RPI, 0) % (RL * 16) == 0, "");
+      const uint32_t piece = piece_at<T, RL * 16>(at, l % RL) % (RL * 16), from = piece < (uint32_t)C * (uint32_t)sizeof(T) ? piece : kNoChan;
 #pragma unroll
-        for (int j0 = 0; j0 < N; j0 += NB) {
-          if (j0 > 0 && r0 + j0 * 4 * RPI >= n) break;       // uniform
-          uint32_t row[NB];
+      for (int j0 = 0; j0 < N; j0 += NB) {
+        if (j0 > 0 && r0 + j0 * 4 * RPI >= n) break;         // uniform
+        uint32_t row[NB];
 #pragma unroll
-          for (int j = 0; j < NB; ++j) row[j] = goff[(turn & 1) * PP + (j0 + j) * 4 * RPI + at];
+        for (int j = 0; j < NB; ++j) row[j] = goff[(turn & 1) * PP + (j0 + j) * 4 * RPI + at];
 #pragma unroll
-          for (int j = 0; j < NB; ++j)
-            load_to_lds16(go_r, gstage + (r0 + (j0 + j) * 4 * RPI) * RL * 16, row[j] + piece_at<T, RL * 16>((j0 + j) * 4 * RPI + at, l % RL) % (RL * 16));
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        return;
+        for (int j = 0; j < NB; ++j) load_to_lds16(go_r, gstage + (r0 + (j0 + j) * 4 * RPI) * RL * 16, row[j] + from);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      const Owner o = owner(arg());
+    };
+    // Rows that end within a piece (2-byte elements, an odd number of groups of four).  The loads end in registers that are put
+    // into LDS: what else the phase asks for comes first, so that there is one wait (44 channels: 749 -> 729 us, sparse 567 -> 536).
+    auto stage_by_registers = [&]() {
+      const auto a = arg();
+      const int Q = a->Q, M = a->M, C = a->C;
+      const T *grad_out = a->grad_out;
+      const Owner o = owner(a);
       const rsrc_t go_r = make_rsrc(grad_out + (size_t)g.b * Q * M * C, (size_t)Q * M * C * sizeof(T));
       const uint32_t *offs_of = goff + (turn & 1) * PP + wave * kRows;
 #pragma unroll
@@ -814,7 +827,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           if (ROWS == 2) put_pixel(now, o, uniform(s_geom[slot_of_item(it - 1)]), u, o.crow < TY && o.group >= TX);   // the second row is complete
         }
         CT_MARK(3);
-        if (!done) stage(g.n_item);
+        if (!done && straight) stage_straight(g.n_item);
         typename LaneChannels<T, VEC, LPR>::Raw vr[4];
         {
           // the four value rows of this group's cell (zero outside the map, when the cell is not part of the tile, or when
@@ -830,6 +843,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
             o.ch.load(value_r, ok ? (uint32_t)(((g.start + y * g.W + x) * M + g.m) * C * (int)sizeof(T)) : kNoRow, vr[k]);
           }
         }
+        if (!done && !straight) stage_by_registers();
         wait_for_loads();
         CT_MARK(6);
         lds_barrier();
@@ -878,7 +892,8 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         lds_barrier();
         CT_MARK(2);
         for (int base = PP; base < g.n_item; base += PP) {   // the item's further passes
-          stage(g.n_item - base);
+          if (straight) stage_straight(g.n_item - base);
+          else stage_by_registers();
           wait_for_loads();
           CT_MARK(6);
           lds_barrier();
