@@ -1651,7 +1651,7 @@ static hipError_t launch_tile_typed(const BwdArgs &a, const BinWorkspace &ws, co
                                     hipStream_t stream) {
   if (c.cells) {
     const int dtype = sizeof(T) == 4 ? DFA3D_F32 : DFA3D_BF16;
-    if (hipError_t e = allow_lds(cell_kernel_symbol(dtype, a.C, a.dist != nullptr), c.lds)) return e;
+    if (hipError_t e = allow_lds(cell_kernel_symbol(a, dtype), c.lds)) return e;
     // two workgroups per CU at most (its registers): a workgroup that had to wait for a place would sit on dealt items
     return launch_cell_kernel(a, dtype, ws, c.lds, tile_grid(c.lds < 80 * 1024 ? 80 * 1024 : c.lds, c.block), gd_heads, stream);
   }

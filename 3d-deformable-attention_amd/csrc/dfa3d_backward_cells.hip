@@ -8,7 +8,7 @@
 //     four dot products and the four weighted sums are formed from it, and nothing is added to an LDS tile during the
 //     passes.  The weighted sums are outer products (4 corners x channels, one point deep) of 4-lane blocks: one
 //     v_mfma_f32_4x4x1 per channel of a lane does what four FMAs per lane would, on the matrix pipe; with 2-byte
-//     elements the dot products are matrix instructions too, four points at a time (walk_fours);
+//     elements, unless points are sparse, the dot products are matrix instructions too, four points at a time (walk_fours);
 //   * a pass sorts its points (256, or 128 with long rows) by cell: one integer LDS atomic per point.
 // (Base pixels run from -1, for a location within half a pixel of the map's upper or left edge, to H - 1 / W - 1;
 // the tiles are laid over that range, so a cell's upper or left pixels may lie outside the map like its lower or
@@ -386,7 +386,9 @@ template <typename T, bool FRESH> __device__ CellArgsPtr<T> args();
 // FUSED: both stages (depth scores recomputed from dist, grad_dist and the z gradient produced).
 // !FUSED: stage 2 alone: scores read from score_in, their gradient written to grad_score_out, no depth tile
 // (the launcher passes D = 0), grad_loc has gl_stride components of which x, y are written.
-template <typename T, int VEC, int LPR, bool FUSED>
+// FOURS: the walkers take the points of a cell four at a time (see walks_fours() below).  Both walks in one kernel, chosen pass by
+// pass, do not fit its registers: base shape, bfloat16, 32 channels 580 -> 742 us for half of its cameras, 64 channels 830 -> 1706.
+template <typename T, int VEC, int LPR, bool FUSED, bool FOURS>
 __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_kernel(CellArgs<T>) {
   constexpr int PP = cell_pass(LPR), BLOCK = kWalkers + PP, TX = kCellTX, TW = TX + 1, ROW = VEC * LPR;
   constexpr int GPW = kWave / LPR, CELLS = 4 * GPW, ROWS = GPW / TX;      // cells and tile rows per walker wavefront
@@ -686,9 +688,9 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     // 2-byte elements: four points per step and group.  Each lane of four takes the row of one of them for the dots, which are
     // products of matrices then (v_mfma_f32_4x4x4, four channels deep), and all four take all of them for the sums.
     // The step takes a third of the vector instructions that four steps of one point do, for two and a half times the reads
-    // from LDS: base shape 1061 -> 1040 us.  With 4-byte elements, where a matrix instruction is one channel deep and a row twice
+    // from LDS, and does the work of four also where a cell has one point (walks_fours()): base shape 1061 -> 1040 us.  With 4-byte elements, where a matrix instruction is one channel deep and a row twice
     // as long, it lost: plain attention 209 -> 227 us, base shape 1194 -> 1277.
-    auto walk_fours = [&](const WholeRow<T, VEC, LPR> &v, f4 (&acc)[VEC]) {
+    auto walk_fours = [&](const auto &v, f4 (&acc)[VEC]) {
       const Owner o = owner(arg());
       const int corner = o.cl & 3, cell = o.crow * TX + o.ccol;
       const bool cell_ok = o.crow < TY;
@@ -733,9 +735,9 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       }
     };
 
-    // 4-byte elements: one point per step and group; the next step's row and weights and the slot after that are asked for while
+    // One point per step and group; the next step's row and weights and the slot after that are asked for while
     // this step's sums are formed, so that no LDS round trip is waited for with nothing to do.
-    auto walk_ones = [&](const float (&v)[4][VEC], f4 (&acc)[VEC]) {
+    auto walk_ones = [&](const auto &v, f4 (&acc)[VEC]) {
       const Owner o = owner(arg());
       const int corner = o.cl & 3, cell = o.crow * TX + o.ccol;
       const bool cell_ok = o.crow < TY;
@@ -768,8 +770,8 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     };
 
     auto walk = [&](const auto &v, f4 (&acc)[VEC]) {
-      if constexpr (sizeof(T) == 4) walk_ones(v, acc);
-      else walk_fours(v, acc);
+      if constexpr (FOURS) walk_fours(v, acc);
+      else walk_ones(v, acc);
     };
 
     if (g.bin >= 0) {
@@ -877,12 +879,12 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           if (r0 + ROWS >= TY) put_rim(now, q, TW, TW);
         }
         if (done) break;
-        typename std::conditional<sizeof(T) == 4, float[4][VEC], WholeRow<T, VEC, LPR>>::type v;      // the four value rows
-        if constexpr (sizeof(T) == 4) {
+        typename std::conditional<FOURS, WholeRow<T, VEC, LPR>, float[4][VEC]>::type v;      // the four value rows
+        if constexpr (FOURS) {
+          whole_rows<T, VEC, LPR>(vr, owner(now).cl, v);
+        } else {
 #pragma unroll
           for (int k = 0; k < 4; ++k) LaneChannels<T, VEC, LPR>::to_float(vr[k], v[k]);
-        } else {
-          whole_rows<T, VEC, LPR>(vr, owner(now).cl, v);
         }
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = (f4){0, 0, 0, 0};
@@ -1161,7 +1163,19 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 // its walkers own.  The row-owned tile kernel keeps the rest.
 bool cell_kernel_applies(int C, int ty, int tx) { return C <= 64 && (C & 3) == 0 && tx == kCellTX && ty >= 1 && ty <= cell_max_ty(C); }
 
-template <typename T, int VEC, int LPR>
+// Whether the walkers take the points of a cell four at a time.  Never with 4-byte elements (walk_fours).  With 2-byte elements a step of
+// four costs about as much as three of one and is wasted on shorter lists, so it is taken from three quarters of a point per
+// pixel on.  Tile kernel, one at a time against four, by points per pixel (uniform locations; the sign turns at 0.5 where they
+// are clustered, + 1.5 % at 0.75):
+//   32 channels, stage 2 on 400 x 400   0.15: 237, 256 us   0.5: 260, 271   0.75: 274, 281   1: 287, 289   1.5: 309, 310   3: 387, 383
+//   32 channels, 16 bins, 232 x 400     0.15: 160, 165      0.5: 168, 171   0.75: 172, 174   1: 179, 180   1.5: 198, 196   3: 257, 254
+//   64 channels, 16 bins, 232 x 400     0.15: 294, 306      0.5: 318, 331   0.75: 332, 339   1: 342, 348   1.5: 363, 363   3: 423, 421
+// Rows of up to 16 channels, whose steps are short, gain at most 1 % below a third of a point, and lose from a half on.
+static bool walks_fours(const BwdArgs &a, int dtype) {
+  return dtype == DFA3D_BF16 && (cell_shape(a.C).vec == 4 || 4LL * a.Q * a.L * a.P >= 3LL * a.S);
+}
+
+template <typename T, int VEC, int LPR, bool FOURS>
 static hipError_t launch_cell_cfg(const BwdArgs &a, const BinWorkspace &ws, size_t lds, int grid, float *gd_heads,
                                   hipStream_t stream) {
   const bool fused = a.dist != nullptr, one = a.dist_heads == 1;
@@ -1174,39 +1188,42 @@ static hipError_t launch_cell_cfg(const BwdArgs &a, const BinWorkspace &ws, size
                          !fused ? 0 : (a.grad_bf16 ? 1 : 0) | (a.grad_bf16 && gd_heads == nullptr ? 2 : 0)
                          DFA3D_DIAG_ARG(a)};
   const dim3 block(kWalkers + cell_pass(LPR));
-  if (fused) hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, true>), dim3(grid), block, lds, stream, c);
-  else hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, false>), dim3(grid), block, lds, stream, c);
+  if (fused) hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, true, FOURS>), dim3(grid), block, lds, stream, c);
+  else hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, false, FOURS>), dim3(grid), block, lds, stream, c);
   return hipGetLastError();
 }
 
-template <typename T, int VEC, int LPR> static const void *symbol_of(bool fused) {
-  return fused ? reinterpret_cast<const void *>(cell_backward_kernel<T, VEC, LPR, true>)
-               : reinterpret_cast<const void *>(cell_backward_kernel<T, VEC, LPR, false>);
+template <typename T, int VEC, int LPR, bool FOURS> static const void *symbol_of(bool fused) {
+  return fused ? reinterpret_cast<const void *>(cell_backward_kernel<T, VEC, LPR, true, FOURS>)
+               : reinterpret_cast<const void *>(cell_backward_kernel<T, VEC, LPR, false, FOURS>);
 }
 
-#define DFA3D_CELL_DISPATCH(dtype, C, CALL)                                  \
+#define DFA3D_CELL_DISPATCH(dtype, a, CALL)                                  \
   do {                                                                       \
-    const CellShape s = cell_shape(C);                                       \
+    const CellShape s = cell_shape((a).C);                                   \
+    const bool fours = walks_fours(a, dtype);                                \
     if (dtype == DFA3D_F32) {                                                \
-      if (s.lpr == 8) return CALL(float, 8, 8);                              \
-      if (s.vec == 8) return CALL(float, 8, 4);                              \
-      return CALL(float, 4, 4);                                              \
+      if (s.lpr == 8) return CALL(float, 8, 8, false);                       \
+      if (s.vec == 8) return CALL(float, 8, 4, false);                       \
+      return CALL(float, 4, 4, false);                                       \
     }                                                                        \
-    if (s.lpr == 8) return CALL(__hip_bfloat16, 8, 8);                       \
-    if (s.vec == 8) return CALL(__hip_bfloat16, 8, 4);                       \
-    return CALL(__hip_bfloat16, 4, 4);                                       \
+    if (s.lpr == 8 && fours) return CALL(__hip_bfloat16, 8, 8, true);        \
+    if (s.lpr == 8) return CALL(__hip_bfloat16, 8, 8, false);                \
+    if (s.vec == 8 && fours) return CALL(__hip_bfloat16, 8, 4, true);        \
+    if (s.vec == 8) return CALL(__hip_bfloat16, 8, 4, false);                \
+    return CALL(__hip_bfloat16, 4, 4, true);                                 \
   } while (0)
 
-const void *cell_kernel_symbol(int dtype, int C, bool fused) {
-#define DFA3D_CELL_SYMBOL(T, V, R) (symbol_of<T, V, R>(fused))
-  DFA3D_CELL_DISPATCH(dtype, C, DFA3D_CELL_SYMBOL);
+const void *cell_kernel_symbol(const BwdArgs &a, int dtype) {
+#define DFA3D_CELL_SYMBOL(T, V, R, F) (symbol_of<T, V, R, F>(a.dist != nullptr))
+  DFA3D_CELL_DISPATCH(dtype, a, DFA3D_CELL_SYMBOL);
 #undef DFA3D_CELL_SYMBOL
 }
 
 hipError_t launch_cell_kernel(const BwdArgs &a, int dtype, const BinWorkspace &ws, size_t lds, int grid, float *gd_heads,
                               hipStream_t stream) {
-#define DFA3D_CELL_LAUNCH(T, V, R) (launch_cell_cfg<T, V, R>(a, ws, lds, grid, gd_heads, stream))
-  DFA3D_CELL_DISPATCH(dtype, a.C, DFA3D_CELL_LAUNCH);
+#define DFA3D_CELL_LAUNCH(T, V, R, F) (launch_cell_cfg<T, V, R, F>(a, ws, lds, grid, gd_heads, stream))
+  DFA3D_CELL_DISPATCH(dtype, a, DFA3D_CELL_LAUNCH);
 #undef DFA3D_CELL_LAUNCH
 }
 

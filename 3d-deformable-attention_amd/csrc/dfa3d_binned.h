@@ -348,7 +348,7 @@ int cell_kernel_pass(int C);           // points per pass
 int cell_kernel_block(int C);          // threads per workgroup
 size_t cell_kernel_lds_bytes(int ty, int C, int D, int elem);
 size_t cell_kernel_half_cu_lds();      // the most dynamic LDS with which two of its workgroups fit a CU
-const void *cell_kernel_symbol(int dtype, int C, bool fused);
+const void *cell_kernel_symbol(const BwdArgs &a, int dtype);
 hipError_t launch_cell_kernel(const BwdArgs &a, int dtype, const BinWorkspace &ws, size_t lds, int grid, float *gd_heads,
                               hipStream_t stream);
 
