@@ -1,12 +1,11 @@
 """Builds libdfa3d_hip.so for gfx950 with hipcc (cross-compiles without a GPU).
 
-    python 3d-deformable-attention_amd/build.py [--force] [--experiment]
+    python 3d-deformable-attention_amd/build.py [--force] [--clocks]
 
 The library lands next to the python package (dfa3D/libdfa3d_hip.so) so that it travels with
 the source tree.  Two more libraries land beside bench.py, which is what uses them: the yardstick kernels
-(libdfa3d_measure.so) and, with --experiment, libdfa3d_hip_experiment.so: the same sources compiled with
--DDFA3D_EXPERIMENT -DDFA3D_TILE_TIMING, i.e. with the switches that cut parts out of the backward kernels and
-the per-phase clocks of the tile kernel (`bench.py --phase-costs`); its results are not the operator's.
+(libdfa3d_measure.so) and, with --clocks, libdfa3d_hip_clocks.so: the same sources compiled with
+-DDFA3D_TILE_TIMING, i.e. with the per-phase clocks of the backward's tile kernels (`bench.py --phase-costs`).
 """
 import os
 import subprocess
@@ -21,8 +20,8 @@ LIB = os.path.join(HERE, "dfa3D", "libdfa3d_hip.so")
 MEASURE_SRC = os.path.join(CSRC, "measure", "dfa3d_measure.hip")
 ROOT = os.path.dirname(HERE)
 MEASURE_LIB = os.path.join(ROOT, "libdfa3d_measure.so")
-EXPERIMENT_LIB = os.path.join(ROOT, "libdfa3d_hip_experiment.so")
-EXPERIMENT_FLAGS = ["-DDFA3D_EXPERIMENT", "-DDFA3D_TILE_TIMING"]
+CLOCKS_LIB = os.path.join(ROOT, "libdfa3d_hip_clocks.so")
+CLOCKS_FLAGS = ["-DDFA3D_TILE_TIMING"]
 SOURCES = ["dfa3d_forward.hip", "dfa3d_backward.hip", "dfa3d_backward_binned.hip", "dfa3d_backward_cells.hip",
            "dfa3d_rebatch.hip", "dfa3d_linear.hip", "dfa3d_locations.hip",
            "dfa3d_api.hip"]
@@ -66,16 +65,16 @@ def _build_lib(lib, obj_dir, extra_flags, force, verbose):
     return lib
 
 
-def build(force=False, verbose=True, experiment=False):
+def build(force=False, verbose=True, clocks=False):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     _build_lib(LIB, OBJ, [], force, verbose)
     if force or _stale(MEASURE_LIB, [MEASURE_SRC, os.path.join(CSRC, "measure", "dfa3d_measure.h")]):
         _run([hipcc, *FLAGS, "-shared", MEASURE_SRC, "-o", MEASURE_LIB], verbose)
-    if experiment:
-        _build_lib(EXPERIMENT_LIB, os.path.join(OBJ, "experiment"), EXPERIMENT_FLAGS, force, verbose)
+    if clocks:
+        _build_lib(CLOCKS_LIB, os.path.join(OBJ, "clocks"), CLOCKS_FLAGS, force, verbose)
     return LIB
 
 
 if __name__ == "__main__":
-    build(force="--force" in sys.argv, experiment="--experiment" in sys.argv)
+    build(force="--force" in sys.argv, clocks="--clocks" in sys.argv)
     print(LIB)

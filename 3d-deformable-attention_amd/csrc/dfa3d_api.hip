@@ -1,7 +1,6 @@
 // C ABI of libdfa3d_hip (declared in include/dfa3d.h): argument checks and dispatch.
 // Errors are returned, never printed-and-ignored (the reference's launchers only printf a failed
 // launch: DFA3D/dfa3D/ops/csrc/cuda/wms_deform_attn_cuda.cu:45-48).
-#include <atomic>
 #include <mutex>
 #include <cstdarg>
 #include <cstdio>
@@ -54,20 +53,9 @@ int check_opts(const char *fn, const dfa3d_launch_options *o, dfa3d_launch_optio
   return 0;
 }
 
-#ifdef DFA3D_EXPERIMENT
-// Development builds only: switches that cut parts out of the backward kernels to see what they cost
-// (results are then incomplete).  Not part of the library's ABI.
-std::atomic<int> g_diag{0};
-std::atomic<int> g_stage{0};
-#endif
-
 void apply_opts(dfa3d::BwdArgs &a, const dfa3d_launch_options &o) {
   a.iters = o.iters; a.vec_hint = o.vec; a.tile_hint = o.tile; a.block_hint = o.block; a.chunk_hint = o.chunk;
   a.pass_hint = o.pass; a.event_binned = o.event_binned; a.clear_grads = o.clear;
-#ifdef DFA3D_EXPERIMENT
-  a.diag = g_diag.load(std::memory_order_relaxed);
-  a.stage = g_stage.load(std::memory_order_relaxed);
-#endif
 }
 
 // Dimension checks shared by every entry point.  `width` is the per-head row length (C or D).
@@ -100,13 +88,8 @@ extern "C" {
 const char *dfa3d_last_error(void) { return g_err; }
 int dfa3d_abi_version(void) { return 9; }
 
-#ifdef DFA3D_EXPERIMENT
-int dfa3d_experiment_set(const char *name, int value) {
-  if (name != nullptr && !strcmp(name, "diag")) { g_diag.store(value, std::memory_order_relaxed); return 0; }
-  if (name != nullptr && !strcmp(name, "bwd_stage")) { g_stage.store(value, std::memory_order_relaxed); return 0; }
-  return fail(DFA3D_EINVAL, "dfa3d_experiment_set: unknown switch");
-}
-size_t dfa3d_experiment_timer_offset(void) { return dfa3d::tile_timer_offset(); }
+#ifdef DFA3D_TILE_TIMING
+size_t dfa3d_tile_timer_offset(void) { return dfa3d::tile_timer_offset(); }
 #endif
 
 int dfa3d_ms_depth_score_sample_forward(const void *dist, const int64_t *shapes3, const int64_t *level_start,

@@ -683,7 +683,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
     const T *__restrict__ grad_out, const T *__restrict__ grad_score_in,
     void *__restrict__ grad_value, void *__restrict__ grad_dist, float *__restrict__ grad_loc, int gl_stride,
     float *__restrict__ grad_attn, float *__restrict__ grad_score_out, const float *__restrict__ grad_wu, int Md,
-    int Mg, int B, int S, int M, int C, int D, int L, int Q, int P, int PP, int grad16 DFA3D_DIAG_PARAM) {
+    int Mg, int B, int S, int M, int C, int D, int L, int Q, int P, int PP, int grad16) {
   // grad16: bit 0 = grad_value is bfloat16, bit 1 = grad_dist is bfloat16 (else float)
   // Md: heads stored in dist (M, or 1 = shared by all heads); Mg: heads of the grad_dist buffer written here
   constexpr int RPI = kWave / LPR;                  // row groups per wavefront
@@ -776,7 +776,6 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
         g = locate_2d<float>(rec.x, rec.y, H, W, start);
         if (FUSED) {
           tap = locate_depth<float>(rec.z, Dd);
-          if (DFA3D_DIAG(diag, 32)) { for (int k = 0; k < 4; ++k) { sc[k] = 0.5f; hl[k] = 0.1f; } } else   // cost of the depth taps
           {
             float lo[4], hi[4];
             corner_scores<T, float, true>(dist_r, g.key, tap, md, Md, D, sc, lo, hi);
@@ -828,7 +827,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
       // a fifth of the taps at 256 points per pass) use the floating-point atomic, after that barrier.  Stale
       // words cannot do harm: one that happens to equal the tag just sends its address's taps to the atomics.
       int *tickets = reinterpret_cast<int *>(gstage);
-      const bool ticketed = FUSED && R * D <= PP * C && !DFA3D_DIAG(diag, 1024);     // uniform over the workgroup
+      const bool ticketed = FUSED && R * D <= PP * C;         // uniform over the workgroup
       ++pass_tag;
       // the previous pass's points as phase A left them
       Point2D<float> g;
@@ -844,7 +843,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
       const size_t gp = st_gp;
       float gs[4] = {0, 0, 0, 0};
       unsigned first_mask = 0;              // bit 2k / 2k+1: this thread took the first ticket of corner k's lower / upper tap
-      if (prev_mine && live && !DFA3D_DIAG(diag, 512)) {               // (development builds: cost of phase C)
+      if (prev_mine && live) {
         float s[4], ga = 0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -875,13 +874,13 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
           int at8[8];                               // tile address of each of the eight taps, -1 = no tap
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            const bool taps = trc[k] >= 0 && tap.inside && gs[k] != 0 && !DFA3D_DIAG(diag, 2);
+            const bool taps = trc[k] >= 0 && tap.inside && gs[k] != 0;
             const int at = trc[k] * D + tap.d0;
             at8[2 * k] = (taps && tap.lo_ok) ? at : -1;
             at8[2 * k + 1] = (taps && tap.hi_ok) ? at + 1 : -1;
             if (!taps) {
               gs[k] = ((on_bits >> k & 1) && tap.inside) ? gs[k] : 0.f;      // no taps below for this corner
-              if (!(trc[k] >= 0 && tap.inside) || DFA3D_DIAG(diag, 2)) trc[k] = -1;
+              if (!(trc[k] >= 0 && tap.inside)) trc[k] = -1;
             }
             gz += ((on_bits >> k & 1) && tap.inside) ? gs[k] * hl[k] : 0.f;
           }
@@ -945,7 +944,6 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
           const bool slot_ok = sub < stage_per_wave;
           const int slot = wave * stage_per_wave + min(sub, stage_per_wave - 1);
           float gg[VEC];
-          if (DFA3D_DIAG(diag, 256)) { for (int i = 0; i < VEC; ++i) gg[i] = 1.f; } else   // cost of the grad_out loads
           RowVec<T, float, VEC>::ld(go_r, goff[slot] + chan_off, gg);
           if (slot_ok && chan < C) LdsVec<VEC>::st(gstage + slot * C + chan, gg);
         }
@@ -991,7 +989,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
         {
           const int r = group;
           const int y = y0 + r / TW, x = x0 + r % TW;
-          const bool ld_ok = r < R && offs[min(r, R - 1) + 1] > offs[min(r, R - 1)] && in_map(y, x, H, W) && !DFA3D_DIAG(diag, 8);
+          const bool ld_ok = r < R && offs[min(r, R - 1) + 1] > offs[min(r, R - 1)] && in_map(y, x, H, W);
           RowVec<T, float, VEC>::ld(value_r, (ld_ok ? (uint32_t)(((start + y * W + x) * M + m) * C * (int)sizeof(T)) : kNoRow) + chan_off, v_next);
         }
         for (int r0 = 0; r0 < R; r0 += kGroups) {        // uniform over the workgroup
@@ -1010,10 +1008,9 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
           {                                              // value row of this group's next round
             const int rn = r + kGroups;
             const int yn = y0 + rn / TW, xn = x0 + rn % TW;
-            const bool ld_ok = rn < R && offs[min(rn, R - 1) + 1] > offs[min(rn, R - 1)] && in_map(yn, xn, H, W) && !DFA3D_DIAG(diag, 8);
+            const bool ld_ok = rn < R && offs[min(rn, R - 1) + 1] > offs[min(rn, R - 1)] && in_map(yn, xn, H, W);
             RowVec<T, float, VEC>::ld(value_r, (ld_ok ? (uint32_t)(((start + yn * W + xn) * M + m) * C * (int)sizeof(T)) : kNoRow) + chan_off, v_next);
           }
-          if (DFA3D_DIAG(diag, 16)) n_max = 0;                      // cost of the task loop
           if (n_max == 0) continue;                      // wave-uniform
           // tasks in flight per group: registers decide (measured: 4 with four channels per lane, 1 with eight;
           // one more costs 1 % .. 10 % of the kernel's time)
@@ -1054,7 +1051,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
               else dots[di] += part[j];
             }
           }
-          if (pix_ok && chan_ok && !DFA3D_DIAG(diag, 1)) {
+          if (pix_ok && chan_ok) {
             float *dst = gv + r * C + chan;
             float cur[VEC];
             LdsVec<VEC>::ld(dst, cur);
@@ -1113,7 +1110,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
         if (nz) *reinterpret_cast<float4 *>(gv + r * C + c) = make_float4(0, 0, 0, 0);
         const int ry = r / TW, rx = r - ry * TW;
         const int y = y0 + ry, x = x0 + rx;
-        if (in_map(y, x, H, W) && !DFA3D_DIAG(diag, 4)) {
+        if (in_map(y, x, H, W)) {
           const uint32_t e = (uint32_t)(((start + y * W + x) * M + m) * C + c);
           const bool store = sole && ry >= 1 && ry < TY && rx >= 1 && rx < TX;
           if (store || nz) put4(gvalue_b, gvalue_r, gv16, e, val, store, true);
@@ -1126,7 +1123,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
         if (nz) *reinterpret_cast<float4 *>(gd + r * D + d) = make_float4(0, 0, 0, 0);
         const int ry = r / TW, rx = r - ry * TW;
         const int y = y0 + ry, x = x0 + rx;
-        if (in_map(y, x, H, W) && !DFA3D_DIAG(diag, 4)) {
+        if (in_map(y, x, H, W)) {
           const uint32_t e = (uint32_t)(((start + y * W + x) * Mg + mg) * D + d);
           const bool store = sole_d && ry >= 1 && ry < TY && rx >= 1 && rx < TX;
           if (store || nz) put4(gdist_b, gdist_r, gd16, e, val, store, false);
@@ -1141,7 +1138,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
           const int r = i / C, c = i - r * C;
           const int ry = r / TW, rx = r % TW;
           const int y = y0 + ry, x = x0 + rx;
-          if (in_map(y, x, H, W) && !DFA3D_DIAG(diag, 4))
+          if (in_map(y, x, H, W))
             scatter_add(gvalue_r, gvalue_f, (uint32_t)((((start + y * W + x) * M + m) * C + c) * 4), val);
         }
       }
@@ -1152,7 +1149,7 @@ __global__ __launch_bounds__(512, 4) void tile_backward_kernel(
           const int r = i / D, d = i - r * D;
           const int ry = r / TW, rx = r % TW;
           const int y = y0 + ry, x = x0 + rx;
-          if (in_map(y, x, H, W) && !DFA3D_DIAG(diag, 4))
+          if (in_map(y, x, H, W))
             scatter_add(gdist_r, gdist_f, (uint32_t)((((start + y * W + x) * Mg + mg) * D + d) * 4), val);
         }
       }
@@ -1441,8 +1438,8 @@ static BinLayout bin_layout(const BwdArgs &a, int ty, int tx, bool float_sums) {
   return o;
 }
 
-#ifdef DFA3D_EXPERIMENT
-// development builds: where in a workspace the tile kernel's phase clocks live (ten 64-bit counters)
+#ifdef DFA3D_TILE_TIMING
+// development builds: where in a workspace the tile kernels' phase clocks live (sixteen 64-bit counters)
 size_t tile_timer_offset() {
   return ((sizeof(BinPlan) + 255) & ~(size_t)255) + (size_t)kClasses * kQueueStride * sizeof(int);
 }
@@ -1631,7 +1628,7 @@ static hipError_t launch_tile_cfg(const BwdArgs &a, const BinWorkspace &ws, cons
                        gd_heads != nullptr ? (void *)gd_heads : a.grad_dist, (float *)a.grad_loc, a.grad_loc_stride, (float *)a.grad_attn,
                        (float *)nullptr, (const float *)a.grad_weight_update, a.dist_heads == 1 ? 1 : a.M,
                        (a.dist_heads == 1 && gd_heads == nullptr) ? 1 : a.M, a.B, a.S, a.M, a.C, a.D, a.L, a.Q, a.P, c.pp,
-                       (a.grad_bf16 ? 1 : 0) | ((a.grad_bf16 && gd_heads == nullptr) ? 2 : 0) DFA3D_DIAG_ARG(a));
+                       (a.grad_bf16 ? 1 : 0) | ((a.grad_bf16 && gd_heads == nullptr) ? 2 : 0));
   } else {
     auto kern = tile_backward_kernel<T, VEC, LPR, false>;
     if (hipError_t e = allow_lds(kern, c.lds)) return e;
@@ -1639,7 +1636,7 @@ static hipError_t launch_tile_cfg(const BwdArgs &a, const BinWorkspace &ws, cons
                        (const T *)a.score_in, (const T *)a.grad_out, (const T *)nullptr, a.grad_value,
                        (void *)nullptr, (float *)a.grad_loc, a.grad_loc_stride, (float *)a.grad_attn,
                        (float *)a.grad_score_out, (const float *)nullptr, a.M, a.M, a.B, a.S, a.M, a.C, 0, a.L, a.Q,
-                       a.P, c.pp, 0 DFA3D_DIAG_ARG(a));
+                       a.P, c.pp, 0);
   }
   return hipGetLastError();
 }
@@ -1770,21 +1767,10 @@ hipError_t launch_backward_binned(const BwdArgs &args, int dtype, void *workspac
     if (!shared_dist(a)) a.grad_dist = static_cast<char *>(workspace) + lay.dist_sums;
   }
   float *gd_heads = shared_dist(a) ? reinterpret_cast<float *>(static_cast<char *>(workspace) + lay.gd_heads) : nullptr;
-#ifdef DFA3D_EXPERIMENT
-  const int stage = a.stage;                     // development builds: 1 = binning launches only, 2 = tile kernel only
-#else
-  constexpr int stage = 0;
-#endif
-  if (stage == 0 || stage == 1) {
-    if (hipError_t e = run_binning(a, ws, cfg, gd_heads, stream)) return e;
-  }
+  if (hipError_t e = run_binning(a, ws, cfg, gd_heads, stream)) return e;
   if (a.event_binned != nullptr) {
     if (hipError_t e = hipEventRecord((hipEvent_t)a.event_binned, stream)) return e;
   }
-  if (stage == 1) return hipSuccess;
-  if (gd_heads != nullptr && stage == 2)
-    hipLaunchKernelGGL(fill_zero_kernel, dim3(2048), dim3(256), 0, stream, reinterpret_cast<float4 *>(gd_heads),
-                       ((size_t)a.B * a.S * a.M * a.D + 3) / 4);
   const hipError_t e = dtype == DFA3D_F32 ? launch_tile_typed<float>(a, ws, cfg, gd_heads, stream)
                                           : launch_tile_typed<__hip_bfloat16>(a, ws, cfg, gd_heads, stream);
   if (e != hipSuccess) return e;

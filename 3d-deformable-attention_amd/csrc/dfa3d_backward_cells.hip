@@ -40,14 +40,16 @@ namespace dfa3d {
 constexpr int kWalkers = 256;         // threads of the walker wavefronts 0-3; the wavefronts after them own the points
 
 #ifdef DFA3D_TILE_TIMING
-// thread 0 (a walker) clocks slots 0-7, thread 256 (a pointer) slots 8-15
-#define CT_DECL unsigned long long ct_acc[8] = {0, 0, 0, 0, 0, 0, 0, 0}; unsigned long long ct_last = clock64();
-#define CT_MARK(i) do { if ((threadIdx.x & 255) == 0) { const unsigned long long ct_now = clock64(); ct_acc[(i) & 7] += ct_now - ct_last; ct_last = ct_now; } } while (0)
-#define CT_FLUSH() do { if ((threadIdx.x & 255) == 0) { unsigned long long *ct_g = reinterpret_cast<unsigned long long *>(ws.queues + kClasses * kQueueStride) + (threadIdx.x ? 8 : 0); for (int i = 0; i < 8; ++i) atomicAdd(ct_g + i, ct_acc[i]); } } while (0)
+// wavefront 0 (walkers) clocks slots 0-7, wavefront 4 (pointers) slots 8-15
+#define CT_DECL TICKS_DECL(16)
+#define CT_MARK(i) TICKS_MARK((wave & 3) == 0, (i) + 2 * wave)
+#define CT_FLUSH() TICKS_FLUSH((wave & 3) == 0, 2 * wave, 8)
+constexpr size_t kTicksLds = 16 * sizeof(unsigned long long);
 #else
 #define CT_DECL
 #define CT_MARK(i) do { } while (0)
 #define CT_FLUSH() do { } while (0)
+constexpr size_t kTicksLds = 0;
 #endif
 
 // Lane groups by row length: LPR lanes of VEC channels per row, 64 / LPR cells per wavefront; points per pass, one per
@@ -135,7 +137,7 @@ constexpr int kItemSlots = 8;      // a power of two; in use: the item before (f
 __device__ __forceinline__ int slot_of_item(int it) { return it & (kItemSlots - 1); }
 // what the kernel declares as static LDS (level tables, the fetching thread's state, item records): the dynamic
 // block of each of two workgroups on a CU may be half of the CU's 160 KB less this
-constexpr size_t kCellStaticLds = 4 * DFA3D_MAX_LEVELS * sizeof(int) + sizeof(CellFetch) + kItemSlots * sizeof(ItemGeom);
+constexpr size_t kCellStaticLds = 4 * DFA3D_MAX_LEVELS * sizeof(int) + sizeof(CellFetch) + kItemSlots * sizeof(ItemGeom) + kTicksLds;
 size_t cell_kernel_half_cu_lds() { return 80 * 1024 - kCellStaticLds; }
 // an item record read from LDS is the same in every lane: keep it in scalar registers
 __device__ __forceinline__ ItemGeom uniform(const ItemGeom &g) {
@@ -367,9 +369,6 @@ template <typename T> struct CellArgs {
   int B, S, M, C, D, L, Q, P;
   FastDiv div_lp;
   int grad16;                 // bit 0 = grad_value is bfloat16, bit 1 = grad_dist is bfloat16 (else float)
-#ifdef DFA3D_EXPERIMENT
-  int diag;
-#endif
 };
 #ifdef __HIP_DEVICE_COMPILE__
 template <typename T> using CellArgsPtr = const __attribute__((address_space(4))) CellArgs<T> *;
@@ -460,7 +459,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       for (int i = first >> sh; i < inner; i += threads >> sh) {
         const int ry = i / (TX - 1) + 1, rx = i % (TX - 1) + 1, r = ry * TW + rx;
         const int y = q.y0 + ry, x = q.x0 + rx;
-        const bool out = y < q.H && x < q.W && !DFA3D_DIAG(arg()->diag, 4);
+        const bool out = y < q.H && x < q.W;
         const uint32_t e0 = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D);
         for (int c = first & ((1 << sh) - 1); c < n; c += 1 << sh) {
           if (d4) {
@@ -489,7 +488,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         ry = i / TW; rx = i % TW;
       }
       const int r = ry * TW + rx, y = q.y0 + ry, x = q.x0 + rx;
-      const bool out = in_map(y, x, q.H, q.W) && !DFA3D_DIAG(arg()->diag, 4);
+      const bool out = in_map(y, x, q.H, q.W);
       const uint32_t e0 = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D);
       for (int c = first & ((1 << sh) - 1); c < n; c += 1 << sh) {
         if (gd16) {
@@ -565,7 +564,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
       void *grad_value = a->grad_value;
       const int y = q.y0 + o.crow, x = q.x0 + o.ccol;
       if (active && (o.crow == 0 || o.ccol == 0)) put_lds(o, rim + rim_index(o.crow, o.ccol, TY, TX) * ROW, u);
-      if (active && o.crow > 0 && o.ccol > 0 && y < q.H && x < q.W && !DFA3D_DIAG(arg()->diag, 4)) {
+      if (active && o.crow > 0 && o.ccol > 0 && y < q.H && x < q.W) {
         char *gvalue_b = static_cast<char *>(grad_value) + (size_t)q.b * S * M * C * (gv16 ? 2 : 4);
         float *gvalue_f = reinterpret_cast<float *>(gvalue_b);
         const rsrc_t gvalue_r = make_rsrc(gvalue_b, (size_t)S * M * C * sizeof(float));
@@ -605,7 +604,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         const int y = q.y0 + ry, x = q.x0 + rx;
         const float *from = rim + k * ROW + c;
         const float f0 = from[0], f1 = gv16 ? from[1] : 0.f;
-        if (c < C && in_map(y, x, q.H, q.W) && (f0 != 0 || f1 != 0) && !DFA3D_DIAG(arg()->diag, 4)) {
+        if (c < C && in_map(y, x, q.H, q.W) && (f0 != 0 || f1 != 0)) {
           const uint32_t e = (uint32_t)(((q.start + y * q.W + x) * M + q.m) * C + c);
           if (gv16) atomic_add_bf16x2(gvalue_b + (size_t)e * 2, f0, f1);
           else scatter_add(gvalue_r, gvalue_f, e * 4, f0);
@@ -841,7 +840,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
             const int y = g.y0 + o.crow + (k >= 2 ? 1 : 0), x = g.x0 + o.ccol + ((k == 1 || k == 2) ? 1 : 0);
-            const bool ok = !done && o.crow < TY && in_map(y, x, g.H, g.W) && !DFA3D_DIAG(arg()->diag, 8);
+            const bool ok = !done && o.crow < TY && in_map(y, x, g.H, g.W);
             o.ch.load(value_r, ok ? (uint32_t)(((g.start + y * g.W + x) * M + g.m) * C * (int)sizeof(T)) : kNoRow, vr[k]);
           }
         }
@@ -889,7 +888,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = (f4){0, 0, 0, 0};
         CT_MARK(5);
-        if (apart() && !DFA3D_DIAG(arg()->diag, 16)) walk(v, acc);
+        if (apart()) walk(v, acc);
         CT_MARK(1);
         lds_barrier();
         CT_MARK(2);
@@ -902,7 +901,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           CT_MARK(4);
           ++turn;
           clear_counts();
-          if (apart() && !DFA3D_DIAG(arg()->diag, 16)) walk(v, acc);
+          if (apart()) walk(v, acc);
           CT_MARK(1);
           lds_barrier();
           CT_MARK(2);
@@ -976,7 +975,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         uint32_t off[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          off[k] = ((on_bits >> k & 1) && tap.inside && !DFA3D_DIAG(arg()->diag, 32)) ? (uint32_t)(((pg.key[k] * Md + md) * D + db) * (int)sizeof(T)) : kNoRow;
+          off[k] = ((on_bits >> k & 1) && tap.inside) ? (uint32_t)(((pg.key[k] * Md + md) * D + db) * (int)sizeof(T)) : kNoRow;
         taps.ask(dist_r, off, D);
       } else if (score_in != nullptr) {                      // uniform
         const T *si = score_in + (size_t)gp * 4;
@@ -1069,7 +1068,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         if (now.bits & 128u) s_slot[offs[(now.bits >> 8) & 63] + rank_now] = (uint16_t)pslot;
       }
       CT_MARK(4);
-      if (valid1 && !DFA3D_DIAG(arg()->diag, 512)) {                // (development builds: cost of phase C)
+      if (valid1) {
         const ItemGeom &q = s_geom[slot_of_item(it1)];
         const int gH = __builtin_amdgcn_readfirstlane(q.H), gW = __builtin_amdgcn_readfirstlane(q.W), gDd = __builtin_amdgcn_readfirstlane(q.Dd);
         const int gb = __builtin_amdgcn_readfirstlane(q.b);
@@ -1122,7 +1121,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ga), ga_r, ga_off, 0, 0);
           // The taps.  One that does not exist adds zero to a word nearby: the four pixels always lie in the tile, the bins
           // are clamped.
-          if (live && !DFA3D_DIAG(arg()->diag, 2)) {
+          if (live) {
             const int row0 = (ccy * TW + ccx) * D, lo_at = max(tap.d0, 0), hi_at = min(tap.d0 + 1, D - 1);
             const float w_lo = tap.lo_ok ? tap.hd : 0.f, w_hi = tap.hi_ok ? tap.ld : 0.f;
             int at[8];
@@ -1185,8 +1184,7 @@ static hipError_t launch_cell_cfg(const BwdArgs &a, const BinWorkspace &ws, size
                          fused ? (const float *)a.grad_weight_update : nullptr, a.grad_loc_stride,
                          fused && one ? 1 : a.M, fused && one && gd_heads == nullptr ? 1 : a.M,
                          a.B, a.S, a.M, a.C, fused ? a.D : 0, a.L, a.Q, a.P, FastDiv((uint32_t)(a.L * a.P)),
-                         !fused ? 0 : (a.grad_bf16 ? 1 : 0) | (a.grad_bf16 && gd_heads == nullptr ? 2 : 0)
-                         DFA3D_DIAG_ARG(a)};
+                         !fused ? 0 : (a.grad_bf16 ? 1 : 0) | (a.grad_bf16 && gd_heads == nullptr ? 2 : 0)};
   const dim3 block(kWalkers + cell_pass(LPR));
   if (fused) hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, true, FOURS>), dim3(grid), block, lds, stream, c);
   else hipLaunchKernelGGL((cell_backward_kernel<T, VEC, LPR, false, FOURS>), dim3(grid), block, lds, stream, c);

@@ -116,13 +116,17 @@ __device__ __forceinline__ int chunk_of(const BinWorkspace &ws, const BinPlan &p
 __device__ __forceinline__ int items_of_bin(int c, int ch) { return c <= ch ? (c > 0 ? 1 : 0) : (c + ch - 1) / ch; }
 __device__ __forceinline__ int share_begin(int c, int k, int t) { const int q = c / k; return t * q + min(t, c - q * k); }
 
-// Optional phase timing of the tile kernel (development builds only, -DDFA3D_TILE_TIMING): thread 0
-// of every workgroup accumulates shader-clock ticks per phase and adds them to 64-bit counters that
-// live in the padding behind the queue counter.
+// Optional phase clocks of the tile kernels (development builds only, -DDFA3D_TILE_TIMING).  A wavefront or two of every
+// workgroup count shader-clock ticks per phase and add them to 64-bit counters that live in the padding behind the queue
+// counters.  The clock is a scalar and the sums are in LDS, so that the kernel keeps the registers that it has without them.
 #ifdef DFA3D_TILE_TIMING
-#define TT_DECL unsigned long long tt_acc[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0}; unsigned long long tt_last = clock64();
-#define TT_MARK(i) do { if (threadIdx.x == 0) { const unsigned long long tt_now = clock64(); tt_acc[i] += tt_now - tt_last; tt_last = tt_now; } } while (0)
-#define TT_FLUSH() do { if (threadIdx.x == 0) { unsigned long long *tt_g = reinterpret_cast<unsigned long long *>(ws.queues + kClasses * kQueueStride); for (int i = 0; i < 10; ++i) atomicAdd(tt_g + i, tt_acc[i]); } } while (0)
+#define TICKS_DECL(n) __shared__ unsigned long long s_ticks[n]; for (int i = threadIdx.x; i < (n); i += blockDim.x) s_ticks[i] = 0; __syncthreads(); unsigned long long ticks_last = clock64();
+#define TICKS_MARK(mine, slot) do { if (mine) { const unsigned long long ticks_now = clock64(); if (threadIdx.x % kWave == 0) atomicAdd(&s_ticks[slot], ticks_now - ticks_last); ticks_last = ticks_now; } } while (0)
+#define TICKS_FLUSH(mine, first, n) do { if ((mine) && threadIdx.x % kWave < (n)) atomicAdd(reinterpret_cast<unsigned long long *>(ws.queues + kClasses * kQueueStride) + (first) + threadIdx.x % kWave, s_ticks[(first) + threadIdx.x % kWave]); } while (0)
+#define TT_MINE (__builtin_amdgcn_readfirstlane(threadIdx.x / kWave) == 0)
+#define TT_DECL TICKS_DECL(10)
+#define TT_MARK(i) TICKS_MARK(TT_MINE, i)
+#define TT_FLUSH() TICKS_FLUSH(TT_MINE, 0, 10)
 #else
 #define TT_DECL
 #define TT_MARK(i) do { } while (0)

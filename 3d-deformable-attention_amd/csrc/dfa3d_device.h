@@ -24,18 +24,6 @@
 
 namespace dfa3d {
 
-// Development builds (-DDFA3D_EXPERIMENT) can cut parts out of the backward kernels to see what they cost;
-// in the library as shipped the switches are constant zero and the compiler drops them.
-#ifdef DFA3D_EXPERIMENT
-#define DFA3D_DIAG(diag, bits) (((diag) & (bits)) != 0)
-#define DFA3D_DIAG_PARAM , int diag          // last kernel parameter, development builds only
-#define DFA3D_DIAG_ARG(a) , (a).diag
-#else
-#define DFA3D_DIAG(diag, bits) false
-#define DFA3D_DIAG_PARAM
-#define DFA3D_DIAG_ARG(a)
-#endif
-
 constexpr int kWave = 64;
 constexpr int kWavesPerBlock = 4;
 constexpr int kBlock = kWave * kWavesPerBlock;

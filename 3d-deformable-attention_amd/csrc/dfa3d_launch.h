@@ -96,10 +96,6 @@ struct BwdArgs {
   int B, S, M, C, D, L, Q, P;
   int iters;
   int vec_hint;
-#ifdef DFA3D_EXPERIMENT
-  int diag;                          // development builds only: parts of the kernels cut out
-  int stage;                         // development builds only: 1 binning kernels only, 2 tile kernel only
-#endif
   int tile_hint;                     // binned path: tile edge as ty * 100 + tx (0 = automatic)
   int block_hint;                    // binned path: threads per tile workgroup (0 = 512)
   int chunk_hint;                    // binned path: points of a bin per work item (0: by the number of points)
@@ -134,7 +130,7 @@ hipError_t launch_depth_score_backward_binned(const DepthScoreBwdArgs &d, int dt
                                               size_t workspace_bytes, int tile_hint, int chunk_hint,
                                               void *event_binned, hipStream_t stream);
 
-#ifdef DFA3D_EXPERIMENT
+#ifdef DFA3D_TILE_TIMING
 size_t tile_timer_offset();
 #endif
 

@@ -4,8 +4,8 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload base|small|unit|dense|base_bf16|base_f64|unittest|base_coherent]
     python bench.py --micro [xcd]                yardsticks of the machine (copy, bare gathers, LDS atomics, XCD map)
     python bench.py --summarize NAME DIR [DIR..] tables from rocprofv3 output directories -> profiles/NAME.txt
-    python bench.py --phase-costs [--workload W] what the parts of the backward's tile kernel cost (development build of
-                                                 the library: `python 3d-deformable-attention_amd/build.py --experiment`)
+    python bench.py --phase-costs [--workload W] where the backward's tile kernel spends its time (build of the library with
+                                                 clocks: `python 3d-deformable-attention_amd/build.py --clocks`)
 
 A step is one forward + backward of the one-stage autograd Function
 (MultiScale3DDeformableAttnFunction.apply -> torch.autograd.grad) over one batch of synthetic
@@ -64,8 +64,8 @@ def parse():
     ap.add_argument("--micro", nargs="?", const="all", choices=("all", "xcd"),
                     help="run the yardstick kernels instead of the operator (xcd: only the workgroup -> XCD map)")
     ap.add_argument("--phase-costs", action="store_true",
-                    help="time the tile kernel of the backward with parts of it cut out, and its per-phase clocks "
-                         "(needs libdfa3d_hip_experiment.so; prints a text table)")
+                    help="per-phase clocks of the backward's tile kernel, and what it takes with and without them "
+                         "(needs libdfa3d_hip_clocks.so; prints a text table)")
     ap.add_argument("--summarize", nargs="+", metavar=("NAME", "DIR"),
                     help="write profiles/NAME.txt (and profiles/hbm_traffic.json) from rocprofv3 output directories")
     ap.add_argument("--summarize-command", action="append", default=[],
@@ -520,21 +520,10 @@ def cpu_baseline(w, budget_s):
                       f"OpenMP over units (forward) and over the {sample.B} batch elements (backward)"}
 
 
-# What the development build can cut out of the tile kernels (dfa3d_experiment_set("diag", bits)): bits, what the
-# cell-owned kernel (cell_backward_kernel) and the row-owned one (tile_backward_kernel) then leave out, None = no such part.
-PHASE_CUTS = ((16, "the walk of the cells' lists (dot products, weighted sums)", "the task loop of the rows phase"),
-              (512, "the per-point gradients and grad_dist taps (finish)", "the per-point gradients and grad_dist taps (phase C)"),
-              (2, "the grad_dist taps alone", "the grad_dist taps alone"),
-              (4, "the device writes of both flushes", "the flush's device writes"),
-              (1, None, "the LDS tile updates of the rows phase"),
-              (256, None, "the grad_out row loads"),
-              (32, "the depth taps' loads (prepare)", "the depth taps of phase A"),
-              (8, "the value row loads", "the value row loads"),
-              (1024, None, "tickets (every grad_dist tap an LDS float atomic)"))
-# The phases that are clocked (-DDFA3D_TILE_TIMING), by slot.  Row-owned kernel: thread 0's clock, ten slots.
+# The phases that are clocked (-DDFA3D_TILE_TIMING), by slot.  Row-owned kernel: wavefront 0's clock, ten slots.
 PHASE_CLOCKS_ROWS = ("item fetch", "barrier after phases A and C", "rank + staging", "scan + placement", "rows",
                      "phases A and C", "flush", "tail", "-", "-")
-# cell-owned kernel: thread 0 (a walker) fills slots 0-7, thread 256 (a pointer) slots 8-15
+# cell-owned kernel: wavefront 0 (walkers) fills slots 0-7, wavefront 4 (pointers) slots 8-15
 PHASE_CLOCKS_CELLS = ("walker: set-up, the next item's record", "walker: walk (phase X)", "walker: wait at the barrier after X",
                       "walker: item record fetched, the old item's sums put together (phase Y)",
                       "walker: wait at the barrier after Y",
@@ -548,19 +537,19 @@ PHASE_CLOCKS_CELLS = ("walker: set-up, the next item's record", "walker: walk (p
 
 
 def phase_costs(a):
-    """Text table: tile kernel duration with each part cut out (the difference to the whole kernel is what that part
-    costs where it stands), and the share of its clock that a thread of each role spends in each phase."""
+    """Text table: the share of its clock that a wavefront of each role spends in each phase of the tile kernel, and the
+    kernel's duration with the clocks and as shipped."""
     import torch
     from dfa3D import _lib
-    _lib.LIB_PATH = os.path.join(ROOT, "libdfa3d_hip_experiment.so")
+    from dfa3D.workloads import WORKLOADS, make_inputs
+    shipped = _lib.lib()
+    _lib.LIB_PATH, _lib._lib = os.path.join(ROOT, "libdfa3d_hip_clocks.so"), None
     if not os.path.exists(_lib.LIB_PATH):
-        print("bench.py: build the development library first: python 3d-deformable-attention_amd/build.py --experiment",
+        print("bench.py: build the library with clocks first: python 3d-deformable-attention_amd/build.py --clocks",
               file=sys.stderr)
         sys.exit(3)
-    from dfa3D.workloads import WORKLOADS, make_inputs
-    L_ = _lib.lib()
-    L_.dfa3d_experiment_set.argtypes = [ctypes.c_char_p, ctypes.c_int]
-    L_.dfa3d_experiment_timer_offset.restype = ctypes.c_size_t
+    clocked = _lib.lib()
+    clocked.dfa3d_tile_timer_offset.restype = ctypes.c_size_t
     bf16 = a.workload.endswith("_bf16")
     w = WORKLOADS["base_peaky" if a.workload == "base_bf16" else a.workload]
     dev = torch.device("cuda:0")
@@ -581,24 +570,24 @@ def phase_costs(a):
     mid.record()
     torch.cuda.synchronize()
     opts = ctypes.pointer(_lib.LaunchOptions(event_binned=mid.cuda_event, **fields))
-    nbytes = L_.dfa3d_fused_backward_workspace_bytes(B, S, M, C, D, L, Q, P, M, code, opts)
+    nbytes = shipped.dfa3d_fused_backward_workspace_bytes(B, S, M, C, D, L, Q, P, M, code, opts)
     assert nbytes > 0, "the binned backward does not take this workload"
     ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
 
-    def call():
-        _lib.check(L_.dfa3d_fused_backward(
+    def call(library):
+        _lib.check(library.dfa3d_fused_backward(
             _lib.ptr(value), _lib.ptr(dist), _lib.ptr(shapes), _lib.ptr(lsi), _lib.ptr(loc), _lib.ptr(attn), _lib.ptr(go),
             None, None, _lib.ptr(gv), _lib.ptr(gd), _lib.ptr(gl), _lib.ptr(ga), _lib.ptr(ws), nbytes, B, S, M, C, D, L, Q,
             P, M, code, opts, _lib.stream_of(value)), "dfa3d_fused_backward")
 
-    def timed(reps):
+    def timed(library, reps):
         bins, tiles = [], []
         for i in range(reps + 3):
             gv.zero_()
             gd.zero_()
             e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             e0.record()
-            call()
+            call(library)
             e1.record()
             e1.synchronize()
             if i >= 3:
@@ -609,32 +598,21 @@ def phase_costs(a):
         return bins[len(bins) // 2], tiles[len(tiles) // 2]
 
     print(f"# python bench.py --phase-costs --workload {a.workload}" + "".join(f" --option {t}" for t in a.option))
-    print(f"# development build (-DDFA3D_EXPERIMENT -DDFA3D_TILE_TIMING) of the kernel sources with digest {sources_digest()[:16]}")
-    print(f"# {torch.cuda.get_device_name(0)}; {w.points} points; medians of {a.kernel_reps} launches; a cut changes results, "
-          "its row says what the kernel takes WITHOUT that part, and whole just before and after")
-    call()                                       # once for the clocks, which say which of the kernels the workload takes
+    print(f"# build with clocks (-DDFA3D_TILE_TIMING) of the kernel sources with digest {sources_digest()[:16]}")
+    print(f"# {torch.cuda.get_device_name(0)}; {w.points} points; medians of {a.kernel_reps} launches")
+    call(clocked)
     ws.zero_()
-    call()
+    call(clocked)
     torch.cuda.synchronize()
-    off = L_.dfa3d_experiment_timer_offset()
+    off = clocked.dfa3d_tile_timer_offset()
     ticks = ws[off:off + 128].view(torch.int64).cpu().tolist()
     cells = any(ticks[10:])                      # only the cell-owned kernel clocks more than ten slots
     names = PHASE_CLOCKS_CELLS if cells else PHASE_CLOCKS_ROWS
-    print(f"{'cut out':72s} {'binning ms':>10s} {'tile ms':>9s} {'whole ms':>9s} {'saves ms':>9s}")
-    timed(a.kernel_reps)
-    b_ms, before = timed(a.kernel_reps)
-    print(f"{'nothing (the kernel as shipped, with the phase clocks compiled in)':72s} {b_ms:10.4f} {before:9.4f}", flush=True)
-    for bits, *labels in PHASE_CUTS:
-        label = labels[0 if cells else 1]
-        if label is None:
-            continue
-        L_.dfa3d_experiment_set(b"diag", bits)
-        b_ms, t_ms = timed(a.kernel_reps)
-        L_.dfa3d_experiment_set(b"diag", 0)
-        _, after = timed(a.kernel_reps)          # the whole kernel before and after each cut: the clock drifts
-        whole, before = (before + after) / 2, after
-        print(f"{label:72s} {b_ms:10.4f} {t_ms:9.4f} {whole:9.4f} {whole - t_ms:9.4f}", flush=True)
-    print("\nshare of a thread's clock per phase, summed over the workgroups of one launch"
+    timed(shipped, a.kernel_reps)
+    print(f"{'':40s} {'binning ms':>10s} {'tile ms':>9s}")
+    for label, library in (("the kernel as shipped", shipped), ("with the clocks", clocked), ("as shipped, again", shipped)):
+        print("{:40s} {:10.4f} {:9.4f}".format(label, *timed(library, a.kernel_reps)), flush=True)
+    print("\nshare of a wavefront's clock per phase, summed over the workgroups of one launch"
           + (" (walkers: wavefronts 0-3, pointers: wavefronts 4-7; each role's shares add up to 100 %)" if cells else ""))
     for lo, hi in ((0, 8), (8, 16)) if cells else ((0, 10),):
         total = sum(ticks[lo:hi]) or 1
