@@ -352,12 +352,7 @@ __device__ __forceinline__ void load_to_lds16(rsrc_t r, const void *lds, uint32_
 }
 __device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }           // vmcnt(0)
 
-// The kernel's arguments.  They are read from the constant segment anew in every phase (args()): there are more of them, and
-// of the numbers that follow from them, than scalar registers.  Passed one by one they were kept from turn to turn, at the
-// cost of 98 others (float, 32 channels; 105 with bfloat16) that went to lanes of vector registers and came back one
-// instruction each.  Base shape, 15.4 M points: 1194 -> 1184 us, bfloat16 1160 -> 1100 us.
-// FRESH: read again at each use.  Stage 2 alone has fewer of them, of which 8 to 16 do not fit, and keeps them (two-stage shape, 14.6 M
-// points: 1037 us against 1040 read anew, 2.6 M points of plain attention 214 against 217).
+// The kernel's arguments.  There are more of them, and of the numbers that follow from them, than scalar registers.
 template <typename T> struct CellArgs {
   BinWorkspace ws;
   const T *value, *dist, *score_in, *grad_out, *grad_score_in;
@@ -370,16 +365,33 @@ template <typename T> struct CellArgs {
   FastDiv div_lp;
   int grad16;                 // bit 0 = grad_value is bfloat16, bit 1 = grad_dist is bfloat16 (else float)
 };
+// Where a kernel has them from:
+//   anew     read from the constant segment in every phase; what a lane owns is worked out anew as well (Owner)
+//   pointer  read there where the compiler wants to
+//   value    kept from the start, as parameters
+// What is kept and does not fit goes to lanes of vector registers and comes back one instruction each (both stages, float: 80 to 100 by
+// value, 40 to 66 by pointer, none anew); what is read is waited for, which counts where phases are short because points are sparse.  Tile
+// kernel, us, anew against what is taken: both stages, float, 32 channels, base shape 1133 -> 1113 (by value 1127), the same maps with
+// 6 x 300 queries 429 -> 417, 400 x 400 at 0.1 points a pixel 254 -> 252; 16 channels 1013 -> 1007, 423 -> 408, 232 -> 222.  Stage 2 alone, 400 x 400
+// at 0.1 and 200 x 200 at 4 (coherent): 32 channels 239 -> 227, 213 -> 209, bfloat16 231 -> 219, 198 -> 189; 16 channels 181 -> 167, 160 -> 153; 64
+// channels 436 -> 419, 381 -> 371.  Both stages in bfloat16 lose with either (base shape 1104 -> 1138, 1124); float rows of over 32 channels
+// gain on the base maps what they lose on others (982 -> 965, 400 x 400 446 -> 453).
+enum class ArgsFrom { anew, pointer, value };
+template <typename T, int LPR, bool FUSED> constexpr ArgsFrom args_from() {
+  return !FUSED ? ArgsFrom::value : sizeof(T) == 4 && LPR == 4 ? ArgsFrom::pointer : ArgsFrom::anew;
+}
 #ifdef __HIP_DEVICE_COMPILE__
-template <typename T> using CellArgsPtr = const __attribute__((address_space(4))) CellArgs<T> *;
-template <typename T, bool FRESH> __device__ __forceinline__ CellArgsPtr<T> args() {
-  auto a = (CellArgsPtr<T>)__builtin_amdgcn_kernarg_segment_ptr();
-  if (FRESH) asm volatile("" : "+s"(a));
-  return a;
+template <typename T, ArgsFrom FROM> __device__ __forceinline__ auto args(const CellArgs<T> &param) {
+  if constexpr (FROM == ArgsFrom::value) {
+    return &param;
+  } else {
+    auto a = (const __attribute__((address_space(4))) CellArgs<T> *)__builtin_amdgcn_kernarg_segment_ptr();
+    if (FROM == ArgsFrom::anew) asm volatile("" : "+s"(a));
+    return a;
+  }
 }
 #else
-template <typename T> using CellArgsPtr = const CellArgs<T> *;
-template <typename T, bool FRESH> __device__ CellArgsPtr<T> args();
+template <typename T, ArgsFrom FROM> __device__ const CellArgs<T> *args(const CellArgs<T> &);
 #endif
 
 // FUSED: both stages (depth scores recomputed from dist, grad_dist and the z gradient produced).
@@ -388,7 +400,7 @@ template <typename T, bool FRESH> __device__ CellArgsPtr<T> args();
 // FOURS: the walkers take the points of a cell four at a time (see walks_fours() below).  Both walks in one kernel, chosen pass by
 // pass, do not fit its registers: base shape, bfloat16, 32 channels 580 -> 742 us for half of its cameras, 64 channels 830 -> 1706.
 template <typename T, int VEC, int LPR, bool FUSED, bool FOURS>
-__global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_kernel(CellArgs<T>) {
+__global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_kernel(const CellArgs<T> param) {
   constexpr int PP = cell_pass(LPR), BLOCK = kWalkers + PP, TX = kCellTX, TW = TX + 1, ROW = VEC * LPR;
   constexpr int GPW = kWave / LPR, CELLS = 4 * GPW, ROWS = GPW / TX;      // cells and tile rows per walker wavefront
   extern __shared__ __align__(16) float smem[];
@@ -396,14 +408,16 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
   __shared__ CellFetch s_fetch;                           // the fetching thread's queue state, between its turns
   __shared__ ItemGeom s_geom[kItemSlots];                // items, decoded by the thread that fetches them
 
-  const auto arg = []() { return args<T, FUSED>(); };
+  constexpr ArgsFrom ARGS = args_from<T, LPR, FUSED>();
+  const auto arg = [&]() { return args<T, ARGS>(param); };
   const auto a0 = arg();
   const BinWorkspace ws = a0->ws;
   const BinPlan &p = *ws.plan;
   if (__builtin_expect(p.bins_per_bm == 0, 0)) {
-    backward_without_bins<T, FUSED>(ws, a0->value, a0->dist, a0->score_in, a0->grad_out, a0->grad_score_in, a0->grad_value, a0->grad_dist,
-                                    a0->grad_loc, a0->gl_stride, a0->grad_attn, a0->grad_score_out, a0->grad_wu, a0->Md, a0->Mg,
-                                    a0->B, a0->S, a0->M, a0->C, a0->D, a0->L, a0->Q, a0->P, a0->grad16);
+    const auto a1 = args<T, ArgsFrom::anew>(param);
+    backward_without_bins<T, FUSED>(a1->ws, a1->value, a1->dist, a1->score_in, a1->grad_out, a1->grad_score_in, a1->grad_value, a1->grad_dist,
+                                    a1->grad_loc, a1->gl_stride, a1->grad_attn, a1->grad_score_out, a1->grad_wu, a1->Md, a1->Mg,
+                                    a1->B, a1->S, a1->M, a1->C, a1->D, a1->L, a1->Q, a1->P, a1->grad16);
     return;
   }
   const int TY = p.ty, R = (TY + 1) * TW;
@@ -515,8 +529,8 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
   //   pass); last2, it2: the same of pass t - 2
   if (walker) {
     // =========================== walkers ===========================
-    // What a lane owns, worked out anew in every block that needs it (from a copy of the lane number that the compiler
-    // does not see through): kept from turn to turn it would cost the registers that the value rows and sums need.
+    // What a lane owns.  With ArgsFrom::anew it is worked out anew in every block that needs it (from a copy of the lane number that
+    // the compiler does not see through): kept from turn to turn it would cost the registers that the value rows and sums need.
     struct Owner {
       int lane, cl, group, crow, ccol;                       // lane of the wavefront, of its group; the group's cell
       LaneChannels<T, VEC, LPR> ch;
@@ -529,7 +543,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     };
     auto owner = [&](auto a) {
       unsigned l = lane;
-      asm volatile("" : "+v"(l));
+      if (ARGS == ArgsFrom::anew) asm volatile("" : "+v"(l));
       return Owner(l, wave, a->C);
     };
     auto decode = [&](const int4 &item, const int4 &geo) {
@@ -792,7 +806,7 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         if (tid == 0 && !done) {
           CellFetch fetch = s_fetch;
           int4 rec, geo;
-          const BinWorkspace w = now->ws;
+          const BinWorkspace w = args<T, ArgsFrom::anew>(param)->ws;
           fetch.advance(w, *w.plan, &rec, &geo);
           s_geom[slot_of_item(it + 3)] = decode(rec, geo);
           s_fetch = fetch;
