@@ -91,7 +91,7 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
     const int64_t *__restrict__ level_start, const A *__restrict__ loc, int loc_stride,
     const A *__restrict__ attn, const T *__restrict__ score_in, T *__restrict__ out, T *__restrict__ score_out,
     A *__restrict__ weight_update, const T *__restrict__ packed_arg, int Md, int B, int S, int M, int C, int D, int L,
-    int Q, int P, int upw, int iters, int q_blocks) {
+    int Q, int P, int upw, int iters, int q_blocks, bool once) {
   // packed: the head-shared distribution as dfa3d_pack_dist lays it out (D >= 2), or nullptr
   __shared__ LevelTable tab;
   __shared__ __align__(16) Task<A> s_tasks[kWavesPerBlock][kWave * 4 + kMaxUnitsPerWave * kTaskPad];
@@ -150,15 +150,23 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
           const int l = lp / P;
           const size_t gp = ((size_t)(b * (size_t)Q + q) * M + m) * ws.LP + lp;   // global point index
           const A *pl = loc + gp * loc_stride;
-          // locations, weights and scores pass through once: non-temporal, so that they do not push the value
-          // rows and distributions that the gathers keep coming back to out of the L2
-          const A x = __builtin_nontemporal_load(pl), y = __builtin_nontemporal_load(pl + 1);
-          const A a = __builtin_nontemporal_load(attn + gp);
+          A x, y, z = 0, a;
+          if (once) {                                    // uniform
+            asm volatile("");                                       // (or the compiler merges the branches into plain loads)
+            x = __builtin_nontemporal_load(pl); y = __builtin_nontemporal_load(pl + 1);
+            if (FUSED) z = __builtin_nontemporal_load(pl + 2);
+            a = __builtin_nontemporal_load(attn + gp);
+            asm volatile("");
+          } else {
+            x = pl[0]; y = pl[1];
+            if (FUSED) z = pl[2];
+            a = attn[gp];
+          }
           const Point2D<A> g = locate_2d<A>(x, y, tab.H[l], tab.W[l], tab.start[l]);
           A sc[4];
           if (FUSED) {
             A lo[4], hi[4];
-            const DepthTap<A> tap = locate_depth<A>(__builtin_nontemporal_load(pl + 2), tab.Dd[l]);
+            const DepthTap<A> tap = locate_depth<A>(z, tab.Dd[l]);
             if (packed != nullptr) {                                // uniform: all eight taps from one line
               const int db = min(max(tap.d0, 0), D - 2);
               const bool lo_x = tap.lo_ok && tap.d0 == db, lo_y = tap.lo_ok && tap.d0 == db + 1;
@@ -395,18 +403,24 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   const int q_blocks = (a.Q + q_per_iter * iters - 1) / (q_per_iter * iters);
   const long long blocks = (long long)a.M * a.B * q_blocks;
   if (blocks <= 0 || blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
+  // Locations and weights pass through once.  Non-temporal loads keep them out of the way of the rows and distributions, but a line that
+  // workgroups on several XCDs share (neighbouring heads, where a unit's points are no whole lines) is then fetched from memory
+  // by each.  6 batch elements, four levels from 80 x 128, 8 points (whole lines), non-temporal and plain, us: 610, 618; bfloat16 556, 572; plain
+  // attention, maps from 116 x 185 360, 380; with 2, 3 or 4 points per level 212, 202; 211, 203; 346, 341; one level of 58 x 92, 4 points
+  // 137, 112; three of 58 x 92 226, 208.  Small operands come from the caches either way (37 x 59, 20 MB, whole lines: 48, 43).
+  const bool once = a.L * a.P * sizeof(A) % 128 == 0 && (long long)a.B * a.Q * a.M * a.L * a.P * (a.loc_stride + 1) * (long long)sizeof(A) > (48LL << 20);
   if (a.dist != nullptr) {
     hipLaunchKernelGGL((fwd_attention_kernel<T, A, VEC, LPR, true>), dim3((unsigned)blocks), dim3(kBlock), 0, stream,
                        (const T *)a.value, (const T *)a.dist, a.shapes, a.shape_stride, a.level_start,
                        (const A *)a.loc, a.loc_stride, (const A *)a.attn, (const T *)nullptr, (T *)a.out,
                        (T *)a.score_out, (A *)a.weight_update, (const T *)a.packed_dist, a.dist_heads == 1 ? 1 : a.M, a.B,
-                       a.S, a.M, a.C, a.D, a.L, a.Q, a.P, upw, iters, q_blocks);
+                       a.S, a.M, a.C, a.D, a.L, a.Q, a.P, upw, iters, q_blocks, once);
   } else {
     hipLaunchKernelGGL((fwd_attention_kernel<T, A, VEC, LPR, false>), dim3((unsigned)blocks), dim3(kBlock), 0, stream,
                        (const T *)a.value, (const T *)nullptr, a.shapes, a.shape_stride, a.level_start,
                        (const A *)a.loc, a.loc_stride, (const A *)a.attn, (const T *)a.score_in, (T *)a.out,
                        (T *)nullptr, (A *)nullptr, (const T *)nullptr, a.M, a.B, a.S, a.M, a.C, a.D, a.L, a.Q, a.P, upw, iters,
-                       q_blocks);
+                       q_blocks, once);
   }
   return hipGetLastError();
 }
