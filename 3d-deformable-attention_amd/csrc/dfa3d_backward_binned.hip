@@ -1582,26 +1582,26 @@ static int current_device() {
   return dev;
 }
 
-static int tile_grid(size_t lds, int block) {
+int cu_count() {
   const int dev = current_device();
-  int cus;
-  {
-    std::lock_guard<std::mutex> lock(g_launch_mutex);
-    if (g_cu_count[dev] == 0) {
-      int n = 0;
-      if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-      g_cu_count[dev] = n;
-    }
-    cus = g_cu_count[dev];
+  std::lock_guard<std::mutex> lock(g_launch_mutex);
+  if (g_cu_count[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    g_cu_count[dev] = n;
   }
+  return g_cu_count[dev];
+}
+
+static int tile_grid(size_t lds, int block) {
   const size_t per_cu = lds > 0 ? (160 * 1024) / lds : 8;
   int wg_per_cu = (int)(per_cu < 1 ? 1 : per_cu > 8 ? 8 : per_cu);
   const int by_waves = 32 / (block / kWave);
   if (wg_per_cu > by_waves) wg_per_cu = by_waves < 1 ? 1 : by_waves;
-  return cus * wg_per_cu;
+  return cu_count() * wg_per_cu;
 }
 
-static hipError_t allow_lds(const void *fn, size_t lds) {
+hipError_t allow_lds(const void *fn, size_t lds) {
   if (lds <= 64 * 1024) return hipSuccess;
   const std::pair<const void *, int> key(fn, current_device());
   std::lock_guard<std::mutex> lock(g_launch_mutex);
@@ -1641,7 +1641,6 @@ static hipError_t launch_tile_cfg(const BwdArgs &a, const BinWorkspace &ws, cons
   return hipGetLastError();
 }
 
-static hipError_t allow_lds(const void *fn, size_t lds);
 
 template <typename T>
 static hipError_t launch_tile_typed(const BwdArgs &a, const BinWorkspace &ws, const TileConfig &c, float *gd_heads,

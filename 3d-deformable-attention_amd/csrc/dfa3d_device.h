@@ -190,6 +190,19 @@ template <typename A> struct RowVec<__hip_bfloat16, A, 8> {      // loads only: 
   }
 };
 
+// The same elements of a row that lies in LDS, and the copy that brings them there (BYTES: of VEC elements, a power of two).
+template <typename T, typename A, int VEC> __device__ __forceinline__ void lds_row(const unsigned char *at, A (&v)[VEC]) {
+  struct alignas(VEC * sizeof(T)) Elems { T e[VEC]; };
+  const Elems x = *reinterpret_cast<const Elems *>(at);
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) v[i] = Elem<T>::ld(&x.e[i]);
+}
+template <int BYTES> struct RawPiece;
+template <> struct RawPiece<2> { uint16_t w; __device__ __forceinline__ void ld(rsrc_t r, uint32_t off) { w = __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0); } };
+template <> struct RawPiece<4> { uint32_t w; __device__ __forceinline__ void ld(rsrc_t r, uint32_t off) { w = __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0); } };
+template <> struct RawPiece<8> { u32x2 w; __device__ __forceinline__ void ld(rsrc_t r, uint32_t off) { w = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0); } };
+template <> struct RawPiece<16> { u32x4 w; __device__ __forceinline__ void ld(rsrc_t r, uint32_t off) { w = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0); } };
+
 // Hardware floating-point scatter-add (no compare-and-swap loop) at byte offset `off` of a
 // gradient slice; an out-of-range offset drops the update.
 __device__ __forceinline__ void scatter_add(rsrc_t r, float *, uint32_t off, float v) {

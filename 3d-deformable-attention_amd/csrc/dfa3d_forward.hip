@@ -21,17 +21,19 @@ __host__ __device__ inline FwdShape fwd_shape(int L, int P, int upw) {
   return FwdShape{L * P, upw, upw > 1 ? 1 : (L * P + kWave - 1) / kWave};
 }
 constexpr int kMaxUnitsPerWave = 16;
+constexpr int kLdsRowsBlock = 1024;    // threads of a workgroup that holds its (batch, head)'s value rows in LDS
 constexpr int kTaskPad = 2;            // tasks left free after each unit's, so that the units start on different LDS banks
+constexpr int kTasksPerWave = kWave * 4 + kMaxUnitsPerWave * kTaskPad;
 
 // Phase B of the forward pass: acc += sum of w * row over the tasks first, first + step, ... below n of one unit.  LPR lanes
 // of VEC channels take a row; the wavefront's 64/LPR row slots may work on the same unit (step > 1) or on units of
 // their own.  Eight rows per lane are in flight, whatever the length of the list: a unit of 8 points has 32 tasks, and
 // walking it one row at a time waited for memory once per row.  A batch is summed in two chains and added to acc as a
 // whole, which keeps the longest chain of additions of a unit at about what a tree over the row slots has.
-// `chan_off` is the lane's byte offset inside a row (kNoChan for a lane beyond the last channel).
-template <typename T, typename A, int VEC>
-__device__ __forceinline__ void gather_rows(rsrc_t value_r, const Task<A> *tasks, int first, int step, int n,
-                                            uint32_t chan_off, A (&acc)[VEC]) {
+// `rows` reads this lane's channels of the row at a byte offset; `none` is the offset of a row of zeros.
+template <typename A, int VEC, typename Rows>
+__device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, const Task<A> *tasks, int first, int step, int n,
+                                            A (&acc)[VEC]) {
   constexpr int U = 8, UT = 4;
   int t = 0;                                             // uniform
   for (; t + step * U <= n; t += step * U) {
@@ -40,7 +42,7 @@ __device__ __forceinline__ void gather_rows(rsrc_t value_r, const Task<A> *tasks
     for (int j = 0; j < U; ++j) e[j] = tasks[t + j * step + first];
     A v[U][VEC];
 #pragma unroll
-    for (int j = 0; j < U; ++j) RowVec<T, A, VEC>::ld(value_r, e[j].off + chan_off, v[j]);
+    for (int j = 0; j < U; ++j) rows(e[j].off, v[j]);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       A s0 = e[0].w * v[0][i], s1 = e[1].w * v[1][i];
@@ -54,14 +56,14 @@ __device__ __forceinline__ void gather_rows(rsrc_t value_r, const Task<A> *tasks
     A v[UT][VEC];
 #pragma unroll
     for (int j = 0; j < UT; ++j) {
-      e[j].off = kNoRow; e[j].w = 0;
+      e[j].off = none; e[j].w = 0;
 #pragma unroll
       for (int i = 0; i < VEC; ++i) v[j][i] = 0;
       if (t + j * step < n) {                            // uniform
         const int at = t + j * step + first;
         e[j] = tasks[min(at, n - 1)];
-        if (at >= n) { e[j].off = kNoRow; e[j].w = 0; }
-        RowVec<T, A, VEC>::ld(value_r, e[j].off + chan_off, v[j]);
+        if (at >= n) { e[j].off = none; e[j].w = 0; }
+        rows(e[j].off, v[j]);
       }
     }
 #pragma unroll
@@ -84,9 +86,15 @@ __device__ __forceinline__ void gather_rows(rsrc_t value_r, const Task<A> *tasks
 //   6 x 10000 queries, 4 levels from 116 x 200, points around the query   664 -> 617 us
 //   6 x 4000 queries, one level of 8 points (training step)               261 -> 239 us
 //   2 x 40000 queries, plain attention, 4 points (training step)          461 -> 427 us
+//
+// A CU's L1 answers in the order in which it was asked, and has 256 lines: 256 lines in flight divided by the latency of the farthest
+// is all that it brings, whichever lines the caches hold.  So where a (batch, head)'s value rows fit in LDS (IN_LDS: small
+// maps), a workgroup of 16 wavefronts brings them there once and walks through a share of the queries: four of a point's eight lines
+// less.  6 x 4000 queries, one level of 23 x 40, 8 points: 53.4 -> 41.0 us (uniform), 41.0 -> 36.4 (points around the query), bfloat16
+// 56.6 -> 51.8, one distribution for all heads 49.1 -> 40.3, plain attention 36.3 -> 28.7; 64 channels, 4 x 4000, 15 x 24: 52.2 -> 32.5.
 // ---------------------------------------------------------------------------------------
-template <typename T, typename A, int VEC, int LPR, bool FUSED>
-__global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
+template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS>
+__global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention_kernel(
     const T *__restrict__ value, const T *__restrict__ dist, const int64_t *__restrict__ shapes, int shape_stride,
     const int64_t *__restrict__ level_start, const A *__restrict__ loc, int loc_stride,
     const A *__restrict__ attn, const T *__restrict__ score_in, T *__restrict__ out, T *__restrict__ score_out,
@@ -94,7 +102,9 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
     int Q, int P, int upw, int iters, int q_blocks, bool once) {
   // packed: the head-shared distribution as dfa3d_pack_dist lays it out (D >= 2), or nullptr
   __shared__ LevelTable tab;
-  __shared__ __align__(16) Task<A> s_tasks[kWavesPerBlock][kWave * 4 + kMaxUnitsPerWave * kTaskPad];
+  constexpr int WAVES = (IN_LDS ? kLdsRowsBlock : kBlock) / kWave;
+  __shared__ __align__(16) Task<A> s_tasks[WAVES][kTasksPerWave];
+  extern __shared__ __align__(16) unsigned char s_rows[];    // IN_LDS: all value rows of (b, m), then a row of zeros
 
   load_level_table(tab, shapes, shape_stride, level_start, L, S, FUSED ? D : 0);
   if (FUSED && packed_arg != nullptr) load_cell_starts(tab, L);      // uniform
@@ -122,7 +132,29 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
   const int md = Md == 1 ? 0 : m;                                    // head whose distribution this head reads
   const size_t packed_slice = (FUSED && packed != nullptr) ? (size_t)tab.cell[L] * D * 4 : 0;   // elements per batch element
   const rsrc_t packed_r = make_rsrc(packed_slice ? packed + (size_t)b * packed_slice : nullptr, packed_slice * sizeof(T));
-  const int q_per_iter = kWavesPerBlock * ws.upw;
+  const int q_per_iter = WAVES * ws.upw;
+  if constexpr (IN_LDS) {
+    // LPR lanes per row as in phase B
+    for (int pass = 0; pass < passes; ++pass) {
+      const int chan = (pass * LPR + cl) * VEC;
+      if (chan >= C) break;
+      for (int s0 = wave * RPI + row_slot; s0 <= S; s0 += 4 * WAVES * RPI) {
+        RawPiece<VEC * sizeof(T)> piece[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int s = s0 + j * WAVES * RPI;
+          piece[j].ld(value_r, s < S ? (uint32_t)(((s * M + m) * C + chan) * (int)sizeof(T)) : kNoRow);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int s = s0 + j * WAVES * RPI;
+          if (s <= S) *reinterpret_cast<decltype(piece[j].w) *>(s_rows + (s * C + chan) * (int)sizeof(T)) = piece[j].w;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  const uint32_t none = IN_LDS ? (uint32_t)(S * C * (int)sizeof(T)) : kNoRow;      // a row of zeros
 
   for (int it = 0; it < iters; ++it) {
     const int q0 = (qb * iters + it) * q_per_iter + wave * ws.upw;   // first query of this wave's group
@@ -131,7 +163,11 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
     for (int pass = 0; pass < passes; ++pass) {
       const int chan = (pass * LPR + cl) * VEC;
       const bool chan_ok = chan < C;
-      const uint32_t chan_off = chan_ok ? (uint32_t)(chan * sizeof(T)) : kNoChan;
+      const uint32_t chan_off = chan_ok ? (uint32_t)(chan * sizeof(T)) : IN_LDS ? 0u : kNoChan;
+      auto rows = [&](uint32_t off, A (&v)[VEC]) {
+        if constexpr (IN_LDS) lds_row<T, A, VEC>(s_rows + off + chan_off, v);
+        else RowVec<T, A, VEC>::ld(value_r, off + chan_off, v);
+      };
       A acc[VEC];
 #pragma unroll
       for (int v = 0; v < VEC; ++v) acc[v] = 0;
@@ -145,13 +181,13 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
         Task<A> t4[4];
         A wu = 0;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) { t4[k].off = kNoRow; t4[k].w = 0; }
+        for (int k = 0; k < 4; ++k) { t4[k].off = none; t4[k].w = 0; }
         if (live) {
           const int l = lp / P;
           const size_t gp = ((size_t)(b * (size_t)Q + q) * M + m) * ws.LP + lp;   // global point index
           const A *pl = loc + gp * loc_stride;
           A x, y, z = 0, a;
-          if (once) {                                    // uniform
+          if (!IN_LDS && once) {                                    // uniform
             asm volatile("");                                       // (or the compiler merges the branches into plain loads)
             x = __builtin_nontemporal_load(pl); y = __builtin_nontemporal_load(pl + 1);
             if (FUSED) z = __builtin_nontemporal_load(pl + 2);
@@ -204,7 +240,7 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
             if (g.key[k] >= 0) {
-              t4[k].off = (uint32_t)((g.key[k] * M + m) * C * (int)sizeof(T));
+              t4[k].off = (uint32_t)((IN_LDS ? g.key[k] : g.key[k] * M + m) * C * (int)sizeof(T));
               t4[k].w = g.bil(k) * sc[k] * a;
             }
           }
@@ -235,7 +271,7 @@ __global__ __launch_bounds__(kBlock) void fwd_attention_kernel(
         for (int u0 = 0; u0 < ws.upw; u0 += par) {              // one round, or three (one where a unit takes several chunks)
           const int u = u0 + row_slot / spu;
           const int n = (ws.upw == 1 ? min(kWave, ws.LP - chunk * kWave) : ws.LP) * 4;
-          gather_rows<T, A, VEC>(value_r, tasks + u * (ws.upw == 1 ? 0 : unit_tasks), row_slot % spu, spu, n, chan_off, acc);
+          gather_rows<A, VEC>(rows, none, tasks + u * (ws.upw == 1 ? 0 : unit_tasks), row_slot % spu, spu, n, acc);
           if (chunk == ws.chunks - 1) {
             for (int off = LPR; off < spu * LPR; off <<= 1) {
 #pragma unroll
@@ -387,6 +423,20 @@ hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int6
 // ---------------------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------------------
+// Workgroups per (batch, head) that hold its value rows in LDS; 0: rows are gathered from memory.  Taken where all rows fit beside
+// the task lists and a workgroup has at least as many points as it brings rows: kernel, us, memory and LDS, 920 rows of 32 channels, points
+// per workgroup 500: 8.6, 11.0   640: 11.6, 12.9   800: 11.9, 12.9   1000: 13.3, 12.6   1600: 19.6, 17.2   6400: 53.4, 41.0; 504 rows, 720 points:
+// 10.7, 10.1; 384 rows, 800 points: 10.9, 10.6.  Rows of whole groups of four channels, up to 64, of 4- or 2-byte elements.
+template <typename T, int VEC, int LPR> constexpr bool kLdsRowsTiling = sizeof(T) <= 4 && VEC == 4 && LPR <= 16;
+static size_t lds_rows_bytes(const FwdArgs &a, size_t elem) { return ((size_t)a.S + 1) * a.C * elem; }
+template <typename T, typename A> static int lds_rows_parts(const FwdArgs &a) {
+  constexpr size_t kStatic = (kLdsRowsBlock / kWave) * sizeof(Task<A>) * kTasksPerWave + sizeof(LevelTable) + 64;
+  if (a.iters > 1 || lds_rows_bytes(a, sizeof(T)) + kStatic > 160 * 1024) return 0;
+  const long long pairs = (long long)a.M * a.B, cus = cu_count(), parts = cus / pairs;      // one workgroup per CU
+  if (4 * pairs * parts < 3 * cus) return 0;                 // too many CUs would be idle
+  return (long long)a.Q * a.L * a.P >= parts * a.S ? (int)parts : 0;
+}
+
 template <typename T, typename A, int VEC, int LPR>
 static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   // Units per wavefront: as many as its 64 lanes have points for.  A call with few units is spread over more wavefronts
@@ -398,31 +448,37 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   if (upw > 1 && upw < kMaxUnitsPerWave && upw / 2 * 3 * a.L * a.P <= kWave) upw = upw / 2 * 3;    // 20 points: 60 lanes, not 40
   while (upw > 1 && (long long)a.M * a.B * ((a.Q + upw - 1) / upw) < kFewWaves) upw /= 2;
   const FwdShape ws = fwd_shape(a.L, a.P, upw);
-  const int q_per_iter = kWavesPerBlock * ws.upw;
-  const int iters = a.iters > 0 ? a.iters : 1;
-  const int q_blocks = (a.Q + q_per_iter * iters - 1) / (q_per_iter * iters);
+  const int parts = kLdsRowsTiling<T, VEC, LPR> ? lds_rows_parts<T, A>(a) : 0;
+  const int q_per_iter = (parts > 0 ? kLdsRowsBlock / kWave : kWavesPerBlock) * ws.upw, groups = (a.Q + q_per_iter - 1) / q_per_iter;
+  const int iters = parts > 0 ? (groups + parts - 1) / parts : a.iters > 0 ? a.iters : 1;
+  const int q_blocks = (groups + iters - 1) / iters;
   const long long blocks = (long long)a.M * a.B * q_blocks;
   if (blocks <= 0 || blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
+  const bool fused = a.dist != nullptr;
   // Locations and weights pass through once.  Non-temporal loads keep them out of the way of the rows and distributions, but a line that
   // workgroups on several XCDs share (neighbouring heads, where a unit's points are no whole lines) is then fetched from memory
   // by each.  6 batch elements, four levels from 80 x 128, 8 points (whole lines), non-temporal and plain, us: 610, 618; bfloat16 556, 572; plain
   // attention, maps from 116 x 185 360, 380; with 2, 3 or 4 points per level 212, 202; 211, 203; 346, 341; one level of 58 x 92, 4 points
   // 137, 112; three of 58 x 92 226, 208.  Small operands come from the caches either way (37 x 59, 20 MB, whole lines: 48, 43).
   const bool once = a.L * a.P * sizeof(A) % 128 == 0 && (long long)a.B * a.Q * a.M * a.L * a.P * (a.loc_stride + 1) * (long long)sizeof(A) > (48LL << 20);
-  if (a.dist != nullptr) {
-    hipLaunchKernelGGL((fwd_attention_kernel<T, A, VEC, LPR, true>), dim3((unsigned)blocks), dim3(kBlock), 0, stream,
-                       (const T *)a.value, (const T *)a.dist, a.shapes, a.shape_stride, a.level_start,
-                       (const A *)a.loc, a.loc_stride, (const A *)a.attn, (const T *)nullptr, (T *)a.out,
-                       (T *)a.score_out, (A *)a.weight_update, (const T *)a.packed_dist, a.dist_heads == 1 ? 1 : a.M, a.B,
-                       a.S, a.M, a.C, a.D, a.L, a.Q, a.P, upw, iters, q_blocks, once);
-  } else {
-    hipLaunchKernelGGL((fwd_attention_kernel<T, A, VEC, LPR, false>), dim3((unsigned)blocks), dim3(kBlock), 0, stream,
-                       (const T *)a.value, (const T *)nullptr, a.shapes, a.shape_stride, a.level_start,
-                       (const A *)a.loc, a.loc_stride, (const A *)a.attn, (const T *)a.score_in, (T *)a.out,
-                       (T *)nullptr, (A *)nullptr, (const T *)nullptr, a.M, a.B, a.S, a.M, a.C, a.D, a.L, a.Q, a.P, upw, iters,
-                       q_blocks, once);
+  auto launch = [&](auto kernel, int threads, size_t bytes) -> hipError_t {
+    if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), bytes)) return e;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), bytes, stream, (const T *)a.value, (const T *)a.dist, a.shapes,
+                       a.shape_stride, a.level_start, (const A *)a.loc, a.loc_stride, (const A *)a.attn,
+                       fused ? nullptr : (const T *)a.score_in, (T *)a.out, fused ? (T *)a.score_out : nullptr,
+                       fused ? (A *)a.weight_update : nullptr, fused ? (const T *)a.packed_dist : nullptr,
+                       fused && a.dist_heads == 1 ? 1 : a.M, a.B, a.S, a.M, a.C, fused ? a.D : 0, a.L, a.Q, a.P, upw, iters, q_blocks, once);
+    return hipGetLastError();
+  };
+  if constexpr (kLdsRowsTiling<T, VEC, LPR>) {
+    if (parts > 0) {
+      const size_t bytes = lds_rows_bytes(a, sizeof(T));
+      return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, true>, kLdsRowsBlock, bytes)
+                   : launch(fwd_attention_kernel<T, A, VEC, LPR, false, true>, kLdsRowsBlock, bytes);
+    }
   }
-  return hipGetLastError();
+  return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false>, kBlock, 0)
+               : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false>, kBlock, 0);
 }
 
 template <typename T, typename A>

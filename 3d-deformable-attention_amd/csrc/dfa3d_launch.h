@@ -110,6 +110,10 @@ struct DepthScoreBwdArgs {
   int clear;                         // grad_dist holds anything on entry (binned kernels; the caller clears for the direct ones)
 };
 
+// Looked up once per device and remembered: the number of CUs; the grant of more than 64 KB of dynamic LDS to a kernel.
+int cu_count();
+hipError_t allow_lds(const void *kernel, size_t bytes);
+
 hipError_t launch_forward(const FwdArgs &a, int dtype, hipStream_t stream);
 hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int64_t *level_start, void *packed, int B,
                             int S, int D, int L, int dtype, hipStream_t stream);
