@@ -92,6 +92,11 @@ __device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, con
 // maps), a workgroup of 16 wavefronts brings them there once and walks through a share of the queries: four of a point's eight lines
 // less.  6 x 4000 queries, one level of 23 x 40, 8 points: 53.4 -> 41.0 us (uniform), 41.0 -> 36.4 (points around the query), bfloat16
 // 56.6 -> 51.8, one distribution for all heads 49.1 -> 40.3, plain attention 36.3 -> 28.7; 64 channels, 4 x 4000, 15 x 24: 52.2 -> 32.5.
+// On larger maps the coarser levels' rows: 6 x 10000 queries, four levels from 116 x 200, 8 points (one level in LDS): 915 -> 864 us,
+// points around the query 605 -> 571; bfloat16 (two levels) 842 -> 787, 572 -> 505; plain attention 297 -> 261.  Groups are taken, not dealt:
+// dealt, a workgroup's slowest wavefront held up the CU (883, 614).  Tried with it and not kept: two workgroups of 8, 10 or 12 wavefronts per CU
+// (908, 870, 1031; 596, 625, 706), 16 gathers in flight (880, 623), the next group's locations asked for ahead (850, 581; bfloat16 951) or
+// brought to the L2 by scalar loads (874, 587); the same workgroups without rows in LDS: 942, 603.
 // ---------------------------------------------------------------------------------------
 template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS>
 __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention_kernel(
@@ -99,12 +104,13 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
     const int64_t *__restrict__ level_start, const A *__restrict__ loc, int loc_stride,
     const A *__restrict__ attn, const T *__restrict__ score_in, T *__restrict__ out, T *__restrict__ score_out,
     A *__restrict__ weight_update, const T *__restrict__ packed_arg, int Md, int B, int S, int M, int C, int D, int L,
-    int Q, int P, int upw, int iters, int q_blocks, bool once) {
+    int Q, int P, int upw, int iters, int q_blocks, bool once, int lds_rows) {
   // packed: the head-shared distribution as dfa3d_pack_dist lays it out (D >= 2), or nullptr
   __shared__ LevelTable tab;
   constexpr int WAVES = (IN_LDS ? kLdsRowsBlock : kBlock) / kWave;
   __shared__ __align__(16) Task<A> s_tasks[WAVES][kTasksPerWave];
-  extern __shared__ __align__(16) unsigned char s_rows[];    // IN_LDS: all value rows of (b, m), then a row of zeros
+  __shared__ int s_next;                                      // IN_LDS: the workgroup's next group of units
+  extern __shared__ __align__(16) unsigned char s_rows[];    // IN_LDS: value rows [key0, S) of (b, m), then a row of zeros
 
   load_level_table(tab, shapes, shape_stride, level_start, L, S, FUSED ? D : 0);
   if (FUSED && packed_arg != nullptr) load_cell_starts(tab, L);      // uniform
@@ -133,41 +139,58 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
   const size_t packed_slice = (FUSED && packed != nullptr) ? (size_t)tab.cell[L] * D * 4 : 0;   // elements per batch element
   const rsrc_t packed_r = make_rsrc(packed_slice ? packed + (size_t)b * packed_slice : nullptr, packed_slice * sizeof(T));
   const int q_per_iter = WAVES * ws.upw;
+  // IN_LDS: levels l0, l0 + 1, ... , whose keys are among the last lds_rows ones
+  int l0 = IN_LDS ? L : 0, key0 = S;
   if constexpr (IN_LDS) {
+    if (threadIdx.x == 0) s_next = 0;
+    while (l0 > 0 && tab.start[l0 - 1] >= S - lds_rows) { --l0; key0 = min(key0, tab.start[l0]); }
+    const int n_rows = S - key0;
     // LPR lanes per row as in phase B
     for (int pass = 0; pass < passes; ++pass) {
       const int chan = (pass * LPR + cl) * VEC;
       if (chan >= C) break;
-      for (int s0 = wave * RPI + row_slot; s0 <= S; s0 += 4 * WAVES * RPI) {
+      for (int s0 = wave * RPI + row_slot; s0 <= n_rows; s0 += 4 * WAVES * RPI) {
         RawPiece<VEC * sizeof(T)> piece[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int s = s0 + j * WAVES * RPI;
-          piece[j].ld(value_r, s < S ? (uint32_t)(((s * M + m) * C + chan) * (int)sizeof(T)) : kNoRow);
+          piece[j].ld(value_r, s < n_rows ? (uint32_t)((((key0 + s) * M + m) * C + chan) * (int)sizeof(T)) : kNoRow);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int s = s0 + j * WAVES * RPI;
-          if (s <= S) *reinterpret_cast<decltype(piece[j].w) *>(s_rows + (s * C + chan) * (int)sizeof(T)) = piece[j].w;
+          if (s <= n_rows) *reinterpret_cast<decltype(piece[j].w) *>(s_rows + (s * C + chan) * (int)sizeof(T)) = piece[j].w;
         }
       }
     }
     __syncthreads();
   }
-  const uint32_t none = IN_LDS ? (uint32_t)(S * C * (int)sizeof(T)) : kNoRow;      // a row of zeros
+  const uint32_t zero_row = (uint32_t)((S - key0) * C * (int)sizeof(T));
 
-  for (int it = 0; it < iters; ++it) {
-    const int q0 = (qb * iters + it) * q_per_iter + wave * ws.upw;   // first query of this wave's group
-    if (q0 >= Q) break;                                              // wave-uniform
+  // Groups of units, WAVES to a round; rounds are dealt to the workgroups of a (batch, head) in turn, so that what they gather at a
+  // time lies together.  IN_LDS: a workgroup's wavefronts take its next group each.
+  for (int it = 0; IN_LDS || it < iters; ++it) {
+    int round = qb * iters + it, slot = wave;
+    if constexpr (IN_LDS) {
+      int n = 0;
+      if (lane == 0) n = atomicAdd(&s_next, 1);
+      n = __builtin_amdgcn_readfirstlane(n);
+      if (n >= iters * WAVES) break;
+      round = n / WAVES * q_blocks + qb;
+      slot = n % WAVES;
+    }
+    const int q0 = round * q_per_iter + slot * ws.upw;               // first query of this wave's group
+    if (q0 >= Q) {                                                   // wave-uniform
+      if (IN_LDS) continue;
+      break;
+    }
     A wu_unit = 0;                                                   // upw == 1: the unit's sum over its chunks
     for (int pass = 0; pass < passes; ++pass) {
       const int chan = (pass * LPR + cl) * VEC;
       const bool chan_ok = chan < C;
-      const uint32_t chan_off = chan_ok ? (uint32_t)(chan * sizeof(T)) : IN_LDS ? 0u : kNoChan;
-      auto rows = [&](uint32_t off, A (&v)[VEC]) {
-        if constexpr (IN_LDS) lds_row<T, A, VEC>(s_rows + off + chan_off, v);
-        else RowVec<T, A, VEC>::ld(value_r, off + chan_off, v);
-      };
+      const uint32_t chan_off = chan_ok ? (uint32_t)(chan * sizeof(T)) : kNoChan, lds_chan = chan_ok ? chan_off : 0u;
+      auto rows = [&](uint32_t off, A (&v)[VEC]) { RowVec<T, A, VEC>::ld(value_r, off + chan_off, v); };
+      auto rows_in_lds = [&](uint32_t off, A (&v)[VEC]) { lds_row<T, A, VEC>(s_rows + off + lds_chan, v); };
       A acc[VEC];
 #pragma unroll
       for (int v = 0; v < VEC; ++v) acc[v] = 0;
@@ -180,6 +203,8 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
         const bool live = ul < ws.upw && q < Q;
         Task<A> t4[4];
         A wu = 0;
+        const bool from_lds = IN_LDS && lp >= l0 * P;
+        const uint32_t none = from_lds ? zero_row : kNoRow;
 #pragma unroll
         for (int k = 0; k < 4; ++k) { t4[k].off = none; t4[k].w = 0; }
         if (live) {
@@ -240,7 +265,7 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
             if (g.key[k] >= 0) {
-              t4[k].off = (uint32_t)((IN_LDS ? g.key[k] : g.key[k] * M + m) * C * (int)sizeof(T));
+              t4[k].off = (uint32_t)((from_lds ? g.key[k] - key0 : g.key[k] * M + m) * C * (int)sizeof(T));
               t4[k].w = g.bil(k) * sc[k] * a;
             }
           }
@@ -271,7 +296,10 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
         for (int u0 = 0; u0 < ws.upw; u0 += par) {              // one round, or three (one where a unit takes several chunks)
           const int u = u0 + row_slot / spu;
           const int n = (ws.upw == 1 ? min(kWave, ws.LP - chunk * kWave) : ws.LP) * 4;
-          gather_rows<A, VEC>(rows, none, tasks + u * (ws.upw == 1 ? 0 : unit_tasks), row_slot % spu, spu, n, acc);
+          const Task<A> *mine = tasks + u * (ws.upw == 1 ? 0 : unit_tasks);
+          const int far = IN_LDS ? min(max((l0 * P - chunk * kWave) * 4, 0), n) : n;
+          gather_rows<A, VEC>(rows, kNoRow, mine, row_slot % spu, spu, far, acc);
+          if constexpr (IN_LDS) gather_rows<A, VEC>(rows_in_lds, zero_row, mine + far, row_slot % spu, spu, n - far, acc);
           if (chunk == ws.chunks - 1) {
             for (int off = LPR; off < spu * LPR; off <<= 1) {
 #pragma unroll
@@ -423,18 +451,38 @@ hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int6
 // ---------------------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------------------
-// Workgroups per (batch, head) that hold its value rows in LDS; 0: rows are gathered from memory.  Taken where all rows fit beside
-// the task lists and a workgroup has at least as many points as it brings rows: kernel, us, memory and LDS, 920 rows of 32 channels, points
-// per workgroup 500: 8.6, 11.0   640: 11.6, 12.9   800: 11.9, 12.9   1000: 13.3, 12.6   1600: 19.6, 17.2   6400: 53.4, 41.0; 504 rows, 720 points:
-// 10.7, 10.1; 384 rows, 800 points: 10.9, 10.6.  Rows of whole groups of four channels, up to 64, of 4- or 2-byte elements.
+// Whether value rows are brought to LDS: those of the last `rows` keys as far as they are whole levels, by `parts` workgroups per (batch, head),
+// one per CU; parts = 0: all rows are gathered from memory.  For rows of whole groups of four channels, up to 64, of 4- or 2-byte elements.
+//   * The whole map fits: the workgroups of all (batch, head) run at once, where each has at least as many points as it brings
+//     rows.  Kernel, us, memory and LDS, 920 rows of 32 channels, points per workgroup 500: 8.6, 11.0   640: 11.6, 12.9   800: 11.9, 12.9
+//     1000: 13.3, 12.6   1600: 19.6, 17.2   6400: 53.4, 41.0; 504 rows, 720 points: 10.7, 10.1; 384 rows, 800 points: 10.9, 10.6.
+//   * The coarser levels of a pyramid fit (the level sizes are on the device; each is taken for a quarter of the one before): one
+//     (batch, head) at a time on an XCD, as its L2 holds no more, so M has to divide 8 or be a multiple of it.  A workgroup's start
+//     and end cost as much as about a thousand points, LDS saves half of a point's lines (plain attention all, packed
+//     distributions 4 of 5): from 2000 points on levels in LDS, so far as one can tell.  Memory and LDS, points per workgroup x share of the levels:
+//     10000 x 1/4: 914, 864   8000 x 1/2: 610, 535   4000 x 1/2: 240, 226; plain 171, 154; 120, 114   3500 x 1/4: 349, 370   3500 x 1/2: plain 52, 54
+//     2000 x 1/2: 106, 109; plain 73, 77   1000 x 3/4: 76, 89.
 template <typename T, int VEC, int LPR> constexpr bool kLdsRowsTiling = sizeof(T) <= 4 && VEC == 4 && LPR <= 16;
-static size_t lds_rows_bytes(const FwdArgs &a, size_t elem) { return ((size_t)a.S + 1) * a.C * elem; }
-template <typename T, typename A> static int lds_rows_parts(const FwdArgs &a) {
+struct LdsRows { int parts, rows; };
+template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a) {
   constexpr size_t kStatic = (kLdsRowsBlock / kWave) * sizeof(Task<A>) * kTasksPerWave + sizeof(LevelTable) + 64;
-  if (a.iters > 1 || lds_rows_bytes(a, sizeof(T)) + kStatic > 160 * 1024) return 0;
-  const long long pairs = (long long)a.M * a.B, cus = cu_count(), parts = cus / pairs;      // one workgroup per CU
-  if (4 * pairs * parts < 3 * cus) return 0;                 // too many CUs would be idle
-  return (long long)a.Q * a.L * a.P >= parts * a.S ? (int)parts : 0;
+  const LdsRows none{0, 0};
+  const long long room = (long long)((160 * 1024 - kStatic) / (a.C * sizeof(T))) - 1, points = (long long)a.Q * a.L * a.P;
+  if (a.iters > 1 || room < 1) return none;
+  const long long cus = cu_count(), pairs = (long long)a.M * a.B;
+  if (room >= a.S) {
+    const long long parts = cus / pairs;
+    if (4 * pairs * parts < 3 * cus || points < parts * a.S) return none;      // idle CUs; too few points
+    return LdsRows{(int)parts, a.S};
+  }
+  const long long parts = cus / a.M;
+  if (parts < 1 || (8 % a.M != 0 && a.M % 8 != 0)) return none;
+  long long all = 1, some = 1;                              // pixels of the pyramid, and of its coarsest levels, in the coarsest one's
+  int in_lds = 0;
+  for (int l = 1; l < a.L; ++l) all = 4 * all + 1;          // (at most 16 levels)
+  for (; in_lds + 1 < a.L && 1.1 * a.S * some <= (double)room * all; ++in_lds) some = 4 * some + 1;
+  if (points * in_lds < parts * 2000 * a.L) return none;
+  return LdsRows{(int)parts, (int)room};
 }
 
 template <typename T, typename A, int VEC, int LPR>
@@ -448,7 +496,8 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   if (upw > 1 && upw < kMaxUnitsPerWave && upw / 2 * 3 * a.L * a.P <= kWave) upw = upw / 2 * 3;    // 20 points: 60 lanes, not 40
   while (upw > 1 && (long long)a.M * a.B * ((a.Q + upw - 1) / upw) < kFewWaves) upw /= 2;
   const FwdShape ws = fwd_shape(a.L, a.P, upw);
-  const int parts = kLdsRowsTiling<T, VEC, LPR> ? lds_rows_parts<T, A>(a) : 0;
+  const LdsRows lds = kLdsRowsTiling<T, VEC, LPR> ? lds_rows_plan<T, A>(a) : LdsRows{0, 0};
+  const int parts = lds.parts;
   const int q_per_iter = (parts > 0 ? kLdsRowsBlock / kWave : kWavesPerBlock) * ws.upw, groups = (a.Q + q_per_iter - 1) / q_per_iter;
   const int iters = parts > 0 ? (groups + parts - 1) / parts : a.iters > 0 ? a.iters : 1;
   const int q_blocks = (groups + iters - 1) / iters;
@@ -467,12 +516,12 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
                        a.shape_stride, a.level_start, (const A *)a.loc, a.loc_stride, (const A *)a.attn,
                        fused ? nullptr : (const T *)a.score_in, (T *)a.out, fused ? (T *)a.score_out : nullptr,
                        fused ? (A *)a.weight_update : nullptr, fused ? (const T *)a.packed_dist : nullptr,
-                       fused && a.dist_heads == 1 ? 1 : a.M, a.B, a.S, a.M, a.C, fused ? a.D : 0, a.L, a.Q, a.P, upw, iters, q_blocks, once);
+                       fused && a.dist_heads == 1 ? 1 : a.M, a.B, a.S, a.M, a.C, fused ? a.D : 0, a.L, a.Q, a.P, upw, iters, q_blocks, once, lds.rows);
     return hipGetLastError();
   };
   if constexpr (kLdsRowsTiling<T, VEC, LPR>) {
     if (parts > 0) {
-      const size_t bytes = lds_rows_bytes(a, sizeof(T));
+      const size_t bytes = ((size_t)lds.rows + 1) * a.C * sizeof(T);
       return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, true>, kLdsRowsBlock, bytes)
                    : launch(fwd_attention_kernel<T, A, VEC, LPR, false, true>, kLdsRowsBlock, bytes);
     }

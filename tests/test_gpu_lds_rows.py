@@ -1,7 +1,7 @@
-"""Forward with the value rows of a (batch, head) in LDS (small maps with many points): row lengths on both sides of every lane
+"""Forward with value rows in LDS, of all of a small map or of a pyramid's coarser levels: row lengths on both sides of every lane
 group, points per unit from one to more than a wavefront holds, a last share of the queries that is not full, and maps on both sides
-of what LDS holds.  Walking several groups per wavefront on request (iters = 2) keeps the gathers from memory, which form the same sums
-in the same order."""
+of what LDS holds.  Walking several groups per wavefront on request (iters = 2) keeps the gathers from memory, which for a whole map form
+the same sums in the same order."""
 import pytest
 import torch
 
@@ -65,3 +65,40 @@ def test_largest_maps_and_other_calls(levels, C, dtype):
     for a, b in zip(got, want):
         torch.testing.assert_close(a, b, rtol=0, atol=0, equal_nan=True)
     assert 0 < got[0].isnan().any(-1).sum() < got[0].shape[1]
+
+
+@pytest.mark.parametrize("levels,M,C,P,dtype", [
+    (((40, 50), (20, 25), (10, 13)), 8, 32, 4, torch.float32),       # two of three levels fit
+    (((40, 50), (20, 25), (10, 13)), 4, 20, 5, torch.float32),
+    (((56, 60), (28, 30), (14, 15), (7, 8)), 8, 32, 3, torch.bfloat16),
+    (((56, 60), (28, 30), (14, 15), (7, 8)), 2, 64, 17, torch.float32),        # two rounds of 64 points per unit
+    (((30, 40), (15, 20), (8, 10)), 8, 32, 4, torch.float32),       # (the finest level just does not fit)
+    (((20, 25), (40, 50), (10, 13)), 8, 32, 4, torch.float32),      # no pyramid: the last level alone fits
+    (((13, 13), (20, 25), (40, 50)), 8, 32, 4, torch.float32),      # coarse to fine: none does
+], ids=str)
+def test_coarser_levels(levels, M, C, P, dtype):
+    from dfa3D import _ext, _lib
+    L, S = len(levels), sum(h * w for h, w in levels)
+    Q = 256 // M * 2200 // P + 29                             # enough points for one workgroup per CU
+    t = _as_inputs(tiny_case(seed=S + P, B=1, M=M, C=C, D=5, Q=Q, P=P, levels=levels))
+    value, dist, sh, lsi, loc, attn = _on(_dev(), t, dtype)
+    value[0, S - 2, 1] = float("nan")
+    sh[0, 1] += 10 ** 6 if L == 4 and M == 2 else 0          # a level that is no level of this map
+    one = dist[:, :, :1].contiguous()
+    packed = _ext.pack_shared_dist(one, sh, lsi)
+
+    def all_calls():
+        out = list(_ext.dfa3d_fused_forward(value, dist, sh, lsi, loc, attn, 64, need_depth_score=True))
+        out += _ext.dfa3d_fused_forward(value, one, sh, lsi, loc, attn, 64, need_depth_score=False, need_weight_update=True, packed_dist=packed)
+        out.append(_ext.ms_deform_attn_forward(value, sh[:, :2].contiguous(), lsi, loc[..., :2].contiguous(), attn, 64))
+        return [o for o in out if o is not None]
+    got = all_calls()
+    with _lib.launch_options(iters=2):
+        want = all_calls()
+    # the same products, added up in another order: at most 8 additions in one chain and a few above it, each rounded to 2^-24 of at
+    # most the sum of the sizes (|value| < 5, weights of a unit sum to at most 1); bfloat16: one rounding of the result
+    tol = dict(rtol=1e-6, atol=4e-6) if dtype == torch.float32 else dict(rtol=2 ** -7, atol=1e-5)
+    assert len(got) == len(want) >= 4
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, equal_nan=True, **tol)
+    assert got[0].isnan().any()
