@@ -3,19 +3,22 @@
     python 3d-deformable-attention_amd/build.py [--force] [--clocks]
 
 The library lands next to the python package (dfa3D/libdfa3d_hip.so) so that it travels with
-the source tree.  Two more libraries land beside bench.py, which is what uses them: the yardstick kernels
+the source tree, as does the module that calls it with torch's tensors (dfa3D/_binding.so, host code).  Two more libraries land beside bench.py, which is what uses them: the yardstick kernels
 (libdfa3d_measure.so) and, with --clocks, libdfa3d_hip_clocks.so: the same sources compiled with
 -DDFA3D_TILE_TIMING, i.e. with the per-phase clocks of the backward's tile kernels (`bench.py --phase-costs`).
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "dfa3D", "libdfa3d_hip.so")
+BINDING_SRC = os.path.join(CSRC, "dfa3d_binding.cpp")
+BINDING = os.path.join(HERE, "dfa3D", "_binding.so")
 # yardstick kernels for bench.py (plain copy, bare gathers, LDS atomics, XCD map): not part of the operator library
 MEASURE_SRC = os.path.join(CSRC, "measure", "dfa3d_measure.hip")
 ROOT = os.path.dirname(HERE)
@@ -65,9 +68,24 @@ def _build_lib(lib, obj_dir, extra_flags, force, verbose):
     return lib
 
 
+def _build_binding(force, verbose):
+    if not (force or _stale(BINDING, [BINDING_SRC, os.path.join(ROOT, "include", "dfa3d.h"), os.path.abspath(__file__)])):
+        return
+    import torch
+    from torch.utils import cpp_extension
+    includes = [f"-isystem{d}" for d in cpp_extension.include_paths()]
+    libs = [f"-L{d}" for d in cpp_extension.library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10"]
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I" + sysconfig.get_paths()["include"], *includes,
+          BINDING_SRC, "-o", BINDING, *libs], verbose)
+
+
 def build(force=False, verbose=True, clocks=False):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    _build_lib(LIB, OBJ, [], force, verbose)
+    with ThreadPoolExecutor(max_workers=1) as ex:
+        binding = ex.submit(_build_binding, force, verbose)
+        _build_lib(LIB, OBJ, [], force, verbose)
+        binding.result()
     if force or _stale(MEASURE_LIB, [MEASURE_SRC, os.path.join(CSRC, "measure", "dfa3d_measure.h")]):
         _run([hipcc, *FLAGS, "-shared", MEASURE_SRC, "-o", MEASURE_LIB], verbose)
     if clocks:

@@ -24,7 +24,19 @@ __all__ = [
     "wms_deform_attn_forward", "wms_deform_attn_backward",
     "ms_depth_score_sample_forward", "ms_depth_score_sample_backward",
     "dfa3d_fused_forward", "dfa3d_fused_backward", "fused_backward_grad_dtype", "pack_shared_dist",
+    "dfa3d_fused_gradients", "attention_gradients", "depth_score_gradients",
 ]
+
+
+def _here(value):
+    """(binding module, current GPU, its current stream) for the short way of a call, or None where it does not lead:
+    launch options are in force, or the operand is not on a GPU.  It declines (None) whatever else is not as its kernels
+    read it, and the long way says what that is.  2 x 100 queries on 16 x 16 maps, forward: 17.3 -> 11.4 us; 2 x 400 queries in
+    float64, training: 158 -> 112."""
+    if _lib.options() is not None or not value.is_cuda:
+        return None
+    at = torch._C._cuda_getDevice()
+    return _lib.binding(), at, torch._C._cuda_getCurrentRawStream(at)
 
 
 def _contig(**tensors):
@@ -96,6 +108,13 @@ def _geometry(shapes, lsi, loc, width, name):
 def ms_depth_score_sample_forward(value, value_spatial_shapes, value_level_start_index,
                                   sampling_locations, im2col_step):
     """value = depth distributions (bs, num_keys, num_heads, D) -> (bs, Q, heads, L, P, 4)."""
+    here = _here(value)
+    if here is not None:
+        native, at, stream = here
+        score = native.score_forward(at, stream, value, value_spatial_shapes, value_level_start_index, sampling_locations,
+                                     im2col_step)
+        if score is not None:
+            return score
     dev = _contig_on_gpu(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
                          sampling_loc=sampling_locations)
     if value.dim() != 4:
@@ -158,6 +177,22 @@ def ms_depth_score_sample_backward_into(value, value_spatial_shapes, value_level
     _lib.check(rc, "dfa3d_ms_depth_score_sample_backward")
 
 
+def depth_score_gradients(value, value_spatial_shapes, value_level_start_index, sampling_locations, grad_output, im2col_step):
+    """Backward of stage 1 into tensors of its own -> gradients of value and sampling_locations, in their types."""
+    here = _here(value)
+    if here is not None:
+        native, at, stream = here
+        got = native.score_gradients(at, stream, value, value_spatial_shapes, value_level_start_index, sampling_locations,
+                                     grad_output, im2col_step)
+        if got is not None:
+            return got
+    grad_value = torch.empty(value.shape, dtype=_aux_dtype(value.dtype), device=value.device)      # cleared by the call (clear=True)
+    grad_sampling_loc = torch.empty_like(sampling_locations)
+    ms_depth_score_sample_backward_into(value, value_spatial_shapes, value_level_start_index, sampling_locations, grad_output,
+                                        grad_value, grad_sampling_loc, im2col_step=im2col_step, clear=True)
+    return grad_value.to(value.dtype), grad_sampling_loc
+
+
 def _wms_dims(value, shapes, lsi, loc, attn, score, name):
     if value.dim() != 4:
         raise RuntimeError(f"value must be (bs, num_keys, num_heads, channels), got {tuple(value.shape)}")
@@ -182,6 +217,13 @@ def _wms_dims(value, shapes, lsi, loc, attn, score, name):
 def wms_deform_attn_forward(value, value_spatial_shapes, value_level_start_index, sampling_locations,
                             attention_weights, depth_scores, im2col_step):
     """Depth-weighted multi-scale deformable attention -> (bs, num_queries, heads*channels)."""
+    here = _here(value)
+    if here is not None and depth_scores is not None:
+        native, at, stream = here
+        out = native.attention_forward(at, stream, value, value_spatial_shapes, value_level_start_index, sampling_locations,
+                                       attention_weights, depth_scores, im2col_step)
+        if out is not None:
+            return out
     dev = _contig_on_gpu(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
                          sampling_loc=sampling_locations, attn_weight=attention_weights, depth_score=depth_scores)
     B, S, M, C, L, Q, P, sw, lw = _wms_dims(value, value_spatial_shapes, value_level_start_index, sampling_locations,
@@ -257,6 +299,13 @@ def ms_deform_attn_forward(value, value_spatial_shapes, value_level_start_index,
     self-attention and decoder load from mmcv's extension
     (BEVFormer_DFA3D/projects/mmdet3d_plugin/bevformer/modules/multi_scale_deformable_attn_function.py:10-12,:47-53).
     Runs the stage-2 kernel without a score tensor."""
+    here = _here(value)
+    if here is not None:
+        native, at, stream = here
+        out = native.attention_forward(at, stream, value, value_spatial_shapes, value_level_start_index, sampling_locations,
+                                       attention_weights, None, im2col_step)
+        if out is not None:
+            return out
     named = dict(value=value, spatial_shapes=value_spatial_shapes, level_start_index=value_level_start_index,
                  sampling_loc=sampling_locations, attn_weight=attention_weights)
     dev = _contig_on_gpu(**named)
@@ -342,6 +391,12 @@ def pack_shared_dist(value_dpt_dist, value_spatial_shapes, value_level_start_ind
     around every base pixel side by side, per bin): pass the result as ``packed_dist`` to ``dfa3d_fused_forward``.
     Returns None where the library does not offer it (D < 2, float64).  Worth keeping: every forward on the same
     distribution (DFA3D-BEVFormer runs six encoder layers on one) can use the same packed tensor."""
+    here = _here(value_dpt_dist)
+    if here is not None:
+        native, at, stream = here
+        packed = native.pack_dist(at, stream, value_dpt_dist, value_spatial_shapes, value_level_start_index)
+        if packed is not None:
+            return packed
     dev = _contig_on_gpu(value_dpt_dist=value_dpt_dist, spatial_shapes=value_spatial_shapes,
                          level_start_index=value_level_start_index)
     if value_dpt_dist.dim() != 4 or value_dpt_dist.shape[2] != 1:
@@ -370,6 +425,14 @@ def dfa3d_fused_forward(value, value_dpt_dist, value_spatial_shapes, value_level
     with ``need_weight_update`` a third result, weight_update (bs, Q, heads, 1) = sum over levels and points of
     attention weight * mean corner score.  ``value_dpt_dist`` is (bs, keys, heads, D), or (bs, keys, 1, D) for one
     distribution shared by all heads; for the latter ``packed_dist`` may be what ``pack_shared_dist`` returned for it."""
+    here = _here(value)
+    if here is not None:
+        native, at, stream = here
+        got = native.fused_forward(at, stream, value, value_dpt_dist, value_spatial_shapes, value_level_start_index,
+                                   sampling_locations, attention_weights, im2col_step, bool(need_depth_score),
+                                   bool(need_weight_update), packed_dist)
+        if got is not None:
+            return got if need_weight_update else got[:2]
     dev = _contig_on_gpu(value=value, value_dpt_dist=value_dpt_dist, spatial_shapes=value_spatial_shapes,
                          level_start_index=value_level_start_index, sampling_loc=sampling_locations,
                          attn_weight=attention_weights)
@@ -470,3 +533,55 @@ def dfa3d_fused_backward(value, value_dpt_dist, value_spatial_shapes, value_leve
                 _lib.ptr(workspace), ws_bytes, B, S, M, C, D, L, Q, P, value_dpt_dist.shape[2], code,
                 _lib.options(), _lib.stream_of(value))
     _lib.check(rc, "dfa3d_fused_backward")
+
+
+def dfa3d_fused_gradients(value, value_dpt_dist, value_spatial_shapes, value_level_start_index, sampling_locations,
+                          attention_weights, grad_output, grad_depth_score, im2col_step, grad_weight_update=None):
+    """``dfa3d_fused_backward`` into tensors of its own -> gradients of value, value_dpt_dist, sampling_locations and
+    attention_weights, in their types."""
+    here = _here(value)
+    if here is not None:
+        native, at, stream = here
+        got = native.fused_gradients(at, stream, value, value_dpt_dist, value_spatial_shapes, value_level_start_index,
+                                     sampling_locations, attention_weights, grad_output, grad_depth_score, grad_weight_update,
+                                     im2col_step)
+        if got is not None:
+            return got
+    gdt = fused_backward_grad_dtype(value, value_dpt_dist, sampling_locations)
+    # not zeroed here: the call clears the part of the two buffers that its kernels add to (clear=True)
+    grad_value = torch.empty(value.shape, dtype=gdt, device=value.device)
+    grad_value_dpt_dist = torch.empty(value_dpt_dist.shape, dtype=gdt, device=value.device)
+    grad_sampling_loc = torch.empty_like(sampling_locations)
+    grad_attn_weight = torch.empty_like(attention_weights)
+    dfa3d_fused_backward(value, value_dpt_dist, value_spatial_shapes, value_level_start_index, sampling_locations,
+                         attention_weights, grad_output, grad_depth_score, grad_value, grad_value_dpt_dist, grad_sampling_loc,
+                         grad_attn_weight, im2col_step=im2col_step, grad_weight_update=grad_weight_update, clear=True)
+    return grad_value.to(value.dtype), grad_value_dpt_dist.to(value_dpt_dist.dtype), grad_sampling_loc, grad_attn_weight
+
+
+def attention_gradients(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
+                        depth_scores, grad_output, im2col_step):
+    """Backward of stage 2, or of plain attention where ``depth_scores`` is None, into tensors of its own -> gradients of
+    value, sampling_locations, attention_weights and depth_scores (None without them), in their types."""
+    here = _here(value)
+    if here is not None:
+        native, at, stream = here
+        got = native.attention_gradients(at, stream, value, value_spatial_shapes, value_level_start_index, sampling_locations,
+                                         attention_weights, depth_scores, grad_output, im2col_step)
+        if got is not None:
+            return got
+    aux = _aux_dtype(value.dtype)
+    grad_value = torch.empty(value.shape, dtype=aux, device=value.device)      # cleared by the call (clear=True)
+    grad_sampling_loc = torch.empty_like(sampling_locations)
+    if sampling_locations.shape[-1] > 2:
+        grad_sampling_loc[..., 2:] = 0
+    grad_attn_weight = torch.empty_like(attention_weights)
+    if depth_scores is None:
+        ms_deform_attn_backward(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
+                                grad_output, grad_value, grad_sampling_loc, grad_attn_weight, im2col_step=im2col_step, clear=True)
+        return grad_value.to(value.dtype), grad_sampling_loc, grad_attn_weight, None
+    grad_depth_score = torch.empty(depth_scores.shape, dtype=aux, device=value.device)
+    wms_deform_attn_backward_into(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
+                                  depth_scores, grad_output, grad_value, grad_sampling_loc, grad_attn_weight, grad_depth_score,
+                                  im2col_step=im2col_step, clear=True)
+    return grad_value.to(value.dtype), grad_sampling_loc, grad_attn_weight, grad_depth_score.to(depth_scores.dtype)

@@ -54,12 +54,26 @@ SIGNATURES = {
     "dfa3d_abi_version": [],
 }
 
+# entry points that the binding module (csrc/dfa3d_binding.cpp) calls by address
+_BOUND = ("dfa3d_last_error", "dfa3d_packed_dist_bytes", "dfa3d_fused_forward", "dfa3d_fused_backward_workspace_bytes",
+          "dfa3d_fused_backward", "dfa3d_wms_deform_attn_forward", "dfa3d_wms_deform_attn_backward_workspace_bytes",
+          "dfa3d_wms_deform_attn_backward", "dfa3d_ms_depth_score_sample_forward",
+          "dfa3d_ms_depth_score_sample_backward_workspace_bytes", "dfa3d_ms_depth_score_sample_backward_into", "dfa3d_pack_dist")
+
 _lib = None
+_binding = None
+
+
+def binding():
+    """The binding module, on the library that ``lib()`` loaded."""
+    if _lib is None:
+        lib()
+    return _binding
 
 
 def lib():
     """Loads the shared library once; raises if it has not been built."""
-    global _lib
+    global _lib, _binding
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise ImportError(
@@ -86,7 +100,13 @@ def lib():
         handle.dfa3d_last_error.restype = ctypes.c_char_p
         if handle.dfa3d_abi_version() != ABI_VERSION:
             raise ImportError(f"{LIB_PATH}: ABI version {handle.dfa3d_abi_version()} != expected {ABI_VERSION}; rebuild")
-        _lib = handle
+        try:
+            from . import _binding as module
+        except ImportError as e:
+            raise ImportError(f"{_HERE}/_binding.so is missing or does not fit this torch: build it with "
+                              f"`python 3d-deformable-attention_amd/build.py` ({e})") from e
+        module.bind({name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in _BOUND})
+        _lib, _binding = handle, module
     return _lib
 
 

@@ -69,7 +69,10 @@ def _with_forward_options(backward):
     would reach the forward kernels only."""
     @functools.wraps(backward)
     def wrapped(ctx, *grads):
-        with _lib.restored_options(getattr(ctx, "launch_fields", {})):
+        fields = getattr(ctx, "launch_fields", {})
+        if not fields and not _lib.current_fields():           # none then, none now
+            return backward(ctx, *grads)
+        with _lib.restored_options(fields):
             return backward(ctx, *grads)
     return wrapped
 
@@ -98,12 +101,10 @@ class MultiScaleDepthScoreSampleFunction(Function):
     @_with_forward_options
     def backward(ctx, grad_output):
         value, value_spatial_shapes, value_level_start_index, sampling_locations = ctx.saved_tensors
-        grad_value = torch.empty(value.shape, dtype=_aux(value), device=value.device)      # cleared by the call (clear=True)
-        grad_sampling_loc = torch.empty_like(sampling_locations)
-        _ext.ms_depth_score_sample_backward_into(
-            value, value_spatial_shapes, value_level_start_index, sampling_locations,
-            _grad_in(grad_output, value.dtype), grad_value, grad_sampling_loc, im2col_step=ctx.im2col_step, clear=True)
-        return grad_value.to(value.dtype), None, None, grad_sampling_loc, None
+        grad_value, grad_sampling_loc = _ext.depth_score_gradients(
+            value, value_spatial_shapes, value_level_start_index, sampling_locations, _grad_in(grad_output, value.dtype),
+            ctx.im2col_step)
+        return grad_value, None, None, grad_sampling_loc, None
 
 
 class WeightedMultiScaleDeformableAttnFunction(Function):
@@ -127,19 +128,10 @@ class WeightedMultiScaleDeformableAttnFunction(Function):
     def backward(ctx, grad_output):
         value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights, \
             depth_score = ctx.saved_tensors
-        aux = _aux(value)
-        grad_value = torch.empty(value.shape, dtype=aux, device=value.device)      # cleared by the call (clear=True)
-        grad_sampling_loc = torch.empty_like(sampling_locations)
-        if sampling_locations.shape[-1] > 2:
-            grad_sampling_loc[..., 2:] = 0
-        grad_attn_weight = torch.empty_like(attention_weights)
-        grad_depth_score = torch.empty(depth_score.shape, dtype=aux, device=value.device)
-        _ext.wms_deform_attn_backward_into(
-            value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
-            depth_score, _grad_in(grad_output, value.dtype), grad_value, grad_sampling_loc, grad_attn_weight,
-            grad_depth_score, im2col_step=ctx.im2col_step, clear=True)
-        return grad_value.to(value.dtype), None, None, grad_sampling_loc, grad_attn_weight, \
-            grad_depth_score.to(depth_score.dtype), None
+        grad_value, grad_sampling_loc, grad_attn_weight, grad_depth_score = _ext.attention_gradients(
+            value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights, depth_score,
+            _grad_in(grad_output, value.dtype), ctx.im2col_step)
+        return grad_value, None, None, grad_sampling_loc, grad_attn_weight, grad_depth_score, None
 
 
 class MultiScaleDeformableAttnFunction(Function):
@@ -164,16 +156,10 @@ class MultiScaleDeformableAttnFunction(Function):
     def backward(ctx, grad_output):
         value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights = \
             ctx.saved_tensors
-        grad_value = torch.empty(value.shape, dtype=_aux(value), device=value.device)   # cleared by the call
-        grad_sampling_loc = torch.empty_like(sampling_locations)
-        if sampling_locations.shape[-1] > 2:
-            grad_sampling_loc[..., 2:] = 0
-        grad_attn_weight = torch.empty_like(attention_weights)
-        _ext.ms_deform_attn_backward(
-            value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
-            _grad_in(grad_output, value.dtype), grad_value, grad_sampling_loc, grad_attn_weight,
-            im2col_step=ctx.im2col_step, clear=True)
-        return grad_value.to(value.dtype), None, None, grad_sampling_loc, grad_attn_weight, None
+        grad_value, grad_sampling_loc, grad_attn_weight, _ = _ext.attention_gradients(
+            value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights, None,
+            _grad_in(grad_output, value.dtype), ctx.im2col_step)
+        return grad_value, None, None, grad_sampling_loc, grad_attn_weight, None
 
 
 class MultiScale3DDeformableAttnFunction(Function):
@@ -203,20 +189,11 @@ class MultiScale3DDeformableAttnFunction(Function):
         if grad_output is None:
             grad_output = torch.zeros(value.shape[0], sampling_locations.shape[1], value.shape[2] * value.shape[3],
                                       dtype=value.dtype, device=value.device)
-        gdt = _ext.fused_backward_grad_dtype(value, value_dpt_dist, sampling_locations)
-        # not zeroed here: the call clears the part of the two buffers that its kernels add to (clear=True)
-        grad_value = torch.empty(value.shape, dtype=gdt, device=value.device)
-        grad_value_dpt_dist = torch.empty(value_dpt_dist.shape, dtype=gdt, device=value.device)
-        grad_sampling_loc = torch.empty_like(sampling_locations)
-        grad_attn_weight = torch.empty_like(attention_weights)
-        _ext.dfa3d_fused_backward(
-            value, value_dpt_dist, value_spatial_shapes, value_level_start_index, sampling_locations,
-            attention_weights, _grad_in(grad_output, value.dtype),
-            None if grad_depth_score is None else _grad_in(grad_depth_score, value.dtype),
-            grad_value, grad_value_dpt_dist, grad_sampling_loc, grad_attn_weight, im2col_step=ctx.im2col_step,
-            clear=True)
-        return grad_value.to(value.dtype), grad_value_dpt_dist.to(value_dpt_dist.dtype), None, None, \
-            grad_sampling_loc, grad_attn_weight, None
+        grad_value, grad_value_dpt_dist, grad_sampling_loc, grad_attn_weight = _ext.dfa3d_fused_gradients(
+            value, value_dpt_dist, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
+            _grad_in(grad_output, value.dtype), None if grad_depth_score is None else _grad_in(grad_depth_score, value.dtype),
+            ctx.im2col_step)
+        return grad_value, grad_value_dpt_dist, None, None, grad_sampling_loc, grad_attn_weight, None
 
 
 class MultiScale3DDeformableAttnWeightUpdateFunction(Function):
@@ -258,20 +235,12 @@ class MultiScale3DDeformableAttnWeightUpdateFunction(Function):
         if grad_output is None:
             grad_output = torch.zeros(value.shape[0], sampling_locations.shape[1], value.shape[2] * value.shape[3],
                                       dtype=value.dtype, device=value.device)
-        gdt = _ext.fused_backward_grad_dtype(value, value_dpt_dist, sampling_locations)
-        grad_value = torch.empty(value.shape, dtype=gdt, device=value.device)
-        grad_value_dpt_dist = torch.empty(value_dpt_dist.shape, dtype=gdt, device=value.device)
-        grad_sampling_loc = torch.empty_like(sampling_locations)
-        grad_attn_weight = torch.empty_like(attention_weights)
-        _ext.dfa3d_fused_backward(
-            value, value_dpt_dist, value_spatial_shapes, value_level_start_index, sampling_locations,
-            attention_weights, _grad_in(grad_output, value.dtype), None,
-            grad_value, grad_value_dpt_dist, grad_sampling_loc, grad_attn_weight, im2col_step=ctx.im2col_step,
-            grad_weight_update=None if grad_weight_update is None else _grad_in(grad_weight_update, aux),
-            clear=True)
+        grad_value, grad_value_dpt_dist, grad_sampling_loc, grad_attn_weight = _ext.dfa3d_fused_gradients(
+            value, value_dpt_dist, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
+            _grad_in(grad_output, value.dtype), None, ctx.im2col_step,
+            grad_weight_update=None if grad_weight_update is None else _grad_in(grad_weight_update, aux))
         # one gradient per forward argument: seven, or eight when the packed distribution was passed in
-        return (grad_value.to(value.dtype), grad_value_dpt_dist.to(value_dpt_dist.dtype), None, None,
-                grad_sampling_loc, grad_attn_weight, None, None)
+        return grad_value, grad_value_dpt_dist, None, None, grad_sampling_loc, grad_attn_weight, None, None
 
 
 def _autocast_twin(base, name, doc):
