@@ -458,10 +458,11 @@ hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int6
 //     1000: 13.3, 12.6   1600: 19.6, 17.2   6400: 53.4, 41.0; 504 rows, 720 points: 10.7, 10.1; 384 rows, 800 points: 10.9, 10.6.
 //   * The coarser levels of a pyramid fit (the level sizes are on the device; each is taken for a quarter of the one before): one
 //     (batch, head) at a time on an XCD, as its L2 holds no more, so M has to divide 8 or be a multiple of it.  A workgroup's start
-//     and end cost as much as about a thousand points, LDS saves half of a point's lines (plain attention all, packed
-//     distributions 4 of 5): from 2000 points on levels in LDS, so far as one can tell.  Memory and LDS, points per workgroup x share of the levels:
+//     and end cost as much as about a thousand points, LDS saves half of a point's lines (plain attention all): from 2000 points on levels in
+//     LDS, so far as one can tell.  Memory and LDS, points per workgroup x share of the levels:
 //     10000 x 1/4: 914, 864   8000 x 1/2: 610, 535   4000 x 1/2: 240, 226; plain 171, 154; 120, 114   3500 x 1/4: 349, 370   3500 x 1/2: plain 52, 54
-//     2000 x 1/2: 106, 109; plain 73, 77   1000 x 3/4: 76, 89.
+//     2000 x 1/2: 106, 109; plain 73, 77   1000 x 3/4: 76, 89.  Not with packed distributions, which a cross-attention layer uses: its
+//     points share a pillar's few pixels, whose rows the L1 has (200 x 200 queries, base maps 412, 432; 120 x 120, 30 x 48 226, 239).
 template <typename T, int VEC, int LPR> constexpr bool kLdsRowsTiling = sizeof(T) <= 4 && VEC == 4 && LPR <= 16;
 struct LdsRows { int parts, rows; };
 template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a) {
@@ -476,7 +477,7 @@ template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a)
     return LdsRows{(int)parts, a.S};
   }
   const long long parts = cus / a.M;
-  if (parts < 1 || (8 % a.M != 0 && a.M % 8 != 0)) return none;
+  if (parts < 1 || (8 % a.M != 0 && a.M % 8 != 0) || a.packed_dist != nullptr) return none;
   long long all = 1, some = 1;                              // pixels of the pyramid, and of its coarsest levels, in the coarsest one's
   int in_lds = 0;
   for (int l = 1; l < a.L; ++l) all = 4 * all + 1;          // (at most 16 levels)
