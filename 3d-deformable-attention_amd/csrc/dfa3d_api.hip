@@ -303,9 +303,8 @@ static dfa3d::BwdArgs fused_bwd_args(const void *value, const void *dist, const 
 static int direct_fused_backward(const char *fn, const dfa3d::BwdArgs &a, int dtype, int dist_heads, hipStream_t stream) {
   if (a.clear_grads) {
     const size_t elem = dtype == DFA3D_F64 ? 8 : 4;
-    if (hipError_t e = dfa3d::launch_zero_fill(a.grad_value, (size_t)a.B * a.S * a.M * a.C * elem, stream))
-      return hip_result(e, fn);
-    if (hipError_t e = dfa3d::launch_zero_fill(a.grad_dist, (size_t)a.B * a.S * dist_heads * a.D * elem, stream))
+    if (hipError_t e = dfa3d::launch_zero_fill(a.grad_value, (size_t)a.B * a.S * a.M * a.C * elem, a.grad_dist,
+                                               (size_t)a.B * a.S * dist_heads * a.D * elem, stream))
       return hip_result(e, fn);
   }
   return hip_result(dfa3d::launch_backward(a, dtype, stream), fn);

@@ -54,6 +54,24 @@ template <int LPR> __device__ __forceinline__ double row_sum(double x) {
   return x;
 }
 
+// the value of the lane next to this one in its pair (lanes 2 i and 2 i + 1); every lane of the wavefront takes part
+__device__ __forceinline__ uint32_t pair_swap(uint32_t x) { return __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, true); }      // quad_perm [1,0,3,2]
+__device__ __forceinline__ float pair_swap(float x) { return __uint_as_float(pair_swap(__float_as_uint(x))); }
+__device__ __forceinline__ double pair_swap(double x) {
+  return __hiloint2double((int)pair_swap((uint32_t)__double2hiint(x)), (int)pair_swap((uint32_t)__double2loint(x)));
+}
+// Adds lo at byte offset off_lo and hi at off_hi, the next element (kNoRow: nothing), for every lane.  The memory side retires (instruction,
+// 64-byte piece) pairs, so a pair of lanes sends both elements of one of them, side by side, then both of the other: half of the pieces.
+// 2 x 400 queries, double, 32 bins: 57 -> 52 us, 15.36 M points with 64 bins 12.2 -> 10.5 ms.
+template <typename A>
+__device__ __forceinline__ void scatter_add_two(rsrc_t r, A *base, uint32_t off_lo, A lo, uint32_t off_hi, A hi) {
+  const bool odd = (threadIdx.x & 1) != 0;
+  const uint32_t off = pair_swap(odd ? off_lo : off_hi);
+  const A x = pair_swap(odd ? lo : hi);
+  scatter_add(r, base, odd ? off : off_lo, odd ? x : lo);
+  scatter_add(r, base, odd ? off_hi : off, odd ? hi : x);
+}
+
 // Phase B of the backward pass over tasks [t_begin, t_end): per task the dot product of the value
 // row with grad_out (left in dots[t]) and the scatter-add of w * grad_out into grad_value.
 //   chan_off   lane's byte offset inside a value row (kNoChan beyond the last channel)
@@ -125,14 +143,15 @@ __global__ __launch_bounds__(kBlock) void bwd_attention_kernel(
     const T *__restrict__ grad_score_in, A *__restrict__ grad_value, A *__restrict__ grad_dist,
     A *__restrict__ grad_loc, int gl_stride, A *__restrict__ grad_attn, A *__restrict__ grad_score_out,
     const A *__restrict__ grad_wu, int Md,
-    int B, int S, int M, int C, int D, int L, int Q, int P, int iters, int q_blocks) {
+    int B, int S, int M, int C, int D, int L, int Q, int P, int upw, int iters, int q_blocks) {
   __shared__ LevelTable tab;
   __shared__ Task<A> s_tasks[kWavesPerBlock][kWave * 4];
   __shared__ A s_dots[kWavesPerBlock][kWave * 4];
 
   load_level_table(tab, shapes, shape_stride, level_start, L, S, FUSED ? D : 0);
 
-  const WaveShape ws = wave_shape(L, P);
+  WaveShape ws = wave_shape(L, P);
+  ws.upw = min(ws.upw, upw);
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int m = blockIdx.x % M;
   const int rest = blockIdx.x / M;
@@ -225,6 +244,8 @@ __global__ __launch_bounds__(kBlock) void bwd_attention_kernel(
       wave_lds_handover();
 
       // ---------------- phase C: one lane per point again ----------------
+      uint32_t tap_off[4] = {kNoRow, kNoRow, kNoRow, kNoRow};      // (FUSED) of the corners' lower bins
+      A tap_add[4] = {0, 0, 0, 0};                                 // what they are to collect, before the weights along depth
       if (live) {
         A dot[4];
 #pragma unroll
@@ -264,9 +285,8 @@ __global__ __launch_bounds__(kBlock) void bwd_attention_kernel(
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
             const bool on = g.key[k] >= 0 && gs[k] != 0;
-            const uint32_t row = (uint32_t)(((g.key[k] * Md + md) * D + tap.d0) * (int)sizeof(A));
-            scatter_add(gdist_r, gdist_b, (on && tap.lo_ok) ? row : kNoRow, tap.hd * gs[k]);
-            scatter_add(gdist_r, gdist_b, (on && tap.hi_ok) ? row + (uint32_t)sizeof(A) : kNoRow, tap.ld * gs[k]);
+            if (on) tap_off[k] = (uint32_t)(((g.key[k] * Md + md) * D + tap.d0) * (int)sizeof(A));
+            tap_add[k] = gs[k];
             gz += (g.key[k] >= 0 && tap.inside) ? gs[k] * (hi[k] - lo[k]) : (A)0;
           }
           gl[2] = gz * (A)tab.Dd[l];
@@ -275,6 +295,12 @@ __global__ __launch_bounds__(kBlock) void bwd_attention_kernel(
 #pragma unroll
           for (int k = 0; k < 4; ++k) go4[k] = gs[k];
         }
+      }
+      if (FUSED) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          scatter_add_two(gdist_r, gdist_b, tap.lo_ok ? tap_off[k] : kNoRow, tap.hd * tap_add[k],
+                          (tap.hi_ok && tap_off[k] != kNoRow) ? tap_off[k] + (uint32_t)sizeof(A) : kNoRow, tap.ld * tap_add[k]);
       }
     }
   }
@@ -301,7 +327,9 @@ __global__ __launch_bounds__(kBlock) void depth_score_bwd_kernel(
   const rsrc_t dist_r = make_rsrc(dist + (size_t)b * S * M * D, (size_t)S * M * D * sizeof(T));
   A *gdist_b = grad_dist + (size_t)b * S * M * D;
   const rsrc_t gdist_r = make_rsrc(gdist_b, (size_t)S * M * D * sizeof(A));
-  for (int i = threadIdx.x; i < nq * LP; i += kBlock) {
+  for (int i0 = 0; i0 < nq * LP; i0 += kBlock) {                  // uniform: all lanes take part in scatter_add_two
+    const bool live = i0 + (int)threadIdx.x < nq * LP;
+    const int i = live ? i0 + (int)threadIdx.x : 0;
     const int ql = i / LP, lp = i - ql * LP;
     const size_t gp = (((size_t)b * Q + q0 + ql) * M + m) * LP + lp;
     const int l = lp / P;
@@ -314,18 +342,20 @@ __global__ __launch_bounds__(kBlock) void depth_score_bwd_kernel(
     A gz = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const bool on = g.key[k] >= 0 && tap.inside;
+      const bool on = live && g.key[k] >= 0 && tap.inside;
       const A gk = Elem<T>::ld(gi + k);
       const uint32_t row = (uint32_t)(((g.key[k] * M + m) * D + tap.d0) * (int)sizeof(A));
-      scatter_add(gdist_r, gdist_b, (on && tap.lo_ok) ? row : kNoRow, tap.hd * gk);
-      scatter_add(gdist_r, gdist_b, (on && tap.hi_ok) ? row + (uint32_t)sizeof(A) : kNoRow, tap.ld * gk);
+      scatter_add_two(gdist_r, gdist_b, (on && tap.lo_ok) ? row : kNoRow, tap.hd * gk,
+                      (on && tap.hi_ok) ? row + (uint32_t)sizeof(A) : kNoRow, tap.ld * gk);
       gz += on ? gk * (hi[k] - lo[k]) : (A)0;
     }
     gz *= (A)tab.Dd[l];
-    A *gl = grad_loc3 + gp * 3;
-    gl[0] = 0;
-    gl[1] = 0;
-    gl[2] = gz;
+    if (live) {
+      A *gl = grad_loc3 + gp * 3;
+      gl[0] = 0;
+      gl[1] = 0;
+      gl[2] = gz;
+    }
   }
 }
 
@@ -334,7 +364,11 @@ __global__ __launch_bounds__(kBlock) void depth_score_bwd_kernel(
 // ---------------------------------------------------------------------------------------
 template <typename T, typename A, int VEC, int LPR>
 static hipError_t launch_bwd_cfg(const BwdArgs &a, hipStream_t stream) {
-  const WaveShape ws = wave_shape(a.L, a.P);
+  // A call with few units is spread over more wavefronts, down to one unit each, whose chains of loads, dots and updates are its
+  // time: 2 x 400 queries of 8 points, double, 52 -> 43 us, with 20 channels 94 -> 50 (from 4096 wavefronts on 44 and 47).
+  constexpr long long kFewWaves = 2048;
+  WaveShape ws = wave_shape(a.L, a.P);
+  while (ws.upw > 1 && (long long)a.M * a.B * ((a.Q + ws.upw - 1) / ws.upw) < kFewWaves) ws.upw /= 2;
   const int q_per_iter = kWavesPerBlock * ws.upw;
   const int iters = a.iters > 0 ? a.iters : 1;
   const int q_blocks = (a.Q + q_per_iter * iters - 1) / (q_per_iter * iters);
@@ -347,14 +381,14 @@ static hipError_t launch_bwd_cfg(const BwdArgs &a, hipStream_t stream) {
                        (const T *)a.grad_out, (const T *)a.grad_score_in, (A *)a.grad_value, (A *)a.grad_dist,
                        (A *)a.grad_loc, a.grad_loc_stride, (A *)a.grad_attn, (A *)nullptr,
                        (const A *)a.grad_weight_update, a.dist_heads == 1 ? 1 : a.M, a.B, a.S, a.M, a.C, a.D,
-                       a.L, a.Q, a.P, iters, q_blocks);
+                       a.L, a.Q, a.P, ws.upw, iters, q_blocks);
   } else {
     hipLaunchKernelGGL((bwd_attention_kernel<T, A, VEC, LPR, false>), dim3((unsigned)blocks), dim3(kBlock), 0, stream,
                        (const T *)a.value, (const T *)nullptr, a.shapes, a.shape_stride, a.level_start,
                        (const A *)a.loc, a.loc_stride, (const A *)a.attn, (const T *)a.score_in,
                        (const T *)a.grad_out, (const T *)nullptr, (A *)a.grad_value, (A *)nullptr, (A *)a.grad_loc,
                        a.grad_loc_stride, (A *)a.grad_attn, (A *)a.grad_score_out, (const A *)nullptr, a.M, a.B, a.S,
-                       a.M, a.C, a.D, a.L, a.Q, a.P, iters, q_blocks);
+                       a.M, a.C, a.D, a.L, a.Q, a.P, ws.upw, iters, q_blocks);
   }
   return hipGetLastError();
 }

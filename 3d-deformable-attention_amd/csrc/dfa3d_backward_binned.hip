@@ -1349,9 +1349,10 @@ constexpr int kMinChunk = 64;        // smallest accepted points-per-item
 // only the fused entry point sets dist_heads
 static bool shared_dist(const BwdArgs &a) { return a.dist_heads == 1 && a.M > 1; }
 
-__global__ __launch_bounds__(256) void fill_zero_kernel(float4 *__restrict__ dst, size_t n4) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256)
-    dst[i] = make_float4(0, 0, 0, 0);
+// Up to two buffers: the direct kernels' two gradients of a small call took as long to clear as two empty launches.
+__global__ __launch_bounds__(256) void fill_zero_kernel(float4 *__restrict__ dst, size_t n4, float4 *__restrict__ other, size_t other4) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4 + other4; i += (size_t)gridDim.x * 256)
+    (i < n4 ? dst[i] : other[i - n4]) = make_float4(0, 0, 0, 0);
 }
 __global__ __launch_bounds__(64) void fill_zero_words_kernel(uint32_t *__restrict__ dst, size_t n) {
   for (size_t i = threadIdx.x; i < n; i += 64) dst[i] = 0;
@@ -1363,9 +1364,18 @@ hipError_t launch_zero_fill(void *dst, size_t bytes, hipStream_t stream) {
   const size_t head = ((uintptr_t)p & 15) ? 16 - ((uintptr_t)p & 15) : 0;        // bytes before the first 16-byte boundary
   const size_t lead = head < bytes ? head : bytes, body = (bytes - lead) & ~(size_t)15, tail = bytes - lead - body;
   if (lead) hipLaunchKernelGGL(fill_zero_words_kernel, dim3(1), dim3(64), 0, stream, reinterpret_cast<uint32_t *>(p), lead / 4);
-  if (body) hipLaunchKernelGGL(fill_zero_kernel, dim3(2048), dim3(256), 0, stream, reinterpret_cast<float4 *>(p + lead), body / 16);
+  if (body) hipLaunchKernelGGL(fill_zero_kernel, dim3(2048), dim3(256), 0, stream, reinterpret_cast<float4 *>(p + lead), body / 16, (float4 *)nullptr, (size_t)0);
   if (tail) hipLaunchKernelGGL(fill_zero_words_kernel, dim3(1), dim3(64), 0, stream, reinterpret_cast<uint32_t *>(p + lead + body), tail / 4);
   return hipGetLastError();
+}
+
+hipError_t launch_zero_fill(void *dst, size_t bytes, void *other, size_t other_bytes, hipStream_t stream) {
+  if (((uintptr_t)dst & 15) == 0 && ((uintptr_t)other & 15) == 0 && (bytes & 15) == 0 && (other_bytes & 15) == 0 && dst != nullptr && other != nullptr) {
+    hipLaunchKernelGGL(fill_zero_kernel, dim3(2048), dim3(256), 0, stream, static_cast<float4 *>(dst), bytes / 16, static_cast<float4 *>(other), other_bytes / 16);
+    return hipGetLastError();
+  }
+  if (hipError_t e = launch_zero_fill(dst, bytes, stream)) return e;
+  return launch_zero_fill(other, other_bytes, stream);
 }
 
 // dst[r, :] = sum over heads m of src[r, m, :], rows of D floats, heads in order; dst is float, or bfloat16

@@ -129,6 +129,7 @@ hipError_t launch_backward_binned(const BwdArgs &a, int dtype, void *workspace, 
                                   hipStream_t stream);
 // Zero fill by a kernel (no memset node: callers may capture the stream in a graph); bytes a multiple of 4.
 hipError_t launch_zero_fill(void *dst, size_t bytes, hipStream_t stream);
+hipError_t launch_zero_fill(void *dst, size_t bytes, void *other, size_t other_bytes, hipStream_t stream);      // both
 size_t binned_depth_score_backward_workspace_bytes(const DepthScoreBwdArgs &d, int dtype, int tile_hint);
 hipError_t launch_depth_score_backward_binned(const DepthScoreBwdArgs &d, int dtype, void *workspace,
                                               size_t workspace_bytes, int tile_hint, int chunk_hint,
