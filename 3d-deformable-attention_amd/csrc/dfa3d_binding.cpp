@@ -3,13 +3,15 @@
 // took 10 of the 17 us that it cost.
 //
 // Every function takes the operands only where all of them are what its kernels read: plain tensors (no subclass, no transform's
-// wrapper) of the right shapes and types, contiguous, on the device that is current, with something to do.  Anything else is declined
+// wrapper) of the right shapes and types, contiguous, on the device that is current, under no dispatch mode, with something to do.  Anything else is declined
 // (None), and the Python form of the call, which says what is wrong, takes it from there.  The library's entry points come as
 // addresses (bind), so this module serves whichever build of the library is loaded.
 #include <Python.h>
 
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -118,10 +120,16 @@ bool numbers(PyObject *const *args, int64_t &device, void *&stream) {
   stream = PyLong_AsVoidPtr(args[1]);
   return !PyErr_Occurred();
 }
+// a dispatch mode (fake tensors, tracing) or a function transform would give the outputs that are allocated here another form
+bool plain_dispatch() {
+  return !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+         !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
 #define TAKES(n)                                                                            \
   if (nargs != (n)) { PyErr_SetString(PyExc_TypeError, "wrong number of arguments"); return nullptr; } \
   Operands in; void *stream;                                                                \
-  if (!numbers(args, in.device, stream)) return nullptr;
+  if (!numbers(args, in.device, stream)) return nullptr;                                    \
+  if (!plain_dispatch()) return declined();
 
 // fused_forward(device, stream, value, dist, shapes, starts, loc, attn, im2col_step, need_score, need_weight_update, packed)
 // -> (out, score or None, weight_update or None), or None

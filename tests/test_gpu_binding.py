@@ -2,6 +2,8 @@
 complaint where an operand is not what the kernels read, and the caller's stream."""
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from forms import tiny_case
 from test_gpu_parity import _as_inputs, _dev
@@ -51,6 +53,7 @@ def test_both_ways(monkeypatch, kind, dtype):
     o = _operands(dtype, one=kind == "weight_update_one")
     kind = kind.replace("_one", "") if kind == "weight_update_one" else kind
     side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
         short = _run(o, kind)
     torch.cuda.current_stream().wait_stream(side)
@@ -99,5 +102,11 @@ def test_subclasses_and_transforms_take_the_long_way():
     seen = []
     torch.func.vmap(lambda v: (seen.append(native.fused_forward(*args(v))), v)[1])(o["value"][None])
     assert seen == [None]
+    torch.func.vmap(lambda v: (seen.append(native.fused_forward(*args(o["value"]))), v)[1])(o["value"][None])
+    with TorchDispatchMode():
+        seen.append(native.fused_forward(*args(o["value"])))
+    with FakeTensorMode():
+        seen.append(native.fused_forward(*args(o["value"])))
+    assert seen == [None] * 4
     with _lib.launch_options(iters=2):
         assert _ext._here(o["value"]) is None
