@@ -527,6 +527,15 @@ static int check_linear(const char *fn, long long N, int O, int K) {
   return 0;
 }
 
+int dfa3d_linear(const float *x, const float *weight, const float *bias, float *y, long long N, int O, int K, int weight_across,
+                 void *stream) {
+  const char *fn = "dfa3d_linear";
+  if (int rc = check_linear(fn, N, O, K)) return rc;
+  if ((K & 3) != 0) return fail(DFA3D_EINVAL, "%s: K must be a multiple of four (K=%d)", fn, K);
+  REQUIRE_PTR(fn, x); REQUIRE_PTR(fn, weight); REQUIRE_PTR(fn, y);
+  return hip_result(dfa3d::launch_linear(x, weight, bias, y, N, O, K, weight_across != 0, (hipStream_t)stream), fn);
+}
+
 size_t dfa3d_linear_grad_workspace_bytes(long long N, int O, int K) {
   if (check_linear("dfa3d_linear_grad_workspace_bytes", N, O, K)) return 0;
   return dfa3d::linear_grad_workspace_bytes(N, O, K);

@@ -1,34 +1,242 @@
-// Weight and bias gradients of the projections around the operator (the value, offset, weight and output layers of the
-// cross-attention module) for gfx950:
+// The projections around the operator (the value, offset, weight and output layers of the cross-attention module) in float32, for gfx950:
 //
-//   grad_weight (O, K) = grad_out (N, O)^T  input (N, K)      grad_bias (O) = column sums of grad_out
+//   y (N, O) = x (N, K) weight (O, K)^T + bias          grad_x (N, K) = grad_out (N, O) weight (O, K)
+//   grad_weight (O, K) = grad_out (N, O)^T x (N, K)     grad_bias (O) = column sums of grad_out
 //
-// in float32.  N is the number of rows (pixels of all cameras, or queries: 10^4 to 10^6), O and K are embedding widths
-// (64 to 1024): a contraction over a very long dimension with a small result.  What bounds it is the float32 matrix
-// rate, and what it needs is parallelism that the 4 to 16 result tiles do not have: the rows are cut into parts, a
-// workgroup forms one 128 x 128 tile of one part's product, and a second kernel adds the parts up in a fixed order.
+// N is the number of rows (pixels of all cameras, or queries: 10^4 to 10^6), O and K are embedding widths (64 to 1024).  Float32
+// matrix instructions have a sixteenth of bfloat16's rate, and bounded these products.  So each float32 is split into three bfloat16 whose
+// sum it is, and a product is six of bfloat16 parts, summed in float32: those whose size is 2^-25 of the whole or less are left out.  What
+// bounds it now is what goes on beside the matrix unit, which is busy for a third of the time: the splitting (one third as many
+// vector cycles as matrix cycles), LDS, rows that come and go.
 //
-//   * v_mfma_f32_32x32x2: a lane holds one element of row n of grad_out and one of input; both operands are read along
-//     their rows, so nothing is transposed and nothing goes through LDS.  A lane reads two neighbouring columns (8 bytes)
-//     and gives them to two tiles (even and odd columns), so a wavefront's load covers whole 256-byte pieces of two rows
-//     and feeds a 64 x 64 tile with four matrix instructions per row pair.
-//   * the loads of the next 16 rows are in flight while the current 16 are multiplied.
-//   * workgroups of one part differ by multiples of the number of parts (a multiple of 8), so they run on one XCD and
-//     share its L2.
-//   * rows beyond a part's end and columns beyond O or K read as zero (buffer range check).
+//   * A workgroup of four wavefronts forms a tile of the result, 16 contraction steps at a time: the next step's operands are split into
+//     LDS and the one after is asked for while this one's parts are multiplied, with one barrier per step.  Steps of 32 with one buffer
+//     and two barriers took as long or longer (184950 rows of 256 x 256, 64 x 128 tiles: 195 us for 184; weight gradient 197 for 193).
+//   * 64 x 128 tiles: 128 x 256, 128 x 128, 64 x 128, 64 x 64 take 210, 199, 184, 206 us for 184950 rows of 256 x 256, 43, 31, 26, 27 for 22500, 35, 21,
+//     13, 12 for 5520; smaller tiles have more workgroups per CU, which wait in turn.
+//   * The result of a weight gradient is small and its contraction long: the rows are cut into parts, a workgroup forms one 128 x 128 tile of
+//     one part's product, and a second kernel adds the parts up in a fixed order.  Workgroups of one part differ by multiples of the
+//     number of parts (a multiple of 8), so they run on one XCD and share its L2.
+//   * Rows beyond the end and columns beyond O or K read as zero (buffer range check).
 //
-// Measured with the library's product and column sum for comparison, us: 184950 rows of 256 x 256 248 (98 TFLOP/s; float32
-// matrix peak 157) against 608; 48000 of 256 x 512 123 against 562; 9000 of 256 x 64 23 against 77; 5000 of 128 x 96 21
-// against 40.  The relative error of grad_weight against float64 is 3e-7 to 1e-6 where the library's is 1e-6 to 5e-6
-// (random signs), that of grad_bias 1e-7 to 3e-7 where it is 1e-7 to 4e-7: the parts shorten the chain of additions.
+// Library (forward and grad_x) or the float32 matrix instructions before (weight gradient), and now, us, between other kernels: 184950 rows of
+// 256 x 256 229, 177 (forward), 220, 171 (grad_x), 227, 147 (weight gradient); 58000 of 256 x 256 80, 56; 22500 45, 26; 5520 20, 12; 6600 of 256 x 64 19, 9.
+// Relative error against float64 (2-norm), the same: forward 2.0e-7, 1.7e-7 (5520 to 10^6 rows); grad_x 2.9e-7, 2.4e-7; weight gradient
+// 184950 rows 6.9e-7, 4.4e-7, 10^6 rows 1.6e-6, 9.6e-7, all positive 6.7e-8, 4.8e-8; grad_bias 2.1e-7, 2.1e-7.
 #include "../../include/dfa3d.h"
+#include "dfa3d_binned.h"
 #include "dfa3d_device.h"
 #include "dfa3d_launch.h"
 
 namespace dfa3d {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-constexpr int kPairs = 8;              // row pairs loaded at once
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+constexpr int kStep = 16;              // contraction steps staged at once: of one matrix instruction
+
+// One operand of a product as its tile of R rows and kStep contraction steps comes through registers into LDS.  Element (row, k) lies at
+// row * ld + k, or (ACROSS) at k * ld + row.  In LDS: three planes of bfloat16, each in two pieces of eight contraction steps, 16 bytes per
+// row and piece; the 64 bytes between the pieces keep writes and reads off each other's banks.
+template <int R, bool ACROSS> struct SplitOperand {
+  static constexpr int kPiece = R * 16 + 64, kPlane = 2 * kPiece, kBytes = 3 * kPlane;
+  static constexpr int kRun = ACROSS ? 8 : 4;                                  // contraction steps of a thread's unit
+  static constexpr int kUnits = (R * kStep / kRun + 255) / 256;
+  float v[kUnits][kRun];
+
+  // r: begins at the tile's first row, or (ACROSS) at the first contraction step, and ends with the last valid one.  `row0` and `rows`: ACROSS,
+  // the tile's first row and how many there are in all.  What lies beyond reads as zero.
+  __device__ __forceinline__ void load(rsrc_t r, int ld, int row0, int rows, int k0, int depth) {
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+      const int idx = (int)threadIdx.x + 256 * u;
+      if constexpr (ACROSS) {
+        const int row = row0 + idx % R, k = k0 + 8 * (idx / R);
+        const uint32_t off = (row < rows && idx < 2 * R) ? (uint32_t)(k * ld + row) * 4 : kNoRow;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[u][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off + (uint32_t)(j * ld) * 4, 0, 0));
+      } else {
+        const int row = idx / 4, k = k0 + 4 * (idx % 4);
+        const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r, k < depth ? (uint32_t)(row * ld + k) * 4 : kNoRow, 0, 0);
+        v[u][0] = __uint_as_float(t.x); v[u][1] = __uint_as_float(t.y);
+        v[u][2] = __uint_as_float(t.z); v[u][3] = __uint_as_float(t.w);
+      }
+    }
+  }
+
+  // x = p1 + p2 + p3, each rounded to nearest: 24 bits and more, so nothing of a float32 is lost
+  __device__ __forceinline__ void to_lds(unsigned char *lds) const {
+    typedef unsigned int words __attribute__((ext_vector_type(kRun / 2)));
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+      const int idx = (int)threadIdx.x + 256 * u;
+      if (2 * R % 256 != 0 && ACROSS && idx >= 2 * R) break;
+      unsigned char *at = lds + (ACROSS ? idx / R * kPiece + idx % R * 16 : idx % 4 / 2 * kPiece + idx / 4 * 16 + idx % 2 * 8);
+      float rest[kRun];
+#pragma unroll
+      for (int j = 0; j < kRun; ++j) rest[j] = v[u][j];
+#pragma unroll
+      for (int plane = 0; plane < 3; ++plane) {
+        words p;
+#pragma unroll
+        for (int j = 0; j < kRun / 2; ++j) {
+          uint32_t two = pack_bf16x2(rest[2 * j], rest[2 * j + 1]);
+          asm("" : "+v"(two));                                 // (or each half is rounded once more for its difference)
+          p[j] = two;
+          if (plane < 2) {
+            rest[2 * j] -= __uint_as_float(two << 16);
+            rest[2 * j + 1] -= __uint_as_float(two & 0xFFFF0000u);
+          }
+        }
+        *reinterpret_cast<words *>(at + plane * kPlane) = p;
+      }
+    }
+  }
+  // this lane's part of a matrix instruction's operand
+  static __device__ __forceinline__ bf16x8 part(const unsigned char *lds, int plane, int half, int row) {
+    return *reinterpret_cast<const bf16x8 *>(lds + plane * kPlane + half * kPiece + row * 16);
+  }
+};
+
+// acc = sum over depth contraction steps of A(m, k) B(n, k) for a TM x TN tile by four wavefronts, 2 x 2; `seen` is called with A's registers
+// once per kStep steps.  FLUSH: the matrix unit does not round its sums to nearest, which a chain of more than some hundred steps feels; its sums
+// start from zero every FLUSH steps and the vector unit adds them up.
+template <int TM, int TN, bool A_ACROSS, bool B_ACROSS, int FLUSH, typename Seen>
+__device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, int lda, int a_row0, int a_rows, rsrc_t b_r, int ldb, int b_row0,
+                                              int b_rows, int depth, f32x16 (&acc)[TM / 64][TN / 64], const Seen &seen) {
+  constexpr int MT = TM / 64, NT = TN / 64;
+  using OpA = SplitOperand<TM, A_ACROSS>;
+  using OpB = SplitOperand<TN, B_ACROSS>;
+  constexpr int kBuffer = OpA::kBytes + OpB::kBytes;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int half = lane / 32, row_a = (wave & 1) * MT * 32 + lane % 32, row_b = (wave >> 1) * NT * 32 + lane % 32;
+  f32x16 sum[MT][NT];
+  auto zero = [](f32x16 (&x)[MT][NT]) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[i][j][r] = 0;
+  };
+  zero(sum);
+  if (FLUSH) zero(acc);
+  OpA a;
+  OpB b;
+  a.load(a_r, lda, a_row0, a_rows, 0, depth);
+  b.load(b_r, ldb, b_row0, b_rows, 0, depth);
+  a.to_lds(lds);
+  b.to_lds(lds + OpA::kBytes);
+  seen(a);
+  a.load(a_r, lda, a_row0, a_rows, kStep, depth);
+  b.load(b_r, ldb, b_row0, b_rows, kStep, depth);
+  for (int k0 = 0, at = 0; k0 < depth; k0 += kStep, at ^= kBuffer) {          // uniform
+    lds_barrier();                                            // this step's parts are there, and nobody reads the last one's any more
+    const unsigned char *const mine = lds + at;
+    unsigned char *const next = lds + (at ^ kBuffer);
+    bf16x8 pa[MT][3], pb[NT][3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) pa[i][p] = OpA::part(mine, p, half, row_a + 32 * i);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) pb[j][p] = OpB::part(mine + OpA::kBytes, p, half, row_b + 32 * j);
+    }
+    a.to_lds(next);                                           // (beyond depth: zeros that nobody reads)
+    b.to_lds(next + OpA::kBytes);
+    seen(a);
+    a.load(a_r, lda, a_row0, a_rows, k0 + 2 * kStep, depth);
+    b.load(b_r, ldb, b_row0, b_rows, k0 + 2 * kStep, depth);
+    constexpr int kOf[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};          // smallest first
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[i][kOf[t][0]], pb[j][kOf[t][1]], sum[i][j], 0, 0, 0);
+    if (FLUSH && (k0 + kStep) % (FLUSH ? FLUSH : 1) == 0) {   // uniform
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[i][j][r] += sum[i][j][r];
+      zero(sum);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = FLUSH ? acc[i][j][r] + sum[i][j][r] : sum[i][j][r];
+}
+
+// Result (m, n) of the tile by plain float32 arithmetic, for the elements that the split gives no number for.
+template <bool A_ACROSS, bool B_ACROSS>
+__device__ __noinline__ float plain_product(rsrc_t a_r, int lda, int m, rsrc_t b_r, int ldb, int n, int depth) {
+  float sum = 0;
+  for (int k = 0; k < depth; ++k)
+    sum = fmaf(BufElem<float>::ld(a_r, (uint32_t)(A_ACROSS ? k * lda + m : m * lda + k) * 4),
+               BufElem<float>::ld(b_r, (uint32_t)(B_ACROSS ? k * ldb + n : n * ldb + k) * 4), sum);
+  return sum;
+}
+
+// A float32 infinity, or a number next to the largest, is no bfloat16 number, and an infinity times a lower part of zero is none either; and
+// the third part of a number below 2^-108 is denormal.  A sum that is no finite number, or tiny, is formed again without parts.
+__device__ __forceinline__ bool odd_sum(float x) { return !(fabsf(x) <= 3.402823466e38f) || (fabsf(x) < 0x1p-96f && x != 0.f); }
+
+// c (TM x TN tile of `ms` x `ns` valid elements, row length ldc) = acc + bias.
+template <int TM, int TN, bool A_ACROSS, bool B_ACROSS>
+__device__ __forceinline__ void store_product(const f32x16 (&acc)[TM / 64][TN / 64], rsrc_t a_r, int lda, int a_row0, rsrc_t b_r, int ldb, int b_row0,
+                                              int depth, float *__restrict__ c, int ldc, int ms, int ns, const float *__restrict__ bias) {
+  constexpr int MT = TM / 64, NT = TN / 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int first_m = (wave & 1) * MT * 32 + 4 * (lane / 32), first_n = (wave >> 1) * NT * 32 + lane % 32;
+  auto row_a = [&](int i, int r) { return first_m + 32 * i + 8 * (r / 4) + r % 4; };
+  auto row_b = [&](int j) { return first_n + 32 * j; };
+  bool odd = false;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int n = row_b(j);
+    const float add = (bias != nullptr && n < ns) ? bias[n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int m = row_a(i, r);
+        odd = odd || odd_sum(acc[i][j][r]);
+        if (m < ms && n < ns) c[(size_t)m * ldc + n] = acc[i][j][r] + add;
+      }
+  }
+  if (odd) {
+    for (int e = 0; e < NT * MT * 16; ++e) {
+      const int m = row_a(e / 16 % MT, e % 16), n = row_b(e / 16 / MT);
+      if (m >= ms || n >= ns) continue;
+      float *to = c + (size_t)m * ldc + n;
+      if (bias == nullptr && !odd_sum(*to)) continue;
+      *to = plain_product<A_ACROSS, B_ACROSS>(a_r, lda, a_row0 + m, b_r, ldb, b_row0 + n, depth) + (bias != nullptr ? bias[n] : 0.f);
+    }
+  }
+}
+
+// y (N, O) = x (N, K) w (O, K)^T + bias, or (B_ACROSS) with w (K, O).  TM rows of one tile of TN columns per workgroup; those of the same rows run
+// on one XCD.
+template <int TM, int TN, bool B_ACROSS>
+__global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
+                                                        float *__restrict__ y, long long N, int O, int K, int o_tiles) {
+  __shared__ __align__(16) unsigned char lds[2 * (SplitOperand<TM, false>::kBytes + SplitOperand<TN, B_ACROSS>::kBytes)];
+  const long long group = blockIdx.x / (8 * o_tiles);
+  const int in_group = blockIdx.x % (8 * o_tiles), o0 = in_group / 8 * TN;
+  const long long n0 = (group * 8 + in_group % 8) * TM;
+  if (n0 >= N) return;                                        // uniform
+  const int ms = N - n0 < TM ? (int)(N - n0) : TM, ns = O - o0 < TN ? O - o0 : TN;
+  const rsrc_t x_r = make_rsrc(x + n0 * K, (size_t)ms * K * 4);
+  const rsrc_t w_r = B_ACROSS ? make_rsrc(w, (size_t)K * O * 4) : make_rsrc(w + (size_t)o0 * K, (size_t)ns * K * 4);
+  const int ldw = B_ACROSS ? O : K, row0 = B_ACROSS ? o0 : 0;
+  f32x16 acc[TM / 64][TN / 64];
+  split_product<TM, TN, false, B_ACROSS, 0>(lds, x_r, K, 0, 0, w_r, ldw, row0, O, K, acc, [](const auto &) {});
+  store_product<TM, TN, false, B_ACROSS>(acc, x_r, K, 0, w_r, ldw, row0, K, y + n0 * O + o0, O, ms, ns, bias != nullptr ? bias + o0 : nullptr);
+}
 
 struct LinearTiles { int o, k, parts, rows; };      // result tiles along O and K; parts of the rows, rows of a part
 static LinearTiles linear_tiles(long long N, int O, int K) {
@@ -48,71 +256,29 @@ static LinearTiles linear_tiles(long long N, int O, int K) {
 __global__ __launch_bounds__(256, 2) void linear_grad_part_kernel(
     const float *__restrict__ x, const float *__restrict__ g, float *__restrict__ partial, long long N, int O, int K,
     int parts, int rows, int o_tiles, int want_bias) {
+  using OpG = SplitOperand<128, true>;
+  __shared__ __align__(16) unsigned char lds[4 * OpG::kBytes];
   const int part = blockIdx.x % parts, tile = blockIdx.x / parts;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
-  const int half = lane / 32, col = lane % 32;
-  const int o0 = (tile % o_tiles) * 128 + (wave & 1) * 64, k0 = (tile / o_tiles) * 128 + (wave >> 1) * 64;
-  if (o0 >= O || k0 >= K) return;                          // uniform per wavefront; no barriers below
+  const int o0 = (tile % o_tiles) * 128, k0 = (tile / o_tiles) * 128;
   const long long n0 = (long long)part * rows;
   const int n_rows = n0 < N ? (int)(N - n0 < rows ? N - n0 : rows) : 0;
   const rsrc_t g_r = make_rsrc(g + (n_rows > 0 ? n0 * O : 0), (size_t)n_rows * O * 4);
   const rsrc_t x_r = make_rsrc(x + (n_rows > 0 ? n0 * K : 0), (size_t)n_rows * K * 4);
-  const int go = o0 + 2 * col, xk = k0 + 2 * col;
-  uint32_t g_off = go < O ? (uint32_t)(half * O + go) * 4 : kNoRow, x_off = xk < K ? (uint32_t)(half * K + xk) * 4 : kNoRow;
-  const uint32_t g_step = 2u * O * 4, x_step = 2u * K * 4;
-
   f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
-  float bias0 = 0, bias1 = 0;
-  u32x2 ga[kPairs], xa[kPairs], gb[kPairs], xb[kPairs];
-  auto load = [&](u32x2 (&gv)[kPairs], u32x2 (&xv)[kPairs]) {
-#pragma unroll
-    for (int j = 0; j < kPairs; ++j) {
-      gv[j] = __builtin_amdgcn_raw_buffer_load_b64(g_r, g_off + j * g_step, 0, 0);
-      xv[j] = __builtin_amdgcn_raw_buffer_load_b64(x_r, x_off + j * x_step, 0, 0);
-    }
-    g_off += kPairs * g_step; x_off += kPairs * x_step;
-  };
-  auto multiply = [&](const u32x2 (&gv)[kPairs], const u32x2 (&xv)[kPairs]) {
-    static_assert(kPairs == 8, "the sums below");
-    auto sum8 = [&](auto of) { return ((of(0) + of(1)) + (of(2) + of(3))) + ((of(4) + of(5)) + (of(6) + of(7))); };
-    bias0 += sum8([&](int j) { return __uint_as_float(gv[j].x); });      // a tree per batch: a chain of rows would round more
-    bias1 += sum8([&](int j) { return __uint_as_float(gv[j].y); });
-#pragma unroll
-    for (int j = 0; j < kPairs; ++j) {
-      const float a0 = __uint_as_float(gv[j].x), a1 = __uint_as_float(gv[j].y);
-      const float b0 = __uint_as_float(xv[j].x), b1 = __uint_as_float(xv[j].y);
-      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc[1][1], 0, 0, 0);
-    }
-  };
-  load(ga, xa);
-  for (int n = 0; n < n_rows; n += 4 * kPairs) {            // uniform; what lies beyond the part's rows reads as zero
-    load(gb, xb);
-    multiply(ga, xa);
-    load(ga, xa);
-    multiply(gb, xb);
-  }
+  float bias_sum = 0;                                       // of this thread's column and every other eight rows
+  split_product<128, 128, true, true, 64>(lds, g_r, O, o0, O, x_r, K, k0, K, n_rows, acc, [&](const OpG &a) {
+    const float *v = a.v[0];                                // a tree per batch: a chain of rows would round more
+    bias_sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  });
   float *mine = partial + (size_t)part * ((size_t)O * K + O);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int o = o0 + 2 * (8 * (r / 4) + 4 * half + r % 4) + i, k = k0 + 2 * col;
-      if (o < O && k < K) *reinterpret_cast<float2 *>(mine + (size_t)o * K + k) = make_float2(acc[i][0][r], acc[i][1][r]);
-    }
-  }
-  if (want_bias && k0 == 0) {
-    bias0 += __shfl_xor(bias0, 32, kWave);
-    bias1 += __shfl_xor(bias1, 32, kWave);
-    if (half == 0 && go < O) *reinterpret_cast<float2 *>(mine + (size_t)O * K + go) = make_float2(bias0, bias1);
+  store_product<128, 128, true, true>(acc, g_r, O, o0, x_r, K, k0, n_rows, mine + (size_t)o0 * K + k0, K, O - o0, K - k0, nullptr);
+  if (want_bias && k0 == 0) {                               // uniform
+    float *s_bias = reinterpret_cast<float *>(lds);
+    lds_barrier();
+    s_bias[threadIdx.x] = bias_sum;
+    lds_barrier();
+    const int col = threadIdx.x;
+    if (col < 128 && o0 + col < O) mine[(size_t)O * K + o0 + col] = s_bias[col] + s_bias[128 + col];
   }
 }
 
@@ -137,6 +303,26 @@ __global__ __launch_bounds__(256) void linear_grad_sum_kernel(const float *__res
     if (i < weights) grad_weight[i] = s;
     else if (grad_bias != nullptr) grad_bias[i - weights] = s;
   }
+}
+
+template <int TM, int TN, bool B_ACROSS>
+static hipError_t launch_linear_cfg(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream) {
+  const long long groups = ((N + TM - 1) / TM + 7) / 8;
+  const int o_tiles = (O + TN - 1) / TN;
+  if (groups * 8 * o_tiles > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((linear_kernel<TM, TN, B_ACROSS>), dim3((unsigned)(groups * 8 * o_tiles)), dim3(256), 0, stream, x, w, bias, y, N, O, K, o_tiles);
+  return hipGetLastError();
+}
+
+template <bool B_ACROSS>
+static hipError_t launch_linear_as(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream) {
+  // at least two workgroups per CU: 4096 rows of 256 x 256 (128 larger tiles) 14 us with them, 10 with 256 smaller ones; 22500 (704) 26, 27
+  if ((N + 63) / 64 * ((O + 127) / 128) < 512 || O <= 64) return launch_linear_cfg<64, 64, B_ACROSS>(x, w, bias, y, N, O, K, stream);
+  return launch_linear_cfg<64, 128, B_ACROSS>(x, w, bias, y, N, O, K, stream);
+}
+
+hipError_t launch_linear(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, bool w_across, hipStream_t stream) {
+  return w_across ? launch_linear_as<true>(x, w, bias, y, N, O, K, stream) : launch_linear_as<false>(x, w, bias, y, N, O, K, stream);
 }
 
 size_t linear_grad_workspace_bytes(long long N, int O, int K) {

@@ -50,6 +50,7 @@ SIGNATURES = {
     "dfa3d_camera_index": [_P] * 4 + [_I] * 3 + [_P],
     "dfa3d_locations": [_P] * 5 + [ctypes.c_longlong] + [_I] * 4 + [_P],
     "dfa3d_locations_grad": [_P] * 4 + [ctypes.c_longlong] + [_I] * 3 + [_P],
+    "dfa3d_linear": [_P] * 4 + [ctypes.c_longlong, _I, _I, _I, _P],
     "dfa3d_linear_grad": [_P] * 5 + [ctypes.c_size_t, ctypes.c_longlong, _I, _I, _P],
     "dfa3d_abi_version": [],
 }

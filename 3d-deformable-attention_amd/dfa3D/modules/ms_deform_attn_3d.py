@@ -82,10 +82,10 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         self.num_levels = num_levels
         self.num_heads = num_heads
         self.num_points = num_points
-        self.sampling_offsets = Projection(embed_dims, num_heads * num_levels * num_points * 2)
+        self.sampling_offsets = Projection(embed_dims, num_heads * num_levels * num_points * 2, library_forward=True)
         self.attention_weights = Projection(embed_dims, num_heads * num_levels * num_points)
         self.value_proj = Projection(embed_dims, embed_dims)
-        self.sampling_offsets_depth = Projection(embed_dims, num_heads * num_levels * num_points)
+        self.sampling_offsets_depth = Projection(embed_dims, num_heads * num_levels * num_points, library_forward=True)
         self.init_weights()
         self.init_smpl_off_weights()
 

@@ -1,5 +1,5 @@
-"""The projections' own weight and bias gradient kernel against float64: row counts around its parts, widths that are not
-multiples of its tiles; and the calls that keep the library's gradients."""
+"""The projections' own kernels against float64: row counts around tiles and parts, widths that are not multiples of the
+tiles, operands that are no ordinary numbers; and the calls that keep the library's operations."""
 import pytest
 import torch
 
@@ -28,6 +28,57 @@ def test_weight_and_bias_gradients(N, K, O):
         assert (a.double().cpu() - b).abs().max() <= 4e-6 * n ** 0.5 * 4
     again = torch.autograd.grad(layer(x), [layer.weight, layer.bias], g)
     assert torch.equal(again[0], got[1]) and torch.equal(again[1], got[2])      # fixed order of summation
+
+
+@pytest.mark.parametrize("N,K,O", [(1, 4, 2), (63, 36, 62), (64, 16, 64), (65, 20, 66), (130, 256, 130), (4097, 12, 128), (16385, 48, 256),
+                                   (20001, 256, 258), (33000, 8, 64)])
+@pytest.mark.parametrize("across", [False, True])
+def test_product(N, K, O, across):
+    from dfa3D.modules import projection
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(N + K + O)
+    x, w, b = (torch.randn(*s, generator=g, device=dev) for s in ((N, K), (O, K), (O,)))
+    assert projection._product_applies(N, O, K)
+    got = projection._product(x, w.t().contiguous() if across else w, None if across else b, across)
+    xd, wd, bd = x.double(), w.double(), torch.zeros_like(b).double() if across else b.double()
+    # three parts hold all of a float32; what is left out is 2^-25 of a product at most, and each of K / 16 steps of six sums, and the bias,
+    # is rounded (or cut) to 2^-23 of the running sum, at most the sum of the sizes
+    bound = (2.0 ** -25 + (6 * (K // 16 + 1) + 16 + 1) * 2.0 ** -23) * (xd.abs() @ wd.abs().t() + bd.abs())
+    assert ((got.double() - (xd @ wd.t() + bd)).abs() <= bound).all()
+    again = projection._product(x, w.t().contiguous() if across else w, None if across else b, across)
+    assert torch.equal(got, again)
+
+
+def test_operands_that_are_no_ordinary_numbers():
+    """Infinities, NaN, numbers that bfloat16 rounds to infinity, and tiny ones, whose parts are denormal: as the library's product."""
+    from dfa3D.modules import projection
+    dev = torch.device("cuda:0")
+    torch.manual_seed(1)
+    x, w, b = torch.randn(4200, 64, device=dev), torch.randn(96, 64, device=dev), torch.randn(96, device=dev)
+    w[:, 1] = 0.5
+    x[3, 5], x[7, 9], x[200, 1], x[201, 1] = float("inf"), float("nan"), 3.402823e38, -3.402823e38
+    x[50] *= 1e-34
+    got, want = projection._product(x, w, b, False), torch.nn.functional.linear(x, w, b)
+    torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-4, equal_nan=True)
+    tiny = projection._product(x[50:51], w, None, False).double()
+    torch.testing.assert_close(tiny, x[50:51].double() @ w.double().t(), rtol=0, atol=64 * 2.0 ** -23 * 1e-34 * 16)
+    across = projection._product(x, w.t().contiguous(), None, True)
+    torch.testing.assert_close(across, x.matmul(w.t()), rtol=1e-5, atol=1e-4, equal_nan=True)
+    g = torch.randn(4200, 96, device=dev)
+    g[9, 3], g[11, 6], x[11, 4], x[7, 9], x[3, 5] = float("inf"), 3.402823e38, 1.5, 0., 0.
+    x[200:202] = 0
+    gw, _ = projection._weight_gradients(x, g, True)
+    torch.testing.assert_close(gw, g.t().mm(x), rtol=1e-4, atol=1e-2, equal_nan=True)
+
+
+def test_offsets_keep_the_librarys_result_in_training():
+    from dfa3D.modules.projection import Projection
+    dev = torch.device("cuda:0")
+    layer = Projection(256, 128, library_forward=True).to(dev)
+    x = torch.randn(5000, 256, device=dev)
+    assert torch.equal(layer(x), torch.nn.functional.linear(x, layer.weight, layer.bias))
+    with torch.no_grad():
+        torch.testing.assert_close(layer(x), torch.nn.functional.linear(x, layer.weight, layer.bias), rtol=1e-5, atol=1e-5)
 
 
 def test_rows_in_other_layouts_and_partial_gradients():
