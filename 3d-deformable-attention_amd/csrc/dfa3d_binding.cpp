@@ -8,8 +8,10 @@
 // addresses (bind), so this module serves whichever build of the library is loaded.
 #include <Python.h>
 
+#include <ATen/autocast_mode.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
@@ -17,6 +19,7 @@
 
 #include <initializer_list>
 #include <limits>
+#include <vector>
 
 #include "../../include/dfa3d.h"
 
@@ -35,6 +38,8 @@ struct Api {
   decltype(&dfa3d_ms_depth_score_sample_backward_workspace_bytes) score_backward_workspace_bytes;
   decltype(&dfa3d_ms_depth_score_sample_backward_into) score_backward;
   decltype(&dfa3d_pack_dist) pack_dist;
+  decltype(&dfa3d_linear) linear;
+  decltype(&dfa3d_linear_sum) linear_sum;
 } api;
 
 using at::Tensor;
@@ -347,6 +352,90 @@ PyObject *pack_dist(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// Where the kernels form a product of rows x width elements, sums of depth terms.  They read four neighbours of a row at a time, and take the
+// library's place except where few rows meet a deep sum: library and kernel, us, 4096 rows of 256 by 256 19, 10; 256 by 64 19, 7; sums of 512 by
+// 256 19, 22; of 2048 by 256 41, 51 to 89; of 1024 by 1024 72, 59; 20000 rows of 512 by 512 98, 70; of 2048 by 256 165, 145; 100000 of 256 by 256 123, 93.
+bool product_applies(int64_t rows, int64_t width, int64_t depth) {
+  return width > 0 && depth > 0 && width <= 4096 && depth <= 4096 && width % 2 == 0 && depth % 4 == 0 && rows > 0 && rows <= (int64_t(1) << 31) &&
+         (depth <= 256 || rows * width >= (int64_t(1) << 22));
+}
+constexpr Py_ssize_t kMaxSets = 4;
+// pairs of a flat tuple, 0 where it is none of 1 to kMaxSets pairs
+Py_ssize_t pairs_of(PyObject *o) {
+  const Py_ssize_t n = PyTuple_CheckExact(o) ? PyTuple_GET_SIZE(o) : 0;
+  return n % 2 == 0 && n / 2 <= kMaxSets ? n / 2 : 0;
+}
+bool is_float_matrix(const Tensor &t) { return t.scalar_type() == at::kFloat && t.dim() == 2; }
+bool recorded(const Tensor &t) { return t.defined() && t.requires_grad() && c10::GradMode::is_enabled(); }
+
+// linear(device, stream, x (..., K), (weight (O, K), bias (O) or None, ...)) -> F.linear of every layer, none of it recorded, or None
+PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TAKES(4)
+  const Tensor &x = in.need(args[2]);
+  const Py_ssize_t n = pairs_of(args[3]);
+  if (!in.ok || n == 0 || x.scalar_type() != at::kFloat || x.dim() < 2 || x.size(-1) == 0 || recorded(x) ||
+      at::autocast::is_autocast_enabled(at::kCUDA) || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer))
+    return declined();
+  const int64_t K = x.size(-1), rows = x.numel() / K;
+  dfa3d_linear_set sets[kMaxSets];
+  Tensor out[kMaxSets];
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const Tensor &w = in.need(PyTuple_GET_ITEM(args[3], 2 * i)), &b = in.may_have(PyTuple_GET_ITEM(args[3], 2 * i + 1));
+    if (!in.ok || !is_float_matrix(w) || w.size(1) != K || recorded(w) || recorded(b) || !product_applies(rows, w.size(0), K) ||
+        (b.defined() && (b.scalar_type() != at::kFloat || !shape_is(b, {w.size(0)}))))
+      return declined();
+    sets[i] = dfa3d_linear_set{static_cast<const float *>(ptr(w)), static_cast<const float *>(ptr(b)), nullptr, static_cast<int>(w.size(0))};
+  }
+  auto sizes = x.sizes().vec();
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    sizes.back() = sets[i].width;
+    out[i] = at::empty(sizes, x.options());
+    sets[i].rows = static_cast<float *>(ptr(out[i]));
+  }
+  int rc;
+  {
+    NoGil no_gil;
+    rc = api.linear(static_cast<const float *>(ptr(x)), sets, (int)n, rows, (int)K, stream);
+  }
+  if (rc != 0) return failed("dfa3d_linear", rc);
+  PyObject *all = PyTuple_New(n);
+  for (Py_ssize_t i = 0; all != nullptr && i < n; ++i) PyTuple_SET_ITEM(all, i, THPVariable_Wrap(out[i]));
+  return all;
+  END_HANDLE_TH_ERRORS
+}
+
+// linear_sum(device, stream, (rows (..., O), weight (O, K), ...)) -> sum of rows times weight (..., K), not recorded, or None
+PyObject *linear_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TAKES(3)
+  const Py_ssize_t n = pairs_of(args[2]);
+  if (n == 0 || at::autocast::is_autocast_enabled(at::kCUDA) || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer)) return declined();
+  dfa3d_linear_set sets[kMaxSets];
+  int64_t K = 0, rows = 0;
+  std::vector<int64_t> sizes;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const Tensor &g = in.need(PyTuple_GET_ITEM(args[2], 2 * i)), &w = in.need(PyTuple_GET_ITEM(args[2], 2 * i + 1));
+    if (!in.ok || g.scalar_type() != at::kFloat || g.dim() < 2 || !is_float_matrix(w) || g.size(-1) != w.size(0) || w.size(0) == 0 || recorded(g) ||
+        recorded(w))
+      return declined();
+    auto shape = g.sizes().vec();
+    shape.back() = w.size(1);
+    if (i == 0) { sizes = shape; K = w.size(1); rows = g.numel() / w.size(0); }
+    if (shape != sizes || !product_applies(rows, K, w.size(0))) return declined();
+    sets[i] = dfa3d_linear_set{static_cast<const float *>(ptr(w)), nullptr, static_cast<float *>(ptr(g)), static_cast<int>(w.size(0))};
+  }
+  Tensor y = at::empty(sizes, THPVariable_Unpack(PyTuple_GET_ITEM(args[2], 0)).options());
+  int rc;
+  {
+    NoGil no_gil;
+    rc = api.linear_sum(sets, (int)n, static_cast<float *>(ptr(y)), rows, (int)K, stream);
+  }
+  if (rc != 0) return failed("dfa3d_linear_sum", rc);
+  return THPVariable_Wrap(y);
+  END_HANDLE_TH_ERRORS
+}
+
 // bind(dict of entry point -> address)
 PyObject *bind(PyObject *, PyObject *table) {
   auto address = [&](const char *name, auto &to) {
@@ -368,7 +457,8 @@ PyObject *bind(PyObject *, PyObject *table) {
       !address("dfa3d_wms_deform_attn_backward", a.attention_backward) ||
       !address("dfa3d_ms_depth_score_sample_forward", a.score_forward) ||
       !address("dfa3d_ms_depth_score_sample_backward_workspace_bytes", a.score_backward_workspace_bytes) ||
-      !address("dfa3d_ms_depth_score_sample_backward_into", a.score_backward) || !address("dfa3d_pack_dist", a.pack_dist))
+      !address("dfa3d_ms_depth_score_sample_backward_into", a.score_backward) || !address("dfa3d_pack_dist", a.pack_dist) ||
+      !address("dfa3d_linear", a.linear) || !address("dfa3d_linear_sum", a.linear_sum))
     return nullptr;
   api = a;
   Py_RETURN_NONE;
@@ -385,6 +475,8 @@ PyMethodDef methods[] = {
     {"score_forward", as_method(score_forward), METH_FASTCALL, nullptr},
     {"score_gradients", as_method(score_gradients), METH_FASTCALL, nullptr},
     {"pack_dist", as_method(pack_dist), METH_FASTCALL, nullptr},
+    {"linear", as_method(linear), METH_FASTCALL, nullptr},
+    {"linear_sum", as_method(linear_sum), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -17,6 +17,9 @@
 //   * The result of a weight gradient is small and its contraction long: the rows are cut into parts, a workgroup forms one 128 x 128 tile of
 //     one part's product, and a second kernel adds the parts up in a fixed order.  Workgroups of one part differ by multiples of the
 //     number of parts (a multiple of 8), so they run on one XCD and share its L2.
+//   * Layers on the same rows go in one launch: 29000 rows of 256 to 128, 64 and 64 columns 20.6 + 13.8 + 13 us one by one, 34 together.  So
+//     does the gradient of those rows, whose sums are added up by the vector unit every 128 steps, as they run over all layers: 58000 rows of 256
+//     from 512, 256 and 256 columns 200 us for three products and 48 for their sums, 185 together.
 //   * Rows beyond the end and columns beyond O or K read as zero (buffer range check).
 //
 // Library (forward and grad_x) or the float32 matrix instructions before (weight gradient), and now, us, between other kernels: 184950 rows of
@@ -97,7 +100,16 @@ template <int R, bool ACROSS> struct SplitOperand {
   }
 };
 
-// acc = sum over depth contraction steps of A(m, k) B(n, k) for a TM x TN tile by four wavefronts, 2 x 2; `seen` is called with A's registers
+template <int MT, int NT> __device__ __forceinline__ void zero_sums(f32x16 (&x)[MT][NT]) {
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) x[i][j][r] = 0;
+}
+
+// acc += sum over depth contraction steps of A(m, k) B(n, k) for a TM x TN tile by four wavefronts, 2 x 2; `seen` is called with A's registers
 // once per kStep steps.  FLUSH: the matrix unit does not round its sums to nearest, which a chain of more than some hundred steps feels; its sums
 // start from zero every FLUSH steps and the vector unit adds them up.
 template <int TM, int TN, bool A_ACROSS, bool B_ACROSS, int FLUSH, typename Seen>
@@ -109,17 +121,9 @@ __device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, in
   constexpr int kBuffer = OpA::kBytes + OpB::kBytes;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int half = lane / 32, row_a = (wave & 1) * MT * 32 + lane % 32, row_b = (wave >> 1) * NT * 32 + lane % 32;
-  f32x16 sum[MT][NT];
-  auto zero = [](f32x16 (&x)[MT][NT]) {
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) x[i][j][r] = 0;
-  };
-  zero(sum);
-  if (FLUSH) zero(acc);
+  f32x16 since[MT][NT];                                       // FLUSH: since the last time
+  f32x16(&sum)[MT][NT] = *(FLUSH ? &since : &acc);
+  if (FLUSH) zero_sums(since);
   OpA a;
   OpB b;
   a.load(a_r, lda, a_row0, a_rows, 0, depth);
@@ -159,16 +163,18 @@ __device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, in
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] += sum[i][j][r];
-      zero(sum);
+          for (int r = 0; r < 16; ++r) acc[i][j][r] += since[i][j][r];
+      zero_sums(since);
     }
   }
+  if (FLUSH) {
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+      for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = FLUSH ? acc[i][j][r] + sum[i][j][r] : sum[i][j][r];
+        for (int r = 0; r < 16; ++r) acc[i][j][r] += since[i][j][r];
+  }
 }
 
 // Result (m, n) of the tile by plain float32 arithmetic, for the elements that the split gives no number for.
@@ -185,10 +191,10 @@ __device__ __noinline__ float plain_product(rsrc_t a_r, int lda, int m, rsrc_t b
 // the third part of a number below 2^-108 is denormal.  A sum that is no finite number, or tiny, is formed again without parts.
 __device__ __forceinline__ bool odd_sum(float x) { return !(fabsf(x) <= 3.402823466e38f) || (fabsf(x) < 0x1p-96f && x != 0.f); }
 
-// c (TM x TN tile of `ms` x `ns` valid elements, row length ldc) = acc + bias.
-template <int TM, int TN, bool A_ACROSS, bool B_ACROSS>
-__device__ __forceinline__ void store_product(const f32x16 (&acc)[TM / 64][TN / 64], rsrc_t a_r, int lda, int a_row0, rsrc_t b_r, int ldb, int b_row0,
-                                              int depth, float *__restrict__ c, int ldc, int ms, int ns, const float *__restrict__ bias) {
+// c (TM x TN tile of `ms` x `ns` valid elements, row length ldc) = acc + bias; `plain` forms one element without parts.
+template <int TM, int TN, typename Plain>
+__device__ __forceinline__ void store_product(const f32x16 (&acc)[TM / 64][TN / 64], float *__restrict__ c, int ldc, int ms, int ns,
+                                              const float *__restrict__ bias, const Plain &plain) {
   constexpr int MT = TM / 64, NT = TN / 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int first_m = (wave & 1) * MT * 32 + 4 * (lane / 32), first_n = (wave >> 1) * NT * 32 + lane % 32;
@@ -214,28 +220,54 @@ __device__ __forceinline__ void store_product(const f32x16 (&acc)[TM / 64][TN / 
       if (m >= ms || n >= ns) continue;
       float *to = c + (size_t)m * ldc + n;
       if (bias == nullptr && !odd_sum(*to)) continue;
-      *to = plain_product<A_ACROSS, B_ACROSS>(a_r, lda, a_row0 + m, b_r, ldb, b_row0 + n, depth) + (bias != nullptr ? bias[n] : 0.f);
+      *to = plain(m, n) + (bias != nullptr ? bias[n] : 0.f);
     }
   }
 }
 
-// y (N, O) = x (N, K) w (O, K)^T + bias, or (B_ACROSS) with w (K, O).  TM rows of one tile of TN columns per workgroup; those of the same rows run
-// on one XCD.
-template <int TM, int TN, bool B_ACROSS>
-__global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
-                                                        float *__restrict__ y, long long N, int O, int K, int o_tiles) {
-  __shared__ __align__(16) unsigned char lds[2 * (SplitOperand<TM, false>::kBytes + SplitOperand<TN, B_ACROSS>::kBytes)];
-  const long long group = blockIdx.x / (8 * o_tiles);
-  const int in_group = blockIdx.x % (8 * o_tiles), o0 = in_group / 8 * TN;
-  const long long n0 = (group * 8 + in_group % 8) * TM;
+// Up to kMaxLinearSets layers on the same rows x (N, K): rows (N, width) = x weight (width, K)^T + bias of each.  TM rows of one tile of TN columns
+// per workgroup; those of the same rows run on one XCD.
+template <int TM, int TN>
+__global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict__ x, LinearSets sets, long long N, int K, int tiles) {
+  __shared__ __align__(16) unsigned char lds[2 * (SplitOperand<TM, false>::kBytes + SplitOperand<TN, false>::kBytes)];
+  const long long n0 = (blockIdx.x / (8 * tiles) * 8 + blockIdx.x % 8) * (long long)TM;
   if (n0 >= N) return;                                        // uniform
-  const int ms = N - n0 < TM ? (int)(N - n0) : TM, ns = O - o0 < TN ? O - o0 : TN;
-  const rsrc_t x_r = make_rsrc(x + n0 * K, (size_t)ms * K * 4);
-  const rsrc_t w_r = B_ACROSS ? make_rsrc(w, (size_t)K * O * 4) : make_rsrc(w + (size_t)o0 * K, (size_t)ns * K * 4);
-  const int ldw = B_ACROSS ? O : K, row0 = B_ACROSS ? o0 : 0;
+  int o0 = blockIdx.x % (8 * tiles) / 8 * TN, i = 0;
+  for (int wide = (sets.set[0].width + TN - 1) / TN * TN; o0 >= wide; wide = (sets.set[i].width + TN - 1) / TN * TN) { o0 -= wide; ++i; }     // uniform
+  const LinearSet set = sets.set[i];
+  const int ms = N - n0 < TM ? (int)(N - n0) : TM, ns = set.width - o0 < TN ? set.width - o0 : TN;
+  const rsrc_t x_r = make_rsrc(x + n0 * K, (size_t)ms * K * 4), w_r = make_rsrc(set.weight + (size_t)o0 * K, (size_t)ns * K * 4);
   f32x16 acc[TM / 64][TN / 64];
-  split_product<TM, TN, false, B_ACROSS, 0>(lds, x_r, K, 0, 0, w_r, ldw, row0, O, K, acc, [](const auto &) {});
-  store_product<TM, TN, false, B_ACROSS>(acc, x_r, K, 0, w_r, ldw, row0, K, y + n0 * O + o0, O, ms, ns, bias != nullptr ? bias + o0 : nullptr);
+  zero_sums(acc);
+  split_product<TM, TN, false, false, 0>(lds, x_r, K, 0, 0, w_r, K, 0, 0, K, acc, [](const auto &) {});
+  store_product<TM, TN>(acc, set.rows + n0 * set.width + o0, set.width, ms, ns, set.bias != nullptr ? set.bias + o0 : nullptr,
+                        [&](int m, int n) { return plain_product<false, false>(x_r, K, m, w_r, K, n, K); });
+}
+
+// y (N, K) = sum of rows (N, width) weight (width, K) over the sets: the gradient of the rows that several layers share.  FLUSH: 0 for one set.
+template <int TM, int TN, int FLUSH>
+__global__ __launch_bounds__(256, 3) void linear_sum_kernel(LinearSets sets, float *__restrict__ y, long long N, int K, int tiles) {
+  __shared__ __align__(16) unsigned char lds[2 * (SplitOperand<TM, false>::kBytes + SplitOperand<TN, true>::kBytes)];
+  const long long n0 = (blockIdx.x / (8 * tiles) * 8 + blockIdx.x % 8) * (long long)TM;
+  if (n0 >= N) return;                                        // uniform
+  const int k0 = blockIdx.x % (8 * tiles) / 8 * TN, ms = N - n0 < TM ? (int)(N - n0) : TM;
+  f32x16 acc[TM / 64][TN / 64];
+  zero_sums(acc);
+  auto rows = [&](const LinearSet &s) { return make_rsrc(s.rows + n0 * s.width, (size_t)ms * s.width * 4); };
+  auto weight = [&](const LinearSet &s) { return make_rsrc(s.weight, (size_t)s.width * K * 4); };
+  for (int i = 0; i < sets.n; ++i) {                          // uniform
+    const LinearSet &s = sets.set[i];
+    if (i > 0) lds_barrier();                                 // nobody reads the last set's parts any more
+    split_product<TM, TN, false, true, FLUSH>(lds, rows(s), s.width, 0, 0, weight(s), K, k0, K, s.width, acc, [](const auto &) {});
+  }
+  store_product<TM, TN>(acc, y + n0 * K + k0, K, ms, K - k0 < TN ? K - k0 : TN, nullptr, [&](int m, int n) {
+    float sum = 0;
+    for (int i = 0; i < sets.n; ++i) {
+      const LinearSet &s = sets.set[i];
+      sum += plain_product<false, true>(rows(s), s.width, m, weight(s), K, k0 + n, s.width);
+    }
+    return sum;
+  });
 }
 
 struct LinearTiles { int o, k, parts, rows; };      // result tiles along O and K; parts of the rows, rows of a part
@@ -265,13 +297,15 @@ __global__ __launch_bounds__(256, 2) void linear_grad_part_kernel(
   const rsrc_t g_r = make_rsrc(g + (n_rows > 0 ? n0 * O : 0), (size_t)n_rows * O * 4);
   const rsrc_t x_r = make_rsrc(x + (n_rows > 0 ? n0 * K : 0), (size_t)n_rows * K * 4);
   f32x16 acc[2][2];
+  zero_sums(acc);
   float bias_sum = 0;                                       // of this thread's column and every other eight rows
   split_product<128, 128, true, true, 64>(lds, g_r, O, o0, O, x_r, K, k0, K, n_rows, acc, [&](const OpG &a) {
     const float *v = a.v[0];                                // a tree per batch: a chain of rows would round more
     bias_sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   });
   float *mine = partial + (size_t)part * ((size_t)O * K + O);
-  store_product<128, 128, true, true>(acc, g_r, O, o0, x_r, K, k0, n_rows, mine + (size_t)o0 * K + k0, K, O - o0, K - k0, nullptr);
+  store_product<128, 128>(acc, mine + (size_t)o0 * K + k0, K, O - o0, K - k0, nullptr,
+                          [&](int m, int n) { return plain_product<true, true>(g_r, O, o0 + m, x_r, K, k0 + n, n_rows); });
   if (want_bias && k0 == 0) {                               // uniform
     float *s_bias = reinterpret_cast<float *>(lds);
     lds_barrier();
@@ -305,24 +339,45 @@ __global__ __launch_bounds__(256) void linear_grad_sum_kernel(const float *__res
   }
 }
 
-template <int TM, int TN, bool B_ACROSS>
-static hipError_t launch_linear_cfg(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream) {
-  const long long groups = ((N + TM - 1) / TM + 7) / 8;
-  const int o_tiles = (O + TN - 1) / TN;
-  if (groups * 8 * o_tiles > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((linear_kernel<TM, TN, B_ACROSS>), dim3((unsigned)(groups * 8 * o_tiles)), dim3(256), 0, stream, x, w, bias, y, N, O, K, o_tiles);
+// Workgroups of TM x TN tiles, rows in groups of eight (one per XCD), or 0 where they are too many for a launch; `tiles`: of one row of them.
+template <int TM, int TN> static unsigned linear_blocks(long long N, int tiles) {
+  const long long blocks = ((N + TM - 1) / TM + 7) / 8 * 8 * tiles;
+  return blocks <= 0x7FFFFFFFLL ? (unsigned)blocks : 0u;
+}
+// 64 x 128 tiles where there are two of them per CU: 4096 rows of 256 x 256 (128) 14 us with them, 10 with 256 smaller ones; 22500 (704) 26, 27
+// and at least three quarters of them are result: the layer with 29000 rows of 256 to 128, 64 and 64 columns 297 us with them, 289 with 64 x 64.
+static bool wide_tiles(long long N, int width, int tiles128) { return 4LL * width >= 3LL * 128 * tiles128 && (N + 63) / 64 * tiles128 >= 512; }
+
+template <int TM, int TN> static hipError_t launch_linear_cfg(const float *x, const LinearSets &sets, long long N, int K, hipStream_t stream) {
+  int tiles = 0;
+  for (int i = 0; i < sets.n; ++i) tiles += (sets.set[i].width + TN - 1) / TN;
+  const unsigned blocks = linear_blocks<TM, TN>(N, tiles);
+  if (blocks == 0) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((linear_kernel<TM, TN>), dim3(blocks), dim3(256), 0, stream, x, sets, N, K, tiles);
   return hipGetLastError();
 }
 
-template <bool B_ACROSS>
-static hipError_t launch_linear_as(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream) {
-  // at least two workgroups per CU: 4096 rows of 256 x 256 (128 larger tiles) 14 us with them, 10 with 256 smaller ones; 22500 (704) 26, 27
-  if ((N + 63) / 64 * ((O + 127) / 128) < 512 || O <= 64) return launch_linear_cfg<64, 64, B_ACROSS>(x, w, bias, y, N, O, K, stream);
-  return launch_linear_cfg<64, 128, B_ACROSS>(x, w, bias, y, N, O, K, stream);
+hipError_t launch_linear(const float *x, const LinearSets &sets, long long N, int K, hipStream_t stream) {
+  int tiles128 = 0, width = 0;
+  for (int i = 0; i < sets.n; ++i) {
+    tiles128 += (sets.set[i].width + 127) / 128;
+    width += sets.set[i].width;
+  }
+  return wide_tiles(N, width, tiles128) ? launch_linear_cfg<64, 128>(x, sets, N, K, stream) : launch_linear_cfg<64, 64>(x, sets, N, K, stream);
 }
 
-hipError_t launch_linear(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, bool w_across, hipStream_t stream) {
-  return w_across ? launch_linear_as<true>(x, w, bias, y, N, O, K, stream) : launch_linear_as<false>(x, w, bias, y, N, O, K, stream);
+template <int TM, int TN, int FLUSH> static hipError_t launch_linear_sum_cfg(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream) {
+  const int tiles = (K + TN - 1) / TN;
+  const unsigned blocks = linear_blocks<TM, TN>(N, tiles);
+  if (blocks == 0) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((linear_sum_kernel<TM, TN, FLUSH>), dim3(blocks), dim3(256), 0, stream, sets, y, N, K, tiles);
+  return hipGetLastError();
+}
+
+hipError_t launch_linear_sum(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream) {
+  const bool wide = wide_tiles(N, K, (K + 127) / 128);
+  if (sets.n == 1) return wide ? launch_linear_sum_cfg<64, 128, 0>(sets, y, N, K, stream) : launch_linear_sum_cfg<64, 64, 0>(sets, y, N, K, stream);
+  return wide ? launch_linear_sum_cfg<64, 128, 128>(sets, y, N, K, stream) : launch_linear_sum_cfg<64, 64, 128>(sets, y, N, K, stream);
 }
 
 size_t linear_grad_workspace_bytes(long long N, int O, int K) {

@@ -20,7 +20,7 @@ from torch.autograd import Function
 from ..functional import (MultiScale3DDeformableAttnFunction_fp32,
                           MultiScale3DDeformableAttnWeightUpdateFunction_fp32)
 from .. import _lib
-from .projection import Projection, ordinary, plain_gradient
+from .projection import Projection, ordinary, plain_gradient, projections
 
 __all__ = ["MSDeformableAttention3D_DFA3D"]
 
@@ -134,22 +134,30 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         """Normalised (x, y, z) of every sampling point, (bs, Q, heads, L, points, 3): the head's learned
         offsets, divided by the level's (W, H, D), around the query's Z-anchor reference points
         (spatial_cross_attention.py:498-537).  Point p belongs to anchor p % num_Z_anchors."""
-        bs, Q, _ = query.shape
-        M, L, P = self.num_heads, self.num_levels, self.num_points
+        self._check_reference_points(reference_points)
+        return self._locations(*projections(query, (self.sampling_offsets, self.sampling_offsets_depth)), reference_points, spatial_shapes_3D,
+                               query.dtype)
+
+    def _check_reference_points(self, reference_points):
+        P, Z = self.num_points, reference_points.shape[2]
         if reference_points.shape[-1] != 3:
             raise ValueError("Last dim of reference_points must be 3 (x, y, depth), but get "
                              f"{reference_points.shape[-1]} instead.")
-        Z = reference_points.shape[2]
         if P % Z:
             raise ValueError(f"num_points ({P}) must be a multiple of the number of Z anchors ({Z})")
-        uv = self.sampling_offsets(query).view(bs, Q, M, L, P, 2)
-        dz = self.sampling_offsets_depth(query).view(bs, Q, M, L, P, 1)
+
+    def _locations(self, uv, dz, reference_points, spatial_shapes_3D, dtype):
+        """``sampling_locations`` from the two offset layers' results (bs, Q, ...)."""
+        bs, Q, _ = uv.shape
+        M, L, P = self.num_heads, self.num_levels, self.num_points
+        Z = reference_points.shape[2]
+        uv, dz = uv.view(bs, Q, M, L, P, 2), dz.view(bs, Q, M, L, P, 1)
         if (ordinary(uv, dz, reference_points) and uv.is_contiguous() and dz.is_contiguous()
                 and reference_points.is_contiguous() and not reference_points.requires_grad
                 and reference_points.shape[:2] == (bs, Q) and spatial_shapes_3D.device == uv.device
                 and spatial_shapes_3D.dtype == torch.int64 and spatial_shapes_3D.shape == (L, 3)):
             return _LocationsFunction.apply(uv, dz, reference_points, spatial_shapes_3D.contiguous())
-        normalizer = spatial_shapes_3D[:, [1, 0, 2]].to(query.dtype)              # (W, H, D) per level
+        normalizer = spatial_shapes_3D[:, [1, 0, 2]].to(dtype)              # (W, H, D) per level
         offsets = torch.cat([uv, dz], dim=-1) / normalizer[None, None, None, :, None, :]
         anchors = reference_points[:, :, None, None, None, :, :]                   # (bs, Q, 1, 1, 1, Z, 3)
         loc = offsets.view(bs, Q, M, L, P // Z, Z, 3) + anchors
@@ -179,17 +187,26 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         if value_dpt_dist is None or value_dpt_dist.dim() != 3 or value_dpt_dist.shape[:2] != value.shape[:2]:
             raise ValueError("value_dpt_dist must be (bs, num_value, D)")
 
+        # the largest launches first: the GPU works on them while the host prepares the others
+        together = getattr(self.sampling_locations, "__func__", None) is MSDeformableAttention3D_DFA3D.sampling_locations
+        if together:
+            self._check_reference_points(reference_points)
+            uv, dz, attention_weights = projections(query, (self.sampling_offsets, self.sampling_offsets_depth, self.attention_weights))
+        else:
+            attention_weights = self.attention_weights(query)
         value = self.value_proj(value)
         if key_padding_mask is not None:
             value = value.masked_fill(key_padding_mask[..., None], 0.0)
         value = value.view(bs, num_value, self.num_heads, -1)
+        attention_weights = attention_weights.view(bs, num_query, self.num_heads, self.num_levels * self.num_points).softmax(-1)
+        attention_weights = attention_weights.view(bs, num_query, self.num_heads, self.num_levels, self.num_points)
         dim_depth = value_dpt_dist.shape[2]
         dist = value_dpt_dist.reshape(bs, num_value, 1, dim_depth).to(value.dtype)
-        attention_weights = self.attention_weights(query).view(
-            bs, num_query, self.num_heads, self.num_levels * self.num_points).softmax(-1)
-        attention_weights = attention_weights.view(bs, num_query, self.num_heads, self.num_levels, self.num_points)
         spatial_shapes_3D = self.get_spatial_shape_3D(spatial_shapes, dim_depth)
-        sampling_locations = self.sampling_locations(query, reference_points, spatial_shapes_3D)
+        if together:
+            sampling_locations = self._locations(uv, dz, reference_points, spatial_shapes_3D, query.dtype)
+        else:
+            sampling_locations = self.sampling_locations(query, reference_points, spatial_shapes_3D)
 
         if not value.is_cuda:
             raise NotImplementedError("the DFA3D operator runs on the GPU only")

@@ -6,10 +6,11 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 from torch.autograd import Function
+from torch.nn.modules import module as _module
 
 from .. import _lib
 
-__all__ = ["Projection"]
+__all__ = ["Projection", "projections"]
 
 
 def ordinary(*tensors):
@@ -22,6 +23,8 @@ def ordinary(*tensors):
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0)
 
+
+_MAX_SHARED = 4        # layers that one launch takes (kMaxLinearSets)
 
 # Fewer rows than this: the library product is as fast and there is one launch less.
 _MIN_ROWS = 4096
@@ -37,33 +40,27 @@ def _widths_apply(O, K):
     return O % 2 == 0 and K % 2 == 0 and max(O, K) <= 2048 and O * K <= 2 ** 20
 
 
-def _product_applies(rows, width, depth):
-    """Where the kernel forms a product of ``rows`` x ``width`` elements, sums of ``depth`` terms.  It reads four neighbours of a
-    row at a time, and takes the library's place except where few rows meet a deep sum: library and kernel, us, 4096 rows
-    of 256 by 256 19, 10; 256 by 64 19, 7; sums of 512 by 256 19, 22; of 2048 by 256 41, 51 to 89; of 1024 by 1024 72, 59; 20000 rows of 512 by
-    512 98, 70; of 2048 by 256 165, 145; 100000 of 256 by 256 123, 93."""
-    return width % 2 == 0 and depth % 4 == 0 and 0 < max(width, depth) <= 4096 and 0 < rows <= 2 ** 31 and \
-        (depth <= 256 or rows * width >= 2 ** 22)
+def _products(x, params):
+    """``F.linear`` of every (weight, bias or None) of the flat tuple in one launch, none of it recorded; None where the kernel does not form
+    them (csrc/dfa3d_binding.cpp says where it does) or they are to be recorded."""
+    if not x.is_cuda or torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
+        return None
+    at = torch._C._cuda_getDevice()
+    return _lib.binding().linear(at, torch._C._cuda_getCurrentRawStream(at), x, params)
 
 
-def _product(x, weight, bias, across):
-    """x (..., K) times weight (O, K) transposed, or (``across``) weight (K, O), plus the bias; contiguous float32 operands."""
-    O = weight.shape[1] if across else weight.shape[0]
-    K = x.shape[-1]
-    y = torch.empty(*x.shape[:-1], O, dtype=torch.float32, device=x.device)
-    with _lib.on_device(x.device):
-        rc = _lib.lib().dfa3d_linear(_lib.ptr(x), _lib.ptr(weight), _lib.ptr(bias), _lib.ptr(y), x.numel() // K, O, K, int(across),
-                                     _lib.stream_of(x))
-    _lib.check(rc, "dfa3d_linear")
-    return y
+def _sum_of_products(operands):
+    """Sum of rows (..., O) times weight (O, K) over the flat tuple of them, or None as above."""
+    if not operands[0].is_cuda:
+        return None
+    at = torch._C._cuda_getDevice()
+    return _lib.binding().linear_sum(at, torch._C._cuda_getCurrentRawStream(at), operands)
 
 
 def _linear(x, weight, bias):
-    """``F.linear`` outside autograd."""
-    if (x.is_cuda and x.is_contiguous() and weight.is_contiguous() and x.shape[-1:] == weight.shape[1:]
-            and (bias is None or (bias.is_contiguous() and bias.shape == weight.shape[:1])) and _product_applies(x.numel() // max(x.shape[-1], 1), *weight.shape)):
-        return _product(x, weight, bias, False)
-    return F.linear(x, weight, bias)
+    """``F.linear``, by the kernel where nothing records it."""
+    got = _products(x, (weight, bias))
+    return F.linear(x, weight, bias) if got is None else got[0]
 
 
 def _weight_gradients(x, grad, want_bias):
@@ -85,7 +82,7 @@ def _weight_gradients(x, grad, want_bias):
 def plain_gradient(grad):
     """A gradient that a kernel may read: float32 on the GPU, not recorded and not a batch of gradients (is_grads_batched)."""
     return (not torch.is_grad_enabled() and grad.is_cuda and grad.dtype == torch.float32
-            and torch._C._len_torch_dispatch_stack() == 0 and not grad.is_neg()
+            and torch._C._len_torch_dispatch_stack() == 0 and torch.autograd.forward_ad._current_level < 0 and not grad.is_neg()
             and not torch._C._functorch.is_batchedtensor(grad) and not torch._C._functorch.is_legacy_batchedtensor(grad))
 
 
@@ -109,36 +106,68 @@ class _ProjectionFunction(Function):
     def backward(ctx, grad):
         x, weight = ctx.saved_tensors
         want_x, want_weight, want_bias = ctx.needs_input_grad[:3]
-        plain = plain_gradient(grad)
-        if plain:
+        if plain_gradient(grad):
             grad = grad.contiguous()
-        grad_x = None
-        if want_x:
-            if plain and _as_plain(weight, grad) and _product_applies(grad.numel() // max(grad.shape[-1], 1), weight.shape[1], weight.shape[0]):
-                grad_x = _product(grad, weight, None, True)
-            else:
-                grad_x = grad.matmul(weight)
-        grad_rows = grad.reshape(-1, grad.shape[-1])
-        if not want_weight:
-            return grad_x, None, grad_rows.sum(0) if want_bias else None, None
-        rows = x.reshape(-1, x.shape[-1]).contiguous()
-        if not (plain and _as_plain(rows, grad)):
-            return grad_x, grad_rows.t().mm(rows), grad_rows.sum(0) if want_bias else None, None
-        return (grad_x, *_weight_gradients(rows, grad_rows, want_bias), None)
+        return (_input_gradient([grad], [weight]) if want_x else None, *_layer_gradients(x, grad, want_weight, want_bias), None)
 
 
-def _applies(x, weight, bias):
-    """Float32 rows on the GPU in ordinary reverse-mode training."""
-    return (not torch.compiler.is_compiling() and bias is not None and torch.is_grad_enabled() and weight.requires_grad
-            and x.dim() >= 2 and _widths_apply(*weight.shape)
-            and _MIN_ROWS <= x.numel() // max(x.shape[-1], 1) <= 2 ** 31 and ordinary(x, weight, bias))
+def _input_gradient(grads, weights):
+    """Gradient of the rows that several layers share, from the gradients of what they gave."""
+    if all(plain_gradient(g) for g in grads):
+        got = _sum_of_products(tuple(t for pair in zip(grads, weights) for t in pair))
+        if got is not None:
+            return got
+    total = grads[0].matmul(weights[0])
+    for g, w in zip(grads[1:], weights[1:]):
+        total = total + g.matmul(w)
+    return total
 
 
-def _no_gradient(x, weight, bias):
-    """Float32 rows on the GPU that nothing records."""
-    operands = (x, weight) if bias is None else (x, weight, bias)
-    return (not torch.compiler.is_compiling() and x.is_cuda and not (torch.is_grad_enabled() and any(t.requires_grad for t in operands))
-            and x.dim() >= 2 and ordinary(*operands))
+def _layer_gradients(x, grad, want_weight, want_bias):
+    """Gradients of a layer's weight and bias from its rows x and the gradient of its result."""
+    grad_rows = grad.reshape(-1, grad.shape[-1])
+    if not want_weight:
+        return None, grad_rows.sum(0) if want_bias else None
+    rows = x.reshape(-1, x.shape[-1]).contiguous()
+    if not (plain_gradient(grad) and _as_plain(rows, grad)):
+        return grad_rows.t().mm(rows), grad_rows.sum(0) if want_bias else None
+    return _weight_gradients(rows, grad_rows.contiguous(), want_bias)
+
+
+class _SharedRowsFunction(Function):
+    """``F.linear(x, weight, bias)`` of several layers (weight, bias, weight, bias, ...) on the same rows; ``library`` says whose forward is
+    the library's.  The gradient of the rows is formed in one kernel instead of one product per layer and the sums of their results."""
+
+    @staticmethod
+    def forward(ctx, library, x, *params):
+        weights, biases = params[::2], params[1::2]
+        ctx.set_materialize_grads(False)
+        want_x, *wanted = ctx.needs_input_grad[1:]
+        ctx.save_for_backward(x if any(wanted[::2]) else None, *(w if want_x else None for w in weights))
+        own = [i for i, lib in enumerate(library) if not lib]
+        made = _products(x, tuple(t for i in own for t in (weights[i], biases[i]))) if own else None
+        made = dict(zip(own, made)) if made is not None else {}
+        return tuple(made[i] if i in made else F.linear(x, weights[i], biases[i]) for i in range(len(weights)))
+
+    @staticmethod
+    def backward(ctx, *grads):
+        x, *weights = ctx.saved_tensors
+        want_x, *wanted = ctx.needs_input_grad[1:]
+        grads = [g.contiguous() if g is not None and plain_gradient(g) else g for g in grads]
+        there = [i for i, g in enumerate(grads) if g is not None]
+        grad_x = _input_gradient([grads[i] for i in there], [weights[i] for i in there]) if want_x and there else None
+        out = []
+        for i, g in enumerate(grads):
+            out += (None, None) if g is None else _layer_gradients(x, g, *wanted[2 * i:2 * i + 2])
+        return (None, grad_x, *out)
+
+
+def _applies(x, *layers):
+    """Float32 rows on the GPU in ordinary reverse-mode training, for layers that all have a bias."""
+    return (not torch.compiler.is_compiling() and torch.is_grad_enabled() and x.dim() >= 2
+            and _MIN_ROWS <= x.numel() // max(x.shape[-1], 1) <= 2 ** 31
+            and all(l.bias is not None and l.weight.requires_grad and _widths_apply(*l.weight.shape) for l in layers)
+            and ordinary(x, *(t for l in layers for t in (l.weight, l.bias))))
 
 
 class Projection(nn.Linear):
@@ -155,8 +184,26 @@ class Projection(nn.Linear):
         self.library_forward = library_forward
 
     def forward(self, input):
-        if _applies(input, self.weight, self.bias):
+        if _applies(input, self):
             return _ProjectionFunction.apply(input, self.weight, self.bias, self.library_forward)
-        if _no_gradient(input, self.weight, self.bias):
-            return _linear(input, self.weight, self.bias)
-        return F.linear(input, self.weight, self.bias)
+        return _linear(input, self.weight, self.bias)
+
+
+def _bare(layer):
+    """A Projection whose call is its ``forward`` and nothing else."""
+    return (type(layer) is Projection and "forward" not in layer.__dict__
+            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks
+                     or _module._global_forward_hooks or _module._global_forward_pre_hooks
+                     or _module._global_backward_hooks or _module._global_backward_pre_hooks))
+
+
+def projections(x, layers):
+    """``[layer(x) for layer in layers]`` in fewer launches where the layers are plain ``Projection``s, at most four.
+    The layer of the base model, training: 3811 -> 3771 us; of the small one, inference: 293 -> 261."""
+    if len(layers) <= _MAX_SHARED and all(_bare(l) for l in layers):
+        if _applies(x, *layers):
+            return list(_SharedRowsFunction.apply(tuple(l.library_forward for l in layers), x, *(t for l in layers for t in (l.weight, l.bias))))
+        got = _products(x, tuple(t for l in layers for t in (l.weight, l.bias)))
+        if got is not None:
+            return list(got)
+    return [layer(x) for layer in layers]

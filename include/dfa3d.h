@@ -264,10 +264,18 @@ int dfa3d_locations(const float *uv, const float *dz, const float *ref, const in
 int dfa3d_locations_grad(const float *grad_loc, const int64_t *shapes3, float *grad_uv, float *grad_dz, long long rows, int M, int L,
                          int P, void *stream);
 
-/* A linear layer in float32: y (N, O) = x (N, K) weight^T + bias, weight (O, K) row-major, or (K, O) when weight_across is not 0 (the gradient
- * of x from that of y); bias (O) or NULL.  O even, K a multiple of four, every element written, the same result every time. */
-int dfa3d_linear(const float *x, const float *weight, const float *bias, float *y, long long N, int O, int K, int weight_across,
-                 void *stream);
+/* Up to four linear layers on the same rows in float32, all matrices row-major:
+ *   dfa3d_linear      rows (N, width) = x (N, K) weight (width, K)^T + bias (width) or NULL, of every layer
+ *   dfa3d_linear_sum  y (N, K) = sum over the layers of rows (N, width) weight (width, K): the gradient of x from those of the rows
+ * K and widths even; K (the first), widths (the second) multiples of four.  Every element written, the same result every time. */
+typedef struct dfa3d_linear_set {
+  const float *weight;
+  const float *bias;
+  float *rows;            /* read only by dfa3d_linear_sum */
+  int width;
+} dfa3d_linear_set;
+int dfa3d_linear(const float *x, const dfa3d_linear_set *layers, int n_layers, long long N, int K, void *stream);
+int dfa3d_linear_sum(const dfa3d_linear_set *layers, int n_layers, float *y, long long N, int K, void *stream);
 
 /* Weight and bias gradients of a linear layer y = x weight^T + bias in float32: grad_weight (O, K) = grad_out^T x,
  * grad_bias (O) = column sums of grad_out, or not formed when it is NULL; x (N, K) and grad_out (N, O) row-major, O and K

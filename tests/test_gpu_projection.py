@@ -30,23 +30,22 @@ def test_weight_and_bias_gradients(N, K, O):
     assert torch.equal(again[0], got[1]) and torch.equal(again[1], got[2])      # fixed order of summation
 
 
-@pytest.mark.parametrize("N,K,O", [(1, 4, 2), (63, 36, 62), (64, 16, 64), (65, 20, 66), (130, 256, 130), (4097, 12, 128), (16385, 48, 256),
-                                   (20001, 256, 258), (33000, 8, 64)])
+@pytest.mark.parametrize("N,K,O", [(1, 4, 4), (63, 36, 64), (64, 16, 64), (65, 20, 68), (130, 256, 132), (4097, 12, 128), (16385, 48, 256),
+                                   (20001, 256, 260), (33000, 8, 64)])
 @pytest.mark.parametrize("across", [False, True])
 def test_product(N, K, O, across):
     from dfa3D.modules import projection
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(N + K + O)
     x, w, b = (torch.randn(*s, generator=g, device=dev) for s in ((N, K), (O, K), (O,)))
-    assert projection._product_applies(N, O, K)
-    got = projection._product(x, w.t().contiguous() if across else w, None if across else b, across)
+    product = lambda: projection._sum_of_products((x, w.t().contiguous())) if across else projection._products(x, (w, b))[0]
+    got = product()
     xd, wd, bd = x.double(), w.double(), torch.zeros_like(b).double() if across else b.double()
     # three parts hold all of a float32; what is left out is 2^-25 of a product at most, and each of K / 16 steps of six sums, and the bias,
     # is rounded (or cut) to 2^-23 of the running sum, at most the sum of the sizes
     bound = (2.0 ** -25 + (6 * (K // 16 + 1) + 16 + 1) * 2.0 ** -23) * (xd.abs() @ wd.abs().t() + bd.abs())
     assert ((got.double() - (xd @ wd.t() + bd)).abs() <= bound).all()
-    again = projection._product(x, w.t().contiguous() if across else w, None if across else b, across)
-    assert torch.equal(got, again)
+    assert torch.equal(got, product())
 
 
 def test_operands_that_are_no_ordinary_numbers():
@@ -58,17 +57,65 @@ def test_operands_that_are_no_ordinary_numbers():
     w[:, 1] = 0.5
     x[3, 5], x[7, 9], x[200, 1], x[201, 1] = float("inf"), float("nan"), 3.402823e38, -3.402823e38
     x[50] *= 1e-34
-    got, want = projection._product(x, w, b, False), torch.nn.functional.linear(x, w, b)
+    got, want = projection._products(x, (w, b))[0], torch.nn.functional.linear(x, w, b)
     torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-4, equal_nan=True)
-    tiny = projection._product(x[50:51], w, None, False).double()
+    tiny = projection._products(x[50:51], (w, None))[0].double()
     torch.testing.assert_close(tiny, x[50:51].double() @ w.double().t(), rtol=0, atol=64 * 2.0 ** -23 * 1e-34 * 16)
-    across = projection._product(x, w.t().contiguous(), None, True)
+    across = projection._sum_of_products((x, w.t().contiguous()))
     torch.testing.assert_close(across, x.matmul(w.t()), rtol=1e-5, atol=1e-4, equal_nan=True)
     g = torch.randn(4200, 96, device=dev)
     g[9, 3], g[11, 6], x[11, 4], x[7, 9], x[3, 5] = float("inf"), 3.402823e38, 1.5, 0., 0.
     x[200:202] = 0
     gw, _ = projection._weight_gradients(x, g, True)
     torch.testing.assert_close(gw, g.t().mm(x), rtol=1e-4, atol=1e-2, equal_nan=True)
+
+
+@pytest.mark.parametrize("N,K,widths", [(4097, 64, (64,)), (5000, 36, (128, 66)), (4160, 256, (128, 64, 64)), (33001, 20, (4, 200, 72, 8))])
+@pytest.mark.parametrize("train", [False, True])
+def test_several_layers_on_the_same_rows(N, K, widths, train):
+    from dfa3D.modules.projection import Projection, projections
+    dev = torch.device("cuda:0")
+    torch.manual_seed(N)
+    layers = [Projection(K, O, library_forward=i == 1).to(dev) for i, O in enumerate(widths)]
+    x = torch.randn(N, K, device=dev, requires_grad=train)
+    gs = [torch.randn(N, O, device=dev) for O in widths]
+    with torch.set_grad_enabled(train):
+        got = projections(x, layers)
+    xd = x.detach().double()
+    for y, l in zip(got, layers):
+        bound = (6 * (K // 16 + 1) + 18) * 2.0 ** -23 * (xd.abs() @ l.weight.detach().double().abs().t() + l.bias.detach().double().abs())
+        assert ((y.detach().double() - (xd @ l.weight.detach().double().t() + l.bias.detach().double())).abs() <= bound).all()
+    if not train:
+        return
+    params = [p for l in layers for p in (l.weight, l.bias)]
+    grads = torch.autograd.grad(got, [x] + params, gs, retain_graph=True)
+    want = sum(g.double() @ l.weight.detach().double() for g, l in zip(gs, layers))
+    size = sum(g.double().abs() @ l.weight.detach().double().abs() for g, l in zip(gs, layers))
+    # sums of at most 128 terms by the matrix unit, the rest to nearest (library products where a width is no multiple of four)
+    assert ((grads[0].double() - want).abs() <= (6 * 9 + 18 + 2 * len(widths)) * 2.0 ** -23 * size).all()
+    for i, (g, l) in enumerate(zip(gs, layers)):
+        gw, gb = torch.autograd.grad(l(x), [l.weight, l.bias], g)
+        assert torch.equal(grads[1 + 2 * i], gw) and torch.equal(grads[2 + 2 * i], gb)
+    # one result's gradient alone; rows that want none; gradients of gradients
+    gx, gw = torch.autograd.grad(got[-1], [x, layers[-1].weight], gs[-1], retain_graph=True)
+    assert torch.equal(gw, grads[1 + 2 * (len(widths) - 1)])
+    torch.testing.assert_close(gx.double(), gs[-1].double() @ layers[-1].weight.detach().double(), rtol=1e-4, atol=1e-4)
+    gw, = torch.autograd.grad(projections(x.detach(), layers)[0], [layers[0].weight], gs[0])
+    assert torch.equal(gw, grads[1])
+    gw, = torch.autograd.grad(sum(y.square().sum() for y in got), [layers[0].weight], create_graph=True)
+    assert torch.autograd.grad(gw.square().sum(), [x])[0].isfinite().all()
+
+
+def test_layers_with_hooks_are_called():
+    from dfa3D.modules.projection import Projection, projections
+    dev = torch.device("cuda:0")
+    layers = [Projection(64, 64).to(dev) for _ in range(2)]
+    seen = []
+    layers[1].register_forward_hook(lambda m, i, o: seen.append(o))
+    x = torch.randn(5000, 64, device=dev)
+    with torch.no_grad():
+        got = projections(x, layers)
+    assert len(seen) == 1 and seen[0] is got[1]
 
 
 def test_offsets_keep_the_librarys_result_in_training():
@@ -115,5 +162,14 @@ def test_calls_that_keep_the_librarys_operation():
     torch.testing.assert_close(tangent, torch.ones_like(x) @ layer.weight.detach().t(), rtol=1e-4, atol=1e-4)
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert layer(x).dtype == torch.bfloat16
+    w, b = layer.weight.detach(), layer.bias.detach()
+    x = x.detach()
+    from dfa3D.modules.projection import _products
+    assert _products(x, (w, b)) is not None
+    for args in ((x, (layer.weight, b)), (x.double(), (w, b)), (x.t(), (w, b)), (x, (w, b[:-1])), (x[:, :-2].contiguous(), (w, b)), (x[0], (w, b)),
+                 (x, (w[:-1].contiguous(), None)), (x, (w.t(), None)), (x, ()), (x, (w, None) * 5), (torch._neg_view(x), (w, b)), (x[:0], (w, b))):
+        assert _products(*args) is None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert _products(x, (w, b)) is None
     few = torch.randn(7, 64, device=dev)
     torch.autograd.grad(layer(few).sum(), [layer.weight])
