@@ -527,36 +527,28 @@ static int check_linear(const char *fn, long long N, int O, int K) {
   return 0;
 }
 
-static int linear_sets(const char *fn, const dfa3d_linear_set *from, int n, long long N, int K, dfa3d::LinearSets &to) {
-  if (n < 1 || n > dfa3d::kMaxLinearSets) return fail(DFA3D_EINVAL, "%s: 1 to %d layers (%d)", fn, dfa3d::kMaxLinearSets, n);
-  REQUIRE_PTR(fn, from);
-  to = dfa3d::LinearSets{};
-  to.n = n;
-  for (int i = 0; i < n; ++i) {
-    if (int rc = check_linear(fn, N, from[i].width, K)) return rc;
-    REQUIRE_PTR(fn, from[i].weight); REQUIRE_PTR(fn, from[i].rows);
-    to.set[i] = dfa3d::LinearSet{from[i].weight, from[i].bias, from[i].rows, from[i].width};
-  }
-  return 0;
-}
-
-int dfa3d_linear(const float *x, const dfa3d_linear_set *sets, int n_sets, long long N, int K, void *stream) {
+int dfa3d_linear(const float *x, const float *weight, const float *bias, float *y, long long N, int O, int K, void *stream) {
   const char *fn = "dfa3d_linear";
-  dfa3d::LinearSets to;
-  if (int rc = linear_sets(fn, sets, n_sets, N, K, to)) return rc;
+  if (int rc = check_linear(fn, N, O, K)) return rc;
   if ((K & 3) != 0) return fail(DFA3D_EINVAL, "%s: K must be a multiple of four (K=%d)", fn, K);
-  REQUIRE_PTR(fn, x);
-  return hip_result(dfa3d::launch_linear(x, to, N, K, (hipStream_t)stream), fn);
+  REQUIRE_PTR(fn, x); REQUIRE_PTR(fn, weight); REQUIRE_PTR(fn, y);
+  return hip_result(dfa3d::launch_linear(x, weight, bias, y, N, O, K, (hipStream_t)stream), fn);
 }
 
-int dfa3d_linear_sum(const dfa3d_linear_set *sets, int n_sets, float *y, long long N, int K, void *stream) {
+int dfa3d_linear_sum(const dfa3d_linear_set *layers, int n_layers, float *y, long long N, int K, void *stream) {
   const char *fn = "dfa3d_linear_sum";
-  dfa3d::LinearSets to;
-  if (int rc = linear_sets(fn, sets, n_sets, N, K, to)) return rc;
-  for (int i = 0; i < n_sets; ++i)
-    if ((sets[i].width & 3) != 0) return fail(DFA3D_EINVAL, "%s: widths must be multiples of four (%d)", fn, sets[i].width);
-  REQUIRE_PTR(fn, y);
-  return hip_result(dfa3d::launch_linear_sum(to, y, N, K, (hipStream_t)stream), fn);
+  if (n_layers < 1 || n_layers > dfa3d::kMaxLinearSets) return fail(DFA3D_EINVAL, "%s: 1 to %d layers (%d)", fn, dfa3d::kMaxLinearSets, n_layers);
+  REQUIRE_PTR(fn, layers); REQUIRE_PTR(fn, y);
+  dfa3d::LinearSets sets{};
+  sets.n = n_layers;
+  for (int i = 0; i < n_layers; ++i) {
+    const dfa3d_linear_set &l = layers[i];
+    if (int rc = check_linear(fn, N, l.width, K)) return rc;
+    if ((l.width & 3) != 0) return fail(DFA3D_EINVAL, "%s: widths must be multiples of four (%d)", fn, l.width);
+    REQUIRE_PTR(fn, l.weight); REQUIRE_PTR(fn, l.rows);
+    sets.set[i] = dfa3d::LinearSet{l.weight, l.rows, l.width};
+  }
+  return hip_result(dfa3d::launch_linear_sum(sets, y, N, K, (hipStream_t)stream), fn);
 }
 
 size_t dfa3d_linear_grad_workspace_bytes(long long N, int O, int K) {

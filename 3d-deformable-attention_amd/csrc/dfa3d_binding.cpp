@@ -368,40 +368,28 @@ Py_ssize_t pairs_of(PyObject *o) {
 bool is_float_matrix(const Tensor &t) { return t.scalar_type() == at::kFloat && t.dim() == 2; }
 bool recorded(const Tensor &t) { return t.defined() && t.requires_grad() && c10::GradMode::is_enabled(); }
 
-// linear(device, stream, x (..., K), (weight (O, K), bias (O) or None, ...)) -> F.linear of every layer, none of it recorded, or None
+// linear(device, stream, x (..., K), weight (O, K), bias (O) or None) -> F.linear, not recorded, or None
 PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  TAKES(4)
-  const Tensor &x = in.need(args[2]);
-  const Py_ssize_t n = pairs_of(args[3]);
-  if (!in.ok || n == 0 || x.scalar_type() != at::kFloat || x.dim() < 2 || x.size(-1) == 0 || recorded(x) ||
+  TAKES(5)
+  const Tensor &x = in.need(args[2]), &w = in.need(args[3]), &b = in.may_have(args[4]);
+  if (!in.ok || x.scalar_type() != at::kFloat || x.dim() < 2 || !is_float_matrix(w) || x.size(-1) != w.size(1) || w.size(1) == 0 ||
+      (b.defined() && (b.scalar_type() != at::kFloat || !shape_is(b, {w.size(0)}))) || recorded(x) || recorded(w) || recorded(b) ||
       at::autocast::is_autocast_enabled(at::kCUDA) || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer))
     return declined();
-  const int64_t K = x.size(-1), rows = x.numel() / K;
-  dfa3d_linear_set sets[kMaxSets];
-  Tensor out[kMaxSets];
-  for (Py_ssize_t i = 0; i < n; ++i) {
-    const Tensor &w = in.need(PyTuple_GET_ITEM(args[3], 2 * i)), &b = in.may_have(PyTuple_GET_ITEM(args[3], 2 * i + 1));
-    if (!in.ok || !is_float_matrix(w) || w.size(1) != K || recorded(w) || recorded(b) || !product_applies(rows, w.size(0), K) ||
-        (b.defined() && (b.scalar_type() != at::kFloat || !shape_is(b, {w.size(0)}))))
-      return declined();
-    sets[i] = dfa3d_linear_set{static_cast<const float *>(ptr(w)), static_cast<const float *>(ptr(b)), nullptr, static_cast<int>(w.size(0))};
-  }
+  const int64_t O = w.size(0), K = w.size(1), rows = x.numel() / K;
+  if (!product_applies(rows, O, K)) return declined();
   auto sizes = x.sizes().vec();
-  for (Py_ssize_t i = 0; i < n; ++i) {
-    sizes.back() = sets[i].width;
-    out[i] = at::empty(sizes, x.options());
-    sets[i].rows = static_cast<float *>(ptr(out[i]));
-  }
+  sizes.back() = O;
+  Tensor y = at::empty(sizes, x.options());
   int rc;
   {
     NoGil no_gil;
-    rc = api.linear(static_cast<const float *>(ptr(x)), sets, (int)n, rows, (int)K, stream);
+    rc = api.linear(static_cast<const float *>(ptr(x)), static_cast<const float *>(ptr(w)), static_cast<const float *>(ptr(b)),
+                    static_cast<float *>(ptr(y)), rows, (int)O, (int)K, stream);
   }
   if (rc != 0) return failed("dfa3d_linear", rc);
-  PyObject *all = PyTuple_New(n);
-  for (Py_ssize_t i = 0; all != nullptr && i < n; ++i) PyTuple_SET_ITEM(all, i, THPVariable_Wrap(out[i]));
-  return all;
+  return THPVariable_Wrap(y);
   END_HANDLE_TH_ERRORS
 }
 
@@ -423,7 +411,7 @@ PyObject *linear_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     shape.back() = w.size(1);
     if (i == 0) { sizes = shape; K = w.size(1); rows = g.numel() / w.size(0); }
     if (shape != sizes || !product_applies(rows, K, w.size(0))) return declined();
-    sets[i] = dfa3d_linear_set{static_cast<const float *>(ptr(w)), nullptr, static_cast<float *>(ptr(g)), static_cast<int>(w.size(0))};
+    sets[i] = dfa3d_linear_set{static_cast<const float *>(ptr(w)), static_cast<const float *>(ptr(g)), static_cast<int>(w.size(0))};
   }
   Tensor y = at::empty(sizes, THPVariable_Unpack(PyTuple_GET_ITEM(args[2], 0)).options());
   int rc;

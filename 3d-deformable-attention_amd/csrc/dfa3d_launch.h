@@ -157,12 +157,12 @@ hipError_t launch_locations(const float *uv, const float *dz, const float *ref, 
 hipError_t launch_locations_grad(const float *grad_loc, const int64_t *shapes3, float *grad_uv, float *grad_dz, long long rows,
                                  int M, int L, int P, hipStream_t stream);
 
-// Linear layers on the same rows (dfa3d_linear.hip): rows = x weight^T + bias (or nullptr) of each set, and y = sum of rows weight over them; K and
-// widths even, K (widths) a multiple of four in the first (second).
+// Linear layers (dfa3d_linear.hip): y (N, O) = x (N, K) w (O, K)^T + bias (or nullptr), and y (N, K) = sum over the sets of rows (N, width) weight
+// (width, K); O, K and widths even, K (widths) a multiple of four in the first (second).
 constexpr int kMaxLinearSets = 4;
-struct LinearSet { const float *weight, *bias; float *rows; int width; };
+struct LinearSet { const float *weight, *rows; int width; };
 struct LinearSets { LinearSet set[kMaxLinearSets]; int n; };
-hipError_t launch_linear(const float *x, const LinearSets &sets, long long N, int K, hipStream_t stream);
+hipError_t launch_linear(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream);
 hipError_t launch_linear_sum(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream);
 // Weight and bias gradients of a linear layer (dfa3d_linear.hip); O and K even.
 size_t linear_grad_workspace_bytes(long long N, int O, int K);

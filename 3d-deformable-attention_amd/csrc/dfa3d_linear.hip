@@ -17,9 +17,8 @@
 //   * The result of a weight gradient is small and its contraction long: the rows are cut into parts, a workgroup forms one 128 x 128 tile of
 //     one part's product, and a second kernel adds the parts up in a fixed order.  Workgroups of one part differ by multiples of the
 //     number of parts (a multiple of 8), so they run on one XCD and share its L2.
-//   * Layers on the same rows go in one launch: 29000 rows of 256 to 128, 64 and 64 columns 20.6 + 13.8 + 13 us one by one, 34 together.  So
-//     does the gradient of those rows, whose sums are added up by the vector unit every 128 steps, as they run over all layers: 58000 rows of 256
-//     from 512, 256 and 256 columns 200 us for three products and 48 for their sums, 185 together.
+//   * The gradient of rows that several layers share is formed in one launch; its sums are added up by the vector unit every 128 steps, as they
+//     run over all layers: 58000 rows of 256 from 512, 256 and 256 columns 200 us for three products and 48 for their sums, 185 together.
 //   * Rows beyond the end and columns beyond O or K read as zero (buffer range check).
 //
 // Library (forward and grad_x) or the float32 matrix instructions before (weight gradient), and now, us, between other kernels: 184950 rows of
@@ -225,22 +224,19 @@ __device__ __forceinline__ void store_product(const f32x16 (&acc)[TM / 64][TN / 
   }
 }
 
-// Up to kMaxLinearSets layers on the same rows x (N, K): rows (N, width) = x weight (width, K)^T + bias of each.  TM rows of one tile of TN columns
-// per workgroup; those of the same rows run on one XCD.
+// y (N, O) = x (N, K) w (O, K)^T + bias.  TM rows of one tile of TN columns per workgroup; those of the same rows run on one XCD.
 template <int TM, int TN>
-__global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict__ x, LinearSets sets, long long N, int K, int tiles) {
+__global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
+                                                        float *__restrict__ y, long long N, int O, int K, int tiles) {
   __shared__ __align__(16) unsigned char lds[2 * (SplitOperand<TM, false>::kBytes + SplitOperand<TN, false>::kBytes)];
   const long long n0 = (blockIdx.x / (8 * tiles) * 8 + blockIdx.x % 8) * (long long)TM;
   if (n0 >= N) return;                                        // uniform
-  int o0 = blockIdx.x % (8 * tiles) / 8 * TN, i = 0;
-  for (int wide = (sets.set[0].width + TN - 1) / TN * TN; o0 >= wide; wide = (sets.set[i].width + TN - 1) / TN * TN) { o0 -= wide; ++i; }     // uniform
-  const LinearSet set = sets.set[i];
-  const int ms = N - n0 < TM ? (int)(N - n0) : TM, ns = set.width - o0 < TN ? set.width - o0 : TN;
-  const rsrc_t x_r = make_rsrc(x + n0 * K, (size_t)ms * K * 4), w_r = make_rsrc(set.weight + (size_t)o0 * K, (size_t)ns * K * 4);
+  const int o0 = blockIdx.x % (8 * tiles) / 8 * TN, ms = N - n0 < TM ? (int)(N - n0) : TM, ns = O - o0 < TN ? O - o0 : TN;
+  const rsrc_t x_r = make_rsrc(x + n0 * K, (size_t)ms * K * 4), w_r = make_rsrc(w + (size_t)o0 * K, (size_t)ns * K * 4);
   f32x16 acc[TM / 64][TN / 64];
   zero_sums(acc);
   split_product<TM, TN, false, false, 0>(lds, x_r, K, 0, 0, w_r, K, 0, 0, K, acc, [](const auto &) {});
-  store_product<TM, TN>(acc, set.rows + n0 * set.width + o0, set.width, ms, ns, set.bias != nullptr ? set.bias + o0 : nullptr,
+  store_product<TM, TN>(acc, y + n0 * O + o0, O, ms, ns, bias != nullptr ? bias + o0 : nullptr,
                         [&](int m, int n) { return plain_product<false, false>(x_r, K, m, w_r, K, n, K); });
 }
 
@@ -345,25 +341,19 @@ template <int TM, int TN> static unsigned linear_blocks(long long N, int tiles) 
   return blocks <= 0x7FFFFFFFLL ? (unsigned)blocks : 0u;
 }
 // 64 x 128 tiles where there are two of them per CU: 4096 rows of 256 x 256 (128) 14 us with them, 10 with 256 smaller ones; 22500 (704) 26, 27
-// and at least three quarters of them are result: the layer with 29000 rows of 256 to 128, 64 and 64 columns 297 us with them, 289 with 64 x 64.
-static bool wide_tiles(long long N, int width, int tiles128) { return 4LL * width >= 3LL * 128 * tiles128 && (N + 63) / 64 * tiles128 >= 512; }
+static bool wide_tiles(long long N, int width) { return width > 64 && (N + 63) / 64 * ((width + 127) / 128) >= 512; }
 
-template <int TM, int TN> static hipError_t launch_linear_cfg(const float *x, const LinearSets &sets, long long N, int K, hipStream_t stream) {
-  int tiles = 0;
-  for (int i = 0; i < sets.n; ++i) tiles += (sets.set[i].width + TN - 1) / TN;
+template <int TM, int TN>
+static hipError_t launch_linear_cfg(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream) {
+  const int tiles = (O + TN - 1) / TN;
   const unsigned blocks = linear_blocks<TM, TN>(N, tiles);
   if (blocks == 0) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((linear_kernel<TM, TN>), dim3(blocks), dim3(256), 0, stream, x, sets, N, K, tiles);
+  hipLaunchKernelGGL((linear_kernel<TM, TN>), dim3(blocks), dim3(256), 0, stream, x, w, bias, y, N, O, K, tiles);
   return hipGetLastError();
 }
 
-hipError_t launch_linear(const float *x, const LinearSets &sets, long long N, int K, hipStream_t stream) {
-  int tiles128 = 0, width = 0;
-  for (int i = 0; i < sets.n; ++i) {
-    tiles128 += (sets.set[i].width + 127) / 128;
-    width += sets.set[i].width;
-  }
-  return wide_tiles(N, width, tiles128) ? launch_linear_cfg<64, 128>(x, sets, N, K, stream) : launch_linear_cfg<64, 64>(x, sets, N, K, stream);
+hipError_t launch_linear(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream) {
+  return wide_tiles(N, O) ? launch_linear_cfg<64, 128>(x, w, bias, y, N, O, K, stream) : launch_linear_cfg<64, 64>(x, w, bias, y, N, O, K, stream);
 }
 
 template <int TM, int TN, int FLUSH> static hipError_t launch_linear_sum_cfg(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream) {
@@ -375,7 +365,7 @@ template <int TM, int TN, int FLUSH> static hipError_t launch_linear_sum_cfg(con
 }
 
 hipError_t launch_linear_sum(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream) {
-  const bool wide = wide_tiles(N, K, (K + 127) / 128);
+  const bool wide = wide_tiles(N, K);
   if (sets.n == 1) return wide ? launch_linear_sum_cfg<64, 128, 0>(sets, y, N, K, stream) : launch_linear_sum_cfg<64, 64, 0>(sets, y, N, K, stream);
   return wide ? launch_linear_sum_cfg<64, 128, 128>(sets, y, N, K, stream) : launch_linear_sum_cfg<64, 64, 128>(sets, y, N, K, stream);
 }

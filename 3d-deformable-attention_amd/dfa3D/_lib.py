@@ -32,7 +32,7 @@ _O = ctypes.POINTER(LaunchOptions)
 
 class LinearSet(ctypes.Structure):
     """dfa3d_linear_set of include/dfa3d.h: one of several linear layers on the same rows."""
-    _fields_ = [("weight", _P), ("bias", _P), ("rows", _P), ("width", _I)]
+    _fields_ = [("weight", _P), ("rows", _P), ("width", _I)]
 
 
 # name -> argument types; every entry point returns int
@@ -56,7 +56,7 @@ SIGNATURES = {
     "dfa3d_camera_index": [_P] * 4 + [_I] * 3 + [_P],
     "dfa3d_locations": [_P] * 5 + [ctypes.c_longlong] + [_I] * 4 + [_P],
     "dfa3d_locations_grad": [_P] * 4 + [ctypes.c_longlong] + [_I] * 3 + [_P],
-    "dfa3d_linear": [_P, ctypes.POINTER(LinearSet), _I, ctypes.c_longlong, _I, _P],
+    "dfa3d_linear": [_P] * 4 + [ctypes.c_longlong, _I, _I, _P],
     "dfa3d_linear_sum": [ctypes.POINTER(LinearSet), _I, _P, ctypes.c_longlong, _I, _P],
     "dfa3d_linear_grad": [_P] * 5 + [ctypes.c_size_t, ctypes.c_longlong, _I, _I, _P],
     "dfa3d_abi_version": [],

@@ -40,13 +40,13 @@ def _widths_apply(O, K):
     return O % 2 == 0 and K % 2 == 0 and max(O, K) <= 2048 and O * K <= 2 ** 20
 
 
-def _products(x, params):
-    """``F.linear`` of every (weight, bias or None) of the flat tuple in one launch, none of it recorded; None where the kernel does not form
-    them (csrc/dfa3d_binding.cpp says where it does) or they are to be recorded."""
+def _product(x, weight, bias):
+    """``F.linear`` that nothing records, or None where the kernel does not form it (csrc/dfa3d_binding.cpp says where it does) or it
+    is to be recorded."""
     if not x.is_cuda or torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
         return None
     at = torch._C._cuda_getDevice()
-    return _lib.binding().linear(at, torch._C._cuda_getCurrentRawStream(at), x, params)
+    return _lib.binding().linear(at, torch._C._cuda_getCurrentRawStream(at), x, weight, bias)
 
 
 def _sum_of_products(operands):
@@ -57,10 +57,10 @@ def _sum_of_products(operands):
     return _lib.binding().linear_sum(at, torch._C._cuda_getCurrentRawStream(at), operands)
 
 
-def _linear(x, weight, bias):
-    """``F.linear``, by the kernel where nothing records it."""
-    got = _products(x, (weight, bias))
-    return F.linear(x, weight, bias) if got is None else got[0]
+def _linear(x, weight, bias, library):
+    """``F.linear``, by the kernel where nothing records it and it is not to be the library's (``library``)."""
+    got = None if library else _product(x, weight, bias)
+    return F.linear(x, weight, bias) if got is None else got
 
 
 def _weight_gradients(x, grad, want_bias):
@@ -100,7 +100,7 @@ class _ProjectionFunction(Function):
         # each operand only where the other one's gradient needs it, as F.linear keeps them: the other may be changed in place
         want_x, want_weight = ctx.needs_input_grad[:2]
         ctx.save_for_backward(x if want_weight else None, weight if want_x else None)
-        return F.linear(x, weight, bias) if library_forward else _linear(x, weight, bias)
+        return _linear(x, weight, bias, library_forward)
 
     @staticmethod
     def backward(ctx, grad):
@@ -144,10 +144,7 @@ class _SharedRowsFunction(Function):
         ctx.set_materialize_grads(False)
         want_x, *wanted = ctx.needs_input_grad[1:]
         ctx.save_for_backward(x if any(wanted[::2]) else None, *(w if want_x else None for w in weights))
-        own = [i for i, lib in enumerate(library) if not lib]
-        made = _products(x, tuple(t for i in own for t in (weights[i], biases[i]))) if own else None
-        made = dict(zip(own, made)) if made is not None else {}
-        return tuple(made[i] if i in made else F.linear(x, weights[i], biases[i]) for i in range(len(weights)))
+        return tuple(_linear(x, w, b, lib) for w, b, lib in zip(weights, biases, library))
 
     @staticmethod
     def backward(ctx, *grads):
@@ -173,7 +170,7 @@ def _applies(x, *layers):
 class Projection(nn.Linear):
     """``nn.Linear``: same parameters, same results.
 
-    ``library_forward``: in training the result is the library's to the bit.  For sampling offsets: the gradient of a sampling
+    ``library_forward``: the result is the library's to the bit.  For sampling offsets: the gradient of a sampling
     location jumps where the location passes from one pixel or depth bin to the next, so two products that round differently, neither
     of them further from the exact one, put some hundred of 15 million points on the other side, and gradients differ by 7e-4."""
 
@@ -186,7 +183,7 @@ class Projection(nn.Linear):
     def forward(self, input):
         if _applies(input, self):
             return _ProjectionFunction.apply(input, self.weight, self.bias, self.library_forward)
-        return _linear(input, self.weight, self.bias)
+        return _linear(input, self.weight, self.bias, self.library_forward)
 
 
 def _bare(layer):
@@ -198,12 +195,8 @@ def _bare(layer):
 
 
 def projections(x, layers):
-    """``[layer(x) for layer in layers]`` in fewer launches where the layers are plain ``Projection``s, at most four.
-    The layer of the base model, training: 3811 -> 3771 us; of the small one, inference: 293 -> 261."""
-    if len(layers) <= _MAX_SHARED and all(_bare(l) for l in layers):
-        if _applies(x, *layers):
-            return list(_SharedRowsFunction.apply(tuple(l.library_forward for l in layers), x, *(t for l in layers for t in (l.weight, l.bias))))
-        got = _products(x, tuple(t for l in layers for t in (l.weight, l.bias)))
-        if got is not None:
-            return list(got)
+    """``[layer(x) for layer in layers]``; where the layers are plain ``Projection``s, at most four, the gradient of ``x`` is formed in one
+    kernel.  The layer of the base model, training: 3811 -> 3771 us."""
+    if len(layers) <= _MAX_SHARED and all(_bare(l) for l in layers) and _applies(x, *layers):
+        return list(_SharedRowsFunction.apply(tuple(l.library_forward for l in layers), x, *(t for l in layers for t in (l.weight, l.bias))))
     return [layer(x) for layer in layers]

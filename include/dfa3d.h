@@ -264,17 +264,17 @@ int dfa3d_locations(const float *uv, const float *dz, const float *ref, const in
 int dfa3d_locations_grad(const float *grad_loc, const int64_t *shapes3, float *grad_uv, float *grad_dz, long long rows, int M, int L,
                          int P, void *stream);
 
-/* Up to four linear layers on the same rows in float32, all matrices row-major:
- *   dfa3d_linear      rows (N, width) = x (N, K) weight (width, K)^T + bias (width) or NULL, of every layer
- *   dfa3d_linear_sum  y (N, K) = sum over the layers of rows (N, width) weight (width, K): the gradient of x from those of the rows
- * K and widths even; K (the first), widths (the second) multiples of four.  Every element written, the same result every time. */
+/* Linear layers in float32, all matrices row-major:
+ *   dfa3d_linear      y (N, O) = x (N, K) weight (O, K)^T + bias (O) or NULL
+ *   dfa3d_linear_sum  y (N, K) = sum over up to four layers of rows (N, width) weight (width, K): the gradient of the rows that the layers
+ *                     share, from those of what they gave
+ * O, K and widths even; K (the first), widths (the second) multiples of four.  Every element written, the same result every time. */
 typedef struct dfa3d_linear_set {
   const float *weight;
-  const float *bias;
-  float *rows;            /* read only by dfa3d_linear_sum */
+  const float *rows;
   int width;
 } dfa3d_linear_set;
-int dfa3d_linear(const float *x, const dfa3d_linear_set *layers, int n_layers, long long N, int K, void *stream);
+int dfa3d_linear(const float *x, const float *weight, const float *bias, float *y, long long N, int O, int K, void *stream);
 int dfa3d_linear_sum(const dfa3d_linear_set *layers, int n_layers, float *y, long long N, int K, void *stream);
 
 /* Weight and bias gradients of a linear layer y = x weight^T + bias in float32: grad_weight (O, K) = grad_out^T x,

@@ -38,7 +38,7 @@ def test_product(N, K, O, across):
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(N + K + O)
     x, w, b = (torch.randn(*s, generator=g, device=dev) for s in ((N, K), (O, K), (O,)))
-    product = lambda: projection._sum_of_products((x, w.t().contiguous())) if across else projection._products(x, (w, b))[0]
+    product = lambda: projection._sum_of_products((x, w.t().contiguous())) if across else projection._product(x, w, b)
     got = product()
     xd, wd, bd = x.double(), w.double(), torch.zeros_like(b).double() if across else b.double()
     # three parts hold all of a float32; what is left out is 2^-25 of a product at most, and each of K / 16 steps of six sums, and the bias,
@@ -57,9 +57,9 @@ def test_operands_that_are_no_ordinary_numbers():
     w[:, 1] = 0.5
     x[3, 5], x[7, 9], x[200, 1], x[201, 1] = float("inf"), float("nan"), 3.402823e38, -3.402823e38
     x[50] *= 1e-34
-    got, want = projection._products(x, (w, b))[0], torch.nn.functional.linear(x, w, b)
+    got, want = projection._product(x, w, b), torch.nn.functional.linear(x, w, b)
     torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-4, equal_nan=True)
-    tiny = projection._products(x[50:51], (w, None))[0].double()
+    tiny = projection._product(x[50:51], w, None).double()
     torch.testing.assert_close(tiny, x[50:51].double() @ w.double().t(), rtol=0, atol=64 * 2.0 ** -23 * 1e-34 * 16)
     across = projection._sum_of_products((x, w.t().contiguous()))
     torch.testing.assert_close(across, x.matmul(w.t()), rtol=1e-5, atol=1e-4, equal_nan=True)
@@ -118,14 +118,15 @@ def test_layers_with_hooks_are_called():
     assert len(seen) == 1 and seen[0] is got[1]
 
 
-def test_offsets_keep_the_librarys_result_in_training():
+def test_offsets_keep_the_librarys_result():
     from dfa3D.modules.projection import Projection
     dev = torch.device("cuda:0")
     layer = Projection(256, 128, library_forward=True).to(dev)
     x = torch.randn(5000, 256, device=dev)
-    assert torch.equal(layer(x), torch.nn.functional.linear(x, layer.weight, layer.bias))
+    want = torch.nn.functional.linear(x, layer.weight, layer.bias)
+    assert torch.equal(layer(x), want)
     with torch.no_grad():
-        torch.testing.assert_close(layer(x), torch.nn.functional.linear(x, layer.weight, layer.bias), rtol=1e-5, atol=1e-5)
+        assert torch.equal(layer(x), want)
 
 
 def test_rows_in_other_layouts_and_partial_gradients():
@@ -164,12 +165,12 @@ def test_calls_that_keep_the_librarys_operation():
         assert layer(x).dtype == torch.bfloat16
     w, b = layer.weight.detach(), layer.bias.detach()
     x = x.detach()
-    from dfa3D.modules.projection import _products
-    assert _products(x, (w, b)) is not None
-    for args in ((x, (layer.weight, b)), (x.double(), (w, b)), (x.t(), (w, b)), (x, (w, b[:-1])), (x[:, :-2].contiguous(), (w, b)), (x[0], (w, b)),
-                 (x, (w[:-1].contiguous(), None)), (x, (w.t(), None)), (x, ()), (x, (w, None) * 5), (torch._neg_view(x), (w, b)), (x[:0], (w, b))):
-        assert _products(*args) is None
+    from dfa3D.modules.projection import _product
+    assert _product(x, w, b) is not None
+    for args in ((x, layer.weight, b), (x.double(), w, b), (x.t(), w, b), (x, w, b[:-1]), (x[:, :-2].contiguous(), w, b), (x[0], w, b),
+                 (x, w[:-1].contiguous(), None), (x, w.t(), None), (torch._neg_view(x), w, b), (x[:0], w, b)):
+        assert _product(*args) is None
     with torch.autocast("cuda", dtype=torch.bfloat16):
-        assert _products(x, (w, b)) is None
+        assert _product(x, w, b) is None
     few = torch.randn(7, 64, device=dev)
     torch.autograd.grad(layer(few).sum(), [layer.weight])
