@@ -163,16 +163,38 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         loc = offsets.view(bs, Q, M, L, P // Z, Z, 3) + anchors
         return loc.view(bs, Q, M, L, P, 3)
 
+    def _check_values(self, value, value_dpt_dist, spatial_shapes):
+        if spatial_shapes.shape[0] != self.num_levels:
+            raise ValueError(f"spatial_shapes has {spatial_shapes.shape[0]} levels, the module {self.num_levels}")
+        if value_dpt_dist is None or value_dpt_dist.dim() != 3 or value_dpt_dist.shape[:2] != value.shape[:2]:
+            raise ValueError("value_dpt_dist must be (bs, num_value, D)")
+
+    def _value_side(self, value, value_dpt_dist, spatial_shapes, key_padding_mask):
+        bs, num_value, _ = value.shape
+        value = self.value_proj(value)
+        if key_padding_mask is not None:
+            value = value.masked_fill(key_padding_mask[..., None], 0.0)
+        value = value.view(bs, num_value, self.num_heads, -1)
+        dim_depth = value_dpt_dist.shape[2]
+        dist = value_dpt_dist.reshape(bs, num_value, 1, dim_depth).to(value.dtype)
+        return value, dist, self.get_spatial_shape_3D(spatial_shapes, dim_depth)
+
+    def value_side(self, value, value_dpt_dist, spatial_shapes):
+        """What ``forward`` makes of ``value`` (bs, keys, embed_dims), ``value_dpt_dist`` and ``spatial_shapes`` alone."""
+        self._check_values(value, value_dpt_dist, spatial_shapes)
+        return self._value_side(value, value_dpt_dist, spatial_shapes, None)
+
     def forward(self, query, key=None, value=None, value_dpt_dist=None, identity=None, query_pos=None,
                 key_padding_mask=None, reference_points=None, spatial_shapes=None, level_start_index=None,
-                return_depth_score=False, packed_dist=None, **kwargs):
+                return_depth_score=False, packed_dist=None, value_side=None, **kwargs):
         """Arguments and results as spatial_cross_attention.py:428-583: ``query`` (bs, Q, embed_dims),
         ``value`` (bs, keys, embed_dims), ``value_dpt_dist`` (bs, keys, D), ``reference_points``
         (bs, Q, num_Z_anchors, 3) normalised, ``spatial_shapes`` (L, 2) as (h, w), ``level_start_index`` (L,).
         Returns ``(output (bs, Q, embed_dims), weight_update (bs, Q, heads, 1))``; with
         ``return_depth_score=True`` a third result, the operator's depth scores.  ``packed_dist``: what
         ``self.pack_dist(value_dpt_dist, spatial_shapes, level_start_index)`` returned for this very distribution;
-        an encoder that runs several of these layers on one distribution packs once and hands it to each."""
+        an encoder that runs several of these layers on one distribution packs once and hands it to each.  ``value_side``:
+        what ``self.value_side(value, value_dpt_dist, spatial_shapes)`` returned, for a caller that has the values before the queries."""
         if value is None:
             value = query
         if query_pos is not None:
@@ -181,12 +203,8 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
             query = query.permute(1, 0, 2)
             value = value.permute(1, 0, 2)
         bs, num_query, _ = query.shape
-        num_value = value.shape[1]
-        if spatial_shapes.shape[0] != self.num_levels:
-            raise ValueError(f"spatial_shapes has {spatial_shapes.shape[0]} levels, the module {self.num_levels}")
-        if value_dpt_dist is None or value_dpt_dist.dim() != 3 or value_dpt_dist.shape[:2] != value.shape[:2]:
-            raise ValueError("value_dpt_dist must be (bs, num_value, D)")
-
+        if value_side is None:
+            self._check_values(value, value_dpt_dist, spatial_shapes)
         # the largest launches first: the GPU works on them while the host prepares the others
         together = getattr(self.sampling_locations, "__func__", None) is MSDeformableAttention3D_DFA3D.sampling_locations
         if together:
@@ -194,15 +212,11 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
             uv, dz, attention_weights = projections(query, (self.sampling_offsets, self.sampling_offsets_depth, self.attention_weights))
         else:
             attention_weights = self.attention_weights(query)
-        value = self.value_proj(value)
-        if key_padding_mask is not None:
-            value = value.masked_fill(key_padding_mask[..., None], 0.0)
-        value = value.view(bs, num_value, self.num_heads, -1)
+        if value_side is None:
+            value_side = self._value_side(value, value_dpt_dist, spatial_shapes, key_padding_mask)
+        value, dist, spatial_shapes_3D = value_side
         attention_weights = attention_weights.view(bs, num_query, self.num_heads, self.num_levels * self.num_points).softmax(-1)
         attention_weights = attention_weights.view(bs, num_query, self.num_heads, self.num_levels, self.num_points)
-        dim_depth = value_dpt_dist.shape[2]
-        dist = value_dpt_dist.reshape(bs, num_value, 1, dim_depth).to(value.dtype)
-        spatial_shapes_3D = self.get_spatial_shape_3D(spatial_shapes, dim_depth)
         if together:
             sampling_locations = self._locations(uv, dz, reference_points, spatial_shapes_3D, query.dtype)
         else:

@@ -186,12 +186,16 @@ class Projection(nn.Linear):
         return _linear(input, self.weight, self.bias, self.library_forward)
 
 
-def _bare(layer):
-    """A Projection whose call is its ``forward`` and nothing else."""
-    return (type(layer) is Projection and "forward" not in layer.__dict__
+def no_hooks(layer):
+    """Whether the module's call is its class's ``forward`` and nothing else."""
+    return ("forward" not in layer.__dict__
             and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks
                      or _module._global_forward_hooks or _module._global_forward_pre_hooks
                      or _module._global_backward_hooks or _module._global_backward_pre_hooks))
+
+
+def _bare(layer):
+    return type(layer) is Projection and no_hooks(layer)
 
 
 def projections(x, layers):

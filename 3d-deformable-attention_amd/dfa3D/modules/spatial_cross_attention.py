@@ -9,7 +9,7 @@ from torch import nn
 
 from ..rebatch import RebatchCombineFunction, RebatchGatherFunction, camera_hits, camera_index, rebatch_gather
 from .ms_deform_attn_3d import MSDeformableAttention3D_DFA3D
-from .projection import Projection
+from .projection import Projection, no_hooks
 
 __all__ = ["SpatialCrossAttention_DFA3D"]
 
@@ -81,24 +81,29 @@ class SpatialCrossAttention_DFA3D(nn.Module):
         Z = reference_points_cam.size(3)
         cams = self.num_cams
 
-        hit, scale = camera_hits(bev_mask)                                       # (cams, Nq), (bs, Nq)
-        index, pos, max_len = camera_index(hit)
-        queries_rebatch = RebatchGatherFunction.apply(query, index, pos)         # (bs, cams, max_len, E)
+        # camera_index waits for the device: what does not need its answer is launched before.  Layer of the small model, inference:
+        # 312 -> 297 us, of the base model, training: 3835 -> 3796.
         ref = reference_points_cam.to(query.dtype).reshape(cams, bs, num_query, Z * 3).contiguous()
-        # The rows that pad the shorter cameras' lists are never read back.  With reference points of zero, as the reference
-        # pads them, all their samples fall on the map's first pixels, which a backward feels: every point of a pass on
-        # one cell and depth (base layer: tile kernel 1.31 against 1.25 ms, training step 4.27 against 4.15).  Far outside the map the operator
-        # skips them.  Another attention module gets the zeros.
-        pad = _OUTSIDE if type(self.deformable_attention) is MSDeformableAttention3D_DFA3D else 0.0
-        reference_points_rebatch = rebatch_gather(ref, index, per_camera=True, pad=pad)     # (bs, cams, max_len, Z*3)
-        L = index.shape[1]
-
         keys = key.shape[1]
         key = key.permute(2, 0, 1, 3).reshape(bs * cams, keys, self.embed_dims)
         value = value.permute(2, 0, 1, 3).reshape(bs * cams, keys, self.embed_dims)
         value_dpt_dist = value_dpt_dist.permute(2, 0, 1, 3).reshape(bs * cams, keys, value_dpt_dist.shape[-1])
+        attention = self.deformable_attention
+        ours = type(attention) is MSDeformableAttention3D_DFA3D
+        if ours and attention.batch_first and no_hooks(attention) and kwargs.get("key_padding_mask") is None:
+            kwargs["value_side"] = attention.value_side(value, value_dpt_dist, spatial_shapes)
+        hit, scale = camera_hits(bev_mask)                                       # (cams, Nq), (bs, Nq)
+        index, pos, max_len = camera_index(hit)
+        queries_rebatch = RebatchGatherFunction.apply(query, index, pos)         # (bs, cams, max_len, E)
+        # The rows that pad the shorter cameras' lists are never read back.  With reference points of zero, as the reference
+        # pads them, all their samples fall on the map's first pixels, which a backward feels: every point of a pass on
+        # one cell and depth (base layer: tile kernel 1.31 against 1.25 ms, training step 4.27 against 4.15).  Far outside the map the operator
+        # skips them.  Another attention module gets the zeros.
+        pad = _OUTSIDE if ours else 0.0
+        reference_points_rebatch = rebatch_gather(ref, index, per_camera=True, pad=pad)     # (bs, cams, max_len, Z*3)
+        L = index.shape[1]
 
-        queries, update_weight = self.deformable_attention(
+        queries, update_weight = attention(
             query=queries_rebatch.view(bs * cams, L, self.embed_dims), key=key, value=value,
             value_dpt_dist=value_dpt_dist, reference_points=reference_points_rebatch.view(bs * cams, L, Z, 3),
             spatial_shapes=spatial_shapes, level_start_index=level_start_index, **kwargs)
