@@ -65,6 +65,31 @@ def test_layer_does_not_depend_on_the_padding(monkeypatch):
         torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4 * b.abs().max().item())
 
 
+@pytest.mark.parametrize("train", [False, True])
+def test_layer_with_the_value_side_first(train):
+    """Launched before the camera lists, and inside the attention module, as it is where a hook looks on: the same result."""
+    from dfa3D.modules import SpatialCrossAttention_DFA3D
+    torch.manual_seed(1)
+    dev, cams, bs, Nq, E, maps = "cuda", 2, 2, 5000, 64, [(9, 14)]
+    layer = SpatialCrossAttention_DFA3D(embed_dims=E, num_cams=cams, bev_h=50, bev_w=100, dropout=0.0, num_head=4,
+                                        deformable_attention=dict(embed_dims=E, num_heads=4, num_levels=1, num_points=4)).to(dev)
+    for p in layer.parameters():
+        torch.nn.init.normal_(p, std=0.1)
+    query = torch.randn(bs, Nq, E, device=dev, requires_grad=train)
+    feats = torch.randn(cams, 126, bs, E, device=dev)
+    args = dict(spatial_shapes=torch.tensor(maps, device=dev), level_start_index=torch.tensor([0], device=dev),
+                reference_points_cam=torch.rand(cams, bs, Nq, 4, 3, device=dev), bev_mask=torch.rand(cams, bs, Nq, 4, device=dev) < 0.3,
+                value_dpt_dist=torch.rand(cams, 126, bs, 8, device=dev).softmax(-1))
+    with torch.set_grad_enabled(train):
+        got = layer(query, feats, feats, **args)
+        seen = []
+        layer.deformable_attention.register_forward_pre_hook(lambda m, a, kw: seen.append(kw.get("value_side")), with_kwargs=True)
+        want = layer(query, feats, feats, **args)
+        with pytest.raises(ValueError, match="levels"):
+            layer(query, feats, feats, **{**args, "spatial_shapes": torch.tensor(maps * 2, device=dev)})
+    assert seen == [None] * 2 and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.bfloat16], ids=["fp64", "fp32", "bf16"])
 def test_scale_has_the_default_dtype(dtype):
     """A program in double precision averages with 1/3 in double precision."""
