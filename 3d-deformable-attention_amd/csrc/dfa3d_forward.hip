@@ -104,7 +104,7 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
     const int64_t *__restrict__ level_start, const A *__restrict__ loc, int loc_stride,
     const A *__restrict__ attn, const T *__restrict__ score_in, T *__restrict__ out, T *__restrict__ score_out,
     A *__restrict__ weight_update, const T *__restrict__ packed_arg, int Md, int B, int S, int M, int C, int D, int L,
-    int Q, int P, int upw, int iters, int q_blocks, bool once, int lds_rows) {
+    int Q, int P, int upw, int iters, int q_blocks, int once, int lds_rows) {
   // packed: the head-shared distribution as dfa3d_pack_dist lays it out (D >= 2), or nullptr
   __shared__ LevelTable tab;
   constexpr int WAVES = (IN_LDS ? kLdsRowsBlock : kBlock) / kWave;
@@ -212,15 +212,20 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
           const size_t gp = ((size_t)(b * (size_t)Q + q) * M + m) * ws.LP + lp;   // global point index
           const A *pl = loc + gp * loc_stride;
           A x, y, z = 0, a;
-          if (!IN_LDS && once) {                                    // uniform
+          if (!IN_LDS && (once & 1) != 0) {                         // uniform
             asm volatile("");                                       // (or the compiler merges the branches into plain loads)
             x = __builtin_nontemporal_load(pl); y = __builtin_nontemporal_load(pl + 1);
             if (FUSED) z = __builtin_nontemporal_load(pl + 2);
-            a = __builtin_nontemporal_load(attn + gp);
             asm volatile("");
           } else {
             x = pl[0]; y = pl[1];
             if (FUSED) z = pl[2];
+          }
+          if (!IN_LDS && (once & 2) != 0) {
+            asm volatile("");
+            a = __builtin_nontemporal_load(attn + gp);
+            asm volatile("");
+          } else {
             a = attn[gp];
           }
           const Point2D<A> g = locate_2d<A>(x, y, tab.H[l], tab.W[l], tab.start[l]);
@@ -458,8 +463,11 @@ hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int6
 //     1000: 13.3, 12.6   1600: 19.6, 17.2   6400: 53.4, 41.0; 504 rows, 720 points: 10.7, 10.1; 384 rows, 800 points: 10.9, 10.6.
 //   * The coarser levels of a pyramid fit (the level sizes are on the device; each is taken for a quarter of the one before): one
 //     (batch, head) at a time on an XCD, as its L2 holds no more, so M has to divide 8 or be a multiple of it.  A workgroup's start
-//     and end cost as much as about a thousand points, LDS saves half of a point's lines (plain attention all): from 2000 points on levels in
-//     LDS, so far as one can tell.  Memory and LDS, points per workgroup x share of the levels:
+//     and end cost as much as about a thousand points, LDS saves half of a point's lines (plain attention all): from 1200 points on levels in
+//     LDS, so far as one can tell.  Memory and LDS, points per workgroup x share of the levels, operands that change from call to call:
+//     5000 x 1/4: 522, 495; scores given 309, 283; plain 266, 252   bfloat16 plain 216, 185   2500 x 1/2: 191, 196; 128, 113; plain 103, 94
+//     3000 x 1/3: 117, 113; 70, 71; plain 49, 54   2800 x 1/3: 127, 124; 82, 84; plain 59, 67   1500 x 1/4: 194, 213; 118, 124; plain 108, 116
+//     and the same operands again and again:
 //     10000 x 1/4: 914, 864   8000 x 1/2: 610, 535   4000 x 1/2: 240, 226; plain 171, 154; 120, 114   3500 x 1/4: 349, 370   3500 x 1/2: plain 52, 54
 //     2000 x 1/2: 106, 109; plain 73, 77   1000 x 3/4: 76, 89.  Not with packed distributions, which a cross-attention layer uses: its
 //     points share a pillar's few pixels, whose rows the L1 has (200 x 200 queries, base maps 412, 432; 120 x 120, 30 x 48 226, 239).
@@ -482,7 +490,7 @@ template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a)
   int in_lds = 0;
   for (int l = 1; l < a.L; ++l) all = 4 * all + 1;          // (at most 16 levels)
   for (; in_lds + 1 < a.L && 1.1 * a.S * some <= (double)room * all; ++in_lds) some = 4 * some + 1;
-  if (points * in_lds < parts * 2000 * a.L) return none;
+  if (points * in_lds < parts * 1200 * a.L) return none;
   return LdsRows{(int)parts, (int)room};
 }
 
@@ -510,7 +518,10 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   // by each.  6 batch elements, four levels from 80 x 128, 8 points (whole lines), non-temporal and plain, us: 610, 618; bfloat16 556, 572; plain
   // attention, maps from 116 x 185 360, 380; with 2, 3 or 4 points per level 212, 202; 211, 203; 346, 341; one level of 58 x 92, 4 points
   // 137, 112; three of 58 x 92 226, 208.  Small operands come from the caches either way (37 x 59, 20 MB, whole lines: 48, 43).
-  const bool once = a.L * a.P * sizeof(A) % 128 == 0 && (long long)a.B * a.Q * a.M * a.L * a.P * (a.loc_stride + 1) * (long long)sizeof(A) > (48LL << 20);
+  // (Plain attention, four levels of 4 points, whose locations are whole lines and whose weights are not: both non-temporal, neither, the
+  // locations alone 272, 269, 267; on the same operands again and again, which the Infinity Cache then holds in part, 230, 258, 238.)
+  const bool large = (long long)a.B * a.Q * a.M * a.L * a.P * (a.loc_stride + 1) * (long long)sizeof(A) > (48LL << 20);
+  const int once = !large ? 0 : (a.L * a.P * a.loc_stride * sizeof(A) % 128 == 0 ? 1 : 0) | (a.L * a.P * sizeof(A) % 128 == 0 ? 2 : 0);
   auto launch = [&](auto kernel, int threads, size_t bytes) -> hipError_t {
     if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), bytes)) return e;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), bytes, stream, (const T *)a.value, (const T *)a.dist, a.shapes,
