@@ -3,8 +3,8 @@
     python 3d-deformable-attention_amd/build.py [--force] [--clocks]
 
 The library lands next to the python package (dfa3D/libdfa3d_hip.so) so that it travels with
-the source tree, as does the module that calls it with torch's tensors (dfa3D/_binding.so, host code).  Two more libraries land beside bench.py, which is what uses them: the yardstick kernels
-(libdfa3d_measure.so) and, with --clocks, libdfa3d_hip_clocks.so: the same sources compiled with
+the source tree, as does the module that calls it with torch's tensors (dfa3D/_binding.so, host code).
+Two more libraries land beside bench.py, which is what uses them: the yardstick kernels (libdfa3d_measure.so) and, with --clocks, libdfa3d_hip_clocks.so: the same sources compiled with
 -DDFA3D_TILE_TIMING, i.e. with the per-phase clocks of the backward's tile kernels (`bench.py --phase-costs`).
 """
 import os

@@ -135,8 +135,8 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         offsets, divided by the level's (W, H, D), around the query's Z-anchor reference points
         (spatial_cross_attention.py:498-537).  Point p belongs to anchor p % num_Z_anchors."""
         self._check_reference_points(reference_points)
-        return self._locations(*projections(query, (self.sampling_offsets, self.sampling_offsets_depth)), reference_points, spatial_shapes_3D,
-                               query.dtype)
+        uv, dz = projections(query, (self.sampling_offsets, self.sampling_offsets_depth))
+        return self._locations(uv, dz, reference_points, spatial_shapes_3D, query.dtype)
 
     def _check_reference_points(self, reference_points):
         P, Z = self.num_points, reference_points.shape[2]
@@ -193,8 +193,9 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         Returns ``(output (bs, Q, embed_dims), weight_update (bs, Q, heads, 1))``; with
         ``return_depth_score=True`` a third result, the operator's depth scores.  ``packed_dist``: what
         ``self.pack_dist(value_dpt_dist, spatial_shapes, level_start_index)`` returned for this very distribution;
-        an encoder that runs several of these layers on one distribution packs once and hands it to each.  ``value_side``:
-        what ``self.value_side(value, value_dpt_dist, spatial_shapes)`` returned, for a caller that has the values before the queries."""
+        an encoder that runs several of these layers on one distribution packs once and hands it to each.
+        ``value_side``: what ``self.value_side(value, value_dpt_dist, spatial_shapes)`` returned, for a caller that has
+        the values before the queries."""
         if value is None:
             value = query
         if query_pos is not None:
@@ -209,7 +210,8 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         together = getattr(self.sampling_locations, "__func__", None) is MSDeformableAttention3D_DFA3D.sampling_locations
         if together:
             self._check_reference_points(reference_points)
-            uv, dz, attention_weights = projections(query, (self.sampling_offsets, self.sampling_offsets_depth, self.attention_weights))
+            uv, dz, attention_weights = projections(
+                query, (self.sampling_offsets, self.sampling_offsets_depth, self.attention_weights))
         else:
             attention_weights = self.attention_weights(query)
         if value_side is None:

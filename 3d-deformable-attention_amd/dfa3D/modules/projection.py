@@ -41,8 +41,8 @@ def _widths_apply(O, K):
 
 
 def _product(x, weight, bias):
-    """``F.linear`` that nothing records, or None where the kernel does not form it (csrc/dfa3d_binding.cpp says where it does) or it
-    is to be recorded."""
+    """``F.linear`` that nothing records, or None where the kernel does not form it (csrc/dfa3d_binding.cpp says where
+    it does) or it is to be recorded."""
     if not x.is_cuda or torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
         return None
     at = torch._C._cuda_getDevice()
@@ -135,8 +135,9 @@ def _layer_gradients(x, grad, want_weight, want_bias):
 
 
 class _SharedRowsFunction(Function):
-    """``F.linear(x, weight, bias)`` of several layers (weight, bias, weight, bias, ...) on the same rows; ``library`` says whose forward is
-    the library's.  The gradient of the rows is formed in one kernel instead of one product per layer and the sums of their results."""
+    """``F.linear(x, weight, bias)`` of several layers (weight, bias, weight, bias, ...) on the same rows; ``library``
+    says whose forward is the library's.  The gradient of the rows is formed in one kernel instead of one product per
+    layer and the sums of their results."""
 
     @staticmethod
     def forward(ctx, library, x, *params):
@@ -171,8 +172,9 @@ class Projection(nn.Linear):
     """``nn.Linear``: same parameters, same results.
 
     ``library_forward``: the result is the library's to the bit.  For sampling offsets: the gradient of a sampling
-    location jumps where the location passes from one pixel or depth bin to the next, so two products that round differently, neither
-    of them further from the exact one, put some hundred of 15 million points on the other side, and gradients differ by 7e-4."""
+    location jumps where the location passes from one pixel or depth bin to the next, so two products that round
+    differently, neither of them further from the exact one, put some hundred of 15 million points on the other side,
+    and gradients differ by 7e-4."""
 
     library_forward = False
 
@@ -199,8 +201,9 @@ def _bare(layer):
 
 
 def projections(x, layers):
-    """``[layer(x) for layer in layers]``; where the layers are plain ``Projection``s, at most four, the gradient of ``x`` is formed in one
-    kernel.  The layer of the base model, training: 3811 -> 3771 us."""
+    """``[layer(x) for layer in layers]``; where the layers are plain ``Projection``s, at most four, the gradient of
+    ``x`` is formed in one kernel.  The layer of the base model, training: 3811 -> 3771 us."""
     if len(layers) <= _MAX_SHARED and all(_bare(l) for l in layers) and _applies(x, *layers):
-        return list(_SharedRowsFunction.apply(tuple(l.library_forward for l in layers), x, *(t for l in layers for t in (l.weight, l.bias))))
+        params = [t for l in layers for t in (l.weight, l.bias)]
+        return list(_SharedRowsFunction.apply(tuple(l.library_forward for l in layers), x, *params))
     return [layer(x) for layer in layers]

@@ -81,8 +81,8 @@ class SpatialCrossAttention_DFA3D(nn.Module):
         Z = reference_points_cam.size(3)
         cams = self.num_cams
 
-        # camera_index waits for the device: what does not need its answer is launched before.  Layer of the small model, inference:
-        # 312 -> 297 us, of the base model, training: 3835 -> 3796.
+        # camera_index waits for the device: what does not need its answer is launched before.  Layer of the small model,
+        # inference: 312 -> 297 us, of the base model, training: 3835 -> 3796.
         ref = reference_points_cam.to(query.dtype).reshape(cams, bs, num_query, Z * 3).contiguous()
         keys = key.shape[1]
         key = key.permute(2, 0, 1, 3).reshape(bs * cams, keys, self.embed_dims)
