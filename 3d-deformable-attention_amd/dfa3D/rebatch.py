@@ -9,35 +9,54 @@ from torch.autograd.function import once_differentiable
 
 from . import _lib
 
-__all__ = ["camera_hits", "camera_index", "rebatch_gather", "rebatch_combine", "RebatchGatherFunction", "RebatchCombineFunction"]
+__all__ = ["camera_hits", "camera_count", "camera_index", "rebatch_gather", "rebatch_combine", "RebatchGatherFunction", "RebatchCombineFunction"]
 
 
-def camera_index(hit):
+def camera_count(hit):
+    """Starts counting the queries of each camera of ``hit`` (cams, Nq) and the copy of the counts to the host: hand the result
+    to ``camera_index``, which then waits for these alone and not for what was launched in between.  None where the lists
+    are not made by the kernels."""
+    cams, Nq = hit.shape
+    if not (hit.is_cuda and hit.dtype == torch.bool and hit.is_contiguous() and 0 < cams <= 65535 and 0 < Nq <= 2 ** 30):
+        return None
+    totals = torch.empty(cams, dtype=torch.int32, device=hit.device)
+    on_host = torch.empty(cams, dtype=torch.int32, pin_memory=True)
+    with _lib.on_device(hit.device):
+        rc = _lib.lib().dfa3d_camera_count(_lib.ptr(hit), _lib.ptr(totals), cams, Nq, _lib.stream_of(hit))
+        _lib.check(rc, "dfa3d_camera_count")
+        on_host.copy_(totals, non_blocking=True)
+        done = torch.cuda.Event()
+        done.record()
+    return totals, on_host, done
+
+
+def camera_index(hit, counted=None):
     """``hit`` (cams, Nq) bool: query q projects into camera i.  Returns ``index`` (cams, max_len) int32, the
     queries of each camera in ascending order padded with -1, and its inverse ``pos`` (cams, Nq) int32
     (position of q in camera i's list, or -1).  ``max_len`` depends on the data, so this synchronises with the
-    device once, like the reference's ``nonzero`` calls (spatial_cross_attention.py:704-707)."""
-    cams, Nq = hit.shape
-    hit = hit.bool()
-    if hit.is_cuda and 0 < cams <= 65535 and 0 < Nq <= 2 ** 30:
-        return _camera_index_on_gpu(hit.contiguous())
+    device once, like the reference's ``nonzero`` calls (spatial_cross_attention.py:704-707).  ``counted``: what
+    ``camera_count`` returned for this very ``hit``."""
+    hit = hit.bool().contiguous()
+    if counted is None:
+        counted = camera_count(hit)
+    if counted is not None:
+        return _camera_index_on_gpu(hit, *counted)
     rank = hit.cumsum(1, dtype=torch.int32) - 1                      # position among the camera's queries
     pos = torch.where(hit, rank, torch.full_like(rank, -1)).contiguous()
     max_len = int(hit.sum(1).max().item()) if hit.numel() else 0
-    index = torch.full((cams, max(max_len, 1)), -1, dtype=torch.int32, device=hit.device)
+    index = torch.full((hit.shape[0], max(max_len, 1)), -1, dtype=torch.int32, device=hit.device)
     cam, q = hit.nonzero(as_tuple=True)
     index[cam, rank[cam, q].long()] = q.to(torch.int32)
     return index, pos, max_len
 
 
-def _camera_index_on_gpu(hit):
+def _camera_index_on_gpu(hit, totals, on_host, done):
     cams, Nq = hit.shape
     dev, lib = hit.device, _lib.lib()
-    totals = torch.empty(cams, dtype=torch.int32, device=dev)
     pos = torch.empty(cams, Nq, dtype=torch.int32, device=dev)
     with _lib.on_device(dev):
-        _lib.check(lib.dfa3d_camera_count(_lib.ptr(hit), _lib.ptr(totals), cams, Nq, _lib.stream_of(hit)), "dfa3d_camera_count")
-        max_len = max(totals.tolist())                              # waits for the device
+        done.synchronize()                                          # waits for the device
+        max_len = max(on_host.tolist())
         index = torch.empty(cams, max(max_len, 1), dtype=torch.int32, device=dev)
         _lib.check(lib.dfa3d_camera_index(_lib.ptr(hit), _lib.ptr(totals), _lib.ptr(index), _lib.ptr(pos), cams, Nq,
                                           max(max_len, 1), _lib.stream_of(hit)), "dfa3d_camera_index")

@@ -65,6 +65,20 @@ def test_layer_does_not_depend_on_the_padding(monkeypatch):
         torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4 * b.abs().max().item())
 
 
+def test_counting_started_ahead():
+    from dfa3D.rebatch import camera_count, camera_index
+    g = torch.Generator(device="cuda").manual_seed(2)
+    for cams, Nq in ((6, 22500), (1, 1), (3, 1000)):
+        hit = torch.rand(cams, Nq, generator=g, device="cuda") < 0.3
+        counted = camera_count(hit)
+        other = torch.ones(1 << 24, device="cuda").cumsum(0)             # work behind the counting
+        index, pos, longest = camera_index(hit, counted)
+        want = camera_index(hit)
+        assert longest == int(hit.sum(1).max()) == want[2] and torch.equal(index, want[0]) and torch.equal(pos, want[1])
+        del other
+    assert camera_count(hit.t()) is None and camera_count(hit.float()) is None and camera_count(hit.cpu()) is None
+
+
 @pytest.mark.parametrize("train", [False, True])
 def test_layer_with_the_value_side_first(train):
     """Launched before the camera lists, and inside the attention module, as it is where a hook looks on: the same result."""
