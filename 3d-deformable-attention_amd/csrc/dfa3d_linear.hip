@@ -176,51 +176,82 @@ __device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, in
   }
 }
 
-// Result (m, n) of the tile by plain float32 arithmetic, for the elements that the split gives no number for.
-template <bool A_ACROSS, bool B_ACROSS>
-__device__ __noinline__ float plain_product(rsrc_t a_r, int lda, int m, rsrc_t b_r, int ldb, int n, int depth) {
-  float sum = 0;
-  for (int k = 0; k < depth; ++k)
-    sum = fmaf(BufElem<float>::ld(a_r, (uint32_t)(A_ACROSS ? k * lda + m : m * lda + k) * 4),
-               BufElem<float>::ld(b_r, (uint32_t)(B_ACROSS ? k * ldb + n : n * ldb + k) * 4), sum);
-  return sum;
+// Whether the wavefront has a sum among its own that parts give no number for.  A float32 infinity, or a number next to the largest, is no
+// bfloat16 number, and an infinity times a lower part of zero is none either; and the third part of a number below 2^-108 is denormal.
+// A sum that is no finite number, or tiny, is formed again without parts.
+template <int MT, int NT> __device__ __forceinline__ bool odd_sums(const f32x16 (&acc)[MT][NT]) {
+  uint32_t least = 0xFFFFFFFFu, most = 0;                     // of the sizes' bits, twice; least: without zeros, less one
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const uint32_t twice = __float_as_uint(acc[i][j][r]) << 1;
+        least = min(least, twice - 1);
+        most = max(most, twice);
+      }
+  const bool odd = most >= 0xFF000000u || least < (__float_as_uint(0x1p-96f) << 1) - 1;
+  return __builtin_amdgcn_ballot_w64(odd) != 0;
 }
 
-// A float32 infinity, or a number next to the largest, is no bfloat16 number, and an infinity times a lower part of zero is none either; and
-// the third part of a number below 2^-108 is denormal.  A sum that is no finite number, or tiny, is formed again without parts.
-__device__ __forceinline__ bool odd_sum(float x) { return !(fabsf(x) <= 3.402823466e38f) || (fabsf(x) < 0x1p-96f && x != 0.f); }
+// This lane's four of eight contraction steps from k0 on of one row, for float32 matrix instructions; arguments as of SplitOperand::load.
+template <bool ACROSS> __device__ __forceinline__ void load_whole(rsrc_t r, int ld, int row0, int rows, int row, int k0, int depth, float (&v)[4]) {
+  const int k = k0 + 4 * ((int)threadIdx.x % kWave / 32);
+  if constexpr (ACROSS) {
+    const uint32_t off = row0 + row < rows ? (uint32_t)(k * ld + row0 + row) * 4 : kNoRow;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off + (uint32_t)(j * ld) * 4, 0, 0));
+  } else {
+    const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r, k < depth ? (uint32_t)(row * ld + k) * 4 : kNoRow, 0, 0);
+    v[0] = __uint_as_float(t.x); v[1] = __uint_as_float(t.y);
+    v[2] = __uint_as_float(t.z); v[3] = __uint_as_float(t.w);
+  }
+}
 
-// c (TM x TN tile of `ms` x `ns` valid elements, row length ldc) = acc + bias; `plain` forms one element without parts.
-template <int TM, int TN, typename Plain>
+// acc += the wavefront's part of the tile by float32 matrix instructions, straight from memory: what split_product forms, for sums that
+// parts give no number for.  Gradients of a loss that is no number are all of that kind, and cost a few times the usual, not a walk
+// over the rows per element: weight gradient of 58000 rows of 256 x 256 56 us, all NaN 119 (by
+// one lane per element 10000); grad_x 59, 124 (3280); with one NaN row in a thousand 125 (6400) and 70 (173).
+template <int TM, int TN, bool A_ACROSS, bool B_ACROSS>
+__device__ __forceinline__ void whole_product(rsrc_t a_r, int lda, int a_row0, int a_rows, rsrc_t b_r, int ldb, int b_row0, int b_rows, int depth,
+                                              f32x16 (&acc)[TM / 64][TN / 64]) {
+  constexpr int MT = TM / 64, NT = TN / 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int row_a = (wave & 1) * MT * 32 + lane % 32, row_b = (wave >> 1) * NT * 32 + lane % 32;
+  for (int k0 = 0; k0 < depth; k0 += 8) {                     // uniform
+    float a[MT][4], b[NT][4];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) load_whole<A_ACROSS>(a_r, lda, a_row0, a_rows, row_a + 32 * i, k0, depth, a[i]);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) load_whole<B_ACROSS>(b_r, ldb, b_row0, b_rows, row_b + 32 * j, k0, depth, b[j]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][k], b[j][k], acc[i][j], 0, 0, 0);
+  }
+}
+
+// c (TM x TN tile of `ms` x `ns` valid elements, row length ldc) = acc + bias.
+template <int TM, int TN>
 __device__ __forceinline__ void store_product(const f32x16 (&acc)[TM / 64][TN / 64], float *__restrict__ c, int ldc, int ms, int ns,
-                                              const float *__restrict__ bias, const Plain &plain) {
+                                              const float *__restrict__ bias) {
   constexpr int MT = TM / 64, NT = TN / 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int first_m = (wave & 1) * MT * 32 + 4 * (lane / 32), first_n = (wave >> 1) * NT * 32 + lane % 32;
-  auto row_a = [&](int i, int r) { return first_m + 32 * i + 8 * (r / 4) + r % 4; };
-  auto row_b = [&](int j) { return first_n + 32 * j; };
-  bool odd = false;
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
-    const int n = row_b(j);
+    const int n = first_n + 32 * j;
     const float add = (bias != nullptr && n < ns) ? bias[n] : 0.f;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int m = row_a(i, r);
-        odd = odd || odd_sum(acc[i][j][r]);
+        const int m = first_m + 32 * i + 8 * (r / 4) + r % 4;
         if (m < ms && n < ns) c[(size_t)m * ldc + n] = acc[i][j][r] + add;
       }
-  }
-  if (odd) {
-    for (int e = 0; e < NT * MT * 16; ++e) {
-      const int m = row_a(e / 16 % MT, e % 16), n = row_b(e / 16 / MT);
-      if (m >= ms || n >= ns) continue;
-      float *to = c + (size_t)m * ldc + n;
-      if (bias == nullptr && !odd_sum(*to)) continue;
-      *to = plain(m, n) + (bias != nullptr ? bias[n] : 0.f);
-    }
   }
 }
 
@@ -236,8 +267,11 @@ __global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict_
   f32x16 acc[TM / 64][TN / 64];
   zero_sums(acc);
   split_product<TM, TN, false, false, 0>(lds, x_r, K, 0, 0, w_r, K, 0, 0, K, acc, [](const auto &) {});
-  store_product<TM, TN>(acc, y + n0 * O + o0, O, ms, ns, bias != nullptr ? bias + o0 : nullptr,
-                        [&](int m, int n) { return plain_product<false, false>(x_r, K, m, w_r, K, n, K); });
+  if (odd_sums(acc)) {                                        // uniform
+    zero_sums(acc);
+    whole_product<TM, TN, false, false>(x_r, K, 0, 0, w_r, K, 0, 0, K, acc);
+  }
+  store_product<TM, TN>(acc, y + n0 * O + o0, O, ms, ns, bias != nullptr ? bias + o0 : nullptr);
 }
 
 // y (N, K) = sum of rows (N, width) weight (width, K) over the sets: the gradient of the rows that several layers share.  FLUSH: 0 for one set.
@@ -256,14 +290,14 @@ __global__ __launch_bounds__(256, 3) void linear_sum_kernel(LinearSets sets, flo
     if (i > 0) lds_barrier();                                 // nobody reads the last set's parts any more
     split_product<TM, TN, false, true, FLUSH>(lds, rows(s), s.width, 0, 0, weight(s), K, k0, K, s.width, acc, [](const auto &) {});
   }
-  store_product<TM, TN>(acc, y + n0 * K + k0, K, ms, K - k0 < TN ? K - k0 : TN, nullptr, [&](int m, int n) {
-    float sum = 0;
+  if (odd_sums(acc)) {                                        // uniform
+    zero_sums(acc);
     for (int i = 0; i < sets.n; ++i) {
       const LinearSet &s = sets.set[i];
-      sum += plain_product<false, true>(rows(s), s.width, m, weight(s), K, k0 + n, s.width);
+      whole_product<TM, TN, false, true>(rows(s), s.width, 0, 0, weight(s), K, k0, K, s.width, acc);
     }
-    return sum;
-  });
+  }
+  store_product<TM, TN>(acc, y + n0 * K + k0, K, ms, K - k0 < TN ? K - k0 : TN, nullptr);
 }
 
 struct LinearTiles { int o, k, parts, rows; };      // result tiles along O and K; parts of the rows, rows of a part
@@ -300,8 +334,11 @@ __global__ __launch_bounds__(256, 2) void linear_grad_part_kernel(
     bias_sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   });
   float *mine = partial + (size_t)part * ((size_t)O * K + O);
-  store_product<128, 128>(acc, mine + (size_t)o0 * K + k0, K, O - o0, K - k0, nullptr,
-                          [&](int m, int n) { return plain_product<true, true>(g_r, O, o0 + m, x_r, K, k0 + n, n_rows); });
+  if (odd_sums(acc)) {                                      // uniform
+    zero_sums(acc);
+    whole_product<128, 128, true, true>(g_r, O, o0, O, x_r, K, k0, K, n_rows, acc);
+  }
+  store_product<128, 128>(acc, mine + (size_t)o0 * K + k0, K, O - o0, K - k0, nullptr);
   if (want_bias && k0 == 0) {                               // uniform
     float *s_bias = reinterpret_cast<float *>(lds);
     lds_barrier();
