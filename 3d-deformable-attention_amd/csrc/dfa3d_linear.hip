@@ -65,8 +65,9 @@ template <int R, bool ACROSS> struct SplitOperand {
     }
   }
 
-  // x = p1 + p2 + p3, each rounded to nearest: 24 bits and more, so nothing of a float32 is lost
-  __device__ __forceinline__ void to_lds(unsigned char *lds) const {
+  // x = p1 + p2 + p3, each rounded to nearest: 24 bits and more, so nothing of a float32 of 2^-108 or more is lost, and of a smaller one
+  // 2^-133 at most (odd_sums).  `most`: the largest size that came by.
+  __device__ __forceinline__ void to_lds(unsigned char *lds, float &most) const {
     typedef unsigned int words __attribute__((ext_vector_type(kRun / 2)));
 #pragma unroll
     for (int u = 0; u < kUnits; ++u) {
@@ -76,6 +77,8 @@ template <int R, bool ACROSS> struct SplitOperand {
       float rest[kRun];
 #pragma unroll
       for (int j = 0; j < kRun; ++j) rest[j] = v[u][j];
+#pragma unroll
+      for (int j = 0; j < kRun; j += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(rest[j]), "v"(rest[j + 1]));
 #pragma unroll
       for (int plane = 0; plane < 3; ++plane) {
         words p;
@@ -110,10 +113,10 @@ template <int MT, int NT> __device__ __forceinline__ void zero_sums(f32x16 (&x)[
 
 // acc += sum over depth contraction steps of A(m, k) B(n, k) for a TM x TN tile by four wavefronts, 2 x 2; `seen` is called with A's registers
 // once per kStep steps.  FLUSH: the matrix unit does not round its sums to nearest, which a chain of more than some hundred steps feels; its sums
-// start from zero every FLUSH steps and the vector unit adds them up.
+// start from zero every FLUSH steps and the vector unit adds them up.  `most`: the largest size among the operands that this thread brought.
 template <int TM, int TN, bool A_ACROSS, bool B_ACROSS, int FLUSH, typename Seen>
 __device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, int lda, int a_row0, int a_rows, rsrc_t b_r, int ldb, int b_row0,
-                                              int b_rows, int depth, f32x16 (&acc)[TM / 64][TN / 64], const Seen &seen) {
+                                              int b_rows, int depth, f32x16 (&acc)[TM / 64][TN / 64], float &most, const Seen &seen) {
   constexpr int MT = TM / 64, NT = TN / 64;
   using OpA = SplitOperand<TM, A_ACROSS>;
   using OpB = SplitOperand<TN, B_ACROSS>;
@@ -127,8 +130,8 @@ __device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, in
   OpB b;
   a.load(a_r, lda, a_row0, a_rows, 0, depth);
   b.load(b_r, ldb, b_row0, b_rows, 0, depth);
-  a.to_lds(lds);
-  b.to_lds(lds + OpA::kBytes);
+  a.to_lds(lds, most);
+  b.to_lds(lds + OpA::kBytes, most);
   seen(a);
   a.load(a_r, lda, a_row0, a_rows, kStep, depth);
   b.load(b_r, ldb, b_row0, b_rows, kStep, depth);
@@ -144,8 +147,8 @@ __device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, in
 #pragma unroll
       for (int j = 0; j < NT; ++j) pb[j][p] = OpB::part(mine + OpA::kBytes, p, half, row_b + 32 * j);
     }
-    a.to_lds(next);                                           // (beyond depth: zeros that nobody reads)
-    b.to_lds(next + OpA::kBytes);
+    a.to_lds(next, most);                                           // (beyond depth: zeros that nobody reads)
+    b.to_lds(next + OpA::kBytes, most);
     seen(a);
     a.load(a_r, lda, a_row0, a_rows, k0 + 2 * kStep, depth);
     b.load(b_r, ldb, b_row0, b_rows, k0 + 2 * kStep, depth);
@@ -176,10 +179,13 @@ __device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, in
   }
 }
 
-// Whether the wavefront has a sum among its own that parts give no number for.  A float32 infinity, or a number next to the largest, is no
-// bfloat16 number, and an infinity times a lower part of zero is none either; and the third part of a number below 2^-108 is denormal.
-// A sum that is no finite number, or tiny, is formed again without parts.
-template <int MT, int NT> __device__ __forceinline__ bool odd_sums(const f32x16 (&acc)[MT][NT]) {
+// Whether the wavefront has a sum among its own that parts give no number for, or too coarse a one; it is then formed again without parts.
+//   * A float32 infinity, or a number next to the largest, is no bfloat16 number, and an infinity times a lower part of zero is none either:
+//     a sum that is no finite number.
+//   * The lowest part of an operand below 2^-108 is denormal, and 2^-133 of it may be lost, times its partner.  Where all partners are 2^32 or
+//     less, 4096 such products lose 2^-89: 2^-25 of a sum of 2^-64 or more.  So: a smaller sum than that (not zero: it may be 2^-89 in
+//     truth), or a larger operand in the workgroup's tile (`large`).
+template <int MT, int NT> __device__ __forceinline__ bool odd_sums(const f32x16 (&acc)[MT][NT], bool large) {
   uint32_t least = 0xFFFFFFFFu, most = 0;                     // of the sizes' bits, twice; least: without zeros, less one
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -191,8 +197,15 @@ template <int MT, int NT> __device__ __forceinline__ bool odd_sums(const f32x16 
         least = min(least, twice - 1);
         most = max(most, twice);
       }
-  const bool odd = most >= 0xFF000000u || least < (__float_as_uint(0x1p-96f) << 1) - 1;
+  const bool odd = large || most >= 0xFF000000u || least < (__float_as_uint(0x1p-64f) << 1) - 1;
   return __builtin_amdgcn_ballot_w64(odd) != 0;
+}
+
+// Whether a thread of the workgroup brought an operand beyond 2^32.  flag: zero since before the last barrier but this one.
+__device__ __forceinline__ bool any_large(float most, int *flag) {
+  if (!(most <= 0x1p32f)) *flag = 1;
+  lds_barrier();
+  return __builtin_amdgcn_readfirstlane(*flag) != 0;
 }
 
 // This lane's four of eight contraction steps from k0 on of one row, for float32 matrix instructions; arguments as of SplitOperand::load.
@@ -260,14 +273,17 @@ template <int TM, int TN>
 __global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
                                                         float *__restrict__ y, long long N, int O, int K, int tiles) {
   __shared__ __align__(16) unsigned char lds[2 * (SplitOperand<TM, false>::kBytes + SplitOperand<TN, false>::kBytes)];
+  __shared__ int large;
   const long long n0 = (blockIdx.x / (8 * tiles) * 8 + blockIdx.x % 8) * (long long)TM;
   if (n0 >= N) return;                                        // uniform
   const int o0 = blockIdx.x % (8 * tiles) / 8 * TN, ms = N - n0 < TM ? (int)(N - n0) : TM, ns = O - o0 < TN ? O - o0 : TN;
   const rsrc_t x_r = make_rsrc(x + n0 * K, (size_t)ms * K * 4), w_r = make_rsrc(w + (size_t)o0 * K, (size_t)ns * K * 4);
   f32x16 acc[TM / 64][TN / 64];
   zero_sums(acc);
-  split_product<TM, TN, false, false, 0>(lds, x_r, K, 0, 0, w_r, K, 0, 0, K, acc, [](const auto &) {});
-  if (odd_sums(acc)) {                                        // uniform
+  float most = 0;
+  if (threadIdx.x == 0) large = 0;
+  split_product<TM, TN, false, false, 0>(lds, x_r, K, 0, 0, w_r, K, 0, 0, K, acc, most, [](const auto &) {});
+  if (odd_sums(acc, any_large(most, &large))) {                                        // uniform
     zero_sums(acc);
     whole_product<TM, TN, false, false>(x_r, K, 0, 0, w_r, K, 0, 0, K, acc);
   }
@@ -278,19 +294,22 @@ __global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict_
 template <int TM, int TN, int FLUSH>
 __global__ __launch_bounds__(256, 3) void linear_sum_kernel(LinearSets sets, float *__restrict__ y, long long N, int K, int tiles) {
   __shared__ __align__(16) unsigned char lds[2 * (SplitOperand<TM, false>::kBytes + SplitOperand<TN, true>::kBytes)];
+  __shared__ int large;
   const long long n0 = (blockIdx.x / (8 * tiles) * 8 + blockIdx.x % 8) * (long long)TM;
   if (n0 >= N) return;                                        // uniform
   const int k0 = blockIdx.x % (8 * tiles) / 8 * TN, ms = N - n0 < TM ? (int)(N - n0) : TM;
   f32x16 acc[TM / 64][TN / 64];
   zero_sums(acc);
+  float most = 0;
+  if (threadIdx.x == 0) large = 0;
   auto rows = [&](const LinearSet &s) { return make_rsrc(s.rows + n0 * s.width, (size_t)ms * s.width * 4); };
   auto weight = [&](const LinearSet &s) { return make_rsrc(s.weight, (size_t)s.width * K * 4); };
   for (int i = 0; i < sets.n; ++i) {                          // uniform
     const LinearSet &s = sets.set[i];
     if (i > 0) lds_barrier();                                 // nobody reads the last set's parts any more
-    split_product<TM, TN, false, true, FLUSH>(lds, rows(s), s.width, 0, 0, weight(s), K, k0, K, s.width, acc, [](const auto &) {});
+    split_product<TM, TN, false, true, FLUSH>(lds, rows(s), s.width, 0, 0, weight(s), K, k0, K, s.width, acc, most, [](const auto &) {});
   }
-  if (odd_sums(acc)) {                                        // uniform
+  if (odd_sums(acc, any_large(most, &large))) {              // uniform
     zero_sums(acc);
     for (int i = 0; i < sets.n; ++i) {
       const LinearSet &s = sets.set[i];
@@ -320,6 +339,7 @@ __global__ __launch_bounds__(256, 2) void linear_grad_part_kernel(
     int parts, int rows, int o_tiles, int want_bias) {
   using OpG = SplitOperand<128, true>;
   __shared__ __align__(16) unsigned char lds[4 * OpG::kBytes];
+  __shared__ int large;
   const int part = blockIdx.x % parts, tile = blockIdx.x / parts;
   const int o0 = (tile % o_tiles) * 128, k0 = (tile / o_tiles) * 128;
   const long long n0 = (long long)part * rows;
@@ -328,13 +348,15 @@ __global__ __launch_bounds__(256, 2) void linear_grad_part_kernel(
   const rsrc_t x_r = make_rsrc(x + (n_rows > 0 ? n0 * K : 0), (size_t)n_rows * K * 4);
   f32x16 acc[2][2];
   zero_sums(acc);
+  float most = 0;
+  if (threadIdx.x == 0) large = 0;
   float bias_sum = 0;                                       // of this thread's column and every other eight rows
-  split_product<128, 128, true, true, 64>(lds, g_r, O, o0, O, x_r, K, k0, K, n_rows, acc, [&](const OpG &a) {
+  split_product<128, 128, true, true, 64>(lds, g_r, O, o0, O, x_r, K, k0, K, n_rows, acc, most, [&](const OpG &a) {
     const float *v = a.v[0];                                // a tree per batch: a chain of rows would round more
     bias_sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   });
   float *mine = partial + (size_t)part * ((size_t)O * K + O);
-  if (odd_sums(acc)) {                                      // uniform
+  if (odd_sums(acc, any_large(most, &large))) {             // uniform
     zero_sums(acc);
     whole_product<128, 128, true, true>(g_r, O, o0, O, x_r, K, k0, K, n_rows, acc);
   }

@@ -70,6 +70,35 @@ def test_operands_that_are_no_ordinary_numbers():
     torch.testing.assert_close(gw, g.t().mm(x), rtol=1e-4, atol=1e-2, equal_nan=True)
 
 
+@pytest.mark.parametrize("tiny,huge", [(-122, 100), (-140, 100), (-112, 33), (-120, 60), (-112, 31), (-109, 25)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_tiny_operands_with_large_partners(tiny, huge, mixed):
+    """The lowest parts of the tiny operands are denormal numbers, or nothing is left of them at all; the sums are ordinary ones.  `mixed`:
+    beside ordinary operands, in tiles of their own and in the same ones."""
+    from dfa3D.modules import projection
+    dev = torch.device("cuda:0")
+    torch.manual_seed(4)
+    x, w, g = torch.randn(4200, 64, device=dev), torch.randn(96, 64, device=dev), torch.randn(4200, 96, device=dev)
+    some = slice(100, 140) if mixed else slice(None)
+    x[some] *= 2.0 ** tiny                                   # denormals of float32 are rounded here: the products are of what is left
+    w *= 2.0 ** huge
+    if mixed:
+        x[:40, 5] *= 2.0 ** tiny
+    rows = slice(some.start, some.stop) if mixed else slice(None)
+    want = x.double() @ w.double().t()
+    for got in (projection._product(x, w, None), projection._sum_of_products((x, w.t().contiguous())), projection._sum_of_products((x, w.t().contiguous()) * 2) / 2):
+        # as ordinary operands (test_product): some 1e-7 of the 2-norm, each part of the rows by itself
+        for part in (rows, slice(None)):
+            assert (got[part].double() - want[part]).norm() <= 1e-6 * want[part].norm()
+    g *= 2.0 ** huge
+    got, _ = projection._weight_gradients(x, g, False)
+    assert (got.double() - g.double().t() @ x.double()).norm() <= 1e-6 * (g.double().t() @ x.double()).norm()
+    if mixed:
+        g[:100], g[140:] = 0, 0                              # the tiny rows alone
+        got, _ = projection._weight_gradients(x, g, False)
+        assert (got.double() - g.double().t() @ x.double()).norm() <= 1e-6 * (g.double().t() @ x.double()).norm()
+
+
 def test_gradients_that_are_no_numbers_take_no_walk():
     """A loss that is NaN or infinite leaves gradients of which every sum is formed again: by matrix instructions (measured: two or
     three times a finite step's time), not by one lane's loop over the rows per element (55 to 105 times)."""
