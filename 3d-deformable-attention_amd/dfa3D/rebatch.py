@@ -20,7 +20,7 @@ def camera_count(hit):
     if not (hit.is_cuda and hit.dtype == torch.bool and hit.is_contiguous() and 0 < cams <= 65535 and 0 < Nq <= 2 ** 30):
         return None
     totals = torch.empty(cams, dtype=torch.int32, device=hit.device)
-    on_host = torch.empty(cams, dtype=torch.int32, pin_memory=True)
+    on_host = torch.empty(cams, dtype=torch.int32, device="cpu", pin_memory=True)      # (whatever the default device)
     with _lib.on_device(hit.device):
         rc = _lib.lib().dfa3d_camera_count(_lib.ptr(hit), _lib.ptr(totals), cams, Nq, _lib.stream_of(hit))
         _lib.check(rc, "dfa3d_camera_count")

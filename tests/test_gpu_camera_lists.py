@@ -79,6 +79,16 @@ def test_counting_started_ahead():
     assert camera_count(hit.t()) is None and camera_count(hit.float()) is None and camera_count(hit.cpu()) is None
 
 
+def test_lists_under_a_default_device():
+    """A program whose new tensors go to the GPU unless it says otherwise: the counts still come to host memory."""
+    from dfa3D.rebatch import camera_index
+    hit = torch.rand(6, 500, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda") < 0.3
+    want = camera_index(hit)
+    with torch.device("cuda"):
+        got = camera_index(hit)
+    assert got[2] == want[2] and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("train", [False, True])
 def test_layer_with_the_value_side_first(train):
     """Launched before the camera lists, and inside the attention module, as it is where a hook looks on: the same result."""
