@@ -43,7 +43,9 @@ def _widths_apply(O, K):
 def _product(x, weight, bias):
     """``F.linear`` that nothing records, or None where the kernel does not form it (csrc/dfa3d_binding.cpp says where
     it does) or it is to be recorded."""
-    if not x.is_cuda or torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
+    # (the type first: a symbolic tracer's proxy has no truth value)
+    if (type(x) not in (torch.Tensor, nn.Parameter) or not x.is_cuda or torch.compiler.is_compiling()
+            or torch.autograd.forward_ad._current_level >= 0):
         return None
     at = torch._C._cuda_getDevice()
     return _lib.binding().linear(at, torch._C._cuda_getCurrentRawStream(at), x, weight, bias)

@@ -187,3 +187,15 @@ def test_projection_workspace_stays_small():
                 for rows in (4096, 48000, 184950, 500000):
                     assert _lib.lib().dfa3d_linear_grad_workspace_bytes(rows, O, K) <= 65 << 20, (rows, O, K)
     assert taken >= 30 and not _widths_apply(2048, 2048) and not _widths_apply(3, 4)
+
+
+@pytest.mark.parametrize("library_forward", [False, True])
+def test_projection_is_traced_symbolically(library_forward):
+    """torch.fx and torch.jit.trace of a layer that nothing records."""
+    import torch.fx
+    from dfa3D.modules.projection import Projection
+    layer, x = Projection(8, 6, library_forward=library_forward), torch.randn(5, 8)
+    with torch.no_grad():
+        want = F.linear(x, layer.weight, layer.bias)
+        assert torch.equal(torch.fx.symbolic_trace(layer)(x), want)
+        assert torch.equal(torch.jit.trace(layer, x)(x), want)
