@@ -179,10 +179,24 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         dist = value_dpt_dist.reshape(bs, num_value, 1, dim_depth).to(value.dtype)
         return value, dist, self.get_spatial_shape_3D(spatial_shapes, dim_depth)
 
-    def value_side(self, value, value_dpt_dist, spatial_shapes):
-        """What ``forward`` makes of ``value`` (bs, keys, embed_dims), ``value_dpt_dist`` and ``spatial_shapes`` alone."""
+    def value_side(self, value, value_dpt_dist, spatial_shapes, key_padding_mask=None):
+        """What ``forward`` makes of ``value`` (bs, keys, embed_dims), ``value_dpt_dist``, ``spatial_shapes`` and
+        ``key_padding_mask`` alone."""
         self._check_values(value, value_dpt_dist, spatial_shapes)
-        return self._value_side(value, value_dpt_dist, spatial_shapes, None)
+        return self._value_side(value, value_dpt_dist, spatial_shapes, key_padding_mask)
+
+    def _check_value_side(self, value_side, bs, value, key_padding_mask):
+        """``value``: (bs, keys, embed_dims) as given to ``forward`` beside ``value_side``, or None."""
+        if key_padding_mask is not None:
+            raise ValueError("key_padding_mask has no effect on a value_side that is given: hand it to value_side()")
+        projected, dist, shapes = value_side
+        if projected.dim() != 4 or projected.shape[0] != bs or projected.shape[2] != self.num_heads:
+            raise ValueError(f"value_side holds values of shape {tuple(projected.shape)}, the queries are {bs} batch elements "
+                             f"for {self.num_heads} heads")
+        if value is not None and value.shape[:2] != projected.shape[:2]:
+            raise ValueError(f"value_side holds {tuple(projected.shape[:2])} values, value {tuple(value.shape[:2])}")
+        if dist.shape[:2] != projected.shape[:2] or shapes.shape[0] != self.num_levels:
+            raise ValueError("value_side is none of this module's")
 
     def forward(self, query, key=None, value=None, value_dpt_dist=None, identity=None, query_pos=None,
                 key_padding_mask=None, reference_points=None, spatial_shapes=None, level_start_index=None,
@@ -194,8 +208,9 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         ``return_depth_score=True`` a third result, the operator's depth scores.  ``packed_dist``: what
         ``self.pack_dist(value_dpt_dist, spatial_shapes, level_start_index)`` returned for this very distribution;
         an encoder that runs several of these layers on one distribution packs once and hands it to each.
-        ``value_side``: what ``self.value_side(value, value_dpt_dist, spatial_shapes)`` returned, for a caller that has
-        the values before the queries."""
+        ``value_side``: what ``self.value_side(value, value_dpt_dist, spatial_shapes, key_padding_mask)`` returned, for a
+        caller that has the values before the queries; there ``value`` is batch first, and the mask is not given again."""
+        given = value
         if value is None:
             value = query
         if query_pos is not None:
@@ -206,6 +221,8 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         bs, num_query, _ = query.shape
         if value_side is None:
             self._check_values(value, value_dpt_dist, spatial_shapes)
+        else:
+            self._check_value_side(value_side, bs, value if given is not None else None, key_padding_mask)
         # the largest launches first: the GPU works on them while the host prepares the others
         together = getattr(self.sampling_locations, "__func__", None) is MSDeformableAttention3D_DFA3D.sampling_locations
         if together:

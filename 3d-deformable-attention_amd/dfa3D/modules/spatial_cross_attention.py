@@ -93,7 +93,7 @@ class SpatialCrossAttention_DFA3D(nn.Module):
         value_dpt_dist = value_dpt_dist.permute(2, 0, 1, 3).reshape(bs * cams, keys, value_dpt_dist.shape[-1])
         attention = self.deformable_attention
         ours = type(attention) is MSDeformableAttention3D_DFA3D
-        if ours and attention.batch_first and no_hooks(attention) and kwargs.get("key_padding_mask") is None:
+        if ours and attention.batch_first and no_hooks(attention):
             kwargs["value_side"] = attention.value_side(value, value_dpt_dist, spatial_shapes)
         index, pos, max_len = camera_index(hit, counted)
         queries_rebatch = RebatchGatherFunction.apply(query, index, pos)         # (bs, cams, max_len, E)

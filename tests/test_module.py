@@ -199,3 +199,34 @@ def test_projection_is_traced_symbolically(library_forward):
         want = F.linear(x, layer.weight, layer.bias)
         assert torch.equal(torch.fx.symbolic_trace(layer)(x), want)
         assert torch.equal(torch.jit.trace(layer, x)(x), want)
+
+
+def test_value_side_is_checked():
+    """A value side prepared ahead: with a mask that it does not hold, or made of other values, it is refused."""
+    m = _randomise(_module(embed_dims=16, num_heads=2, num_levels=3, num_points=4).double())
+    query, value, dist, ref, shapes, lsi, _ = _inputs()
+    kw = dict(value=value, value_dpt_dist=dist, reference_points=ref, spatial_shapes=shapes, level_start_index=lsi)
+    side = m.value_side(value, dist, shapes)
+    with pytest.raises(NotImplementedError):                  # accepted (and no GPU)
+        m(query, value_side=side, **kw)
+    mask = torch.zeros(value.shape[:2], dtype=torch.bool)
+    with pytest.raises(ValueError, match="key_padding_mask"):
+        m(query, value_side=side, key_padding_mask=mask, **kw)
+    for other in (m.value_side(value[:1], dist[:1], shapes), m.value_side(value[:, :-1], dist[:, :-1], shapes),
+                  (side[0].flatten(2), *side[1:]), (*side[:2], side[2][:2]), (side[0], side[1][:, 1:], side[2])):
+        with pytest.raises(ValueError, match="value_side"):
+            m(query, value_side=other, **kw)
+    mask[:, 7:] = True
+    assert (m.value_side(value, dist, shapes, mask)[0][:, 7:] == 0).all() and torch.equal(m.value_side(value, dist, shapes, mask)[0][:, :7], side[0][:, :7])
+
+
+@pytest.mark.gpu
+def test_masked_value_side_and_masked_call():
+    dev = torch.device("cuda:0")
+    m = _randomise(_module(embed_dims=16, num_heads=2, num_levels=3, num_points=4)).to(dev)
+    query, value, dist, ref, shapes, lsi, _ = (t.to(dev) if torch.is_tensor(t) else t for t in _inputs(dtype=torch.float32))
+    kw = dict(value=value, value_dpt_dist=dist, reference_points=ref, spatial_shapes=shapes, level_start_index=lsi)
+    mask = torch.rand(value.shape[:2], generator=torch.Generator().manual_seed(5)).to(dev) < 0.4
+    want = m(query, key_padding_mask=mask, **kw)
+    got = m(query, value_side=m.value_side(value, dist, shapes, mask), **kw)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and not torch.equal(want[0], m(query, **kw)[0])
