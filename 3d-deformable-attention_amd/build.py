@@ -3,7 +3,8 @@
     python 3d-deformable-attention_amd/build.py [--force] [--clocks]
 
 The library lands next to the python package (dfa3D/libdfa3d_hip.so) so that it travels with
-the source tree, as does the module that calls it with torch's tensors (dfa3D/_binding.so, host code).
+the source tree, as does the module that calls it with torch's tensors (dfa3D/_binding.*.so, host code).  That module fits
+one torch and one Python and is built again when either is another; where it cannot be built, calls go through ctypes.
 Two more libraries land beside bench.py, which is what uses them: the yardstick kernels (libdfa3d_measure.so) and, with --clocks, libdfa3d_hip_clocks.so: the same sources compiled with
 -DDFA3D_TILE_TIMING, i.e. with the per-phase clocks of the backward's tile kernels (`bench.py --phase-costs`).
 """
@@ -18,7 +19,8 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "dfa3D", "libdfa3d_hip.so")
 BINDING_SRC = os.path.join(CSRC, "dfa3d_binding.cpp")
-BINDING = os.path.join(HERE, "dfa3D", "_binding.so")
+BINDING = os.path.join(HERE, "dfa3D", "_binding" + sysconfig.get_config_var("EXT_SUFFIX"))      # named for this Python
+BINDING_STAMP = os.path.join(OBJ, "binding.built_for")
 # yardstick kernels for bench.py (plain copy, bare gathers, LDS atomics, XCD map): not part of the operator library
 MEASURE_SRC = os.path.join(CSRC, "measure", "dfa3d_measure.hip")
 ROOT = os.path.dirname(HERE)
@@ -68,16 +70,37 @@ def _build_lib(lib, obj_dir, extra_flags, force, verbose):
     return lib
 
 
+def _binding_stale(built_for):
+    """`built_for`: the torch that is installed (dfa3D/_lib.py compares it with what the module was built for)."""
+    if (_stale(BINDING, [BINDING_SRC, os.path.join(ROOT, "include", "dfa3d.h"), os.path.abspath(__file__)])
+            or not os.path.exists(BINDING_STAMP)):
+        return True
+    with open(BINDING_STAMP) as f:
+        return f.read() != built_for
+
+
 def _build_binding(force, verbose):
-    if not (force or _stale(BINDING, [BINDING_SRC, os.path.join(ROOT, "include", "dfa3d.h"), os.path.abspath(__file__)])):
-        return
-    import torch
-    from torch.utils import cpp_extension
-    includes = [f"-isystem{d}" for d in cpp_extension.include_paths()]
-    libs = [f"-L{d}" for d in cpp_extension.library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10"]
-    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
-          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I" + sysconfig.get_paths()["include"], *includes,
-          BINDING_SRC, "-o", BINDING, *libs], verbose)
+    """Whether the module is there and up to date."""
+    try:
+        import torch
+        from torch.utils import cpp_extension
+        built_for = f"{torch.__version__} {torch.version.git_version}"
+        if not (force or _binding_stale(built_for)):
+            return True
+        includes = [f"-isystem{d}" for d in cpp_extension.include_paths()]
+        libs = [f"-L{d}" for d in cpp_extension.library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10"]
+        _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DDFA3D_BUILT_FOR="{built_for}"',
+              "-I" + sysconfig.get_paths()["include"], *includes, BINDING_SRC, "-o", BINDING, *libs], verbose)
+    except (ImportError, OSError, subprocess.CalledProcessError) as e:
+        print(f"{BINDING} is not built ({e}): calls go through ctypes, which takes 5 to 10 us longer each", file=sys.stderr)
+        if os.path.exists(BINDING):
+            os.remove(BINDING)                   # of other sources or another torch
+        return False
+    os.makedirs(os.path.dirname(BINDING_STAMP), exist_ok=True)
+    with open(BINDING_STAMP, "w") as f:
+        f.write(built_for)
+    return True
 
 
 def build(force=False, verbose=True, clocks=False):

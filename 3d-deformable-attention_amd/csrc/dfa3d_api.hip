@@ -86,7 +86,7 @@ int check_dims(const char *fn, int B, int S, int M, int width, int L, int Q, int
 extern "C" {
 
 const char *dfa3d_last_error(void) { return g_err; }
-int dfa3d_abi_version(void) { return 9; }
+int dfa3d_abi_version(void) { return DFA3D_ABI_VERSION; }
 
 #ifdef DFA3D_TILE_TIMING
 size_t dfa3d_tile_timer_offset(void) { return dfa3d::tile_timer_offset(); }

@@ -424,6 +424,10 @@ PyObject *linear_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// built_for() -> (version of the torch that this module was compiled against, version of the library's interface).  It touches no
+// tensor and nothing of torch's: another torch's module says so before anything of it runs.
+PyObject *built_for(PyObject *, PyObject *) { return Py_BuildValue("(si)", DFA3D_BUILT_FOR, DFA3D_ABI_VERSION); }
+
 // bind(dict of entry point -> address)
 PyObject *bind(PyObject *, PyObject *table) {
   auto address = [&](const char *name, auto &to) {
@@ -455,6 +459,7 @@ PyObject *bind(PyObject *, PyObject *table) {
 typedef PyObject *(*Fast)(PyObject *, PyObject *const *, Py_ssize_t);
 PyCFunction as_method(Fast f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)); }
 PyMethodDef methods[] = {
+    {"built_for", built_for, METH_NOARGS, nullptr},
     {"bind", bind, METH_O, nullptr},
     {"fused_forward", as_method(fused_forward), METH_FASTCALL, nullptr},
     {"fused_gradients", as_method(fused_gradients), METH_FASTCALL, nullptr},

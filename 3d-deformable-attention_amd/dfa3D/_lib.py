@@ -5,8 +5,10 @@ shared object is missing or a tensor is not on a GPU, the call raises.
 """
 import contextlib
 import ctypes
+import importlib
 import os
 import threading
+import warnings
 
 import torch
 
@@ -74,10 +76,28 @@ _binding = None
 
 
 def binding():
-    """The binding module, on the library that ``lib()`` loaded."""
+    """The binding module, on the library that ``lib()`` loaded, or None: calls then go through ctypes."""
     if _lib is None:
         lib()
     return _binding
+
+
+def _load_binding(handle):
+    """The binding module, told where the library's entry points are; None (and a warning) where it is not built, or was built
+    for another torch, whose tensors it would misread, or for another version of the library's interface."""
+    try:
+        module = importlib.import_module(__package__ + "._binding")
+        built_for, abi = module.built_for()
+        here = f"{torch.__version__} {torch.version.git_version}"
+        if built_for != here or abi != ABI_VERSION:
+            raise ImportError(f"it was built for torch {built_for} and ABI version {abi}, this is {here} and {ABI_VERSION}")
+    except (ImportError, AttributeError) as e:
+        warnings.warn(f"dfa3D: calls go through ctypes, which takes 5 to 10 us longer each, and projections by the library where "
+                      f"nothing is recorded: the binding module does not load ({e}); "
+                      "`python 3d-deformable-attention_amd/build.py --force` builds it", RuntimeWarning, stacklevel=3)
+        return None
+    module.bind({name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in _BOUND})
+    return module
 
 
 def lib():
@@ -109,13 +129,7 @@ def lib():
         handle.dfa3d_last_error.restype = ctypes.c_char_p
         if handle.dfa3d_abi_version() != ABI_VERSION:
             raise ImportError(f"{LIB_PATH}: ABI version {handle.dfa3d_abi_version()} != expected {ABI_VERSION}; rebuild")
-        try:
-            from . import _binding as module
-        except ImportError as e:
-            raise ImportError(f"{_HERE}/_binding.so is missing or does not fit this torch: build it with "
-                              f"`python 3d-deformable-attention_amd/build.py` ({e})") from e
-        module.bind({name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in _BOUND})
-        _lib, _binding = handle, module
+        _binding, _lib = _load_binding(handle), handle           # in this order: binding() of another thread looks at _lib
     return _lib
 
 

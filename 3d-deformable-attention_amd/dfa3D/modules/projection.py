@@ -47,16 +47,22 @@ def _product(x, weight, bias):
     if (type(x) not in (torch.Tensor, nn.Parameter) or not x.is_cuda or torch.compiler.is_compiling()
             or torch.autograd.forward_ad._current_level >= 0):
         return None
+    native = _lib.binding()
+    if native is None:
+        return None
     at = torch._C._cuda_getDevice()
-    return _lib.binding().linear(at, torch._C._cuda_getCurrentRawStream(at), x, weight, bias)
+    return native.linear(at, torch._C._cuda_getCurrentRawStream(at), x, weight, bias)
 
 
 def _sum_of_products(operands):
     """Sum of rows (..., O) times weight (O, K) over the flat tuple of them, or None as above."""
     if not operands[0].is_cuda:
         return None
+    native = _lib.binding()
+    if native is None:
+        return None
     at = torch._C._cuda_getDevice()
-    return _lib.binding().linear_sum(at, torch._C._cuda_getCurrentRawStream(at), operands)
+    return native.linear_sum(at, torch._C._cuda_getCurrentRawStream(at), operands)
 
 
 def _linear(x, weight, bias, library):
