@@ -462,15 +462,23 @@ hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int6
 //     rows.  Kernel, us, memory and LDS, 920 rows of 32 channels, points per workgroup 500: 8.6, 11.0   640: 11.6, 12.9   800: 11.9, 12.9
 //     1000: 13.3, 12.6   1600: 19.6, 17.2   6400: 53.4, 41.0; 504 rows, 720 points: 10.7, 10.1; 384 rows, 800 points: 10.9, 10.6.
 //   * The coarser levels of a pyramid fit (the level sizes are on the device; each is taken for a quarter of the one before): one
-//     (batch, head) at a time on an XCD, as its L2 holds no more, so M has to divide 8 or be a multiple of it.  A workgroup's start
-//     and end cost as much as about a thousand points, LDS saves half of a point's lines (plain attention all): from 1200 points on levels in
-//     LDS, so far as one can tell.  Memory and LDS, points per workgroup x share of the levels, operands that change from call to call:
-//     5000 x 1/4: 522, 495; scores given 309, 283; plain 266, 252   bfloat16 plain 216, 185   2500 x 1/2: 191, 196; 128, 113; plain 103, 94
-//     3000 x 1/3: 117, 113; 70, 71; plain 49, 54   2800 x 1/3: 127, 124; 82, 84; plain 59, 67   1500 x 1/4: 194, 213; 118, 124; plain 108, 116
-//     and the same operands again and again:
-//     10000 x 1/4: 914, 864   8000 x 1/2: 610, 535   4000 x 1/2: 240, 226; plain 171, 154; 120, 114   3500 x 1/4: 349, 370   3500 x 1/2: plain 52, 54
-//     2000 x 1/2: 106, 109; plain 73, 77   1000 x 3/4: 76, 89.  Not with packed distributions, which a cross-attention layer uses: its
-//     points share a pillar's few pixels, whose rows the L1 has (200 x 200 queries, base maps 412, 432; 120 x 120, 30 x 48 226, 239).
+//     (batch, head) at a time on an XCD, as its L2 holds no more, so M has to divide 8 or be a multiple of it.  What a workgroup spends on
+//     its start, its end and fewer wavefronts is worth some thousand points; what LDS saves of a point on a level that it holds is half of its
+//     lines of float32 rows and of bfloat16 ones, which cost less (plain attention all).  Memory over LDS, maps from 58 x 100, 80 x 128 and 116 x 200 in
+//     three or four levels, locations anywhere and around the query, operands that change from call to call, lowest and highest:
+//       points per workgroup, share of the levels in LDS   2500 x 1/2    3500 x 1/2    5000 x 1/4    5000 x 1/3    5000 x 1/2    8000 x 1/2
+//       float32, one stage                                 0.94 - 1.01   0.96 - 1.02   0.99 - 1.05   0.96 - 1.10   1.07 - 1.12   1.06 - 1.15
+//       scores given                                       0.99 - 1.14   0.99 - 1.14   1.03 - 1.09   1.02 - 1.05   1.13 - 1.19   1.21 - 1.24
+//       plain attention                                    0.97 - 1.11   0.94 - 1.08   1.03 - 1.04   1.02 - 1.03   1.05 - 1.12   1.10 - 1.17
+//       bfloat16, one stage                                0.87 - 0.92   0.87 - 0.93                 0.93 - 0.97   0.99 - 1.02   0.99 - 1.07
+//       scores given                                       0.90 - 1.01   0.89 - 0.99                 0.95 - 0.99   0.98 - 1.08   1.04 - 1.13
+//       plain attention                                    0.87 - 1.04   0.89 - 1.02                 1.01 - 1.06   1.05 - 1.14   1.10 - 1.19
+//     (12000 x 1/2: bfloat16, one stage 1.03 - 1.09; float32, scores given, below 1000 points on levels in LDS 0.84 - 1.05.)  On the same operands again
+//     and again, which the Infinity Cache then holds, plain attention 0.88 - 0.92 at 5000 x 1/4, 1.22 at 8000 x 1/4.  So: from 5000 points (bfloat16 in one
+//     stage 8000; float32 with scores fewer) of which 1300 (bfloat16 2400) are on levels in LDS.
+//     Levels that are no such pyramid (equal ones, or coarse to fine) may have none that fits; such a call takes 1 to 12 % longer than from memory.
+//     Not with packed distributions, which a cross-attention layer uses: its points share a pillar's few pixels, whose rows the L1 has
+//     (200 x 200 queries, base maps 412, 432; 120 x 120, 30 x 48 226, 239).
 template <typename T, int VEC, int LPR> constexpr bool kLdsRowsTiling = sizeof(T) <= 4 && VEC == 4 && LPR <= 16;
 struct LdsRows { int parts, rows; };
 template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a) {
@@ -490,7 +498,9 @@ template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a)
   int in_lds = 0;
   for (int l = 1; l < a.L; ++l) all = 4 * all + 1;          // (at most 16 levels)
   for (; in_lds + 1 < a.L && 1.1 * a.S * some <= (double)room * all; ++in_lds) some = 4 * some + 1;
-  if (points * in_lds < parts * 1200 * a.L) return none;
+  constexpr bool k16 = sizeof(T) == 2;
+  const long long least = a.dist != nullptr ? (k16 ? 8000 : 5000) : (!k16 && a.score_in != nullptr) ? 0 : 5000;
+  if (points < parts * least || points * in_lds < parts * (k16 ? 2400 : 1300) * a.L) return none;
   return LdsRows{(int)parts, (int)room};
 }
 
