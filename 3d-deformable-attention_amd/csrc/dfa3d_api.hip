@@ -537,7 +537,7 @@ int dfa3d_linear(const float *x, const float *weight, const float *bias, float *
 
 int dfa3d_linear_sum(const dfa3d_linear_set *layers, int n_layers, float *y, long long N, int K, void *stream) {
   const char *fn = "dfa3d_linear_sum";
-  if (n_layers < 1 || n_layers > dfa3d::kMaxLinearSets) return fail(DFA3D_EINVAL, "%s: 1 to %d layers (%d)", fn, dfa3d::kMaxLinearSets, n_layers);
+  if (n_layers < 1 || n_layers > DFA3D_MAX_LINEAR_SETS) return fail(DFA3D_EINVAL, "%s: 1 to %d layers (%d)", fn, DFA3D_MAX_LINEAR_SETS, n_layers);
   REQUIRE_PTR(fn, layers); REQUIRE_PTR(fn, y);
   dfa3d::LinearSets sets{};
   sets.n = n_layers;

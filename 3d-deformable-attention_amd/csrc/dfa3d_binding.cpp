@@ -359,11 +359,10 @@ bool product_applies(int64_t rows, int64_t width, int64_t depth) {
   return width > 0 && depth > 0 && width <= 4096 && depth <= 4096 && width % 2 == 0 && depth % 4 == 0 && rows > 0 && rows <= (int64_t(1) << 31) &&
          (depth <= 256 || rows * width >= (int64_t(1) << 22));
 }
-constexpr Py_ssize_t kMaxSets = 4;
-// pairs of a flat tuple, 0 where it is none of 1 to kMaxSets pairs
+// pairs of a flat tuple, 0 where it is none of 1 to as many pairs as a call takes
 Py_ssize_t pairs_of(PyObject *o) {
   const Py_ssize_t n = PyTuple_CheckExact(o) ? PyTuple_GET_SIZE(o) : 0;
-  return n % 2 == 0 && n / 2 <= kMaxSets ? n / 2 : 0;
+  return n % 2 == 0 && n / 2 <= DFA3D_MAX_LINEAR_SETS ? n / 2 : 0;
 }
 bool is_float_matrix(const Tensor &t) { return t.scalar_type() == at::kFloat && t.dim() == 2; }
 bool recorded(const Tensor &t) { return t.defined() && t.requires_grad() && c10::GradMode::is_enabled(); }
@@ -399,7 +398,7 @@ PyObject *linear_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   TAKES(3)
   const Py_ssize_t n = pairs_of(args[2]);
   if (n == 0 || at::autocast::is_autocast_enabled(at::kCUDA) || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer)) return declined();
-  dfa3d_linear_set sets[kMaxSets];
+  dfa3d_linear_set sets[DFA3D_MAX_LINEAR_SETS];
   int64_t K = 0, rows = 0;
   std::vector<int64_t> sizes;
   for (Py_ssize_t i = 0; i < n; ++i) {

@@ -190,7 +190,7 @@ template <typename A> struct RowVec<__hip_bfloat16, A, 8> {      // loads only: 
   }
 };
 
-// The same elements of a row that lies in LDS, and the copy that brings them there (BYTES: of VEC elements, a power of two).
+// The same elements of a row that lies in LDS, and the copy that brings them there (BYTES: of four elements).
 template <typename T, typename A, int VEC> __device__ __forceinline__ void lds_row(const unsigned char *at, A (&v)[VEC]) {
   struct alignas(VEC * sizeof(T)) Elems { T e[VEC]; };
   const Elems x = *reinterpret_cast<const Elems *>(at);
@@ -198,8 +198,6 @@ template <typename T, typename A, int VEC> __device__ __forceinline__ void lds_r
   for (int i = 0; i < VEC; ++i) v[i] = Elem<T>::ld(&x.e[i]);
 }
 template <int BYTES> struct RawPiece;
-template <> struct RawPiece<2> { uint16_t w; __device__ __forceinline__ void ld(rsrc_t r, uint32_t off) { w = __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0); } };
-template <> struct RawPiece<4> { uint32_t w; __device__ __forceinline__ void ld(rsrc_t r, uint32_t off) { w = __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0); } };
 template <> struct RawPiece<8> { u32x2 w; __device__ __forceinline__ void ld(rsrc_t r, uint32_t off) { w = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0); } };
 template <> struct RawPiece<16> { u32x4 w; __device__ __forceinline__ void ld(rsrc_t r, uint32_t off) { w = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0); } };
 

@@ -159,9 +159,8 @@ hipError_t launch_locations_grad(const float *grad_loc, const int64_t *shapes3, 
 
 // Linear layers (dfa3d_linear.hip): y (N, O) = x (N, K) w (O, K)^T + bias (or nullptr), and y (N, K) = sum over the sets of rows (N, width) weight
 // (width, K); O, K and widths even, K (widths) a multiple of four in the first (second).
-constexpr int kMaxLinearSets = 4;
 struct LinearSet { const float *weight, *rows; int width; };
-struct LinearSets { LinearSet set[kMaxLinearSets]; int n; };
+struct LinearSets { LinearSet set[DFA3D_MAX_LINEAR_SETS]; int n; };
 hipError_t launch_linear(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream);
 hipError_t launch_linear_sum(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream);
 // Weight and bias gradients of a linear layer (dfa3d_linear.hip); O and K even.

@@ -24,8 +24,6 @@ def ordinary(*tensors):
             and torch.autograd.forward_ad._current_level < 0)
 
 
-_MAX_SHARED = 4        # layers that one launch takes (kMaxLinearSets)
-
 # Fewer rows than this: the library product is as fast and there is one launch less.
 _MIN_ROWS = 4096
 
@@ -211,7 +209,7 @@ def _bare(layer):
 def projections(x, layers):
     """``[layer(x) for layer in layers]``; where the layers are plain ``Projection``s, at most four, the gradient of
     ``x`` is formed in one kernel.  The layer of the base model, training: 3811 -> 3771 us."""
-    if len(layers) <= _MAX_SHARED and all(_bare(l) for l in layers) and _applies(x, *layers):
+    if len(layers) <= _lib.MAX_LINEAR_SETS and all(_bare(l) for l in layers) and _applies(x, *layers):
         params = [t for l in layers for t in (l.weight, l.bias)]
         return list(_SharedRowsFunction.apply(tuple(l.library_forward for l in layers), x, *params))
     return [layer(x) for layer in layers]

@@ -52,6 +52,7 @@ extern "C" {
 #define DFA3D_BF16G 3
 
 #define DFA3D_MAX_LEVELS 16
+#define DFA3D_MAX_LINEAR_SETS 4   /* layers of one dfa3d_linear_sum call */
 
 /* Launch options of ONE call.  NULL, or a zero-filled structure, means the defaults.  They choose how the
  * work is laid out on the machine (and, `clear`, who zeroes two output buffers) and never what is computed:
