@@ -49,21 +49,48 @@ def _run(o, kind):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16], ids=["fp32", "fp64", "bf16"])
 @pytest.mark.parametrize("kind", ["one_stage", "weight_update", "weight_update_one", "stage_1", "stage_2", "plain"])
 def test_both_ways(monkeypatch, kind, dtype):
-    from dfa3D import _ext
-    o = _operands(dtype, one=kind == "weight_update_one")
+    from dfa3D import _ext, _lib
+
+    class Watched:
+        """The binding module; notes what was called and whether it took the call."""
+        def __init__(self):
+            self.took = {}
+
+        def __getattr__(self, name):
+            call = getattr(_lib.binding(), name)
+
+            def watched(*args):
+                got = call(*args)
+                self.took[name] = self.took.get(name, True) and got is not None
+                return got
+            return watched
+    watched, here = Watched(), _ext._here
+    monkeypatch.setattr(_ext, "_here", lambda value: (watched, *here(value)[1:]))
+    one = kind == "weight_update_one"
+    o = _operands(dtype, one=one)
     kind = kind.replace("_one", "") if kind == "weight_update_one" else kind
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
         short = _run(o, kind)
     torch.cuda.current_stream().wait_stream(side)
+    names = {"stage_1": ("score_forward", "score_gradients"), "one_stage": ("fused_forward", "fused_gradients"),
+             "weight_update": ("fused_forward", "fused_gradients")}.get(kind, ("attention_forward", "attention_gradients"))
+    assert all(watched.took.get(n) for n in names) and all(took for n, took in watched.took.items() if n != "pack_dist")
+    if one and dtype != torch.float64:
+        assert watched.took["pack_dist"]
     monkeypatch.setattr(_ext, "_here", lambda value: None)
     long = _run(o, kind)
     assert len(short) == len(long)
-    for a, b in zip(short, long):
+    outputs = 1 if kind in ("stage_1", "stage_2", "plain") else 2
+    # gradients are added up atomically in no fixed order: a few hundred terms per element
+    tol = {torch.float32: dict(rtol=1e-5, atol=1e-4), torch.float64: dict(rtol=1e-12, atol=1e-12), torch.bfloat16: dict(rtol=2 ** -6, atol=1e-2)}[dtype]
+    for i, (a, b) in enumerate(zip(short, long)):
         assert a.dtype == b.dtype and a.shape == b.shape
-        # gradients are added up atomically in no fixed order: a few hundred terms per element
-        torch.testing.assert_close(a.double(), b.double(), rtol=2 ** -6 if dtype == torch.bfloat16 else 1e-5, atol=1e-2 if dtype == torch.bfloat16 else 1e-4)
+        if i < outputs:
+            assert torch.equal(a, b)                                        # no atomics
+        else:
+            torch.testing.assert_close(a, b, **tol)
 
 
 def _strided(t):

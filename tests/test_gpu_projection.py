@@ -70,6 +70,66 @@ def test_operands_that_are_no_ordinary_numbers():
     torch.testing.assert_close(gw, g.t().mm(x), rtol=1e-4, atol=1e-2, equal_nan=True)
 
 
+def _error(got, want):
+    return ((got.double() - want).norm() / want.norm()).item()
+
+
+@pytest.mark.parametrize("N,depth,width", [(4096, 64, 64), (5520, 256, 256), (16500, 512, 256), (4100, 1024, 1028), (8200, 2048, 516), (4096, 4096, 1024)])
+@pytest.mark.parametrize("signs", ["random", "positive"])
+def test_products_round_no_more_than_the_librarys(N, depth, width, signs):
+    """Up to the deepest sums that the kernels take: the 2-norm error against float64 is no larger than the library's for the same product
+    (measured: 0.63 to 0.87 of it from 256 terms on), and with random signs what the rounding of the sums alone makes.  Every other
+    number of parts would show: two parts leave 2.3e-6 whatever the depth."""
+    from dfa3D.modules import projection
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(depth)
+    make = torch.randn if signs == "random" else torch.rand
+    x, w = make(N, depth, generator=g, device=dev), make(width, depth, generator=g, device=dev)
+    wt, want = w.t().contiguous(), x.double() @ w.double().t()
+    for got, library in ((projection._product(x, w, None), torch.nn.functional.linear(x, w)), (projection._sum_of_products((x, wt)), x @ wt)):
+        assert got is not None
+        assert _error(got, want) <= 1.1 * _error(library, want)
+        if signs == "random":
+            # six roundings per 16 terms, each at most 2^-23 of a running sum of sqrt(terms so far) and 0.4 of that in size:
+            # (6 / 16 depth)^(1/2) 0.4 2^-23 of the result, 3e-8 depth^(1/2)
+            assert _error(got, want) <= 3e-8 * depth ** 0.5
+    # the same terms dealt to several layers
+    cut = depth // 4
+    parts = tuple(t for i in range(4) for t in (x[:, i * cut:(i + 1) * cut].contiguous(), wt[i * cut:(i + 1) * cut].contiguous()))
+    got = projection._sum_of_products(parts)
+    if got is not None:
+        assert _error(got, want) <= 1.1 * _error(x @ wt, want)
+    assert got is not None or cut > 256
+
+
+@pytest.mark.parametrize("N,widths", [(16500, (512, 256, 256)), (5520, (256, 64)), (33000, (512, 512, 512, 512))])
+def test_gradient_of_rows_that_deep_layers_share(N, widths):
+    """The offset and weight layers of the base model (512, 256 and 256 columns) and deeper sums, against the library's products and sums."""
+    from dfa3D.modules import projection
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(N)
+    gs = [torch.randn(N, o, generator=g, device=dev) for o in widths]
+    ws = [torch.randn(o, 256, generator=g, device=dev) for o in widths]
+    got = projection._sum_of_products(tuple(t for pair in zip(gs, ws) for t in pair))
+    assert got is not None
+    want = sum(a.double() @ b.double() for a, b in zip(gs, ws))
+    assert _error(got, want) <= min(1.1 * _error(sum(a @ b for a, b in zip(gs, ws)), want), 3e-8 * sum(widths) ** 0.5)
+
+
+@pytest.mark.parametrize("N", [4096, 184950, 600000])
+@pytest.mark.parametrize("signs", ["random", "positive"])
+def test_weight_gradients_round_no_more_than_the_librarys(N, signs):
+    from dfa3D.modules import projection
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(N)
+    make = torch.randn if signs == "random" else torch.rand
+    x, y = make(N, 128, generator=g, device=dev), make(N, 64, generator=g, device=dev)
+    got, bias = projection._weight_gradients(x, y, True)
+    want = y.double().t() @ x.double()
+    assert _error(got, want) <= 1.1 * _error(y.t().mm(x), want)
+    assert _error(bias, y.double().sum(0)) <= 5e-7
+
+
 @pytest.mark.parametrize("tiny,huge", [(-122, 100), (-140, 100), (-112, 33), (-120, 60), (-112, 31), (-109, 25)])
 @pytest.mark.parametrize("mixed", [False, True])
 def test_tiny_operands_with_large_partners(tiny, huge, mixed):
