@@ -353,8 +353,10 @@ PyObject *pack_dist(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 }
 
 // Where the kernels form a product of rows x width elements, sums of depth terms.  They read four neighbours of a row at a time, and take the
-// library's place except where few rows meet a deep sum: library and kernel, us, 4096 rows of 256 by 256 19, 10; 256 by 64 19, 7; sums of 512 by
-// 256 19, 22; of 2048 by 256 41, 51 to 89; of 1024 by 1024 72, 59; 20000 rows of 512 by 512 98, 70; of 2048 by 256 165, 145; 100000 of 256 by 256 123, 93.
+// library's place except where few rows meet a deep sum.  Library and kernel, us a call one after the other: 4096 rows of 256 by 256 19, 9; 256 by 64
+// 19, 8; sums of 512 by 256 19, 22; of 2048 by 256 41, 51 to 89; of 1024 by 1024 72, 58; 20000 rows of 512 by 512 98, 70; of 2048 by 256 165, 145; 100000 of
+// 256 by 256 123, 93.  The 18 to 19 are the library call's host time, which bounds it up to some 5000 rows; on the device alone (captured in a graph)
+// 100 rows of 256 by 256 30, 8, 625 rows 5.5, 8.0, 1500 rows 5.6, 8.2, 4096 rows 10, 9; of 256 by 64 4096 rows 5.4, 7.8, 10000 rows 7.3, 8.2.
 bool product_applies(int64_t rows, int64_t width, int64_t depth) {
   return width > 0 && depth > 0 && width <= 4096 && depth <= 4096 && width % 2 == 0 && depth % 4 == 0 && rows > 0 && rows <= (int64_t(1) << 31) &&
          (depth <= 256 || rows * width >= (int64_t(1) << 22));

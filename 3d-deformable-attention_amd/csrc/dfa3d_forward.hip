@@ -92,7 +92,7 @@ __device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, con
 // maps), a workgroup of 16 wavefronts brings them there once and walks through a share of the queries: four of a point's eight lines
 // less.  6 x 4000 queries, one level of 23 x 40, 8 points: 53.4 -> 41.0 us (uniform), 41.0 -> 36.4 (points around the query), bfloat16
 // 56.6 -> 51.8, one distribution for all heads 49.1 -> 40.3, plain attention 36.3 -> 28.7; 64 channels, 4 x 4000, 15 x 24: 52.2 -> 32.5.
-// On larger maps the coarser levels' rows: 6 x 10000 queries, four levels from 116 x 200, 8 points (one level in LDS): 915 -> 864 us,
+// On larger maps the coarser levels' rows: 6 x 10000 queries, four levels from 116 x 200, 8 points (one level in LDS): 915 -> 864 us (one box; 884 on others),
 // points around the query 605 -> 571; bfloat16 (two levels) 842 -> 787, 572 -> 505; plain attention 297 -> 261.  Groups are taken, not dealt:
 // dealt, a workgroup's slowest wavefront held up the CU (883, 614).  Tried with it and not kept: two workgroups of 8, 10 or 12 wavefronts per CU
 // (908, 870, 1031; 596, 625, 706), 16 gathers in flight (880, 623), the next group's locations asked for ahead (850, 581; bfloat16 951) or
@@ -463,8 +463,8 @@ hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int6
 //     1000: 13.3, 12.6   1600: 19.6, 17.2   6400: 53.4, 41.0; 504 rows, 720 points: 10.7, 10.1; 384 rows, 800 points: 10.9, 10.6.
 //   * The coarser levels of a pyramid fit (the level sizes are on the device; each is taken for a quarter of the one before): one
 //     (batch, head) at a time on an XCD, as its L2 holds no more, so M has to divide 8 or be a multiple of it.  What a workgroup spends on
-//     its start, its end and fewer wavefronts is worth some thousand points; what LDS saves of a point on a level that it holds is half of its
-//     lines of float32 rows and of bfloat16 ones, which cost less (plain attention all).  Memory over LDS, maps from 58 x 100, 80 x 128 and 116 x 200 in
+//     its start, its end and fewer wavefronts is worth some thousand points; LDS saves half of the lines of a point on a level that it holds
+//     (plain attention all), which cost less where rows are bfloat16.  Memory over LDS, maps from 58 x 100, 80 x 128 and 116 x 200 in
 //     three or four levels, locations anywhere and around the query, operands that change from call to call, lowest and highest:
 //       points per workgroup, share of the levels in LDS   2500 x 1/2    3500 x 1/2    5000 x 1/4    5000 x 1/3    5000 x 1/2    8000 x 1/2
 //       float32, one stage                                 0.94 - 1.01   0.96 - 1.02   0.99 - 1.05   0.96 - 1.10   1.07 - 1.12   1.06 - 1.15
@@ -474,8 +474,9 @@ hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int6
 //       scores given                                       0.90 - 1.01   0.89 - 0.99                 0.95 - 0.99   0.98 - 1.08   1.04 - 1.13
 //       plain attention                                    0.87 - 1.04   0.89 - 1.02                 1.01 - 1.06   1.05 - 1.14   1.10 - 1.19
 //     (12000 x 1/2: bfloat16, one stage 1.03 - 1.09; float32, scores given, below 1000 points on levels in LDS 0.84 - 1.05.)  On the same operands again
-//     and again, which the Infinity Cache then holds, plain attention 0.88 - 0.92 at 5000 x 1/4, 1.22 at 8000 x 1/4.  So: from 5000 points (bfloat16 in one
-//     stage 8000; float32 with scores fewer) of which 1300 (bfloat16 2400) are on levels in LDS.
+//     and again, part of which the Infinity Cache then holds: plain attention, 6 x 10000 queries on base maps, 4 points 265, 250 (the same ones 237, 241),
+//     8 points 457, 438 (415, 434).  So: from 5000 points (bfloat16 in one stage 8000; float32 with scores fewer) of which 1200 (bfloat16 2400)
+//     are on levels in LDS.
 //     Levels that are no such pyramid (equal ones, or coarse to fine) may have none that fits; such a call takes 1 to 12 % longer than from memory.
 //     Not with packed distributions, which a cross-attention layer uses: its points share a pillar's few pixels, whose rows the L1 has
 //     (200 x 200 queries, base maps 412, 432; 120 x 120, 30 x 48 226, 239).
@@ -500,7 +501,7 @@ template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a)
   for (; in_lds + 1 < a.L && 1.1 * a.S * some <= (double)room * all; ++in_lds) some = 4 * some + 1;
   constexpr bool k16 = sizeof(T) == 2;
   const long long least = a.dist != nullptr ? (k16 ? 8000 : 5000) : (!k16 && a.score_in != nullptr) ? 0 : 5000;
-  if (points < parts * least || points * in_lds < parts * (k16 ? 2400 : 1300) * a.L) return none;
+  if (points < parts * least || points * in_lds < parts * (k16 ? 2400 : 1200) * a.L) return none;
   return LdsRows{(int)parts, (int)room};
 }
 

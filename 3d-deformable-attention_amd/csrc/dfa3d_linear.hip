@@ -24,7 +24,9 @@
 // Library (forward and grad_x) or the float32 matrix instructions before (weight gradient), and now, us, between other kernels: 184950 rows of
 // 256 x 256 229, 177 (forward), 220, 171 (grad_x), 227, 147 (weight gradient); 58000 of 256 x 256 80, 56; 22500 45, 26; 5520 20, 12; 6600 of 256 x 64 19, 9.
 // Relative error against float64 (2-norm), the same: forward 2.0e-7, 1.7e-7 (5520 to 10^6 rows); grad_x 2.9e-7, 2.4e-7; weight gradient
-// 184950 rows 6.9e-7, 4.4e-7, 10^6 rows 1.6e-6, 9.6e-7, all positive 6.7e-8, 4.8e-8; grad_bias 2.1e-7, 2.1e-7.
+// 184950 rows 6.9e-7, 4.4e-7, 10^6 rows 1.6e-6, 9.6e-7, all positive 6.7e-8, 4.8e-8; grad_bias 2.1e-7, 2.1e-7.  Library's and these, forward
+// and grad_x alike, random signs (all positive): sums of 256 2.9e-7, 2.4e-7 (2.2e-7, 1.8e-7), 512 4.1e-7, 3.4e-7 (3.1e-7, 2.4e-7), 1024 5.7e-7, 4.9e-7
+// (4.3e-7, 2.9e-7), 2048 8.1e-7, 7.0e-7 (6.0e-7, 3.8e-7), 4096 1.2e-6, 1.0e-6 (8.5e-7, 5.3e-7).
 #include "../../include/dfa3d.h"
 #include "dfa3d_binned.h"
 #include "dfa3d_device.h"
@@ -112,8 +114,9 @@ template <int MT, int NT> __device__ __forceinline__ void zero_sums(f32x16 (&x)[
 }
 
 // acc += sum over depth contraction steps of A(m, k) B(n, k) for a TM x TN tile by four wavefronts, 2 x 2; `seen` is called with A's registers
-// once per kStep steps.  FLUSH: the matrix unit does not round its sums to nearest, which a chain of more than some hundred steps feels; its sums
-// start from zero every FLUSH steps and the vector unit adds them up.  `most`: the largest size among the operands that this thread brought.
+// once per kStep steps.  FLUSH: an instruction cuts off what lies about 2^-24 below the largest of its terms instead of rounding it (16 products of
+// 2^-27 on a sum of 1 leave 1, 16 of -2^-27 leave 1 - 2^-23; one of 3 2^-25 is rounded up), which a chain over thousands of rows of a weight
+// gradient feels; its sums start from zero every FLUSH steps and the vector unit adds them up.  Without, up to 4096 terms: see above.  `most`: the largest size among the operands that this thread brought.
 template <int TM, int TN, bool A_ACROSS, bool B_ACROSS, int FLUSH, typename Seen>
 __device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, int lda, int a_row0, int a_rows, rsrc_t b_r, int ldb, int b_row0,
                                               int b_rows, int depth, f32x16 (&acc)[TM / 64][TN / 64], float &most, const Seen &seen) {

@@ -269,7 +269,9 @@ int dfa3d_locations_grad(const float *grad_loc, const int64_t *shapes3, float *g
  *   dfa3d_linear      y (N, O) = x (N, K) weight (O, K)^T + bias (O) or NULL
  *   dfa3d_linear_sum  y (N, K) = sum over up to four layers of rows (N, width) weight (width, K): the gradient of the rows that the layers
  *                     share, from those of what they gave
- * O, K and widths even; K (the first), widths (the second) multiples of four.  Every element written, the same result every time. */
+ * O, K and widths even; K (the first), widths (the second) multiples of four.  Every element written, the same result every time.
+ * Precision: that of float32 products and sums; operands and results may have any value (infinities and NaN as in float32 arithmetic; a
+ * sum below 2^-89 in size of which an operand is denormal may come out as zero). */
 typedef struct dfa3d_linear_set {
   const float *weight;
   const float *rows;
