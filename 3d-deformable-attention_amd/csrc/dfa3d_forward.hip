@@ -92,7 +92,7 @@ __device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, con
 // maps), a workgroup of 16 wavefronts brings them there once and walks through a share of the queries: four of a point's eight lines
 // less.  6 x 4000 queries, one level of 23 x 40, 8 points: 53.4 -> 41.0 us (uniform), 41.0 -> 36.4 (points around the query), bfloat16
 // 56.6 -> 51.8, one distribution for all heads 49.1 -> 40.3, plain attention 36.3 -> 28.7; 64 channels, 4 x 4000, 15 x 24: 52.2 -> 32.5.
-// On larger maps the coarser levels' rows: 6 x 10000 queries, four levels from 116 x 200, 8 points (one level in LDS): 915 -> 864 us (one box; 884 on others),
+// On larger maps the coarser levels' rows: 6 x 10000 queries, four levels from 116 x 200, 8 points (one level in LDS): 915 -> 864 us (884 on another card),
 // points around the query 605 -> 571; bfloat16 (two levels) 842 -> 787, 572 -> 505; plain attention 297 -> 261.  Groups are taken, not dealt:
 // dealt, a workgroup's slowest wavefront held up the CU (883, 614).  Tried with it and not kept: two workgroups of 8, 10 or 12 wavefronts per CU
 // (908, 870, 1031; 596, 625, 706), 16 gathers in flight (880, 623), the next group's locations asked for ahead (850, 581; bfloat16 951) or
