@@ -338,18 +338,6 @@ template <typename T> struct TapsInFlight {
   }
 };
 
-// 16 bytes per lane from a buffer to consecutive LDS addresses (`lds`: the wavefront's first byte).  Written out because
-// behind the builtin the compiler waits for the data before the next LDS read of any kind; here wait_for_loads() does,
-// when the phase ends.  (The compiler does not count these loads: where it waits for an older
-// one, it waits for more than it has to, never for less.)
-__device__ __forceinline__ void load_to_lds16(rsrc_t r, const void *lds, uint32_t off) {
-#ifdef __HIP_DEVICE_COMPILE__
-  const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)lds);
-  uint32_t kept;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
-               : "=&s"(kept) : "s"(at), "v"(off), "s"(r) : "memory");
-#endif
-}
 __device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }           // vmcnt(0)
 
 // The kernel's arguments.  There are more of them, and of the numbers that follow from them, than scalar registers.

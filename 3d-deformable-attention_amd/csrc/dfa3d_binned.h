@@ -66,6 +66,19 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// 16 bytes per lane from a buffer to consecutive LDS addresses (`lds`: the wavefront's first byte).  Written out because
+// behind the builtin the compiler waits for the data before the next LDS read of any kind; here the kernel
+// waits for itself, as late as it can.  (The compiler does not count these loads: where it waits for an older one, it waits for more
+// than it has to, never for less.)
+__device__ __forceinline__ void load_to_lds16(rsrc_t r, const void *lds, uint32_t off) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)lds);
+  uint32_t kept;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
+               : "=&s"(kept) : "s"(at), "v"(off), "s"(r) : "memory");
+#endif
+}
+
 struct BinWorkspace {      // device pointers into the caller's workspace
   BinPlan *plan;
   int *queues;             // kClasses counters, kQueueStride ints apart; beside each, a part of the number of points counted

@@ -38,6 +38,30 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int kStep = 16;              // contraction steps staged at once: of one matrix instruction
 
+// x = p1 + p2 + p3, each rounded to nearest: 24 bits and more, so nothing of a float32 of 2^-108 or more is lost, and of a smaller one
+// 2^-133 at most (odd_sums).  p: two numbers to a word.  `most`: the largest size that came by.
+template <int N> __device__ __forceinline__ void split_parts(const float (&v)[N], uint32_t (&p)[3][N / 2], float &most) {
+  float rest[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) rest[j] = v[j];
+#pragma unroll
+  for (int j = 0; j < N; j += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(rest[j]), "v"(rest[j + 1]));
+#pragma unroll
+  for (int plane = 0; plane < 3; ++plane)
+#pragma unroll
+    for (int j = 0; j < N / 2; ++j) {
+      uint32_t two = pack_bf16x2(rest[2 * j], rest[2 * j + 1]);
+      asm("" : "+v"(two));                                     // (or each half is rounded once more for its difference)
+      p[plane][j] = two;
+      if (plane < 2) {
+        rest[2 * j] -= __uint_as_float(two << 16);
+        rest[2 * j + 1] -= __uint_as_float(two & 0xFFFF0000u);
+      }
+    }
+}
+// the six products of parts, smallest first: part of the one operand, part of the other
+constexpr int kProducts[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+
 // One operand of a product as its tile of R rows and kStep contraction steps comes through registers into LDS.  Element (row, k) lies at
 // row * ld + k, or (ACROSS) at k * ld + row.  In LDS: three planes of bfloat16, each in two pieces of eight contraction steps, 16 bytes per
 // row and piece; the 64 bytes between the pieces keep writes and reads off each other's banks.
@@ -67,8 +91,6 @@ template <int R, bool ACROSS> struct SplitOperand {
     }
   }
 
-  // x = p1 + p2 + p3, each rounded to nearest: 24 bits and more, so nothing of a float32 of 2^-108 or more is lost, and of a smaller one
-  // 2^-133 at most (odd_sums).  `most`: the largest size that came by.
   __device__ __forceinline__ void to_lds(unsigned char *lds, float &most) const {
     typedef unsigned int words __attribute__((ext_vector_type(kRun / 2)));
 #pragma unroll
@@ -76,24 +98,13 @@ template <int R, bool ACROSS> struct SplitOperand {
       const int idx = (int)threadIdx.x + 256 * u;
       if (2 * R % 256 != 0 && ACROSS && idx >= 2 * R) break;
       unsigned char *at = lds + (ACROSS ? idx / R * kPiece + idx % R * 16 : idx % 4 / 2 * kPiece + idx / 4 * 16 + idx % 2 * 8);
-      float rest[kRun];
-#pragma unroll
-      for (int j = 0; j < kRun; ++j) rest[j] = v[u][j];
-#pragma unroll
-      for (int j = 0; j < kRun; j += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(rest[j]), "v"(rest[j + 1]));
+      uint32_t parts[3][kRun / 2];
+      split_parts(v[u], parts, most);
 #pragma unroll
       for (int plane = 0; plane < 3; ++plane) {
         words p;
 #pragma unroll
-        for (int j = 0; j < kRun / 2; ++j) {
-          uint32_t two = pack_bf16x2(rest[2 * j], rest[2 * j + 1]);
-          asm("" : "+v"(two));                                 // (or each half is rounded once more for its difference)
-          p[j] = two;
-          if (plane < 2) {
-            rest[2 * j] -= __uint_as_float(two << 16);
-            rest[2 * j + 1] -= __uint_as_float(two & 0xFFFF0000u);
-          }
-        }
+        for (int j = 0; j < kRun / 2; ++j) p[j] = parts[plane][j];
         *reinterpret_cast<words *>(at + plane * kPlane) = p;
       }
     }
@@ -155,13 +166,12 @@ __device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, in
     seen(a);
     a.load(a_r, lda, a_row0, a_rows, k0 + 2 * kStep, depth);
     b.load(b_r, ldb, b_row0, b_rows, k0 + 2 * kStep, depth);
-    constexpr int kOf[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};          // smallest first
 #pragma unroll
     for (int t = 0; t < 6; ++t)
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[i][kOf[t][0]], pb[j][kOf[t][1]], sum[i][j], 0, 0, 0);
+        for (int j = 0; j < NT; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[i][kProducts[t][0]], pb[j][kProducts[t][1]], sum[i][j], 0, 0, 0);
     if (FLUSH && (k0 + kStep) % (FLUSH ? FLUSH : 1) == 0) {   // uniform
 #pragma unroll
       for (int i = 0; i < MT; ++i)
@@ -226,15 +236,12 @@ template <bool ACROSS> __device__ __forceinline__ void load_whole(rsrc_t r, int 
 }
 
 // acc += the wavefront's part of the tile by float32 matrix instructions, straight from memory: what split_product forms, for sums that
-// parts give no number for.  Gradients of a loss that is no number are all of that kind, and cost a few times the usual, not a walk
+// parts give no number for; row_a, row_b: this lane's first rows within the tile.  Gradients of a loss that is no number are all of that kind, and cost a few times the usual, not a walk
 // over the rows per element: weight gradient of 58000 rows of 256 x 256 56 us, all NaN 119 (by
 // one lane per element 10000); grad_x 59, 124 (3280); with one NaN row in a thousand 125 (6400) and 70 (173).
-template <int TM, int TN, bool A_ACROSS, bool B_ACROSS>
+template <int MT, int NT, bool A_ACROSS, bool B_ACROSS>
 __device__ __forceinline__ void whole_product(rsrc_t a_r, int lda, int a_row0, int a_rows, rsrc_t b_r, int ldb, int b_row0, int b_rows, int depth,
-                                              f32x16 (&acc)[TM / 64][TN / 64]) {
-  constexpr int MT = TM / 64, NT = TN / 64;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
-  const int row_a = (wave & 1) * MT * 32 + lane % 32, row_b = (wave >> 1) * NT * 32 + lane % 32;
+                                              int row_a, int row_b, f32x16 (&acc)[MT][NT]) {
   for (int k0 = 0; k0 < depth; k0 += 8) {                     // uniform
     float a[MT][4], b[NT][4];
 #pragma unroll
@@ -248,6 +255,15 @@ __device__ __forceinline__ void whole_product(rsrc_t a_r, int lda, int a_row0, i
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][k], b[j][k], acc[i][j], 0, 0, 0);
   }
+}
+
+// the same for the tiles of split_product
+template <int TM, int TN, bool A_ACROSS, bool B_ACROSS>
+__device__ __forceinline__ void whole_tile(rsrc_t a_r, int lda, int a_row0, int a_rows, rsrc_t b_r, int ldb, int b_row0, int b_rows, int depth,
+                                           f32x16 (&acc)[TM / 64][TN / 64]) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  whole_product<TM / 64, TN / 64, A_ACROSS, B_ACROSS>(a_r, lda, a_row0, a_rows, b_r, ldb, b_row0, b_rows, depth,
+                                                      (wave & 1) * (TM / 2) + lane % 32, (wave >> 1) * (TN / 2) + lane % 32, acc);
 }
 
 // c (TM x TN tile of `ms` x `ns` valid elements, row length ldc) = acc + bias.
@@ -288,7 +304,7 @@ __global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict_
   split_product<TM, TN, false, false, 0>(lds, x_r, K, 0, 0, w_r, K, 0, 0, K, acc, most, [](const auto &) {});
   if (odd_sums(acc, any_large(most, &large))) {                                        // uniform
     zero_sums(acc);
-    whole_product<TM, TN, false, false>(x_r, K, 0, 0, w_r, K, 0, 0, K, acc);
+    whole_tile<TM, TN, false, false>(x_r, K, 0, 0, w_r, K, 0, 0, K, acc);
   }
   store_product<TM, TN>(acc, y + n0 * O + o0, O, ms, ns, bias != nullptr ? bias + o0 : nullptr);
 }
@@ -316,10 +332,218 @@ __global__ __launch_bounds__(256, 3) void linear_sum_kernel(LinearSets sets, flo
     zero_sums(acc);
     for (int i = 0; i < sets.n; ++i) {
       const LinearSet &s = sets.set[i];
-      whole_product<TM, TN, false, true>(rows(s), s.width, 0, 0, weight(s), K, k0, K, s.width, acc);
+      whole_tile<TM, TN, false, true>(rows(s), s.width, 0, 0, weight(s), K, k0, K, s.width, acc);
     }
   }
   store_product<TM, TN>(acc, y + n0 * K + k0, K, ms, K - k0 < TN ? K - k0 : TN, nullptr);
+}
+
+// y (N, cols) = x (N, depth) times the weight of one layer, whose parts for 32 columns and all of the depth (up to KS * 16 steps) a wavefront keeps in
+// registers: 192 of its 256.  A workgroup (8 wavefronts, one per CU) splits its 256 columns once and walks through tiles of 32 rows; what is left of a
+// tile is its rows: straight to LDS two tiles ahead (a thread's own 16 bytes each, so no register holds them and no barrier is needed), split once,
+// read by all eight.  Power bounds it: 32x32x16 products of random numbers alone run at 1.8 of 2.4 GHz, so every split, access to LDS and load that is
+// left out counts, not only those that something waits for.  Same products and sums in the same order as by linear_kernel and linear_sum_kernel, to
+// the bit.  With those, and with this one, us, new operands each time: 184950 rows of 256 x 256 200, 151 (x W^T), 178, 130 (g W); 49536 60, 44 and 58,
+// 43; 40000 47, 33 and 45, 33; 22500 28, 22 and 27, 23; 58000 of 256 x 512 117, 92.
+constexpr int kRowTile = 32, kRowThreads = 512, kRowCols = 256;
+constexpr int kOddTiles = 256;         // a wavefront's tiles with odd sums, a bit each; of more tiles, several share one
+template <int KS> struct RowTile {
+  static constexpr int kPiece = kRowTile * 16 + 16, kPlane = 2 * KS * kPiece, kParts = 3 * kPlane;      // (pieces begin on other banks)
+  static constexpr int kQuads = 4 * KS, kUnits = kRowTile * kQuads / kRowThreads, kRaw = kRowTile * kQuads * 16;
+  static constexpr int kLds = 2 * kParts + kRaw;
+  // unit u of the rows straight to this thread's place in LDS; beyond the depth or the last row: zeros
+  static __device__ __forceinline__ void ask(int u, unsigned char *raw, rsrc_t r, int depth) {
+    int idx = (int)threadIdx.x;
+    asm volatile("" : "+v"(idx));                              // (not worth registers from tile to tile)
+    idx += kRowThreads * u;
+    const int row = idx / kQuads, k = 4 * (idx % kQuads);
+    load_to_lds16(r, raw + (kRowThreads * u + (int)threadIdx.x / kWave * kWave) * 16, k < depth ? (uint32_t)(row * depth + k) * 4 : kNoRow);
+  }
+  static __device__ __forceinline__ void split(int u, const unsigned char *raw, unsigned char *parts, float &most) {
+    const int idx = (int)threadIdx.x + kRowThreads * u, row = idx / kQuads, quad = idx % kQuads;
+    const float4 t = *reinterpret_cast<const float4 *>(raw + idx * 16);
+    const float v[4] = {t.x, t.y, t.z, t.w};
+    uint32_t p[3][2];
+    split_parts(v, p, most);
+#pragma unroll
+    for (int plane = 0; plane < 3; ++plane)
+      *reinterpret_cast<uint2 *>(parts + plane * kPlane + quad / 2 * kPiece + row * 16 + quad % 2 * 8) = make_uint2(p[plane][0], p[plane][1]);
+  }
+  static __device__ __forceinline__ bf16x8 part(const unsigned char *parts, int plane, int step, int half, int row) {
+    return *reinterpret_cast<const bf16x8 *>(parts + plane * kPlane + (2 * step + half) * kPiece + row * 16);
+  }
+};
+// waits until at most N of the wavefront's loads and stores are under way: those before them have arrived
+template <int N> __device__ __forceinline__ void wait_until_left() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+// waits for the wavefront's accesses to LDS
+__device__ __forceinline__ void wave_lds_read() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// The parts of a wavefront's 32 columns of a weight, eight contraction steps of one column to a lane and step.
+template <int KS> using ColumnParts = bf16x8[KS][3];
+__device__ __forceinline__ void column_parts(const float (&v)[8], bf16x8 (&parts)[3], float &most) {
+  uint32_t p[3][4];
+  split_parts(v, p, most);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const u32x4 words = {p[i][0], p[i][1], p[i][2], p[i][3]};
+    parts[i] = __builtin_bit_cast(bf16x8, words);
+  }
+}
+// Element (column, k) lies at k * ld + column: 32 lanes take a whole line at a time.
+template <int KS> __device__ __forceinline__ void load_columns_across(rsrc_t r, int ld, int col, int cols, ColumnParts<KS> &parts, float &most) {
+  float v[KS][8];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const uint32_t off = col < cols ? (uint32_t)((16 * s + 8 * ((int)threadIdx.x % kWave / 32)) * ld + col) * 4 : kNoRow;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[s][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off + (uint32_t)(j * ld) * 4, 0, 0));
+  }
+  __builtin_amdgcn_sched_barrier(0);                           // (all of them under way before the first is waited for)
+#pragma unroll
+  for (int s = 0; s < KS; ++s) column_parts(v[s], parts[s], most);
+}
+// Element (column, k) lies at column * depth + k: a lane per column would take 64 pieces of 16 bytes with an instruction, which cost 7 us
+// for 256 x 256.  So they come through LDS, whole lines of 32 steps of each column, three such rounds of 4 KB (`ring`: the wavefront's) under way.
+constexpr int kRing = 3, kRound = 32 * 32 * 4;
+template <int KS> __device__ __forceinline__ void load_columns(rsrc_t r, int col0, int cols, int depth, unsigned char *ring, ColumnParts<KS> &parts, float &most) {
+  const int lane = threadIdx.x % kWave;
+  constexpr int kRounds = KS / 2;
+  auto ask = [&](int round) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {                              // eight columns each; a column's pieces in an order that depends on it
+      const int c = 8 * i + lane / 8, k = 32 * round + 4 * (lane % 8 ^ c / 2 % 8);
+      load_to_lds16(r, ring + round % kRing * kRound + i * 1024, col0 + c < cols && k < depth ? (uint32_t)((col0 + c) * depth + k) * 4 : kNoRow);
+    }
+  };
+  auto wait = [&](int rounds_left) {                           // rounds asked for after the one that is waited for
+    if (rounds_left >= 2) wait_until_left<8>();
+    else if (rounds_left == 1) wait_until_left<4>();
+    else wait_until_left<0>();
+  };
+#pragma unroll
+  for (int round = 0; round < kRing; ++round) ask(round);
+#pragma unroll
+  for (int round = 0; round < kRounds; ++round) {
+    wait(kRounds - 1 - round);
+    float v[2][8];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const int c = lane % 32, piece = 4 * (h / 2) + 2 * (lane / 32) + h % 2;
+      const float4 t = *reinterpret_cast<const float4 *>(ring + round % kRing * kRound + c * 128 + 16 * (piece ^ c / 2 % 8));
+      v[h / 2][4 * (h % 2)] = t.x; v[h / 2][4 * (h % 2) + 1] = t.y; v[h / 2][4 * (h % 2) + 2] = t.z; v[h / 2][4 * (h % 2) + 3] = t.w;
+    }
+    wave_lds_read();                                           // they are read: their place is free
+    if (round + kRing < kRounds) ask(round + kRing);
+    column_parts(v[0], parts[2 * round], most);
+    column_parts(v[1], parts[2 * round + 1], most);
+  }
+}
+
+template <int KS, bool ACROSS>
+__global__ __launch_bounds__(kRowThreads, 2) void linear_rows_kernel(const float *__restrict__ x, const float *__restrict__ weight,
+                                                                     const float *__restrict__ bias, float *__restrict__ y, long long N, int cols,
+                                                                     int depth) {
+  using Tile = RowTile<KS>;
+  constexpr int kStores = 16;
+  extern __shared__ __align__(16) unsigned char lds[];
+  __shared__ int s_large[3];                                   // an operand beyond 2^32 in this tile, the next, the one before
+  __shared__ uint32_t s_odd[kRowThreads / kWave][kOddTiles / 32];
+  unsigned char *const raw = lds + 2 * Tile::kParts;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, half = lane / 32;
+  const int c0 = blockIdx.y * kRowCols, col = wave * 32 + lane % 32, ldw = ACROSS ? cols : depth;
+  const rsrc_t w_r = ACROSS ? make_rsrc(weight + c0, ((size_t)depth * cols - c0) * 4) : make_rsrc(weight + (size_t)c0 * depth, (size_t)(cols - c0) * depth * 4);
+  const int tiles = (int)((N + kRowTile - 1) / kRowTile), stride = gridDim.x;
+  auto rows_of = [&](int t) {
+    const long long n0 = (long long)t * kRowTile, left = N - n0;
+    return make_rsrc(x + (left > 0 ? n0 * depth : 0), left > 0 ? (size_t)(left < kRowTile ? left : kRowTile) * depth * 4 : 0);
+  };
+  auto result_of = [&](int t) {
+    const long long n0 = (long long)t * kRowTile, left = N - n0;
+    return make_rsrc(y + n0 * cols, (size_t)(left < kRowTile ? left : kRowTile) * cols * 4);
+  };
+  const uint32_t y_off = c0 + col < cols ? (uint32_t)(4 * half * cols + c0 + col) * 4 : kNoRow;
+  const float add = bias != nullptr && c0 + col < cols ? bias[c0 + col] : 0.f;
+  // always the same number of stores, as their number is part of what is waited for
+  auto put = [&](const f32x16 &acc, rsrc_t r, uint32_t off) {
+    asm volatile("" : "+v"(off));
+#pragma unroll
+    for (int i = 0; i < kStores; ++i) {
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i] + add), r, off, 0, 2);      // 2: non-temporal
+      off += (uint32_t)(i % 4 == 3 ? 5 : 1) * cols * 4;
+    }
+  };
+
+  int t = blockIdx.x;
+#pragma unroll
+  for (int u = 0; u < Tile::kUnits; ++u) Tile::ask(u, raw, rows_of(t), depth);
+  if (threadIdx.x < 3) s_large[threadIdx.x] = 0;
+  for (int i = lane; i < kOddTiles / 32; i += kWave) s_odd[wave][i] = 0;
+  ColumnParts<KS> w;
+  bool large_weight;
+  {
+    float most = 0;
+    if constexpr (ACROSS) load_columns_across<KS>(w_r, ldw, col, cols - c0, w, most);
+    else load_columns<KS>(w_r, wave * 32, cols - c0, depth, lds + wave * kRing * kRound, w, most);
+    large_weight = __builtin_amdgcn_ballot_w64(!(most <= 0x1p32f)) != 0;
+  }
+  static_assert(kRowThreads / kWave * kRing * kRound <= 2 * Tile::kParts, "");
+  lds_barrier();                                               // s_large is zero, and nobody uses a ring any more
+  float most = 0;
+  wait_until_left<0>();
+#pragma unroll
+  for (int u = 0; u < Tile::kUnits; ++u) Tile::split(u, raw, lds, most);
+  if (!(most <= 0x1p32f)) s_large[0] = 1;
+#pragma unroll
+  for (int u = 0; u < Tile::kUnits; ++u) Tile::ask(u, raw, rows_of(t + stride), depth);
+
+  bool any_odd = false;
+  int i = 0, at = 0, now = 0;                                  // number of the tile; its parts; i % 3
+  for (; t < tiles; t += stride, ++i, at ^= Tile::kParts) {
+    lds_barrier();                                             // this tile's parts are there, and nobody reads the last one's any more
+    const unsigned char *const mine = lds + at;
+    unsigned char *const next = lds + (at ^ Tile::kParts);
+    const int after = now == 2 ? 0 : now + 1;
+    if (threadIdx.x == 0) s_large[after == 2 ? 0 : after + 1] = 0;
+    const rsrc_t ahead = rows_of(t + 2 * stride);
+    f32x16 acc[1][1];
+    zero_sums(acc);
+    most = 0;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      bf16x8 px[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) px[p] = Tile::part(mine, p, s, half, lane % 32);
+      constexpr int kEvery = KS / Tile::kUnits;
+      if (s % kEvery == kEvery - 1) {
+        // the next tile's rows of this unit, asked for a tile ago: after them the other units' and the stores
+        if (i == 0) wait_until_left<Tile::kUnits - 1>();       // uniform
+        else wait_until_left<Tile::kUnits - 1 + kStores>();
+        Tile::split(s / kEvery, raw, next, most);
+        Tile::ask(s / kEvery, raw, ahead, depth);
+      }
+#pragma unroll
+      for (int q = 0; q < 6; ++q) acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(px[kProducts[q][0]], w[s][kProducts[q][1]], acc[0][0], 0, 0, 0);
+    }
+    if (!(most <= 0x1p32f)) s_large[after] = 1;
+    const bool odd = odd_sums(acc, large_weight || __builtin_amdgcn_readfirstlane(s_large[now]) != 0);
+    if (odd) {                                                 // uniform over the wavefront
+      any_odd = true;
+      if (lane == 0) s_odd[wave][i % kOddTiles / 32] |= 1u << (i % 32);
+    }
+    put(acc[0][0], result_of(t), odd ? kNoRow : y_off);
+    now = after;
+  }
+  wait_until_left<0>();                                        // nothing is on its way to LDS when the workgroup ends
+  if (any_odd) {                                               // uniform over the wavefront
+    wave_lds_handover();
+    for (t = blockIdx.x, i = 0; t < tiles; t += stride, ++i) {
+      if (!(__builtin_amdgcn_readfirstlane(s_odd[wave][i % kOddTiles / 32]) >> (i % 32) & 1)) continue;
+      f32x16 acc[1][1];
+      zero_sums(acc);
+      whole_product<1, 1, false, ACROSS>(rows_of(t), depth, 0, 0, w_r, ldw, 0, cols - c0, depth, lane % 32, col, acc);
+      put(acc[0][0], result_of(t), y_off);
+    }
+  }
 }
 
 struct LinearTiles { int o, k, parts, rows; };      // result tiles along O and K; parts of the rows, rows of a part
@@ -361,7 +585,7 @@ __global__ __launch_bounds__(256, 2) void linear_grad_part_kernel(
   float *mine = partial + (size_t)part * ((size_t)O * K + O);
   if (odd_sums(acc, any_large(most, &large))) {             // uniform
     zero_sums(acc);
-    whole_product<128, 128, true, true>(g_r, O, o0, O, x_r, K, k0, K, n_rows, acc);
+    whole_tile<128, 128, true, true>(g_r, O, o0, O, x_r, K, k0, K, n_rows, acc);
   }
   store_product<128, 128>(acc, mine + (size_t)o0 * K + k0, K, O - o0, K - k0, nullptr);
   if (want_bias && k0 == 0) {                               // uniform
@@ -414,7 +638,29 @@ static hipError_t launch_linear_cfg(const float *x, const float *w, const float 
   return hipGetLastError();
 }
 
+// Where linear_rows_kernel takes a product.  A wavefront multiplies by 32 columns and 256 steps whether they are there or not, and a workgroup
+// begins with 5 us of weights: so more than half of the columns, more than three quarters of the depth, and rows that give the CUs
+// about a tile each or one and a half and more.  The others and this one, us (x W^T; g W is the same or better), 256 x 256: 2048 rows 11.4, 13.1;
+// 4096 12.4, 13.5; 6000 14.6, 13.9; 8200 15.6, 18.0; 10500 17.8, 18.0; 12500 20.8, 18.4; 25000 33.2, 27.1; 16500 rows of 256 x 160 24.9, 21.5, 192 x 192
+// 21.6, 21.1, 160 x 256 20.4, 21.8; 27850 of 256 x 128 21.1, 25.1; 40000 of 128 x 256 27.3, 28.5.  (16-byte loads to LDS want their addresses whole.)
+static bool rows_kernel_applies(const float *x, const float *weight, long long N, int cols, int depth) {
+  if (cols <= 128 || depth <= 192 || depth > 256 || (depth & 3) != 0 || (((uintptr_t)x | (uintptr_t)weight) & 15) != 0) return false;
+  const long long tiles = (N + kRowTile - 1) / kRowTile, cus = cu_count();
+  return 2 * tiles >= 3 * cus || (cols <= kRowCols && tiles <= cus && 5 * tiles >= 3 * cus);
+}
+template <int KS, bool ACROSS>
+static hipError_t launch_linear_rows(const float *x, const float *w, const float *bias, float *y, long long N, int cols, int depth, hipStream_t stream) {
+  const auto kernel = linear_rows_kernel<KS, ACROSS>;
+  if (const hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), RowTile<KS>::kLds); e != hipSuccess) return e;
+  const long long tiles = (N + kRowTile - 1) / kRowTile;
+  const int cus = cu_count();
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles < cus ? tiles : cus), (cols + kRowCols - 1) / kRowCols), dim3(kRowThreads), RowTile<KS>::kLds, stream,
+                     x, w, bias, y, N, cols, depth);
+  return hipGetLastError();
+}
+
 hipError_t launch_linear(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream) {
+  if (rows_kernel_applies(x, w, N, O, K)) return launch_linear_rows<16, false>(x, w, bias, y, N, O, K, stream);
   return wide_tiles(N, O) ? launch_linear_cfg<64, 128>(x, w, bias, y, N, O, K, stream) : launch_linear_cfg<64, 64>(x, w, bias, y, N, O, K, stream);
 }
 
@@ -427,6 +673,8 @@ template <int TM, int TN, int FLUSH> static hipError_t launch_linear_sum_cfg(con
 }
 
 hipError_t launch_linear_sum(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream) {
+  const LinearSet &s = sets.set[0];
+  if (sets.n == 1 && rows_kernel_applies(s.rows, s.weight, N, K, s.width)) return launch_linear_rows<16, true>(s.rows, s.weight, nullptr, y, N, K, s.width, stream);
   const bool wide = wide_tiles(N, K);
   if (sets.n == 1) return wide ? launch_linear_sum_cfg<64, 128, 0>(sets, y, N, K, stream) : launch_linear_sum_cfg<64, 64, 0>(sets, y, N, K, stream);
   return wide ? launch_linear_sum_cfg<64, 128, 128>(sets, y, N, K, stream) : launch_linear_sum_cfg<64, 64, 128>(sets, y, N, K, stream);

@@ -70,6 +70,51 @@ def test_operands_that_are_no_ordinary_numbers():
     torch.testing.assert_close(gw, g.t().mm(x), rtol=1e-4, atol=1e-2, equal_nan=True)
 
 
+@pytest.mark.parametrize("N,K,O", [(4928, 256, 130), (8192, 256, 256), (12289, 196, 256), (12320, 252, 258), (24607, 256, 512), (50000, 256, 160)])
+@pytest.mark.parametrize("across", [False, True])
+def test_product_with_the_weight_in_registers(N, K, O, across):
+    """Row tiles that end early, one tile per workgroup and several, depths and widths that are no whole steps or columns of a wavefront; rows with
+    an infinity, a NaN, huge and tiny numbers in the first, a middle and the last tile, next to rows without."""
+    from dfa3D.modules import projection
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(N + K + O)
+    x, w, b = (torch.randn(*s, generator=g, device=dev) for s in ((N, K), (O, K), (O,)))
+    wt = w.t().contiguous()
+    product = lambda: projection._sum_of_products((x, wt)) if across else projection._product(x, w, b)
+    want = x.double() @ w.double().t() + (0 if across else b.double())
+    bound = (2.0 ** -25 + (6 * (K // 16 + 1) + 16 + 1) * 2.0 ** -23) * (x.double().abs() @ w.double().abs().t() + b.double().abs())      # as in test_product
+    got = product()
+    assert ((got.double() - want).abs() <= bound).all()
+    assert torch.equal(got, product())
+    odd = torch.tensor([3, N // 2, N // 2 + 33, N - 1], device=dev)
+    x[odd[0], 5], x[odd[1], K - 1], x[odd[2], 0] = float("inf"), float("nan"), 3e38
+    x[odd[3]] *= 1e-34
+    again = product()
+    library = x[odd] @ wt if across else torch.nn.functional.linear(x[odd], w, b)
+    torch.testing.assert_close(again[odd[:3]], library[:3], rtol=1e-5, atol=1e-4, equal_nan=True)
+    tiny = (again[odd[3]].double() - (x[odd[3]].double() @ w.double().t() + (0 if across else b.double()))).abs()
+    assert (tiny <= bound[odd[3]] * 1e-34 + (0 if across else 2.0 ** -23 * b.double().abs())).all()
+    same = torch.ones(N, dtype=torch.bool, device=dev)
+    same[odd] = False
+    assert ((again.double() - want).abs() <= bound)[same].all()
+
+
+def test_product_with_the_weight_in_registers_and_more_odd_tiles_than_bits():
+    """A workgroup remembers which of its tiles had odd sums in 256 bits; row 5 of the first tile and its namesake 256 tiles on share one."""
+    from dfa3D.modules import projection
+    dev = torch.device("cuda:0")
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    N = 32 * cus * 258 + 7
+    x, wt = torch.randn(4096, 196, device=dev).repeat(N // 4096 + 1, 1)[:N].contiguous(), torch.randn(196, 132, device=dev)
+    x[5, 7] = float("nan")
+    got = projection._sum_of_products((x, wt))
+    assert got[5].isnan().all() and got.isnan().sum() == 132
+    first = 32 * cus * 256
+    for rows in (slice(0, 5), slice(6, 64), slice(first, first + 64), slice(N - 64, N)):
+        want = x[rows].double() @ wt.double()
+        assert ((got[rows].double() - want).abs() <= 100 * 2.0 ** -23 * (x[rows].double().abs() @ wt.double().abs())).all()
+
+
 def _error(got, want):
     return ((got.double() - want).norm() / want.norm()).item()
 
