@@ -440,9 +440,12 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
   // the pairs: this kernel's flushes alone were worth 1 ms at the BEVFormer-base shape).
 
   // The depth tile of the item in slot `which` goes out and is left zeroed, by `threads` threads of which this one is
-  // number `first`, in the phase in which nobody adds to the tile.  A tile row (one pixel) takes 2^sh threads; no
-  // divisions.  Pixels 1..TY-1 x 1..7 belong to no neighbour's halo: when the item writes its tile alone they are stored,
-  // the others are added.
+  // number `first`, in the phase in which nobody adds to the tile.  A tile row (one pixel) takes 2^sh threads.  Pixels
+  // 1..TY-1 x 1..7 belong to no neighbour's halo: when the item writes its tile alone they are stored, the others are added.
+  // What bounds it are the vector instructions that find a pixel's place, so what is the same for a wavefront stays in scalars: the tile row
+  // that it takes of the inner pixels, the pixel that it takes of the rim where that is all its lanes have room for.  (With a pixel's number
+  // divided into row and column by every lane, tile kernel, one card: base shape 1210 us for 1110, bfloat16 1090 for 1025, dense 4349 for 4100, 59
+  // bins and 20 channels 124.7 for 117.5, one level of 23 x 40 113.6 for 107.  Several pixels of a lane read at once instead: registers spill, + 9 %.)
   auto flush_gd = [&](int which, int first, int threads) {
     const auto a = arg();
     const int D = a->D, S = a->S, M = a->M, Mg = a->Mg;
@@ -456,58 +459,70 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     const bool sole_d = q.sole != 0 && Mg == M;       // a gradient shared by the heads collects from all of them
     const bool d4 = (D & 3) == 0;
     auto lanes_log2 = [](int n) { return n > 32 ? 6 : n > 16 ? 5 : n > 8 ? 4 : n > 4 ? 3 : 2; };
+    const uint32_t col_step = (uint32_t)(Mg * D), row_step = (uint32_t)q.W * col_step;
+    const uint32_t e_tile = (uint32_t)(q.start + q.y0 * q.W + q.x0) * col_step + (uint32_t)(mg * D);      // of the tile's pixel (0, 0), where that exists
     if (sole_d) {
-      const int n = d4 ? D >> 2 : D, sh = lanes_log2(n), inner = (TY - 1) * (TX - 1);
-      for (int i = first >> sh; i < inner; i += threads >> sh) {
-        const int ry = i / (TX - 1) + 1, rx = i % (TX - 1) + 1, r = ry * TW + rx;
-        const int y = q.y0 + ry, x = q.x0 + rx;
-        const bool out = y < q.H && x < q.W;
-        const uint32_t e0 = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D);
-        for (int c = first & ((1 << sh) - 1); c < n; c += 1 << sh) {
-          if (d4) {
-            float4 *at = reinterpret_cast<float4 *>(gd + r * D) + c;
-            const float4 val = *at;
-            *at = make_float4(0, 0, 0, 0);
-            if (out) {
-              if (gd16) *reinterpret_cast<uint2 *>(gdist_b + (size_t)(e0 + 4 * c) * 2) = make_uint2(pack_bf16x2(val.x, val.y), pack_bf16x2(val.z, val.w));
-              else *reinterpret_cast<float4 *>(gdist_f + e0 + 4 * c) = val;
+      // a wavefront takes as many pixels of a tile row as it has lanes for; the row is a scalar
+      const int n = d4 ? D >> 2 : D, sh = lanes_log2(n), at_once = 6 - sh, parts = sh >= 3 ? sh - 3 : 0;   // pixels at once, parts of a row (log2)
+      const int lane_px = (first & (kWave - 1)) >> sh, c0 = first & ((1 << sh) - 1);
+      const int waves = threads / kWave, wave0 = __builtin_amdgcn_readfirstlane(first / kWave);
+      for (int k = wave0; k < (TY - 1) << parts; k += waves) {                // uniform
+        const int ry = 1 + (k >> parts), rx = 1 + ((k & ((1 << parts) - 1)) << at_once) + lane_px;
+        const bool in_row = rx < TX, out = q.y0 + ry < q.H && q.x0 + rx < q.W;
+        float *row = gd + (ry * TW + rx) * D;
+        const uint32_t e0 = e_tile + (uint32_t)ry * row_step + (uint32_t)rx * col_step;
+        if (in_row) {
+          for (int c = c0; c < n; c += 1 << sh) {
+            if (d4) {
+              float4 *at = reinterpret_cast<float4 *>(row) + c;
+              const float4 val = *at;
+              *at = make_float4(0, 0, 0, 0);
+              if (out) {
+                if (gd16) *reinterpret_cast<uint2 *>(gdist_b + (size_t)(e0 + 4 * c) * 2) = make_uint2(pack_bf16x2(val.x, val.y), pack_bf16x2(val.z, val.w));
+                else *reinterpret_cast<float4 *>(gdist_f + e0 + 4 * c) = val;
+              }
+            } else {                                        // float gradients only (the launcher sees to it)
+              const float val = row[c];
+              row[c] = 0;
+              if (out) gdist_f[e0 + c] = val;
             }
-          } else {                                        // float gradients only (the launcher sees to it)
-            const float val = gd[r * D + c];
-            gd[r * D + c] = 0;
-            if (out) gdist_f[e0 + c] = val;
           }
         }
       }
     }
     const int n = gd16 ? D >> 1 : D, sh = lanes_log2(n);
     const int rows = sole_d ? rim_pixels(TY, TX) : R;
-    for (int i = first >> sh; i < rows; i += threads >> sh) {
+    auto add_pixel = [&](int i) {
       int ry, rx;
       if (sole_d) {
         rim_decode(i, TY, TX, ry, rx);
       } else {
         ry = i / TW; rx = i % TW;
       }
-      const int r = ry * TW + rx, y = q.y0 + ry, x = q.x0 + rx;
-      const bool out = in_map(y, x, q.H, q.W);
-      const uint32_t e0 = (uint32_t)(((q.start + y * q.W + x) * Mg + mg) * D);
+      float *row = gd + (ry * TW + rx) * D;
+      const bool out = in_map(q.y0 + ry, q.x0 + rx, q.H, q.W);
+      const uint32_t e0 = e_tile + (uint32_t)ry * row_step + (uint32_t)rx * col_step;
       for (int c = first & ((1 << sh) - 1); c < n; c += 1 << sh) {
         if (gd16) {
-          float2 *at = reinterpret_cast<float2 *>(gd + r * D) + c;
+          float2 *at = reinterpret_cast<float2 *>(row) + c;
           const float2 val = *at;
           if (val.x != 0 || val.y != 0) {
             *at = make_float2(0, 0);
             if (out) atomic_add_bf16x2(gdist_b + (size_t)(e0 + 2 * c) * 2, val.x, val.y);
           }
         } else {
-          const float val = gd[r * D + c];
+          const float val = row[c];
           if (val != 0) {
-            gd[r * D + c] = 0;
+            row[c] = 0;
             if (out) scatter_add(gdist_r, gdist_f, (e0 + c) * 4, val);
           }
         }
       }
+    };
+    if (sh == 6) {                                          // a pixel per wavefront: its place is a scalar
+      for (int i = __builtin_amdgcn_readfirstlane(first / kWave); i < rows; i += threads / kWave) add_pixel(i);
+    } else {
+      for (int i = first >> sh; i < rows; i += threads >> sh) add_pixel(i);
     }
   };
 
