@@ -31,9 +31,10 @@ and their ``_fp32`` / ``_fp16`` twins.  Differences from the reference, all on p
 import functools
 
 import torch
-from torch.autograd.function import Function, once_differentiable
+from torch.autograd.function import once_differentiable
 
 from . import _ext, _lib
+from .recording import OperatorFunction
 
 __all__ = [
     "MultiScaleDepthScoreSampleFunction", "WeightedMultiScaleDeformableAttnFunction",
@@ -83,8 +84,10 @@ def _grad_in(g, like):
     return g if g.dtype == like else g.to(like)
 
 
-class MultiScaleDepthScoreSampleFunction(Function):
+class MultiScaleDepthScoreSampleFunction(OperatorFunction):
     """Stage 1: depth scores of the four pixels around every sampling point."""
+
+    own = True
 
     @staticmethod
     def forward(ctx, value, value_spatial_shapes, value_level_start_index, sampling_locations, im2col_step):
@@ -107,8 +110,10 @@ class MultiScaleDepthScoreSampleFunction(Function):
         return grad_value, None, None, grad_sampling_loc, None
 
 
-class WeightedMultiScaleDeformableAttnFunction(Function):
+class WeightedMultiScaleDeformableAttnFunction(OperatorFunction):
     """Stage 2: multi-scale deformable attention with every corner weighted by its depth score."""
+
+    own = True
 
     @staticmethod
     def forward(ctx, value, value_spatial_shapes, value_level_start_index, sampling_locations,
@@ -134,10 +139,12 @@ class WeightedMultiScaleDeformableAttnFunction(Function):
         return grad_value, None, None, grad_sampling_loc, grad_attn_weight, grad_depth_score, None
 
 
-class MultiScaleDeformableAttnFunction(Function):
+class MultiScaleDeformableAttnFunction(OperatorFunction):
     """Plain (2-D) multi-scale deformable attention: stage 2 with every depth score equal to 1.  Same signature
     as the Function BEVFormer's temporal self-attention and decoder cross-attention use
     (BEVFormer_DFA3D/projects/mmdet3d_plugin/bevformer/modules/multi_scale_deformable_attn_function.py:90-163)."""
+
+    own = True
 
     @staticmethod
     def forward(ctx, value, value_spatial_shapes, value_level_start_index, sampling_locations,
@@ -162,8 +169,10 @@ class MultiScaleDeformableAttnFunction(Function):
         return grad_value, None, None, grad_sampling_loc, grad_attn_weight, None
 
 
-class MultiScale3DDeformableAttnFunction(Function):
+class MultiScale3DDeformableAttnFunction(OperatorFunction):
     """One-stage DFA3D: returns ``(output, depth_score)``."""
+
+    own = True
 
     @staticmethod
     def forward(ctx, value, value_dpt_dist, value_spatial_shapes, value_level_start_index,
@@ -196,7 +205,7 @@ class MultiScale3DDeformableAttnFunction(Function):
         return grad_value, grad_value_dpt_dist, None, None, grad_sampling_loc, grad_attn_weight, None
 
 
-class MultiScale3DDeformableAttnWeightUpdateFunction(Function):
+class MultiScale3DDeformableAttnWeightUpdateFunction(OperatorFunction):
     """One-stage DFA3D that returns ``(output, weight_update)`` instead of the depth scores:
     ``weight_update`` (bs, Q, heads, 1) is the reduction the reference's caller applies to the score tensor,
     ``(depth_score.mean(-1) * attention_weights).flatten(-2).sum(-1, keepdim=True)``
@@ -207,6 +216,8 @@ class MultiScale3DDeformableAttnWeightUpdateFunction(Function):
     ``dfa3D._ext.pack_shared_dist`` lays it out for the forward's depth taps: a caller that runs several layers on
     one distribution (DFA3D-BEVFormer's six encoder layers) packs once and passes it to each; without it the
     forward packs for itself when that pays."""
+
+    own = True
 
     @staticmethod
     def forward(ctx, value, value_dpt_dist, value_spatial_shapes, value_level_start_index,
@@ -259,7 +270,7 @@ def _autocast_twin(base, name, doc):
             return base.backward(ctx, *grads)
 
     return type(name, (base,), {"forward": staticmethod(forward), "backward": staticmethod(backward),
-                                "__doc__": doc, "__module__": __name__})
+                                "own": True, "__doc__": doc, "__module__": __name__})
 
 
 _FP32_DOC = "Autocast-safe twin: inputs are cast to float32 when autocast is on."

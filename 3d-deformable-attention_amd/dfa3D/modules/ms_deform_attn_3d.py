@@ -15,19 +15,21 @@ import warnings
 
 import torch
 from torch import nn
-from torch.autograd import Function
 
 from ..functional import (MultiScale3DDeformableAttnFunction_fp32,
                           MultiScale3DDeformableAttnWeightUpdateFunction_fp32)
 from .. import _lib
+from ..recording import OperatorFunction
 from .projection import Projection, ordinary, plain_gradient, projections
 
 __all__ = ["MSDeformableAttention3D_DFA3D"]
 
 
-class _LocationsFunction(Function):
+class _LocationsFunction(OperatorFunction):
     """uv (bs, Q, M, L, P, 2), dz (bs, Q, M, L, P, 1), reference points (bs, Q, Z, 3) and shapes (L, 3) to sampling locations
     in one kernel; differentiable in uv and dz, any number of times."""
+
+    own = True
 
     @staticmethod
     def forward(ctx, uv, dz, reference_points, shapes3):

@@ -4,10 +4,10 @@ afterwards.  The reference does both in python loops over batch x cameras
 (BEVFormer_DFA3D/projects/mmdet3d_plugin/bevformer/modules/spatial_cross_attention.py:716-722, 741-748);
 here each direction is one HIP kernel (csrc/dfa3d_rebatch.hip), and each kernel is the other's backward."""
 import torch
-from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 
 from . import _lib
+from .recording import OperatorFunction
 
 __all__ = ["camera_hits", "camera_count", "camera_index", "rebatch_gather", "rebatch_combine", "RebatchGatherFunction", "RebatchCombineFunction"]
 
@@ -147,8 +147,10 @@ def rebatch_combine(src, pos, scale=None):
     return dst
 
 
-class RebatchGatherFunction(Function):
+class RebatchGatherFunction(OperatorFunction):
     """``apply(src (bs, Nq, E), index, pos) -> (bs, cams, max_len, E)``; differentiable in ``src``."""
+
+    own = True
 
     @staticmethod
     def forward(ctx, src, index, pos):
@@ -162,9 +164,11 @@ class RebatchGatherFunction(Function):
         return rebatch_combine(grad.contiguous(), pos), None, None
 
 
-class RebatchCombineFunction(Function):
+class RebatchCombineFunction(OperatorFunction):
     """``apply(src (bs, cams, max_len, E), index, pos, scale (bs, Nq) or None) -> (bs, Nq, E)``; differentiable in
     ``src`` (``scale`` is a constant: the reciprocal camera count)."""
+
+    own = True
 
     @staticmethod
     def forward(ctx, src, index, pos, scale):

@@ -1,0 +1,106 @@
+"""Functions whose ``apply`` is their ``forward`` where nothing records: the same results, and a node all the same where somebody looks."""
+import threading
+
+import pytest
+import torch
+from torch.autograd import Function
+from torch.autograd.function import once_differentiable
+
+from dfa3D.recording import OperatorFunction
+
+
+def _body():
+    def forward(ctx, x, s):
+        ctx.s = s
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(x)
+        _body.seen.append(type(ctx).__name__)
+        return x * ctx.s, x + 1
+
+    def backward(ctx, g, h):
+        return g * ctx.s, None
+    return {"forward": staticmethod(forward), "backward": staticmethod(once_differentiable(backward))}
+
+
+_body.seen = []
+Plain = type("Plain", (Function,), _body())
+Own = type("Own", (OperatorFunction,), dict(_body(), own=True))
+Theirs = type("Theirs", (Own,), {})
+
+
+def _took_the_short_way(call):
+    _body.seen.clear()
+    out = call()
+    return out, _body.seen[-1] == "_Notes"
+
+
+def test_without_gradients_the_forward_alone_runs():
+    x = torch.randn(5, requires_grad=True)
+    for mode in (torch.no_grad, torch.inference_mode):
+        with mode():
+            out, short = _took_the_short_way(lambda: Own.apply(x, 3))
+            want = Plain.apply(x, 3)
+        assert short
+        for a, b in zip(out, want):
+            assert torch.equal(a, b) and not a.requires_grad and a.grad_fn is None and a.is_inference() == b.is_inference()
+
+
+def test_with_gradients_a_node_is_made():
+    x = torch.randn(5, requires_grad=True)
+    out, short = _took_the_short_way(lambda: Own.apply(x, 3))
+    assert not short and torch.equal(torch.autograd.grad(out[0].sum(), x)[0], torch.full((5,), 3.0))
+    out, short = _took_the_short_way(lambda: Own.apply(x.detach(), 3))
+    assert not short and not out[0].requires_grad
+
+
+def test_a_subclass_from_elsewhere_gets_a_context_of_torchs():
+    with torch.no_grad():
+        assert not _took_the_short_way(lambda: Theirs.apply(torch.ones(2), 3))[1]
+
+
+def test_tracing_forward_mode_and_transforms_see_the_call():
+    x = torch.randn(4)
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda t: Own.apply(t, 3)[0], x, check_trace=False)
+        assert any(n.kind() == "prim::PythonOp" for n in traced.graph.nodes())
+        assert torch.equal(torch.compile(lambda t: Own.apply(t.sin(), 3)[0], backend="eager", fullgraph=True)(x), x.sin() * 3)
+        for F in (Plain, Own):
+            with pytest.raises(RuntimeError):
+                torch.func.vmap(lambda t: F.apply(t, 3)[0])(x)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones(4))
+        answers = []
+        for F in (Plain, Own):
+            with torch.no_grad():
+                try:
+                    answers.append(torch.autograd.forward_ad.unpack_dual(F.apply(dual, 3)[0]).tangent)
+                except (RuntimeError, NotImplementedError) as e:
+                    answers.append(type(e))
+        assert answers[0] == answers[1]
+
+
+def test_a_wrapper_left_over_from_a_transform_is_unwrapped():
+    left = []
+    torch.func.vmap(lambda t: (left.append(t), t)[1])(torch.ones(3, 2))
+    outs = []
+    for F in (Plain, Own):
+        with torch.no_grad():
+            try:
+                outs.append(torch.equal(F.apply(left[0], 3)[0], F.apply(left[0], 3)[0]))
+            except RuntimeError as e:
+                outs.append(type(e))
+    assert outs[0] == outs[1]
+
+
+def test_threads_do_not_share_a_context():
+    results = [None] * 8
+
+    def work(i):
+        with torch.no_grad():
+            results[i] = all(torch.equal(Own.apply(torch.full((3,), float(i)), i)[0], torch.full((3,), float(i * i))) for _ in range(200))
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(results)
