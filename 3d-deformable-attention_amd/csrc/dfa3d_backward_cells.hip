@@ -605,24 +605,27 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
         }
       }
     };
-    // Rim pixels [first, first + n) of item q, whose sums this wavefront left in LDS.
-    auto put_rim = [&](auto a, const ItemGeom &q, int first, int n) {
+    // Rim pixels of tile row `ry` of item q, whose sums this wavefront left in LDS: the whole row where it is the tile's first or last, else its
+    // first and last pixel.  What is the same for the row is in scalars.
+    auto put_rim = [&](auto a, const ItemGeom &q, int ry) {
+      if ((unsigned)(q.y0 + ry) >= (unsigned)q.H) return;   // uniform
       const int S = a->S, M = a->M, C = a->C;
-      const bool gv16 = (a->grad16 & 1) != 0;               // uniform
+      const bool gv16 = (a->grad16 & 1) != 0, whole = ry == 0 || ry == TY;      // uniform
       void *grad_value = a->grad_value;
       char *gvalue_b = static_cast<char *>(grad_value) + (size_t)q.b * S * M * C * (gv16 ? 2 : 4);
       float *gvalue_f = reinterpret_cast<float *>(gvalue_b);
       const rsrc_t gvalue_r = make_rsrc(gvalue_b, (size_t)S * M * C * sizeof(float));
-      const int per = gv16 ? ROW / 2 : ROW;                 // lanes per pixel: a float, or a pair of bfloat16
-      for (int i = lane; i < n * per; i += kWave) {
-        const int k = first + i / per, c = (i % per) * (gv16 ? 2 : 1);
-        int ry, rx;
-        rim_decode(k, TY, TX, ry, rx);
-        const int y = q.y0 + ry, x = q.x0 + rx;
-        const float *from = rim + k * ROW + c;
-        const float f0 = from[0], f1 = gv16 ? from[1] : 0.f;
-        if (c < C && in_map(y, x, q.H, q.W) && (f0 != 0 || f1 != 0)) {
-          const uint32_t e = (uint32_t)(((q.start + y * q.W + x) * M + q.m) * C + c);
+      constexpr int kRowLog2 = ROW == 64 ? 6 : ROW == 32 ? 5 : 4;
+      const int sh = gv16 ? kRowLog2 - 1 : kRowLog2;        // lanes per pixel: a float, or a pair of bfloat16 (log2)
+      const int c = (lane & ((1 << sh) - 1)) * (gv16 ? 2 : 1), pixels = whole ? TW : 2, apart = whole ? 1 : TX;
+      const uint32_t col_step = (uint32_t)(M * C), e_row = (uint32_t)(q.start + (q.y0 + ry) * q.W + q.x0) * col_step + (uint32_t)(q.m * C);
+      const float *row = rim + rim_index(ry, 0, TY, TX) * ROW + c;
+#pragma unroll 1
+      for (int i = lane >> sh; i < pixels; i += kWave >> sh) {
+        const int rx = i * apart;
+        const float f0 = row[i * ROW], f1 = gv16 ? row[i * ROW + 1] : 0.f;
+        if (c < C && (unsigned)(q.x0 + rx) < (unsigned)q.W && (f0 != 0 || f1 != 0)) {
+          const uint32_t e = e_row + (uint32_t)rx * col_step + (uint32_t)c;
           if (gv16) atomic_add_bf16x2(gvalue_b + (size_t)e * 2, f0, f1);
           else scatter_add(gvalue_r, gvalue_f, e * 4, f0);
         }
@@ -903,10 +906,9 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
           }
           put_pixel(now, o, q, u, mine);
           wave_lds_handover();
-          const int ra = max(r0, 1), n_side = min(r0 + ROWS, TY) - ra;
-          if (wave == 0) put_rim(now, q, 0, TW);
-          if (n_side > 0) put_rim(now, q, rim_index(ra, 0, TY, TX), 2 * n_side);
-          if (r0 + ROWS >= TY) put_rim(now, q, TW, TW);
+#pragma unroll 1
+          for (int ry = r0; ry < min(r0 + ROWS, TY); ++ry) put_rim(now, q, ry);      // uniform
+          if (r0 + ROWS >= TY) put_rim(now, q, TY);
         }
         if (done) break;
         typename std::conditional<FOURS, WholeRow<T, VEC, LPR>, float[4][VEC]>::type v;      // the four value rows
