@@ -334,6 +334,34 @@ template <typename A> struct Point2D {
   }
 };
 
+// The same without keys: which of the four pixels exist, for callers that count in bytes.
+template <typename A> struct Grid2D {
+  A lh, lw, hh, hw;
+  int h0, w0;
+  bool inside, h_lo, h_hi, w_lo, w_hi;      // h_lo ...: rows h0, h0 + 1, columns w0, w0 + 1 are in the map
+  __device__ __forceinline__ A bil(int k) const {
+    return k == 0 ? hh * hw : k == 1 ? hh * lw : k == 2 ? lh * lw : lh * hw;
+  }
+  __device__ __forceinline__ bool on(int k) const { return inside && (k >= 2 ? h_hi : h_lo) && (k == 1 || k == 2 ? w_hi : w_lo); }
+};
+
+template <typename A>
+__device__ __forceinline__ Grid2D<A> locate_grid(A x, A y, int H, int W) {
+  Grid2D<A> g;
+  const A h_im = to_pixel(y, H), w_im = to_pixel(x, W);
+  g.inside = h_im > -1 && w_im > -1 && h_im < H && w_im < W;
+  // as in locate_2d: harmless geometry for a point that fails the test
+  g.h0 = g.inside ? floor_index(h_im) : 0;
+  g.w0 = g.inside ? floor_index(w_im) : 0;
+  g.lh = g.inside ? h_im - g.h0 : (A)0;
+  g.lw = g.inside ? w_im - g.w0 : (A)0;
+  g.hh = 1 - g.lh;
+  g.hw = 1 - g.lw;
+  g.h_lo = (unsigned)g.h0 < (unsigned)H; g.h_hi = (unsigned)(g.h0 + 1) < (unsigned)H;
+  g.w_lo = (unsigned)g.w0 < (unsigned)W; g.w_hi = (unsigned)(g.w0 + 1) < (unsigned)W;
+  return g;
+}
+
 template <typename A>
 __device__ __forceinline__ Point2D<A> locate_2d(A x, A y, int H, int W, int start) {
   Point2D<A> g;
@@ -489,6 +517,50 @@ __device__ __forceinline__ void corner_scores(rsrc_t dist_r, const int (&key)[4]
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) score[k] = depth_lerp(lo[k], hi[k], tap.hd, tap.ld);
+}
+
+// A point's taps as weights of the pair of bins (db, db + 1), D >= 2: the lower tap is the pair's first bin, or its second where it is
+// the row's last; the upper one the second, or the first where it is bin 0.  A bin that is no tap counts as zero, whatever it holds.
+// Rounds like depth_lerp.
+template <typename A> struct DepthPair {
+  int db;
+  A wx, wy;
+  bool use_x, use_y;
+  __device__ __forceinline__ DepthPair(const DepthTap<A> &tap, int D) : db(min(max(tap.d0, 0), D - 2)) {
+    const bool first = tap.d0 == db;                         // else d0 = db - 1 (the upper tap is bin 0) or db + 1 (the lower one is the last)
+    use_x = (first & tap.lo_ok) | ((tap.d0 < db) & tap.hi_ok);
+    use_y = (first & tap.hi_ok) | ((tap.d0 > db) & tap.lo_ok);
+    wx = first ? tap.hd : tap.ld;
+    wy = first ? tap.ld : tap.hd;
+  }
+  __device__ __forceinline__ A score(A x, A y) const { return depth_lerp(use_x ? x : (A)0, use_y ? y : (A)0, wx, wy); }
+};
+// corner_scores() for callers that count in bytes: the distribution of pixel (y, x) lies at base + y * row + x * col
+template <typename T, typename A>
+__device__ __forceinline__ void grid_scores(rsrc_t dist_r, const Grid2D<A> &g, const DepthTap<A> &tap, uint32_t base, uint32_t row, uint32_t col,
+                                            int D, A (&score)[4]) {
+  const uint32_t at = (uint32_t)g.h0 * row + (uint32_t)g.w0 * col + base;
+  if (D >= 2) {
+    const DepthPair<A> pair(tap, D);
+    const uint32_t at_pair = at + (uint32_t)(pair.db * (int)sizeof(T));
+    uint32_t off[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      off[k] = g.on(k) && tap.inside ? at_pair + (k >= 2 ? row : 0) + (k == 1 || k == 2 ? col : 0) : kNoRow;
+    A x[4], y[4];
+    __builtin_amdgcn_sched_barrier(0);                       // the loads one behind the other: corner_scores()
+    PairLoader<T, false>::ld(dist_r, off, D, x, y);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) score[k] = pair.score(x[k], y[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t bin = at + (k >= 2 ? row : 0) + (k == 1 || k == 2 ? col : 0) + (uint32_t)(tap.d0 * (int)sizeof(T));
+      const A lo = BufElem<T>::ld(dist_r, (g.on(k) && tap.lo_ok) ? bin : kNoRow);
+      const A hi = BufElem<T>::ld(dist_r, (g.on(k) && tap.hi_ok) ? bin + (uint32_t)sizeof(T) : kNoRow);
+      score[k] = depth_lerp(lo, hi, tap.hd, tap.ld);
+    }
+  }
 }
 
 // one task of phase B: byte offset of a value row inside the batch element (kNoRow = nothing

@@ -7,6 +7,7 @@
 //                                           (wms_deform_attn_cuda_kernel.cuh:240-303)
 //   depth_score_kernel                      stage 1 alone
 //                                           (ms_depth_score_sample_cuda_kernel.cuh:94-148)
+#include <algorithm>
 #include <type_traits>
 
 #include "dfa3d_device.h"
@@ -22,24 +23,29 @@ __host__ __device__ inline FwdShape fwd_shape(int L, int P, int upw) {
 }
 constexpr int kMaxUnitsPerWave = 16;
 constexpr int kLdsRowsBlock = 1024;    // threads of a workgroup that holds its (batch, head)'s value rows in LDS
-constexpr int kTaskPad = 2;            // tasks left free after each unit's, so that the units start on different LDS banks
-constexpr int kTasksPerWave = kWave * 4 + kMaxUnitsPerWave * kTaskPad;
+constexpr int kTasksPerWave = kWave * 4 + 32;      // room for its tasks, padding included (task_run)
+// Places that a row slot's run of a unit's tasks takes.  Two runs are read at 16 bytes each at a time, so they start 16 bytes apart on the LDS banks
+// (two places more than a multiple of four), but for 21 points a unit on eight slots, for which there is no room.
+__device__ __forceinline__ int task_run(int longest, int runs) {
+  const int padded = ((longest + 1) & ~3) + 2;
+  return runs * padded <= kTasksPerWave ? padded : longest;
+}
 
-// Phase B of the forward pass: acc += sum of w * row over the tasks first, first + step, ... below n of one unit.  LPR lanes
-// of VEC channels take a row; the wavefront's 64/LPR row slots may work on the same unit (step > 1) or on units of
-// their own.  Eight rows per lane are in flight, whatever the length of the list: a unit of 8 points has 32 tasks, and
-// walking it one row at a time waited for memory once per row.  A batch is summed in two chains and added to acc as a
-// whole, which keeps the longest chain of additions of a unit at about what a tree over the row slots has.
-// `rows` reads this lane's channels of the row at a byte offset; `none` is the offset of a row of zeros.
+// Phase B of the forward pass: acc += sum of w * row over a row slot's tasks.  LPR lanes of VEC channels take a row; the
+// wavefront's 64/LPR row slots may share a unit, each with a run of its tasks, or work on units of their own.  `all` tasks every slot
+// of the unit has, `most` the longest run (both uniform), `mine` this slot's.  Eight rows per lane are in flight, whatever the length
+// of the list: a unit of 8 points has 32 tasks, and walking it one row at a time waited for memory once per row.  A batch is summed in
+// two chains and added to acc as a whole, which keeps the longest chain of additions of a unit at about what a tree over the
+// row slots has.  `rows` reads this lane's channels of the row at a byte offset; `none` is the offset of a row of zeros.
 template <typename A, int VEC, typename Rows>
-__device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, const Task<A> *tasks, int first, int step, int n,
+__device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, const Task<A> *tasks, int all, int most, int mine,
                                             A (&acc)[VEC]) {
   constexpr int U = 8, UT = 4;
   int t = 0;                                             // uniform
-  for (; t + step * U <= n; t += step * U) {
+  for (; t + U <= all; t += U) {
     Task<A> e[U];
 #pragma unroll
-    for (int j = 0; j < U; ++j) e[j] = tasks[t + j * step + first];
+    for (int j = 0; j < U; ++j) e[j] = tasks[t + j];
     A v[U][VEC];
 #pragma unroll
     for (int j = 0; j < U; ++j) rows(e[j].off, v[j]);
@@ -51,7 +57,7 @@ __device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, con
       acc[i] += s0 + s1;
     }
   }
-  for (; t < n; t += step * UT) {                       // the rest: no load is issued that no slot has a row for
+  for (; t < most; t += UT) {                            // the rest: no load is issued that no slot has a row for
     Task<A> e[UT];
     A v[UT][VEC];
 #pragma unroll
@@ -59,10 +65,10 @@ __device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, con
       e[j].off = none; e[j].w = 0;
 #pragma unroll
       for (int i = 0; i < VEC; ++i) v[j][i] = 0;
-      if (t + j * step < n) {                            // uniform
-        const int at = t + j * step + first;
-        e[j] = tasks[min(at, n - 1)];
-        if (at >= n) { e[j].off = none; e[j].w = 0; }
+      if (t + j < most) {                                // uniform
+        const bool has = t + j < mine;
+        e[j] = tasks[has ? t + j : 0];
+        if (!has) { e[j].off = none; e[j].w = 0; }
         rows(e[j].off, v[j]);
       }
     }
@@ -71,6 +77,35 @@ __device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, con
 #pragma unroll
       for (int i = 0; i < VEC; ++i) acc[i] += e[j].w * v[j][i];
     }
+  }
+}
+// x summed over the lanes that differ in the bits FROM, 2 FROM, ... below `to` (uniform) of their number
+template <int FROM, int VEC> __device__ __forceinline__ void sum_over_slots(int to, float (&x)[VEC]) {
+  if constexpr (FROM < kWave) {
+    if (FROM < to) {
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        const int v = __float_as_int(x[i]);
+        if constexpr (FROM == 8) {
+          x[i] += __int_as_float(__builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true));              // row_ror:8
+        } else if constexpr (FROM == 16) {
+          const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+          x[i] = __int_as_float(r[0]) + __int_as_float(r[1]);
+        } else if constexpr (FROM == 32) {
+          const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+          x[i] = __int_as_float(r[0]) + __int_as_float(r[1]);
+        } else {
+          x[i] += __shfl_xor(x[i], FROM, kWave);
+        }
+      }
+      sum_over_slots<2 * FROM, VEC>(to, x);
+    }
+  }
+}
+template <int FROM, int VEC> __device__ __forceinline__ void sum_over_slots(int to, double (&x)[VEC]) {
+  for (int off = FROM; off < to; off <<= 1) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) x[i] += __shfl_xor(x[i], off, kWave);
   }
 }
 
@@ -97,6 +132,15 @@ __device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, con
 // dealt, a workgroup's slowest wavefront held up the CU (883, 614).  Tried with it and not kept: two workgroups of 8, 10 or 12 wavefronts per CU
 // (908, 870, 1031; 596, 625, 706), 16 gathers in flight (880, 623), the next group's locations asked for ahead (850, 581; bfloat16 951) or
 // brought to the L2 by scalar loads (874, 587); the same workgroups without rows in LDS: 942, 603.
+//
+// A quarter of the instructions found places: divisions by the points of a unit and of a level, 64-bit indexes, a product per corner.  What a
+// lane's point has from its place in the group and its level is kept from group to group (IN_LDS), the group's part is in scalars, corners
+// are a row and a column apart, and a slot's tasks lie side by side (656 -> 498 vector instructions per 64 points).  And the wavefronts of a SIMD,
+// which meet at the L1, go by what they hold: one that gathers value rows comes before one that looks for its points' corners, and that before one
+// that begins a group (s_setprio 2, 1, 0; the other way round 3120 us for the 3047 of two steps and 3000 of three, 24 planes and 128 bins).  Together, one card, us:
+//   6 x 10000 queries, 4 levels from 116 x 200, 8 points: 885 -> 872, around the query 574 -> 571 (bfloat16 483 -> 476), plain attention 436 -> 389;
+//   6 x 40000 clustered, 128 bins: 3067 -> 3000; the two separate stages without gradients, 112 bins: 1013 -> 936; one level of 23 x 40: 39.7 -> 38.0;
+//   plain attention, 2 x 40000 queries of 4 points: 109 -> 99.  (6 heads of 20 channels, three levels of 5 points: 44.1 -> 45.0.)
 // ---------------------------------------------------------------------------------------
 template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS>
 __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention_kernel(
@@ -113,7 +157,7 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
   extern __shared__ __align__(16) unsigned char s_rows[];    // IN_LDS: value rows [key0, S) of (b, m), then a row of zeros
 
   const FwdShape ws = fwd_shape(L, P, upw);
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int m = blockIdx.x % M;
   const int rest = blockIdx.x / M;
   const int qb = rest % q_blocks, b = rest / q_blocks;
@@ -121,40 +165,55 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
   const int passes = (C + VEC * LPR - 1) / (VEC * LPR);
   Task<A> *tasks = s_tasks[wave];
   const int q_per_iter = WAVES * ws.upw;
-  // what this lane's point of a chunk of the group that begins with query q0 has
+  // This lane's point of chunk `chunk` of a group: unit and point within the unit, and the point's number counted from the group's
+  // first unit's first point.  The same for all groups (of one chunk): what a group adds is in scalars.
+  struct Place { int ul, lp; uint32_t idx; };
+  auto place = [&](int chunk) {
+    const int pt = chunk * kWave + lane, ul = pt / ws.LP, lp = pt - ul * ws.LP;
+    return Place{ul, lp, (uint32_t)ul * (uint32_t)(M * ws.LP) + (uint32_t)lp};
+  };
+  auto first_point = [&](int q0) { return ((size_t)(b * (size_t)Q + q0) * M + m) * ws.LP; };      // of the group that begins with query q0
   struct Operands { A x, y, z, a; };
-  auto fetch = [&](int q0, int chunk) {
-    const int pt = chunk * kWave + lane, ul = pt / ws.LP, lp = pt - ul * ws.LP, q = q0 + ul;
+  auto fetch = [&](int q0, const Place &pl) {
     Operands o{0, 0, 0, 0};
-    if (ul < ws.upw && q < Q) {
-      const size_t gp = ((size_t)(b * (size_t)Q + q) * M + m) * ws.LP + lp;   // global point index
-      const A *pl = loc + gp * loc_stride;
+    if (pl.ul < min(ws.upw, Q - q0)) {
+      const size_t first = first_point(q0);
+      const A *pt = reinterpret_cast<const A *>(reinterpret_cast<const char *>(loc + first * loc_stride) + pl.idx * (uint32_t)(loc_stride * (int)sizeof(A)));
+      const A *pa = reinterpret_cast<const A *>(reinterpret_cast<const char *>(attn + first) + pl.idx * (uint32_t)sizeof(A));
       if (!IN_LDS && (once & 1) != 0) {                         // uniform
         asm volatile("");                                       // (or the compiler merges the branches into plain loads)
-        o.x = __builtin_nontemporal_load(pl); o.y = __builtin_nontemporal_load(pl + 1);
-        if (FUSED) o.z = __builtin_nontemporal_load(pl + 2);
+        o.x = __builtin_nontemporal_load(pt); o.y = __builtin_nontemporal_load(pt + 1);
+        if (FUSED) o.z = __builtin_nontemporal_load(pt + 2);
         asm volatile("");
       } else {
-        o.x = pl[0]; o.y = pl[1];
-        if (FUSED) o.z = pl[2];
+        o.x = pt[0]; o.y = pt[1];
+        if (FUSED) o.z = pt[2];
       }
       if (!IN_LDS && (once & 2) != 0) {
         asm volatile("");
-        o.a = __builtin_nontemporal_load(attn + gp);
+        o.a = __builtin_nontemporal_load(pa);
         asm volatile("");
       } else {
-        o.a = attn[gp];
+        o.a = *pa;
       }
     }
     return o;
   };
   // The first group's are on their way while the level table is: a workgroup of one group otherwise waits for one after the other (2 x 40000
   // queries of plain attention, 4 points: 98.7 -> 94 us; 2 x 100 queries 6.24 -> 6.04; larger calls +- 0.5 %).
-  const Operands first = IN_LDS ? Operands{0, 0, 0, 0} : fetch((qb * iters * WAVES + wave) * ws.upw, 0);
+  Place pl = place(0);
+  const Operands first = IN_LDS ? Operands{0, 0, 0, 0} : fetch((qb * iters * WAVES + wave) * ws.upw, pl);
   // phase B: `par` units at a time, `spu` row slots each
   constexpr int RPI = kWave / LPR;
-  const int par = min(ws.upw & -ws.upw, RPI), spu = RPI / par;
-  const int unit_tasks = ws.LP * 4 + kTaskPad;              // where the next unit's tasks start (upw > 1)
+  const int par = min(ws.upw & -ws.upw, RPI), spu = RPI / par, spu_log2 = 31 - __builtin_clz(spu);
+  // Task i of a unit belongs to its slot i % spu.  A slot's tasks lie side by side, so that a batch of them is read from one address.
+  const int unit_points = ws.upw == 1 ? min(kWave, ws.LP) : ws.LP;                 // of a chunk
+  const int run = task_run((unit_points * 4 + spu - 1) >> spu_log2, ws.upw * spu);
+  const int my_point = ws.upw == 1 ? lane : pl.lp, my_unit = ws.upw == 1 ? 0 : pl.ul;
+  const bool my_tasks = my_point < unit_points && my_unit < ws.upw;
+  Task<A> *const to = tasks + (my_unit * spu + ((my_point * 4) & (spu - 1))) * run + ((my_point * 4) >> spu_log2);
+  const int to1 = spu > 1 ? run : 1, to2 = spu > 2 ? 2 * run : spu == 2 ? 1 : 2, to3 = spu == 2 ? run + 1 : to1 + to2;
+  const int part = row_slot % spu;
 
   load_level_table(tab, shapes, shape_stride, level_start, L, S, FUSED ? D : 0);
   if (FUSED && packed_arg != nullptr) load_cell_starts(tab, L);      // uniform
@@ -196,6 +255,25 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
     __syncthreads();
   }
   const uint32_t zero_row = (uint32_t)((S - key0) * C * (int)sizeof(T));
+  // What the geometry of a lane's point takes from its level: sizes, and byte offsets (modulo 2^32) of value rows and distributions, those of
+  // a map's pixel (y, x) being base + y * row + x * col.  Kept from group to group, like the lane's place.
+  struct Level { int H, W, Dd, cell; uint32_t v_col, v_row, v_base, d_row, d_base; bool in_lds; };
+  const uint32_t d_col = (uint32_t)(Md * D * (int)sizeof(T));
+  auto level = [&](const Place &at) {
+    const int l = min(at.lp / P, L - 1), start = tab.start[l];
+    Level v;
+    v.H = tab.H[l]; v.W = tab.W[l]; v.Dd = tab.Dd[l];
+    v.cell = FUSED && packed != nullptr ? tab.cell[l] : 0;
+    v.in_lds = IN_LDS && l >= l0;
+    v.v_col = (uint32_t)((v.in_lds ? C : M * C) * (int)sizeof(T));
+    v.v_row = (uint32_t)v.W * v.v_col;
+    v.v_base = v.in_lds ? (uint32_t)((start - key0) * C * (int)sizeof(T)) : (uint32_t)((start * M + m) * C * (int)sizeof(T));
+    v.d_row = (uint32_t)v.W * d_col;
+    v.d_base = (uint32_t)((start * Md + md) * D * (int)sizeof(T));
+    return v;
+  };
+  Level lv{};
+  if (IN_LDS) lv = level(pl);                                // (else worked out where it is needed: most workgroups have one group, and registers are wavefronts)
 
   // Groups of units, WAVES to a round; rounds are dealt to the workgroups of a (batch, head) in turn, so that what they gather at a
   // time lies together.  IN_LDS: a workgroup's wavefronts take its next group each.
@@ -226,47 +304,39 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
       for (int v = 0; v < VEC; ++v) acc[v] = 0;
 
       for (int chunk = 0; chunk < ws.chunks; ++chunk) {
+        __builtin_amdgcn_s_setprio(0);                       // a group begins
         // ---------------- phase A: one lane per sampling point ----------------
-        const int pt = chunk * kWave + lane;                 // point within the group of units
-        const int ul = pt / ws.LP, lp = pt - ul * ws.LP;     // unit within group, point within unit
-        const int q = q0 + ul;
-        const bool live = ul < ws.upw && q < Q;
+        if (ws.chunks > 1) pl = place(chunk);                // uniform
+        if (!IN_LDS || ws.chunks > 1) lv = level(pl);
+        const int ul = pl.ul, lp = pl.lp, q = q0 + ul;       // unit within group, point within unit
+        const bool live = ul < min(ws.upw, Q - q0);
         Operands in = first;
-        if (IN_LDS || it > 0 || pass > 0 || chunk > 0) in = fetch(q0, chunk);      // uniform
+        if (IN_LDS || it > 0 || pass > 0 || chunk > 0) in = fetch(q0, pl);      // uniform
         Task<A> t4[4];
         A wu = 0;
-        const bool from_lds = IN_LDS && lp >= l0 * P;
-        const uint32_t none = from_lds ? zero_row : kNoRow;
+        const uint32_t none = lv.in_lds ? zero_row : kNoRow;
 #pragma unroll
         for (int k = 0; k < 4; ++k) { t4[k].off = none; t4[k].w = 0; }
         if (live) {
-          const int l = lp / P;
-          const size_t gp = ((size_t)(b * (size_t)Q + q) * M + m) * ws.LP + lp;   // global point index
           const A a = in.a;
-          const Point2D<A> g = locate_2d<A>(in.x, in.y, tab.H[l], tab.W[l], tab.start[l]);
+        __builtin_amdgcn_s_setprio(1);
+          const Grid2D<A> g = locate_grid<A>(in.x, in.y, lv.H, lv.W);
           A sc[4];
           if (FUSED) {
-            A lo[4], hi[4];
-            const DepthTap<A> tap = locate_depth<A>(in.z, tab.Dd[l]);
+            const DepthTap<A> tap = locate_depth<A>(in.z, lv.Dd);
             if (packed != nullptr) {                                // uniform: all eight taps from one line
-              const int db = min(max(tap.d0, 0), D - 2);
-              const bool lo_x = tap.lo_ok && tap.d0 == db, lo_y = tap.lo_ok && tap.d0 == db + 1;
-              const bool hi_x = tap.hi_ok && tap.d0 + 1 == db, hi_y = tap.hi_ok && tap.d0 + 1 == db + 1;
-              const int cell = tab.cell[l] + (g.h0 + 1) * (tab.W[l] + 1) + g.w0 + 1;
+              const DepthPair<A> pair(tap, D);
+              const int cell = lv.cell + (g.h0 + 1) * (lv.W + 1) + g.w0 + 1;
               A x4[4], y4[4];
-              PackedTap<T>::ld(packed_r, (g.inside && tap.inside) ? (uint32_t)((cell * D + db) * 4 * (int)sizeof(T)) : kNoRow,
+              PackedTap<T>::ld(packed_r, (g.inside && tap.inside) ? (uint32_t)((cell * D + pair.db) * 4 * (int)sizeof(T)) : kNoRow,
                                x4, y4);
 #pragma unroll
-              for (int k = 0; k < 4; ++k) {
-                lo[k] = lo_x ? x4[k] : lo_y ? y4[k] : (A)0;
-                hi[k] = hi_x ? x4[k] : hi_y ? y4[k] : (A)0;
-                sc[k] = depth_lerp(lo[k], hi[k], tap.hd, tap.ld);
-              }
+              for (int k = 0; k < 4; ++k) sc[k] = pair.score(x4[k], y4[k]);
             } else {
-              corner_scores<T, A>(dist_r, g.key, tap, md, Md, D, sc, lo, hi);
+              grid_scores<T, A>(dist_r, g, tap, lv.d_base, lv.d_row, d_col, D, sc);
             }
             if (score_out != nullptr && pass == 0) {
-              T *so = score_out + gp * 4;
+              T *so = reinterpret_cast<T *>(reinterpret_cast<char *>(score_out + first_point(q0) * 4) + pl.idx * (uint32_t)(4 * sizeof(T)));
               if constexpr (sizeof(T) == 4) {                     // one 16-byte store
                 typedef float f4 __attribute__((ext_vector_type(4)));
                 f4 v4 = {(float)sc[0], (float)sc[1], (float)sc[2], (float)sc[3]};
@@ -278,16 +348,22 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
             }
             wu = a * ((sc[0] + sc[1] + sc[2] + sc[3]) * (A)0.25);
           } else {
-            const T *si = score_in + gp * 4;        // no scores given: plain deformable attention
+            // no scores given: plain deformable attention
 #pragma unroll
-            for (int k = 0; k < 4; ++k) sc[k] = score_in != nullptr ? Elem<T>::ld(si + k) : (A)1;
+            for (int k = 0; k < 4; ++k) sc[k] = (A)1;
+            if (score_in != nullptr) {                              // uniform
+              const T *si = reinterpret_cast<const T *>(reinterpret_cast<const char *>(score_in + first_point(q0) * 4) + pl.idx * (uint32_t)(4 * sizeof(T)));
+#pragma unroll
+              for (int k = 0; k < 4; ++k) sc[k] = Elem<T>::ld(si + k);
+            }
           }
+          const uint32_t at = (uint32_t)g.h0 * lv.v_row + (uint32_t)g.w0 * lv.v_col + lv.v_base;
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            if (g.key[k] >= 0) {
-              t4[k].off = (uint32_t)((from_lds ? g.key[k] - key0 : g.key[k] * M + m) * C * (int)sizeof(T));
-              t4[k].w = g.bil(k) * sc[k] * a;
-            }
+            const uint32_t off = at + (k >= 2 ? lv.v_row : 0) + (k == 1 || k == 2 ? lv.v_col : 0);
+            const A w = g.bil(k) * sc[k] * a;
+            t4[k].off = g.on(k) ? off : none;
+            t4[k].w = g.on(k) ? w : (A)0;
           }
         }
         if (FUSED && weight_update != nullptr && pass == 0) {      // wave-uniform
@@ -305,29 +381,29 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
           }
         }
         wave_lds_handover();     // previous phase B has consumed the task list
-        if (ws.upw == 1 || ul < ws.upw) {
-          Task<A> *to = tasks + (ws.upw == 1 ? lane * 4 : ul * unit_tasks + lp * 4);
-#pragma unroll
-          for (int k = 0; k < 4; ++k) to[k] = t4[k];
+        if (my_tasks) {
+          to[0] = t4[0]; to[to1] = t4[1]; to[to2] = t4[2]; to[to3] = t4[3];
         }
         wave_lds_handover();
 
+        __builtin_amdgcn_s_setprio(2);
         // ---------------- phase B: lanes over channels ----------------
         for (int u0 = 0; u0 < ws.upw; u0 += par) {              // one round, or three (one where a unit takes several chunks)
           const int u = u0 + row_slot / spu;
           const int n = (ws.upw == 1 ? min(kWave, ws.LP - chunk * kWave) : ws.LP) * 4;
-          const Task<A> *mine = tasks + u * (ws.upw == 1 ? 0 : unit_tasks);
+          const Task<A> *mine = tasks + (u0 * spu + row_slot) * run;
           const int far = IN_LDS ? min(max((l0 * P - chunk * kWave) * 4, 0), n) : n;
-          gather_rows<A, VEC>(rows, kNoRow, mine, row_slot % spu, spu, far, acc);
-          if constexpr (IN_LDS) gather_rows<A, VEC>(rows_in_lds, zero_row, mine + far, row_slot % spu, spu, n - far, acc);
+          const int n_far = (far + spu - 1 - part) >> spu_log2;
+          gather_rows<A, VEC>(rows, kNoRow, mine, far >> spu_log2, (far + spu - 1) >> spu_log2, n_far, acc);
+          if constexpr (IN_LDS)
+            gather_rows<A, VEC>(rows_in_lds, zero_row, mine + n_far, (n - far) >> spu_log2, (n - far + spu - 1) >> spu_log2,
+                                ((n + spu - 1 - part) >> spu_log2) - n_far, acc);
           if (chunk == ws.chunks - 1) {
-            for (int off = LPR; off < spu * LPR; off <<= 1) {
-#pragma unroll
-              for (int i = 0; i < VEC; ++i) acc[i] += __shfl_xor(acc[i], off, kWave);
-            }
-            if (row_slot % spu == 0 && chan_ok && q0 + u < Q) {
-              const size_t unit = ((size_t)b * Q + (q0 + u)) * M + m;
-              RowVec<T, A, VEC>::st(out + unit * C + chan, acc);
+        __builtin_amdgcn_s_setprio(1);
+            sum_over_slots<LPR, VEC>(spu * LPR, acc);
+            if (part == 0 && chan_ok && q0 + u < Q) {
+              T *group_out = out + ((size_t)(b * (size_t)Q + q0) * M + m) * C;
+              RowVec<T, A, VEC>::st(reinterpret_cast<T *>(reinterpret_cast<char *>(group_out) + ((uint32_t)u * (uint32_t)(M * C) + (uint32_t)chan) * (uint32_t)sizeof(T)), acc);
             }
 #pragma unroll
             for (int i = 0; i < VEC; ++i) acc[i] = 0;
@@ -530,6 +606,8 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   while (upw < kMaxUnitsPerWave && 2 * upw * a.L * a.P <= kWave) upw *= 2;
   if (upw > 1 && upw < kMaxUnitsPerWave && upw / 2 * 3 * a.L * a.P <= kWave) upw = upw / 2 * 3;    // 20 points: 60 lanes, not 40
   while (upw > 1 && (long long)a.M * a.B * ((a.Q + upw - 1) / upw) < kFewWaves) upw /= 2;
+  // (the kernel counts bytes from a group's first point, and from its first output row, in 32 bits)
+  while (upw > 1 && (long long)upw * a.M * std::max((long long)a.L * a.P * std::max<int>(a.loc_stride * sizeof(A), 4 * sizeof(T)), (long long)a.C * (long long)sizeof(T)) > 0x7FFFFFFFLL) upw /= 2;
   const FwdShape ws = fwd_shape(a.L, a.P, upw);
   const LdsRows lds = kLdsRowsTiling<T, VEC, LPR> ? lds_rows_plan<T, A>(a) : LdsRows{0, 0};
   const int parts = lds.parts;

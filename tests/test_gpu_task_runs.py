@@ -1,0 +1,53 @@
+"""The forward's tasks, which each row slot of a unit has side by side: slots that get unequal numbers of them, units in three rounds, a
+run that LDS has no room to pad; and the two taps of a distribution as weights of a pair of bins, where what is no tap must not be felt."""
+import pytest
+import torch
+
+from forms import tiny_case
+from test_gpu_parity import F32_FWD, _as_inputs, _dev
+
+pytestmark = pytest.mark.gpu
+
+LEVELS = ((9, 13), (5, 7), (3, 4), (2, 2))
+
+
+# enough queries that a wavefront keeps as many units as it has lanes for
+@pytest.mark.parametrize("L,P,C,Q", [(3, 7, 32, 1031), (3, 7, 16, 1031), (1, 9, 32, 2051), (1, 17, 64, 1025), (1, 19, 128, 1027), (1, 13, 20, 1367),
+                                     (4, 11, 32, 519), (1, 65, 32, 130)])
+@pytest.mark.parametrize("levels", [LEVELS, ((40, 61), (20, 31), (10, 16), (5, 8))], ids=["in LDS", "from memory"])
+def test_unequal_runs(oracle, L, P, C, Q, levels):
+    from dfa3D import _ext
+    dev = _dev()
+    t = _as_inputs(tiny_case(seed=17 * P + C, B=2, M=2, C=C, D=6, Q=Q, P=P, levels=levels[:L]))
+    args = [t[k].float() if t[k].is_floating_point() else t[k] for k in
+            ("value", "value_dpt_dist", "spatial_shapes", "level_start_index", "sampling_locations", "attention_weights")]
+    want, want_score = oracle.dfa3d_forward(*args)
+    got, score = _ext.dfa3d_fused_forward(*(x.to(dev) for x in args), 64, need_depth_score=True)
+    torch.testing.assert_close(got.cpu(), want, **F32_FWD)
+    torch.testing.assert_close(score.cpu(), want_score, **F32_FWD)
+
+
+@pytest.mark.parametrize("D,extent", [(2, 2), (3, 2), (7, 7), (7, 4), (1, 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64], ids=["fp32", "bf16", "fp64"])
+def test_bins_that_are_no_taps(oracle, D, extent, dtype):
+    """Depths on both sides of the first and of the last bin; bins beyond a level's depth extent hold NaN and infinities."""
+    from dfa3D import _ext
+    dev = _dev()
+    t = _as_inputs(tiny_case(seed=D, B=1, M=2, C=8, D=D, Q=64, P=4, levels=((5, 6), (3, 3))))
+    aux = torch.float64 if dtype == torch.float64 else torch.float32
+    dist = t["value_dpt_dist"].to(dtype)
+    clean = dist.clone()
+    clean[..., extent:] = 0
+    dist[..., extent:] = torch.tensor([float("nan"), float("inf"), float("-inf"), float("nan"), float("inf")], dtype=dtype)[:D - extent]
+    sh = t["spatial_shapes"].clone()
+    sh[:, 2] = extent
+    loc = t["sampling_locations"].to(aux)
+    edges = torch.linspace(-0.75, extent + 0.25, 64, dtype=aux) / extent
+    loc[..., 2] = edges.view(1, -1, 1, 1, 1)
+    rest = [loc, t["attention_weights"].to(aux)]
+    value = t["value"].to(dtype)
+    want, want_score = oracle.dfa3d_forward(value.to(aux), clean.to(aux), sh, t["level_start_index"], *rest)
+    got, score = _ext.dfa3d_fused_forward(*(x.to(dev) for x in (value, dist, sh, t["level_start_index"], *rest)), 64, need_depth_score=True)
+    tol = {torch.float32: F32_FWD, torch.float64: dict(rtol=1e-10, atol=1e-11), torch.bfloat16: dict(rtol=2 ** -8, atol=1e-5)}[dtype]
+    torch.testing.assert_close(got.cpu().to(aux), want, **tol)
+    torch.testing.assert_close(score.cpu().to(aux), want_score, **tol)
