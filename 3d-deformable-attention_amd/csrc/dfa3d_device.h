@@ -246,19 +246,46 @@ struct LevelTable {
   int cell[DFA3D_MAX_LEVELS + 1];   // packed distributions only (load_cell_starts): first cell of each level, total
 };
 
+// A level's sizes and first key; all zero where they do not fit S keys and D bins (D <= 0: depth extent unused).
+struct LevelSize { int H, W, Dd, start; };
+__device__ __forceinline__ LevelSize level_size(int64_t H, int64_t W, int64_t Dd, int64_t start, int S, int D) {
+  // 32 bits hold all that fits: a negative or larger number has bits above them
+  const uint32_t above = (uint32_t)((uint64_t)(H | W | start | (D > 0 ? Dd : 0)) >> 32);
+  const uint64_t keys = (uint64_t)(uint32_t)H * (uint32_t)W;
+  const bool ok = (above | (uint32_t)(keys >> 32)) == 0 && (uint32_t)keys != 0 && (uint32_t)keys <= (uint32_t)S &&
+                  (uint32_t)start <= (uint32_t)S - (uint32_t)keys && (D <= 0 || (uint32_t)Dd - 1u < (uint32_t)D);
+  return LevelSize{ok ? (int)H : 0, ok ? (int)W : 0, ok ? (int)Dd : 0, ok ? (int)start : 0};
+}
+// The sizes of level 0, 1, ... in turn as each(l, size): scalar loads, four levels' on their way at a time.
+template <typename Each>
+__device__ __forceinline__ void for_each_level(const int64_t *shapes, int shape_stride, const int64_t *level_start, int L, int S, int D,
+                                               const Each &each) {
+  const bool depth = shape_stride > 2 && D > 0;
+  for (int l0 = 0; l0 < L; l0 += 4) {
+    int64_t H[4], W[4], Dd[4], start[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int l = min(l0 + k, L - 1);
+      H[k] = shapes[l * shape_stride]; W[k] = shapes[l * shape_stride + 1];
+      Dd[k] = depth ? shapes[l * shape_stride + 2] : 1;
+      start[k] = level_start[l];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (l0 + k < L) each(l0 + k, level_size(H[k], W[k], Dd[k], start[k], S, D));
+  }
+}
+
 __device__ __forceinline__ void load_level_table(LevelTable &tab, const int64_t *shapes, int shape_stride,
                                                  const int64_t *level_start, int L, int S, int D) {
   if ((int)threadIdx.x < L) {
     const int l = threadIdx.x;
-    const int64_t H = shapes[l * shape_stride], W = shapes[l * shape_stride + 1];
-    const int64_t Dd = (shape_stride > 2 && D > 0) ? shapes[l * shape_stride + 2] : 1;   // D <= 0: depth extent unused
-    const int64_t st = level_start[l];
-    const bool ok = H > 0 && W > 0 && st >= 0 && H <= S && W <= S && st + H * W <= (int64_t)S &&
-                    Dd > 0 && (D <= 0 || Dd <= D);
-    tab.H[l] = ok ? (int)H : 0;
-    tab.W[l] = ok ? (int)W : 0;
-    tab.Dd[l] = ok ? (int)Dd : 0;
-    tab.start[l] = ok ? (int)st : 0;
+    const LevelSize v = level_size(shapes[l * shape_stride], shapes[l * shape_stride + 1],
+                                   (shape_stride > 2 && D > 0) ? shapes[l * shape_stride + 2] : 1, level_start[l], S, D);
+    tab.H[l] = v.H;
+    tab.W[l] = v.W;
+    tab.Dd[l] = v.Dd;
+    tab.start[l] = v.start;
   }
   __syncthreads();
 }

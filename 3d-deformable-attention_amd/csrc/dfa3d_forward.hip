@@ -32,20 +32,20 @@ __device__ __forceinline__ int task_run(int longest, int runs) {
 }
 
 // Phase B of the forward pass: acc += sum of w * row over a row slot's tasks.  LPR lanes of VEC channels take a row; the
-// wavefront's 64/LPR row slots may share a unit, each with a run of its tasks, or work on units of their own.  `all` tasks every slot
+// wavefront's 64/LPR row slots may share a unit, each with its tasks, `step` apart, or work on units of their own.  `all` tasks every slot
 // of the unit has, `most` the longest run (both uniform), `mine` this slot's.  Eight rows per lane are in flight, whatever the length
 // of the list: a unit of 8 points has 32 tasks, and walking it one row at a time waited for memory once per row.  A batch is summed in
 // two chains and added to acc as a whole, which keeps the longest chain of additions of a unit at about what a tree over the
 // row slots has.  `rows` reads this lane's channels of the row at a byte offset; `none` is the offset of a row of zeros.
 template <typename A, int VEC, typename Rows>
-__device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, const Task<A> *tasks, int all, int most, int mine,
-                                            A (&acc)[VEC]) {
+__device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, const Task<A> *tasks, int step, int all, int most,
+                                            int mine, A (&acc)[VEC]) {
   constexpr int U = 8, UT = 4;
   int t = 0;                                             // uniform
   for (; t + U <= all; t += U) {
     Task<A> e[U];
 #pragma unroll
-    for (int j = 0; j < U; ++j) e[j] = tasks[t + j];
+    for (int j = 0; j < U; ++j) e[j] = tasks[(t + j) * step];
     A v[U][VEC];
 #pragma unroll
     for (int j = 0; j < U; ++j) rows(e[j].off, v[j]);
@@ -67,7 +67,7 @@ __device__ __forceinline__ void gather_rows(const Rows &rows, uint32_t none, con
       for (int i = 0; i < VEC; ++i) v[j][i] = 0;
       if (t + j < most) {                                // uniform
         const bool has = t + j < mine;
-        e[j] = tasks[has ? t + j : 0];
+        e[j] = tasks[has ? (t + j) * step : 0];
         if (!has) { e[j].off = none; e[j].w = 0; }
         rows(e[j].off, v[j]);
       }
@@ -140,10 +140,19 @@ template <int FROM, int VEC> __device__ __forceinline__ void sum_over_slots(int 
 // that begins a group (s_setprio 2, 1, 0; the other way round 3120 us for the 3047 of two steps and 3000 of three, 24 planes and 128 bins).  Together, one card, us:
 //   6 x 10000 queries, 4 levels from 116 x 200, 8 points: 885 -> 872, around the query 574 -> 571 (bfloat16 483 -> 476), plain attention 436 -> 389;
 //   6 x 40000 clustered, 128 bins: 3067 -> 3000; the two separate stages without gradients, 112 bins: 1013 -> 936; one level of 23 x 40: 39.7 -> 38.0;
-//   plain attention, 2 x 40000 queries of 4 points: 109 -> 99.  (6 heads of 20 channels, three levels of 5 points: 44.1 -> 45.0.)
+// Where a workgroup has one group (not IN_LDS) these priorities took more than they gave for rows that the L2 holds (plain attention, 4 x 10000
+// queries of 4 points on 116 x 197: 59.5 -> 63.7) and gave where it does not (2 x 40000 on 200 x 200, around the query 103 -> 96, anywhere 65 -> 69): none.
+//
+// Without rows in LDS each wavefront with depth taps finds its levels' sizes for itself (kOwnLevels), which with the order of tasks that
+// launch_fwd_cfg chooses gives, us, 4 x 4000 queries on three levels from 60 x 100, 4 points, around the query: 63 -> 57, 16 channels 38.5 -> 33.7, 20 channels
+// 43 -> 38.6, bfloat16 49 -> 45.7; four levels of 8 points 118 -> 111; 64 channels 82.6 -> 78.6; 6 heads of 20 channels, three levels of 5 points
+// 45.2 -> 43.5.  Plain attention and given scores gain nothing from it (96 -> 100) but from six wavefronts a SIMD (kFwdWaves, 80 registers): 3 x 3 points
+// 33.5 -> 30.1.  (One distribution in bfloat16, packed, four levels of 8 points: 140 -> 141, around the query 116 -> 119.)
 // ---------------------------------------------------------------------------------------
-template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS>
-__global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention_kernel(
+// wavefronts a SIMD that the registers have to leave room for (1: as the compiler likes)
+template <typename T, int VEC, bool FUSED, bool IN_LDS> constexpr int kFwdWaves = !FUSED && !IN_LDS && sizeof(T) == 4 && VEC == 4 ? 6 : 1;
+template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS, bool IN_TURN>
+__global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC, FUSED, IN_LDS>)) void fwd_attention_kernel(
     const T *__restrict__ value, const T *__restrict__ dist, const int64_t *__restrict__ shapes, int shape_stride,
     const int64_t *__restrict__ level_start, const A *__restrict__ loc, int loc_stride,
     const A *__restrict__ attn, const T *__restrict__ score_in, T *__restrict__ out, T *__restrict__ score_out,
@@ -199,10 +208,11 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
     }
     return o;
   };
-  // The first group's are on their way while the level table is: a workgroup of one group otherwise waits for one after the other (2 x 40000
-  // queries of plain attention, 4 points: 98.7 -> 94 us; 2 x 100 queries 6.24 -> 6.04; larger calls +- 0.5 %).
+  // Plain attention and given scores, rows from memory: the first group's are on their way while the level table is; a workgroup of one group
+  // otherwise waits for one after the other (2 x 40000 queries of plain attention, 4 points: 100 -> 97 us).  With depth taps see kOwnLevels.
+  constexpr bool kAhead = !FUSED && !IN_LDS;
   Place pl = place(0);
-  const Operands first = IN_LDS ? Operands{0, 0, 0, 0} : fetch((qb * iters * WAVES + wave) * ws.upw, pl);
+  const Operands first = kAhead ? fetch((qb * iters * WAVES + wave) * ws.upw, pl) : Operands{0, 0, 0, 0};
   // phase B: `par` units at a time, `spu` row slots each
   constexpr int RPI = kWave / LPR;
   const int par = min(ws.upw & -ws.upw, RPI), spu = RPI / par, spu_log2 = 31 - __builtin_clz(spu);
@@ -211,22 +221,37 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
   const int run = task_run((unit_points * 4 + spu - 1) >> spu_log2, ws.upw * spu);
   const int my_point = ws.upw == 1 ? lane : pl.lp, my_unit = ws.upw == 1 ? 0 : pl.ul;
   const bool my_tasks = my_point < unit_points && my_unit < ws.upw;
-  Task<A> *const to = tasks + (my_unit * spu + ((my_point * 4) & (spu - 1))) * run + ((my_point * 4) >> spu_log2);
-  const int to1 = spu > 1 ? run : 1, to2 = spu > 2 ? 2 * run : spu == 2 ? 1 : 2, to3 = spu == 2 ? run + 1 : to1 + to2;
+  // IN_TURN: as they come instead, a unit's side by side.
+  const int unit_room = unit_points * 4 + (ws.upw == 1 ? 0 : 2);
+  Task<A> *const to = tasks + (IN_TURN ? my_unit * unit_room + my_point * 4
+                                       : (my_unit * spu + ((my_point * 4) & (spu - 1))) * run + ((my_point * 4) >> spu_log2));
+  const int to1 = !IN_TURN && spu > 1 ? run : 1, to2 = !IN_TURN && spu > 2 ? 2 * run : !IN_TURN && spu == 2 ? 1 : 2;
+  const int to3 = !IN_TURN && spu == 2 ? run + 1 : to1 + to2;
   const int part = row_slot % spu;
 
-  load_level_table(tab, shapes, shape_stride, level_start, L, S, FUSED ? D : 0);
-  if (FUSED && packed_arg != nullptr) load_cell_starts(tab, L);      // uniform
+  // Depth taps, rows from memory: no level table.  Its barrier held a workgroup's four wavefronts in step, so that they looked for corners and
+  // gathered rows all at once; each now reads the levels' sizes as scalars and goes its own way.
+  constexpr bool kOwnLevels = FUSED && !IN_LDS;
+  int cells = 0;
+  if constexpr (!kOwnLevels) {
+    load_level_table(tab, shapes, shape_stride, level_start, L, S, FUSED ? D : 0);
+    if (FUSED && packed_arg != nullptr) {                              // uniform
+      load_cell_starts(tab, L);
+      cells = tab.cell[L];
+    }
+  } else if (packed_arg != nullptr) {
+    for_each_level(shapes, shape_stride, level_start, L, S, D, [&](int, const LevelSize &z) { cells += (z.H + 1) * (z.W + 1); });
+  }
   // The packed table was sized on the host for levels that share no keys (at most 2 S + 2 L cells).  A level
   // table whose levels overlap can ask for more: then the table is not used (nor was it written) and the taps
   // come from dist itself.
-  const T *packed = (FUSED && packed_arg != nullptr && tab.cell[L] <= packed_cell_capacity(S, L)) ? packed_arg : nullptr;
+  const T *packed = (FUSED && packed_arg != nullptr && cells <= packed_cell_capacity(S, L)) ? packed_arg : nullptr;
 
   const rsrc_t value_r = make_rsrc(value + (size_t)b * S * M * C, (size_t)S * M * C * sizeof(T));
   const rsrc_t dist_r = make_rsrc(FUSED ? dist + (size_t)b * S * Md * D : nullptr,
                                   FUSED ? (size_t)S * Md * D * sizeof(T) : 0);
   const int md = Md == 1 ? 0 : m;                                    // head whose distribution this head reads
-  const size_t packed_slice = (FUSED && packed != nullptr) ? (size_t)tab.cell[L] * D * 4 : 0;   // elements per batch element
+  const size_t packed_slice = (FUSED && packed != nullptr) ? (size_t)cells * D * 4 : 0;   // elements per batch element
   const rsrc_t packed_r = make_rsrc(packed_slice ? packed + (size_t)b * packed_slice : nullptr, packed_slice * sizeof(T));
   // IN_LDS: levels l0, l0 + 1, ... , whose keys are among the last lds_rows ones
   int l0 = IN_LDS ? L : 0, key0 = S;
@@ -260,10 +285,21 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
   struct Level { int H, W, Dd, cell; uint32_t v_col, v_row, v_base, d_row, d_base; bool in_lds; };
   const uint32_t d_col = (uint32_t)(Md * D * (int)sizeof(T));
   auto level = [&](const Place &at) {
-    const int l = min(at.lp / P, L - 1), start = tab.start[l];
-    Level v;
-    v.H = tab.H[l]; v.W = tab.W[l]; v.Dd = tab.Dd[l];
-    v.cell = FUSED && packed != nullptr ? tab.cell[l] : 0;
+    const int l = min(at.lp / P, L - 1);
+    Level v{};
+    int start = 0;
+    if constexpr (kOwnLevels) {
+      int cell = 0;
+      for_each_level(shapes, shape_stride, level_start, L, S, D, [&](int i, const LevelSize &z) {
+        const bool here = i == l;
+        v.H = here ? z.H : v.H; v.W = here ? z.W : v.W; v.Dd = here ? z.Dd : v.Dd; v.cell = here ? cell : v.cell;
+        start = here ? z.start : start;
+        cell += (z.H + 1) * (z.W + 1);
+      });
+    } else {
+      v.H = tab.H[l]; v.W = tab.W[l]; v.Dd = tab.Dd[l]; start = tab.start[l];
+      v.cell = FUSED && packed != nullptr ? tab.cell[l] : 0;
+    }
     v.in_lds = IN_LDS && l >= l0;
     v.v_col = (uint32_t)((v.in_lds ? C : M * C) * (int)sizeof(T));
     v.v_row = (uint32_t)v.W * v.v_col;
@@ -304,14 +340,14 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
       for (int v = 0; v < VEC; ++v) acc[v] = 0;
 
       for (int chunk = 0; chunk < ws.chunks; ++chunk) {
-        __builtin_amdgcn_s_setprio(0);                       // a group begins
+        if (IN_LDS) __builtin_amdgcn_s_setprio(0);                       // a group begins
         // ---------------- phase A: one lane per sampling point ----------------
         if (ws.chunks > 1) pl = place(chunk);                // uniform
-        if (!IN_LDS || ws.chunks > 1) lv = level(pl);
         const int ul = pl.ul, lp = pl.lp, q = q0 + ul;       // unit within group, point within unit
         const bool live = ul < min(ws.upw, Q - q0);
         Operands in = first;
-        if (IN_LDS || it > 0 || pass > 0 || chunk > 0) in = fetch(q0, pl);      // uniform
+        if (!kAhead || it > 0 || pass > 0 || chunk > 0) in = fetch(q0, pl);      // uniform
+        if (!IN_LDS || ws.chunks > 1) lv = level(pl);
         Task<A> t4[4];
         A wu = 0;
         const uint32_t none = lv.in_lds ? zero_row : kNoRow;
@@ -319,7 +355,7 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
         for (int k = 0; k < 4; ++k) { t4[k].off = none; t4[k].w = 0; }
         if (live) {
           const A a = in.a;
-        __builtin_amdgcn_s_setprio(1);
+          if (IN_LDS) __builtin_amdgcn_s_setprio(1);
           const Grid2D<A> g = locate_grid<A>(in.x, in.y, lv.H, lv.W);
           A sc[4];
           if (FUSED) {
@@ -386,20 +422,20 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock) void fwd_attention
         }
         wave_lds_handover();
 
-        __builtin_amdgcn_s_setprio(2);
+        if (IN_LDS) __builtin_amdgcn_s_setprio(2);
         // ---------------- phase B: lanes over channels ----------------
         for (int u0 = 0; u0 < ws.upw; u0 += par) {              // one round, or three (one where a unit takes several chunks)
           const int u = u0 + row_slot / spu;
           const int n = (ws.upw == 1 ? min(kWave, ws.LP - chunk * kWave) : ws.LP) * 4;
-          const Task<A> *mine = tasks + (u0 * spu + row_slot) * run;
           const int far = IN_LDS ? min(max((l0 * P - chunk * kWave) * 4, 0), n) : n;
           const int n_far = (far + spu - 1 - part) >> spu_log2;
-          gather_rows<A, VEC>(rows, kNoRow, mine, far >> spu_log2, (far + spu - 1) >> spu_log2, n_far, acc);
+          const Task<A> *mine = tasks + (IN_TURN ? u * unit_room + part : (u0 * spu + row_slot) * run);
+          gather_rows<A, VEC>(rows, kNoRow, mine, IN_TURN ? spu : 1, far >> spu_log2, (far + spu - 1) >> spu_log2, n_far, acc);
           if constexpr (IN_LDS)
-            gather_rows<A, VEC>(rows_in_lds, zero_row, mine + n_far, (n - far) >> spu_log2, (n - far + spu - 1) >> spu_log2,
+            gather_rows<A, VEC>(rows_in_lds, zero_row, mine + n_far, 1, (n - far) >> spu_log2, (n - far + spu - 1) >> spu_log2,
                                 ((n + spu - 1 - part) >> spu_log2) - n_far, acc);
           if (chunk == ws.chunks - 1) {
-        __builtin_amdgcn_s_setprio(1);
+            if (IN_LDS) __builtin_amdgcn_s_setprio(1);
             sum_over_slots<LPR, VEC>(spu * LPR, acc);
             if (part == 0 && chan_ok && q0 + u < Q) {
               T *group_out = out + ((size_t)(b * (size_t)Q + q0) * M + m) * C;
@@ -626,6 +662,13 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   // locations alone 272, 269, 267; on the same operands again and again, which the Infinity Cache then holds in part, 230, 258, 238.)
   const bool large = (long long)a.B * a.Q * a.M * a.L * a.P * (a.loc_stride + 1) * (long long)sizeof(A) > (48LL << 20);
   const int once = !large ? 0 : (a.L * a.P * a.loc_stride * sizeof(A) % 128 == 0 ? 1 : 0) | (a.L * a.P * sizeof(A) % 128 == 0 ? 2 : 0);
+  // How a unit's tasks lie in LDS where several row slots share it: in the order of its points, or a run for each slot, which takes half the
+  // instructions to read.  Runs where the XCD's L2 does not hold a (batch, head)'s value rows well: half of it, 2 MB.  In turn and runs, us, 4 x 4000
+  // queries, 8 points on four levels, value rows of 1 MB: 110.7, 113; plain attention 81.4, 89 and with 4 points 45.5, 49.7; 12 points, 16 channels
+  // 33.7, 35.8.  3.9 MB, 3000 queries 159.5, 151; 2.3 MB, 4 points a level 116, 111; their second stage alone 133, 129.  A packed float32
+  // distribution, 1 MB: 160.6, 149.5 (3.9 MB: 167, 155); bfloat16 141, 143.
+  const int par = std::min(upw & -upw, kWave / LPR);
+  const bool in_turn = kWave / LPR > par && (long long)a.S * a.C * (long long)sizeof(T) <= (2LL << 20) && !(fused && a.packed_dist != nullptr && sizeof(T) == 4);
   auto launch = [&](auto kernel, int threads, size_t bytes) -> hipError_t {
     if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), bytes)) return e;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), bytes, stream, (const T *)a.value, (const T *)a.dist, a.shapes,
@@ -638,12 +681,15 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   if constexpr (kLdsRowsTiling<T, VEC, LPR>) {
     if (parts > 0) {
       const size_t bytes = ((size_t)lds.rows + 1) * a.C * sizeof(T);
-      return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, true>, kLdsRowsBlock, bytes)
-                   : launch(fwd_attention_kernel<T, A, VEC, LPR, false, true>, kLdsRowsBlock, bytes);
+      return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, true, false>, kLdsRowsBlock, bytes)
+                   : launch(fwd_attention_kernel<T, A, VEC, LPR, false, true, false>, kLdsRowsBlock, bytes);
     }
   }
-  return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false>, kBlock, 0)
-               : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false>, kBlock, 0);
+  if (in_turn)
+    return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, true>, kBlock, 0)
+                 : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, true>, kBlock, 0);
+  return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, false>, kBlock, 0)
+               : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, false>, kBlock, 0);
 }
 
 template <typename T, typename A>

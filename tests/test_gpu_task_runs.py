@@ -51,3 +51,61 @@ def test_bins_that_are_no_taps(oracle, D, extent, dtype):
     tol = {torch.float32: F32_FWD, torch.float64: dict(rtol=1e-10, atol=1e-11), torch.bfloat16: dict(rtol=2 ** -8, atol=1e-5)}[dtype]
     torch.testing.assert_close(got.cpu().to(aux), want, **tol)
     torch.testing.assert_close(score.cpu().to(aux), want_score, **tol)
+
+
+# value rows of one (batch, head) on both sides of 2 MB, where the order of a unit's tasks changes: 128 and 64 channels, 4096 and 8192 keys
+@pytest.mark.parametrize("C,levels", [(128, ((64, 63), (8, 8))), (128, ((64, 63), (8, 8), (1, 1))), (64, ((91, 90),)), (64, ((91, 90), (2, 2)))])
+@pytest.mark.parametrize("call", ["one stage", "packed", "scores", "plain"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_order_of_tasks(oracle, C, levels, call, dtype):
+    from dfa3D import _ext
+    dev = _dev()
+    t = _as_inputs(tiny_case(seed=C + len(levels), B=1, M=2, C=C, D=4, Q=1301, P=7, levels=levels))
+    value, dist = (t[k].to(dtype) for k in ("value", "value_dpt_dist"))
+    sh, lsi, loc, attn = t["spatial_shapes"], t["level_start_index"], t["sampling_locations"].float(), t["attention_weights"].float()
+    if call == "packed":
+        dist = dist[:, :, :1].contiguous()
+    want, score = oracle.dfa3d_forward(value.float(), dist.float().expand(-1, -1, 2, -1).contiguous(), sh, lsi, loc, attn)
+    on = [x.to(dev) for x in (value, dist, sh, lsi, loc, attn)]
+    if call in ("one stage", "packed"):
+        packed = _ext.pack_shared_dist(*on[1:4]) if call == "packed" else None
+        got = _ext.dfa3d_fused_forward(*on, 64, need_depth_score=False, packed_dist=packed)[0]
+    else:
+        from dfa3D import functional
+        xy, sh2 = on[4][..., :2].contiguous(), on[2][:, :2].contiguous()
+        if call == "plain":
+            got = functional.MultiScaleDeformableAttnFunction.apply(on[0], sh2, on[3], xy, on[5], 64)
+            want = oracle.dfa3d_forward(value.float(), torch.ones_like(t["value_dpt_dist"][..., :1]).float(),
+                                        torch.cat([sh[:, :2], torch.ones_like(sh[:, :1])], 1), lsi,
+                                        torch.cat([loc[..., :2], torch.full_like(loc[..., :1], 0.5)], -1), attn)[0]
+        else:
+            given = score.to(dtype)
+            got = functional.WeightedMultiScaleDeformableAttnFunction.apply(on[0], sh2, on[3], xy, on[5], given.to(dev), 64)
+    # bfloat16: the output's own rounding, and that of the scores that are handed over
+    tol = F32_FWD if dtype == torch.float32 else dict(rtol=2 ** -7, atol=2 ** -7)
+    torch.testing.assert_close(got.float().cpu(), want, **tol)
+
+
+@pytest.mark.parametrize("L", [1, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("packed", [False, True])
+def test_levels_four_at_a_time(oracle, L, packed):
+    """Levels' sizes, four read at a time; one that does not fit the keys or bins adds nothing, as with weights of zero."""
+    from dfa3D import _ext
+    dev = _dev()
+    t = _as_inputs(tiny_case(seed=L, B=2, M=2, C=16, D=5, Q=37, P=3, levels=tuple((3 + l % 4, 2 + l % 3) for l in range(L))))
+    value, dist, sh, lsi, loc, attn = (t[k].float() if t[k].is_floating_point() else t[k] for k in
+                                       ("value", "value_dpt_dist", "spatial_shapes", "level_start_index", "sampling_locations", "attention_weights"))
+    if packed:
+        dist = dist[:, :, :1].contiguous()
+    bad, bad_lsi, kept = sh.clone(), lsi.clone(), attn.clone()
+    for l, column, number in ((1, 0, 2 ** 32 + 3), (4, 2, 6), (7, 1, -2), (8, 0, 2 ** 31), (15, 2, 2 ** 32 + 5)):
+        if l < L:
+            bad[l, column] = number
+            kept[:, :, :, l] = 0
+    if L > 2:
+        bad_lsi[2] = -1
+        kept[:, :, :, 2] = 0
+    want, _ = oracle.dfa3d_forward(value, dist.expand(-1, -1, 2, -1).contiguous(), sh, lsi, loc, kept)
+    on = [x.to(dev) for x in (value, dist, bad, bad_lsi, loc, attn)]
+    got = _ext.dfa3d_fused_forward(*on, 64, need_depth_score=False, packed_dist=_ext.pack_shared_dist(*on[1:4]) if packed else None)[0]
+    torch.testing.assert_close(got.cpu(), want, **F32_FWD)
