@@ -109,3 +109,24 @@ def test_levels_four_at_a_time(oracle, L, packed):
     on = [x.to(dev) for x in (value, dist, bad, bad_lsi, loc, attn)]
     got = _ext.dfa3d_fused_forward(*on, 64, need_depth_score=False, packed_dist=_ext.pack_shared_dist(*on[1:4]) if packed else None)[0]
     torch.testing.assert_close(got.cpu(), want, **F32_FWD)
+
+
+@pytest.mark.parametrize("D", [2, 31, 64, 255, 256, 257, 600])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_packed_table_as_laid_out(D, dtype):
+    """Every cell and bin against the four pixels around it: rows of cells of one run and of several, an empty level, a map of one pixel."""
+    from dfa3D import _ext
+    dev = _dev()
+    levels, B = ((5, 130), (1, 1), (7, 3)), 3
+    S = sum(h * w for h, w in levels) + 4
+    dist = torch.rand(B, S, 1, D, generator=torch.Generator().manual_seed(D)).to(dtype)
+    sh = torch.tensor([(h, w, D) for h, w in levels] + [(S + 1, 2, D)])                  # the last does not fit: empty
+    start = [0, 650, 651, 0]
+    got = _ext.pack_shared_dist(dist.to(dev), sh.to(dev), torch.tensor(start).to(dev))
+    want = []
+    for (h, w), s in zip(levels + ((0, 0),), start):
+        m = torch.nn.functional.pad(dist[:, s:s + h * w, 0].reshape(B, h, w, D), (0, 0, 1, 1, 1, 1))
+        four = torch.stack([m[:, :-1, :-1], m[:, :-1, 1:], m[:, 1:, 1:], m[:, 1:, :-1]], -1)
+        want.append(four.reshape(B, (h + 1) * (w + 1) * D * 4))
+    want = torch.cat(want, 1)
+    assert torch.equal(got.view(dtype)[:want.numel()].cpu(), want.view(-1))
