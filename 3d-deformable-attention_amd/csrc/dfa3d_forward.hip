@@ -146,13 +146,14 @@ template <int FROM, int VEC> __device__ __forceinline__ void sum_over_slots(int 
 // Without rows in LDS each wavefront with depth taps finds its levels' sizes for itself (kOwnLevels), which with the order of tasks that
 // launch_fwd_cfg chooses gives, us, 4 x 4000 queries on three levels from 60 x 100, 4 points, around the query: 63 -> 57, 16 channels 38.5 -> 33.7, 20 channels
 // 43 -> 38.6, bfloat16 49 -> 45.7; four levels of 8 points 118 -> 111; 64 channels 82.6 -> 78.6; 6 heads of 20 channels, three levels of 5 points
-// 45.2 -> 43.5.  Plain attention and given scores gain nothing from it (96 -> 100) but from six wavefronts a SIMD (kFwdWaves, 80 registers): 3 x 3 points
-// 33.5 -> 30.1.  (One distribution in bfloat16, packed, four levels of 8 points: 140 -> 141, around the query 116 -> 119.)
+// 45.2 -> 43.5.  Plain attention and given scores gain nothing from it (96 -> 100).  Six wavefronts a SIMD (kFwdWaves: 80 registers, which nothing is
+// spilled for) where five were: plain attention, 3 x 3 points 33.5 -> 30.1; one distribution for all heads, packed, four levels of 8 points, around the query 125 ->
+// 118.5, anywhere 150 -> 144, 9000 queries, 116 x 197 326 -> 315; other calls with runs +- 0.5 %.  Seven spill (118.5 -> 141).  (One distribution in bfloat16, packed, four levels of 8 points: 140 -> 141, around the query 116 -> 119.)
 // ---------------------------------------------------------------------------------------
 // wavefronts a SIMD that the registers have to leave room for (1: as the compiler likes)
-template <typename T, int VEC, bool FUSED, bool IN_LDS> constexpr int kFwdWaves = !FUSED && !IN_LDS && sizeof(T) == 4 && VEC == 4 ? 6 : 1;
+template <typename T, int VEC, bool IN_LDS> constexpr int kFwdWaves = !IN_LDS && sizeof(T) == 4 && VEC == 4 ? 6 : 1;
 template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS, bool IN_TURN>
-__global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC, FUSED, IN_LDS>)) void fwd_attention_kernel(
+__global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC, IN_LDS>)) void fwd_attention_kernel(
     const T *__restrict__ value, const T *__restrict__ dist, const int64_t *__restrict__ shapes, int shape_stride,
     const int64_t *__restrict__ level_start, const A *__restrict__ loc, int loc_stride,
     const A *__restrict__ attn, const T *__restrict__ score_in, T *__restrict__ out, T *__restrict__ score_out,
@@ -666,7 +667,7 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   // instructions to read.  Runs where the XCD's L2 does not hold a (batch, head)'s value rows well: half of it, 2 MB.  In turn and runs, us, 4 x 4000
   // queries, 8 points on four levels, value rows of 1 MB: 110.7, 113; plain attention 81.4, 89 and with 4 points 45.5, 49.7; 12 points, 16 channels
   // 33.7, 35.8.  3.9 MB, 3000 queries 159.5, 151; 2.3 MB, 4 points a level 116, 111; their second stage alone 133, 129.  A packed float32
-  // distribution, 1 MB: 160.6, 149.5 (3.9 MB: 167, 155); bfloat16 141, 143.
+  // distribution, 1 MB: 160.6, 144 (3.9 MB: 167, 155); bfloat16 141, 143.
   const int par = std::min(upw & -upw, kWave / LPR);
   const bool in_turn = kWave / LPR > par && (long long)a.S * a.C * (long long)sizeof(T) <= (2LL << 20) && !(fused && a.packed_dist != nullptr && sizeof(T) == 4);
   auto launch = [&](auto kernel, int threads, size_t bytes) -> hipError_t {
