@@ -152,7 +152,7 @@ template <int FROM, int VEC> __device__ __forceinline__ void sum_over_slots(int 
 // ---------------------------------------------------------------------------------------
 // wavefronts a SIMD that the registers have to leave room for (1: as the compiler likes)
 template <typename T, int VEC, bool IN_LDS> constexpr int kFwdWaves = !IN_LDS && sizeof(T) == 4 && VEC == 4 ? 6 : 1;
-template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS, bool IN_TURN>
+template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS, bool IN_TURN, bool EARLY>
 __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC, IN_LDS>)) void fwd_attention_kernel(
     const T *__restrict__ value, const T *__restrict__ dist, const int64_t *__restrict__ shapes, int shape_stride,
     const int64_t *__restrict__ level_start, const A *__restrict__ loc, int loc_stride,
@@ -209,9 +209,8 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC,
     }
     return o;
   };
-  // Plain attention and given scores, rows from memory: the first group's are on their way while the level table is; a workgroup of one group
-  // otherwise waits for one after the other (2 x 40000 queries of plain attention, 4 points: 100 -> 97 us).  With depth taps see kOwnLevels.
-  constexpr bool kAhead = !FUSED && !IN_LDS;
+  // EARLY, no depth taps: the first group's are on their way while the level table is (launch_fwd_cfg)
+  constexpr bool kAhead = EARLY && !FUSED;
   Place pl = place(0);
   const Operands first = kAhead ? fetch((qb * iters * WAVES + wave) * ws.upw, pl) : Operands{0, 0, 0, 0};
   // phase B: `par` units at a time, `spu` row slots each
@@ -669,7 +668,16 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   // 33.7, 35.8.  3.9 MB, 3000 queries 159.5, 151; 2.3 MB, 4 points a level 116, 111; their second stage alone 133, 129.  A packed float32
   // distribution, 1 MB: 160.6, 144 (3.9 MB: 167, 155); bfloat16 141, 143.
   const int par = std::min(upw & -upw, kWave / LPR);
-  const bool in_turn = kWave / LPR > par && (long long)a.S * a.C * (long long)sizeof(T) <= (2LL << 20) && !(fused && a.packed_dist != nullptr && sizeof(T) == 4);
+  const long long map_bytes = (long long)a.S * a.C * (long long)sizeof(T);                  // a (batch, head)'s value rows
+  const bool in_turn = kWave / LPR > par && map_bytes <= (2LL << 20) && !(fused && a.packed_dist != nullptr && sizeof(T) == 4);
+  // Plain attention, the first group's locations and weights before the level table: a wavefront of one group then waits once, not twice, but all of
+  // them gather rows the sooner together, which costs more where caches serve them.  Float32 units of four points with rows of whole lines on maps above
+  // 1.5 MB gain.  4 x 31250 queries around the query and anywhere, table first and early, us: 32 channels, 1.1 MB 110, 110 and 106, 107; 2.2 MB
+  // 136, 133 and 137, 139; 8.7 MB 206, 204 and 269, 268; two levels of 2 points, 2.7 MB 137, 134 and 155, 156; 64 channels, 2.1 MB 203, 196 and
+  // 189, 186; 4.4 MB 238, 229 and 269, 271.  16 channels, 4.4 MB 143, 145 and 220, 219; 20 channels, 5.4 MB 189, 202 and 308, 307; 2 points a unit,
+  // 2.2 MB 120, 122 and 127, 130.  Early over table first, 32 channels, four sizes of map: 8 to 64
+  // points 1.00 - 1.12 (20 points 0.96 - 1.01), bfloat16 0.99 - 1.07 (15 and 20 points 0.95 - 1.02), float64 up to 1.08.
+  const bool early = !fused && a.score_in == nullptr && sizeof(T) == 4 && a.L * a.P == 4 && a.C >= 32 && 2 * map_bytes > (3LL << 20);
   auto launch = [&](auto kernel, int threads, size_t bytes) -> hipError_t {
     if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), bytes)) return e;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), bytes, stream, (const T *)a.value, (const T *)a.dist, a.shapes,
@@ -682,15 +690,18 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   if constexpr (kLdsRowsTiling<T, VEC, LPR>) {
     if (parts > 0) {
       const size_t bytes = ((size_t)lds.rows + 1) * a.C * sizeof(T);
-      return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, true, false>, kLdsRowsBlock, bytes)
-                   : launch(fwd_attention_kernel<T, A, VEC, LPR, false, true, false>, kLdsRowsBlock, bytes);
+      return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, true, false, false>, kLdsRowsBlock, bytes)
+                   : launch(fwd_attention_kernel<T, A, VEC, LPR, false, true, false, false>, kLdsRowsBlock, bytes);
     }
   }
   if (in_turn)
-    return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, true>, kBlock, 0)
-                 : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, true>, kBlock, 0);
-  return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, false>, kBlock, 0)
-               : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, false>, kBlock, 0);
+    return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, true, false>, kBlock, 0)
+                 : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, true, false>, kBlock, 0);
+  if constexpr (std::is_same<T, float>::value) {
+    if (early) return launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, false, true>, kBlock, 0);
+  }
+  return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, false, false>, kBlock, 0)
+               : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, false, false>, kBlock, 0);
 }
 
 template <typename T, typename A>

@@ -86,6 +86,28 @@ def test_order_of_tasks(oracle, C, levels, call, dtype):
     torch.testing.assert_close(got.float().cpu(), want, **tol)
 
 
+# value rows of one (batch, head) on both sides of 1.5 MB, above which units of four points have their first operands asked for before the level table:
+# 12288 rows of 32 channels, 6144 of 64, 1512 of 260 (two passes over the channels)
+@pytest.mark.parametrize("C,levels,P", [(32, ((96, 128),), 4), (32, ((97, 128),), 4), (32, ((96, 128), (1, 1)), 2), (64, ((64, 97), (2, 1), (1, 1), (1, 1)), 1),
+                                        (260, ((36, 42),), 4), (260, ((37, 42),), 4), (28, ((120, 128),), 4), (32, ((97, 128),), 3)])
+@pytest.mark.parametrize("Q", [1, 301, 8201])
+@pytest.mark.parametrize("scores", [False, True])
+def test_units_of_four_points(oracle, C, levels, P, Q, scores):
+    """Plain attention and given scores, from one unit per wavefront up to sixteen."""
+    from dfa3D import functional
+    dev = _dev()
+    t = _as_inputs(tiny_case(seed=C + P + Q, B=1, M=2, C=C, D=2, Q=Q, P=P, levels=levels))
+    value, dist, sh, lsi, loc, attn = (t[k].float() if t[k].is_floating_point() else t[k] for k in
+                                       ("value", "value_dpt_dist", "spatial_shapes", "level_start_index", "sampling_locations", "attention_weights"))
+    if not scores:
+        dist, sh, loc = torch.ones_like(dist[..., :1]), torch.cat([sh[:, :2], torch.ones_like(sh[:, :1])], 1), torch.cat([loc[..., :2], torch.full_like(loc[..., :1], 0.5)], -1)
+    want, score = oracle.dfa3d_forward(value, dist.contiguous(), sh, lsi, loc, attn)
+    v, s2, start, xy, a = (x.to(dev) for x in (value, sh[:, :2].contiguous(), lsi, loc[..., :2].contiguous(), attn))
+    got = (functional.WeightedMultiScaleDeformableAttnFunction.apply(v, s2, start, xy, a, score.to(dev), 64) if scores else
+           functional.MultiScaleDeformableAttnFunction.apply(v, s2, start, xy, a, 64))
+    torch.testing.assert_close(got.cpu(), want, **F32_FWD)
+
+
 @pytest.mark.parametrize("L", [1, 3, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("packed", [False, True])
 def test_levels_four_at_a_time(oracle, L, packed):
