@@ -143,12 +143,9 @@ template <int FROM, int VEC> __device__ __forceinline__ void sum_over_slots(int 
 // Where a workgroup has one group (not IN_LDS) these priorities took more than they gave for rows that the L2 holds (plain attention, 4 x 10000
 // queries of 4 points on 116 x 197: 59.5 -> 63.7) and gave where it does not (2 x 40000 on 200 x 200, around the query 103 -> 96, anywhere 65 -> 69): none.
 //
-// Without rows in LDS each wavefront with depth taps finds its levels' sizes for itself (kOwnLevels), which with the order of tasks that
-// launch_fwd_cfg chooses gives, us, 4 x 4000 queries on three levels from 60 x 100, 4 points, around the query: 63 -> 57, 16 channels 38.5 -> 33.7, 20 channels
-// 43 -> 38.6, bfloat16 49 -> 45.7; four levels of 8 points 118 -> 111; 64 channels 82.6 -> 78.6; 6 heads of 20 channels, three levels of 5 points
-// 45.2 -> 43.5.  Plain attention and given scores gain nothing from it (96 -> 100).  Six wavefronts a SIMD (kFwdWaves: 80 registers, which nothing is
-// spilled for) where five were: plain attention, 3 x 3 points 33.5 -> 30.1; one distribution for all heads, packed, four levels of 8 points, around the query 125 ->
-// 118.5, anywhere 150 -> 144, 9000 queries, 116 x 197 326 -> 315; other calls with runs +- 0.5 %.  Seven spill (118.5 -> 141).  (One distribution in bfloat16, packed, four levels of 8 points: 140 -> 141, around the query 116 -> 119.)
+// Six wavefronts a SIMD (kFwdWaves: 80 vector registers, none of which is spilled; of the scalars 64 are with depth taps, 84 with EARLY, to vector lanes) where five were: plain
+// attention, 3 x 3 points 33.5 -> 30.1; one distribution for all heads, packed, four levels of 8 points, around the query 125 -> 118.5, anywhere 150 -> 144,
+// 9000 queries, 116 x 197 326 -> 315; other calls with runs +- 0.5 %.  Seven spill (118.5 -> 141).
 // ---------------------------------------------------------------------------------------
 // wavefronts a SIMD that the registers have to leave room for (1: as the compiler likes)
 template <typename T, int VEC, bool IN_LDS> constexpr int kFwdWaves = !IN_LDS && sizeof(T) == 4 && VEC == 4 ? 6 : 1;
@@ -229,9 +226,8 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC,
   const int to3 = !IN_TURN && spu == 2 ? run + 1 : to1 + to2;
   const int part = row_slot % spu;
 
-  // Depth taps, rows from memory: no level table.  Its barrier held a workgroup's four wavefronts in step, so that they looked for corners and
-  // gathered rows all at once; each now reads the levels' sizes as scalars and goes its own way.
-  constexpr bool kOwnLevels = FUSED && !IN_LDS;
+  // EARLY, depth taps: no level table, each wavefront reads the levels' sizes as scalars (launch_fwd_cfg)
+  constexpr bool kOwnLevels = EARLY && FUSED;
   int cells = 0;
   if constexpr (!kOwnLevels) {
     load_level_table(tab, shapes, shape_stride, level_start, L, S, FUSED ? D : 0);
@@ -677,7 +673,16 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   // 189, 186; 4.4 MB 238, 229 and 269, 271.  16 channels, 4.4 MB 143, 145 and 220, 219; 20 channels, 5.4 MB 189, 202 and 308, 307; 2 points a unit,
   // 2.2 MB 120, 122 and 127, 130.  Early over table first, 32 channels, four sizes of map: 8 to 64
   // points 1.00 - 1.12 (20 points 0.96 - 1.01), bfloat16 0.99 - 1.07 (15 and 20 points 0.95 - 1.02), float64 up to 1.08.
-  const bool early = !fused && a.score_in == nullptr && sizeof(T) == 4 && a.L * a.P == 4 && a.C >= 32 && 2 * map_bytes > (3LL << 20);
+  // Depth taps, each wavefront reading the levels' sizes by scalar loads instead of the table: no faster with a barrier in the table's place and slower with a
+  // table for each wavefront, so it is not the barrier that makes the difference but when the first rows are asked for.  Gains where a packed float32
+  // distribution leaves the value rows of a map above 1.5 MB to the caches.  Table and own sizes, us, around the query and anywhere, 4 levels of 8 points,
+  // 4 x 9000 queries on 116 x 197, 112 bins 300, 284 and 424, 405; 4 x 3906 on 100 x 170 117, 114 and 169, 162; 64 channels 191, 188 and 258, 251;
+  // on 70 x 119 (1.4 MB) 96, 100 and 132, 129; 16 channels 80, 93 and 117, 113; 3 levels of 4 points 119, 122 and 150, 145, 16 channels 95, 113 and
+  // 129, 125.  Bfloat16, packed, 60 x 102, 3 levels of 4 points 62, 69 and 73, 74; 4 levels of 8, 16 channels 80, 96 and 102, 105; 116 x 197 244, 251 and 349,
+  // 351.  A distribution per head, 60 x 102, 4 levels of 8 points 111, 111 and 157, 162 (bfloat16 106, 107 and 160, 167); other shapes 0.98 - 1.06
+  // around the query and 0.99 - 1.02 anywhere, own over table.
+  const bool early = sizeof(T) == 4 && !in_turn && 2 * map_bytes > (3LL << 20) &&
+                     (fused ? a.packed_dist != nullptr : a.score_in == nullptr && a.L * a.P == 4 && a.C >= 32);
   auto launch = [&](auto kernel, int threads, size_t bytes) -> hipError_t {
     if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), bytes)) return e;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), bytes, stream, (const T *)a.value, (const T *)a.dist, a.shapes,
@@ -694,12 +699,14 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
                    : launch(fwd_attention_kernel<T, A, VEC, LPR, false, true, false, false>, kLdsRowsBlock, bytes);
     }
   }
+  if constexpr (std::is_same<T, float>::value) {
+    if (early)
+      return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, false, true>, kBlock, 0)
+                   : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, false, true>, kBlock, 0);
+  }
   if (in_turn)
     return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, true, false>, kBlock, 0)
                  : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, true, false>, kBlock, 0);
-  if constexpr (std::is_same<T, float>::value) {
-    if (early) return launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, false, true>, kBlock, 0);
-  }
   return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, false, false>, kBlock, 0)
                : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, false, false>, kBlock, 0);
 }

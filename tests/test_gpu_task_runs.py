@@ -133,6 +133,33 @@ def test_levels_four_at_a_time(oracle, L, packed):
     torch.testing.assert_close(got.cpu(), want, **F32_FWD)
 
 
+@pytest.mark.parametrize("L", [1, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("map_rows", [95, 97])
+@pytest.mark.parametrize("Q", [37, 1301])
+def test_packed_levels_of_large_maps(oracle, L, map_rows, Q):
+    """A packed float32 distribution on both sides of 1.5 MB of value rows, above which each wavefront reads the levels' sizes itself: as above, and
+    with levels that share keys, whose cells are more than the packed table holds."""
+    from dfa3D import _ext
+    dev = _dev()
+    levels = ((map_rows, 127),) + tuple((3 + l % 4, 2 + l % 3) for l in range(1, L))
+    t = _as_inputs(tiny_case(seed=L, B=2, M=2, C=32, D=5, Q=Q, P=3, levels=levels))
+    value, dist, sh, lsi, loc, attn = (t[k].float() if t[k].is_floating_point() else t[k] for k in
+                                       ("value", "value_dpt_dist", "spatial_shapes", "level_start_index", "sampling_locations", "attention_weights"))
+    dist = dist[:, :, :1].contiguous()
+    both = dist.expand(-1, -1, 2, -1).contiguous()
+    bad, kept = sh.clone(), attn.clone()
+    for l, column, number in ((2, 0, 2 ** 32 + 3), (4, 2, 6), (7, 1, -2), (8, 0, 2 ** 31), (15, 2, 2 ** 32 + 5)):
+        if l < L:
+            bad[l, column] = number
+            kept[:, :, :, l] = 0
+    shared, from_zero = sh[:1].expand(L, -1).contiguous(), torch.zeros_like(lsi)
+    for given, shapes, start, weights in ((bad, sh, lsi, kept), (shared, shared, from_zero, attn)):
+        want, _ = oracle.dfa3d_forward(value, both, shapes, start, loc, weights)
+        on = [x.to(dev) for x in (value, dist, given, start, loc, attn)]
+        got = _ext.dfa3d_fused_forward(*on, 64, need_depth_score=False, packed_dist=_ext.pack_shared_dist(*on[1:4]))[0]
+        torch.testing.assert_close(got.cpu(), want, **F32_FWD)
+
+
 @pytest.mark.parametrize("D", [2, 31, 64, 255, 256, 257, 600])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 def test_packed_table_as_laid_out(D, dtype):
