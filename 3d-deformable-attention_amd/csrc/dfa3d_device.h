@@ -457,8 +457,7 @@ template <> struct BufPair<__hip_bfloat16> {
   // One 8-byte load from the 4-byte boundary at or below the pair: it holds the pair whichever half of its
   // first word the pair starts in.  The load may reach up to four bytes past the buffer's end; the hardware
   // checks the range word by word, so the words inside come back and the one outside reads as zero.  Needs a
-  // buffer whose size is a multiple of 4 bytes (an even number of bins per row), or the last word could be
-  // cut in the middle and dropped.
+  // buffer whose size is a multiple of 4 bytes, or the last word could be cut in the middle and dropped.
   static __device__ __forceinline__ void ld_word_aligned(rsrc_t r, uint32_t off, float &x, float &y) {
     const uint32_t shift = (off & 2u) << 3;              // 0 or 16 bits into the first word
     const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(r, off == kNoRow ? kNoRow : (off & ~3u), 0, 0);
@@ -488,17 +487,20 @@ __device__ __forceinline__ double depth_lerp(double lo, double hi, double hd, do
 // meet after each load, and every corner waits for the one before.
 // LOCAL: the caller's taps mostly hit lines its workgroup has just used (tile kernels)
 template <typename T, bool LOCAL> struct PairLoader {
-  static __device__ __forceinline__ void ld(rsrc_t r, const uint32_t (&off)[4], int, T (&x)[4], T (&y)[4]) {
+  static __device__ __forceinline__ void ld(rsrc_t r, const uint32_t (&off)[4], int, bool, T (&x)[4], T (&y)[4]) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) BufPair<T>::ld(r, off[k], x[k], y[k]);
   }
 };
 template <bool LOCAL> struct PairLoader<__hip_bfloat16, LOCAL> {
-  static __device__ __forceinline__ void ld(rsrc_t r, const uint32_t (&off)[4], int D, float (&x)[4], float (&y)[4]) {
+  // whole_words: the buffer begins and ends on 4-byte boundaries, whatever the number of bins.  Eight 2-byte loads at once spread a point's lines too thin where
+  // caches miss: forward, 4 x 3331 queries, 59 bins, three levels from 37 x 62, 20 channels, anywhere and around the query, corner by corner
+  // 57.6, 45 us, all at once 65, 39, by words 49.4, 38; 4 x 9000 queries, 63 bins, four levels of 8 points from 116 x 197 524, 321; 548, 309; 436, 278.
+  static __device__ __forceinline__ void ld(rsrc_t r, const uint32_t (&off)[4], int D, bool whole_words, float (&x)[4], float (&y)[4]) {
     if (LOCAL && (D & 3) == 0) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) BufPair<__hip_bfloat16>::ld_aligned4(r, off[k], x[k], y[k]);
-    } else if ((D & 1) == 0) {
+    } else if (whole_words) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) BufPair<__hip_bfloat16>::ld_word_aligned(r, off[k], x[k], y[k]);
     } else {
@@ -527,7 +529,7 @@ __device__ __forceinline__ void corner_scores(rsrc_t dist_r, const int (&key)[4]
     for (int k = 0; k < 4; ++k)
       off[k] = key[k] >= 0 && tap.inside ? (uint32_t)(((key[k] * M + m) * D + db) * (int)sizeof(T)) : kNoRow;
     A x[4], y[4];
-    PairLoader<T, LOCAL>::ld(dist_r, off, D, x, y);
+    PairLoader<T, LOCAL>::ld(dist_r, off, D, (D & 1) == 0, x, y);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       lo[k] = lo_x ? x[k] : lo_y ? y[k] : (A)0;
@@ -565,7 +567,7 @@ template <typename A> struct DepthPair {
 // corner_scores() for callers that count in bytes: the distribution of pixel (y, x) lies at base + y * row + x * col
 template <typename T, typename A>
 __device__ __forceinline__ void grid_scores(rsrc_t dist_r, const Grid2D<A> &g, const DepthTap<A> &tap, uint32_t base, uint32_t row, uint32_t col,
-                                            int D, A (&score)[4]) {
+                                            int D, bool whole_words, A (&score)[4]) {
   const uint32_t at = (uint32_t)g.h0 * row + (uint32_t)g.w0 * col + base;
   if (D >= 2) {
     const DepthPair<A> pair(tap, D);
@@ -576,7 +578,7 @@ __device__ __forceinline__ void grid_scores(rsrc_t dist_r, const Grid2D<A> &g, c
       off[k] = g.on(k) && tap.inside ? at_pair + (k >= 2 ? row : 0) + (k == 1 || k == 2 ? col : 0) : kNoRow;
     A x[4], y[4];
     __builtin_amdgcn_sched_barrier(0);                       // the loads one behind the other: corner_scores()
-    PairLoader<T, false>::ld(dist_r, off, D, x, y);
+    PairLoader<T, false>::ld(dist_r, off, D, whole_words, x, y);
 #pragma unroll
     for (int k = 0; k < 4; ++k) score[k] = pair.score(x[k], y[k]);
   } else {

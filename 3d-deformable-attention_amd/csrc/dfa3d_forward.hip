@@ -280,6 +280,7 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC,
   // a map's pixel (y, x) being base + y * row + x * col.  Kept from group to group, like the lane's place.
   struct Level { int H, W, Dd, cell; uint32_t v_col, v_row, v_base, d_row, d_base; bool in_lds; };
   const uint32_t d_col = (uint32_t)(Md * D * (int)sizeof(T));
+  const bool whole_words = (S * Md * D & 1) == 0 && ((uintptr_t)dist & 3) == 0;      // 2-byte elements: what each batch element has of dist
   auto level = [&](const Place &at) {
     const int l = min(at.lp / P, L - 1);
     Level v{};
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC,
 #pragma unroll
               for (int k = 0; k < 4; ++k) sc[k] = pair.score(x4[k], y4[k]);
             } else {
-              grid_scores<T, A>(dist_r, g, tap, lv.d_base, lv.d_row, d_col, D, sc);
+              grid_scores<T, A>(dist_r, g, tap, lv.d_base, lv.d_row, d_col, D, whole_words, sc);
             }
             if (score_out != nullptr && pass == 0) {
               T *so = reinterpret_cast<T *>(reinterpret_cast<char *>(score_out + first_point(q0) * 4) + pl.idx * (uint32_t)(4 * sizeof(T)));

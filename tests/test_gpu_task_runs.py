@@ -53,6 +53,30 @@ def test_bins_that_are_no_taps(oracle, D, extent, dtype):
     torch.testing.assert_close(score.cpu().to(aux), want_score, **tol)
 
 
+@pytest.mark.parametrize("M,levels", [(2, ((5, 6), (3, 3))), (3, ((4, 6), (2, 3))), (1, ((5, 7), (3, 3))), (1, ((5, 7), (2, 3)))])
+@pytest.mark.parametrize("D", [2, 3, 7, 8, 59])
+@pytest.mark.parametrize("first", [0, 1])
+def test_pairs_of_2_byte_bins(oracle, M, levels, D, first):
+    """Batch elements whose distributions begin and end on words and ones that do not, in memory of NaN; half of the points at the ends of the last
+    pixel's distribution."""
+    from dfa3D import _ext
+    dev = _dev()
+    t = _as_inputs(tiny_case(seed=D + M, B=3, M=M, C=8, D=D, Q=64, P=4, levels=levels))
+    value, dist, attn, loc = t["value"].bfloat16(), t["value_dpt_dist"].bfloat16(), t["attention_weights"].float(), t["sampling_locations"].float()
+    for l, (h, w) in enumerate(levels):
+        loc[:, ::2, :, l, :, 0], loc[:, ::2, :, l, :, 1] = (w - 0.4) / w, (h - 0.6) / h
+    loc[:, ::4, ..., 2] = torch.linspace(-0.3, 0.7, 16).view(1, -1, 1, 1, 1) / D
+    loc[:, 2::4, ..., 2] = 1 + torch.linspace(-0.9, 0.3, 16).view(1, -1, 1, 1, 1) / D
+    memory = torch.full((dist.numel() + 16,), float("nan"), dtype=torch.bfloat16, device=dev)
+    given = memory[8 + first:8 + first + dist.numel()].view(dist.shape).copy_(dist)
+    want, want_score = oracle.dfa3d_forward(value.float(), dist.float(), t["spatial_shapes"], t["level_start_index"], loc, attn)
+    got, score = _ext.dfa3d_fused_forward(value.to(dev), given, t["spatial_shapes"].to(dev), t["level_start_index"].to(dev), loc.to(dev), attn.to(dev), 64,
+                                          need_depth_score=True)
+    # one rounding to bfloat16 is 2^-9 of a number; another 2^-9 for float32 sums in another order, which may tip it the other way
+    torch.testing.assert_close(got.cpu().float(), want, rtol=2 ** -8, atol=1e-5)
+    torch.testing.assert_close(score.cpu().float(), want_score, rtol=2 ** -8, atol=1e-5)
+
+
 # value rows of one (batch, head) on both sides of 2 MB, where the order of a unit's tasks changes: 128 and 64 channels, 4096 and 8192 keys
 @pytest.mark.parametrize("C,levels", [(128, ((64, 63), (8, 8))), (128, ((64, 63), (8, 8), (1, 1))), (64, ((91, 90),)), (64, ((91, 90), (2, 2)))])
 @pytest.mark.parametrize("call", ["one stage", "packed", "scores", "plain"])
