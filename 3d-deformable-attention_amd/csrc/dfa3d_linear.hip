@@ -638,15 +638,28 @@ static hipError_t launch_linear_cfg(const float *x, const float *w, const float 
   return hipGetLastError();
 }
 
-// Where linear_rows_kernel takes a product.  A wavefront multiplies by 32 columns and 256 steps whether they are there or not, and a workgroup
-// begins with 5 us of weights: so more than half of the columns, more than three quarters of the depth, and rows that give the CUs
-// about a tile each or one and a half and more.  The others and this one, us (x W^T; g W is the same or better), 256 x 256: 2048 rows 11.4, 13.1;
-// 4096 12.4, 13.5; 6000 14.6, 13.9; 8200 15.6, 18.0; 10500 17.8, 18.0; 12500 20.8, 18.4; 25000 33.2, 27.1; 16500 rows of 256 x 160 24.9, 21.5, 192 x 192
-// 21.6, 21.1, 160 x 256 20.4, 21.8; 27850 of 256 x 128 21.1, 25.1; 40000 of 128 x 256 27.3, 28.5.  (16-byte loads to LDS want their addresses whole.)
-static bool rows_kernel_applies(const float *x, const float *weight, long long N, int cols, int depth) {
+// Where linear_rows_kernel takes a product.  A workgroup multiplies by 256 columns and 256 steps whether they are there or not and begins with 5 us of
+// weights, more where they lie along the depth; the other kernels' tiles end where a multiple of 64 columns does.  So the share of the products that the
+// others would form too, in sixteenths, has to be the larger the fewer row tiles a CU gets and the more blocks of columns there are.  Time over that of the
+// others, 4928 to 185000 rows, depths 196 to 256, 130 to 1024 columns, lowest and highest where this kernel is taken and where not:
+//   row tiles per CU        0.6 - 1                    1.5 - 2                    2 - 4                      4 - 8                      8 and more
+//   256 columns or fewer    x W^T from 15, g W 12      from 14                    from 10                    all                        all
+//     taken, not            0.77 - 1.01, 0.93 - 1.35   0.81 - 0.97, 0.89 - 1.19   0.83 - 1.02, 0.93 - 1.06   0.77 - 0.96                0.67 - 0.88
+//   more                    none                       none                       512 from 14 (more: below)  from 12                    from 9
+//     taken, not                                       0.95 - 1.54                0.87 - 1.05, 0.88 - 1.44   0.80 - 1.06, 0.89 - 1.23   0.72 - 0.93
+// More than 512 columns gain from three tiles per CU on if they are whole blocks (25000 rows, 768 columns 0.88, 1024 0.96; 16500 rows 1.02, 1.08).  In us, the
+// others and this one: 4928 rows of 256 x 256 10.7, 10.8 (x W^T), 13.0, 11.1 (g W); 12500 17.8, 15.2 and 18.5, 15.2; 12500 of 258 columns 22.5, 27.6 and 21.8, 29.5;
+// 25000 of 320 38.7, 42.5; 58000 of 320 77.5, 78.5; 58000 of 512 108, 89; of 128 columns 27850 21.1, 25.1.  (16-byte loads to LDS want their addresses whole.)
+static bool rows_kernel_applies(const float *x, const float *weight, long long N, int cols, int depth, bool across) {
   if (cols <= 128 || depth <= 192 || depth > 256 || (depth & 3) != 0 || (((uintptr_t)x | (uintptr_t)weight) & 15) != 0) return false;
-  const long long tiles = (N + kRowTile - 1) / kRowTile, cus = cu_count();
-  return 2 * tiles >= 3 * cus || (cols <= kRowCols && tiles <= cus && 5 * tiles >= 3 * cus);
+  const long long tiles = (N + kRowTile - 1) / kRowTile, cus = cu_count(), blocks = (cols + kRowCols - 1) / kRowCols;
+  const long long sixteenth = blocks * kRowCols * 256 / 16, share = (cols + 63) / 64 * 64 * (long long)depth;
+  if (tiles >= 8 * cus) return share >= 9 * sixteenth;
+  if (tiles >= 4 * cus) return blocks == 1 || share >= 12 * sixteenth;
+  if (tiles >= 2 * cus) return share >= (blocks == 1 ? 10 : blocks == 2 ? 14 : 16) * sixteenth && (blocks <= 2 || tiles >= 3 * cus);
+  if (blocks > 1) return false;
+  if (2 * tiles >= 3 * cus) return share >= 14 * sixteenth;
+  return tiles <= cus && 5 * tiles >= 3 * cus && share >= (across ? 12 : 15) * sixteenth;
 }
 template <int KS, bool ACROSS>
 static hipError_t launch_linear_rows(const float *x, const float *w, const float *bias, float *y, long long N, int cols, int depth, hipStream_t stream) {
@@ -660,7 +673,7 @@ static hipError_t launch_linear_rows(const float *x, const float *w, const float
 }
 
 hipError_t launch_linear(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream) {
-  if (rows_kernel_applies(x, w, N, O, K)) return launch_linear_rows<16, false>(x, w, bias, y, N, O, K, stream);
+  if (rows_kernel_applies(x, w, N, O, K, false)) return launch_linear_rows<16, false>(x, w, bias, y, N, O, K, stream);
   return wide_tiles(N, O) ? launch_linear_cfg<64, 128>(x, w, bias, y, N, O, K, stream) : launch_linear_cfg<64, 64>(x, w, bias, y, N, O, K, stream);
 }
 
@@ -674,7 +687,7 @@ template <int TM, int TN, int FLUSH> static hipError_t launch_linear_sum_cfg(con
 
 hipError_t launch_linear_sum(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream) {
   const LinearSet &s = sets.set[0];
-  if (sets.n == 1 && rows_kernel_applies(s.rows, s.weight, N, K, s.width)) return launch_linear_rows<16, true>(s.rows, s.weight, nullptr, y, N, K, s.width, stream);
+  if (sets.n == 1 && rows_kernel_applies(s.rows, s.weight, N, K, s.width, true)) return launch_linear_rows<16, true>(s.rows, s.weight, nullptr, y, N, K, s.width, stream);
   const bool wide = wide_tiles(N, K);
   if (sets.n == 1) return wide ? launch_linear_sum_cfg<64, 128, 0>(sets, y, N, K, stream) : launch_linear_sum_cfg<64, 64, 0>(sets, y, N, K, stream);
   return wide ? launch_linear_sum_cfg<64, 128, 128>(sets, y, N, K, stream) : launch_linear_sum_cfg<64, 64, 128>(sets, y, N, K, stream);

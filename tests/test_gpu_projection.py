@@ -70,7 +70,10 @@ def test_operands_that_are_no_ordinary_numbers():
     torch.testing.assert_close(gw, g.t().mm(x), rtol=1e-4, atol=1e-2, equal_nan=True)
 
 
-@pytest.mark.parametrize("N,K,O", [(4928, 256, 130), (8192, 256, 256), (12289, 196, 256), (12320, 252, 258), (24607, 256, 512), (50000, 256, 160)])
+# on both sides of the lines that the launcher draws: one tile of 32 rows per workgroup, two, three, five and nine, of one block of 256 columns, two and three
+@pytest.mark.parametrize("N,K,O", [(4928, 256, 130), (8192, 256, 256), (12289, 196, 256), (12320, 252, 258), (24607, 256, 512), (50000, 256, 160),
+                                   (5001, 252, 250), (12300, 228, 254), (16411, 196, 200), (16500, 228, 506), (25003, 256, 642), (25003, 252, 706), (32801, 200, 130),
+                                   (33000, 256, 386), (33000, 196, 450), (65600, 196, 196), (65600, 212, 324), (65600, 200, 258)])
 @pytest.mark.parametrize("across", [False, True])
 def test_product_with_the_weight_in_registers(N, K, O, across):
     """Row tiles that end early, one tile per workgroup and several, depths and widths that are no whole steps or columns of a wavefront; rows with
@@ -113,6 +116,48 @@ def test_product_with_the_weight_in_registers_and_more_odd_tiles_than_bits():
     for rows in (slice(0, 5), slice(6, 64), slice(first, first + 64), slice(N - 64, N)):
         want = x[rows].double() @ wt.double()
         assert ((got[rows].double() - want).abs() <= 100 * 2.0 ** -23 * (x[rows].double().abs() @ wt.double().abs())).all()
+
+
+@pytest.mark.parametrize("tiny,huge", [(-122, 100), (-140, 100), (-112, 33), (-109, 25)])
+@pytest.mark.parametrize("across", [False, True])
+def test_tiny_operands_with_large_partners_and_the_weight_in_registers(tiny, huge, across):
+    """As test_tiny_operands_with_large_partners, with five tiles per workgroup: large weights in some columns of one wavefront; large rows in one tile
+    each of five workgroups, the first, the second ... that it takes."""
+    from dfa3D.modules import projection
+    dev = torch.device("cuda:0")
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    N, K, O = 32 * cus * 5 - 7, 256, 250
+    g = torch.Generator(device=dev).manual_seed(-tiny)
+    product = lambda x, w: projection._sum_of_products((x, w.t().contiguous())) if across else projection._product(x, w, None)
+
+    def close(got, want):
+        return (got.double() - want).norm() <= 1e-6 * want.norm()                   # as for ordinary operands
+    x, w = torch.randn(N, K, generator=g, device=dev) * 2.0 ** tiny, torch.randn(O, K, generator=g, device=dev)
+    columns = torch.arange(40, 50, device=dev)
+    w[columns] *= 2.0 ** huge
+    assert close(product(x, w)[:, columns], x.double() @ w[columns].double().t())
+    x, w = torch.randn(N, K, generator=g, device=dev), torch.randn(O, K, generator=g, device=dev) * 2.0 ** tiny
+    large = torch.cat([32 * (i * cus + 3 * i + 1) + torch.arange(5, device=dev) for i in range(5)])
+    x[large] *= 2.0 ** huge
+    got, want = product(x, w)[large], x[large].double() @ w.double().t()
+    for i in range(5):
+        assert close(got[5 * i:5 * i + 5], want[5 * i:5 * i + 5]), i
+
+
+@pytest.mark.parametrize("N,K,O", [(8192, 256, 256), (16500, 256, 512), (50001, 200, 250)])
+@pytest.mark.parametrize("across", [False, True])
+def test_kernels_agree_to_the_bit(N, K, O, across):
+    """The same products and sums in the same order, whichever kernel a call's size takes: rows by themselves, in calls too small for the weight in registers."""
+    from dfa3D.modules import projection
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(N + O)
+    x, w, b = (torch.randn(*s, generator=g, device=dev) for s in ((N, K), (O, K), (O,)))
+    wt = w.t().contiguous()
+    product = lambda rows: projection._sum_of_products((rows, wt)) if across else projection._product(rows, w, b)
+    got = product(x)
+    for first in (0, 33, N - 4100):
+        some = x[first:first + 4100].contiguous()
+        assert torch.equal(product(some), got[first:first + 4100])
 
 
 def _error(got, want):
