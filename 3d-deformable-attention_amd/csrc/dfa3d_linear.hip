@@ -39,25 +39,28 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int kStep = 16;              // contraction steps staged at once: of one matrix instruction
 
 // x = p1 + p2 + p3, each rounded to nearest: 24 bits and more, so nothing of a float32 of 2^-108 or more is lost, and of a smaller one
-// 2^-133 at most (odd_sums).  p: two numbers to a word.  `most`: the largest size that came by.
-template <int N> __device__ __forceinline__ void split_parts(const float (&v)[N], uint32_t (&p)[3][N / 2], float &most) {
+// 2^-133 at most (odd_sums).  put(i, p): the numbers' parts i, two to a word, before the next ones are formed.  `most`: the largest size that came by.
+template <int N, typename Put> __device__ __forceinline__ void split_parts(const float (&v)[N], float &most, const Put &put) {
   float rest[N];
 #pragma unroll
   for (int j = 0; j < N; ++j) rest[j] = v[j];
 #pragma unroll
   for (int j = 0; j < N; j += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(rest[j]), "v"(rest[j + 1]));
 #pragma unroll
-  for (int plane = 0; plane < 3; ++plane)
+  for (int plane = 0; plane < 3; ++plane) {
+    uint32_t p[N / 2];
 #pragma unroll
     for (int j = 0; j < N / 2; ++j) {
       uint32_t two = pack_bf16x2(rest[2 * j], rest[2 * j + 1]);
       asm("" : "+v"(two));                                     // (or each half is rounded once more for its difference)
-      p[plane][j] = two;
+      p[j] = two;
       if (plane < 2) {
         rest[2 * j] -= __uint_as_float(two << 16);
         rest[2 * j + 1] -= __uint_as_float(two & 0xFFFF0000u);
       }
     }
+    put(plane, p);
+  }
 }
 // the six products of parts, smallest first: part of the one operand, part of the other
 constexpr int kProducts[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
@@ -98,15 +101,12 @@ template <int R, bool ACROSS> struct SplitOperand {
       const int idx = (int)threadIdx.x + 256 * u;
       if (2 * R % 256 != 0 && ACROSS && idx >= 2 * R) break;
       unsigned char *at = lds + (ACROSS ? idx / R * kPiece + idx % R * 16 : idx % 4 / 2 * kPiece + idx / 4 * 16 + idx % 2 * 8);
-      uint32_t parts[3][kRun / 2];
-      split_parts(v[u], parts, most);
+      split_parts(v[u], most, [&](int plane, const uint32_t (&p)[kRun / 2]) {
+        words w;
 #pragma unroll
-      for (int plane = 0; plane < 3; ++plane) {
-        words p;
-#pragma unroll
-        for (int j = 0; j < kRun / 2; ++j) p[j] = parts[plane][j];
-        *reinterpret_cast<words *>(at + plane * kPlane) = p;
-      }
+        for (int j = 0; j < kRun / 2; ++j) w[j] = p[j];
+        *reinterpret_cast<words *>(at + plane * kPlane) = w;
+      });
     }
   }
   // this lane's part of a matrix instruction's operand
@@ -363,11 +363,9 @@ template <int KS> struct RowTile {
     const int idx = (int)threadIdx.x + kRowThreads * u, row = idx / kQuads, quad = idx % kQuads;
     const float4 t = *reinterpret_cast<const float4 *>(raw + idx * 16);
     const float v[4] = {t.x, t.y, t.z, t.w};
-    uint32_t p[3][2];
-    split_parts(v, p, most);
-#pragma unroll
-    for (int plane = 0; plane < 3; ++plane)
-      *reinterpret_cast<uint2 *>(parts + plane * kPlane + quad / 2 * kPiece + row * 16 + quad % 2 * 8) = make_uint2(p[plane][0], p[plane][1]);
+    split_parts(v, most, [&](int plane, const uint32_t (&p)[2]) {
+      *reinterpret_cast<uint2 *>(parts + plane * kPlane + quad / 2 * kPiece + row * 16 + quad % 2 * 8) = make_uint2(p[0], p[1]);
+    });
   }
   static __device__ __forceinline__ bf16x8 part(const unsigned char *parts, int plane, int step, int half, int row) {
     return *reinterpret_cast<const bf16x8 *>(parts + plane * kPlane + (2 * step + half) * kPiece + row * 16);
@@ -381,13 +379,10 @@ __device__ __forceinline__ void wave_lds_read() { asm volatile("s_waitcnt lgkmcn
 // The parts of a wavefront's 32 columns of a weight, eight contraction steps of one column to a lane and step.
 template <int KS> using ColumnParts = bf16x8[KS][3];
 __device__ __forceinline__ void column_parts(const float (&v)[8], bf16x8 (&parts)[3], float &most) {
-  uint32_t p[3][4];
-  split_parts(v, p, most);
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const u32x4 words = {p[i][0], p[i][1], p[i][2], p[i][3]};
+  split_parts(v, most, [&](int i, const uint32_t (&p)[4]) {
+    const u32x4 words = {p[0], p[1], p[2], p[3]};
     parts[i] = __builtin_bit_cast(bf16x8, words);
-  }
+  });
 }
 // Element (column, k) lies at k * ld + column: 32 lanes take a whole line at a time.
 template <int KS> __device__ __forceinline__ void load_columns_across(rsrc_t r, int ld, int col, int cols, ColumnParts<KS> &parts, float &most) {
