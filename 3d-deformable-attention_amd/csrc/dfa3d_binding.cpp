@@ -11,6 +11,7 @@
 #include <ATen/autocast_mode.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <ATen/record_function.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -429,6 +430,9 @@ PyObject *linear_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 // tensor and nothing of torch's: another torch's module says so before anything of it runs.
 PyObject *built_for(PyObject *, PyObject *) { return Py_BuildValue("(si)", DFA3D_BUILT_FOR, DFA3D_ABI_VERSION); }
 
+// observed() -> whether a profiler or another observer is told of calls on this thread
+PyObject *observed(PyObject *, PyObject *) { return PyBool_FromLong(at::hasCallbacks()); }
+
 // bind(dict of entry point -> address)
 PyObject *bind(PyObject *, PyObject *table) {
   auto address = [&](const char *name, auto &to) {
@@ -462,6 +466,7 @@ PyCFunction as_method(Fast f) { return reinterpret_cast<PyCFunction>(reinterpret
 PyMethodDef methods[] = {
     {"built_for", built_for, METH_NOARGS, nullptr},
     {"bind", bind, METH_O, nullptr},
+    {"observed", observed, METH_NOARGS, nullptr},
     {"fused_forward", as_method(fused_forward), METH_FASTCALL, nullptr},
     {"fused_gradients", as_method(fused_gradients), METH_FASTCALL, nullptr},
     {"attention_forward", as_method(attention_forward), METH_FASTCALL, nullptr},

@@ -3,6 +3,8 @@ import torch
 from torch import _functorch
 from torch.autograd.function import Function
 
+from . import _lib
+
 __all__ = ["OperatorFunction"]
 
 
@@ -20,9 +22,10 @@ class _Notes:
 
 class OperatorFunction(Function):
     """A Function whose ``apply`` is its ``forward`` where gradients are off: making a node and wrapping what comes back is 4 of
-    the 12 us that a forward of 2 x 100 queries takes.  Tracing, compilation, functorch transforms and forward mode,
-    which see a call or refuse it, have the node made all the same, as do subclasses from elsewhere: a class says with
-    ``own = True`` in its own body that its ``forward`` asks no more of its context than ``_Notes`` has."""
+    the 12 us that a forward of 2 x 100 queries takes.  Tracing, compilation, functorch transforms, forward mode, and profilers and
+    other observers, which see a call or refuse it, have the node made all the same, as do subclasses from elsewhere (and all calls where there is no
+    binding module to say who observes).  A class says with ``own = True`` in its own body that its ``forward`` asks no more of its context than ``_Notes``
+    has and returns none of its operands: ``Function`` hands out another tensor where a forward does, this the operand itself."""
 
     own = False
 
@@ -30,6 +33,6 @@ class OperatorFunction(Function):
     def apply(cls, *args, **kwargs):
         if (torch.compiler.is_compiling() or torch.is_grad_enabled() or kwargs or not cls.__dict__.get("own", False)
                 or torch._C._get_tracing_state() is not None or torch._C._are_functorch_transforms_active()
-                or torch.autograd.forward_ad._current_level >= 0):
+                or torch.autograd.forward_ad._current_level >= 0 or (native := _lib.binding()) is None or native.observed()):
             return super().apply(*args, **kwargs)
         return cls.forward(_Notes(), *_functorch.utils.unwrap_dead_wrappers(args))

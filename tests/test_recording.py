@@ -92,6 +92,34 @@ def test_a_wrapper_left_over_from_a_transform_is_unwrapped():
     assert outs[0] == outs[1]
 
 
+def test_a_profiler_sees_the_call(tmp_path):
+    x = torch.randn(4)
+    observer = torch.profiler.ExecutionTraceObserver().register_callback(str(tmp_path / "calls.json"))
+    for mode in (torch.no_grad, torch.inference_mode):
+        with mode():
+            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as seen:
+                short = _took_the_short_way(lambda: Own.apply(x, 3))[1]
+            assert not short and "Own" in [e.key for e in seen.key_averages()]
+            observer.start()
+            try:
+                short = _took_the_short_way(lambda: Own.apply(x, 3))[1]
+            finally:
+                observer.stop()
+            assert not short
+            assert _took_the_short_way(lambda: Own.apply(x, 3))[1]
+    observer.unregister_callback()
+    assert '"Own"' in (tmp_path / "calls.json").read_text()
+
+
+def test_without_a_binding_module_a_node_is_made(monkeypatch):
+    from dfa3D import _lib
+    _lib.lib()
+    monkeypatch.setattr(_lib, "_binding", None)
+    with torch.no_grad():
+        out, short = _took_the_short_way(lambda: Own.apply(torch.ones(2), 3))
+    assert not short and torch.equal(out[0], torch.full((2,), 3.0))
+
+
 def test_threads_do_not_share_a_context():
     results = [None] * 8
 
