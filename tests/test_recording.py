@@ -81,15 +81,30 @@ def test_tracing_forward_mode_and_transforms_see_the_call():
 
 def test_a_wrapper_left_over_from_a_transform_is_unwrapped():
     left = []
-    torch.func.vmap(lambda t: (left.append(t), t)[1])(torch.ones(3, 2))
-    outs = []
-    for F in (Plain, Own):
+    torch.func.grad(lambda t: (left.append(t), t.sum())[1])(torch.ones(3))
+    assert torch._C._functorch.is_functorch_wrapped_tensor(left[0])
+    wrapped = []
+
+    def forward(ctx, x):
+        wrapped.append(torch._C._functorch.is_functorch_wrapped_tensor(x))
+        return x * 3
+    for base in (Function, OperatorFunction):
+        F = type("F", (base,), {"own": True, "forward": staticmethod(forward)})
         with torch.no_grad():
-            try:
-                outs.append(torch.equal(F.apply(left[0], 3)[0], F.apply(left[0], 3)[0]))
-            except RuntimeError as e:
-                outs.append(type(e))
-    assert outs[0] == outs[1]
+            out = F.apply(left[0])
+        assert torch.equal(out, torch.full((3,), 3.0)) and not torch._C._functorch.is_functorch_wrapped_tensor(out)
+    assert wrapped == [False, False]
+
+
+def test_export_sees_the_call():
+    """Export without Dynamo runs ``apply`` itself, on tensors that hold nothing."""
+    class M(torch.nn.Module):
+        def forward(self, t):
+            return Own.apply(t, 3)[0]
+    x = torch.randn(4)
+    with torch.no_grad():
+        program, short = _took_the_short_way(lambda: torch.export.export(M(), (x,), strict=False))
+        assert not short and torch.equal(program.module()(x), x * 3)
 
 
 def test_a_profiler_sees_the_call(tmp_path):
