@@ -77,14 +77,10 @@ def test_pairs_of_2_byte_bins(oracle, M, levels, D, first):
     torch.testing.assert_close(score.cpu().float(), want_score, rtol=2 ** -8, atol=1e-5)
 
 
-# value rows of one (batch, head) on both sides of 2 MB, where the order of a unit's tasks changes: 128 and 64 channels, 4096 and 8192 keys
-@pytest.mark.parametrize("C,levels", [(128, ((64, 63), (8, 8))), (128, ((64, 63), (8, 8), (1, 1))), (64, ((91, 90),)), (64, ((91, 90), (2, 2)))])
-@pytest.mark.parametrize("call", ["one stage", "packed", "scores", "plain"])
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-def test_order_of_tasks(oracle, C, levels, call, dtype):
+def _forward_against_oracle(oracle, C, levels, call, dtype, Q, P, B=1):
     from dfa3D import _ext
     dev = _dev()
-    t = _as_inputs(tiny_case(seed=C + len(levels), B=1, M=2, C=C, D=4, Q=1301, P=7, levels=levels))
+    t = _as_inputs(tiny_case(seed=C + len(levels), B=B, M=2, C=C, D=4, Q=Q, P=P, levels=levels))
     value, dist = (t[k].to(dtype) for k in ("value", "value_dpt_dist"))
     sh, lsi, loc, attn = t["spatial_shapes"], t["level_start_index"], t["sampling_locations"].float(), t["attention_weights"].float()
     if call == "packed":
@@ -108,6 +104,33 @@ def test_order_of_tasks(oracle, C, levels, call, dtype):
     # bfloat16: the output's own rounding, and that of the scores that are handed over
     tol = F32_FWD if dtype == torch.float32 else dict(rtol=2 ** -7, atol=2 ** -7)
     torch.testing.assert_close(got.float().cpu(), want, **tol)
+
+
+# value rows of one (batch, head) on both sides of 2 MB, where the order of a unit's tasks changes: 128 and 64 channels, 4096 and 8192 keys
+@pytest.mark.parametrize("C,levels", [(128, ((64, 63), (8, 8))), (128, ((64, 63), (8, 8), (1, 1))), (64, ((91, 90),)), (64, ((91, 90), (2, 2)))])
+@pytest.mark.parametrize("call", ["one stage", "packed", "scores", "plain"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_order_of_tasks(oracle, C, levels, call, dtype):
+    _forward_against_oracle(oracle, C, levels, call, dtype, 1301, 7)
+
+
+# the same with several slots a unit on both sides: one unit of 128 channels a wavefront, two of 64, and bfloat16 rows of half the bytes
+@pytest.mark.parametrize("dtype,C,Q,levels", [(torch.float32, 128, 400, ((64, 64),)), (torch.float32, 128, 400, ((64, 64), (1, 1))),
+                                              (torch.bfloat16, 128, 400, ((91, 90), (1, 2))), (torch.bfloat16, 128, 400, ((91, 90), (3, 1))),
+                                              (torch.bfloat16, 64, 1301, ((128, 128),)), (torch.bfloat16, 64, 1301, ((128, 128), (1, 1)))])
+@pytest.mark.parametrize("call", ["one stage", "packed", "scores", "plain"])
+def test_order_of_tasks_where_units_have_several_slots(oracle, dtype, C, Q, levels, call):
+    _forward_against_oracle(oracle, C, levels, call, dtype, Q, 7)
+
+
+# runs from memory: above 2 MB, so that 2, 4, 8 and 16 slots share a unit, with the shapes of test_unequal_runs
+@pytest.mark.parametrize("L,P,C,Q", [(3, 7, 32, 1031), (3, 7, 16, 1031), (1, 9, 32, 2051), (1, 17, 64, 1025), (1, 19, 128, 1027), (1, 13, 20, 1367),
+                                     (4, 11, 32, 519), (1, 65, 32, 130)])
+@pytest.mark.parametrize("call", ["one stage", "packed", "scores", "plain"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_unequal_runs_of_large_maps(oracle, L, P, C, Q, call, dtype):
+    rows = (2 << 20) // (C * (4 if dtype == torch.float32 else 2)) + 1
+    _forward_against_oracle(oracle, C, (((rows + 126) // 127, 127),) + LEVELS[1:L], call, dtype, Q, P, B=2)
 
 
 # value rows of one (batch, head) on both sides of 1.5 MB, above which units of four points have their first operands asked for before the level table:
@@ -135,7 +158,7 @@ def test_units_of_four_points(oracle, C, levels, P, Q, scores):
 @pytest.mark.parametrize("L", [1, 3, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("packed", [False, True])
 def test_levels_four_at_a_time(oracle, L, packed):
-    """Levels' sizes, four read at a time; one that does not fit the keys or bins adds nothing, as with weights of zero."""
+    """Tables of one to sixteen levels; a level that does not fit the keys or bins adds nothing, as with weights of zero."""
     from dfa3D import _ext
     dev = _dev()
     t = _as_inputs(tiny_case(seed=L, B=2, M=2, C=16, D=5, Q=37, P=3, levels=tuple((3 + l % 4, 2 + l % 3) for l in range(L))))
