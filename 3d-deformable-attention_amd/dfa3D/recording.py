@@ -31,7 +31,8 @@ class OperatorFunction(Function):
 
     @classmethod
     def apply(cls, *args, **kwargs):
-        if (torch.compiler.is_compiling() or torch.is_grad_enabled() or kwargs or not cls.__dict__.get("own", False)
+        # gradients first: a training step's calls are not to pay for the other questions (1.5 us of 27 a forward, of which 0.5 is left)
+        if (torch.is_grad_enabled() or torch.compiler.is_compiling() or kwargs or not cls.__dict__.get("own", False)
                 or torch._C._get_tracing_state() is not None or torch._C._are_functorch_transforms_active()
                 or torch.autograd.forward_ad._current_level >= 0 or (native := _lib.binding()) is None or native.observed()):
             return super().apply(*args, **kwargs)

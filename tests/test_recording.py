@@ -135,6 +135,15 @@ def test_without_a_binding_module_a_node_is_made(monkeypatch):
     assert not short and torch.equal(out[0], torch.full((2,), 3.0))
 
 
+def test_with_gradients_nothing_else_is_asked(monkeypatch):
+    """What a call that is recorded pays for the choice is the one question whether it is."""
+    def asked():
+        raise AssertionError("asked")
+    monkeypatch.setattr(torch.compiler, "is_compiling", asked)
+    x = torch.randn(4, requires_grad=True)
+    assert Own.apply(x, 3)[0].requires_grad
+
+
 def test_threads_do_not_share_a_context():
     results = [None] * 8
 
