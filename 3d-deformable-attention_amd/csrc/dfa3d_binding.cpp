@@ -17,6 +17,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <initializer_list>
 #include <limits>
@@ -430,8 +431,12 @@ PyObject *linear_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 // tensor and nothing of torch's: another torch's module says so before anything of it runs.
 PyObject *built_for(PyObject *, PyObject *) { return Py_BuildValue("(si)", DFA3D_BUILT_FOR, DFA3D_ABI_VERSION); }
 
-// observed() -> whether a profiler or another observer is told of calls on this thread
-PyObject *observed(PyObject *, PyObject *) { return PyBool_FromLong(at::hasCallbacks()); }
+// seen() -> whether a tracer, a functorch transform, a profiler or another observer sees what this thread calls
+PyObject *seen(PyObject *, PyObject *) {
+  const c10::DispatchKeySet modes = c10::impl::tls_local_dispatch_key_set().included_;
+  return PyBool_FromLong(at::hasCallbacks() || torch::jit::tracer::isTracing() || modes.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+                         modes.has(c10::DispatchKey::FuncTorchDynamicLayerBackMode));
+}
 
 // bind(dict of entry point -> address)
 PyObject *bind(PyObject *, PyObject *table) {
@@ -466,7 +471,7 @@ PyCFunction as_method(Fast f) { return reinterpret_cast<PyCFunction>(reinterpret
 PyMethodDef methods[] = {
     {"built_for", built_for, METH_NOARGS, nullptr},
     {"bind", bind, METH_O, nullptr},
-    {"observed", observed, METH_NOARGS, nullptr},
+    {"seen", seen, METH_NOARGS, nullptr},
     {"fused_forward", as_method(fused_forward), METH_FASTCALL, nullptr},
     {"fused_gradients", as_method(fused_gradients), METH_FASTCALL, nullptr},
     {"attention_forward", as_method(attention_forward), METH_FASTCALL, nullptr},

@@ -88,7 +88,7 @@ def _load_binding(handle):
     for another torch, whose tensors it would misread, or for another version of the library's interface."""
     try:
         module = importlib.import_module(__package__ + "._binding")
-        built_for, abi, _ = *module.built_for(), module.observed
+        built_for, abi, _ = *module.built_for(), module.seen
         here = f"{torch.__version__} {torch.version.git_version}"
         if built_for != here or abi != ABI_VERSION:
             raise ImportError(f"it was built for torch {built_for} and ABI version {abi}, this is {here} and {ABI_VERSION}")

@@ -24,7 +24,7 @@ class OperatorFunction(Function):
     """A Function whose ``apply`` is its ``forward`` where gradients are off: making a node and wrapping what comes back is 4 of
     the 12 us that a forward of 2 x 100 queries takes.  Tracing, compilation, functorch transforms, forward mode, and profilers and
     other observers, which see a call or refuse it, have the node made all the same, as do subclasses from elsewhere (and all calls where there is no
-    binding module to say who observes).  A class says with ``own = True`` in its own body that its ``forward`` asks no more of its context than ``_Notes``
+    binding module to say who sees them; asked one by one from here they are 0.2 us of 9).  A class says with ``own = True`` in its own body that its ``forward`` asks no more of its context than ``_Notes``
     has and returns none of its operands: ``Function`` hands out another tensor where a forward does, this the operand itself."""
 
     own = False
@@ -33,7 +33,6 @@ class OperatorFunction(Function):
     def apply(cls, *args, **kwargs):
         # gradients first: a training step's calls are not to pay for the other questions (1.5 us of 27 a forward, of which 0.5 is left)
         if (torch.is_grad_enabled() or torch.compiler.is_compiling() or kwargs or not cls.__dict__.get("own", False)
-                or torch._C._get_tracing_state() is not None or torch._C._are_functorch_transforms_active()
-                or torch.autograd.forward_ad._current_level >= 0 or (native := _lib.binding()) is None or native.observed()):
+                or torch.autograd.forward_ad._current_level >= 0 or (native := _lib.binding()) is None or native.seen()):
             return super().apply(*args, **kwargs)
         return cls.forward(_Notes(), *_functorch.utils.unwrap_dead_wrappers(args))
