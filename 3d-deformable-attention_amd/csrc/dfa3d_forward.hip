@@ -140,8 +140,8 @@ template <int FROM, int VEC> __device__ __forceinline__ void sum_over_slots(int 
 // that begins a group (s_setprio 2, 1, 0; the other way round 3120 us for the 3047 of two steps and 3000 of three, 24 planes and 128 bins).  Together, one card, us:
 //   6 x 10000 queries, 4 levels from 116 x 200, 8 points: 885 -> 872, around the query 574 -> 571 (bfloat16 483 -> 476), plain attention 436 -> 389;
 //   6 x 40000 clustered, 128 bins: 3067 -> 3000; the two separate stages without gradients, 112 bins: 1013 -> 936; one level of 23 x 40: 39.7 -> 38.0;
-// Where a workgroup has one group (not IN_LDS) these priorities took more than they gave for rows that the L2 holds (plain attention, 4 x 10000
-// queries of 4 points on 116 x 197: 59.5 -> 63.7) and gave where it does not (2 x 40000 on 200 x 200, around the query 103 -> 96, anywhere 65 -> 69): none.
+// Where a workgroup has one group (not IN_LDS) there are none: plain attention, 4 points, 2 x 40000 queries on 200 x 200 gained from them (103 -> 96),
+// 4 x 10000 on 116 x 197 lost (59.5 -> 63.7).
 //
 // Six wavefronts a SIMD (kFwdWaves: 80 vector registers, none of which is spilled; of the scalars 64 are with depth taps, 84 with EARLY, to vector lanes) where five were: plain
 // attention, 3 x 3 points 33.5 -> 30.1; one distribution for all heads, packed, four levels of 8 points, around the query 125 -> 118.5, anywhere 150 -> 144,

@@ -339,12 +339,13 @@ __global__ __launch_bounds__(256, 3) void linear_sum_kernel(LinearSets sets, flo
 }
 
 // y (N, cols) = x (N, depth) times the weight of one layer, whose parts for 32 columns and all of the depth (up to KS * 16 steps) a wavefront keeps in
-// registers: 192 of its 256.  A workgroup (8 wavefronts, one per CU) splits its 256 columns once and walks through tiles of 32 rows; what is left of a
-// tile is its rows: straight to LDS two tiles ahead (a thread's own 16 bytes each, so no register holds them and no barrier is needed), split once,
-// read by all eight.  Power bounds it: 32x32x16 products of random numbers alone run at 1.8 of 2.4 GHz, so every split, access to LDS and load that is
-// left out counts, not only those that something waits for.  Same products and sums in the same order as by linear_kernel and linear_sum_kernel, to
-// the bit.  With those, and with this one, us, new operands each time: 184950 rows of 256 x 256 200, 151 (x W^T), 178, 130 (g W); 49536 60, 44 and 58,
-// 43; 40000 47, 33 and 45, 33; 22500 28, 22 and 27, 23; 58000 of 256 x 512 117, 92.
+// registers: 192 of its 256 (the others are taken too; one or two are spilled, outside of the loop).  A workgroup (8 wavefronts, one per CU) splits
+// its 256 columns once and walks through tiles of 32 rows; what is left of a tile is its rows: straight to LDS two tiles ahead (a thread's own 16
+// bytes each, so no register holds them and no barrier is needed), split once, read by all eight.  Power bounds it: 32x32x16 products of random
+// numbers alone run at 1.8 of 2.4 GHz, so every split, access to LDS and load that is left out counts, not only those that something waits for.  Same
+// products and sums in the same order as by linear_kernel and linear_sum_kernel, to the bit but where odd sums are formed again (here for 32 rows and
+// columns at a time, there for a wavefront's part of a tile).  With those, and with this one, us, new operands each time: 184950 rows of 256 x 256
+// 200, 151 (x W^T), 178, 130 (g W); 49536 60, 44 and 58, 43; 40000 47, 33 and 45, 33; 22500 28, 22 and 27, 23; 58000 of 256 x 512 117, 92.
 constexpr int kRowTile = 32, kRowThreads = 512, kRowCols = 256;
 constexpr int kOddTiles = 256;         // a wavefront's tiles with odd sums, a bit each; of more tiles, several share one
 template <int KS> struct RowTile {

@@ -100,13 +100,18 @@ WORKLOADS = {
     "base_fine": Workload("base_fine", B=6, Q=10000, levels=_BASE_LEVELS[:1], D=64, P=8, depth_sigma=2.0),
     "base_fine_band": Workload("base_fine_band", B=6, Q=10000, levels=_BASE_LEVELS[:1], D=64, P=8, depth_sigma=2.0,
                                loc="band"),
+    # sizes that are no multiple of anything, some locations out of bounds
+    "ragged": Workload("ragged", B=3, Q=3331, levels=((37, 67), (19, 34), (10, 17)), D=59, P=5, M=6, C=20,
+                       loc_lo=-0.05, loc_hi=1.05, depth_sigma=2.0),
+    # self-attention over the 200 x 200 BEV map of two frames, no depth
+    "bev_self": Workload("bev_self", B=2, Q=40000, levels=((200, 200),), D=1, P=4, loc="coherent", loc_std=0.02),
     # dense BEV grid, clustered locations
     "dense": Workload("dense", B=6, Q=40000, levels=_BASE_LEVELS, D=128, P=8, loc="normal",
                       loc_lo=-0.1, loc_hi=1.1, depth_sigma=2.0),
 }
 
 SEEDS = {"unit": 1, "small": 2, "base": 3, "base_peaky": 4, "dense": 5, "unittest": 6, "base_coherent": 7,
-         "base_coarse": 3, "base_band": 3, "base_fine": 3, "base_fine_band": 3}
+         "base_coarse": 3, "base_band": 3, "base_fine": 3, "base_fine_band": 3, "ragged": 8, "bev_self": 9}
 
 
 def scaled(w: Workload, B=None, Q=None, name=None) -> Workload:

@@ -570,11 +570,20 @@ def phase_costs(a):
     mid.record()
     torch.cuda.synchronize()
     opts = ctypes.pointer(_lib.LaunchOptions(event_binned=mid.cuda_event, **fields))
-    nbytes = shipped.dfa3d_fused_backward_workspace_bytes(B, S, M, C, D, L, Q, P, M, code, opts)
+    plain = D == 1                               # plain attention: no depth taps
+    nbytes = (shipped.dfa3d_wms_deform_attn_backward_workspace_bytes(B, S, M, C, L, Q, P, code, opts) if plain else
+              shipped.dfa3d_fused_backward_workspace_bytes(B, S, M, C, D, L, Q, P, M, code, opts))
     assert nbytes > 0, "the binned backward does not take this workload"
     ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
 
+    xy, gxy, shapes2 = loc[..., :2].contiguous(), torch.empty_like(loc[..., :2].contiguous()), shapes[:, :2].contiguous()
+
     def call(library):
+        if plain:
+            return _lib.check(library.dfa3d_wms_deform_attn_backward(
+                _lib.ptr(value), _lib.ptr(shapes2), 2, _lib.ptr(lsi), _lib.ptr(xy), 2, _lib.ptr(attn), None, _lib.ptr(go),
+                _lib.ptr(gv), _lib.ptr(gxy), 2, _lib.ptr(ga), None, _lib.ptr(ws), nbytes, B, S, M, C, L, Q, P, code, opts,
+                _lib.stream_of(value)), "dfa3d_wms_deform_attn_backward")
         _lib.check(library.dfa3d_fused_backward(
             _lib.ptr(value), _lib.ptr(dist), _lib.ptr(shapes), _lib.ptr(lsi), _lib.ptr(loc), _lib.ptr(attn), _lib.ptr(go),
             None, None, _lib.ptr(gv), _lib.ptr(gd), _lib.ptr(gl), _lib.ptr(ga), _lib.ptr(ws), nbytes, B, S, M, C, D, L, Q,
