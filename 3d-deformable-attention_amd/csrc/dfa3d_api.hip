@@ -58,6 +58,17 @@ void apply_opts(dfa3d::BwdArgs &a, const dfa3d_launch_options &o) {
   a.pass_hint = o.pass; a.event_binned = o.event_binned; a.clear_grads = o.clear;
 }
 
+// Whether a backward goes to the direct kernels, whatever scratch it has.
+bool goes_direct(const dfa3d_launch_options &o, const dfa3d::BwdArgs &a, int kind, int dtype) {
+  return o.direct == DFA3D_FEW_POINTS ? dfa3d::few_points(a, kind, dtype) : o.direct != 0;
+}
+// dimensions of a stage 1 backward
+dfa3d::BwdArgs stage1_dims(int B, int S, int M, int D, int L, int Q, int P) {
+  dfa3d::BwdArgs a{};
+  a.B = B; a.S = S; a.M = M; a.C = 0; a.D = D; a.L = L; a.Q = Q; a.P = P;
+  return a;
+}
+
 // Dimension checks shared by every entry point.  `width` is the per-head row length (C or D).
 int check_dims(const char *fn, int B, int S, int M, int width, int L, int Q, int P, int dtype) {
   if (dtype != DFA3D_F32 && dtype != DFA3D_F64 && dtype != DFA3D_BF16)
@@ -110,7 +121,7 @@ size_t dfa3d_ms_depth_score_sample_backward_workspace_bytes(int B, int S, int M,
   const char *fn = "dfa3d_ms_depth_score_sample_backward_workspace_bytes";
   dfa3d_launch_options o;
   if (check_dims(fn, B, S, M, D, L, Q, P, dtype) || check_opts(fn, opts, &o)) return 0;
-  if (o.direct) return 0;
+  if (goes_direct(o, stage1_dims(B, S, M, D, L, Q, P), 2, dtype)) return 0;
   dfa3d::DepthScoreBwdArgs a{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, B, S, M, D, L, Q, P, 0};
   return dfa3d::binned_depth_score_backward_workspace_bytes(a, dtype, o.tile);
 }
@@ -125,7 +136,7 @@ static int depth_score_backward(const char *fn, bool clear, const void *dist, co
   REQUIRE_PTR(fn, dist); REQUIRE_PTR(fn, shapes3); REQUIRE_PTR(fn, level_start); REQUIRE_PTR(fn, loc3);
   REQUIRE_PTR(fn, grad_score); REQUIRE_PTR(fn, grad_dist); REQUIRE_PTR(fn, grad_loc3);
   dfa3d::DepthScoreBwdArgs a{dist, shapes3, level_start, loc3, grad_score, grad_dist, grad_loc3, B, S, M, D, L, Q, P, clear ? 1 : 0};
-  if (workspace != nullptr && !o.direct) {
+  if (workspace != nullptr && !goes_direct(o, stage1_dims(B, S, M, D, L, Q, P), 2, dtype)) {
     const hipError_t e = dfa3d::launch_depth_score_backward_binned(a, dtype, workspace, workspace_bytes, o.tile, o.chunk,
                                                                    o.event_binned, (hipStream_t)stream);
     if (e != hipErrorNotSupported) return hip_result(e, fn);
@@ -196,9 +207,9 @@ size_t dfa3d_wms_deform_attn_backward_workspace_bytes(int B, int S, int M, int C
   const char *fn = "dfa3d_wms_deform_attn_backward_workspace_bytes";
   dfa3d_launch_options o;
   if (check_dims(fn, B, S, M, C, L, Q, P, dtype) || check_opts(fn, opts, &o, true)) return 0;
-  if (o.direct) return 0;
   const dfa3d::BwdArgs a = wms_bwd_args(nullptr, nullptr, 2, nullptr, nullptr, 2, nullptr, nullptr, nullptr, nullptr,
                                         nullptr, 2, nullptr, nullptr, B, S, M, C, L, Q, P, o);
+  if (goes_direct(o, a, 1, dtype)) return 0;
   return dfa3d::binned_backward_workspace_bytes(a, 1, dtype);
 }
 
@@ -222,7 +233,7 @@ int dfa3d_wms_deform_attn_backward(const void *value, const int64_t *shapes, int
   const dfa3d::BwdArgs a = wms_bwd_args(value, shapes, shape_stride, level_start, loc, loc_stride, attn, score,
                                         grad_out, grad_value, grad_loc, grad_loc_stride, grad_attn, grad_score, B, S,
                                         M, C, L, Q, P, o);
-  if (workspace != nullptr && !o.direct) {
+  if (workspace != nullptr && !goes_direct(o, a, 1, dtype)) {
     const hipError_t e = dfa3d::launch_backward_binned(a, dtype, workspace, workspace_bytes, (hipStream_t)stream);
     if (e != hipErrorNotSupported) return hip_result(e, fn);
   }
@@ -319,11 +330,11 @@ size_t dfa3d_fused_backward_workspace_bytes(int B, int S, int M, int C, int D, i
   if (check_dims(fn, B, S, M, C, L, Q, P, dtype) || check_dims(fn, B, S, M, D, L, Q, P, dtype) ||
       check_opts(fn, opts, &o, true))
     return 0;
-  if (o.direct) return 0;
   dfa3d::BwdArgs a = fused_bwd_args(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                                     nullptr, nullptr, nullptr, nullptr, nullptr, B, S, M, C, D, L, Q, P,
                                     dist_heads == 1 ? 1 : M, o);
   a.grad_bf16 = g16;
+  if (goes_direct(o, a, 0, dtype)) return g16 && o.direct == DFA3D_FEW_POINTS ? dfa3d::few_points_workspace_bytes(a) : 0;
   return dfa3d::binned_backward_workspace_bytes(a, 0, dtype);
 }
 
@@ -348,11 +359,16 @@ int dfa3d_fused_backward(const void *value, const void *dist, const int64_t *sha
                                     grad_weight_update, grad_value, grad_dist, grad_loc3, grad_attn, B, S, M, C,
                                     D, L, Q, P, dist_heads, o);
   a.grad_bf16 = g16;
-  if (workspace != nullptr && !o.direct) {
+  const bool direct = goes_direct(o, a, 0, dtype);
+  if (workspace != nullptr && direct && g16 && o.direct == DFA3D_FEW_POINTS) {
+    const hipError_t e = dfa3d::launch_few_points_rounded(a, dtype, workspace, workspace_bytes, (hipStream_t)stream);
+    if (e != hipErrorNotSupported) return hip_result(e, fn);
+  }
+  if (workspace != nullptr && !direct) {
     const hipError_t e = dfa3d::launch_backward_binned(a, dtype, workspace, workspace_bytes, (hipStream_t)stream);
     if (e != hipErrorNotSupported) return hip_result(e, fn);
   }
-  if (g16) return fail(DFA3D_EINVAL, "%s: DFA3D_BF16G (bfloat16 gradients) runs on the binned kernels only: pass a "
+  if (g16) return fail(DFA3D_EINVAL, "%s: DFA3D_BF16G (bfloat16 gradients) needs scratch: pass a "
                        "workspace of dfa3d_fused_backward_workspace_bytes(..., DFA3D_BF16G, ...) bytes (0 = not offered "
                        "for these dimensions: use DFA3D_BF16 with float gradients)", fn);
   return direct_fused_backward(fn, a, dtype, dist_heads, (hipStream_t)stream);
@@ -409,7 +425,7 @@ int dfa3d_fused_backward_static(const void *value, const void *dist, const int64
                                     grad_weight_update, grad_value, grad_dist, grad_loc3, grad_attn, B, S, M, C,
                                     D, L, Q, P, dist_heads, o);
   a.grad_bf16 = g16;
-  const size_t need = o.direct ? 0 : dfa3d::binned_backward_least_workspace_bytes(a, 0, dtype);
+  const size_t need = goes_direct(o, a, 0, dtype) && !(g16 && o.direct == DFA3D_FEW_POINTS) ? 0 : dfa3d::binned_backward_least_workspace_bytes(a, 0, dtype);
   if (need > DFA3D_STATIC_SCRATCH_BYTES)
     return fail(DFA3D_ERANGE, "%s: these dimensions need %zu bytes of scratch, the static buffer holds %zu; use "
                 "dfa3d_fused_backward with a workspace", fn, need, (size_t)DFA3D_STATIC_SCRATCH_BYTES);

@@ -72,6 +72,19 @@ __device__ __forceinline__ void scatter_add_two(rsrc_t r, A *base, uint32_t off_
   scatter_add(r, base, odd ? off_hi : off, odd ? hi : x);
 }
 
+// w * go added to the gradient row at byte offset `row` (kNoRow: none), of which this lane has the channels from `chan` on (kNoChan: none).  What adds
+// nothing is dropped instead of sent to memory: floats by the product, so that a zero weight on an infinite gradient arrives as NaN, as it does
+// from the tile kernels; doubles by the weight.
+template <typename A, int VEC>
+__device__ __forceinline__ void add_row(rsrc_t r, A *base, uint32_t row, uint32_t chan, A w, const A (&go)[VEC]) {
+  const uint32_t at = (sizeof(A) == 8 && w == 0 ? kNoRow : row) + chan;
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) {
+    const A add = w * go[i];
+    scatter_add(r, base, sizeof(A) == 4 && add == 0 ? kNoRow : at + i * (uint32_t)sizeof(A), add);
+  }
+}
+
 // Phase B of the backward pass over tasks [t_begin, t_end): per task the dot product of the value
 // row with grad_out (left in dots[t]) and the scatter-add of w * grad_out into grad_value.
 //   chan_off   lane's byte offset inside a value row (kNoChan beyond the last channel)
@@ -94,11 +107,7 @@ __device__ __forceinline__ void dots_and_scatter(rsrc_t value_r, rsrc_t gvalue_r
     for (int j = 0; j < U; ++j) RowVec<T, A, VEC>::ld(value_r, e[j].off + chan_off, v[j]);
 #pragma unroll
     for (int j = 0; j < U; ++j) {
-      // a zero weight adds nothing: drop the update instead of sending it to memory
-      const uint32_t goff = ((e[j].w != 0 && e[j].off != kNoRow) ? (e[j].off << GSHIFT) : kNoRow) +
-                            (chan_off == kNoChan ? kNoChan : (chan_off << GSHIFT));
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) scatter_add(gvalue_r, gvalue_b, goff + i * (uint32_t)sizeof(A), e[j].w * go[i]);
+      add_row<A, VEC>(gvalue_r, gvalue_b, e[j].off == kNoRow ? kNoRow : e[j].off << GSHIFT, chan_off == kNoChan ? kNoChan : chan_off << GSHIFT, e[j].w, go);
     }
 #pragma unroll
     for (int j = 0; j < U; ++j) {
@@ -117,14 +126,10 @@ __device__ __forceinline__ void dots_and_scatter(rsrc_t value_r, rsrc_t gvalue_r
     const uint32_t off = in ? e.off : kNoRow;
     A v[VEC];
     RowVec<T, A, VEC>::ld(value_r, off + chan_off, v);
-    const uint32_t goff = ((e.w != 0 && off != kNoRow) ? (off << GSHIFT) : kNoRow) +
-                          (chan_off == kNoChan ? kNoChan : (chan_off << GSHIFT));
+    add_row<A, VEC>(gvalue_r, gvalue_b, off == kNoRow ? kNoRow : off << GSHIFT, chan_off == kNoChan ? kNoChan : chan_off << GSHIFT, e.w, go);
     A part = 0;
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      scatter_add(gvalue_r, gvalue_b, goff + i * (uint32_t)sizeof(A), e.w * go[i]);
-      part += v[i] * go[i];
-    }
+    for (int i = 0; i < VEC; ++i) part += v[i] * go[i];
     part = row_sum<LPR>(part);
     if (cl == 0 && in) dots[t] = first_pass ? part : dots[t] + part;
   }

@@ -1580,6 +1580,35 @@ static size_t workspace_bytes_for(const BwdArgs &a, int kind, int dtype, bool le
 size_t binned_backward_workspace_bytes(const BwdArgs &a, int kind, int dtype) { return workspace_bytes_for(a, kind, dtype); }
 size_t binned_backward_least_workspace_bytes(const BwdArgs &a, int kind, int dtype) { return workspace_bytes_for(a, kind, dtype, true); }
 
+// A backward on the tile kernels is five launches (six for a distribution shared by the heads), of which each takes its 5 us however few points there
+// are, and visits every tile that has one.  The direct kernels are two launches, whose time is the clearing and one atomic per 64-byte
+// piece of what a point adds to, 20 G of which the L2 executes a second: 0.6 ns a point with rows of 32 floats and depth bins.  So the line is where
+// those atomics cost what the tile kernels' launches and tiles do.  The call's kernels alone (captured in a graph), 2 batch elements, 8 heads of 32
+// channels, 64 bins, us, tile kernels and direct, by thousands of points:
+//   40 x 60 and 20 x 30            12: 47, 22    51: 51, 47    128: 58, 91     one distribution for all heads   12: 55, 22    51: 58, 47    128: 66, 90
+//   80 x 120, three levels         19: 94, 33    76: 102, 69   153: 110, 116   16 channels                      12: 45, 19    51: 48, 36    128: 55, 65
+//   116 x 200, four levels         25: 139, 50  102: 175, 100  256: 188, 189   64 channels                      12: 59, 29    51: 62, 68    128: 70, 140
+//   plain attention, 40 x 60       12: 40, 19    51: 42, 35    128: 49, 66     on one level of 200 x 200        12: 113, 26   51: 142, 42   204: 152, 109
+//   stage 1 alone, 40 x 60         12: 55, 20    51: 57, 25    204: 61, 56     116 x 200, 112 bins              25: 104, 55  204: 121, 91   409: 127, 141
+// The lines below lie a tenth or so under the crossings.  With bfloat16 gradients the float sums are written, read and rounded besides.
+bool few_points(const BwdArgs &a, int kind, int dtype) {
+  if (dtype == DFA3D_F64) return true;                       // (no tile kernels)
+  const double points = (double)a.B * a.Q * a.M * a.L * a.P, rows = (double)a.B * a.S * a.M;
+  const int pieces = (kind == 2 ? 0 : 4 * ((a.C * 4 + 63) / 64)) + (kind == 1 ? 0 : 4);        // that a point adds to
+  const double atomics_us = points * pieces * 0.05e-3;
+  if (kind == 2) return atomics_us < 35 + rows * 0.06e-3;
+  if (kind == 1) return atomics_us < 18 + rows * 0.17e-3;
+  if (a.grad_bf16) return atomics_us < 19 + rows * 0.07e-3;
+  return atomics_us < (shared_dist(a) ? 30 + rows * 0.3e-3 : 25 + rows * 0.2e-3);
+}
+
+static size_t few_points_value_bytes(const BwdArgs &a) { return ((size_t)a.B * a.S * a.M * a.C * sizeof(float) + 255) & ~(size_t)255; }
+static size_t few_points_dist_rows(const BwdArgs &a) { return (size_t)a.B * a.S * (a.dist_heads == 1 ? 1 : a.M); }
+size_t few_points_workspace_bytes(const BwdArgs &a) {
+  if (((a.C | a.D) & 3) != 0) return 0;                      // bfloat16 gradients: whole 8-byte groups
+  return few_points_value_bytes(a) + few_points_dist_rows(a) * a.D * sizeof(float);
+}
+
 // Per-device facts and per-kernel attributes are looked up once and remembered (a launch then costs no
 // runtime queries).
 static std::mutex g_launch_mutex;
@@ -1791,6 +1820,23 @@ hipError_t launch_backward_binned(const BwdArgs &args, int dtype, void *workspac
     hipLaunchKernelGGL(round_rows_kernel, dim3(2048), dim3(256), 0, stream, (const float4 *)a.grad_value, (uint2 *)args.grad_value,
                        rows * a.C / 4, (const float4 *)a.grad_dist, (uint2 *)args.grad_dist, gd_heads != nullptr ? 0 : rows * a.D / 4);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_few_points_rounded(const BwdArgs &args, int dtype, void *workspace, size_t workspace_bytes, hipStream_t stream) {
+  const size_t need = few_points_workspace_bytes(args);
+  if (dtype != DFA3D_BF16 || need == 0 || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0 ||
+      (((uintptr_t)args.grad_value | (uintptr_t)args.grad_dist) & 7) != 0)
+    return hipErrorNotSupported;
+  BwdArgs a = args;
+  a.grad_bf16 = 0;
+  a.grad_value = workspace;
+  a.grad_dist = static_cast<char *>(workspace) + few_points_value_bytes(a);
+  const size_t value_elems = (size_t)a.B * a.S * a.M * a.C, dist_elems = few_points_dist_rows(a) * a.D;
+  if (hipError_t e = launch_zero_fill(a.grad_value, value_elems * sizeof(float), a.grad_dist, dist_elems * sizeof(float), stream)) return e;
+  if (hipError_t e = launch_backward(a, dtype, stream)) return e;
+  hipLaunchKernelGGL(round_rows_kernel, dim3(2048), dim3(256), 0, stream, (const float4 *)a.grad_value, (uint2 *)args.grad_value, value_elems / 4,
+                     (const float4 *)a.grad_dist, (uint2 *)args.grad_dist, dist_elems / 4);
   return hipGetLastError();
 }
 

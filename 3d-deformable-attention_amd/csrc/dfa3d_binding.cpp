@@ -103,6 +103,14 @@ struct NoGil {
   ~NoGil() { PyEval_RestoreThread(state); }
 };
 
+// options of a backward into tensors of its own
+dfa3d_launch_options own_gradients(bool clear) {
+  dfa3d_launch_options o{};
+  o.direct = DFA3D_FEW_POINTS;
+  o.clear = clear ? 1 : 0;
+  return o;
+}
+
 // shapes of a one-stage call
 struct FusedDims {
   int64_t B, S, M, C, D, L, Q, P, heads;
@@ -179,12 +187,11 @@ PyObject *fused_gradients(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (grad_out.numel() != d.B * d.Q * d.M * d.C || grad_out.scalar_type() != d.type) return declined();
   if (grad_score.defined() && (!shape_is(grad_score, {d.B, d.Q, d.M, d.L, d.P, 4}) || grad_score.scalar_type() != d.type)) return declined();
   if (grad_wu.defined() && (grad_wu.numel() != d.B * d.Q * d.M || grad_wu.scalar_type() != d.aux)) return declined();
-  // bfloat16 gradients are written as such where the tile kernels apply
+  // bfloat16 gradients are written as such where that is offered
+  const dfa3d_launch_options clear = own_gradients(true);
   const bool g16 = d.type == at::kBFloat16 &&
-                   api.fused_backward_workspace_bytes(d.B, d.S, d.M, d.C, d.D, d.L, d.Q, d.P, d.heads, DFA3D_BF16G, nullptr) > 0;
+                   api.fused_backward_workspace_bytes(d.B, d.S, d.M, d.C, d.D, d.L, d.Q, d.P, d.heads, DFA3D_BF16G, &clear) > 0;
   const int code = g16 ? DFA3D_BF16G : d.code;
-  dfa3d_launch_options clear{};
-  clear.clear = 1;
   const size_t bytes = api.fused_backward_workspace_bytes(d.B, d.S, d.M, d.C, d.D, d.L, d.Q, d.P, d.heads, code, &clear);
   const auto aux = value.options().dtype(d.aux), sums = g16 ? value.options() : aux;
   Tensor grad_value = at::empty(value.sizes(), sums), grad_dist = at::empty(dist.sizes(), sums), grad_loc = at::empty(loc.sizes(), aux),
@@ -252,8 +259,7 @@ PyObject *attention_gradients(PyObject *, PyObject *const *args, Py_ssize_t narg
   AttentionDims d;
   if (!in.ok || !attention_dims(value, shapes, starts, loc, attn, score, d) || d.loc_width != 2 || !step_ok(d.B, args[9])) return declined();
   if (grad_out.numel() != d.B * d.Q * d.M * d.C || grad_out.scalar_type() != d.type) return declined();
-  dfa3d_launch_options clear{};
-  clear.clear = 1;
+  const dfa3d_launch_options clear = own_gradients(true);
   const size_t bytes = api.attention_backward_workspace_bytes(d.B, d.S, d.M, d.C, d.L, d.Q, d.P, d.code, &clear);
   const auto aux = value.options().dtype(d.aux);
   Tensor grad_value = at::empty(value.sizes(), aux), grad_loc = at::empty(loc.sizes(), aux), grad_attn = at::empty(attn.sizes(), aux), grad_score,
@@ -315,7 +321,8 @@ PyObject *score_gradients(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   ScoreDims d;
   if (!in.ok || !score_dims(dist, shapes, starts, loc, d) || !step_ok(d.B, args[7])) return declined();
   if (!shape_is(grad_score, {d.B, d.Q, d.M, d.L, d.P, 4}) || grad_score.scalar_type() != d.type) return declined();
-  const size_t bytes = api.score_backward_workspace_bytes(d.B, d.S, d.M, d.D, d.L, d.Q, d.P, d.code, nullptr);
+  const dfa3d_launch_options options = own_gradients(false);      // (this entry point clears by itself)
+  const size_t bytes = api.score_backward_workspace_bytes(d.B, d.S, d.M, d.D, d.L, d.Q, d.P, d.code, &options);
   const auto aux = dist.options().dtype(d.aux);
   Tensor grad_dist = at::empty(dist.sizes(), aux), grad_loc = at::empty(loc.sizes(), aux), workspace;
   if (bytes > 0) workspace = at::empty({(int64_t)bytes}, dist.options().dtype(at::kByte));
@@ -323,7 +330,7 @@ PyObject *score_gradients(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   {
     NoGil no_gil;
     rc = api.score_backward(ptr(dist), keys(shapes), keys(starts), ptr(loc), ptr(grad_score), ptr(grad_dist), ptr(grad_loc), ptr(workspace), bytes,
-                            d.B, d.S, d.M, d.D, d.L, d.Q, d.P, d.code, nullptr, stream);
+                            d.B, d.S, d.M, d.D, d.L, d.Q, d.P, d.code, &options, stream);
   }
   if (rc != 0) return failed("dfa3d_ms_depth_score_sample_backward", rc);
   return tuple_of({grad_dist.to(d.type), grad_loc});

@@ -110,6 +110,13 @@ struct DepthScoreBwdArgs {
   int clear;                         // grad_dist holds anything on entry (binned kernels; the caller clears for the direct ones)
 };
 
+// Whether a backward has too few points for the tile kernels to pay (dfa3d_launch_options.direct = DFA3D_FEW_POINTS).  kind 0: both stages,
+// 1: stage 2 alone, 2: stage 1 alone.
+bool few_points(const BwdArgs &a, int kind, int dtype);
+// Such a backward with bfloat16 gradients (a.grad_bf16): sums in float in the workspace, rounded once at the end.
+size_t few_points_workspace_bytes(const BwdArgs &a);
+hipError_t launch_few_points_rounded(const BwdArgs &a, int dtype, void *workspace, size_t workspace_bytes, hipStream_t stream);
+
 // Looked up once per device and remembered: the number of CUs; the grant of more than 64 KB of dynamic LDS to a kernel.
 int cu_count();
 hipError_t allow_lds(const void *kernel, size_t bytes);

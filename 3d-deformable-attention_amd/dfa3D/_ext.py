@@ -42,6 +42,12 @@ def _here(value):
     return native, at, torch._C._cuda_getCurrentRawStream(at)
 
 
+def _by_size():
+    """A backward into tensors of its own takes the direct kernels where it has too few points for the tile kernels, unless
+    the caller's launch options say how it is to run."""
+    return contextlib.nullcontext() if _lib.options() is not None else _lib.launch_options(direct=_lib.DFA3D_FEW_POINTS)
+
+
 def _contig(**tensors):
     for name, t in tensors.items():
         if not t.is_contiguous():
@@ -191,8 +197,9 @@ def depth_score_gradients(value, value_spatial_shapes, value_level_start_index, 
             return got
     grad_value = torch.empty(value.shape, dtype=_aux_dtype(value.dtype), device=value.device)      # cleared by the call (clear=True)
     grad_sampling_loc = torch.empty_like(sampling_locations)
-    ms_depth_score_sample_backward_into(value, value_spatial_shapes, value_level_start_index, sampling_locations, grad_output,
-                                        grad_value, grad_sampling_loc, im2col_step=im2col_step, clear=True)
+    with _by_size():
+        ms_depth_score_sample_backward_into(value, value_spatial_shapes, value_level_start_index, sampling_locations, grad_output,
+                                            grad_value, grad_sampling_loc, im2col_step=im2col_step, clear=True)
     return grad_value.to(value.dtype), grad_sampling_loc
 
 
@@ -550,15 +557,16 @@ def dfa3d_fused_gradients(value, value_dpt_dist, value_spatial_shapes, value_lev
                                      im2col_step)
         if got is not None:
             return got
-    gdt = fused_backward_grad_dtype(value, value_dpt_dist, sampling_locations)
-    # not zeroed here: the call clears the part of the two buffers that its kernels add to (clear=True)
-    grad_value = torch.empty(value.shape, dtype=gdt, device=value.device)
-    grad_value_dpt_dist = torch.empty(value_dpt_dist.shape, dtype=gdt, device=value.device)
-    grad_sampling_loc = torch.empty_like(sampling_locations)
-    grad_attn_weight = torch.empty_like(attention_weights)
-    dfa3d_fused_backward(value, value_dpt_dist, value_spatial_shapes, value_level_start_index, sampling_locations,
-                         attention_weights, grad_output, grad_depth_score, grad_value, grad_value_dpt_dist, grad_sampling_loc,
-                         grad_attn_weight, im2col_step=im2col_step, grad_weight_update=grad_weight_update, clear=True)
+    with _by_size():
+        gdt = fused_backward_grad_dtype(value, value_dpt_dist, sampling_locations)
+        # not zeroed here: the call clears the part of the two buffers that its kernels add to (clear=True)
+        grad_value = torch.empty(value.shape, dtype=gdt, device=value.device)
+        grad_value_dpt_dist = torch.empty(value_dpt_dist.shape, dtype=gdt, device=value.device)
+        grad_sampling_loc = torch.empty_like(sampling_locations)
+        grad_attn_weight = torch.empty_like(attention_weights)
+        dfa3d_fused_backward(value, value_dpt_dist, value_spatial_shapes, value_level_start_index, sampling_locations,
+                             attention_weights, grad_output, grad_depth_score, grad_value, grad_value_dpt_dist, grad_sampling_loc,
+                             grad_attn_weight, im2col_step=im2col_step, grad_weight_update=grad_weight_update, clear=True)
     return grad_value.to(value.dtype), grad_value_dpt_dist.to(value_dpt_dist.dtype), grad_sampling_loc, grad_attn_weight
 
 
@@ -580,11 +588,13 @@ def attention_gradients(value, value_spatial_shapes, value_level_start_index, sa
         grad_sampling_loc[..., 2:] = 0
     grad_attn_weight = torch.empty_like(attention_weights)
     if depth_scores is None:
-        ms_deform_attn_backward(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
-                                grad_output, grad_value, grad_sampling_loc, grad_attn_weight, im2col_step=im2col_step, clear=True)
+        with _by_size():
+            ms_deform_attn_backward(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
+                                    grad_output, grad_value, grad_sampling_loc, grad_attn_weight, im2col_step=im2col_step, clear=True)
         return grad_value.to(value.dtype), grad_sampling_loc, grad_attn_weight, None
     grad_depth_score = torch.empty(depth_scores.shape, dtype=aux, device=value.device)
-    wms_deform_attn_backward_into(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
-                                  depth_scores, grad_output, grad_value, grad_sampling_loc, grad_attn_weight, grad_depth_score,
-                                  im2col_step=im2col_step, clear=True)
+    with _by_size():
+        wms_deform_attn_backward_into(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
+                                      depth_scores, grad_output, grad_value, grad_sampling_loc, grad_attn_weight, grad_depth_score,
+                                      im2col_step=im2col_step, clear=True)
     return grad_value.to(value.dtype), grad_sampling_loc, grad_attn_weight, grad_depth_score.to(depth_scores.dtype)

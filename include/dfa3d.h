@@ -60,7 +60,9 @@ extern "C" {
 typedef struct dfa3d_launch_options {
   int iters;    /* groups of units each wavefront walks through; 0 = 1, at most 64 */
   int vec;      /* channels per lane in the row gathers: 0 = automatic, 1, 2 or 4 (8: tile kernels only) */
-  int direct;   /* non-zero: a backward ignores its workspace and adds straight into device memory */
+  int direct;   /* a backward on the direct kernels, which add straight into device memory and need no scratch: 0 = where the
+                 * tile kernels are not offered, DFA3D_FEW_POINTS = there and where the call has too few points for the tile
+                 * kernels to pay, any other value = always (bfloat16 gradients, DFA3D_BF16G, only with DFA3D_FEW_POINTS) */
   int tile;     /* binned backward: tile edge in pixels as ty*100+tx, 0 = automatic */
   int block;    /* binned backward: threads per tile workgroup, 256 or 0/512 */
   int pass;     /* binned backward: points a tile workgroup takes per pass, 64, 128 or 256; 0 = automatic */
@@ -72,6 +74,8 @@ typedef struct dfa3d_launch_options {
   void *event_binned;   /* a hipEvent_t, or NULL: a binned backward records it on `stream` between its binning
                          * kernels and its tile kernel, so that a profiler can time the two parts of the call */
 } dfa3d_launch_options;
+
+#define DFA3D_FEW_POINTS 2   /* dfa3d_launch_options.direct */
 
 #define DFA3D_EINVAL (-1)   /* null pointer, non-positive dimension, bad stride or dtype */
 #define DFA3D_ERANGE (-2)   /* a dimension exceeds what the kernels index (see dfa3d_last_error) */
