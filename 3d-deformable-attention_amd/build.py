@@ -87,10 +87,11 @@ def _build_binding(force, verbose):
         built_for = f"{torch.__version__} {torch.version.git_version}"
         if not (force or _binding_stale(built_for)):
             return True
-        includes = [f"-isystem{d}" for d in cpp_extension.include_paths()]
-        libs = [f"-L{d}" for d in cpp_extension.library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10"]
+        rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+        includes = [f"-isystem{d}" for d in [*cpp_extension.include_paths(), os.path.join(rocm, "include")]]
+        libs = [f"-L{d}" for d in cpp_extension.library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
         _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
-              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DDFA3D_BUILT_FOR="{built_for}"',
+              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f'-DDFA3D_BUILT_FOR="{built_for}"',
               "-I" + sysconfig.get_paths()["include"], *includes, BINDING_SRC, "-o", BINDING, *libs], verbose)
     except (ImportError, OSError, subprocess.CalledProcessError) as e:
         print(f"{BINDING} is not built ({e}): calls go through ctypes, which takes 5 to 10 us longer each", file=sys.stderr)

@@ -11,16 +11,22 @@
 #include <ATen/autocast_mode.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <ATen/ops/zeros.h>
 #include <ATen/record_function.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
 #include <initializer_list>
 #include <limits>
+#include <stdexcept>
+#include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/dfa3d.h"
@@ -46,18 +52,23 @@ struct Api {
 
 using at::Tensor;
 
+// strided, with storage of its own, on `device`
+bool is_plain(const Tensor &t, int64_t device) {
+  return t.defined() && t.is_cuda() && t.get_device() == device && t.layout() == at::kStrided && t.has_storage() && !t.is_neg() && !t.is_conj();
+}
 // the operands of one call; `ok` says whether all of them can be read as they are
 struct Operands {
   int64_t device;
   bool ok = true;
+  bool locked = true;          // this thread holds the interpreter's lock
   // a tensor that is no wrapper: on this device, contiguous, with storage of its own
   const Tensor &need(PyObject *o) {
     static const Tensor none;
     if (!THPVariable_CheckExact(o)) { ok = false; return none; }
-    const Tensor &t = THPVariable_Unpack(o);
-    if (!t.defined() || !t.is_cuda() || t.get_device() != device || t.layout() != at::kStrided || !t.has_storage() || !t.is_contiguous() ||
-        t.is_neg() || t.is_conj())
-      ok = false;
+    return need(THPVariable_Unpack(o));
+  }
+  const Tensor &need(const Tensor &t) {
+    if (!is_plain(t, device) || !t.is_contiguous()) ok = false;
     return t;
   }
   const Tensor &may_have(PyObject *o) {
@@ -79,8 +90,19 @@ void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 const int64_t *keys(const Tensor &t) { return static_cast<const int64_t *>(t.data_ptr()); }
 
 PyObject *declined() { Py_RETURN_NONE; }
-PyObject *failed(const char *name, int rc) {
-  PyErr_Format(PyExc_RuntimeError, "%s failed with code %d: %s", name, rc, api.last_error());
+// What became of a call: taken, declined, or refused by the library, whose entry point is then named.
+struct Outcome {
+  bool taken;
+  const char *refused_by = nullptr;
+  int rc = 0;
+  std::string message() const { return std::string(refused_by) + " failed with code " + std::to_string(rc) + ": " + api.last_error(); }
+};
+constexpr Outcome kDeclined{false};
+Outcome outcome(const char *name, int rc) { return rc == 0 ? Outcome{true} : Outcome{false, name, rc}; }
+// the Python answer where there are no results
+PyObject *without_results(const Outcome &o) {
+  if (o.refused_by == nullptr) return declined();
+  PyErr_SetString(PyExc_RuntimeError, o.message().c_str());
   return nullptr;
 }
 // a tuple that owns the tensors; an undefined one is None
@@ -92,15 +114,24 @@ PyObject *tuple_of(std::initializer_list<Tensor> tensors) {
   return out;
 }
 // im2col_step as the reference checks it
-bool step_ok(int64_t batch, PyObject *o) {
-  if (!PyLong_CheckExact(o)) return false;
-  const long long given = PyLong_AsLongLong(o), step = given < batch ? given : batch;
-  if (given == -1 && PyErr_Occurred()) { PyErr_Clear(); return false; }
+bool step_ok(int64_t batch, int64_t given) {
+  const int64_t step = given < batch ? given : batch;
   return step > 0 && batch % step == 0;
 }
+// an im2col_step that is no number is one that no batch has
+int64_t step_of(PyObject *o) {
+  if (!PyLong_CheckExact(o)) return 0;
+  const long long given = PyLong_AsLongLong(o);
+  if (given == -1 && PyErr_Occurred()) { PyErr_Clear(); return 0; }
+  return given;
+}
+// without the interpreter's lock, where this thread holds it
 struct NoGil {
-  PyThreadState *state = PyEval_SaveThread();
-  ~NoGil() { PyEval_RestoreThread(state); }
+  PyThreadState *state;
+  explicit NoGil(bool locked) : state(locked ? PyEval_SaveThread() : nullptr) {}
+  ~NoGil() {
+    if (state != nullptr) PyEval_RestoreThread(state);
+  }
 };
 
 // options of a backward into tensors of its own
@@ -146,6 +177,24 @@ bool plain_dispatch() {
   if (!numbers(args, in.device, stream)) return nullptr;                                    \
   if (!plain_dispatch()) return declined();
 
+struct FusedResults { Tensor out, score, wu; };
+Outcome fused_forward(const Operands &in, void *stream, const Tensor &value, const Tensor &dist, const Tensor &shapes, const Tensor &starts,
+                      const Tensor &loc, const Tensor &attn, int64_t step, bool need_score, bool need_wu, const Tensor &packed, FusedResults &to) {
+  FusedDims d;
+  if (!in.ok || !fused_dims(value, dist, shapes, starts, loc, attn, d) || !step_ok(d.B, step)) return kDeclined;
+  if (packed.defined()) {
+    const size_t least = d.heads == 1 ? api.packed_dist_bytes(d.B, d.S, d.D, d.L, d.code) : 0;
+    if (least == 0 || packed.nbytes() < least) return kDeclined;
+  }
+  const auto store = value.options(), aux = store.dtype(d.aux);
+  to.out = at::empty({d.B, d.Q, d.M * d.C}, store);
+  if (need_score) to.score = at::empty({d.B, d.Q, d.M, d.L, d.P, 4}, store);
+  if (need_wu) to.wu = at::empty({d.B, d.Q, d.M, 1}, aux);
+  NoGil no_gil(in.locked);
+  return outcome("dfa3d_fused_forward",
+                 api.fused_forward(ptr(value), ptr(dist), keys(shapes), keys(starts), ptr(loc), ptr(attn), ptr(to.out), ptr(to.score), ptr(to.wu),
+                                   ptr(packed), d.B, d.S, d.M, d.C, d.D, d.L, d.Q, d.P, d.heads, d.code, nullptr, stream));
+}
 // fused_forward(device, stream, value, dist, shapes, starts, loc, attn, im2col_step, need_score, need_weight_update, packed)
 // -> (out, score or None, weight_update or None), or None
 PyObject *fused_forward(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
@@ -153,27 +202,45 @@ PyObject *fused_forward(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   TAKES(12)
   const Tensor &value = in.need(args[2]), &dist = in.need(args[3]), &shapes = in.need(args[4]), &starts = in.need(args[5]),
                &loc = in.need(args[6]), &attn = in.need(args[7]), &packed = in.may_have(args[11]);
-  FusedDims d;
-  if (!in.ok || !fused_dims(value, dist, shapes, starts, loc, attn, d) || !step_ok(d.B, args[8])) return declined();
-  if (packed.defined()) {
-    const size_t least = d.heads == 1 ? api.packed_dist_bytes(d.B, d.S, d.D, d.L, d.code) : 0;
-    if (least == 0 || packed.nbytes() < least) return declined();
-  }
-  const auto store = value.options(), aux = store.dtype(d.aux);
-  Tensor out = at::empty({d.B, d.Q, d.M * d.C}, store), score, wu;
-  if (args[9] == Py_True) score = at::empty({d.B, d.Q, d.M, d.L, d.P, 4}, store);
-  if (args[10] == Py_True) wu = at::empty({d.B, d.Q, d.M, 1}, aux);
-  int rc;
-  {
-    NoGil no_gil;
-    rc = api.fused_forward(ptr(value), ptr(dist), keys(shapes), keys(starts), ptr(loc), ptr(attn), ptr(out), ptr(score), ptr(wu), ptr(packed),
-                           d.B, d.S, d.M, d.C, d.D, d.L, d.Q, d.P, d.heads, d.code, nullptr, stream);
-  }
-  if (rc != 0) return failed("dfa3d_fused_forward", rc);
-  return tuple_of({out, score, wu});
+  FusedResults r;
+  const Outcome o = fused_forward(in, stream, value, dist, shapes, starts, loc, attn, step_of(args[8]), args[9] == Py_True, args[10] == Py_True,
+                                  packed, r);
+  return o.taken ? tuple_of({r.out, r.score, r.wu}) : without_results(o);
   END_HANDLE_TH_ERRORS
 }
 
+struct FusedGradients { Tensor value, dist, loc, attn; };
+Outcome fused_gradients(const Operands &in, void *stream, const Tensor &value, const Tensor &dist, const Tensor &shapes, const Tensor &starts,
+                        const Tensor &loc, const Tensor &attn, const Tensor &grad_out, const Tensor &grad_score, const Tensor &grad_wu, int64_t step,
+                        FusedGradients &to) {
+  FusedDims d;
+  if (!in.ok || !fused_dims(value, dist, shapes, starts, loc, attn, d) || !step_ok(d.B, step)) return kDeclined;
+  if (grad_out.numel() != d.B * d.Q * d.M * d.C || grad_out.scalar_type() != d.type) return kDeclined;
+  if (grad_score.defined() && (!shape_is(grad_score, {d.B, d.Q, d.M, d.L, d.P, 4}) || grad_score.scalar_type() != d.type)) return kDeclined;
+  if (grad_wu.defined() && (grad_wu.numel() != d.B * d.Q * d.M || grad_wu.scalar_type() != d.aux)) return kDeclined;
+  // bfloat16 gradients are written as such where that is offered
+  const dfa3d_launch_options clear = own_gradients(true);
+  const bool g16 = d.type == at::kBFloat16 &&
+                   api.fused_backward_workspace_bytes(d.B, d.S, d.M, d.C, d.D, d.L, d.Q, d.P, d.heads, DFA3D_BF16G, &clear) > 0;
+  const int code = g16 ? DFA3D_BF16G : d.code;
+  const size_t bytes = api.fused_backward_workspace_bytes(d.B, d.S, d.M, d.C, d.D, d.L, d.Q, d.P, d.heads, code, &clear);
+  const auto aux = value.options().dtype(d.aux), sums = g16 ? value.options() : aux;
+  to = FusedGradients{at::empty(value.sizes(), sums), at::empty(dist.sizes(), sums), at::empty(loc.sizes(), aux), at::empty(attn.sizes(), aux)};
+  Tensor workspace;
+  if (bytes > 0) workspace = at::empty({(int64_t)bytes}, value.options().dtype(at::kByte));
+  Outcome o{false};
+  {
+    NoGil no_gil(in.locked);
+    o = outcome("dfa3d_fused_backward",
+                api.fused_backward(ptr(value), ptr(dist), keys(shapes), keys(starts), ptr(loc), ptr(attn), ptr(grad_out), ptr(grad_score), ptr(grad_wu),
+                                   ptr(to.value), ptr(to.dist), ptr(to.loc), ptr(to.attn), ptr(workspace), bytes, d.B, d.S, d.M, d.C, d.D, d.L, d.Q,
+                                   d.P, d.heads, code, &clear, stream));
+  }
+  if (!o.taken) return o;
+  to.value = to.value.to(d.type);
+  to.dist = to.dist.to(d.type);
+  return o;
+}
 // fused_gradients(device, stream, value, dist, shapes, starts, loc, attn, grad_out, grad_score, grad_weight_update, im2col_step)
 // -> gradients of value, dist, loc and attn in their types, or None
 PyObject *fused_gradients(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
@@ -182,30 +249,9 @@ PyObject *fused_gradients(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   const Tensor &value = in.need(args[2]), &dist = in.need(args[3]), &shapes = in.need(args[4]), &starts = in.need(args[5]),
                &loc = in.need(args[6]), &attn = in.need(args[7]), &grad_out = in.need(args[8]), &grad_score = in.may_have(args[9]),
                &grad_wu = in.may_have(args[10]);
-  FusedDims d;
-  if (!in.ok || !fused_dims(value, dist, shapes, starts, loc, attn, d) || !step_ok(d.B, args[11])) return declined();
-  if (grad_out.numel() != d.B * d.Q * d.M * d.C || grad_out.scalar_type() != d.type) return declined();
-  if (grad_score.defined() && (!shape_is(grad_score, {d.B, d.Q, d.M, d.L, d.P, 4}) || grad_score.scalar_type() != d.type)) return declined();
-  if (grad_wu.defined() && (grad_wu.numel() != d.B * d.Q * d.M || grad_wu.scalar_type() != d.aux)) return declined();
-  // bfloat16 gradients are written as such where that is offered
-  const dfa3d_launch_options clear = own_gradients(true);
-  const bool g16 = d.type == at::kBFloat16 &&
-                   api.fused_backward_workspace_bytes(d.B, d.S, d.M, d.C, d.D, d.L, d.Q, d.P, d.heads, DFA3D_BF16G, &clear) > 0;
-  const int code = g16 ? DFA3D_BF16G : d.code;
-  const size_t bytes = api.fused_backward_workspace_bytes(d.B, d.S, d.M, d.C, d.D, d.L, d.Q, d.P, d.heads, code, &clear);
-  const auto aux = value.options().dtype(d.aux), sums = g16 ? value.options() : aux;
-  Tensor grad_value = at::empty(value.sizes(), sums), grad_dist = at::empty(dist.sizes(), sums), grad_loc = at::empty(loc.sizes(), aux),
-         grad_attn = at::empty(attn.sizes(), aux), workspace;
-  if (bytes > 0) workspace = at::empty({(int64_t)bytes}, value.options().dtype(at::kByte));
-  int rc;
-  {
-    NoGil no_gil;
-    rc = api.fused_backward(ptr(value), ptr(dist), keys(shapes), keys(starts), ptr(loc), ptr(attn), ptr(grad_out), ptr(grad_score), ptr(grad_wu),
-                            ptr(grad_value), ptr(grad_dist), ptr(grad_loc), ptr(grad_attn), ptr(workspace), bytes, d.B, d.S, d.M, d.C, d.D, d.L,
-                            d.Q, d.P, d.heads, code, &clear, stream);
-  }
-  if (rc != 0) return failed("dfa3d_fused_backward", rc);
-  return tuple_of({grad_value.to(d.type), grad_dist.to(d.type), grad_loc, grad_attn});
+  FusedGradients g;
+  const Outcome o = fused_gradients(in, stream, value, dist, shapes, starts, loc, attn, grad_out, grad_score, grad_wu, step_of(args[11]), g);
+  return o.taken ? tuple_of({g.value, g.dist, g.loc, g.attn}) : without_results(o);
   END_HANDLE_TH_ERRORS
 }
 
@@ -229,26 +275,54 @@ bool attention_dims(const Tensor &value, const Tensor &shapes, const Tensor &sta
          (!score.defined() || (shape_is(score, {d.B, d.Q, d.M, d.L, d.P, 4}) && score.scalar_type() == d.type));
 }
 
+Outcome attention_forward(const Operands &in, void *stream, const Tensor &value, const Tensor &shapes, const Tensor &starts, const Tensor &loc,
+                          const Tensor &attn, const Tensor &score, int64_t step, Tensor &out) {
+  AttentionDims d;
+  if (!in.ok || !attention_dims(value, shapes, starts, loc, attn, score, d) || !step_ok(d.B, step)) return kDeclined;
+  out = at::empty({d.B, d.Q, d.M * d.C}, value.options());
+  NoGil no_gil(in.locked);
+  return outcome("dfa3d_wms_deform_attn_forward",
+                 api.attention_forward(ptr(value), keys(shapes), d.shape_width, keys(starts), ptr(loc), d.loc_width, ptr(attn), ptr(score), ptr(out),
+                                       d.B, d.S, d.M, d.C, d.L, d.Q, d.P, d.code, nullptr, stream));
+}
 // attention_forward(device, stream, value, shapes, starts, loc, attn, score or None, im2col_step) -> out, or None
 PyObject *attention_forward(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   TAKES(9)
   const Tensor &value = in.need(args[2]), &shapes = in.need(args[3]), &starts = in.need(args[4]), &loc = in.need(args[5]),
                &attn = in.need(args[6]), &score = in.may_have(args[7]);
-  AttentionDims d;
-  if (!in.ok || !attention_dims(value, shapes, starts, loc, attn, score, d) || !step_ok(d.B, args[8])) return declined();
-  Tensor out = at::empty({d.B, d.Q, d.M * d.C}, value.options());
-  int rc;
-  {
-    NoGil no_gil;
-    rc = api.attention_forward(ptr(value), keys(shapes), d.shape_width, keys(starts), ptr(loc), d.loc_width, ptr(attn), ptr(score), ptr(out),
-                               d.B, d.S, d.M, d.C, d.L, d.Q, d.P, d.code, nullptr, stream);
-  }
-  if (rc != 0) return failed("dfa3d_wms_deform_attn_forward", rc);
-  return THPVariable_Wrap(out);
+  Tensor out;
+  const Outcome o = attention_forward(in, stream, value, shapes, starts, loc, attn, score, step_of(args[8]), out);
+  return o.taken ? THPVariable_Wrap(out) : without_results(o);
   END_HANDLE_TH_ERRORS
 }
 
+struct AttentionGradients { Tensor value, loc, attn, score; };
+Outcome attention_gradients(const Operands &in, void *stream, const Tensor &value, const Tensor &shapes, const Tensor &starts, const Tensor &loc,
+                            const Tensor &attn, const Tensor &score, const Tensor &grad_out, int64_t step, AttentionGradients &to) {
+  AttentionDims d;
+  if (!in.ok || !attention_dims(value, shapes, starts, loc, attn, score, d) || d.loc_width != 2 || !step_ok(d.B, step)) return kDeclined;
+  if (grad_out.numel() != d.B * d.Q * d.M * d.C || grad_out.scalar_type() != d.type) return kDeclined;
+  const dfa3d_launch_options clear = own_gradients(true);
+  const size_t bytes = api.attention_backward_workspace_bytes(d.B, d.S, d.M, d.C, d.L, d.Q, d.P, d.code, &clear);
+  const auto aux = value.options().dtype(d.aux);
+  to = AttentionGradients{at::empty(value.sizes(), aux), at::empty(loc.sizes(), aux), at::empty(attn.sizes(), aux), Tensor()};
+  Tensor workspace;
+  if (score.defined()) to.score = at::empty(score.sizes(), aux);
+  if (bytes > 0) workspace = at::empty({(int64_t)bytes}, value.options().dtype(at::kByte));
+  Outcome o{false};
+  {
+    NoGil no_gil(in.locked);
+    o = outcome("dfa3d_wms_deform_attn_backward",
+                api.attention_backward(ptr(value), keys(shapes), d.shape_width, keys(starts), ptr(loc), d.loc_width, ptr(attn), ptr(score), ptr(grad_out),
+                                       ptr(to.value), ptr(to.loc), d.loc_width, ptr(to.attn), ptr(to.score), ptr(workspace), bytes, d.B, d.S, d.M, d.C,
+                                       d.L, d.Q, d.P, d.code, &clear, stream));
+  }
+  if (!o.taken) return o;
+  to.value = to.value.to(d.type);
+  if (score.defined()) to.score = to.score.to(d.type);
+  return o;
+}
 // attention_gradients(device, stream, value, shapes, starts, loc (2 wide), attn, score or None, grad_out, im2col_step)
 // -> gradients of value, loc, attn and score (None without one) in their types, or None
 PyObject *attention_gradients(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
@@ -256,25 +330,9 @@ PyObject *attention_gradients(PyObject *, PyObject *const *args, Py_ssize_t narg
   TAKES(10)
   const Tensor &value = in.need(args[2]), &shapes = in.need(args[3]), &starts = in.need(args[4]), &loc = in.need(args[5]),
                &attn = in.need(args[6]), &score = in.may_have(args[7]), &grad_out = in.need(args[8]);
-  AttentionDims d;
-  if (!in.ok || !attention_dims(value, shapes, starts, loc, attn, score, d) || d.loc_width != 2 || !step_ok(d.B, args[9])) return declined();
-  if (grad_out.numel() != d.B * d.Q * d.M * d.C || grad_out.scalar_type() != d.type) return declined();
-  const dfa3d_launch_options clear = own_gradients(true);
-  const size_t bytes = api.attention_backward_workspace_bytes(d.B, d.S, d.M, d.C, d.L, d.Q, d.P, d.code, &clear);
-  const auto aux = value.options().dtype(d.aux);
-  Tensor grad_value = at::empty(value.sizes(), aux), grad_loc = at::empty(loc.sizes(), aux), grad_attn = at::empty(attn.sizes(), aux), grad_score,
-         workspace;
-  if (score.defined()) grad_score = at::empty(score.sizes(), aux);
-  if (bytes > 0) workspace = at::empty({(int64_t)bytes}, value.options().dtype(at::kByte));
-  int rc;
-  {
-    NoGil no_gil;
-    rc = api.attention_backward(ptr(value), keys(shapes), d.shape_width, keys(starts), ptr(loc), d.loc_width, ptr(attn), ptr(score), ptr(grad_out),
-                                ptr(grad_value), ptr(grad_loc), d.loc_width, ptr(grad_attn), ptr(grad_score), ptr(workspace), bytes, d.B, d.S,
-                                d.M, d.C, d.L, d.Q, d.P, d.code, &clear, stream);
-  }
-  if (rc != 0) return failed("dfa3d_wms_deform_attn_backward", rc);
-  return tuple_of({grad_value.to(d.type), grad_loc, grad_attn, grad_score.defined() ? grad_score.to(d.type) : grad_score});
+  AttentionGradients g;
+  const Outcome o = attention_gradients(in, stream, value, shapes, starts, loc, attn, score, grad_out, step_of(args[9]), g);
+  return o.taken ? tuple_of({g.value, g.loc, g.attn, g.score}) : without_results(o);
   END_HANDLE_TH_ERRORS
 }
 
@@ -294,71 +352,259 @@ bool score_dims(const Tensor &dist, const Tensor &shapes, const Tensor &starts, 
          starts.scalar_type() == at::kLong;
 }
 
+Outcome score_forward(const Operands &in, void *stream, const Tensor &dist, const Tensor &shapes, const Tensor &starts, const Tensor &loc, int64_t step,
+                      Tensor &score) {
+  ScoreDims d;
+  if (!in.ok || !score_dims(dist, shapes, starts, loc, d) || !step_ok(d.B, step)) return kDeclined;
+  score = at::empty({d.B, d.Q, d.M, d.L, d.P, 4}, dist.options());
+  NoGil no_gil(in.locked);
+  return outcome("dfa3d_ms_depth_score_sample_forward", api.score_forward(ptr(dist), keys(shapes), keys(starts), ptr(loc), ptr(score), d.B, d.S, d.M,
+                                                                          d.D, d.L, d.Q, d.P, d.code, nullptr, stream));
+}
 // score_forward(device, stream, dist, shapes, starts, loc, im2col_step) -> score, or None
 PyObject *score_forward(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   TAKES(7)
   const Tensor &dist = in.need(args[2]), &shapes = in.need(args[3]), &starts = in.need(args[4]), &loc = in.need(args[5]);
-  ScoreDims d;
-  if (!in.ok || !score_dims(dist, shapes, starts, loc, d) || !step_ok(d.B, args[6])) return declined();
-  Tensor score = at::empty({d.B, d.Q, d.M, d.L, d.P, 4}, dist.options());
-  int rc;
-  {
-    NoGil no_gil;
-    rc = api.score_forward(ptr(dist), keys(shapes), keys(starts), ptr(loc), ptr(score), d.B, d.S, d.M, d.D, d.L, d.Q, d.P, d.code, nullptr, stream);
-  }
-  if (rc != 0) return failed("dfa3d_ms_depth_score_sample_forward", rc);
-  return THPVariable_Wrap(score);
+  Tensor score;
+  const Outcome o = score_forward(in, stream, dist, shapes, starts, loc, step_of(args[6]), score);
+  return o.taken ? THPVariable_Wrap(score) : without_results(o);
   END_HANDLE_TH_ERRORS
 }
 
+struct ScoreGradients { Tensor dist, loc; };
+Outcome score_gradients(const Operands &in, void *stream, const Tensor &dist, const Tensor &shapes, const Tensor &starts, const Tensor &loc,
+                        const Tensor &grad_score, int64_t step, ScoreGradients &to) {
+  ScoreDims d;
+  if (!in.ok || !score_dims(dist, shapes, starts, loc, d) || !step_ok(d.B, step)) return kDeclined;
+  if (!shape_is(grad_score, {d.B, d.Q, d.M, d.L, d.P, 4}) || grad_score.scalar_type() != d.type) return kDeclined;
+  const dfa3d_launch_options options = own_gradients(false);      // (this entry point clears by itself)
+  const size_t bytes = api.score_backward_workspace_bytes(d.B, d.S, d.M, d.D, d.L, d.Q, d.P, d.code, &options);
+  const auto aux = dist.options().dtype(d.aux);
+  to = ScoreGradients{at::empty(dist.sizes(), aux), at::empty(loc.sizes(), aux)};
+  Tensor workspace;
+  if (bytes > 0) workspace = at::empty({(int64_t)bytes}, dist.options().dtype(at::kByte));
+  Outcome o{false};
+  {
+    NoGil no_gil(in.locked);
+    o = outcome("dfa3d_ms_depth_score_sample_backward",
+                api.score_backward(ptr(dist), keys(shapes), keys(starts), ptr(loc), ptr(grad_score), ptr(to.dist), ptr(to.loc), ptr(workspace), bytes, d.B,
+                                   d.S, d.M, d.D, d.L, d.Q, d.P, d.code, &options, stream));
+  }
+  if (!o.taken) return o;
+  to.dist = to.dist.to(d.type);
+  return o;
+}
 // score_gradients(device, stream, dist, shapes, starts, loc, grad_score, im2col_step) -> gradients of dist and loc in their types, or None
 PyObject *score_gradients(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   TAKES(8)
   const Tensor &dist = in.need(args[2]), &shapes = in.need(args[3]), &starts = in.need(args[4]), &loc = in.need(args[5]),
                &grad_score = in.need(args[6]);
-  ScoreDims d;
-  if (!in.ok || !score_dims(dist, shapes, starts, loc, d) || !step_ok(d.B, args[7])) return declined();
-  if (!shape_is(grad_score, {d.B, d.Q, d.M, d.L, d.P, 4}) || grad_score.scalar_type() != d.type) return declined();
-  const dfa3d_launch_options options = own_gradients(false);      // (this entry point clears by itself)
-  const size_t bytes = api.score_backward_workspace_bytes(d.B, d.S, d.M, d.D, d.L, d.Q, d.P, d.code, &options);
-  const auto aux = dist.options().dtype(d.aux);
-  Tensor grad_dist = at::empty(dist.sizes(), aux), grad_loc = at::empty(loc.sizes(), aux), workspace;
-  if (bytes > 0) workspace = at::empty({(int64_t)bytes}, dist.options().dtype(at::kByte));
-  int rc;
-  {
-    NoGil no_gil;
-    rc = api.score_backward(ptr(dist), keys(shapes), keys(starts), ptr(loc), ptr(grad_score), ptr(grad_dist), ptr(grad_loc), ptr(workspace), bytes,
-                            d.B, d.S, d.M, d.D, d.L, d.Q, d.P, d.code, &options, stream);
-  }
-  if (rc != 0) return failed("dfa3d_ms_depth_score_sample_backward", rc);
-  return tuple_of({grad_dist.to(d.type), grad_loc});
+  ScoreGradients g;
+  const Outcome o = score_gradients(in, stream, dist, shapes, starts, loc, grad_score, step_of(args[7]), g);
+  return o.taken ? tuple_of({g.dist, g.loc}) : without_results(o);
   END_HANDLE_TH_ERRORS
 }
 
+Outcome pack_dist(const Operands &in, void *stream, const Tensor &dist, const Tensor &shapes, const Tensor &starts, Tensor &packed) {
+  if (!in.ok || dist.dim() != 4 || dist.size(2) != 1 || shapes.dim() != 2 || shapes.size(1) != 3 || !shape_is(starts, {shapes.size(0)}) ||
+      shapes.scalar_type() != at::kLong || starts.scalar_type() != at::kLong)
+    return kDeclined;
+  const int64_t B = dist.size(0), S = dist.size(1), D = dist.size(3), L = shapes.size(0);
+  const int code = code_of(dist.scalar_type());
+  if (!(code == DFA3D_F32 || code == DFA3D_BF16) || !fits_int({B, S, D, L})) return kDeclined;
+  const size_t bytes = api.packed_dist_bytes(B, S, D, L, code);
+  if (bytes == 0) return kDeclined;
+  packed = at::empty({(int64_t)bytes}, dist.options().dtype(at::kByte));
+  NoGil no_gil(in.locked);
+  return outcome("dfa3d_pack_dist", api.pack_dist(ptr(dist), keys(shapes), keys(starts), ptr(packed), bytes, B, S, D, L, code, stream));
+}
 // pack_dist(device, stream, dist (bs, keys, 1, D), shapes, starts) -> packed distribution, or None
 PyObject *pack_dist(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   TAKES(5)
   const Tensor &dist = in.need(args[2]), &shapes = in.need(args[3]), &starts = in.need(args[4]);
-  if (!in.ok || dist.dim() != 4 || dist.size(2) != 1 || shapes.dim() != 2 || shapes.size(1) != 3 || !shape_is(starts, {shapes.size(0)}) ||
-      shapes.scalar_type() != at::kLong || starts.scalar_type() != at::kLong)
-    return declined();
-  const int64_t B = dist.size(0), S = dist.size(1), D = dist.size(3), L = shapes.size(0);
-  const int code = code_of(dist.scalar_type());
-  if (!(code == DFA3D_F32 || code == DFA3D_BF16) || !fits_int({B, S, D, L})) return declined();
-  const size_t bytes = api.packed_dist_bytes(B, S, D, L, code);
-  if (bytes == 0) return declined();
-  Tensor packed = at::empty({(int64_t)bytes}, dist.options().dtype(at::kByte));
-  int rc;
-  {
-    NoGil no_gil;
-    rc = api.pack_dist(ptr(dist), keys(shapes), keys(starts), ptr(packed), bytes, B, S, D, L, code, stream);
-  }
-  if (rc != 0) return failed("dfa3d_pack_dist", rc);
-  return THPVariable_Wrap(packed);
+  Tensor packed;
+  const Outcome o = pack_dist(in, stream, dist, shapes, starts, packed);
+  return o.taken ? THPVariable_Wrap(packed) : without_results(o);
   END_HANDLE_TH_ERRORS
+}
+
+// Calls of the Functions as a whole: forward, and the node of the graph where one is recorded, whose backward runs without the interpreter.  A
+// node of Python's needs the interpreter's lock on the engine's thread, which is handed over twice a backward, and costs its context and two wrappers:
+// 1 x 50 queries on 15 x 25 maps, a training pass in a row of them, 99 -> 68 us (backward 69 -> 54; with the engine on the caller's own thread the pass
+// 50 -> 42), the forward 11.7 -> 8.3 recorded and 9.4 -> 7.6 not.
+enum Kind { kScore, kStage2, kPlain, kFused, kWeightUpdate };      // numbered as in recording.py
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// (kind, im2col_step, saved tensors, gradients of the outputs) -> gradients of the saved tensors: a Function's own backward, for what is not as the
+// kernels read it, and for a backward that is recorded itself
+PyObject *python_backward = nullptr;
+
+struct WithGil {
+  PyGILState_STATE state = PyGILState_Ensure();
+  ~WithGil() { PyGILState_Release(state); }
+};
+PyObject *python_tuple(const variable_list &t) {
+  PyObject *to = PyTuple_New((Py_ssize_t)t.size());
+  for (size_t i = 0; to != nullptr && i < t.size(); ++i)
+    PyTuple_SET_ITEM(to, (Py_ssize_t)i, t[i].defined() ? THPVariable_Wrap(t[i]) : Py_NewRef(Py_None));
+  return to;
+}
+variable_list gradients_by_python(Kind kind, int64_t step, const variable_list &t, const variable_list &grads) {
+  WithGil gil;
+  PyObject *saved = python_tuple(t), *incoming = python_tuple(grads), *got = nullptr;
+  if (saved != nullptr && incoming != nullptr && python_backward != nullptr)
+    got = PyObject_CallFunction(python_backward, "iLOO", (int)kind, (long long)step, saved, incoming);
+  Py_XDECREF(saved);
+  Py_XDECREF(incoming);
+  variable_list to(t.size());
+  if (got != nullptr && PyTuple_CheckExact(got) && (size_t)PyTuple_GET_SIZE(got) == t.size()) {
+    for (size_t i = 0; i < t.size(); ++i)
+      if (PyObject *g = PyTuple_GET_ITEM(got, (Py_ssize_t)i); THPVariable_Check(g)) to[i] = THPVariable_Unpack(g);
+    Py_DECREF(got);
+    return to;
+  }
+  if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "no gradients");
+  Py_XDECREF(got);
+  python_error e;
+  e.persist();
+  throw e;
+}
+// an incoming gradient as a contiguous tensor of the output's type
+Tensor incoming(const Tensor &g, at::ScalarType like, int64_t device, bool &ok) {
+  if (!g.defined()) return g;
+  if (!is_plain(g, device) || g.unsafeGetTensorImpl()->is_python_dispatch()) { ok = false; return g; }
+  return g.contiguous().to(like);
+}
+// the saved tensors' gradients, or false
+bool gradients_of(Kind kind, int64_t step, const variable_list &t, const variable_list &grads, variable_list &to) {
+  if (c10::GradMode::is_enabled() || !plain_dispatch() || !t[0].defined() || !t[0].is_cuda()) return false;
+  Operands in{t[0].get_device()};
+  in.locked = false;
+  if (c10::hip::current_device() != in.device) return false;
+  for (const Tensor &x : t) in.need(x);
+  const Tensor &loc = t[kind == kFused || kind == kWeightUpdate ? 4 : 3];
+  if (!in.ok || loc.dim() != 6 || t[0].dim() != 4) return false;
+  const at::ScalarType type = t[0].scalar_type();
+  Tensor g = incoming(grads[0], type, in.device, in.ok), score, wu;
+  if (kind == kFused) score = incoming(grads[1], type, in.device, in.ok);
+  if (kind == kWeightUpdate) wu = incoming(grads[1], aux_of(type), in.device, in.ok);
+  if (!in.ok) return false;
+  if (!g.defined()) {
+    g = kind == kScore ? at::zeros({t[0].size(0), loc.size(1), t[0].size(2), loc.size(3), loc.size(4), 4}, t[0].options())
+                       : at::zeros({t[0].size(0), loc.size(1), t[0].size(2) * t[0].size(3)}, t[0].options());
+  }
+  void *stream = c10::hip::getCurrentHIPStream(in.device).stream();
+  Outcome o{false};
+  if (kind == kScore) {
+    ScoreGradients r;
+    o = score_gradients(in, stream, t[0], t[1], t[2], t[3], g, step, r);
+    to = {r.dist, Tensor(), Tensor(), r.loc};
+  } else if (kind == kStage2 || kind == kPlain) {
+    AttentionGradients r;
+    o = attention_gradients(in, stream, t[0], t[1], t[2], t[3], t[4], kind == kStage2 ? t[5] : Tensor(), g, step, r);
+    to = {r.value, Tensor(), Tensor(), r.loc, r.attn};
+    if (kind == kStage2) to.push_back(r.score);
+  } else {
+    FusedGradients r;
+    o = fused_gradients(in, stream, t[0], t[1], t[2], t[3], t[4], t[5], g, score, wu, step, r);
+    to = {r.value, r.dist, Tensor(), Tensor(), r.loc, r.attn};
+  }
+  if (o.refused_by != nullptr) throw std::runtime_error(o.message());
+  return o.taken;
+}
+
+// The nodes, which hand out outputs that are there already.
+template <typename Self, Kind KIND> struct Recorded : torch::autograd::Function<Self> {
+  template <typename... Tensors>
+  static variable_list forward(AutogradContext *ctx, int64_t step, const variable_list *outputs, const Tensors &...saved) {
+    ctx->set_materialize_grads(false);
+    ctx->save_for_backward({saved...});
+    ctx->saved_data["step"] = step;
+    return *outputs;
+  }
+  static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
+    const int64_t step = ctx->saved_data["step"].toInt();
+    const variable_list saved = ctx->get_saved_variables();
+    variable_list to;
+    if (!gradients_of(KIND, step, saved, grads, to)) to = gradients_by_python(KIND, step, saved, grads);
+    to.insert(to.begin(), 2, Tensor());                      // of the step and the outputs
+    return to;
+  }
+};
+}  // namespace
+namespace dfa3d {      // (their names are what a graph shows)
+struct MultiScaleDepthScoreSampleFunction : Recorded<MultiScaleDepthScoreSampleFunction, kScore> {};
+struct WeightedMultiScaleDeformableAttnFunction : Recorded<WeightedMultiScaleDeformableAttnFunction, kStage2> {};
+struct MultiScaleDeformableAttnFunction : Recorded<MultiScaleDeformableAttnFunction, kPlain> {};
+struct MultiScale3DDeformableAttnFunction : Recorded<MultiScale3DDeformableAttnFunction, kFused> {};
+struct MultiScale3DDeformableAttnWeightUpdateFunction : Recorded<MultiScale3DDeformableAttnWeightUpdateFunction, kWeightUpdate> {};
+}  // namespace dfa3d
+namespace {
+// the outputs with a node behind them, where one is to be made
+template <typename F, typename... Tensors> variable_list recorded_outputs(variable_list outputs, int64_t step, const Tensors &...inputs) {
+  if (!c10::GradMode::is_enabled() || !(inputs.requires_grad() || ...)) return outputs;
+  return F::apply(step, (const variable_list *)&outputs, inputs...);
+}
+
+// call(device, stream, kind, arguments of a Function's apply) -> what apply returns, or None
+PyObject *call(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TAKES(4)
+  const long kind = PyLong_AsLong(args[2]);
+  if (kind == -1 && PyErr_Occurred()) return nullptr;
+  if (!PyTuple_CheckExact(args[3]) || at::autocast::is_autocast_enabled(at::kCUDA)) return declined();
+  const Py_ssize_t given = PyTuple_GET_SIZE(args[3]);
+  const auto arg = [&](Py_ssize_t i) { return PyTuple_GET_ITEM(args[3], i); };
+  if (kind == kScore && given == 5) {
+    const Tensor &dist = in.need(arg(0)), &shapes = in.need(arg(1)), &starts = in.need(arg(2)), &loc = in.need(arg(3));
+    const int64_t step = step_of(arg(4));
+    Tensor score;
+    const Outcome o = score_forward(in, stream, dist, shapes, starts, loc, step, score);
+    if (!o.taken) return without_results(o);
+    return THPVariable_Wrap(recorded_outputs<dfa3d::MultiScaleDepthScoreSampleFunction>({score}, step, dist, shapes, starts, loc)[0]);
+  }
+  if ((kind == kStage2 && given == 7) || (kind == kPlain && given == 6)) {
+    const Tensor &value = in.need(arg(0)), &shapes = in.need(arg(1)), &starts = in.need(arg(2)), &loc = in.need(arg(3)), &attn = in.need(arg(4));
+    const Tensor score = kind == kStage2 ? in.need(arg(5)) : Tensor();
+    const int64_t step = step_of(arg(given - 1));
+    Tensor out;
+    const Outcome o = attention_forward(in, stream, value, shapes, starts, loc, attn, score, step, out);
+    if (!o.taken) return without_results(o);
+    return THPVariable_Wrap(
+        (kind == kStage2 ? recorded_outputs<dfa3d::WeightedMultiScaleDeformableAttnFunction>({out}, step, value, shapes, starts, loc, attn, score)
+                         : recorded_outputs<dfa3d::MultiScaleDeformableAttnFunction>({out}, step, value, shapes, starts, loc, attn))[0]);
+  }
+  if ((kind == kFused && given == 7) || (kind == kWeightUpdate && (given == 7 || given == 8))) {
+    const Tensor &value = in.need(arg(0)), &dist = in.need(arg(1)), &shapes = in.need(arg(2)), &starts = in.need(arg(3)), &loc = in.need(arg(4)),
+                 &attn = in.need(arg(5));
+    const int64_t step = step_of(arg(6));
+    Tensor packed = given == 8 ? in.may_have(arg(7)) : Tensor();
+    if (!in.ok) return declined();
+    // the packed form of a distribution shared by all heads, where making it pays: functional._packed_for_forward
+    if (!packed.defined() && dist.dim() == 4 && dist.size(2) == 1 && loc.numel() / 3 >= dist.size(0) * dist.size(1) * dist.size(3)) {
+      const Outcome o = pack_dist(in, stream, dist, shapes, starts, packed);
+      if (o.refused_by != nullptr) return without_results(o);
+    }
+    FusedResults r;
+    const Outcome o = fused_forward(in, stream, value, dist, shapes, starts, loc, attn, step, kind == kFused, kind == kWeightUpdate, packed, r);
+    if (!o.taken) return without_results(o);
+    const variable_list out =
+        kind == kFused ? recorded_outputs<dfa3d::MultiScale3DDeformableAttnFunction>({r.out, r.score}, step, value, dist, shapes, starts, loc, attn)
+                       : recorded_outputs<dfa3d::MultiScale3DDeformableAttnWeightUpdateFunction>({r.out, r.wu}, step, value, dist, shapes, starts, loc, attn);
+    return tuple_of({out[0], out[1]});
+  }
+  return declined();
+  END_HANDLE_TH_ERRORS
+}
+PyObject *set_python_backward(PyObject *, PyObject *f) {
+  Py_INCREF(f);
+  PyObject *before = std::exchange(python_backward, f);
+  Py_XDECREF(before);
+  Py_RETURN_NONE;
 }
 
 // Where the kernels form a product of rows x width elements, sums of depth terms.  They read four neighbours of a row at a time, and take the
@@ -394,11 +640,11 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   Tensor y = at::empty(sizes, x.options());
   int rc;
   {
-    NoGil no_gil;
+    NoGil no_gil(in.locked);
     rc = api.linear(static_cast<const float *>(ptr(x)), static_cast<const float *>(ptr(w)), static_cast<const float *>(ptr(b)),
                     static_cast<float *>(ptr(y)), rows, (int)O, (int)K, stream);
   }
-  if (rc != 0) return failed("dfa3d_linear", rc);
+  if (rc != 0) return without_results(outcome("dfa3d_linear", rc));
   return THPVariable_Wrap(y);
   END_HANDLE_TH_ERRORS
 }
@@ -426,10 +672,10 @@ PyObject *linear_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   Tensor y = at::empty(sizes, THPVariable_Unpack(PyTuple_GET_ITEM(args[2], 0)).options());
   int rc;
   {
-    NoGil no_gil;
+    NoGil no_gil(in.locked);
     rc = api.linear_sum(sets, (int)n, static_cast<float *>(ptr(y)), rows, (int)K, stream);
   }
-  if (rc != 0) return failed("dfa3d_linear_sum", rc);
+  if (rc != 0) return without_results(outcome("dfa3d_linear_sum", rc));
   return THPVariable_Wrap(y);
   END_HANDLE_TH_ERRORS
 }
@@ -486,6 +732,8 @@ PyMethodDef methods[] = {
     {"score_forward", as_method(score_forward), METH_FASTCALL, nullptr},
     {"score_gradients", as_method(score_gradients), METH_FASTCALL, nullptr},
     {"pack_dist", as_method(pack_dist), METH_FASTCALL, nullptr},
+    {"call", as_method(call), METH_FASTCALL, nullptr},
+    {"set_python_backward", set_python_backward, METH_O, nullptr},
     {"linear", as_method(linear), METH_FASTCALL, nullptr},
     {"linear_sum", as_method(linear_sum), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

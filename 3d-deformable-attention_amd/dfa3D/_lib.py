@@ -18,7 +18,7 @@ LIB_PATH = os.path.join(_HERE, "libdfa3d_hip.so")
 DFA3D_F32, DFA3D_F64, DFA3D_BF16, DFA3D_BF16G = 0, 1, 2, 3
 DFA3D_FEW_POINTS = 2        # launch option `direct`
 MAX_LINEAR_SETS = 4        # DFA3D_MAX_LINEAR_SETS
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 _P, _I = ctypes.c_void_p, ctypes.c_int
 _DIMS7 = [_I] * 7      # B S M (C|D) L Q P
@@ -89,7 +89,7 @@ def _load_binding(handle):
     for another torch, whose tensors it would misread, or for another version of the library's interface."""
     try:
         module = importlib.import_module(__package__ + "._binding")
-        built_for, abi, _ = *module.built_for(), module.seen
+        built_for, abi, _ = *module.built_for(), module.call
         here = f"{torch.__version__} {torch.version.git_version}"
         if built_for != here or abi != ABI_VERSION:
             raise ImportError(f"it was built for torch {built_for} and ABI version {abi}, this is {here} and {ABI_VERSION}")
@@ -99,7 +99,13 @@ def _load_binding(handle):
                       "`python 3d-deformable-attention_amd/build.py --force` builds it", RuntimeWarning, stacklevel=3)
         return None
     module.bind({name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in _BOUND})
+    module.set_python_backward(_python_backward)
     return module
+
+
+def _python_backward(*args):
+    from . import functional
+    return functional.backward_of(*args)
 
 
 def lib():

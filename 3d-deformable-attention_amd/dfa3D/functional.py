@@ -33,7 +33,7 @@ import functools
 import torch
 from torch.autograd.function import once_differentiable
 
-from . import _ext, _lib
+from . import _ext, _lib, recording
 from .recording import OperatorFunction
 
 __all__ = [
@@ -88,6 +88,7 @@ class MultiScaleDepthScoreSampleFunction(OperatorFunction):
     """Stage 1: depth scores of the four pixels around every sampling point."""
 
     own = True
+    kind = recording.SCORE
 
     @staticmethod
     def forward(ctx, value, value_spatial_shapes, value_level_start_index, sampling_locations, im2col_step):
@@ -114,6 +115,7 @@ class WeightedMultiScaleDeformableAttnFunction(OperatorFunction):
     """Stage 2: multi-scale deformable attention with every corner weighted by its depth score."""
 
     own = True
+    kind = recording.STAGE2
 
     @staticmethod
     def forward(ctx, value, value_spatial_shapes, value_level_start_index, sampling_locations,
@@ -145,6 +147,7 @@ class MultiScaleDeformableAttnFunction(OperatorFunction):
     (BEVFormer_DFA3D/projects/mmdet3d_plugin/bevformer/modules/multi_scale_deformable_attn_function.py:90-163)."""
 
     own = True
+    kind = recording.PLAIN
 
     @staticmethod
     def forward(ctx, value, value_spatial_shapes, value_level_start_index, sampling_locations,
@@ -173,6 +176,7 @@ class MultiScale3DDeformableAttnFunction(OperatorFunction):
     """One-stage DFA3D: returns ``(output, depth_score)``."""
 
     own = True
+    kind = recording.FUSED
 
     @staticmethod
     def forward(ctx, value, value_dpt_dist, value_spatial_shapes, value_level_start_index,
@@ -218,6 +222,7 @@ class MultiScale3DDeformableAttnWeightUpdateFunction(OperatorFunction):
     forward packs for itself when that pays."""
 
     own = True
+    kind = recording.WEIGHT_UPDATE
 
     @staticmethod
     def forward(ctx, value, value_dpt_dist, value_spatial_shapes, value_level_start_index,
@@ -254,6 +259,28 @@ class MultiScale3DDeformableAttnWeightUpdateFunction(OperatorFunction):
         return grad_value, grad_value_dpt_dist, None, None, grad_sampling_loc, grad_attn_weight, None, None
 
 
+class _Saved:
+    """What a Function's backward asks of its context, from a native node (whose calls carry no launch options)."""
+
+    launch_fields = {}
+
+    def __init__(self, saved_tensors, im2col_step):
+        self.saved_tensors, self.im2col_step = saved_tensors, im2col_step
+
+
+_OF_KIND = {cls.kind: cls for cls in (MultiScaleDepthScoreSampleFunction, WeightedMultiScaleDeformableAttnFunction, MultiScaleDeformableAttnFunction,
+                                      MultiScale3DDeformableAttnFunction, MultiScale3DDeformableAttnWeightUpdateFunction)}
+
+
+def backward_of(kind, im2col_step, saved, grads):
+    """A Function's backward for a native node -> gradients of the tensors it saved (the Function's first operands)."""
+    if kind in (recording.SCORE, recording.STAGE2, recording.PLAIN) and grads[0] is None:
+        like, loc = saved[0], saved[3]
+        B, Q, M, L, P = loc.shape[:5]
+        grads = (like.new_zeros((B, Q, M, L, P, 4) if kind == recording.SCORE else (B, Q, M * like.shape[3])),)
+    return tuple(_OF_KIND[kind].backward(_Saved(saved, im2col_step), *grads)[:len(saved)])
+
+
 def _autocast_twin(base, name, doc):
     """Subclass whose forward casts floating inputs to float32 under ``torch.autocast`` (what the
     reference's ``custom_fwd(cast_inputs=torch.float32)`` twins do) and runs outside autocast."""
@@ -270,7 +297,7 @@ def _autocast_twin(base, name, doc):
             return base.backward(ctx, *grads)
 
     return type(name, (base,), {"forward": staticmethod(forward), "backward": staticmethod(backward),
-                                "own": True, "__doc__": doc, "__module__": __name__})
+                                "own": True, "kind": base.__dict__["kind"], "__doc__": doc, "__module__": __name__})
 
 
 _FP32_DOC = "Autocast-safe twin: inputs are cast to float32 when autocast is on."

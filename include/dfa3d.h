@@ -296,7 +296,7 @@ int dfa3d_linear_grad(const float *x, const float *grad_out, float *grad_weight,
 const char *dfa3d_last_error(void);
 
 /* Library ABI version (bumped when a signature changes). */
-#define DFA3D_ABI_VERSION 9
+#define DFA3D_ABI_VERSION 10
 int dfa3d_abi_version(void);
 
 #ifdef __cplusplus
