@@ -22,6 +22,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
+#include <algorithm>
 #include <initializer_list>
 #include <limits>
 #include <stdexcept>
@@ -612,9 +613,12 @@ PyObject *set_python_backward(PyObject *, PyObject *f) {
 // 19, 8; sums of 512 by 256 19, 22; of 2048 by 256 41, 51 to 89; of 1024 by 1024 72, 58; 20000 rows of 512 by 512 98, 70; of 2048 by 256 165, 145; 100000 of
 // 256 by 256 123, 93.  The 18 to 19 are the library call's host time, which bounds it up to some 5000 rows; on the device alone (captured in a graph)
 // 100 rows of 256 by 256 30, 8, 625 rows 5.5, 8.0, 1500 rows 5.6, 8.2, 4096 rows 10, 9; of 256 by 64 4096 rows 5.4, 7.8, 10000 rows 7.3, 8.2.
-bool product_applies(int64_t rows, int64_t width, int64_t depth) {
+// Where several layers' terms are summed (of_several), the library takes a call each and their sums: up to 1024 terms in all the kernel whatever the rows. Three
+// layers of 512, 256 and 256 columns, library and kernel, 64 rows 74, 35; 1000 67, 36 (on the device alone 21, 36); 4000 67, 43 (42, 43); 16000 95, 69; of 256,
+// 128 and 128 67, 21 (18, 21); 32, 24 at 4000; four of 512 1000 rows 92, 74 (40, 74).
+bool product_applies(int64_t rows, int64_t width, int64_t depth, bool of_several = false) {
   return width > 0 && depth > 0 && width <= 4096 && depth <= 4096 && width % 2 == 0 && depth % 4 == 0 && rows > 0 && rows <= (int64_t(1) << 31) &&
-         (depth <= 256 || rows * width >= (int64_t(1) << 22));
+         (depth <= 256 || of_several || rows * width >= (int64_t(1) << 22));
 }
 // pairs of a flat tuple, 0 where it is none of 1 to as many pairs as a call takes
 Py_ssize_t pairs_of(PyObject *o) {
@@ -656,7 +660,7 @@ PyObject *linear_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   const Py_ssize_t n = pairs_of(args[2]);
   if (n == 0 || at::autocast::is_autocast_enabled(at::kCUDA) || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer)) return declined();
   dfa3d_linear_set sets[DFA3D_MAX_LINEAR_SETS];
-  int64_t K = 0, rows = 0;
+  int64_t K = 0, rows = 0, depth = 0, deepest = 0;
   std::vector<int64_t> sizes;
   for (Py_ssize_t i = 0; i < n; ++i) {
     const Tensor &g = in.need(PyTuple_GET_ITEM(args[2], 2 * i)), &w = in.need(PyTuple_GET_ITEM(args[2], 2 * i + 1));
@@ -666,9 +670,13 @@ PyObject *linear_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     auto shape = g.sizes().vec();
     shape.back() = w.size(1);
     if (i == 0) { sizes = shape; K = w.size(1); rows = g.numel() / w.size(0); }
-    if (shape != sizes || !product_applies(rows, K, w.size(0))) return declined();
+    if (shape != sizes) return declined();
+    depth += w.size(0);
+    deepest = std::max(deepest, w.size(0));
+    if (w.size(0) % 4 != 0) return declined();
     sets[i] = dfa3d_linear_set{static_cast<const float *>(ptr(w)), static_cast<const float *>(ptr(g)), static_cast<int>(w.size(0))};
   }
+  if (!product_applies(rows, K, deepest, n > 1 && depth <= 1024)) return declined();
   Tensor y = at::empty(sizes, THPVariable_Unpack(PyTuple_GET_ITEM(args[2], 0)).options());
   int rc;
   {

@@ -24,16 +24,13 @@ def ordinary(*tensors):
             and torch.autograd.forward_ad._current_level < 0)
 
 
-# Fewer rows than this: the library product is as fast and there is one launch less.
-_MIN_ROWS = 4096
-
-
 def _widths_apply(O, K):
     """Where the kernel takes the gradient of an O x K weight: even widths of up to 2048 whose product is at most 2^20.  The
     library's product is slow where the result has few tiles, and has caught up at about 64 tiles of 128 x 128.  Times as
     fast as the library's product and column sum, 4096 / 20000 / 100000 rows: 256 x 512 1.5 / 4.5 / 4.1, 256 x 2048 1.2 /
     1.8 / 1.3, 512 x 1024 1.2 / 1.0 / 1.0, 1024 x 1024 1.05 / 0.95 / 1.1; beyond, 1024 x 2048 0.89 / 0.87 / 0.87, 2048 x 2048
-    0.84 / 0.87 / 0.85, 64 x 4096 1.1 / 0.9 / 0.8.  The rule also bounds the workspace, 512 to 1024 tiles of 64 KB (2048 x
+    0.84 / 0.87 / 0.85, 64 x 4096 1.1 / 0.9 / 0.8.  Fewer rows, library and kernels, us a call: 256 x 256 16 rows 25 / 13, 128 41 / 13,
+    1000 235 / 14, 2000 28 / 20; 512 x 256 24 / 13, 24 / 13, 28 / 15, 29 / 22 (on the device alone 6.6 / 10 at 16 rows, else as good or better).  The rule also bounds the workspace, 512 to 1024 tiles of 64 KB (2048 x
     2048 would take 134 MB, 16384 x 16384 8.6 GB)."""
     return O % 2 == 0 and K % 2 == 0 and max(O, K) <= 2048 and O * K <= 2 ** 20
 
@@ -169,7 +166,7 @@ class _SharedRowsFunction(Function):
 def _applies(x, *layers):
     """Float32 rows on the GPU in ordinary reverse-mode training, for layers that all have a bias."""
     return (not torch.compiler.is_compiling() and torch.is_grad_enabled() and x.dim() >= 2
-            and _MIN_ROWS <= x.numel() // max(x.shape[-1], 1) <= 2 ** 31
+            and 0 < x.numel() // max(x.shape[-1], 1) <= 2 ** 31
             and all(l.bias is not None and l.weight.requires_grad and _widths_apply(*l.weight.shape) for l in layers)
             and ordinary(x, *(t for l in layers for t in (l.weight, l.bias))))
 
