@@ -471,6 +471,16 @@ int dfa3d_rebatch_gather_padded(const void *src, long long cam_stride, long long
                         dtype, pad, stream);
 }
 
+int dfa3d_rebatch_queries(const void *src, const void *plus, const void *ref, const int32_t *index, void *dst, void *ref_dst, int bs, int cams,
+                          int max_len, int Nq, int E, int R, int dtype, double ref_pad, void *stream) {
+  const char *fn = "dfa3d_rebatch_queries";
+  if (int rc = check_rebatch(fn, bs, cams, max_len, Nq, E, dtype)) return rc;
+  if (R <= 0) return fail(DFA3D_EINVAL, "%s: dimensions must be positive (R=%d)", fn, R);
+  REQUIRE_PTR(fn, src); REQUIRE_PTR(fn, ref); REQUIRE_PTR(fn, index); REQUIRE_PTR(fn, dst); REQUIRE_PTR(fn, ref_dst);
+  const dfa3d::RebatchQueries a = {src, plus, ref, index, dst, ref_dst, bs, cams, max_len, Nq, E, R, ref_pad};
+  return hip_result(dfa3d::launch_rebatch_queries(a, dtype, (hipStream_t)stream), fn);
+}
+
 int dfa3d_rebatch_combine(const void *src, const int32_t *pos, const void *scale, void *dst, int bs, int cams,
                           int max_len, int Nq, int E, int dtype, void *stream) {
   const char *fn = "dfa3d_rebatch_combine";
@@ -495,6 +505,16 @@ int dfa3d_camera_hits(const uint8_t *mask, uint8_t *hit, float *scale, int cams,
   return hip_result(dfa3d::launch_camera_hits(mask, hit, scale, cams, bs, Nq, Z, (hipStream_t)stream), fn);
 }
 
+int dfa3d_camera_hits_counted(const uint8_t *mask, uint8_t *hit, float *scale, int32_t *counts, int parts, int cams, int bs, int Nq, int Z,
+                              void *stream) {
+  const char *fn = "dfa3d_camera_hits_counted";
+  if (int rc = check_cameras(fn, cams, bs, Nq, Z)) return rc;
+  if (cams > 1024) return fail(DFA3D_ERANGE, "%s: at most 1024 cameras", fn);
+  if (parts <= 0) return fail(DFA3D_EINVAL, "%s: parts must be positive", fn);
+  REQUIRE_PTR(fn, mask); REQUIRE_PTR(fn, hit); REQUIRE_PTR(fn, scale); REQUIRE_PTR(fn, counts);
+  return hip_result(dfa3d::launch_camera_hits_counted(mask, hit, scale, counts, parts, cams, bs, Nq, Z, (hipStream_t)stream), fn);
+}
+
 int dfa3d_camera_count(const uint8_t *hit, int32_t *totals, int cams, int Nq, void *stream) {
   const char *fn = "dfa3d_camera_count";
   if (int rc = check_cameras(fn, cams, 1, Nq, 1)) return rc;
@@ -508,7 +528,14 @@ int dfa3d_camera_index(const uint8_t *hit, const int32_t *totals, int32_t *index
   if (int rc = check_cameras(fn, cams, 1, Nq, 1)) return rc;
   if (max_len <= 0 || max_len > Nq) return fail(DFA3D_EINVAL, "%s: max_len must be in [1, Nq]", fn);
   REQUIRE_PTR(fn, hit); REQUIRE_PTR(fn, totals); REQUIRE_PTR(fn, index); REQUIRE_PTR(fn, pos);
-  return hip_result(dfa3d::launch_camera_index(hit, totals, index, pos, cams, Nq, max_len, (hipStream_t)stream), fn);
+  return hip_result(dfa3d::launch_camera_index(hit, index, pos, cams, Nq, max_len, (hipStream_t)stream), fn);
+}
+
+int dfa3d_level_table(const int64_t *shapes, int64_t *shapes3, int L, int D, void *stream) {
+  const char *fn = "dfa3d_level_table";
+  if (L <= 0) return fail(DFA3D_EINVAL, "%s: dimensions must be positive (L=%d)", fn, L);
+  REQUIRE_PTR(fn, shapes); REQUIRE_PTR(fn, shapes3);
+  return hip_result(dfa3d::launch_level_table(shapes, shapes3, L, D, (hipStream_t)stream), fn);
 }
 
 static int check_locations(const char *fn, long long rows, int M, int L, int P, int Z) {

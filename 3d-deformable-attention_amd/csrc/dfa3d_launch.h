@@ -153,10 +153,23 @@ hipError_t launch_rebatch_gather(const void *src, long long cam_stride, long lon
 hipError_t launch_rebatch_combine(const void *src, const int *pos, const void *scale, void *dst, int bs, int cams,
                                   int max_len, int Nq, int E, int dtype, hipStream_t stream);
 
+struct RebatchQueries {                // src, plus (or nullptr) (bs, Nq, E) and ref (cams, bs, Nq, R) to dst and ref_dst (bs, cams, max_len, ...)
+  const void *src, *plus, *ref;
+  const int *index;
+  void *dst, *ref_dst;
+  int bs, cams, max_len, Nq, E, R;
+  double ref_pad;
+};
+hipError_t launch_rebatch_queries(const RebatchQueries &a, int dtype, hipStream_t stream);
+
 hipError_t launch_camera_hits(const uint8_t *mask, uint8_t *hit, float *scale, int cams, int bs, int Nq, int Z, hipStream_t stream);
 hipError_t launch_camera_count(const uint8_t *hit, int *totals, int cams, int Nq, hipStream_t stream);
-hipError_t launch_camera_index(const uint8_t *hit, const int *totals, int *index, int *pos, int cams, int Nq, int max_len,
-                               hipStream_t stream);
+hipError_t launch_camera_hits_counted(const uint8_t *mask, uint8_t *hit, float *scale, int *counts, int parts, int cams, int bs, int Nq, int Z,
+                                      hipStream_t stream);
+hipError_t launch_camera_index(const uint8_t *hit, int *index, int *pos, int cams, int Nq, int max_len, hipStream_t stream);
+
+// (L, 2) to (L, 3) with D as the third extent (dfa3d_locations.hip).
+hipError_t launch_level_table(const int64_t *shapes, int64_t *shapes3, int L, int D, hipStream_t stream);
 
 // Sampling locations of a layer and their gradients (dfa3d_locations.hip).
 hipError_t launch_locations(const float *uv, const float *dz, const float *ref, const int64_t *shapes3, float *loc, long long rows,

@@ -56,6 +56,14 @@ __global__ __launch_bounds__(256) void locations_grad_kernel(const float *__rest
   }
 }
 
+__global__ __launch_bounds__(64) void level_table_kernel(const int64_t *__restrict__ shapes, int64_t *__restrict__ shapes3, int L, int D) {
+  for (int i = threadIdx.x; i < 3 * L; i += 64) shapes3[i] = i % 3 == 2 ? D : shapes[i / 3 * 2 + i % 3];
+}
+
+hipError_t launch_level_table(const int64_t *shapes, int64_t *shapes3, int L, int D, hipStream_t stream) {
+  hipLaunchKernelGGL(level_table_kernel, dim3(1), dim3(64), 0, stream, shapes, shapes3, L, D);
+  return hipGetLastError();
+}
 hipError_t launch_locations(const float *uv, const float *dz, const float *ref, const int64_t *shapes3, float *loc, long long rows,
                             int M, int L, int P, int Z, hipStream_t stream) {
   hipLaunchKernelGGL(locations_kernel, dim3((unsigned)((rows + kLocRows - 1) / kLocRows)), dim3(256), 0, stream, uv, dz, ref,

@@ -54,10 +54,13 @@ SIGNATURES = {
     "dfa3d_rebatch_gather": [_P, ctypes.c_longlong, ctypes.c_longlong, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "dfa3d_rebatch_gather_padded": [_P, ctypes.c_longlong, ctypes.c_longlong, _P, _P, _P, _I, _I, _I, _I, _I, _I,
                                     ctypes.c_double, _P],
+    "dfa3d_rebatch_queries": [_P] * 6 + [_I] * 7 + [ctypes.c_double, _P],
     "dfa3d_rebatch_combine": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "dfa3d_camera_hits": [_P] * 3 + [_I] * 4 + [_P],
+    "dfa3d_camera_hits_counted": [_P] * 4 + [_I] * 5 + [_P],
     "dfa3d_camera_count": [_P, _P, _I, _I, _P],
     "dfa3d_camera_index": [_P] * 4 + [_I] * 3 + [_P],
+    "dfa3d_level_table": [_P, _P, _I, _I, _P],
     "dfa3d_locations": [_P] * 5 + [ctypes.c_longlong] + [_I] * 4 + [_P],
     "dfa3d_locations_grad": [_P] * 4 + [ctypes.c_longlong] + [_I] * 3 + [_P],
     "dfa3d_linear": [_P] * 4 + [ctypes.c_longlong, _I, _I, _P],

@@ -13,12 +13,12 @@ from .. import _lib
 __all__ = ["Projection", "projections"]
 
 
-def ordinary(*tensors):
-    """Plain float32 tensors on one GPU, outside autocast, functorch transforms, dispatch modes, forward-mode derivatives,
+def ordinary(*tensors, dtype=torch.float32):
+    """Plain tensors of ``dtype`` on one GPU, outside autocast, functorch transforms, dispatch modes, forward-mode derivatives,
     tracing and compilation: what this package's kernels may stand in for torch operations on."""
     return (not torch.compiler.is_compiling() and not torch.jit.is_tracing() and not torch.is_autocast_enabled()
             and torch._C._len_torch_dispatch_stack() == 0
-            and all(type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.dtype == torch.float32 and not t.is_neg()
+            and all(type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.dtype == dtype and not t.is_neg()
                     and t.device == tensors[0].device for t in tensors)
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0)

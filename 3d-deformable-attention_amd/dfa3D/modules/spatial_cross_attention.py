@@ -7,13 +7,22 @@ re-batching (python loops over batch x cameras in the reference, :716-722 and :7
 import torch
 from torch import nn
 
-from ..rebatch import RebatchCombineFunction, RebatchGatherFunction, camera_count, camera_hits, camera_index, rebatch_gather
+from ..rebatch import RebatchCombineFunction, RebatchQueriesFunction, camera_hits_counted, camera_index
 from .ms_deform_attn_3d import MSDeformableAttention3D_DFA3D
 from .projection import Projection, no_hooks
 
 __all__ = ["SpatialCrossAttention_DFA3D"]
 
+_PLAIN = (torch.Tensor, nn.Parameter)
 _OUTSIDE = -64.0        # a normalised coordinate: 64 maps away
+
+
+def _added_as_gathered(query, query_pos):
+    """Whether the gather may add ``query_pos`` to the queries that it reads: two plain tensors that lie alike.  What is broadcast, laid out otherwise,
+    of another type or somebody's subclass is added by torch."""
+    return (type(query) in _PLAIN and type(query_pos) in _PLAIN and query.is_cuda and query_pos.device == query.device
+            and query_pos.dtype == query.dtype and query_pos.shape == query.shape and query.is_contiguous() and query_pos.is_contiguous()
+            and not (query.is_neg() or query_pos.is_neg()))
 
 
 class SpatialCrossAttention_DFA3D(nn.Module):
@@ -75,18 +84,17 @@ class SpatialCrossAttention_DFA3D(nn.Module):
         if value is None:
             value = key
         inp_residual = query if residual is None else residual
-        if query_pos is not None:
-            query = query + query_pos
+        if query_pos is not None and not _added_as_gathered(query, query_pos):
+            query, query_pos = query + query_pos, None
         bs, num_query, _ = query.shape
         Z = reference_points_cam.size(3)
         cams = self.num_cams
 
-        hit, scale = camera_hits(bev_mask)                                       # (cams, Nq), (bs, Nq)
+        hit, scale, counted = camera_hits_counted(bev_mask)                      # (cams, Nq), (bs, Nq)
         # The host waits for the lists' length, and the device has what does not need it to do meanwhile.  Inference of the
         # layer of the small model 292 -> 277 us against waiting behind that work; two samples of six cameras, 90 x 134 and
         # 45 x 67 maps, 51 x 51 queries 552 us in the order of the operations, 562 behind that work, 492 so.
-        counted = camera_count(hit)
-        ref = reference_points_cam.to(query.dtype).reshape(cams, bs, num_query, Z * 3).contiguous()
+        ref = reference_points_cam.to(query.dtype).reshape(cams, bs, num_query, Z * 3).contiguous().detach()
         keys = key.shape[1]
         key = key.permute(2, 0, 1, 3).reshape(bs * cams, keys, self.embed_dims)
         value = value.permute(2, 0, 1, 3).reshape(bs * cams, keys, self.embed_dims)
@@ -96,13 +104,13 @@ class SpatialCrossAttention_DFA3D(nn.Module):
         if ours and attention.batch_first and no_hooks(attention):
             kwargs["value_side"] = attention.value_side(value, value_dpt_dist, spatial_shapes)
         index, pos, max_len = camera_index(hit, counted)
-        queries_rebatch = RebatchGatherFunction.apply(query, index, pos)         # (bs, cams, max_len, E)
         # The rows that pad the shorter cameras' lists are never read back.  With reference points of zero, as the reference
         # pads them, all their samples fall on the map's first pixels, which a backward feels: every point of a pass on
         # one cell and depth (base layer: tile kernel 1.31 against 1.25 ms, training step 4.27 against 4.15).  Far outside the map the operator
         # skips them.  Another attention module gets the zeros.
         pad = _OUTSIDE if ours else 0.0
-        reference_points_rebatch = rebatch_gather(ref, index, per_camera=True, pad=pad)     # (bs, cams, max_len, Z*3)
+        queries_rebatch, reference_points_rebatch = RebatchQueriesFunction.apply(       # (bs, cams, max_len, E), (bs, cams, max_len, Z*3)
+            query, query_pos, ref, index, pos, pad)
         L = index.shape[1]
 
         queries, update_weight = attention(

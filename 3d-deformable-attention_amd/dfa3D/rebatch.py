@@ -9,7 +9,8 @@ from torch.autograd.function import once_differentiable
 from . import _lib
 from .recording import OperatorFunction
 
-__all__ = ["camera_hits", "camera_count", "camera_index", "rebatch_gather", "rebatch_combine", "RebatchGatherFunction", "RebatchCombineFunction"]
+__all__ = ["camera_hits", "camera_count", "camera_hits_counted", "camera_index", "rebatch_gather", "rebatch_queries", "rebatch_combine",
+           "RebatchGatherFunction", "RebatchQueriesFunction", "RebatchCombineFunction"]
 
 
 def camera_count(hit):
@@ -19,15 +20,43 @@ def camera_count(hit):
     cams, Nq = hit.shape
     if not (hit.is_cuda and hit.dtype == torch.bool and hit.is_contiguous() and 0 < cams <= 65535 and 0 < Nq <= 2 ** 30):
         return None
-    totals = torch.empty(cams, dtype=torch.int32, device=hit.device)
-    on_host = torch.empty(cams, dtype=torch.int32, device="cpu", pin_memory=True)      # (whatever the default device)
+    totals = torch.empty(cams, 1, dtype=torch.int32, device=hit.device)
     with _lib.on_device(hit.device):
         rc = _lib.lib().dfa3d_camera_count(_lib.ptr(hit), _lib.ptr(totals), cams, Nq, _lib.stream_of(hit))
         _lib.check(rc, "dfa3d_camera_count")
-        on_host.copy_(totals, non_blocking=True)
-        done = torch.cuda.Event()
-        done.record()
-    return totals, on_host, done
+        return _on_their_way(totals)
+
+
+def _on_their_way(counts):
+    """``counts`` (cams, parts) on the GPU, the same on the host, and the event after which the host has them."""
+    on_host = torch.empty(counts.shape, dtype=torch.int32, device="cpu", pin_memory=True)      # (whatever the default device)
+    on_host.copy_(counts, non_blocking=True)
+    done = torch.cuda.Event()
+    done.record()
+    return counts, on_host, done
+
+
+# Workgroups that count, 1024 queries each at a time, and up to how many queries of all batch elements they count as they mark the hits; with more of them,
+# workgroups that mark alone are as many as there are queries for.
+_PARTS, _COUNTED_QUERIES = 64, 2 ** 18
+
+
+def camera_hits_counted(bev_mask):
+    """``camera_hits(bev_mask)`` and ``camera_count`` of its first result, in one launch where both are the kernels' and queries are not many."""
+    cams, bs, Nq, Z = bev_mask.shape
+    if not (_hits_by_kernel(bev_mask) and cams <= 1024 and bs * Nq <= _COUNTED_QUERIES):
+        hit, scale = camera_hits(bev_mask)
+        return hit, scale, camera_count(hit)
+    mask = bev_mask.contiguous()
+    parts = min(-(-bs * Nq // 1024), _PARTS)
+    hit = torch.empty(cams, Nq, dtype=torch.bool, device=mask.device)
+    scale = torch.empty(bs, Nq, dtype=torch.float32, device=mask.device)
+    counts = torch.empty(cams, parts, dtype=torch.int32, device=mask.device)
+    with _lib.on_device(mask.device):
+        rc = _lib.lib().dfa3d_camera_hits_counted(_lib.ptr(mask), _lib.ptr(hit), _lib.ptr(scale), _lib.ptr(counts), parts, cams, bs, Nq, Z,
+                                                  _lib.stream_of(mask))
+        _lib.check(rc, "dfa3d_camera_hits_counted")
+        return hit, scale, _on_their_way(counts)
 
 
 def camera_index(hit, counted=None):
@@ -56,11 +85,17 @@ def _camera_index_on_gpu(hit, totals, on_host, done):
     pos = torch.empty(cams, Nq, dtype=torch.int32, device=dev)
     with _lib.on_device(dev):
         done.synchronize()                                          # waits for the device
-        max_len = max(on_host.tolist())
+        max_len = max(map(sum, on_host.tolist()))
         index = torch.empty(cams, max(max_len, 1), dtype=torch.int32, device=dev)
         _lib.check(lib.dfa3d_camera_index(_lib.ptr(hit), _lib.ptr(totals), _lib.ptr(index), _lib.ptr(pos), cams, Nq,
                                           max(max_len, 1), _lib.stream_of(hit)), "dfa3d_camera_index")
     return index, pos, max_len
+
+
+def _hits_by_kernel(bev_mask):
+    cams, _, Nq, _ = bev_mask.shape
+    return (bev_mask.is_cuda and bev_mask.dtype == torch.bool and bev_mask.numel() and cams <= 65535 and Nq <= 2 ** 30
+            and torch.get_default_dtype() == torch.float32)            # what the kernel writes
 
 
 def camera_hits(bev_mask):
@@ -68,8 +103,7 @@ def camera_hits(bev_mask):
     camera, and ``scale`` (bs, Nq) of the default dtype, one over the number of cameras with any anchor of a query (at
     least 1)."""
     cams, bs, Nq, Z = bev_mask.shape
-    if (bev_mask.is_cuda and bev_mask.dtype == torch.bool and bev_mask.numel() and cams <= 65535 and Nq <= 2 ** 30
-            and torch.get_default_dtype() == torch.float32):           # what the kernel writes
+    if _hits_by_kernel(bev_mask):
         mask = bev_mask.contiguous()
         hit = torch.empty(cams, Nq, dtype=torch.bool, device=mask.device)
         scale = torch.empty(bs, Nq, dtype=torch.float32, device=mask.device)
@@ -122,6 +156,28 @@ def rebatch_gather(src, index, scale=None, per_camera=False, pad=0.0):
     return dst
 
 
+def rebatch_queries(src, plus, ref, index, ref_pad=0.0):
+    """``src`` and ``plus`` (bs, Nq, E; or None), ``ref`` (cams, bs, Nq, R) -> (bs, cams, max_len, E) and (bs, cams, max_len, R): what
+    ``rebatch_gather(src + plus, index)`` and ``rebatch_gather(ref, index, per_camera=True, pad=ref_pad)`` give."""
+    for t, name, dtype in ((src, "src", None), (plus, "plus", src.dtype), (ref, "ref", src.dtype), (index, "index", torch.int32)):
+        if t is not None:
+            _check(t, name, dtype)
+    cams, max_len = index.shape
+    if src.dim() != 3 or ref.dim() != 4 or tuple(ref.shape[:3]) != (cams, *src.shape[:2]) or (plus is not None and plus.shape != src.shape):
+        raise RuntimeError(f"src and plus must be (bs, Nq, E) and ref (cams, bs, Nq, R), got {tuple(src.shape)}, "
+                           f"{None if plus is None else tuple(plus.shape)}, {tuple(ref.shape)}")
+    bs, Nq, E = src.shape
+    R = ref.shape[3]
+    dst, ref_dst = src.new_empty(bs, cams, max_len, E), src.new_empty(bs, cams, max_len, R)
+    if dst.numel() == 0 or ref_dst.numel() == 0:
+        return rebatch_gather(src if plus is None else src + plus, index), rebatch_gather(ref, index, per_camera=True, pad=ref_pad)
+    with _lib.on_device(src.device):
+        rc = _lib.lib().dfa3d_rebatch_queries(_lib.ptr(src), _lib.ptr(plus), _lib.ptr(ref), _lib.ptr(index), _lib.ptr(dst), _lib.ptr(ref_dst),
+                                              bs, cams, max_len, Nq, E, R, _lib.dtype_code(src), ref_pad, _lib.stream_of(src))
+    _lib.check(rc, "dfa3d_rebatch_queries")
+    return dst, ref_dst
+
+
 def rebatch_combine(src, pos, scale=None):
     """``src`` (bs, cams, max_len, E) -> (bs, Nq, E): row [j, q] = scale[j, q] * sum over the cameras i that see q
     of src[j, i, pos[i, q]]."""
@@ -162,6 +218,29 @@ class RebatchGatherFunction(OperatorFunction):
     def backward(ctx, grad):
         pos, = ctx.saved_tensors
         return rebatch_combine(grad.contiguous(), pos), None, None
+
+
+class RebatchQueriesFunction(OperatorFunction):
+    """``apply(src, plus or None, ref, index, pos, ref_pad)``: ``rebatch_queries``, differentiable in ``src`` and ``plus``."""
+
+    own = True
+
+    @staticmethod
+    def forward(ctx, src, plus, ref, index, pos, ref_pad):
+        ctx.save_for_backward(pos)
+        ctx.set_materialize_grads(False)
+        queries, refs = rebatch_queries(src.contiguous(), plus, ref, index, ref_pad)
+        ctx.mark_non_differentiable(refs)
+        return queries, refs
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad, _):
+        if grad is None:
+            return (None,) * 6
+        pos, = ctx.saved_tensors
+        grad = rebatch_combine(grad.contiguous(), pos)
+        return tuple(grad if want else None for want in ctx.needs_input_grad[:2]) + (None,) * 4
 
 
 class RebatchCombineFunction(OperatorFunction):

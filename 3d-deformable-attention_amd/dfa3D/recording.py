@@ -21,6 +21,9 @@ class _Notes:
     def set_materialize_grads(self, value):
         pass
 
+    def mark_non_differentiable(self, *results):
+        pass
+
 
 class OperatorFunction(Function):
     """A Function whose ``apply`` is its ``forward`` where gradients are off, and one call of the binding module, node and all, where that knows

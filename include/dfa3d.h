@@ -246,6 +246,10 @@ int dfa3d_rebatch_gather(const void *src, long long cam_stride, long long batch_
 int dfa3d_rebatch_gather_padded(const void *src, long long cam_stride, long long batch_stride, const int32_t *index,
                                 const void *scale, void *dst, int bs, int cams, int max_len, int Nq, int E, int dtype,
                                 double pad, void *stream);
+/* What a cross-attention layer gathers, in one launch: dst[j,i,k,:] = src[j,q,:] + plus[j,q,:] (plus may be NULL), zeros for padding, and
+ * ref_dst[j,i,k,:] = ref[i,j,q,:], ref_pad for padding; src and plus (bs, Nq, E), ref (cams, bs, Nq, R). */
+int dfa3d_rebatch_queries(const void *src, const void *plus, const void *ref, const int32_t *index, void *dst, void *ref_dst, int bs, int cams,
+                          int max_len, int Nq, int E, int R, int dtype, double ref_pad, void *stream);
 int dfa3d_rebatch_combine(const void *src, const int32_t *pos, const void *scale, void *dst, int bs, int cams,
                           int max_len, int Nq, int E, int dtype, void *stream);
 
@@ -254,12 +258,19 @@ int dfa3d_rebatch_combine(const void *src, const int32_t *pos, const void *scale
  * hits:  hit[i,q] = any anchor of query q of the FIRST batch element; scale[j,q] = 1 / max(cameras that see query q of
  *        batch element j, 1).
  * count: totals[i] = number of queries camera i hits.
+ * hits_counted: hits, and counts (cams, parts), whose rows add up to the totals; at most 1024 cameras.  A part is a workgroup, 1024 queries at a
+ *        time.
  * index: index (cams, max_len) lists the queries of each camera in ascending order, padded with -1, and pos (cams, Nq) is
- *        its inverse (-1: not seen); 1 <= max_len <= Nq, the largest of totals (or 1). */
+ *        its inverse (-1: not seen); 1 <= max_len <= Nq, the largest of totals (or 1).  totals: its place is kept, its values are not read. */
 int dfa3d_camera_hits(const uint8_t *mask, uint8_t *hit, float *scale, int cams, int bs, int Nq, int Z, void *stream);
+int dfa3d_camera_hits_counted(const uint8_t *mask, uint8_t *hit, float *scale, int32_t *counts, int parts, int cams, int bs, int Nq, int Z,
+                              void *stream);
 int dfa3d_camera_count(const uint8_t *hit, int32_t *totals, int cams, int Nq, void *stream);
 int dfa3d_camera_index(const uint8_t *hit, const int32_t *totals, int32_t *index, int32_t *pos, int cams, int Nq, int max_len,
                        void *stream);
+
+/* shapes (L, 2) = (H, W) to shapes3 (L, 3) = (H, W, D), both on the device. */
+int dfa3d_level_table(const int64_t *shapes, int64_t *shapes3, int L, int D, void *stream);
 
 /* Sampling locations of a cross-attention layer in float32: loc (rows, M, L, P, 3) = (uv / (W, H), dz / D) of the level plus
  * ref[row, p % Z], with uv (rows, M, L, P, 2), dz (rows, M, L, P), ref (rows, Z, 3) and shapes3 (L, 3) = (H, W, D) on the
