@@ -570,12 +570,18 @@ static int check_linear(const char *fn, long long N, int O, int K) {
   return 0;
 }
 
-int dfa3d_linear(const float *x, const float *weight, const float *bias, float *y, long long N, int O, int K, void *stream) {
-  const char *fn = "dfa3d_linear";
+static int linear(const char *fn, const float *x, const float *weight, const float *bias, const float *addend, float *y, long long N, int O, int K,
+                  void *stream) {
   if (int rc = check_linear(fn, N, O, K)) return rc;
   if ((K & 3) != 0) return fail(DFA3D_EINVAL, "%s: K must be a multiple of four (K=%d)", fn, K);
   REQUIRE_PTR(fn, x); REQUIRE_PTR(fn, weight); REQUIRE_PTR(fn, y);
-  return hip_result(dfa3d::launch_linear(x, weight, bias, y, N, O, K, (hipStream_t)stream), fn);
+  return hip_result(dfa3d::launch_linear(x, weight, bias, addend, y, N, O, K, (hipStream_t)stream), fn);
+}
+int dfa3d_linear(const float *x, const float *weight, const float *bias, float *y, long long N, int O, int K, void *stream) {
+  return linear("dfa3d_linear", x, weight, bias, nullptr, y, N, O, K, stream);
+}
+int dfa3d_linear_add(const float *x, const float *weight, const float *bias, const float *addend, float *y, long long N, int O, int K, void *stream) {
+  return linear("dfa3d_linear_add", x, weight, bias, addend, y, N, O, K, stream);
 }
 
 int dfa3d_linear_sum(const dfa3d_linear_set *layers, int n_layers, float *y, long long N, int K, void *stream) {

@@ -47,7 +47,7 @@ struct Api {
   decltype(&dfa3d_ms_depth_score_sample_backward_workspace_bytes) score_backward_workspace_bytes;
   decltype(&dfa3d_ms_depth_score_sample_backward_into) score_backward;
   decltype(&dfa3d_pack_dist) pack_dist;
-  decltype(&dfa3d_linear) linear;
+  decltype(&dfa3d_linear_add) linear_add;
   decltype(&dfa3d_linear_sum) linear_sum;
 } api;
 
@@ -628,27 +628,29 @@ Py_ssize_t pairs_of(PyObject *o) {
 bool is_float_matrix(const Tensor &t) { return t.scalar_type() == at::kFloat && t.dim() == 2; }
 bool recorded(const Tensor &t) { return t.defined() && t.requires_grad() && c10::GradMode::is_enabled(); }
 
-// linear(device, stream, x (..., K), weight (O, K), bias (O) or None) -> F.linear, not recorded, or None
+// linear(device, stream, x (..., K), weight (O, K), bias (O) or None, addend (..., O) or None) -> F.linear + addend, not recorded, or None
 PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  TAKES(5)
-  const Tensor &x = in.need(args[2]), &w = in.need(args[3]), &b = in.may_have(args[4]);
+  TAKES(6)
+  const Tensor &x = in.need(args[2]), &w = in.need(args[3]), &b = in.may_have(args[4]), &addend = in.may_have(args[5]);
   if (!in.ok || x.scalar_type() != at::kFloat || x.dim() < 2 || !is_float_matrix(w) || x.size(-1) != w.size(1) || w.size(1) == 0 ||
       (b.defined() && (b.scalar_type() != at::kFloat || !shape_is(b, {w.size(0)}))) || recorded(x) || recorded(w) || recorded(b) ||
+      (addend.defined() && (addend.scalar_type() != at::kFloat || recorded(addend))) ||
       at::autocast::is_autocast_enabled(at::kCUDA) || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer))
     return declined();
   const int64_t O = w.size(0), K = w.size(1), rows = x.numel() / K;
   if (!product_applies(rows, O, K)) return declined();
   auto sizes = x.sizes().vec();
   sizes.back() = O;
+  if (addend.defined() && addend.sizes() != at::IntArrayRef(sizes)) return declined();
   Tensor y = at::empty(sizes, x.options());
   int rc;
   {
     NoGil no_gil(in.locked);
-    rc = api.linear(static_cast<const float *>(ptr(x)), static_cast<const float *>(ptr(w)), static_cast<const float *>(ptr(b)),
-                    static_cast<float *>(ptr(y)), rows, (int)O, (int)K, stream);
+    rc = api.linear_add(static_cast<const float *>(ptr(x)), static_cast<const float *>(ptr(w)), static_cast<const float *>(ptr(b)),
+                        static_cast<const float *>(ptr(addend)), static_cast<float *>(ptr(y)), rows, (int)O, (int)K, stream);
   }
-  if (rc != 0) return without_results(outcome("dfa3d_linear", rc));
+  if (rc != 0) return without_results(outcome("dfa3d_linear_add", rc));
   return THPVariable_Wrap(y);
   END_HANDLE_TH_ERRORS
 }
@@ -721,7 +723,7 @@ PyObject *bind(PyObject *, PyObject *table) {
       !address("dfa3d_ms_depth_score_sample_forward", a.score_forward) ||
       !address("dfa3d_ms_depth_score_sample_backward_workspace_bytes", a.score_backward_workspace_bytes) ||
       !address("dfa3d_ms_depth_score_sample_backward_into", a.score_backward) || !address("dfa3d_pack_dist", a.pack_dist) ||
-      !address("dfa3d_linear", a.linear) || !address("dfa3d_linear_sum", a.linear_sum))
+      !address("dfa3d_linear_add", a.linear_add) || !address("dfa3d_linear_sum", a.linear_sum))
     return nullptr;
   api = a;
   Py_RETURN_NONE;

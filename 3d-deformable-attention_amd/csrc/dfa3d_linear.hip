@@ -266,31 +266,47 @@ __device__ __forceinline__ void whole_tile(rsrc_t a_r, int lda, int a_row0, int 
                                                       (wave & 1) * (TM / 2) + lane % 32, (wave >> 1) * (TN / 2) + lane % 32, acc);
 }
 
-// c (TM x TN tile of `ms` x `ns` valid elements, row length ldc) = acc + bias.
+// c (TM x TN tile of `ms` x `ns` valid elements, row length ldc) = acc + bias, + addend (as c) where there is one, asked for
+// 16 elements at a time (one by one, each between two stores, 2500 rows of 256 x 256 14.5 us; product 8.5, product and sum 12.3, so 9.6; 22500 of 128 x 128 17.4; 11.0,
+// 19.3, 11.5; 40000 of 512 x 512 178; 134, 168, 143).
 template <int TM, int TN>
 __device__ __forceinline__ void store_product(const f32x16 (&acc)[TM / 64][TN / 64], float *__restrict__ c, int ldc, int ms, int ns,
-                                              const float *__restrict__ bias) {
+                                              const float *__restrict__ bias, const float *__restrict__ addend = nullptr) {
   constexpr int MT = TM / 64, NT = TN / 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int first_m = (wave & 1) * MT * 32 + 4 * (lane / 32), first_n = (wave >> 1) * NT * 32 + lane % 32;
+  const rsrc_t from = make_rsrc(addend, addend != nullptr ? ((size_t)(ms - 1) * ldc + ns) * 4 : 0);      // (none: zeros)
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int n = first_n + 32 * j;
     const float add = (bias != nullptr && n < ns) ? bias[n] : 0.f;
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i) {
+      const int m0 = first_m + 32 * i;
+      float sum[16], plus[16];
+      if (addend != nullptr) {                               // uniform
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          plus[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, n < ns ? (uint32_t)((m0 + 8 * (r / 4) + r % 4) * ldc + n) * 4 : kNoRow, 0, 0));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[r] = acc[i][j][r] + add + plus[r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[r] = acc[i][j][r] + add;
+      }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int m = first_m + 32 * i + 8 * (r / 4) + r % 4;
-        if (m < ms && n < ns) c[(size_t)m * ldc + n] = acc[i][j][r] + add;
+        const int m = m0 + 8 * (r / 4) + r % 4;
+        if (m < ms && n < ns) c[(size_t)m * ldc + n] = sum[r];
       }
+    }
   }
 }
 
-// y (N, O) = x (N, K) w (O, K)^T + bias.  TM rows of one tile of TN columns per workgroup; those of the same rows run on one XCD.
+// y (N, O) = x (N, K) w (O, K)^T + bias + addend.  TM rows of one tile of TN columns per workgroup; those of the same rows run on one XCD.
 template <int TM, int TN>
 __global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
-                                                        float *__restrict__ y, long long N, int O, int K, int tiles) {
+                                                        const float *__restrict__ addend, float *__restrict__ y, long long N, int O, int K, int tiles) {
   __shared__ __align__(16) unsigned char lds[2 * (SplitOperand<TM, false>::kBytes + SplitOperand<TN, false>::kBytes)];
   __shared__ int large;
   const long long n0 = (blockIdx.x / (8 * tiles) * 8 + blockIdx.x % 8) * (long long)TM;
@@ -306,7 +322,8 @@ __global__ __launch_bounds__(256, 3) void linear_kernel(const float *__restrict_
     zero_sums(acc);
     whole_tile<TM, TN, false, false>(x_r, K, 0, 0, w_r, K, 0, 0, K, acc);
   }
-  store_product<TM, TN>(acc, y + n0 * O + o0, O, ms, ns, bias != nullptr ? bias + o0 : nullptr);
+  store_product<TM, TN>(acc, y + n0 * O + o0, O, ms, ns, bias != nullptr ? bias + o0 : nullptr,
+                        addend != nullptr ? addend + n0 * O + o0 : nullptr);
 }
 
 // y (N, K) = sum of rows (N, width) weight (width, K) over the sets: the gradient of the rows that several layers share.  FLUSH: 0 for one set.
@@ -435,10 +452,13 @@ template <int KS> __device__ __forceinline__ void load_columns(rsrc_t r, int col
   }
 }
 
-template <int KS, bool ACROSS>
+// ADD: `addend` (N, cols) is added to the result: its elements are asked for when the tile's last product is under way (there are no registers to hold them before),
+// and what their way takes per tile is less than a pass over the result: product, product and sum, and both in one, 22500 rows of 256 x 256 23.2, 37.6 and 29.6 us;
+// 40000 34.2, 56.5, 45.7; 80000 67, 101, 82.
+template <int KS, bool ACROSS, bool ADD>
 __global__ __launch_bounds__(kRowThreads, 2) void linear_rows_kernel(const float *__restrict__ x, const float *__restrict__ weight,
-                                                                     const float *__restrict__ bias, float *__restrict__ y, long long N, int cols,
-                                                                     int depth) {
+                                                                     const float *__restrict__ bias, const float *__restrict__ addend,
+                                                                     float *__restrict__ y, long long N, int cols, int depth) {
   using Tile = RowTile<KS>;
   constexpr int kStores = 16;
   extern __shared__ __align__(16) unsigned char lds[];
@@ -453,18 +473,31 @@ __global__ __launch_bounds__(kRowThreads, 2) void linear_rows_kernel(const float
     const long long n0 = (long long)t * kRowTile, left = N - n0;
     return make_rsrc(x + (left > 0 ? n0 * depth : 0), left > 0 ? (size_t)(left < kRowTile ? left : kRowTile) * depth * 4 : 0);
   };
-  auto result_of = [&](int t) {
+  auto result_in = [&](const float *in, int t) {
     const long long n0 = (long long)t * kRowTile, left = N - n0;
-    return make_rsrc(y + n0 * cols, (size_t)(left < kRowTile ? left : kRowTile) * cols * 4);
+    return make_rsrc(in + n0 * cols, (size_t)(left < kRowTile ? left : kRowTile) * cols * 4);
   };
   const uint32_t y_off = c0 + col < cols ? (uint32_t)(4 * half * cols + c0 + col) * 4 : kNoRow;
   const float add = bias != nullptr && c0 + col < cols ? bias[c0 + col] : 0.f;
   // always the same number of stores, as their number is part of what is waited for
-  auto put = [&](const f32x16 &acc, rsrc_t r, uint32_t off) {
+  auto put = [&](f32x16 &acc, int t, uint32_t off) {
+    const rsrc_t r = result_in(y, t);
     asm volatile("" : "+v"(off));
+    if constexpr (ADD) {
+      const rsrc_t from = result_in(addend, t);
+      float plus[kStores];
+      uint32_t at = off;
+#pragma unroll
+      for (int i = 0; i < kStores; ++i) {
+        plus[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0));
+        at += (uint32_t)(i % 4 == 3 ? 5 : 1) * cols * 4;
+      }
+#pragma unroll
+      for (int i = 0; i < kStores; ++i) acc[i] = acc[i] + add + plus[i];
+    }
 #pragma unroll
     for (int i = 0; i < kStores; ++i) {
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i] + add), r, off, 0, 2);      // 2: non-temporal
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ADD ? acc[i] : acc[i] + add), r, off, 0, 2);      // 2: non-temporal
       off += (uint32_t)(i % 4 == 3 ? 5 : 1) * cols * 4;
     }
   };
@@ -526,7 +559,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void linear_rows_kernel(const float
       any_odd = true;
       if (lane == 0) s_odd[wave][i % kOddTiles / 32] |= 1u << (i % 32);
     }
-    put(acc[0][0], result_of(t), odd ? kNoRow : y_off);
+    put(acc[0][0], t, odd ? kNoRow : y_off);
     now = after;
   }
   wait_until_left<0>();                                        // nothing is on its way to LDS when the workgroup ends
@@ -537,7 +570,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void linear_rows_kernel(const float
       f32x16 acc[1][1];
       zero_sums(acc);
       whole_product<1, 1, false, ACROSS>(rows_of(t), depth, 0, 0, w_r, ldw, 0, cols - c0, depth, lane % 32, col, acc);
-      put(acc[0][0], result_of(t), y_off);
+      put(acc[0][0], t, y_off);
     }
   }
 }
@@ -626,11 +659,11 @@ template <int TM, int TN> static unsigned linear_blocks(long long N, int tiles) 
 static bool wide_tiles(long long N, int width) { return width > 64 && (N + 63) / 64 * ((width + 127) / 128) >= 512; }
 
 template <int TM, int TN>
-static hipError_t launch_linear_cfg(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream) {
+static hipError_t launch_linear_cfg(const float *x, const float *w, const float *bias, const float *addend, float *y, long long N, int O, int K, hipStream_t stream) {
   const int tiles = (O + TN - 1) / TN;
   const unsigned blocks = linear_blocks<TM, TN>(N, tiles);
   if (blocks == 0) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((linear_kernel<TM, TN>), dim3(blocks), dim3(256), 0, stream, x, w, bias, y, N, O, K, tiles);
+  hipLaunchKernelGGL((linear_kernel<TM, TN>), dim3(blocks), dim3(256), 0, stream, x, w, bias, addend, y, N, O, K, tiles);
   return hipGetLastError();
 }
 
@@ -657,20 +690,24 @@ static bool rows_kernel_applies(const float *x, const float *weight, long long N
   if (2 * tiles >= 3 * cus) return share >= 14 * sixteenth;
   return tiles <= cus && 5 * tiles >= 3 * cus && share >= (across ? 12 : 15) * sixteenth;
 }
-template <int KS, bool ACROSS>
-static hipError_t launch_linear_rows(const float *x, const float *w, const float *bias, float *y, long long N, int cols, int depth, hipStream_t stream) {
-  const auto kernel = linear_rows_kernel<KS, ACROSS>;
+template <int KS, bool ACROSS, bool ADD>
+static hipError_t launch_linear_rows(const float *x, const float *w, const float *bias, const float *addend, float *y, long long N, int cols, int depth,
+                                     hipStream_t stream) {
+  const auto kernel = linear_rows_kernel<KS, ACROSS, ADD>;
   if (const hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), RowTile<KS>::kLds); e != hipSuccess) return e;
   const long long tiles = (N + kRowTile - 1) / kRowTile;
   const int cus = cu_count();
   hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles < cus ? tiles : cus), (cols + kRowCols - 1) / kRowCols), dim3(kRowThreads), RowTile<KS>::kLds, stream,
-                     x, w, bias, y, N, cols, depth);
+                     x, w, bias, addend, y, N, cols, depth);
   return hipGetLastError();
 }
 
-hipError_t launch_linear(const float *x, const float *w, const float *bias, float *y, long long N, int O, int K, hipStream_t stream) {
-  if (rows_kernel_applies(x, w, N, O, K, false)) return launch_linear_rows<16, false>(x, w, bias, y, N, O, K, stream);
-  return wide_tiles(N, O) ? launch_linear_cfg<64, 128>(x, w, bias, y, N, O, K, stream) : launch_linear_cfg<64, 64>(x, w, bias, y, N, O, K, stream);
+hipError_t launch_linear(const float *x, const float *w, const float *bias, const float *addend, float *y, long long N, int O, int K, hipStream_t stream) {
+  if (rows_kernel_applies(x, w, N, O, K, false))
+    return addend != nullptr ? launch_linear_rows<16, false, true>(x, w, bias, addend, y, N, O, K, stream)
+                             : launch_linear_rows<16, false, false>(x, w, bias, nullptr, y, N, O, K, stream);
+  return wide_tiles(N, O) ? launch_linear_cfg<64, 128>(x, w, bias, addend, y, N, O, K, stream)
+                          : launch_linear_cfg<64, 64>(x, w, bias, addend, y, N, O, K, stream);
 }
 
 template <int TM, int TN, int FLUSH> static hipError_t launch_linear_sum_cfg(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream) {
@@ -683,7 +720,7 @@ template <int TM, int TN, int FLUSH> static hipError_t launch_linear_sum_cfg(con
 
 hipError_t launch_linear_sum(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream) {
   const LinearSet &s = sets.set[0];
-  if (sets.n == 1 && rows_kernel_applies(s.rows, s.weight, N, K, s.width, true)) return launch_linear_rows<16, true>(s.rows, s.weight, nullptr, y, N, K, s.width, stream);
+  if (sets.n == 1 && rows_kernel_applies(s.rows, s.weight, N, K, s.width, true)) return launch_linear_rows<16, true, false>(s.rows, s.weight, nullptr, nullptr, y, N, K, s.width, stream);
   const bool wide = wide_tiles(N, K);
   if (sets.n == 1) return wide ? launch_linear_sum_cfg<64, 128, 0>(sets, y, N, K, stream) : launch_linear_sum_cfg<64, 64, 0>(sets, y, N, K, stream);
   return wide ? launch_linear_sum_cfg<64, 128, 128>(sets, y, N, K, stream) : launch_linear_sum_cfg<64, 64, 128>(sets, y, N, K, stream);

@@ -64,6 +64,7 @@ SIGNATURES = {
     "dfa3d_locations": [_P] * 5 + [ctypes.c_longlong] + [_I] * 4 + [_P],
     "dfa3d_locations_grad": [_P] * 4 + [ctypes.c_longlong] + [_I] * 3 + [_P],
     "dfa3d_linear": [_P] * 4 + [ctypes.c_longlong, _I, _I, _P],
+    "dfa3d_linear_add": [_P] * 5 + [ctypes.c_longlong, _I, _I, _P],
     "dfa3d_linear_sum": [ctypes.POINTER(LinearSet), _I, _P, ctypes.c_longlong, _I, _P],
     "dfa3d_linear_grad": [_P] * 5 + [ctypes.c_size_t, ctypes.c_longlong, _I, _I, _P],
     "dfa3d_abi_version": [],
@@ -74,7 +75,7 @@ _BOUND = ("dfa3d_last_error", "dfa3d_packed_dist_bytes", "dfa3d_fused_forward", 
           "dfa3d_fused_backward", "dfa3d_wms_deform_attn_forward", "dfa3d_wms_deform_attn_backward_workspace_bytes",
           "dfa3d_wms_deform_attn_backward", "dfa3d_ms_depth_score_sample_forward",
           "dfa3d_ms_depth_score_sample_backward_workspace_bytes", "dfa3d_ms_depth_score_sample_backward_into", "dfa3d_pack_dist",
-          "dfa3d_linear", "dfa3d_linear_sum")
+          "dfa3d_linear_add", "dfa3d_linear_sum")
 
 _lib = None
 _binding = None

@@ -9,7 +9,7 @@ from torch import nn
 
 from ..rebatch import RebatchCombineFunction, RebatchQueriesFunction, camera_hits_counted, camera_index
 from .ms_deform_attn_3d import MSDeformableAttention3D_DFA3D
-from .projection import Projection, no_hooks
+from .projection import Projection, no_hooks, projection_plus
 
 __all__ = ["SpatialCrossAttention_DFA3D"]
 
@@ -127,5 +127,7 @@ class SpatialCrossAttention_DFA3D(nn.Module):
             queries = queries + ((1 - update_weight) * empty[None]).mean(dim=-2)
 
         slots = RebatchCombineFunction.apply(queries, index, pos, scale.to(queries.dtype).contiguous())     # (bs, Nq, E)
-        slots = self.output_proj(slots)
-        return self.dropout(slots) + inp_residual
+        drops = self.dropout
+        if type(drops) is nn.Dropout and no_hooks(drops) and not (drops.training and drops.p):
+            return projection_plus(self.output_proj, slots, inp_residual)
+        return drops(self.output_proj(slots)) + inp_residual

@@ -282,9 +282,10 @@ int dfa3d_locations_grad(const float *grad_loc, const int64_t *shapes3, float *g
 
 /* Linear layers in float32, all matrices row-major:
  *   dfa3d_linear      y (N, O) = x (N, K) weight (O, K)^T + bias (O) or NULL
+ *   dfa3d_linear_add  the same plus addend (N, O), or NULL: the residual beside a layer
  *   dfa3d_linear_sum  y (N, K) = sum over up to four layers of rows (N, width) weight (width, K): the gradient of the rows that the layers
  *                     share, from those of what they gave
- * O, K and widths even; K (the first), widths (the second) multiples of four.  Every element written, the same result every time.
+ * O, K and widths even; K (the first two), widths (the third) multiples of four.  Every element written, the same result every time.
  * Precision: that of float32 products and sums; operands and results may have any value (infinities and NaN as in float32 arithmetic; a
  * sum below 2^-89 in size of which an operand is denormal may come out as zero). */
 typedef struct dfa3d_linear_set {
@@ -293,6 +294,7 @@ typedef struct dfa3d_linear_set {
   int width;
 } dfa3d_linear_set;
 int dfa3d_linear(const float *x, const float *weight, const float *bias, float *y, long long N, int O, int K, void *stream);
+int dfa3d_linear_add(const float *x, const float *weight, const float *bias, const float *addend, float *y, long long N, int O, int K, void *stream);
 int dfa3d_linear_sum(const dfa3d_linear_set *layers, int n_layers, float *y, long long N, int K, void *stream);
 
 /* Weight and bias gradients of a linear layer y = x weight^T + bias in float32: grad_weight (O, K) = grad_out^T x,
