@@ -612,8 +612,28 @@ int dfa3d_linear_grad(const float *x, const float *grad_out, float *grad_weight,
   REQUIRE_PTR(fn, x); REQUIRE_PTR(fn, grad_out); REQUIRE_PTR(fn, grad_weight); REQUIRE_PTR(fn, workspace);
   if (workspace_bytes < dfa3d::linear_grad_workspace_bytes(N, O, K) || ((uintptr_t)workspace & 15) != 0)
     return fail(DFA3D_EINVAL, "%s: workspace too small or not on a 16-byte boundary", fn);
-  return hip_result(dfa3d::launch_linear_grad(x, grad_out, grad_weight, grad_bias, (float *)workspace, N, O, K,
-                                              (hipStream_t)stream), fn);
+  const dfa3d::LinearGradSets sets = {{{grad_out, grad_weight, grad_bias, O}}, 1};
+  return hip_result(dfa3d::launch_linear_grads(x, sets, (float *)workspace, N, K, (hipStream_t)stream), fn);
+}
+
+int dfa3d_linear_grads(const float *x, const dfa3d_linear_grad_set *layers, int n_layers, void *workspace, size_t workspace_bytes, long long N, int K,
+                       void *stream) {
+  const char *fn = "dfa3d_linear_grads";
+  if (n_layers < 1 || n_layers > DFA3D_MAX_LINEAR_SETS) return fail(DFA3D_EINVAL, "%s: 1 to %d layers (%d)", fn, DFA3D_MAX_LINEAR_SETS, n_layers);
+  REQUIRE_PTR(fn, x); REQUIRE_PTR(fn, layers); REQUIRE_PTR(fn, workspace);
+  dfa3d::LinearGradSets sets{};
+  sets.n = n_layers;
+  size_t bytes = 0;
+  for (int i = 0; i < n_layers; ++i) {
+    const dfa3d_linear_grad_set &l = layers[i];
+    if (int rc = check_linear(fn, N, l.width, K)) return rc;
+    REQUIRE_PTR(fn, l.grad_out); REQUIRE_PTR(fn, l.grad_weight);
+    sets.set[i] = dfa3d::LinearGradSet{l.grad_out, l.grad_weight, l.grad_bias, l.width};
+    bytes += dfa3d::linear_grad_workspace_bytes(N, l.width, K);
+  }
+  if (workspace_bytes < bytes || ((uintptr_t)workspace & 15) != 0)
+    return fail(DFA3D_EINVAL, "%s: workspace too small or not on a 16-byte boundary", fn);
+  return hip_result(dfa3d::launch_linear_grads(x, sets, (float *)workspace, N, K, (hipStream_t)stream), fn);
 }
 
 }  // extern "C"

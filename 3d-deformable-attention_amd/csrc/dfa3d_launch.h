@@ -185,7 +185,8 @@ hipError_t launch_linear(const float *x, const float *w, const float *bias, cons
 hipError_t launch_linear_sum(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream);
 // Weight and bias gradients of a linear layer (dfa3d_linear.hip); O and K even.
 size_t linear_grad_workspace_bytes(long long N, int O, int K);
-hipError_t launch_linear_grad(const float *x, const float *g, float *grad_weight, float *grad_bias, float *workspace,
-                              long long N, int O, int K, hipStream_t stream);
+struct LinearGradSet { const float *rows; float *grad_weight, *grad_bias; int width; };
+struct LinearGradSets { LinearGradSet set[DFA3D_MAX_LINEAR_SETS]; int n; };
+hipError_t launch_linear_grads(const float *x, const LinearGradSets &sets, float *workspace, long long N, int K, hipStream_t stream);
 
 }  // namespace dfa3d

@@ -39,6 +39,11 @@ class LinearSet(ctypes.Structure):
     _fields_ = [("weight", _P), ("rows", _P), ("width", _I)]
 
 
+class LinearGradSet(ctypes.Structure):
+    """dfa3d_linear_grad_set of include/dfa3d.h: the gradients of one of several linear layers on the same rows."""
+    _fields_ = [("grad_out", _P), ("grad_weight", _P), ("grad_bias", _P), ("width", _I)]
+
+
 # name -> argument types; every entry point returns int
 SIGNATURES = {
     "dfa3d_ms_depth_score_sample_forward": [_P] * 5 + _DIMS7 + [_I, _O, _P],
@@ -67,6 +72,7 @@ SIGNATURES = {
     "dfa3d_linear_add": [_P] * 5 + [ctypes.c_longlong, _I, _I, _P],
     "dfa3d_linear_sum": [ctypes.POINTER(LinearSet), _I, _P, ctypes.c_longlong, _I, _P],
     "dfa3d_linear_grad": [_P] * 5 + [ctypes.c_size_t, ctypes.c_longlong, _I, _I, _P],
+    "dfa3d_linear_grads": [_P, ctypes.POINTER(LinearGradSet), _I, _P, ctypes.c_size_t, ctypes.c_longlong, _I, _P],
     "dfa3d_abi_version": [],
 }
 

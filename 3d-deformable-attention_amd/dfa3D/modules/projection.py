@@ -88,6 +88,20 @@ def _weight_gradients(x, grad, want_bias):
     return grad_weight, grad_bias
 
 
+def _several_weight_gradients(x, grads, want_bias):
+    """``_weight_gradients`` of several layers on the same rows, in the launches of one."""
+    N, K = x.shape
+    lib = _lib.lib()
+    sizes = [lib.dfa3d_linear_grad_workspace_bytes(N, g.shape[1], K) for g in grads]
+    workspace = torch.empty(sum(sizes), dtype=torch.uint8, device=x.device)
+    out = [(x.new_empty(g.shape[1], K), x.new_empty(g.shape[1]) if want else None) for g, want in zip(grads, want_bias)]
+    sets = (_lib.LinearGradSet * len(grads))(*((_lib.ptr(g), _lib.ptr(w), _lib.ptr(b), g.shape[1]) for g, (w, b) in zip(grads, out)))
+    with _lib.on_device(x.device):
+        rc = lib.dfa3d_linear_grads(_lib.ptr(x), sets, len(grads), _lib.ptr(workspace), sum(sizes), N, K, _lib.stream_of(x))
+    _lib.check(rc, "dfa3d_linear_grads")
+    return out
+
+
 def plain_gradient(grad):
     """A gradient that a kernel may read: float32 on the GPU, not recorded and not a batch of gradients (is_grads_batched)."""
     return (not torch.is_grad_enabled() and grad.is_cuda and grad.dtype == torch.float32
@@ -177,9 +191,19 @@ class _SharedRowsFunction(Function):
         grads = [g.contiguous() if g is not None and plain_gradient(g) else g for g in grads]
         there = [i for i, g in enumerate(grads) if g is not None]
         grad_x = _input_gradient([grads[i] for i in there], [weights[i] for i in there]) if want_x and there else None
-        out = []
-        for i, g in enumerate(grads):
-            out += (None, None) if g is None else _layer_gradients(x, g, *wanted[2 * i:2 * i + 2])
+        out = [None] * (2 * len(grads))
+        together = [i for i in there if wanted[2 * i]]         # (the layers whose weight's gradient is wanted)
+        rows = x.reshape(-1, x.shape[-1]).contiguous() if len(together) > 1 else None
+        if rows is not None and all(plain_gradient(grads[i]) and _as_plain(rows, grads[i]) for i in together):
+            formed = _several_weight_gradients(rows, [grads[i].reshape(-1, grads[i].shape[-1]) for i in together],
+                                               [wanted[2 * i + 1] for i in together])
+            for i, pair in zip(together, formed):
+                out[2 * i:2 * i + 2] = pair
+        else:
+            together = ()
+        for i in there:
+            if i not in together:
+                out[2 * i:2 * i + 2] = _layer_gradients(x, grads[i], *wanted[2 * i:2 * i + 2])
         return (None, grad_x, *out)
 
 

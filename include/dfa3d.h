@@ -304,6 +304,15 @@ int dfa3d_linear_sum(const dfa3d_linear_set *layers, int n_layers, float *y, lon
 size_t dfa3d_linear_grad_workspace_bytes(long long N, int O, int K);
 int dfa3d_linear_grad(const float *x, const float *grad_out, float *grad_weight, float *grad_bias, void *workspace,
                       size_t workspace_bytes, long long N, int O, int K, void *stream);
+/* The same of several layers on the same rows x, each with its result's gradient (N, width); `workspace` of the sum of their sizes. */
+typedef struct dfa3d_linear_grad_set {
+  const float *grad_out;
+  float *grad_weight;
+  float *grad_bias;
+  int width;
+} dfa3d_linear_grad_set;
+int dfa3d_linear_grads(const float *x, const dfa3d_linear_grad_set *layers, int n_layers, void *workspace, size_t workspace_bytes, long long N, int K,
+                       void *stream);
 
 /* Message for the last non-zero return on the calling thread ("" if none). */
 const char *dfa3d_last_error(void);
