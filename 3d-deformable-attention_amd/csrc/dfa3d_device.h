@@ -564,10 +564,40 @@ template <typename A> struct DepthPair {
   }
   __device__ __forceinline__ A score(A x, A y) const { return depth_lerp(use_x ? x : (A)0, use_y ? y : (A)0, wx, wy); }
 };
-// corner_scores() for callers that count in bytes: the distribution of pixel (y, x) lies at base + y * row + x * col
-template <typename T, typename A>
+// Pairs of floats at the byte offsets `off` of the wavefront's active lanes in `lanes`, by scalar loads: they go round the vector path, whose front end is what gathers
+// wait for.  Four points at a time (more, or fewer, of the scalar registers' room for their results are slower), each place read from its lane and the results
+// written back to it.  Offsets are read whether the lane has use for them or not: they have to lie in the array.
+extern "C" __device__ __attribute__((const)) int dfa3d_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+__device__ __forceinline__ void scalar_pairs(const float *base, unsigned long long lanes, const uint32_t (&off)[4], float (&x)[4], float (&y)[4]) {
+  constexpr int kPoints = 4;
+  typedef int i2 __attribute__((ext_vector_type(2), aligned(4)));
+  typedef const __attribute__((address_space(4))) char *Scalar;
+  const Scalar from = (Scalar)(uintptr_t)base;
+  int xs[4] = {0, 0, 0, 0}, ys[4] = {0, 0, 0, 0};
+  while (lanes != 0) {                                       // uniform
+    int at[kPoints];
+    i2 t[kPoints][4];
+#pragma unroll
+    for (int j = 0; j < kPoints; ++j) {
+      at[j] = j == 0 || lanes != 0 ? __builtin_ctzll(lanes) : at[j > 0 ? j - 1 : 0];      // (the last one again)
+      lanes &= lanes - 1;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        t[j][k] = *(const __attribute__((address_space(4))) i2 *)(from + (uint32_t)__builtin_amdgcn_readlane((int)off[k], at[j]));
+    }
+#pragma unroll
+    for (int j = 0; j < kPoints; ++j)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) { xs[k] = dfa3d_writelane(t[j][k].x, at[j], xs[k]); ys[k] = dfa3d_writelane(t[j][k].y, at[j], ys[k]); }
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) { x[k] = __int_as_float(xs[k]); y[k] = __int_as_float(ys[k]); }
+}
+// corner_scores() for callers that count in bytes: the distribution of pixel (y, x) lies at base + y * row + x * col.  SCALAR: lanes with `by_scalar`
+// take their taps by scalar loads, from `dist` (the batch element's).
+template <typename T, typename A, bool SCALAR = false>
 __device__ __forceinline__ void grid_scores(rsrc_t dist_r, const Grid2D<A> &g, const DepthTap<A> &tap, uint32_t base, uint32_t row, uint32_t col,
-                                            int D, bool whole_words, A (&score)[4]) {
+                                            int D, bool whole_words, A (&score)[4], const T *dist = nullptr, bool by_scalar = false) {
   const uint32_t at = (uint32_t)g.h0 * row + (uint32_t)g.w0 * col + base;
   if (D >= 2) {
     const DepthPair<A> pair(tap, D);
@@ -578,7 +608,20 @@ __device__ __forceinline__ void grid_scores(rsrc_t dist_r, const Grid2D<A> &g, c
       off[k] = g.on(k) && tap.inside ? at_pair + (k >= 2 ? row : 0) + (k == 1 || k == 2 ? col : 0) : kNoRow;
     A x[4], y[4];
     __builtin_amdgcn_sched_barrier(0);                       // the loads one behind the other: corner_scores()
-    PairLoader<T, false>::ld(dist_r, off, D, whole_words, x, y);
+    if constexpr (SCALAR) {
+      const unsigned long long lanes = __builtin_amdgcn_ballot_w64(by_scalar);
+      uint32_t in_array[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) { in_array[k] = off[k] == kNoRow ? 0u : off[k]; x[k] = 0; y[k] = 0; }
+      if (!by_scalar) PairLoader<T, false>::ld(dist_r, off, D, whole_words, x, y);
+      A xs[4], ys[4];
+      scalar_pairs(dist, lanes, in_array, xs, ys);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (by_scalar) { x[k] = off[k] == kNoRow ? (A)0 : xs[k]; y[k] = off[k] == kNoRow ? (A)0 : ys[k]; }
+    } else {
+      PairLoader<T, false>::ld(dist_r, off, D, whole_words, x, y);
+    }
 #pragma unroll
     for (int k = 0; k < 4; ++k) score[k] = pair.score(x[k], y[k]);
   } else {

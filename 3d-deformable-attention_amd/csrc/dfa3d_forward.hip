@@ -149,13 +149,13 @@ template <int FROM, int VEC> __device__ __forceinline__ void sum_over_slots(int 
 // ---------------------------------------------------------------------------------------
 // wavefronts a SIMD that the registers have to leave room for (1: as the compiler likes)
 template <typename T, int VEC, bool IN_LDS> constexpr int kFwdWaves = !IN_LDS && sizeof(T) == 4 && VEC == 4 ? 6 : 1;
-template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS, bool IN_TURN, bool EARLY>
+template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS, bool IN_TURN, bool EARLY, bool SCALAR = false>
 __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC, IN_LDS>)) void fwd_attention_kernel(
     const T *__restrict__ value, const T *__restrict__ dist, const int64_t *__restrict__ shapes, int shape_stride,
     const int64_t *__restrict__ level_start, const A *__restrict__ loc, int loc_stride,
     const A *__restrict__ attn, const T *__restrict__ score_in, T *__restrict__ out, T *__restrict__ score_out,
     A *__restrict__ weight_update, const T *__restrict__ packed_arg, int Md, int B, int S, int M, int C, int D, int L,
-    int Q, int P, int upw, int iters, int q_blocks, int once, int lds_rows) {
+    int Q, int P, int upw, int iters, int q_blocks, int once, int lds_rows, int by_scalar) {
   // packed: the head-shared distribution as dfa3d_pack_dist lays it out (D >= 2), or nullptr
   __shared__ LevelTable tab;
   constexpr int WAVES = (IN_LDS ? kLdsRowsBlock : kBlock) / kWave;
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC,
 #pragma unroll
               for (int k = 0; k < 4; ++k) sc[k] = pair.score(x4[k], y4[k]);
             } else {
-              grid_scores<T, A>(dist_r, g, tap, lv.d_base, lv.d_row, d_col, D, whole_words, sc);
+              grid_scores<T, A, SCALAR>(dist_r, g, tap, lv.d_base, lv.d_row, d_col, D, whole_words, sc, dist + (size_t)b * S * Md * D, lp < by_scalar);
             }
             if (score_out != nullptr && pass == 0) {
               T *so = reinterpret_cast<T *>(reinterpret_cast<char *>(score_out + first_point(q0) * 4) + pl.idx * (uint32_t)(4 * sizeof(T)));
@@ -602,20 +602,32 @@ hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int6
 //     8 points 457, 438 (415, 434).  So: from 5000 points (bfloat16 in one stage 8000; float32 with scores fewer) of which 1200 (bfloat16 2400)
 //     are on levels in LDS.
 //     Levels that are no such pyramid (equal ones, or coarse to fine) may have none that fits; such a call takes 1 to 12 % longer than from memory.
+//     There an eighth of a unit's points take their depth taps by scalar loads (by_scalar points; float32), which the vector path's front end, what bounds the
+//     others, does not see: it answers a scattered line in 2 to 10 clocks, the scalar path a load in 10 to 14, side by side.  Kernel, all by vector loads and so, us,
+//     6 x 10000 queries, four levels of 8 points, 32 channels, around the query, anywhere and clustered, by what a (batch, head) has of values and
+//     distributions:
+//       58 x 100, 16 bins   1.5 MB   323, 359   499, 478   517, 483      80 x 128, 3 x 8, 64 bins  5.2 MB   680, 697   1027, 998   965, 925
+//       80 x 128, 16 bins   2.6 MB   359, 382   565, 530   564, 515      116 x 200, 16 bins        5.9 MB   487, 474    769, 737   721, 675
+//       58 x 100, 64 bins   3.0 MB   367, 384   533, 510   565, 520      16 channels, 64 bins      9.9 MB   488, 454    759, 721   691, 640
+//       70 x 119, 64 bins   4.2 MB   403, 408   610, 577   605, 554      32 channels, 64 bins     11.8 MB   571, 538    869, 839   803, 766
+//       58 x 100, 112 bins  4.4 MB   406, 411   620, 603   599, 563      128 bins                 19.7 MB   630, 587    983, 947   849, 806
+//     Neighbouring points find each other's lines in the L1 where maps are small, and the scalar path has none that would know: so from 5.5 MB on.  A quarter of
+//     the points: anywhere 816, around the query 631 (64 bins).  On maps that are in LDS whole 3 to 20 % slower; where all rows come from memory,
+//     or in stage 1 alone, 0 to 2 % either way.
 //     Not with packed distributions, which a cross-attention layer uses: its points share a pillar's few pixels, whose rows the L1 has
 //     (200 x 200 queries, base maps 412, 432; 120 x 120, 30 x 48 226, 239).
 template <typename T, int VEC, int LPR> constexpr bool kLdsRowsTiling = sizeof(T) <= 4 && VEC == 4 && LPR <= 16;
-struct LdsRows { int parts, rows; };
+struct LdsRows { int parts, rows, by_scalar; };
 template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a) {
   constexpr size_t kStatic = (kLdsRowsBlock / kWave) * sizeof(Task<A>) * kTasksPerWave + sizeof(LevelTable) + 64;
-  const LdsRows none{0, 0};
+  const LdsRows none{0, 0, 0};
   const long long room = (long long)((160 * 1024 - kStatic) / (a.C * sizeof(T))) - 1, points = (long long)a.Q * a.L * a.P;
   if (a.iters > 1 || room < 1) return none;
   const long long cus = cu_count(), pairs = (long long)a.M * a.B;
   if (room >= a.S) {
     const long long parts = cus / pairs;
     if (4 * pairs * parts < 3 * cus || points < parts * a.S) return none;      // idle CUs; too few points
-    return LdsRows{(int)parts, a.S};
+    return LdsRows{(int)parts, a.S, 0};
   }
   const long long parts = cus / a.M;
   if (parts < 1 || (8 % a.M != 0 && a.M % 8 != 0) || a.packed_dist != nullptr) return none;
@@ -626,7 +638,8 @@ template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a)
   constexpr bool k16 = sizeof(T) == 2;
   const long long least = a.dist != nullptr ? (k16 ? 8000 : 5000) : (!k16 && a.score_in != nullptr) ? 0 : 5000;
   if (points < parts * least || points * in_lds < parts * (k16 ? 2400 : 1200) * a.L) return none;
-  return LdsRows{(int)parts, (int)room};
+  const bool scalar_taps = sizeof(T) == 4 && a.dist != nullptr && a.D >= 2 && (long long)(a.C + a.D) * 4 * a.S > (11LL << 19);
+  return LdsRows{(int)parts, (int)room, scalar_taps ? a.L * a.P / 8 : 0};
 }
 
 template <typename T, typename A, int VEC, int LPR>
@@ -642,7 +655,7 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   // (the kernel counts bytes from a group's first point, and from its first output row, in 32 bits)
   while (upw > 1 && (long long)upw * a.M * std::max((long long)a.L * a.P * std::max<int>(a.loc_stride * sizeof(A), 4 * sizeof(T)), (long long)a.C * (long long)sizeof(T)) > 0x7FFFFFFFLL) upw /= 2;
   const FwdShape ws = fwd_shape(a.L, a.P, upw);
-  const LdsRows lds = kLdsRowsTiling<T, VEC, LPR> ? lds_rows_plan<T, A>(a) : LdsRows{0, 0};
+  const LdsRows lds = kLdsRowsTiling<T, VEC, LPR> ? lds_rows_plan<T, A>(a) : LdsRows{0, 0, 0};
   const int parts = lds.parts;
   const int q_per_iter = (parts > 0 ? kLdsRowsBlock / kWave : kWavesPerBlock) * ws.upw, groups = (a.Q + q_per_iter - 1) / q_per_iter;
   const int iters = parts > 0 ? (groups + parts - 1) / parts : a.iters > 0 ? a.iters : 1;
@@ -690,12 +703,15 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
                        a.shape_stride, a.level_start, (const A *)a.loc, a.loc_stride, (const A *)a.attn,
                        fused ? nullptr : (const T *)a.score_in, (T *)a.out, fused ? (T *)a.score_out : nullptr,
                        fused ? (A *)a.weight_update : nullptr, fused ? (const T *)a.packed_dist : nullptr,
-                       fused && a.dist_heads == 1 ? 1 : a.M, a.B, a.S, a.M, a.C, fused ? a.D : 0, a.L, a.Q, a.P, upw, iters, q_blocks, once, lds.rows);
+                       fused && a.dist_heads == 1 ? 1 : a.M, a.B, a.S, a.M, a.C, fused ? a.D : 0, a.L, a.Q, a.P, upw, iters, q_blocks, once, lds.rows, lds.by_scalar);
     return hipGetLastError();
   };
   if constexpr (kLdsRowsTiling<T, VEC, LPR>) {
     if (parts > 0) {
       const size_t bytes = ((size_t)lds.rows + 1) * a.C * sizeof(T);
+      if constexpr (sizeof(T) == 4) {
+        if (lds.by_scalar > 0) return launch(fwd_attention_kernel<T, A, VEC, LPR, true, true, false, false, true>, kLdsRowsBlock, bytes);
+      }
       return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, true, false, false>, kLdsRowsBlock, bytes)
                    : launch(fwd_attention_kernel<T, A, VEC, LPR, false, true, false, false>, kLdsRowsBlock, bytes);
     }
