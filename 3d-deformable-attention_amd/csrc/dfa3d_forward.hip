@@ -602,32 +602,20 @@ hipError_t launch_pack_dist(const void *dist, const int64_t *shapes3, const int6
 //     8 points 457, 438 (415, 434).  So: from 5000 points (bfloat16 in one stage 8000; float32 with scores fewer) of which 1200 (bfloat16 2400)
 //     are on levels in LDS.
 //     Levels that are no such pyramid (equal ones, or coarse to fine) may have none that fits; such a call takes 1 to 12 % longer than from memory.
-//     There an eighth of a unit's points take their depth taps by scalar loads (by_scalar points; float32), which the vector path's front end, what bounds the
-//     others, does not see: it answers a scattered line in 2 to 10 clocks, the scalar path a load in 10 to 14, side by side.  Kernel, all by vector loads and so, us,
-//     6 x 10000 queries, four levels of 8 points, 32 channels, around the query, anywhere and clustered, by what a (batch, head) has of values and
-//     distributions:
-//       58 x 100, 16 bins   1.5 MB   323, 359   499, 478   517, 483      80 x 128, 3 x 8, 64 bins  5.2 MB   680, 697   1027, 998   965, 925
-//       80 x 128, 16 bins   2.6 MB   359, 382   565, 530   564, 515      116 x 200, 16 bins        5.9 MB   487, 474    769, 737   721, 675
-//       58 x 100, 64 bins   3.0 MB   367, 384   533, 510   565, 520      16 channels, 64 bins      9.9 MB   488, 454    759, 721   691, 640
-//       70 x 119, 64 bins   4.2 MB   403, 408   610, 577   605, 554      32 channels, 64 bins     11.8 MB   571, 538    869, 839   803, 766
-//       58 x 100, 112 bins  4.4 MB   406, 411   620, 603   599, 563      128 bins                 19.7 MB   630, 587    983, 947   849, 806
-//     Neighbouring points find each other's lines in the L1 where maps are small, and the scalar path has none that would know: so from 5.5 MB on.  A quarter of
-//     the points: anywhere 816, around the query 631 (64 bins).  On maps that are in LDS whole 3 to 20 % slower; where all rows come from memory,
-//     or in stage 1 alone, 0 to 2 % either way.
 //     Not with packed distributions, which a cross-attention layer uses: its points share a pillar's few pixels, whose rows the L1 has
 //     (200 x 200 queries, base maps 412, 432; 120 x 120, 30 x 48 226, 239).
 template <typename T, int VEC, int LPR> constexpr bool kLdsRowsTiling = sizeof(T) <= 4 && VEC == 4 && LPR <= 16;
-struct LdsRows { int parts, rows, by_scalar; };
+struct LdsRows { int parts, rows; };
 template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a) {
   constexpr size_t kStatic = (kLdsRowsBlock / kWave) * sizeof(Task<A>) * kTasksPerWave + sizeof(LevelTable) + 64;
-  const LdsRows none{0, 0, 0};
+  const LdsRows none{0, 0};
   const long long room = (long long)((160 * 1024 - kStatic) / (a.C * sizeof(T))) - 1, points = (long long)a.Q * a.L * a.P;
   if (a.iters > 1 || room < 1) return none;
   const long long cus = cu_count(), pairs = (long long)a.M * a.B;
   if (room >= a.S) {
     const long long parts = cus / pairs;
     if (4 * pairs * parts < 3 * cus || points < parts * a.S) return none;      // idle CUs; too few points
-    return LdsRows{(int)parts, a.S, 0};
+    return LdsRows{(int)parts, a.S};
   }
   const long long parts = cus / a.M;
   if (parts < 1 || (8 % a.M != 0 && a.M % 8 != 0) || a.packed_dist != nullptr) return none;
@@ -638,8 +626,33 @@ template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a)
   constexpr bool k16 = sizeof(T) == 2;
   const long long least = a.dist != nullptr ? (k16 ? 8000 : 5000) : (!k16 && a.score_in != nullptr) ? 0 : 5000;
   if (points < parts * least || points * in_lds < parts * (k16 ? 2400 : 1200) * a.L) return none;
-  const bool scalar_taps = sizeof(T) == 4 && a.dist != nullptr && a.D >= 2 && (long long)(a.C + a.D) * 4 * a.S > (11LL << 19);
-  return LdsRows{(int)parts, (int)room, scalar_taps ? a.L * a.P / 8 : 0};
+  return LdsRows{(int)parts, (int)room};
+}
+
+// How many of a unit's points, the first ones, take their depth taps by scalar loads (float32, a distribution that is not packed).  The vector path's front end is what
+// bounds the gathers, a scattered line in 2 to 10 clocks; the scalar path answers a load in 10 to 14, side by side.  But neighbouring points find each
+// other's lines in the L1 where maps are small, and the scalar path has nothing of the kind: so the line lies by what a (batch, head) has of values and
+// distributions.  Kernel, us, points around the query, anywhere, clustered, 6 batch elements, 32 channels and four levels of 8 points unless noted.
+//   Rows from memory, 4000 queries, none / an eighth / three sixteenths:
+//     58 x 100, 16 bins          1.4 MB   159, 228, 226   164, 231, 228   169, 231, 224      80 x 128, 64 bins, 1 x 8   3.8 MB   123, 144, 150   117, 140, 142   120, 136, 140
+//     80 x 128, 16 bins          2.5 MB   185, 264, 268   181, 266, 262   193, 266, 258      58 x 100, 112 bins, 3 x 4  4.2 MB   156, 213, 203   150, 206, 194   159, 195, 183
+//     46 x 80, 128 bins, 3 x 8   3.0 MB   153, 225, 231   159, 222, 222   171, 217, 216      70 x 119, 112 bins         6.1 MB   240, 367, 335   226, 354, 317   232, 340, 303
+//     58 x 100, 80 bins          3.3 MB   197, 300, 293   193, 294, 281   200, 284, 270      116 x 200, 16 channels     9.4 MB   244, 375, 338   225, 358, 320   230, 344, 310
+//     100 x 170, 16 bins, 1 x 4  3.1 MB   106, 125, 121   106, 123, 116   106, 123, 116      116 x 200, 64 bins        11.3 MB   283, 415, 376   263, 401, 360   268, 389, 354
+//     so an eighth from 3.5 MB, three sixteenths from 6 MB on, one point at least (of 3 or 4: 116 x 200, one level 154, 179, 149 -> 146, 171, 140 and 168, 212, 172 -> 161,
+//     205, 162); a quarter: 64 bins 292, 385, 343.
+//   The coarser levels in LDS, 10000 queries, none / an eighth:
+//     58 x 100, 16 bins    1.5 MB   323, 499, 517   359, 478, 483      80 x 128, 64 bins, 3 x 8   5.2 MB   680, 1027, 965   697, 998, 925
+//     80 x 128, 16 bins    2.6 MB   359, 565, 564   382, 530, 515      116 x 200, 16 bins         5.9 MB   487, 769, 721    474, 737, 675
+//     58 x 100, 64 bins    3.0 MB   367, 533, 565   384, 510, 520      16 channels, 64 bins       9.9 MB   488, 759, 691    454, 721, 640
+//     70 x 119, 64 bins    4.2 MB   403, 610, 605   408, 577, 554      64 bins                   11.8 MB   571, 869, 803    538, 839, 766
+//     so an eighth from 5.5 MB on (three sixteenths: 64 bins 578, 825, 752; 16 bins 515, 749, 680).  On a map that is in LDS whole 3 to 20 % slower.
+template <typename T> static int points_by_scalar(const FwdArgs &a, const LdsRows &lds) {
+  const int LP = a.L * a.P;
+  if (sizeof(T) != 4 || a.dist == nullptr || a.packed_dist != nullptr || a.D < 2 || LP < 3 || (lds.parts > 0 && lds.rows == a.S)) return 0;
+  const long long bytes = (long long)(a.C + a.D) * a.S * 4;
+  if (lds.parts > 0) return bytes > (11LL << 19) ? LP / 8 : 0;
+  return bytes > (6LL << 20) ? (3 * LP + 15) / 16 : bytes > (7LL << 19) ? std::max(LP / 8, 1) : 0;
 }
 
 template <typename T, typename A, int VEC, int LPR>
@@ -655,8 +668,8 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   // (the kernel counts bytes from a group's first point, and from its first output row, in 32 bits)
   while (upw > 1 && (long long)upw * a.M * std::max((long long)a.L * a.P * std::max<int>(a.loc_stride * sizeof(A), 4 * sizeof(T)), (long long)a.C * (long long)sizeof(T)) > 0x7FFFFFFFLL) upw /= 2;
   const FwdShape ws = fwd_shape(a.L, a.P, upw);
-  const LdsRows lds = kLdsRowsTiling<T, VEC, LPR> ? lds_rows_plan<T, A>(a) : LdsRows{0, 0, 0};
-  const int parts = lds.parts;
+  const LdsRows lds = kLdsRowsTiling<T, VEC, LPR> ? lds_rows_plan<T, A>(a) : LdsRows{0, 0};
+  const int parts = lds.parts, by_scalar = points_by_scalar<T>(a, lds);
   const int q_per_iter = (parts > 0 ? kLdsRowsBlock / kWave : kWavesPerBlock) * ws.upw, groups = (a.Q + q_per_iter - 1) / q_per_iter;
   const int iters = parts > 0 ? (groups + parts - 1) / parts : a.iters > 0 ? a.iters : 1;
   const int q_blocks = (groups + iters - 1) / iters;
@@ -703,14 +716,14 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
                        a.shape_stride, a.level_start, (const A *)a.loc, a.loc_stride, (const A *)a.attn,
                        fused ? nullptr : (const T *)a.score_in, (T *)a.out, fused ? (T *)a.score_out : nullptr,
                        fused ? (A *)a.weight_update : nullptr, fused ? (const T *)a.packed_dist : nullptr,
-                       fused && a.dist_heads == 1 ? 1 : a.M, a.B, a.S, a.M, a.C, fused ? a.D : 0, a.L, a.Q, a.P, upw, iters, q_blocks, once, lds.rows, lds.by_scalar);
+                       fused && a.dist_heads == 1 ? 1 : a.M, a.B, a.S, a.M, a.C, fused ? a.D : 0, a.L, a.Q, a.P, upw, iters, q_blocks, once, lds.rows, by_scalar);
     return hipGetLastError();
   };
   if constexpr (kLdsRowsTiling<T, VEC, LPR>) {
     if (parts > 0) {
       const size_t bytes = ((size_t)lds.rows + 1) * a.C * sizeof(T);
       if constexpr (sizeof(T) == 4) {
-        if (lds.by_scalar > 0) return launch(fwd_attention_kernel<T, A, VEC, LPR, true, true, false, false, true>, kLdsRowsBlock, bytes);
+        if (by_scalar > 0) return launch(fwd_attention_kernel<T, A, VEC, LPR, true, true, false, false, true>, kLdsRowsBlock, bytes);
       }
       return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, true, false, false>, kLdsRowsBlock, bytes)
                    : launch(fwd_attention_kernel<T, A, VEC, LPR, false, true, false, false>, kLdsRowsBlock, bytes);
@@ -720,6 +733,11 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
     if (early)
       return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, false, true>, kBlock, 0)
                    : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, false, true>, kBlock, 0);
+  }
+  if constexpr (std::is_same<T, float>::value) {
+    if (by_scalar > 0)
+      return in_turn ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, true, false, true>, kBlock, 0)
+                     : launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, false, false, true>, kBlock, 0);
   }
   if (in_turn)
     return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, true, false>, kBlock, 0)

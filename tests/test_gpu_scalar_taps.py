@@ -1,5 +1,5 @@
-"""Depth taps of a part of the points by scalar loads (large maps whose coarser levels are in LDS): the scores are those of the path that gathers everything
-from memory (iters = 2) to the bit, the sums but for their order.  Units of one to more points than a wavefront has lanes, few and odd bins, a distribution that begins
+"""Depth taps of a part of the points by scalar loads (large maps, whose coarser levels are in LDS or not): the scores are those of the kernel of stage 1, which
+takes them all by vector loads, to the bit, and the sums those of stage 2 with them, but for their order.  Units of one to more points than a wavefront has lanes, few and odd bins, a distribution that begins
 between two cache lines, locations outside the map and the depth range, levels that do not fit the keys, and numbers that are none."""
 import pytest
 import torch
@@ -19,10 +19,13 @@ PYRAMID = ((116, 120), (58, 60), (29, 30), (15, 15))
     (PYRAMID, 4, 8, 97, 17, 4803),                         # 68 points: two rounds
     (((160, 190), (80, 95), (40, 48), (20, 24)), 8, 48, 2, 4, 10003),     # two bins
     (PYRAMID[:2] + PYRAMID[:1:-1], 8, 32, 64, 8, 5101),    # no pyramid
+    # all rows from memory, an eighth of a unit's points (3.5 MB and more) and three sixteenths (6 MB and more)
+    (PYRAMID, 3, 32, 64, 8, 70), (PYRAMID, 2, 5, 64, 5, 33), (PYRAMID[:1], 2, 64, 33, 3, 130), (PYRAMID[:1], 1, 72, 60, 1, 7), (PYRAMID[:1], 2, 8, 97, 4, 9),
+    (PYRAMID[:2], 5, 16, 77, 1, 31), (PYRAMID[:2], 2, 130, 6, 70, 5), (PYRAMID, 8, 12, 101, 2, 1), (PYRAMID[:1], 2, 64, 33, 90, 11),
 ], ids=str)
 @pytest.mark.parametrize("shared", [False, True])
 def test_same_taps_as_from_memory(levels, M, C, D, P, Q, shared):
-    from dfa3D import _ext, _lib
+    from dfa3D import _ext
     torch.manual_seed(Q)
     dev, B, L = "cuda", 2, len(levels)
     S = sum(h * w for h, w in levels)
@@ -33,8 +36,8 @@ def test_same_taps_as_from_memory(levels, M, C, D, P, Q, shared):
     starts = [sum(h * w for h, w in levels[:l]) for l in range(L)]
     lsi = torch.tensor(starts, device=dev)
     loc = torch.rand(B, Q, M, L, P, 3, device=dev) * 1.3 - 0.15
-    loc[0, 1, 0, 0, 0] = float("nan")
-    loc[1, 2, M - 1, L - 1, P - 1, 2] = float("inf")
+    loc[0, Q - 1, 0, 0, 0] = float("nan")
+    loc[1, Q // 2, M - 1, L - 1, P - 1, 2] = float("inf")
     attn = torch.rand(B, Q, M, L, P, device=dev)
     dist[1, S - 1, -1, -1] = float("nan")                  # the last number of all
     dist[0, 0, 0, 0] = float("inf")
@@ -43,8 +46,9 @@ def test_same_taps_as_from_memory(levels, M, C, D, P, Q, shared):
             sh = sh.clone()
             sh[L - 1, 0] += 50
         got = _ext.dfa3d_fused_forward(value, dist, sh, lsi, loc, attn, 64, need_depth_score=True, need_weight_update=True)
-        with _lib.launch_options(iters=2):
-            want = _ext.dfa3d_fused_forward(value, dist, sh, lsi, loc, attn, 64, need_depth_score=True, need_weight_update=True)
-        assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32))
-        torch.testing.assert_close(got[2], want[2], rtol=0, atol=0, equal_nan=True)
-        torch.testing.assert_close(got[0], want[0], **F32_FWD, equal_nan=True)
+        want = _ext.ms_depth_score_sample_forward(dist.expand(B, S, M, D).contiguous(), sh, lsi, loc, 64)
+        assert torch.equal(got[1].view(torch.int32), want.view(torch.int32))
+        out = _ext.wms_deform_attn_forward(value, sh[:, :2].contiguous(), lsi, loc[..., :2].contiguous(), attn, want, 64)
+        torch.testing.assert_close(got[0], out, **F32_FWD, equal_nan=True)
+        update = (want.double().mean(-1) * attn).sum((-1, -2)).float()
+        torch.testing.assert_close(got[2].view(update.shape), update, **F32_FWD, equal_nan=True)
