@@ -149,6 +149,7 @@ template <int FROM, int VEC> __device__ __forceinline__ void sum_over_slots(int 
 // ---------------------------------------------------------------------------------------
 // wavefronts a SIMD that the registers have to leave room for (1: as the compiler likes)
 template <typename T, int VEC, bool IN_LDS> constexpr int kFwdWaves = !IN_LDS && sizeof(T) == 4 && VEC == 4 ? 6 : 1;
+// SCALAR: the first by_scalar points of a unit take their depth taps by scalar loads (points_by_scalar)
 template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS, bool IN_TURN, bool EARLY, bool SCALAR = false>
 __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC, IN_LDS>)) void fwd_attention_kernel(
     const T *__restrict__ value, const T *__restrict__ dist, const int64_t *__restrict__ shapes, int shape_stride,
@@ -366,7 +367,8 @@ __global__ __launch_bounds__(IN_LDS ? kLdsRowsBlock : kBlock, (kFwdWaves<T, VEC,
 #pragma unroll
               for (int k = 0; k < 4; ++k) sc[k] = pair.score(x4[k], y4[k]);
             } else {
-              grid_scores<T, A, SCALAR>(dist_r, g, tap, lv.d_base, lv.d_row, d_col, D, whole_words, sc, dist + (size_t)b * S * Md * D, lp < by_scalar);
+              grid_scores<T, A, SCALAR>(dist_r, g, tap, lv.d_base, lv.d_row, d_col, D, whole_words, sc, dist + (size_t)b * S * Md * D,
+                                         (uint32_t)(S * Md * D * (int)sizeof(T)) - 8, lp < by_scalar);
             }
             if (score_out != nullptr && pass == 0) {
               T *so = reinterpret_cast<T *>(reinterpret_cast<char *>(score_out + first_point(q0) * 4) + pl.idx * (uint32_t)(4 * sizeof(T)));
@@ -629,7 +631,8 @@ template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a)
   return LdsRows{(int)parts, (int)room};
 }
 
-// How many of a unit's points, the first ones, take their depth taps by scalar loads (float32, a distribution that is not packed).  The vector path's front end is what
+// How many of a unit's points, the first ones, take their depth taps by scalar loads (a distribution that is not packed: with one line a point instead of four, 4 %
+// either way).  The vector path's front end is what
 // bounds the gathers, a scattered line in 2 to 10 clocks; the scalar path answers a load in 10 to 14, side by side.  But neighbouring points find each
 // other's lines in the L1 where maps are small, and the scalar path has nothing of the kind: so the line lies by what a (batch, head) has of values and
 // distributions.  Kernel, us, points around the query, anywhere, clustered, 6 batch elements, 32 channels and four levels of 8 points unless noted.
@@ -647,12 +650,17 @@ template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a)
 //     58 x 100, 64 bins    3.0 MB   367, 533, 565   384, 510, 520      16 channels, 64 bins       9.9 MB   488, 759, 691    454, 721, 640
 //     70 x 119, 64 bins    4.2 MB   403, 610, 605   408, 577, 554      64 bins                   11.8 MB   571, 869, 803    538, 839, 766
 //     so an eighth from 5.5 MB on (three sixteenths: 64 bins 578, 825, 752; 16 bins 515, 749, 680).  On a map that is in LDS whole 3 to 20 % slower.
+//   Bfloat16, rows from memory, 4000 queries, none / three sixteenths: 70 x 119, 112 bins 3.1 MB 190, 299, 263 -> 213, 282, 241 (an eighth 194, 290, 250); 116 x 200, 59 bins
+//     5.6 MB 231, 355, 327 -> 228, 335, 302; 64 bins 5.9 MB 250, 379, 351 -> 229, 341, 302: from 5 MB on.  The coarser levels in LDS, 10000 queries, 64 bins, a sixteenth /
+//     an eighth: 475, 795, 738 -> 482, 760, 684 / 486, 738, 663; 128 bins 498, 763, 697 -> 505, 748, 676 / 515, 733, 665: not, for the points around the query.
 template <typename T> static int points_by_scalar(const FwdArgs &a, const LdsRows &lds) {
   const int LP = a.L * a.P;
-  if (sizeof(T) != 4 || a.dist == nullptr || a.packed_dist != nullptr || a.D < 2 || LP < 3 || (lds.parts > 0 && lds.rows == a.S)) return 0;
-  const long long bytes = (long long)(a.C + a.D) * a.S * 4;
-  if (lds.parts > 0) return bytes > (11LL << 19) ? LP / 8 : 0;
-  return bytes > (6LL << 20) ? (3 * LP + 15) / 16 : bytes > (7LL << 19) ? std::max(LP / 8, 1) : 0;
+  if (sizeof(T) > 4 || a.dist == nullptr || a.packed_dist != nullptr || a.D < 2 || LP < 3 || (lds.parts > 0 && lds.rows == a.S)) return 0;
+  const long long bytes = (long long)(a.C + a.D) * a.S * (long long)sizeof(T);
+  const int eighth = LP / 8, three_sixteenths = (3 * LP + 15) / 16;
+  if (sizeof(T) == 2) return lds.parts == 0 && bytes > (5LL << 20) ? three_sixteenths : 0;
+  if (lds.parts > 0) return bytes > (11LL << 19) ? eighth : 0;
+  return bytes > (6LL << 20) ? three_sixteenths : bytes > (7LL << 19) ? std::max(eighth, 1) : 0;
 }
 
 template <typename T, typename A, int VEC, int LPR>
@@ -734,7 +742,7 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
       return fused ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, false, true>, kBlock, 0)
                    : launch(fwd_attention_kernel<T, A, VEC, LPR, false, false, false, true>, kBlock, 0);
   }
-  if constexpr (std::is_same<T, float>::value) {
+  if constexpr (sizeof(T) <= 4) {
     if (by_scalar > 0)
       return in_turn ? launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, true, false, true>, kBlock, 0)
                      : launch(fwd_attention_kernel<T, A, VEC, LPR, true, false, false, false, true>, kBlock, 0);
