@@ -551,7 +551,33 @@ int dfa3d_locations(const float *uv, const float *dz, const float *ref, const in
   const char *fn = "dfa3d_locations";
   if (int rc = check_locations(fn, rows, M, L, P, Z)) return rc;
   REQUIRE_PTR(fn, uv); REQUIRE_PTR(fn, dz); REQUIRE_PTR(fn, ref); REQUIRE_PTR(fn, shapes3); REQUIRE_PTR(fn, loc);
-  return hip_result(dfa3d::launch_locations(uv, dz, ref, shapes3, loc, rows, M, L, P, Z, (hipStream_t)stream), fn);
+  return hip_result(dfa3d::launch_locations(uv, dz, nullptr, ref, shapes3, loc, nullptr, rows, M, L, P, Z, (hipStream_t)stream), fn);
+}
+
+static int check_sampling(const char *fn, int L, int P) {
+  const long long n = (long long)L * P;
+  if (n > 64 || (n & (n - 1)) != 0) return fail(DFA3D_EINVAL, "%s: L * P must be a power of two up to 64 (L=%d P=%d)", fn, L, P);
+  return 0;
+}
+
+int dfa3d_sampling(const float *uv, const float *dz, const float *logits, const float *ref, const int64_t *shapes3, float *loc, float *attn,
+                   long long rows, int M, int L, int P, int Z, void *stream) {
+  const char *fn = "dfa3d_sampling";
+  if (int rc = check_locations(fn, rows, M, L, P, Z)) return rc;
+  if (int rc = check_sampling(fn, L, P)) return rc;
+  REQUIRE_PTR(fn, uv); REQUIRE_PTR(fn, dz); REQUIRE_PTR(fn, logits); REQUIRE_PTR(fn, ref); REQUIRE_PTR(fn, shapes3); REQUIRE_PTR(fn, loc);
+  REQUIRE_PTR(fn, attn);
+  return hip_result(dfa3d::launch_locations(uv, dz, logits, ref, shapes3, loc, attn, rows, M, L, P, Z, (hipStream_t)stream), fn);
+}
+
+int dfa3d_sampling_grad(const float *grad_loc, const float *grad_attn, const float *attn, const int64_t *shapes3, float *grad_uv, float *grad_dz,
+                        float *grad_logits, long long rows, int M, int L, int P, void *stream) {
+  const char *fn = "dfa3d_sampling_grad";
+  if (int rc = check_locations(fn, rows, M, L, P, 1)) return rc;
+  if (int rc = check_sampling(fn, L, P)) return rc;
+  REQUIRE_PTR(fn, grad_loc); REQUIRE_PTR(fn, grad_attn); REQUIRE_PTR(fn, attn); REQUIRE_PTR(fn, shapes3); REQUIRE_PTR(fn, grad_uv);
+  REQUIRE_PTR(fn, grad_dz); REQUIRE_PTR(fn, grad_logits);
+  return hip_result(dfa3d::launch_locations_grad(grad_loc, grad_attn, attn, shapes3, grad_uv, grad_dz, grad_logits, rows, M, L, P, (hipStream_t)stream), fn);
 }
 
 int dfa3d_locations_grad(const float *grad_loc, const int64_t *shapes3, float *grad_uv, float *grad_dz, long long rows, int M, int L,
@@ -559,7 +585,7 @@ int dfa3d_locations_grad(const float *grad_loc, const int64_t *shapes3, float *g
   const char *fn = "dfa3d_locations_grad";
   if (int rc = check_locations(fn, rows, M, L, P, 1)) return rc;
   REQUIRE_PTR(fn, grad_loc); REQUIRE_PTR(fn, shapes3); REQUIRE_PTR(fn, grad_uv); REQUIRE_PTR(fn, grad_dz);
-  return hip_result(dfa3d::launch_locations_grad(grad_loc, shapes3, grad_uv, grad_dz, rows, M, L, P, (hipStream_t)stream), fn);
+  return hip_result(dfa3d::launch_locations_grad(grad_loc, nullptr, nullptr, shapes3, grad_uv, grad_dz, nullptr, rows, M, L, P, (hipStream_t)stream), fn);
 }
 
 static int check_linear(const char *fn, long long N, int O, int K) {

@@ -171,11 +171,12 @@ hipError_t launch_camera_index(const uint8_t *hit, int *index, int *pos, int cam
 // (L, 2) to (L, 3) with D as the third extent (dfa3d_locations.hip).
 hipError_t launch_level_table(const int64_t *shapes, int64_t *shapes3, int L, int D, hipStream_t stream);
 
-// Sampling locations of a layer and their gradients (dfa3d_locations.hip).
-hipError_t launch_locations(const float *uv, const float *dz, const float *ref, const int64_t *shapes3, float *loc, long long rows,
-                            int M, int L, int P, int Z, hipStream_t stream);
-hipError_t launch_locations_grad(const float *grad_loc, const int64_t *shapes3, float *grad_uv, float *grad_dz, long long rows,
-                                 int M, int L, int P, hipStream_t stream);
+// Sampling locations of a layer and their gradients, without or with the weights (logits, attn and their gradients, or nullptr; L * P a power of two
+// up to 64 then) (dfa3d_locations.hip).
+hipError_t launch_locations(const float *uv, const float *dz, const float *logits, const float *ref, const int64_t *shapes3, float *loc, float *attn,
+                            long long rows, int M, int L, int P, int Z, hipStream_t stream);
+hipError_t launch_locations_grad(const float *grad_loc, const float *grad_attn, const float *attn, const int64_t *shapes3, float *grad_uv, float *grad_dz,
+                                 float *grad_logits, long long rows, int M, int L, int P, hipStream_t stream);
 
 // Linear layers (dfa3d_linear.hip): y (N, O) = x (N, K) w (O, K)^T + bias + addend (N, O) (or nullptr), and y (N, K) = sum over the sets of rows (N, width) weight
 // (width, K); O, K and widths even, K (widths) a multiple of four in the first (second).

@@ -68,6 +68,8 @@ SIGNATURES = {
     "dfa3d_level_table": [_P, _P, _I, _I, _P],
     "dfa3d_locations": [_P] * 5 + [ctypes.c_longlong] + [_I] * 4 + [_P],
     "dfa3d_locations_grad": [_P] * 4 + [ctypes.c_longlong] + [_I] * 3 + [_P],
+    "dfa3d_sampling": [_P] * 7 + [ctypes.c_longlong] + [_I] * 4 + [_P],
+    "dfa3d_sampling_grad": [_P] * 7 + [ctypes.c_longlong] + [_I] * 3 + [_P],
     "dfa3d_linear": [_P] * 4 + [ctypes.c_longlong, _I, _I, _P],
     "dfa3d_linear_add": [_P] * 5 + [ctypes.c_longlong, _I, _I, _P],
     "dfa3d_linear_sum": [ctypes.POINTER(LinearSet), _I, _P, ctypes.c_longlong, _I, _P],

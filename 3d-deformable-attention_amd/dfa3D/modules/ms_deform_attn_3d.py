@@ -20,7 +20,7 @@ from ..functional import (MultiScale3DDeformableAttnFunction_fp32,
                           MultiScale3DDeformableAttnWeightUpdateFunction_fp32)
 from .. import _lib
 from ..recording import OperatorFunction
-from .projection import Projection, ordinary, plain_gradient, projections
+from .projection import Projection, as_plain, ordinary, plain_gradient, projections
 
 __all__ = ["MSDeformableAttention3D_DFA3D"]
 
@@ -57,6 +57,40 @@ class _LocationsFunction(OperatorFunction):
                                                  M, L, P, _lib.stream_of(grad))
         _lib.check(rc, "dfa3d_locations_grad")
         return grad_uv, grad_dz, None, None
+
+
+class _SamplingFunction(OperatorFunction):
+    """As ``_LocationsFunction``, and logits (bs, Q, M, L, P) to their softmax over a head's points: ``apply(uv, dz, logits, reference_points, shapes3)``."""
+
+    own = True
+
+    @staticmethod
+    def forward(ctx, uv, dz, logits, reference_points, shapes3):
+        bs, Q, M, L, P = logits.shape
+        loc, attn = logits.new_empty(bs, Q, M, L, P, 3), logits.new_empty(bs, Q, M, L, P)
+        if attn.numel():
+            with _lib.on_device(uv.device):
+                rc = _lib.lib().dfa3d_sampling(_lib.ptr(uv), _lib.ptr(dz), _lib.ptr(logits), _lib.ptr(reference_points), _lib.ptr(shapes3),
+                                               _lib.ptr(loc), _lib.ptr(attn), bs * Q, M, L, P, reference_points.shape[2], _lib.stream_of(uv))
+            _lib.check(rc, "dfa3d_sampling")
+        ctx.save_for_backward(shapes3, attn)
+        return loc, attn
+
+    @staticmethod
+    def backward(ctx, grad_loc, grad_attn):
+        shapes3, attn = ctx.saved_tensors
+        if not (plain_gradient(grad_loc) and plain_gradient(grad_attn) and as_plain(attn, grad_attn)) or attn.numel() == 0:
+            scaled = grad_loc / shapes3[:, [1, 0, 2]].to(grad_loc.dtype)[None, None, None, :, None, :]
+            weighted = grad_attn * attn
+            return scaled[..., :2], scaled[..., 2:], weighted - attn * weighted.sum((-1, -2), keepdim=True), None, None
+        grad_loc, grad_attn = grad_loc.contiguous(), grad_attn.contiguous()
+        bs, Q, M, L, P = attn.shape
+        grad_uv, grad_dz, grad_logits = attn.new_empty(bs, Q, M, L, P, 2), attn.new_empty(bs, Q, M, L, P, 1), attn.new_empty(attn.shape)
+        with _lib.on_device(attn.device):
+            rc = _lib.lib().dfa3d_sampling_grad(_lib.ptr(grad_loc), _lib.ptr(grad_attn), _lib.ptr(attn), _lib.ptr(shapes3), _lib.ptr(grad_uv),
+                                                _lib.ptr(grad_dz), _lib.ptr(grad_logits), bs * Q, M, L, P, _lib.stream_of(attn))
+        _lib.check(rc, "dfa3d_sampling_grad")
+        return grad_uv, grad_dz, grad_logits, None, None
 
 
 class MSDeformableAttention3D_DFA3D(nn.Module):
@@ -162,16 +196,29 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         M, L, P = self.num_heads, self.num_levels, self.num_points
         Z = reference_points.shape[2]
         uv, dz = uv.view(bs, Q, M, L, P, 2), dz.view(bs, Q, M, L, P, 1)
-        if (ordinary(uv, dz, reference_points) and uv.is_contiguous() and dz.is_contiguous()
-                and reference_points.is_contiguous() and not reference_points.requires_grad
-                and reference_points.shape[:2] == (bs, Q) and spatial_shapes_3D.device == uv.device
-                and spatial_shapes_3D.dtype == torch.int64 and spatial_shapes_3D.shape == (L, 3)):
+        if self._by_kernel(uv, dz, reference_points, spatial_shapes_3D):
             return _LocationsFunction.apply(uv, dz, reference_points, spatial_shapes_3D.contiguous())
         normalizer = spatial_shapes_3D[:, [1, 0, 2]].to(dtype)              # (W, H, D) per level
         offsets = torch.cat([uv, dz], dim=-1) / normalizer[None, None, None, :, None, :]
         anchors = reference_points[:, :, None, None, None, :, :]                   # (bs, Q, 1, 1, 1, Z, 3)
         loc = offsets.view(bs, Q, M, L, P // Z, Z, 3) + anchors
         return loc.view(bs, Q, M, L, P, 3)
+
+    def _by_kernel(self, uv, dz, reference_points, spatial_shapes_3D, *others):
+        return (ordinary(uv, dz, reference_points, *others) and all(t.is_contiguous() for t in (uv, dz, reference_points, *others))
+                and not reference_points.requires_grad and reference_points.shape[:2] == uv.shape[:2] and spatial_shapes_3D.device == uv.device
+                and spatial_shapes_3D.dtype == torch.int64 and spatial_shapes_3D.shape == (self.num_levels, 3))
+
+    def _sampling(self, uv, dz, logits, reference_points, spatial_shapes_3D, dtype):
+        """Locations (as ``_locations``) and attention weights from the results of the three layers of the queries.  In one kernel where a head's
+        points are a power of two that a wavefront has lanes for; else the softmax is torch's."""
+        bs, Q, _ = uv.shape
+        M, L, P = self.num_heads, self.num_levels, self.num_points
+        if L * P <= 64 and L * P & (L * P - 1) == 0 and self._by_kernel(uv, dz, reference_points, spatial_shapes_3D, logits):
+            return _SamplingFunction.apply(uv.view(bs, Q, M, L, P, 2), dz.view(bs, Q, M, L, P, 1), logits.view(bs, Q, M, L, P), reference_points,
+                                           spatial_shapes_3D.contiguous())
+        weights = logits.view(bs, Q, M, L * P).softmax(-1).view(bs, Q, M, L, P)
+        return self._locations(uv, dz, reference_points, spatial_shapes_3D, dtype), weights
 
     def _check_values(self, value, value_dpt_dist, spatial_shapes):
         if spatial_shapes.shape[0] != self.num_levels:
@@ -244,11 +291,11 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
         if value_side is None:
             value_side = self._value_side(value, value_dpt_dist, spatial_shapes, key_padding_mask)
         value, dist, spatial_shapes_3D = value_side
-        attention_weights = attention_weights.view(bs, num_query, self.num_heads, self.num_levels * self.num_points).softmax(-1)
-        attention_weights = attention_weights.view(bs, num_query, self.num_heads, self.num_levels, self.num_points)
         if together:
-            sampling_locations = self._locations(uv, dz, reference_points, spatial_shapes_3D, query.dtype)
+            sampling_locations, attention_weights = self._sampling(uv, dz, attention_weights, reference_points, spatial_shapes_3D, query.dtype)
         else:
+            attention_weights = attention_weights.view(bs, num_query, self.num_heads, self.num_levels * self.num_points).softmax(-1)
+            attention_weights = attention_weights.view(bs, num_query, self.num_heads, self.num_levels, self.num_points)
             sampling_locations = self.sampling_locations(query, reference_points, spatial_shapes_3D)
 
         if not value.is_cuda:

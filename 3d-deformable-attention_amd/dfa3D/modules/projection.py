@@ -109,7 +109,7 @@ def plain_gradient(grad):
             and not torch._C._functorch.is_batchedtensor(grad) and not torch._C._functorch.is_legacy_batchedtensor(grad))
 
 
-def _as_plain(saved, grad):
+def as_plain(saved, grad):
     """A saved tensor (whatever a hook made of it) that a kernel may read beside the gradient."""
     return saved.dtype == grad.dtype and saved.device == grad.device and saved.is_contiguous() and not saved.is_neg()
 
@@ -166,7 +166,7 @@ def _layer_gradients(x, grad, want_weight, want_bias):
     if not want_weight:
         return None, grad_rows.sum(0) if want_bias else None
     rows = x.reshape(-1, x.shape[-1]).contiguous()
-    if not (plain_gradient(grad) and _as_plain(rows, grad)):
+    if not (plain_gradient(grad) and as_plain(rows, grad)):
         return grad_rows.t().mm(rows), grad_rows.sum(0) if want_bias else None
     return _weight_gradients(rows, grad_rows.contiguous(), want_bias)
 
@@ -194,7 +194,7 @@ class _SharedRowsFunction(Function):
         out = [None] * (2 * len(grads))
         together = [i for i in there if wanted[2 * i]]         # (the layers whose weight's gradient is wanted)
         rows = x.reshape(-1, x.shape[-1]).contiguous() if len(together) > 1 else None
-        if rows is not None and all(plain_gradient(grads[i]) and _as_plain(rows, grads[i]) for i in together):
+        if rows is not None and all(plain_gradient(grads[i]) and as_plain(rows, grads[i]) for i in together):
             formed = _several_weight_gradients(rows, [grads[i].reshape(-1, grads[i].shape[-1]) for i in together],
                                                [wanted[2 * i + 1] for i in together])
             for i, pair in zip(together, formed):
