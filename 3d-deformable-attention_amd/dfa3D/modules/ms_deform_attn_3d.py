@@ -25,6 +25,11 @@ from .projection import Projection, as_plain, ordinary, plain_gradient, projecti
 __all__ = ["MSDeformableAttention3D_DFA3D"]
 
 
+def _readable(shapes3, grad):
+    """Whether a kernel may read the saved level table (whatever a hook made of it) beside the gradient."""
+    return shapes3.device == grad.device and shapes3.dtype == torch.int64 and shapes3.is_contiguous()
+
+
 class _LocationsFunction(OperatorFunction):
     """uv (bs, Q, M, L, P, 2), dz (bs, Q, M, L, P, 1), reference points (bs, Q, Z, 3) and shapes (L, 3) to sampling locations
     in one kernel; differentiable in uv and dz, any number of times."""
@@ -46,8 +51,8 @@ class _LocationsFunction(OperatorFunction):
     @staticmethod
     def backward(ctx, grad):
         shapes3, = ctx.saved_tensors
-        if not plain_gradient(grad) or grad.numel() == 0:
-            scaled = grad / shapes3[:, [1, 0, 2]].to(grad.dtype)[None, None, None, :, None, :]
+        if not plain_gradient(grad) or not _readable(shapes3, grad) or grad.numel() == 0:
+            scaled = grad / shapes3[:, [1, 0, 2]].to(grad.device, grad.dtype)[None, None, None, :, None, :]
             return scaled[..., :2], scaled[..., 2:], None, None
         grad = grad.contiguous()
         bs, Q, M, L, P, _ = grad.shape
@@ -79,8 +84,8 @@ class _SamplingFunction(OperatorFunction):
     @staticmethod
     def backward(ctx, grad_loc, grad_attn):
         shapes3, attn = ctx.saved_tensors
-        if not (plain_gradient(grad_loc) and plain_gradient(grad_attn) and as_plain(attn, grad_attn)) or attn.numel() == 0:
-            scaled = grad_loc / shapes3[:, [1, 0, 2]].to(grad_loc.dtype)[None, None, None, :, None, :]
+        if not (plain_gradient(grad_loc) and plain_gradient(grad_attn) and as_plain(attn, grad_attn) and _readable(shapes3, attn)) or attn.numel() == 0:
+            scaled = grad_loc / shapes3[:, [1, 0, 2]].to(grad_loc.device, grad_loc.dtype)[None, None, None, :, None, :]
             weighted = grad_attn * attn
             return scaled[..., :2], scaled[..., 2:], weighted - attn * weighted.sum((-1, -2), keepdim=True), None, None
         grad_loc, grad_attn = grad_loc.contiguous(), grad_attn.contiguous()

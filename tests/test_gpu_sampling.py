@@ -68,3 +68,22 @@ def test_module_takes_it_where_it_may(L, P, kernel):
     with torch.autocast("cuda", torch.bfloat16):
         loc, attn = mod._sampling(uv, dz, logits, ref, shapes, torch.float32)
         assert "Sampling" not in attn.grad_fn.name()
+
+
+def test_with_saved_tensors_elsewhere():
+    """Hooks that keep saved tensors on the host, or bring them back as others: the gradients stay the same."""
+    from dfa3D.modules.ms_deform_attn_3d import _LocationsFunction, _SamplingFunction
+    torch.manual_seed(0)
+    uv, dz, logits = (torch.randn(1, 9, 2, 2, 4, *s, device="cuda", requires_grad=True) for s in ((2,), (1,), ()))
+    ref, shapes = torch.rand(1, 9, 1, 3, device="cuda"), torch.tensor([[20, 30, 8], [10, 15, 8]], device="cuda")
+    want = torch.autograd.grad([t.square().sum() for t in _SamplingFunction.apply(uv, dz, logits, ref, shapes)], (uv, dz, logits))
+    # back on the GPU; left on the host (the level table alone: what meets the gradients has to be where they are); strided
+    for unpack in (lambda t: t.cuda(), lambda t: t if t.dtype == torch.int64 else t.cuda(), lambda t: t.cuda().t().contiguous().t() if t.dim() == 2 else t.cuda()):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), unpack):
+            loc, attn = _SamplingFunction.apply(uv, dz, logits, ref, shapes)
+            alone = _LocationsFunction.apply(uv, dz, ref, shapes)
+        g = 2 * loc.detach(), 2 * attn.detach()
+        for a, b in zip(torch.autograd.grad((loc, attn), (uv, dz, logits), g), want):
+            torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-6)
+        for a, b in zip(torch.autograd.grad(alone, (uv, dz), g[0]), want):
+            torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-6)
