@@ -20,7 +20,7 @@ def camera_count(hit):
     cams, Nq = hit.shape
     if not (hit.is_cuda and hit.dtype == torch.bool and hit.is_contiguous() and 0 < cams <= 65535 and 0 < Nq <= 2 ** 30):
         return None
-    totals = torch.empty(cams, 1, dtype=torch.int32, device=hit.device)
+    totals = torch.empty(cams, dtype=torch.int32, device=hit.device)
     with _lib.on_device(hit.device):
         rc = _lib.lib().dfa3d_camera_count(_lib.ptr(hit), _lib.ptr(totals), cams, Nq, _lib.stream_of(hit))
         _lib.check(rc, "dfa3d_camera_count")
@@ -28,7 +28,7 @@ def camera_count(hit):
 
 
 def _on_their_way(counts):
-    """``counts`` (cams, parts) on the GPU, the same on the host, and the event after which the host has them."""
+    """``counts`` (cams,) or (cams, parts) on the GPU, the same on the host, and the event after which the host has them."""
     on_host = torch.empty(counts.shape, dtype=torch.int32, device="cpu", pin_memory=True)      # (whatever the default device)
     on_host.copy_(counts, non_blocking=True)
     done = torch.cuda.Event()
@@ -85,7 +85,7 @@ def _camera_index_on_gpu(hit, totals, on_host, done):
     pos = torch.empty(cams, Nq, dtype=torch.int32, device=dev)
     with _lib.on_device(dev):
         done.synchronize()                                          # waits for the device
-        max_len = max(map(sum, on_host.tolist()))
+        max_len = max(map(sum, on_host.view(cams, -1).tolist()))
         index = torch.empty(cams, max(max_len, 1), dtype=torch.int32, device=dev)
         _lib.check(lib.dfa3d_camera_index(_lib.ptr(hit), _lib.ptr(totals), _lib.ptr(index), _lib.ptr(pos), cams, Nq,
                                           max(max_len, 1), _lib.stream_of(hit)), "dfa3d_camera_index")

@@ -54,7 +54,7 @@ def test_counts_with_the_hits(cams, bs, Nq, Z, share):
     assert torch.equal(hit.cpu(), want_hit) and torch.equal(scale.cpu(), want_scale)
     got, want = camera_index(hit, counted), camera_index(want_hit)
     assert got[2] == want[2] and torch.equal(got[0].cpu(), want[0]) and torch.equal(got[1].cpu(), want[1])
-    assert torch.equal(counted[0].sum(1).cpu(), want_hit.sum(1))
+    assert torch.equal(counted[0].view(cams, -1).sum(1).cpu(), want_hit.sum(1))
 
 
 def test_counts_of_other_masks():
