@@ -642,7 +642,9 @@ template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a)
 //     46 x 80, 128 bins, 3 x 8   3.0 MB   153, 225, 231   159, 222, 222   171, 217, 216      70 x 119, 112 bins         6.1 MB   240, 367, 335   226, 354, 317   232, 340, 303
 //     58 x 100, 80 bins          3.3 MB   197, 300, 293   193, 294, 281   200, 284, 270      116 x 200, 16 channels     9.4 MB   244, 375, 338   225, 358, 320   230, 344, 310
 //     100 x 170, 16 bins, 1 x 4  3.1 MB   106, 125, 121   106, 123, 116   106, 123, 116      116 x 200, 64 bins        11.3 MB   283, 415, 376   263, 401, 360   268, 389, 354
-//     so an eighth from 3.5 MB, three sixteenths from 6 MB on, one point at least (of 3 or 4: 116 x 200, one level 154, 179, 149 -> 146, 171, 140 and 168, 212, 172 -> 161,
+//     one distribution for all heads (not packed: few points), none / an eighth: 65 x 116, 128 bins, 2 x 8, 2000 queries 6.0 MB 18.1, 18.2 around the query; 116 x 200, 64 bins
+//     11.3 MB 232, 357, 328 -> 224, 347, 318: from 8 MB on.
+//     So an eighth from 3.5 MB, three sixteenths from 6 MB on, one point at least (of 3 or 4: 116 x 200, one level 154, 179, 149 -> 146, 171, 140 and 168, 212, 172 -> 161,
 //     205, 162); a quarter: 64 bins 292, 385, 343.
 //   The coarser levels in LDS, 10000 queries, none / an eighth:
 //     58 x 100, 16 bins    1.5 MB   323, 499, 517   359, 478, 483      80 x 128, 64 bins, 3 x 8   5.2 MB   680, 1027, 965   697, 998, 925
@@ -660,6 +662,7 @@ template <typename T> static int points_by_scalar(const FwdArgs &a, const LdsRow
   const int eighth = LP / 8, three_sixteenths = (3 * LP + 15) / 16;
   if (sizeof(T) == 2) return lds.parts == 0 && bytes > (5LL << 20) ? three_sixteenths : 0;
   if (lds.parts > 0) return bytes > (11LL << 19) ? eighth : 0;
+  if (a.dist_heads == 1) return bytes > (8LL << 20) ? eighth : 0;
   return bytes > (6LL << 20) ? three_sixteenths : bytes > (7LL << 19) ? std::max(eighth, 1) : 0;
 }
 
