@@ -353,6 +353,22 @@ __global__ __launch_bounds__(kIndexBlock) void camera_count_kernel(const uint8_t
   if (threadIdx.x == 0) totals[blockIdx.x] = n;
 }
 
+// This thread's share of the number of bytes among hit[0 .. n) that are not zero: whole words, and the bytes before and after them.  (Byte by
+// byte, lists of six cameras, 22500 queries 5.6 us for 3.6, 40000 7.8 for 4.0, 160000 37 for 11.)
+__device__ __forceinline__ int hits_before(const uint8_t *__restrict__ hit, int n) {
+  const int head = min((int)(-(uintptr_t)hit & 3), n), words = (n - head) / 4, rest = n - 4 * words;      // rest: the bytes that are in no word
+  const uint32_t *__restrict__ const word = reinterpret_cast<const uint32_t *>(hit + head);
+  int sum = 0;
+#pragma unroll 4
+  for (int k = threadIdx.x; k < words; k += kIndexBlock) {
+    const uint32_t w = word[k];
+    sum += __popc((((w & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | w) & 0x80808080u);
+  }
+  const int t = threadIdx.x;
+  if (t < rest) sum += hit[t < head ? t : t + 4 * words] != 0;
+  return sum;
+}
+
 // A block ranks kIndexBlock queries of one camera; it counts the hits before them itself instead of waiting for the
 // blocks that rank those.  pos is written whole, index from 0 to max_len: ranks, then the padding, in which a query that is no hit takes the place from
 // the end that it has among those.
@@ -362,9 +378,7 @@ __global__ __launch_bounds__(kIndexBlock) void camera_index_kernel(const uint8_t
   const int cam = blockIdx.y, first = blockIdx.x * kIndexBlock, q = first + threadIdx.x;
   const uint8_t *mine = hit + (long long)cam * Nq;
   int *index_row = index + (long long)cam * max_len;
-  int before = 0;
-  for (int k = threadIdx.x; k < first; k += kIndexBlock) before += mine[k] != 0;
-  before = block_sum(before, s_part);
+  const int before = block_sum(hits_before(mine, first), s_part);
   const bool on = q < Nq && mine[q] != 0;
   const unsigned long long lanes = __ballot(on);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;

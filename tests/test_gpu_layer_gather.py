@@ -99,3 +99,15 @@ def test_layer_with_positions_in_other_forms():
             torch.testing.assert_close(g.float(), w, rtol=1e-5, atol=1e-5)
     few = pos[:1].detach().expand(bs, Nq, E)
     torch.testing.assert_close(layer(query, feats, feats, query_pos=few, **args), layer(query, feats, feats, query_pos=pos[:1].detach(), **args), rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("Nq", [1023, 1024, 1025, 1026, 1027, 3073, 4099])
+@pytest.mark.parametrize("by", [0, 1, 2, 3])
+def test_lists_of_hits_at_any_byte(Nq, by):
+    """A block counts the hits before its own by whole words, and the bytes around them."""
+    from dfa3D.rebatch import camera_index
+    g = torch.Generator().manual_seed(Nq)
+    hit = torch.rand(3, Nq, generator=g) < 0.4
+    on = torch.zeros(3 * Nq + by, dtype=torch.bool, device="cuda")[by:].view(3, Nq).copy_(hit)
+    got, want = camera_index(on), camera_index(hit)
+    assert got[2] == want[2] and torch.equal(got[0].cpu(), want[0]) and torch.equal(got[1].cpu(), want[1])
