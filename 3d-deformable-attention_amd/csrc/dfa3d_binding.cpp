@@ -69,7 +69,7 @@ struct Operands {
     return need(THPVariable_Unpack(o));
   }
   const Tensor &need(const Tensor &t) {
-    if (!is_plain(t, device) || !t.is_contiguous()) ok = false;
+    if (!is_plain(t, device) || !t.is_contiguous() || t.unsafeGetTensorImpl()->is_python_dispatch()) ok = false;
     return t;
   }
   const Tensor &may_have(PyObject *o) {

@@ -27,7 +27,7 @@ __all__ = ["MSDeformableAttention3D_DFA3D"]
 
 def _readable(shapes3, grad):
     """Whether a kernel may read the saved level table (whatever a hook made of it) beside the gradient."""
-    return shapes3.device == grad.device and shapes3.dtype == torch.int64 and shapes3.is_contiguous()
+    return type(shapes3) is torch.Tensor and shapes3.device == grad.device and shapes3.dtype == torch.int64 and shapes3.is_contiguous()
 
 
 class _LocationsFunction(OperatorFunction):

@@ -12,13 +12,15 @@ from .. import _lib
 
 __all__ = ["Projection", "projections", "projection_plus"]
 
+_PLAIN = (torch.Tensor, nn.Parameter)
+
 
 def ordinary(*tensors, dtype=torch.float32):
     """Plain tensors of ``dtype`` on one GPU, outside autocast, functorch transforms, dispatch modes, forward-mode derivatives,
     tracing and compilation: what this package's kernels may stand in for torch operations on."""
     return (not torch.compiler.is_compiling() and not torch.jit.is_tracing() and not torch.is_autocast_enabled()
             and torch._C._len_torch_dispatch_stack() == 0
-            and all(type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.dtype == dtype and not t.is_neg()
+            and all(type(t) in _PLAIN and t.is_cuda and t.dtype == dtype and not t.is_neg()
                     and t.device == tensors[0].device for t in tensors)
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0)
@@ -39,7 +41,7 @@ def _product(x, weight, bias, addend=None):
     """``F.linear`` (plus ``addend``) that nothing records, or None where the kernel does not form it (csrc/dfa3d_binding.cpp says where
     it does) or it is to be recorded."""
     # (the type first: a symbolic tracer's proxy has no truth value)
-    if (type(x) not in (torch.Tensor, nn.Parameter) or not x.is_cuda or torch.compiler.is_compiling()
+    if (type(x) not in _PLAIN or not x.is_cuda or torch.compiler.is_compiling()
             or torch.autograd.forward_ad._current_level >= 0):
         return None
     native = _lib.binding()
@@ -103,15 +105,15 @@ def _several_weight_gradients(x, grads, want_bias):
 
 
 def plain_gradient(grad):
-    """A gradient that a kernel may read: float32 on the GPU, not recorded and not a batch of gradients (is_grads_batched)."""
-    return (not torch.is_grad_enabled() and grad.is_cuda and grad.dtype == torch.float32
+    """A gradient that a kernel may read: a plain float32 tensor on the GPU, not recorded and not a batch of gradients (is_grads_batched)."""
+    return (type(grad) in _PLAIN and not torch.is_grad_enabled() and grad.is_cuda and grad.dtype == torch.float32
             and torch._C._len_torch_dispatch_stack() == 0 and torch.autograd.forward_ad._current_level < 0 and not grad.is_neg()
             and not torch._C._functorch.is_batchedtensor(grad) and not torch._C._functorch.is_legacy_batchedtensor(grad))
 
 
 def as_plain(saved, grad):
     """A saved tensor (whatever a hook made of it) that a kernel may read beside the gradient."""
-    return saved.dtype == grad.dtype and saved.device == grad.device and saved.is_contiguous() and not saved.is_neg()
+    return type(saved) in _PLAIN and saved.dtype == grad.dtype and saved.device == grad.device and saved.is_contiguous() and not saved.is_neg()
 
 
 class _ProjectionFunction(Function):
@@ -249,7 +251,7 @@ def _bare(layer):
 
 def projection_plus(layer, x, addend):
     """``layer(x) + addend`` without a pass over the result for the sum: the layer of the small model, inference, 252 -> 246 us."""
-    if _bare(layer) and not layer.library_forward and type(addend) in (torch.Tensor, nn.Parameter) and addend.shape == (*x.shape[:-1], layer.out_features):
+    if _bare(layer) and not layer.library_forward and type(addend) in _PLAIN and addend.shape == (*x.shape[:-1], layer.out_features):
         if _applies(x, layer) and ordinary(x, addend):
             if addend.is_contiguous():
                 return _ProjectionPlusFunction.apply(x, layer.weight, layer.bias, addend)
