@@ -172,6 +172,12 @@ bool plain_dispatch() {
   return !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
          !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
 }
+// a tracer, a functorch transform, a profiler or another observer sees what this thread calls
+bool observed() {
+  const c10::DispatchKeySet modes = c10::impl::tls_local_dispatch_key_set().included_;
+  return at::hasCallbacks() || torch::jit::tracer::isTracing() || modes.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+         modes.has(c10::DispatchKey::FuncTorchDynamicLayerBackMode);
+}
 #define TAKES(n)                                                                            \
   if (nargs != (n)) { PyErr_SetString(PyExc_TypeError, "wrong number of arguments"); return nullptr; } \
   Operands in; void *stream;                                                                \
@@ -482,7 +488,7 @@ Tensor incoming(const Tensor &g, at::ScalarType like, int64_t device, bool &ok) 
 }
 // the saved tensors' gradients, or false
 bool gradients_of(Kind kind, int64_t step, const variable_list &t, const variable_list &grads, variable_list &to) {
-  if (c10::GradMode::is_enabled() || !plain_dispatch() || !t[0].defined() || !t[0].is_cuda()) return false;
+  if (c10::GradMode::is_enabled() || !plain_dispatch() || observed() || !t[0].defined() || !t[0].is_cuda()) return false;
   Operands in{t[0].get_device()};
   in.locked = false;
   if (c10::hip::current_device() != in.device) return false;
@@ -695,11 +701,7 @@ PyObject *linear_sum(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 PyObject *built_for(PyObject *, PyObject *) { return Py_BuildValue("(si)", DFA3D_BUILT_FOR, DFA3D_ABI_VERSION); }
 
 // seen() -> whether a tracer, a functorch transform, a profiler or another observer sees what this thread calls
-PyObject *seen(PyObject *, PyObject *) {
-  const c10::DispatchKeySet modes = c10::impl::tls_local_dispatch_key_set().included_;
-  return PyBool_FromLong(at::hasCallbacks() || torch::jit::tracer::isTracing() || modes.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
-                         modes.has(c10::DispatchKey::FuncTorchDynamicLayerBackMode));
-}
+PyObject *seen(PyObject *, PyObject *) { return PyBool_FromLong(observed()); }
 
 // bind(dict of entry point -> address)
 PyObject *bind(PyObject *, PyObject *table) {

@@ -84,3 +84,16 @@ def test_layers_whose_saved_tensors_are_held_elsewhere(rows):
     for a, b in zip(torch.autograd.grad(out, leaves, up), want):
         assert type(a) is torch.Tensor
         assert (a - b).norm() <= 2e-6 * b.norm()               # sums in another order
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_profiler_that_comes_for_the_backward_sees_it(kind, by_python):
+    args = _args(kind)
+    out, leaves = _record(kind, args)
+    up = _upstream(out)
+    want = torch.autograd.grad(out, leaves, up, retain_graph=True)
+    assert _is_native(out[0]) and not by_python
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+        got = torch.autograd.grad(out, leaves, up)
+    _close(got, want)
+    assert len(by_python) == 1
