@@ -19,6 +19,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -551,6 +552,44 @@ struct MultiScale3DDeformableAttnFunction : Recorded<MultiScale3DDeformableAttnF
 struct MultiScale3DDeformableAttnWeightUpdateFunction : Recorded<MultiScale3DDeformableAttnWeightUpdateFunction, kWeightUpdate> {};
 }  // namespace dfa3d
 namespace {
+// What Python sees of a node: the name of its class and what a node made in Python has of its context.
+template <typename F> torch::autograd::CppNode<F> &node_of(PyObject *o) {
+  return *static_cast<torch::autograd::CppNode<F> *>(reinterpret_cast<torch::autograd::THPCppFunction *>(o)->cdata.get());
+}
+template <typename F> PyObject *saved_tensors(PyObject *o, void *) {
+  HANDLE_TH_ERRORS
+  return python_tuple(node_of<F>(o).ctx_.get_saved_variables());
+  END_HANDLE_TH_ERRORS
+}
+template <typename F> PyObject *im2col_step(PyObject *o, void *) {
+  HANDLE_TH_ERRORS
+  return PyLong_FromLongLong(node_of<F>(o).ctx_.saved_data.at("step").toInt());
+  END_HANDLE_TH_ERRORS
+}
+// of the tensors and the step
+template <typename F> PyObject *needs_input_grad(PyObject *o, void *) {
+  HANDLE_TH_ERRORS
+  const auto &edges = node_of<F>(o).next_edges();
+  PyObject *to = PyTuple_New((Py_ssize_t)edges.size() + 1);
+  if (to == nullptr) return nullptr;
+  for (size_t i = 0; i <= edges.size(); ++i) PyTuple_SET_ITEM(to, (Py_ssize_t)i, PyBool_FromLong(i < edges.size() && edges[i].is_valid()));
+  return to;
+  END_HANDLE_TH_ERRORS
+}
+template <typename F> void show_as(const char *name) {
+  using namespace torch::autograd;
+  static PyGetSetDef properties[] = {THP_FUNCTION_DEFAULT_PROPERTIES,
+                                     {"saved_tensors", saved_tensors<F>, nullptr, nullptr, nullptr},
+                                     {"im2col_step", im2col_step<F>, nullptr, nullptr, nullptr},
+                                     {"needs_input_grad", needs_input_grad<F>, nullptr, nullptr, nullptr},
+                                     {nullptr, nullptr, nullptr, nullptr, nullptr}};
+  static PyTypeObject type;
+  if (type.tp_name != nullptr) return;                       // (already)
+  torch::autograd::_initFunctionPyTypeObject(type, name, properties, nullptr);
+  Py_INCREF(&type);
+  torch::autograd::registerCppFunction(typeid(torch::autograd::CppNode<F>), &type);
+}
+
 // the outputs with a node behind them, where one is to be made
 template <typename F, typename... Tensors> variable_list recorded_outputs(variable_list outputs, int64_t step, const Tensors &...inputs) {
   if (!c10::GradMode::is_enabled() || !(inputs.requires_grad() || ...)) return outputs;
@@ -705,6 +744,7 @@ PyObject *seen(PyObject *, PyObject *) { return PyBool_FromLong(observed()); }
 
 // bind(dict of entry point -> address)
 PyObject *bind(PyObject *, PyObject *table) {
+  HANDLE_TH_ERRORS
   auto address = [&](const char *name, auto &to) {
     PyObject *o = PyDict_Check(table) ? PyDict_GetItemString(table, name) : nullptr;
     void *p = o != nullptr ? PyLong_AsVoidPtr(o) : nullptr;
@@ -728,7 +768,13 @@ PyObject *bind(PyObject *, PyObject *table) {
       !address("dfa3d_linear_add", a.linear_add) || !address("dfa3d_linear_sum", a.linear_sum))
     return nullptr;
   api = a;
+  show_as<dfa3d::MultiScaleDepthScoreSampleFunction>("MultiScaleDepthScoreSampleFunctionBackward");
+  show_as<dfa3d::WeightedMultiScaleDeformableAttnFunction>("WeightedMultiScaleDeformableAttnFunctionBackward");
+  show_as<dfa3d::MultiScaleDeformableAttnFunction>("MultiScaleDeformableAttnFunctionBackward");
+  show_as<dfa3d::MultiScale3DDeformableAttnFunction>("MultiScale3DDeformableAttnFunctionBackward");
+  show_as<dfa3d::MultiScale3DDeformableAttnWeightUpdateFunction>("MultiScale3DDeformableAttnWeightUpdateFunctionBackward");
   Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
 }
 
 typedef PyObject *(*Fast)(PyObject *, PyObject *const *, Py_ssize_t);

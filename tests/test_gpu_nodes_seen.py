@@ -97,3 +97,33 @@ def test_a_profiler_that_comes_for_the_backward_sees_it(kind, by_python):
         got = torch.autograd.grad(out, leaves, up)
     _close(got, want)
     assert len(by_python) == 1
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_what_a_node_shows(monkeypatch, kind):
+    """The class's name, the tensors that are saved and the step, as a node made in Python has them."""
+    args = _args(kind)
+    args[-1] = 32
+    shown = []
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(KINDS[kind], "kind", None)
+        out, leaves = _record(kind, args)
+        node = out[0].grad_fn
+        assert _is_native(out[0]) == native and node.im2col_step == 32 and isinstance(node.saved_tensors, tuple)
+        for t, a in zip(node.saved_tensors, args):
+            assert torch.equal(t, a) and t.requires_grad == a.is_floating_point()
+        shown.append((type(node).__name__, len(node.saved_tensors), tuple(node.needs_input_grad)[:len(args)], [n is None for n, _ in node.next_functions]))
+        torch.autograd.grad(out, leaves, _upstream(out))
+        with pytest.raises(RuntimeError, match="second time"):
+            node.saved_tensors
+    assert shown[0] == shown[1]
+    monkeypatch.undo()
+    hooked = torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.cuda())
+    with hooked:
+        out, _ = _record(kind, args)
+    assert _is_native(out[0]) and all(t.is_cuda and torch.equal(t, a) for t, a in zip(out[0].grad_fn.saved_tensors, args))
+    first = [a.requires_grad_() if i == 0 else a for i, a in enumerate(_args(kind))]
+    out = KINDS[kind].apply(*first)
+    node = (out if torch.is_tensor(out) else out[0]).grad_fn
+    assert node.needs_input_grad == (True,) + (False,) * (len(first) - 1)
