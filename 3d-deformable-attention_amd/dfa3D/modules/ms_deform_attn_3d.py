@@ -161,8 +161,9 @@ class MSDeformableAttention3D_DFA3D(nn.Module):
     def get_spatial_shape_3D(spatial_shape, depth_dim):
         """(L, 2) -> (L, 3) with the number of depth bins as third extent (spatial_cross_attention.py:584-587)."""
         # one launch for two: a pass of the small model's layer has 18 others, most of them shorter than the host takes to make them
-        if (spatial_shape.dim() == 2 and spatial_shape.shape[1] == 2 and len(spatial_shape) and ordinary(spatial_shape, dtype=torch.int64)
-                and spatial_shape.is_contiguous()):
+        # (for a number that the call takes as it is: numpy's, tensors, floats and what does not fit an int are torch's)
+        if (type(depth_dim) is int and abs(depth_dim) < 2 ** 31 and spatial_shape.dim() == 2 and spatial_shape.shape[1] == 2
+                and len(spatial_shape) and ordinary(spatial_shape, dtype=torch.int64) and spatial_shape.is_contiguous()):
             table = spatial_shape.new_empty(len(spatial_shape), 3)
             with _lib.on_device(table.device):
                 rc = _lib.lib().dfa3d_level_table(_lib.ptr(spatial_shape), _lib.ptr(table), len(table), depth_dim, _lib.stream_of(table))
