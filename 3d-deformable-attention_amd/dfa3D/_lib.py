@@ -16,9 +16,9 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdfa3d_hip.so")
 
 DFA3D_F32, DFA3D_F64, DFA3D_BF16, DFA3D_BF16G = 0, 1, 2, 3
-DFA3D_FEW_POINTS = 2        # launch option `direct`
+DFA3D_FEW_POINTS = 0xDFA3D  # launch option `direct`
 MAX_LINEAR_SETS = 4        # DFA3D_MAX_LINEAR_SETS
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 _P, _I = ctypes.c_void_p, ctypes.c_int
 _DIMS7 = [_I] * 7      # B S M (C|D) L Q P

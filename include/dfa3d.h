@@ -75,7 +75,7 @@ typedef struct dfa3d_launch_options {
                          * kernels and its tile kernel, so that a profiler can time the two parts of the call */
 } dfa3d_launch_options;
 
-#define DFA3D_FEW_POINTS 2   /* dfa3d_launch_options.direct */
+#define DFA3D_FEW_POINTS 0xDFA3D   /* dfa3d_launch_options.direct: none of the values that say yes */
 
 #define DFA3D_EINVAL (-1)   /* null pointer, non-positive dimension, bad stride or dtype */
 #define DFA3D_ERANGE (-2)   /* a dimension exceeds what the kernels index (see dfa3d_last_error) */
@@ -325,7 +325,7 @@ int dfa3d_linear_grads(const float *x, const dfa3d_linear_grad_set *layers, int 
 const char *dfa3d_last_error(void);
 
 /* Library ABI version (bumped when a signature changes). */
-#define DFA3D_ABI_VERSION 10
+#define DFA3D_ABI_VERSION 11
 int dfa3d_abi_version(void);
 
 #ifdef __cplusplus
