@@ -527,7 +527,7 @@ int dfa3d_camera_index(const uint8_t *hit, const int32_t *totals, int32_t *index
   const char *fn = "dfa3d_camera_index";
   if (int rc = check_cameras(fn, cams, 1, Nq, 1)) return rc;
   if (max_len <= 0 || max_len > Nq) return fail(DFA3D_EINVAL, "%s: max_len must be in [1, Nq]", fn);
-  REQUIRE_PTR(fn, hit); REQUIRE_PTR(fn, totals); REQUIRE_PTR(fn, index); REQUIRE_PTR(fn, pos);
+  REQUIRE_PTR(fn, hit); REQUIRE_PTR(fn, index); REQUIRE_PTR(fn, pos);
   return hip_result(dfa3d::launch_camera_index(hit, index, pos, cams, Nq, max_len, (hipStream_t)stream), fn);
 }
 

@@ -79,7 +79,7 @@ def camera_index(hit, counted=None):
     return index, pos, max_len
 
 
-def _camera_index_on_gpu(hit, totals, on_host, done):
+def _camera_index_on_gpu(hit, _, on_host, done):
     cams, Nq = hit.shape
     dev, lib = hit.device, _lib.lib()
     pos = torch.empty(cams, Nq, dtype=torch.int32, device=dev)
@@ -87,7 +87,7 @@ def _camera_index_on_gpu(hit, totals, on_host, done):
         done.synchronize()                                          # waits for the device
         max_len = max(map(sum, on_host.view(cams, -1).tolist()))
         index = torch.empty(cams, max(max_len, 1), dtype=torch.int32, device=dev)
-        _lib.check(lib.dfa3d_camera_index(_lib.ptr(hit), _lib.ptr(totals), _lib.ptr(index), _lib.ptr(pos), cams, Nq,
+        _lib.check(lib.dfa3d_camera_index(_lib.ptr(hit), None, _lib.ptr(index), _lib.ptr(pos), cams, Nq,
                                           max(max_len, 1), _lib.stream_of(hit)), "dfa3d_camera_index")
     return index, pos, max_len
 

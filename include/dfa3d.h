@@ -261,7 +261,7 @@ int dfa3d_rebatch_combine(const void *src, const int32_t *pos, const void *scale
  * hits_counted: hits, and counts (cams, parts), whose rows add up to the totals; at most 1024 cameras.  A part is a workgroup, 1024 queries at a
  *        time.
  * index: index (cams, max_len) lists the queries of each camera in ascending order, padded with -1, and pos (cams, Nq) is
- *        its inverse (-1: not seen); 1 <= max_len <= Nq, the largest of totals (or 1).  totals: its place is kept, its values are not read. */
+ *        its inverse (-1: not seen); 1 <= max_len <= Nq, the largest of totals (or 1).  totals: not read, NULL or anything. */
 int dfa3d_camera_hits(const uint8_t *mask, uint8_t *hit, float *scale, int cams, int bs, int Nq, int Z, void *stream);
 int dfa3d_camera_hits_counted(const uint8_t *mask, uint8_t *hit, float *scale, int32_t *counts, int parts, int cams, int bs, int Nq, int Z,
                               void *stream);
