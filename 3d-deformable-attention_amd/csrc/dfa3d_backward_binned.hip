@@ -1580,26 +1580,48 @@ static size_t workspace_bytes_for(const BwdArgs &a, int kind, int dtype, bool le
 size_t binned_backward_workspace_bytes(const BwdArgs &a, int kind, int dtype) { return workspace_bytes_for(a, kind, dtype); }
 size_t binned_backward_least_workspace_bytes(const BwdArgs &a, int kind, int dtype) { return workspace_bytes_for(a, kind, dtype, true); }
 
-// A backward on the tile kernels is five launches (six for a distribution shared by the heads), of which each takes its 5 us however few points there
-// are, and visits every tile that has one.  The direct kernels are two launches, whose time is the clearing and one atomic per 64-byte
-// piece of what a point adds to, 20 G of which the L2 executes a second: 0.6 ns a point with rows of 32 floats and depth bins.  So the line is where
-// those atomics cost what the tile kernels' launches and tiles do.  The call's kernels alone (captured in a graph), 2 batch elements, 8 heads of 32
-// channels, 64 bins, us, tile kernels and direct, by thousands of points:
-//   40 x 60 and 20 x 30            12: 47, 22    51: 51, 47    128: 58, 91     one distribution for all heads   12: 55, 22    51: 58, 47    128: 66, 90
-//   80 x 120, three levels         19: 94, 33    76: 102, 69   153: 110, 116   16 channels                      12: 45, 19    51: 48, 36    128: 55, 65
-//   116 x 200, four levels         25: 139, 50  102: 175, 100  256: 188, 189   64 channels                      12: 59, 29    51: 62, 68    128: 70, 140
-//   plain attention, 40 x 60       12: 40, 19    51: 42, 35    128: 49, 66     on one level of 200 x 200        12: 113, 26   51: 142, 42   204: 152, 109
-//   stage 1 alone, 40 x 60         12: 55, 20    51: 57, 25    204: 61, 56     116 x 200, 112 bins              25: 104, 55  204: 121, 91   409: 127, 141
-// The lines below lie a tenth or so under the crossings.  With bfloat16 gradients the float sums are written, read and rounded besides.
+// A backward on the tile kernels is five launches (six for a distribution shared by the heads), of which each takes its 5 us however
+// few points there are, and visits every tile that has one.  The direct kernels are two launches, whose time is the clearing and one
+// atomic per 64-byte piece of what a point adds to, 20 G of which the L2 executes a second where points are spread; adds to the same
+// few lines wait for one another, some 40 ns each.  So the direct kernels take calls
+//   * whose atomics, as of spread points, cost less than launches and tiles do: the lines below, drawn where neither points all over the
+//     map, nor around the query, nor clustered (a normal distribution about the middle, 0.15 of the map) lose;
+//   * with at most 6000 points of a batch element, head and level: all of them may lie in one cell;
+//   * with float sums of 80 MB at most, where those are formed for bfloat16 gradients alone: the tile kernels add bfloat16 in place (384
+//     points, 6 x 116 x 200, 66 us; 222 for the direct kernels, whatever the points.  For a shared distribution 240 us and more).
+// The call's kernels alone (captured in a graph), 8 heads of 32 channels, 64 bins, float32, at the line, thousands of points: tile kernels,
+// direct; all over, around the query, clustered | normal, 0.02 of the map | all in one cell:
+//   2 x 40 x 60 and 20 x 30       43: 45, 37   46, 36   45, 42 | 73, 93 | 85, 104       16 channels     64: 45, 36   45, 35   47, 40 | 66, 114 | 83, 186
+//   2 x 80 x 120, 3 levels        84: 100, 69   98, 68   89, 75 | 81, 139 | 126, 199    64 channels     26: 56, 37   56, 37   53, 39 | 67, 57 | 83, 81
+//   2 x 116 x 200, 4 levels       161: 183, 140   179, 136   146, 144 | 125, 258 | 193, 334
+//   6 x 116 x 200, 4 levels       249: 430, 281   417, 276   311, 286 | 213, 376 | 310, 548    (500: 451, 424   452, 413   352, 431 | 288, 712 | 491, 1057)
+//   one distribution for all heads, 2 x 40 x 60 43: 53, 34   53, 34   53, 41 | 81, 135 | 94, 220
+//     6 x 116 x 200, 4 levels     424: 528, 303   513, 296   426, 328 | 355, 667 | 534, 970
+//   plain, 2 x 40 x 60            55: 36, 31   36, 31   38, 32 | 45, 58 | 81, 117
+//     6 x 116 x 200, 4 levels     375: 303, 185   292, 187   221, 193 | 142, 316 | 254, 497
+//   stage 1 alone, 2 x 40 x 60    54: 48, 20   49, 18   52, 20 | 52, 33 | 65, 136       2 x 116 x 200, 112 bins   87: 99, 61   99, 61   90, 57 | 84, 52 | 112, 251
+//     6 x 116 x 200, 4 levels     140: 157, 137   148, 141   154, 133 | 134, 120 | 158, 130
+//   bfloat16, 2 x 40 x 60         32: 42, 35   43, 35   44, 39 | 148, 71 | 281, 92
+//     2 x 80 x 120, 3 levels      35: 91, 56   87, 55   77, 58 | 125, 79 | 220, 107
+//     sums of 95 MB, 0.5: 41, 49   37: 101, 64   100, 63   81, 63 | 115, 111 | 329, 145   of 189 MB, 25: 129, 99   108, 97   94, 97 | 69, 108 | 140, 122
+//     one distribution for all heads, 6 x 116 x 200, 4 levels   286: 518, 276   507, 274   408, 292 | 409, 507 | 585, 631
+//   more than 6000: 1 x 116 x 200, 10000 of each head 79: 92, 67   92, 65   83, 66 | 61, 105 | 121, 381
 bool few_points(const BwdArgs &a, int kind, int dtype) {
   if (dtype == DFA3D_F64) return true;                       // (no tile kernels)
   const double points = (double)a.B * a.Q * a.M * a.L * a.P, rows = (double)a.B * a.S * a.M;
+  if ((double)a.Q * a.P > 6000) return false;
   const int pieces = (kind == 2 ? 0 : 4 * ((a.C * 4 + 63) / 64)) + (kind == 1 ? 0 : 4);        // that a point adds to
-  const double atomics_us = points * pieces * 0.05e-3;
-  if (kind == 2) return atomics_us < 35 + rows * 0.06e-3;
-  if (kind == 1) return atomics_us < 18 + rows * 0.17e-3;
-  if (a.grad_bf16) return atomics_us < 19 + rows * 0.07e-3;
-  return atomics_us < (shared_dist(a) ? 30 + rows * 0.3e-3 : 25 + rows * 0.2e-3);
+  double atomics_us = points * pieces * 0.05e-3;
+  if (kind == 2) return atomics_us < std::min(10 + rows * 0.02e-3, 28.0);
+  if (kind == 1) return atomics_us < std::min(18 + rows * 0.10e-3, 150.0);
+  // float sums that the tile kernels would not form are cleared, written, read and rounded besides
+  if (a.grad_bf16 && !sums_in_float(a, kind, dtype, tile_config_of(a, kind, dtype))) {
+    const double sums = 4 * rows * a.C + 4 * (double)a.B * a.S * (shared_dist(a) ? 1 : a.M) * a.D;
+    if (sums > 80e6 && !shared_dist(a)) return false;
+    atomics_us += sums * 0.35e-6;
+  }
+  const double line = 16 + rows * 0.16e-3;
+  return atomics_us < (shared_dist(a) ? line : std::min(line, 150.0));
 }
 
 static size_t few_points_value_bytes(const BwdArgs &a) { return ((size_t)a.B * a.S * a.M * a.C * sizeof(float) + 255) & ~(size_t)255; }
