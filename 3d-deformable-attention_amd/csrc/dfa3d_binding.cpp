@@ -653,14 +653,17 @@ PyObject *set_python_backward(PyObject *, PyObject *f) {
   Py_RETURN_NONE;
 }
 
-// Where the kernels form a product of rows x width elements, sums of depth terms.  They read four neighbours of a row at a time, and take the
-// library's place except where few rows meet a deep sum.  Library and kernel, us a call one after the other: 4096 rows of 256 by 256 19, 9; 256 by 64
-// 19, 8; sums of 512 by 256 19, 22; of 2048 by 256 41, 51 to 89; of 1024 by 1024 72, 58; 20000 rows of 512 by 512 98, 70; of 2048 by 256 165, 145; 100000 of
-// 256 by 256 123, 93.  The 18 to 19 are the library call's host time, which bounds it up to some 5000 rows; on the device alone (captured in a graph)
-// 100 rows of 256 by 256 30, 8, 625 rows 5.5, 8.0, 1500 rows 5.6, 8.2, 4096 rows 10, 9; of 256 by 64 4096 rows 5.4, 7.8, 10000 rows 7.3, 8.2.
-// Where several layers' terms are summed (of_several), the library takes a call each and their sums: up to 1024 terms in all the kernel whatever the rows. Three
-// layers of 512, 256 and 256 columns, library and kernel, 64 rows 74, 35; 1000 67, 36 (on the device alone 21, 36); 4000 67, 43 (42, 43); 16000 95, 69; of 256,
-// 128 and 128 67, 21 (18, 21); 32, 24 at 4000; four of 512 1000 rows 92, 74 (40, 74).
+// Where the kernels form a product of rows x width elements, sums of depth terms, in the library's place: they read four neighbours of a
+// row at a time; not where few rows meet a deep sum of one layer; where several layers' terms are summed (of_several), for which the
+// library takes a call each and their sums, with up to 1024 terms in all whatever the rows.  Library and kernels, us:
+//   a call after the other   4096 rows of 256 by 256 20, 8     of 256 by 64 20, 8     20000 of 512 by 512 98, 70     100000 of 256 by 256 123, 93
+//     deep sums of one layer, 4096 rows: of 512 by 256 19, 22     of 2048 by 256 41, 51 to 89     of 1024 by 1024 72, 58
+//   The library's 20 are its host's time, which bounds it up to some 5000 rows.  On the device alone (captured in a graph)
+//     256 by 256   16 rows 9.6, 5.5   100 31, 5.9   625 6.3, 6.1   1500 6.4, 8.1   4096 10.7, 9.2     512 by 256   16 4.5, 5.4   625 6.6, 8.0   2500 10.8, 11.4
+//     256 by 64    100 11.7, 5.8   2500 6.1, 6.2   6600 6.4, 8.4   10000 8.4, 8.7
+//     512, 256 and 256 terms   16 rows 30, 9.1   1000 22, 12   4000 41, 29   16000 100, 74     512 and 512   1000 16, 12   8000 48, 49
+//     256, 128 and 128         1000 18, 9.2   4000 33, 22     128, 64 and 64   1000 17, 8.5   8000 39, 17
+//   So the device alone is up to 2 us slower with the kernels for one layer of some rows and widths; the host's 12 weigh more.
 bool product_applies(int64_t rows, int64_t width, int64_t depth, bool of_several = false) {
   return width > 0 && depth > 0 && width <= 4096 && depth <= 4096 && width % 2 == 0 && depth % 4 == 0 && rows > 0 && rows <= (int64_t(1) << 31) &&
          (depth <= 256 || of_several || rows * width >= (int64_t(1) << 22));

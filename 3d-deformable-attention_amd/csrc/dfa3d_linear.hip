@@ -26,7 +26,10 @@
 // Relative error against float64 (2-norm), the same: forward 2.0e-7, 1.7e-7 (5520 to 10^6 rows); grad_x 2.9e-7, 2.4e-7; weight gradient
 // 184950 rows 6.9e-7, 4.4e-7, 10^6 rows 1.6e-6, 9.6e-7, all positive 6.7e-8, 4.8e-8; grad_bias 2.1e-7, 2.1e-7.  Library's and these, forward
 // and grad_x alike, random signs (all positive): sums of 256 2.9e-7, 2.4e-7 (2.2e-7, 1.8e-7), 512 4.1e-7, 3.4e-7 (3.1e-7, 2.4e-7), 1024 5.7e-7, 4.9e-7
-// (4.3e-7, 2.9e-7), 2048 8.1e-7, 7.0e-7 (6.0e-7, 3.8e-7), 4096 1.2e-6, 1.0e-6 (8.5e-7, 5.3e-7).
+// (4.3e-7, 2.9e-7), 2048 8.1e-7, 7.0e-7 (6.0e-7, 3.8e-7), 4096 1.2e-6, 1.0e-6 (8.5e-7, 5.3e-7).  Of few rows (linear_few_kernel): sums of 256
+// 2.9e-7, 1.2e-7 (2.4e-7, 0.6e-7), of 512, 256 and 256 terms of three layers 3.5e-7, 1.3e-7 (2.0e-7, 0.4e-7).
+#include <algorithm>
+
 #include "../../include/dfa3d.h"
 #include "dfa3d_binned.h"
 #include "dfa3d_device.h"
@@ -214,6 +217,11 @@ template <int MT, int NT> __device__ __forceinline__ bool odd_sums(const f32x16 
   return __builtin_amdgcn_ballot_w64(odd) != 0;
 }
 
+__device__ __forceinline__ bool odd_sum(float sum) {           // of one, but for `large`
+  const uint32_t twice = __float_as_uint(sum) << 1;
+  return twice >= 0xFF000000u || twice - 1 < (__float_as_uint(0x1p-64f) << 1) - 1;
+}
+
 // Whether a thread of the workgroup brought an operand beyond 2^32.  flag: zero since before the last barrier but this one.
 __device__ __forceinline__ bool any_large(float most, int *flag) {
   if (!(most <= 0x1p32f)) *flag = 1;
@@ -355,6 +363,123 @@ __global__ __launch_bounds__(256, 3) void linear_sum_kernel(LinearSets sets, flo
   store_product<TM, TN>(acc, y + n0 * K + k0, K, ms, K - k0 < TN ? K - k0 : TN, nullptr);
 }
 
+// eight contraction steps of one row or column, as a matrix instruction takes them from a lane, and their parts
+__device__ __forceinline__ void column_parts(const float (&v)[8], bf16x8 (&parts)[3], float &most) {
+  split_parts(v, most, [&](int i, const uint32_t (&p)[4]) {
+    const u32x4 words = {p[0], p[1], p[2], p[3]};
+    parts[i] = __builtin_bit_cast(bf16x8, words);
+  });
+}
+// Element (row, k) lies at row * ld + k, or (ACROSS) at k * ld + row; `r` begins with both and ends with the last valid one.
+template <bool ACROSS> __device__ __forceinline__ void load_eight(rsrc_t r, int ld, int row, int rows, int k, int depth, float (&v)[8]) {
+  if constexpr (ACROSS) {
+    const uint32_t off = row < rows ? (uint32_t)(k * ld + row) * 4 : kNoRow;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off + (uint32_t)(j * ld) * 4, 0, 0));
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; j += 4) {
+      const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r, k + j < depth ? (uint32_t)(row * ld + k + j) * 4 : kNoRow, 0, 0);
+      v[j] = __uint_as_float(t.x); v[j + 1] = __uint_as_float(t.y); v[j + 2] = __uint_as_float(t.z); v[j + 3] = __uint_as_float(t.w);
+    }
+  }
+}
+
+// The same products and sums where the tiles of the two kernels above are few: y (N, cols) = sum over the sets of rows (N, width) weight (cols, width)^T, or
+// (ACROSS) weight (width, cols), + bias + addend.  A workgroup forms 32 x 32, and its four wavefronts take every fourth 16 steps each, straight
+// from memory into registers, four of their steps at a time: a chain a sixteenth as long as those kernels', on up to four times as many workgroups.
+// Sums start from zero every four steps (split_product, FLUSH) and the vector unit adds them up; those of the wavefronts meet in LDS.
+constexpr int kFewTile = 32, kFewSteps = 4;
+template <bool ACROSS>
+__global__ __launch_bounds__(256, 2) void linear_few_kernel(LinearSets sets, const float *__restrict__ bias, const float *__restrict__ addend,
+                                                            float *__restrict__ y, long long N, int cols, int tiles) {
+  __shared__ float s_sum[4][16][kWave];
+  __shared__ int large, any_odd;
+  const long long n0 = (blockIdx.x / (8 * tiles) * 8 + blockIdx.x % 8) * (long long)kFewTile;
+  if (n0 >= N) return;                                        // uniform
+  const int c0 = blockIdx.x % (8 * tiles) / 8 * kFewTile, ms = N - n0 < kFewTile ? (int)(N - n0) : kFewTile;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, half = lane / 32, at = lane % 32;
+  if (threadIdx.x == 0) { large = 0; any_odd = 0; }
+  lds_barrier();
+  auto rows = [&](const LinearSet &s) { return make_rsrc(s.rows + n0 * s.width, (size_t)ms * s.width * 4); };
+  auto weight = [&](const LinearSet &s) {
+    return ACROSS ? make_rsrc(s.weight, (size_t)s.width * cols * 4)
+                  : make_rsrc(s.weight + (size_t)c0 * s.width, (size_t)min(cols - c0, kFewTile) * s.width * 4);
+  };
+  f32x16 acc[1][1], since;
+  zero_sums(acc);
+  float most = 0;
+  for (int i = 0; i < sets.n; ++i) {                          // uniform
+    const LinearSet &s = sets.set[i];
+    const rsrc_t a_r = rows(s), b_r = weight(s);
+    for (int k0 = kStep * wave; k0 < s.width; k0 += 4 * kFewSteps * kStep) {         // uniform
+      float a[kFewSteps][8], b[kFewSteps][8];
+#pragma unroll
+      for (int u = 0; u < kFewSteps; ++u) {
+        const int k = k0 + 4 * u * kStep + 8 * half;
+        load_eight<false>(a_r, s.width, at, kFewTile, k, s.width, a[u]);
+        load_eight<ACROSS>(b_r, ACROSS ? cols : s.width, ACROSS ? c0 + at : at, ACROSS ? cols : kFewTile, k, s.width, b[u]);
+      }
+      __builtin_amdgcn_sched_barrier(0);                       // (all of them under way before the first is waited for)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) since[r] = 0;
+#pragma unroll
+      for (int u = 0; u < kFewSteps; ++u) {
+        bf16x8 pa[3], pb[3];
+        column_parts(a[u], pa, most);
+        column_parts(b[u], pb, most);
+#pragma unroll
+        for (int t = 0; t < 6; ++t) since = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[kProducts[t][0]], pb[kProducts[t][1]], since, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][0][r] += since[r];
+    }
+  }
+  // this thread's four sums: of rows 8 * wave + 4 * half and the three below, column `at`
+  float sum[4];
+  auto meet = [&]() {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s_sum[wave][r][lane] = acc[0][0][r];
+    lds_barrier();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int e = 4 * wave + r;
+      sum[r] = (s_sum[0][e][lane] + s_sum[1][e][lane]) + (s_sum[2][e][lane] + s_sum[3][e][lane]);
+    }
+  };
+  if (!(most <= 0x1p32f)) large = 1;
+  meet();
+  bool odd = large != 0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) odd |= odd_sum(sum[r]);
+  if (odd) any_odd = 1;
+  lds_barrier();
+  if (__builtin_amdgcn_readfirstlane(any_odd) != 0) {         // uniform over the workgroup
+    zero_sums(acc);
+    for (int i = 0; i < sets.n; ++i) {
+      const LinearSet &s = sets.set[i];
+      const rsrc_t a_r = rows(s), b_r = weight(s);
+      for (int k0 = 8 * wave; k0 < s.width; k0 += 32) {
+        float a[4], b[4];
+        load_whole<false>(a_r, s.width, 0, 0, at, k0, s.width, a);
+        load_whole<ACROSS>(b_r, ACROSS ? cols : s.width, ACROSS ? c0 : 0, cols, at, k0, s.width, b);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[k], b[k], acc[0][0], 0, 0, 0);
+      }
+    }
+    meet();
+  }
+  const int col = c0 + at, row = 8 * wave + 4 * half;
+  if (col >= cols) return;
+  const float add = bias != nullptr ? bias[col] : 0.f;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (row + r < ms) {
+      const size_t to = (size_t)(n0 + row + r) * cols + col;
+      y[to] = addend != nullptr ? sum[r] + add + addend[to] : sum[r] + add;
+    }
+}
+
 // y (N, cols) = x (N, depth) times the weight of one layer, whose parts for 32 columns and all of the depth (up to KS * 16 steps) a wavefront keeps in
 // registers: 192 of its 256 (the others are taken too; one or two are spilled, outside of the loop).  A workgroup (8 wavefronts, one per CU) splits
 // its 256 columns once and walks through tiles of 32 rows; what is left of a tile is its rows: straight to LDS two tiles ahead (a thread's own 16
@@ -396,12 +521,6 @@ __device__ __forceinline__ void wave_lds_read() { asm volatile("s_waitcnt lgkmcn
 
 // The parts of a wavefront's 32 columns of a weight, eight contraction steps of one column to a lane and step.
 template <int KS> using ColumnParts = bf16x8[KS][3];
-__device__ __forceinline__ void column_parts(const float (&v)[8], bf16x8 (&parts)[3], float &most) {
-  split_parts(v, most, [&](int i, const uint32_t (&p)[4]) {
-    const u32x4 words = {p[0], p[1], p[2], p[3]};
-    parts[i] = __builtin_bit_cast(bf16x8, words);
-  });
-}
 // Element (column, k) lies at k * ld + column: 32 lanes take a whole line at a time.
 template <int KS> __device__ __forceinline__ void load_columns_across(rsrc_t r, int ld, int col, int cols, ColumnParts<KS> &parts, float &most) {
   float v[KS][8];
@@ -724,7 +843,31 @@ static hipError_t launch_linear_rows(const float *x, const float *w, const float
   return hipGetLastError();
 }
 
+// Where linear_few_kernel takes a product: few 64 x 64 tiles for the depth of the sums, as its own 32 x 32 read operands twice as often.  On the device alone
+// (captured in a graph), the other kernels and this one, us:
+//   x W^T, 256 columns of 256 terms   100 rows 8.0, 5.9   625 (40 tiles) 8.1, 6.2   1500 (96) 8.3, 8.1   2500 (160) 8.7, 10.3     64 columns  6600 (104) 8.4, 8.2
+//     128 columns of 128 terms        625 (20) 5.9, 5.5   1500 (48) 5.9, 5.5   2500 (80) 6.0, 6.8     256 of 64 terms 100 (8) 4.7, 5.0
+//   sums of 512, 256 and 256 terms    16 rows 35.6, 9.1   1000 (64) 37.1, 12.0   4000 (252) 43.0, 27.8   5500 (344) 47.0, 36.8   8000 (500) 50.3, 52.2
+//     of 256, 128 and 128             1000 20.5, 8.3   4000 (252) 22.7, 20.9   5500 (344) 25.7, 26.8     of 128, 64 and 64  2000 (128) 13.2, 12.1   4000 13.9, 18.8
+//     of 64, 32 and 32                1000 (64) 9.0, 7.9   2000 (128) 9.2, 10.8
+static bool few_rows(long long N, int cols, int depth, bool across) {
+  const long long tiles = (N + 63) / 64 * ((cols + 63) / 64);
+  return across ? tiles <= std::min(depth / 2, 384) : depth >= 128 && tiles <= std::min(depth * 3 / 8, 96);
+}
+template <bool ACROSS>
+static hipError_t launch_linear_few(const LinearSets &sets, const float *bias, const float *addend, float *y, long long N, int cols, hipStream_t stream) {
+  const int tiles = (cols + kFewTile - 1) / kFewTile;
+  const unsigned blocks = linear_blocks<kFewTile, kFewTile>(N, tiles);
+  if (blocks == 0) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL(linear_few_kernel<ACROSS>, dim3(blocks), dim3(256), 0, stream, sets, bias, addend, y, N, cols, tiles);
+  return hipGetLastError();
+}
+
 hipError_t launch_linear(const float *x, const float *w, const float *bias, const float *addend, float *y, long long N, int O, int K, hipStream_t stream) {
+  if (few_rows(N, O, K, false)) {
+    const LinearSets one = {{{w, x, K}}, 1};
+    return launch_linear_few<false>(one, bias, addend, y, N, O, stream);
+  }
   if (rows_kernel_applies(x, w, N, O, K, false))
     return addend != nullptr ? launch_linear_rows<16, false, true>(x, w, bias, addend, y, N, O, K, stream)
                              : launch_linear_rows<16, false, false>(x, w, bias, nullptr, y, N, O, K, stream);
@@ -741,6 +884,9 @@ template <int TM, int TN, int FLUSH> static hipError_t launch_linear_sum_cfg(con
 }
 
 hipError_t launch_linear_sum(const LinearSets &sets, float *y, long long N, int K, hipStream_t stream) {
+  int depth = 0;
+  for (int i = 0; i < sets.n; ++i) depth += sets.set[i].width;
+  if (few_rows(N, K, depth, true)) return launch_linear_few<true>(sets, nullptr, nullptr, y, N, K, stream);
   const LinearSet &s = sets.set[0];
   if (sets.n == 1 && rows_kernel_applies(s.rows, s.weight, N, K, s.width, true)) return launch_linear_rows<16, true, false>(s.rows, s.weight, nullptr, nullptr, y, N, K, s.width, stream);
   const bool wide = wide_tiles(N, K);
