@@ -1584,44 +1584,46 @@ size_t binned_backward_least_workspace_bytes(const BwdArgs &a, int kind, int dty
 // few points there are, and visits every tile that has one.  The direct kernels are two launches, whose time is the clearing and one
 // atomic per 64-byte piece of what a point adds to, 20 G of which the L2 executes a second where points are spread; adds to the same
 // few lines wait for one another, some 40 ns each.  So the direct kernels take calls
-//   * whose atomics, as of spread points, cost less than launches and tiles do: the lines below, drawn where neither points all over the
-//     map, nor around the query, nor clustered (a normal distribution about the middle, 0.15 of the map) lose;
-//   * with at most 6000 points of a batch element, head and level: all of them may lie in one cell;
+//   * whose atomics, as of spread points, cost less than launches and tiles do: lines drawn where neither points all over the map, nor
+//     around the query, nor clustered (a normal distribution about the middle, 0.15 of the map) lose more than a few percent;
+//   * with at most 8000 (stage 1: 4000) points of a batch element, head and level, ten of a row, four of a line of a shared
+//     distribution: they may lie closer together;
 //   * with float sums of 80 MB at most, where those are formed for bfloat16 gradients alone: the tile kernels add bfloat16 in place (384
 //     points, 6 x 116 x 200, 66 us; 222 for the direct kernels, whatever the points.  For a shared distribution 240 us and more).
 // The call's kernels alone (captured in a graph), 8 heads of 32 channels, 64 bins, float32, at the line, thousands of points: tile kernels,
 // direct; all over, around the query, clustered | normal, 0.02 of the map | all in one cell:
-//   2 x 40 x 60 and 20 x 30       43: 45, 37   46, 36   45, 42 | 73, 93 | 85, 104       16 channels     64: 45, 36   45, 35   47, 40 | 66, 114 | 83, 186
-//   2 x 80 x 120, 3 levels        84: 100, 69   98, 68   89, 75 | 81, 139 | 126, 199    64 channels     26: 56, 37   56, 37   53, 39 | 67, 57 | 83, 81
-//   2 x 116 x 200, 4 levels       161: 183, 140   179, 136   146, 144 | 125, 258 | 193, 334
-//   6 x 116 x 200, 4 levels       249: 430, 281   417, 276   311, 286 | 213, 376 | 310, 548    (500: 451, 424   452, 413   352, 431 | 288, 712 | 491, 1057)
-//   one distribution for all heads, 2 x 40 x 60 43: 53, 34   53, 34   53, 41 | 81, 135 | 94, 220
-//     6 x 116 x 200, 4 levels     424: 528, 303   513, 296   426, 328 | 355, 667 | 534, 970
-//   plain, 2 x 40 x 60            55: 36, 31   36, 31   38, 32 | 45, 58 | 81, 117
-//     6 x 116 x 200, 4 levels     375: 303, 185   292, 187   221, 193 | 142, 316 | 254, 497
-//   stage 1 alone, 2 x 40 x 60    54: 48, 20   49, 18   52, 20 | 52, 33 | 65, 136       2 x 116 x 200, 112 bins   87: 99, 61   99, 61   90, 57 | 84, 52 | 112, 251
-//     6 x 116 x 200, 4 levels     140: 157, 137   148, 141   154, 133 | 134, 120 | 158, 130
-//   bfloat16, 2 x 40 x 60         32: 42, 35   43, 35   44, 39 | 148, 71 | 281, 92
-//     2 x 80 x 120, 3 levels      35: 91, 56   87, 55   77, 58 | 125, 79 | 220, 107
-//     sums of 95 MB, 0.5: 41, 49   37: 101, 64   100, 63   81, 63 | 115, 111 | 329, 145   of 189 MB, 25: 129, 99   108, 97   94, 97 | 69, 108 | 140, 122
-//     one distribution for all heads, 6 x 116 x 200, 4 levels   286: 518, 276   507, 274   408, 292 | 409, 507 | 585, 631
-//   more than 6000: 1 x 116 x 200, 10000 of each head 79: 92, 67   92, 65   83, 66 | 61, 105 | 121, 381
+//   2 x 40 x 60 and 20 x 30       42: 45, 36   46, 36   45, 42 | 75, 89 | 84, 109      16 channels   62: 45, 35   45, 34   46, 39 | 65, 114 | 80, 158
+//                                                                                      64 channels   27: 56, 39   56, 38   53, 40 | 69, 62 | 85, 90
+//   2 x 80 x 120, 3 levels        87: 99, 71   99, 70   89, 76 | 83, 131 | 121, 221
+//   2 x 116 x 200, 128 bins       128: 192, 137   190, 133   155, 131 | 96, 158 | 147, 432
+//   2 x 116 x 200, 4 levels       173: 180, 143   181, 138   147, 147 | 123, 322 | 193, 371
+//   6 x 116 x 200, 4 levels       283: 435, 303   413, 300   318, 314 | 219, 421 | 327, 554     (500: 451, 424   452, 413   352, 431 | 288, 712 | 491, 1057)
+//   one distribution for all heads, 2 x 40 x 60   53: 54, 42   54, 40   56, 49 | 73, 165 | 96, 268
+//     6 x 116 x 200, 4 levels     554: 536, 372   536, 359   443, 408 | 392, 881 | 624, 1182
+//   plain, 2 x 40 x 60            63: 36, 34   36, 33   39, 35 | 48, 67 | 84, 138
+//     6 x 116 x 200, 4 levels     412: 306, 203   304, 203   226, 211 | 152, 347 | 273, 545
+//   stage 1 alone, 2 x 40 x 60    64: 48, 22   49, 20   53, 22 | 53, 36 | 66, 170               (177: 59, 46   61, 41   55, 46 | 61, 91 | 86, 528)
+//     6 x 116 x 200, 4 levels     151: 159, 141   154, 122   158, 148 | 141, 137 | 156, 135
+//   bfloat16, 2 x 40 x 60         31: 42, 35   42, 34   44, 39 | 145, 75 | 275, 88              2 x 80 x 120, 3 levels   42: 93, 60   89, 59   80, 63 | 143, 86 | 259, 129
+//     sums of 95 MB, 0.5: 41, 49   37: 101, 64   100, 63   81, 63 | 115, 111 | 329, 145         of 189 MB   25: 129, 99   108, 97   94, 97 | 69, 108 | 140, 122
+//     one distribution for all heads, 6 x 116 x 200, 4 levels   416: 533, 353   528, 345   420, 374 | 470, 705 | 745, 940
+//   beyond ten of a row: plain, 15 x 21 51: 38, 31   40, 31   48, 61 | 72, 255 | 96, 265; beyond four of a line: 4 x 45 x 70, 4 levels, 16 bins 84: 78, 70   79, 63   74, 109
 bool few_points(const BwdArgs &a, int kind, int dtype) {
   if (dtype == DFA3D_F64) return true;                       // (no tile kernels)
   const double points = (double)a.B * a.Q * a.M * a.L * a.P, rows = (double)a.B * a.S * a.M;
-  if ((double)a.Q * a.P > 6000) return false;
+  if ((double)a.Q * a.P > (kind == 2 ? 4000 : 8000) || points > 10 * rows) return false;
   const int pieces = (kind == 2 ? 0 : 4 * ((a.C * 4 + 63) / 64)) + (kind == 1 ? 0 : 4);        // that a point adds to
   double atomics_us = points * pieces * 0.05e-3;
-  if (kind == 2) return atomics_us < std::min(10 + rows * 0.02e-3, 28.0);
-  if (kind == 1) return atomics_us < std::min(18 + rows * 0.10e-3, 150.0);
+  if (kind == 2) return atomics_us < std::max(40 - rows * 0.01e-3, 10.0);
+  if (kind == 1) return atomics_us < std::min(20 + rows * 0.14e-3, 165.0);
   // float sums that the tile kernels would not form are cleared, written, read and rounded besides
   if (a.grad_bf16 && !sums_in_float(a, kind, dtype, tile_config_of(a, kind, dtype))) {
     const double sums = 4 * rows * a.C + 4 * (double)a.B * a.S * (shared_dist(a) ? 1 : a.M) * a.D;
     if (sums > 80e6 && !shared_dist(a)) return false;
     atomics_us += sums * 0.35e-6;
   }
-  const double line = 16 + rows * 0.16e-3;
-  return atomics_us < (shared_dist(a) ? line : std::min(line, 150.0));
+  if (shared_dist(a)) return points < 4.0 * a.B * a.S * ((a.D * 4 + 63) / 64) && atomics_us < 22 + rows * 0.21e-3;
+  return atomics_us < std::min(17 + rows * (0.08e-3 + 0.001e-3 * (a.C + a.D)), 170.0);
 }
 
 static size_t few_points_value_bytes(const BwdArgs &a) { return ((size_t)a.B * a.S * a.M * a.C * sizeof(float) + 255) & ~(size_t)255; }

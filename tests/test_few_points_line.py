@@ -1,5 +1,5 @@
 """Where the line between the direct and the tile kernels of a backward lies, asked on the host: by the scratch that a call wants.  On both sides of each
-term of the rule: atomics against tiles, points of a batch element, head and level, float sums of bfloat16 gradients."""
+term of the rule: atomics against tiles, points that may lie close together, float sums of bfloat16 gradients."""
 import ctypes
 
 import pytest
@@ -22,19 +22,22 @@ def _direct(kind, B, S, L, Q, P, C=32, D=64, M=8, heads=8, code=_lib.DFA3D_F32):
 
 
 @pytest.mark.parametrize("kind,B,S,L,P,last,options", [
-    ("fused", 2, 3000, 2, 8, 154, {}), ("fused", 2, 3000, 2, 8, 154, dict(heads=1)), ("fused", 2, 3000, 2, 8, 92, dict(C=64)),
-    ("fused", 2, 30825, 4, 8, 308, {}), ("fused", 6, 30825, 4, 8, 162, {}), ("fused", 6, 30825, 4, 8, 274, dict(heads=1)),
-    ("plain", 2, 2400, 1, 4, 853, {}), ("plain", 6, 30825, 4, 8, 244, {}),
-    ("stage 1", 2, 2400, 1, 8, 420, {}), ("stage 1", 6, 30825, 4, 8, 91, {})])
+    ("fused", 2, 3000, 2, 8, 165, {}), ("fused", 2, 3000, 2, 8, 208, dict(heads=1)), ("fused", 2, 3000, 2, 8, 105, dict(C=64)),
+    ("fused", 2, 30825, 4, 8, 337, {}), ("fused", 6, 30825, 4, 8, 184, {}), ("fused", 6, 30825, 4, 8, 361, dict(heads=1)),
+    ("plain", 2, 2400, 1, 4, 991, {}), ("plain", 6, 30825, 4, 8, 268, {}),
+    ("stage 1", 2, 3000, 4, 2, 1543, {}), ("stage 1", 6, 30825, 4, 8, 82, {})])
 def test_last_call_of_the_direct_kernels(kind, B, S, L, P, last, options):
     """A point has an atomic per 64 bytes of its four rows and four for its bins, 0.05 ns each; a call has its base and its rows.  The first:
-    (16 us + 48000 rows * 0.16 ns) / (256 points a query * 12 * 0.05 ns) = 154.2."""
+    (17 us + 48000 rows * 0.176 ns) / (256 points a query * 12 * 0.05 ns) = 165.7."""
     assert _direct(kind, B, S, L, last, P, **options) and not _direct(kind, B, S, L, last + 1, P, **options)
 
 
-def test_points_that_may_lie_in_one_cell():
-    assert _direct("plain", 2, 40000, 1, 1500, 4) and not _direct("plain", 2, 40000, 1, 1501, 4)
-    assert _direct("fused", 2, 23200, 1, 750, 8, D=128) and not _direct("fused", 2, 23200, 1, 751, 8, D=128)
+@pytest.mark.parametrize("kind,B,S,L,P,last,options", [
+    ("plain", 2, 40000, 1, 4, 2000, {}), ("fused", 2, 23200, 1, 8, 1000, dict(D=128)), ("stage 1", 2, 23200, 1, 8, 500, dict(D=112)),
+    ("plain", 1, 315, 1, 4, 787, {}), ("fused", 3, 1040, 4, 4, 32, dict(D=16, heads=1))])
+def test_points_that_may_lie_close_together(kind, B, S, L, P, last, options):
+    """8000 points of a batch element, head and level (4000), ten of a row (2520 rows, 32 points a query), four of a line (3120 lines, 384)."""
+    assert _direct(kind, B, S, L, last, P, **options) and not _direct(kind, B, S, L, last + 1, P, **options)
 
 
 def test_float_sums_of_bfloat16_gradients():
