@@ -1586,7 +1586,7 @@ size_t binned_backward_least_workspace_bytes(const BwdArgs &a, int kind, int dty
 // few lines wait for one another, some 40 ns each.  So the direct kernels take calls
 //   * whose atomics, as of spread points, cost less than launches and tiles do: lines drawn where neither points all over the map, nor
 //     around the query, nor clustered (a normal distribution about the middle, 0.15 of the map) lose more than a few percent;
-//   * with at most 8000 (stage 1: 4000) points of a batch element, head and level, ten of a row, four of a line of a shared
+//   * with at most 8000 (stage 1: 4000) points of a batch element, head and level, ten of a row, three of a line of a shared
 //     distribution: they may lie closer together;
 //   * with float sums of 80 MB at most, where those are formed for bfloat16 gradients alone: the tile kernels add bfloat16 in place (384
 //     points, 6 x 116 x 200, 66 us; 222 for the direct kernels, whatever the points.  For a shared distribution 240 us and more).
@@ -1607,7 +1607,7 @@ size_t binned_backward_least_workspace_bytes(const BwdArgs &a, int kind, int dty
 //   bfloat16, 2 x 40 x 60         31: 42, 35   42, 34   44, 39 | 145, 75 | 275, 88              2 x 80 x 120, 3 levels   42: 93, 60   89, 59   80, 63 | 143, 86 | 259, 129
 //     sums of 95 MB, 0.5: 41, 49   37: 101, 64   100, 63   81, 63 | 115, 111 | 329, 145         of 189 MB   25: 129, 99   108, 97   94, 97 | 69, 108 | 140, 122
 //     one distribution for all heads, 6 x 116 x 200, 4 levels   416: 533, 353   528, 345   420, 374 | 470, 705 | 745, 940
-//   beyond ten of a row: plain, 15 x 21 51: 38, 31   40, 31   48, 61 | 72, 255 | 96, 265; beyond four of a line: 4 x 45 x 70, 4 levels, 16 bins 84: 78, 70   79, 63   74, 109
+//   beyond ten of a row: plain, 15 x 21 51: 38, 31   40, 31   48, 61 | 72, 255 | 96, 265; beyond three of a line: 4 x 45 x 70, 4 levels, 16 bins 84: 78, 70   79, 63   74, 109
 bool few_points(const BwdArgs &a, int kind, int dtype) {
   if (dtype == DFA3D_F64) return true;                       // (no tile kernels)
   const double points = (double)a.B * a.Q * a.M * a.L * a.P, rows = (double)a.B * a.S * a.M;
@@ -1622,7 +1622,7 @@ bool few_points(const BwdArgs &a, int kind, int dtype) {
     if (sums > 80e6 && !shared_dist(a)) return false;
     atomics_us += sums * 0.35e-6;
   }
-  if (shared_dist(a)) return points < 4.0 * a.B * a.S * ((a.D * 4 + 63) / 64) && atomics_us < 22 + rows * 0.21e-3;
+  if (shared_dist(a)) return points < 3.0 * a.B * a.S * ((a.D * 4 + 63) / 64) && atomics_us < 22 + rows * 0.21e-3;
   return atomics_us < std::min(17 + rows * (0.08e-3 + 0.001e-3 * (a.C + a.D)), 170.0);
 }
 

@@ -34,9 +34,9 @@ def test_last_call_of_the_direct_kernels(kind, B, S, L, P, last, options):
 
 @pytest.mark.parametrize("kind,B,S,L,P,last,options", [
     ("plain", 2, 40000, 1, 4, 2000, {}), ("fused", 2, 23200, 1, 8, 1000, dict(D=128)), ("stage 1", 2, 23200, 1, 8, 500, dict(D=112)),
-    ("plain", 1, 315, 1, 4, 787, {}), ("fused", 3, 1040, 4, 4, 32, dict(D=16, heads=1))])
+    ("plain", 1, 315, 1, 4, 787, {}), ("fused", 3, 1040, 4, 4, 24, dict(D=16, heads=1))])
 def test_points_that_may_lie_close_together(kind, B, S, L, P, last, options):
-    """8000 points of a batch element, head and level (4000), ten of a row (2520 rows, 32 points a query), four of a line (3120 lines, 384)."""
+    """8000 points of a batch element, head and level (4000), ten of a row (2520 rows, 32 points a query), three of a line (3120 lines, 384)."""
     assert _direct(kind, B, S, L, last, P, **options) and not _direct(kind, B, S, L, last + 1, P, **options)
 
 
