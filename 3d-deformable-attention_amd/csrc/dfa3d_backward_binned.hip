@@ -1597,17 +1597,22 @@ size_t binned_backward_least_workspace_bytes(const BwdArgs &a, int kind, int dty
 //   2 x 80 x 120, 3 levels        87: 99, 71   99, 70   89, 76 | 83, 131 | 121, 221
 //   2 x 116 x 200, 128 bins       128: 192, 137   190, 133   155, 131 | 96, 158 | 147, 432
 //   2 x 116 x 200, 4 levels       173: 180, 143   181, 138   147, 147 | 123, 322 | 193, 371
-//   6 x 116 x 200, 4 levels       283: 435, 303   413, 300   318, 314 | 219, 421 | 327, 554     (500: 451, 424   452, 413   352, 431 | 288, 712 | 491, 1057)
+//   6 x 116 x 200, 4 levels       283: 435, 303   413, 300   318, 314 | 219, 421 | 327, 554
+//     (beyond the line              500: 451, 424   452, 413   352, 431 | 288, 712 | 491, 1057)
 //   one distribution for all heads, 2 x 40 x 60   53: 54, 42   54, 40   56, 49 | 73, 165 | 96, 268
 //     6 x 116 x 200, 4 levels     554: 536, 372   536, 359   443, 408 | 392, 881 | 624, 1182
 //   plain, 2 x 40 x 60            63: 36, 34   36, 33   39, 35 | 48, 67 | 84, 138
 //     6 x 116 x 200, 4 levels     412: 306, 203   304, 203   226, 211 | 152, 347 | 273, 545
-//   stage 1 alone, 2 x 40 x 60    64: 48, 22   49, 20   53, 22 | 53, 36 | 66, 170               (177: 59, 46   61, 41   55, 46 | 61, 91 | 86, 528)
+//   stage 1 alone, 2 x 40 x 60    64: 48, 22   49, 20   53, 22 | 53, 36 | 66, 170
+//     (beyond the line            177: 59, 46   61, 41   55, 46 | 61, 91 | 86, 528)
 //     6 x 116 x 200, 4 levels     151: 159, 141   154, 122   158, 148 | 141, 137 | 156, 135
-//   bfloat16, 2 x 40 x 60         31: 42, 35   42, 34   44, 39 | 145, 75 | 275, 88              2 x 80 x 120, 3 levels   42: 93, 60   89, 59   80, 63 | 143, 86 | 259, 129
-//     sums of 95 MB, 0.5: 41, 49   37: 101, 64   100, 63   81, 63 | 115, 111 | 329, 145         of 189 MB   25: 129, 99   108, 97   94, 97 | 69, 108 | 140, 122
+//   bfloat16, 2 x 40 x 60         31: 42, 35   42, 34   44, 39 | 145, 75 | 275, 88
+//     2 x 80 x 120, 3 levels      42: 93, 60   89, 59   80, 63 | 143, 86 | 259, 129
+//     sums of 95 MB               0.5: 41, 49   37: 101, 64   100, 63   81, 63 | 115, 111 | 329, 145
+//     of 189 MB                   25: 129, 99   108, 97   94, 97 | 69, 108 | 140, 122
 //     one distribution for all heads, 6 x 116 x 200, 4 levels   416: 533, 353   528, 345   420, 374 | 470, 705 | 745, 940
-//   beyond ten of a row: plain, 15 x 21 51: 38, 31   40, 31   48, 61 | 72, 255 | 96, 265; beyond three of a line: 4 x 45 x 70, 4 levels, 16 bins 84: 78, 70   79, 63   74, 109
+//   beyond ten of a row: plain, 15 x 21                            51: 38, 31   40, 31   48, 61 | 72, 255 | 96, 265
+//   beyond three of a line: 4 x 45 x 70, 4 levels, 16 bins         84: 78, 70   79, 63   74, 109
 bool few_points(const BwdArgs &a, int kind, int dtype) {
   if (dtype == DFA3D_F64) return true;                       // (no tile kernels)
   const double points = (double)a.B * a.Q * a.M * a.L * a.P, rows = (double)a.B * a.S * a.M;

@@ -17,8 +17,8 @@
 // The 8 wavefronts of a workgroup have two roles.  "Walkers" (wavefronts 0-3, one or two tile rows of 8 cells each)
 // walk the cells' lists; "pointers" (wavefronts 4-7, one point of the pass per thread) do everything that is per point:
 // geometry, depth taps, corner weights, the sort, and afterwards the point's gradients and its grad_dist taps into the
-// LDS depth tile.  The roles meet at two barriers per turn and otherwise overlap.  Turns follow one another without a gap, whatever item their passes belong to (pass t: one of
-// the item's passes), so that an item of a single pass costs a single turn:
+// LDS depth tile.  The roles meet at two barriers per turn and otherwise overlap.  Turns follow one another without a gap, whatever item their
+// passes belong to (pass t: one of the item's passes), so that an item of a single pass costs a single turn:
 //   phase X(t):  walkers: walk(t-1)        pointers: scores and corner weights of t, prepare(t+1)
 //   phase Y(t):  walkers: stage(t)         pointers: place(t) (scan + sorted slots), finish(t-1)
 // and where pass t-1 was its item's last:
@@ -310,7 +310,8 @@ __device__ __forceinline__ f4 corner_dots(const WholeRow<T, VEC, LPR> &v, const 
 
 // The two taps (bins db, db + 1) of each of a point's four corners, asked for one phase before they are looked at.
 // The choice between the two ways of 2-byte elements is made once for all four corners: made per corner, each load was followed
-// by a wait for the one before, because the two ways' registers meet after it (six cameras, 30825 rows, 8 x 32 channels, bf16: 990 us for the kernel, now 951).
+// by a wait for the one before, because the two ways' registers meet after it (six cameras, 30825 rows, 8 x 32 channels, bf16: 990 us for the
+// kernel, now 951).
 template <typename T> struct TapsInFlight {
   u32x2 t[4];
   // off: byte offset of bin db of each corner's distribution, kNoRow where there is nothing to fetch
@@ -709,8 +710,8 @@ __global__ __launch_bounds__(kWalkers + cell_pass(LPR), 4) void cell_backward_ke
     // 2-byte elements: four points per step and group.  Each lane of four takes the row of one of them for the dots, which are
     // products of matrices then (v_mfma_f32_4x4x4, four channels deep), and all four take all of them for the sums.
     // The step takes a third of the vector instructions that four steps of one point do, for two and a half times the reads
-    // from LDS, and does the work of four also where a cell has one point (walks_fours()): base shape 1061 -> 1040 us.  With 4-byte elements, where a matrix instruction is one channel deep and a row twice
-    // as long, it lost: plain attention 209 -> 227 us, base shape 1194 -> 1277.
+    // from LDS, and does the work of four also where a cell has one point (walks_fours()): base shape 1061 -> 1040 us.  With 4-byte elements, where
+    // a matrix instruction is one channel deep and a row twice as long, it lost: plain attention 209 -> 227 us, base shape 1194 -> 1277.
     auto walk_fours = [&](const auto &v, f4 (&acc)[VEC]) {
       const Owner o = owner(arg());
       const int corner = o.cl & 3, cell = o.crow * TX + o.ccol;

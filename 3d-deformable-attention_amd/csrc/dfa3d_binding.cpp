@@ -3,9 +3,9 @@
 // took 10 of the 17 us that it cost.
 //
 // Every function takes the operands only where all of them are what its kernels read: plain tensors (no subclass, no transform's
-// wrapper) of the right shapes and types, contiguous, on the device that is current, under no dispatch mode, with something to do.  Anything else is declined
-// (None), and the Python form of the call, which says what is wrong, takes it from there.  The library's entry points come as
-// addresses (bind), so this module serves whichever build of the library is loaded.
+// wrapper) of the right shapes and types, contiguous, on the device that is current, under no dispatch mode, with something to do.  Anything else
+// is declined (None), and the Python form of the call, which says what is wrong, takes it from there.  The library's entry points come as addresses
+// (bind), so this module serves whichever build of the library is loaded.
 #include <Python.h>
 
 #include <ATen/autocast_mode.h>
@@ -659,7 +659,8 @@ PyObject *set_python_backward(PyObject *, PyObject *f) {
 //   a call after the other   4096 rows of 256 by 256 20, 8     of 256 by 64 20, 8     20000 of 512 by 512 98, 70     100000 of 256 by 256 123, 93
 //     deep sums of one layer, 4096 rows: of 512 by 256 19, 22     of 2048 by 256 41, 51 to 89     of 1024 by 1024 72, 58
 //   The library's 20 are its host's time, which bounds it up to some 5000 rows.  On the device alone (captured in a graph)
-//     256 by 256   16 rows 9.6, 5.5   100 31, 5.9   625 6.3, 6.1   1500 6.4, 8.1   4096 10.7, 9.2     512 by 256   16 4.5, 5.4   625 6.6, 8.0   2500 10.8, 11.4
+//     256 by 256   16 rows 9.6, 5.5   100 31, 5.9   625 6.3, 6.1   1500 6.4, 8.1   4096 10.7, 9.2
+//     512 by 256   16 rows 4.5, 5.4   100 6.1, 5.9   625 6.6, 8.0   2500 10.8, 11.4
 //     256 by 64    100 11.7, 5.8   2500 6.1, 6.2   6600 6.4, 8.4   10000 8.4, 8.7
 //     512, 256 and 256 terms   16 rows 30, 9.1   1000 22, 12   4000 41, 29   16000 100, 74     512 and 512   1000 16, 12   8000 48, 49
 //     256, 128 and 128         1000 18, 9.2   4000 33, 22     128, 64 and 64   1000 17, 8.5   8000 39, 17

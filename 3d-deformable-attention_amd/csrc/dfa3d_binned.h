@@ -253,8 +253,8 @@ template <int VEC> __device__ __forceinline__ void lds_ld(const float *p, float 
 // found there is replaced by itself.  With a branch around each of them the round waited for one after the other: tile
 // kernel 1185 -> 1153 us at the base shape, 4366 -> 4251 us dense, 117.3 -> 112.6 us small.
 // Such a round costs the wavefront 60 vector instructions and eight swaps by all lanes.  The float atomic's time goes with the lanes that
-// take part, so it comes at once where few are left (none, 8, 20, 40 of the active ones: tile kernel 1104, 1094, 1081, 1087 us at the base shape, 4092, 4052,
-// 3981, 3987 dense, 106.6, 104.9, 103, 104.8 small), and nothing is looked at again where none is.
+// take part, so it comes at once where few are left (none, 8, 20, 40 of the active ones: tile kernel 1104, 1094, 1081, 1087 us at the base shape,
+// 4092, 4052, 3981, 3987 dense, 106.6, 104.9, 103, 104.8 small), and nothing is looked at again where none is.
 constexpr int kFewLanes = 32;
 __device__ __forceinline__ void lds_add_taps(float *tile, const int (&at)[8], const float (&tv)[8]) {
   uint32_t *words = reinterpret_cast<uint32_t *>(tile);

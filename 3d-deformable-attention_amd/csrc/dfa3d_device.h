@@ -493,9 +493,10 @@ template <typename T, bool LOCAL> struct PairLoader {
   }
 };
 template <bool LOCAL> struct PairLoader<__hip_bfloat16, LOCAL> {
-  // whole_words: the buffer begins and ends on 4-byte boundaries, whatever the number of bins.  Eight 2-byte loads at once spread a point's lines too thin where
-  // caches miss: forward, 4 x 3331 queries, 59 bins, three levels from 37 x 62, 20 channels, anywhere and around the query, corner by corner
-  // 57.6, 45 us, all at once 65, 39, by words 49.4, 38; 4 x 9000 queries, 63 bins, four levels of 8 points from 116 x 197 524, 321; 548, 309; 436, 278.
+  // whole_words: the buffer begins and ends on 4-byte boundaries, whatever the number of bins.  Eight 2-byte loads at once spread a point's lines
+  // too thin where caches miss: forward, 4 x 3331 queries, 59 bins, three levels from 37 x 62, 20 channels, anywhere and around the query, corner
+  // by corner 57.6, 45 us, all at once 65, 39, by words 49.4, 38; 4 x 9000 queries, 63 bins, four levels of 8 points from 116 x 197 524, 321; 548,
+  // 309; 436, 278.
   static __device__ __forceinline__ void ld(rsrc_t r, const uint32_t (&off)[4], int D, bool whole_words, float (&x)[4], float (&y)[4]) {
     if (LOCAL && (D & 3) == 0) {
 #pragma unroll
@@ -564,10 +565,11 @@ template <typename A> struct DepthPair {
   }
   __device__ __forceinline__ A score(A x, A y) const { return depth_lerp(use_x ? x : (A)0, use_y ? y : (A)0, wx, wy); }
 };
-// The two words at each of the four byte offsets `off` of the wavefront's active lanes in `lanes`, by scalar loads: they go round the vector path, whose front end is
-// what gathers wait for.  Four points at a time, all loads before the first result is written back to its lane: left to the compiler, which waits in between, three
-// sixteenths of the base shape's points 577 us for 558 around the query, 824 for 820 anywhere; two or three at a time, an eighth, bfloat16 with 128 bins 525, 520 for 515.  Offsets
-// are read whether the lane has use for them or not: they have to lie in the array.
+// The two words at each of the four byte offsets `off` of the wavefront's active lanes in `lanes`, by scalar loads: they go round the vector path,
+// whose front end is what gathers wait for.  Four points at a time, all loads before the first result is written back to its lane: left to the
+// compiler, which waits in between, three sixteenths of the base shape's points 577 us for 558 around the query, 824 for 820 anywhere; two or three
+// at a time, an eighth, bfloat16 with 128 bins 525, 520 for 515.  Offsets are read whether the lane has use for them or not: they have to lie in
+// the array.
 extern "C" __device__ __attribute__((const)) int dfa3d_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 __device__ __forceinline__ void scalar_pairs(const void *base, unsigned long long lanes, const uint32_t (&off)[4], uint32_t (&first)[4], uint32_t (&second)[4]) {
   constexpr int kPoints = 4;

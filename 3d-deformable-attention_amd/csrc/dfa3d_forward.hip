@@ -127,27 +127,28 @@ template <int FROM, int VEC> __device__ __forceinline__ void sum_over_slots(int 
 // maps), a workgroup of 16 wavefronts brings them there once and walks through a share of the queries: four of a point's eight lines
 // less.  6 x 4000 queries, one level of 23 x 40, 8 points: 53.4 -> 41.0 us (uniform), 41.0 -> 36.4 (points around the query), bfloat16
 // 56.6 -> 51.8, one distribution for all heads 49.1 -> 40.3, plain attention 36.3 -> 28.7; 64 channels, 4 x 4000, 15 x 24: 52.2 -> 32.5.
-// On larger maps the coarser levels' rows: 6 x 10000 queries, four levels from 116 x 200, 8 points (one level in LDS): 915 -> 864 us (884 on another card),
-// points around the query 605 -> 571; bfloat16 (two levels) 842 -> 787, 572 -> 505; plain attention 297 -> 261.  Groups are taken, not dealt:
-// dealt, a workgroup's slowest wavefront held up the CU (883, 614).  Tried with it and not kept: two workgroups of 8, 10 or 12 wavefronts per CU
-// (908, 870, 1031; 596, 625, 706), 16 gathers in flight (880, 623), the next group's locations asked for ahead (850, 581; bfloat16 951) or
-// brought to the L2 by scalar loads (874, 587); the same workgroups without rows in LDS: 942, 603.
+// On larger maps the coarser levels' rows: 6 x 10000 queries, four levels from 116 x 200, 8 points (one level in LDS): 915 -> 864 us (884 on
+// another card), points around the query 605 -> 571; bfloat16 (two levels) 842 -> 787, 572 -> 505; plain attention 297 -> 261.  Groups are taken,
+// not dealt: dealt, a workgroup's slowest wavefront held up the CU (883, 614).  Tried with it and not kept: two workgroups of 8, 10 or 12
+// wavefronts per CU (908, 870, 1031; 596, 625, 706), 16 gathers in flight (880, 623), the next group's locations asked for ahead (850, 581;
+// bfloat16 951) or brought to the L2 by scalar loads (874, 587); the same workgroups without rows in LDS: 942, 603.
 //
 // A quarter of the instructions found places: divisions by the points of a unit and of a level, 64-bit indexes, a product per corner.  What a
 // lane's point has from its place in the group and its level is kept from group to group (IN_LDS), the group's part is in scalars, corners
 // are a row and a column apart, and a slot's tasks lie side by side (656 -> 498 vector instructions per 64 points).  And the wavefronts of a SIMD,
 // which meet at the L1, go by what they hold: one that gathers value rows comes before one that looks for its points' corners, and that before one
-// that begins a group (s_setprio 2, 1, 0; the other way round 3120 us for the 3047 of two steps and 3000 of three, 24 planes and 128 bins).  Together, one card, us:
+// that begins a group (s_setprio 2, 1, 0; the other way round 3120 us for the 3047 of two steps and 3000 of three, 24 planes and 128 bins).
+// Together, one card, us:
 //   6 x 10000 queries, 4 levels from 116 x 200, 8 points: 885 -> 872, around the query 574 -> 571 (bfloat16 483 -> 476), plain attention 436 -> 389;
 //   6 x 40000 clustered, 128 bins: 3067 -> 3000; the two separate stages without gradients, 112 bins: 1013 -> 936; one level of 23 x 40: 39.7 -> 38.0;
 // Where a workgroup has one group (not IN_LDS) there are none: plain attention, 4 points, 2 x 40000 queries on 200 x 200 gained from them (103 -> 96),
 // 4 x 10000 on 116 x 197 lost (59.5 -> 63.7).
 //
-// Six wavefronts a SIMD (kFwdWaves: 80 vector registers, none of which is spilled; of the scalars 64 are with depth taps, 84 with EARLY, to vector lanes) where five were: plain
-// attention, 3 x 3 points 33.5 -> 30.1; one distribution for all heads, packed, four levels of 8 points, around the query 125 -> 118.5, anywhere 150 -> 144,
-// 9000 queries, 116 x 197 326 -> 315; other calls with runs +- 0.5 %.  Seven spill (118.5 -> 141).
-// ---------------------------------------------------------------------------------------
-// wavefronts a SIMD that the registers have to leave room for (1: as the compiler likes)
+// Six wavefronts a SIMD (kFwdWaves: 80 vector registers, none of which is spilled; of the scalars 64 are with depth taps, 84 with EARLY, to vector
+// lanes) where five were: plain attention, 3 x 3 points 33.5 -> 30.1; one distribution for all heads, packed, four levels of 8 points, around the
+// query 125 -> 118.5, anywhere 150 -> 144, 9000 queries, 116 x 197 326 -> 315; other calls with runs +- 0.5 %.  Seven spill (118.5 -> 141).
+// --------------------------------------------------------------------------------------- wavefronts a SIMD that the registers have to leave room
+// for (1: as the compiler likes)
 template <typename T, int VEC, bool IN_LDS> constexpr int kFwdWaves = !IN_LDS && sizeof(T) == 4 && VEC == 4 ? 6 : 1;
 // SCALAR: the first by_scalar points of a unit take their depth taps by scalar loads (points_by_scalar)
 template <typename T, typename A, int VEC, int LPR, bool FUSED, bool IN_LDS, bool IN_TURN, bool EARLY, bool SCALAR = false>
@@ -631,30 +632,53 @@ template <typename T, typename A> static LdsRows lds_rows_plan(const FwdArgs &a)
   return LdsRows{(int)parts, (int)room};
 }
 
-// How many of a unit's points, the first ones, take their depth taps by scalar loads (a distribution that is not packed: with one line a point instead of four, 4 %
-// either way).  The vector path's front end is what
-// bounds the gathers, a scattered line in 2 to 10 clocks; the scalar path answers a load in 10 to 14, side by side.  But neighbouring points find each
-// other's lines in the L1 where maps are small, and the scalar path has nothing of the kind: so the line lies by what a (batch, head) has of values and
-// distributions.  Kernel, us, points around the query, anywhere, clustered, 6 batch elements, 32 channels and four levels of 8 points unless noted.
+// How many of a unit's points, the first ones, take their depth taps by scalar loads, where a (batch, head) has this much of values and
+// distributions:
+//   rows from memory                  an eighth above 3.5 MB (one point at least), three sixteenths above 6 MB
+//     one distribution for all heads  an eighth above 8 MB
+//     bfloat16                        three sixteenths above 5 MB
+//   the coarser levels in LDS         an eighth above 5.5 MB; bfloat16, or a map that is in LDS whole (3 to 20 % slower): none
+//   a packed distribution             none: with one line a point instead of four, 4 % either way
+// The vector path's front end is what bounds the gathers, a scattered line in 2 to 10 clocks; the scalar path answers a load in 10 to 14,
+// side by side.  But neighbouring points find each other's lines in the L1 where maps are small, and the scalar path has nothing of the
+// kind: so the lines lie where points around the query stop losing.  Kernel, us, points around the query, anywhere, clustered, 6 batch
+// elements, 32 channels and four levels of 8 points unless noted.
 //   Rows from memory, 4000 queries, none / an eighth / three sixteenths:
-//     58 x 100, 16 bins          1.4 MB   159, 228, 226   164, 231, 228   169, 231, 224      80 x 128, 64 bins, 1 x 8   3.8 MB   123, 144, 150   117, 140, 142   120, 136, 140
-//     80 x 128, 16 bins          2.5 MB   185, 264, 268   181, 266, 262   193, 266, 258      58 x 100, 112 bins, 3 x 4  4.2 MB   156, 213, 203   150, 206, 194   159, 195, 183
-//     46 x 80, 128 bins, 3 x 8   3.0 MB   153, 225, 231   159, 222, 222   171, 217, 216      70 x 119, 112 bins         6.1 MB   240, 367, 335   226, 354, 317   232, 340, 303
-//     58 x 100, 80 bins          3.3 MB   197, 300, 293   193, 294, 281   200, 284, 270      116 x 200, 16 channels     9.4 MB   244, 375, 338   225, 358, 320   230, 344, 310
-//     100 x 170, 16 bins, 1 x 4  3.1 MB   106, 125, 121   106, 123, 116   106, 123, 116      116 x 200, 64 bins        11.3 MB   283, 415, 376   263, 401, 360   268, 389, 354
-//     one distribution for all heads (not packed: few points), none / an eighth: 65 x 116, 128 bins, 2 x 8, 2000 queries 6.0 MB 18.1, 18.2 around the query; 116 x 200, 64 bins
-//     11.3 MB 232, 357, 328 -> 224, 347, 318: from 8 MB on.
-//     So an eighth from 3.5 MB, three sixteenths from 6 MB on, one point at least (of 3 or 4: 116 x 200, one level 154, 179, 149 -> 146, 171, 140 and 168, 212, 172 -> 161,
-//     205, 162); a quarter: 64 bins 292, 385, 343.
+//     58 x 100, 16 bins          1.4 MB   159, 228, 226   164, 231, 228   169, 231, 224
+//     80 x 128, 16 bins          2.5 MB   185, 264, 268   181, 266, 262   193, 266, 258
+//     46 x 80, 128 bins, 3 x 8   3.0 MB   153, 225, 231   159, 222, 222   171, 217, 216
+//     100 x 170, 16 bins, 1 x 4  3.1 MB   106, 125, 121   106, 123, 116   106, 123, 116
+//     58 x 100, 80 bins          3.3 MB   197, 300, 293   193, 294, 281   200, 284, 270
+//     80 x 128, 64 bins, 1 x 8   3.8 MB   123, 144, 150   117, 140, 142   120, 136, 140
+//     58 x 100, 112 bins, 3 x 4  4.2 MB   156, 213, 203   150, 206, 194   159, 195, 183
+//     70 x 119, 112 bins         6.1 MB   240, 367, 335   226, 354, 317   232, 340, 303
+//     116 x 200, 16 channels     9.4 MB   244, 375, 338   225, 358, 320   230, 344, 310
+//     116 x 200, 64 bins        11.3 MB   283, 415, 376   263, 401, 360   268, 389, 354   (a quarter 292, 385, 343)
+//   Units of few points, for which one or two are a larger part, none / by the rule:
+//     3 points   100 x 170, 32 bins  4.2 MB   84, 90, 69   77, 82, 63         116 x 200, 64 bins  8.5 MB   87, 91, 74   87, 90, 71
+//                three levels of 1 from 58 x 100, 112 bins  4.2 MB   61, 70, 47   58, 63, 44
+//     4 points   80 x 128, 64 bins   3.8 MB   74, 78, 68   73, 77, 65         70 x 119, 112 bins  4.6 MB   76, 84, 69   74, 83, 65
+//                116 x 200, 16 bins  4.2 MB   80, 89, 73   82, 89, 72         116 x 200, 64 bins  8.5 MB   99, 106, 86   98, 103, 82
+//                two levels of 2 from 80 x 128  4.7 MB   73, 83, 71   72, 81, 68   from 116 x 200  10.6 MB   97, 104, 87   96, 102, 84
+//     5 and 7    116 x 200, 64 bins  8.5 MB   116, 129, 107   113, 124, 102   and   141, 159, 134   135, 152, 126
+//     6 points   three levels of 2 from 116 x 200  11.2 MB   112, 130, 116   113, 128, 112   two of 3, 40 bins  8.0 MB   116, 135, 114   117, 132, 111
+//   One distribution for all heads (not packed: few points), none / an eighth:
+//     65 x 116, 128 bins, 2 x 8, 2000 queries  6.0 MB   18.1, 18.2 around the query     116 x 200, 64 bins  11.3 MB   232, 357, 328   224, 347, 318
 //   The coarser levels in LDS, 10000 queries, none / an eighth:
-//     58 x 100, 16 bins    1.5 MB   323, 499, 517   359, 478, 483      80 x 128, 64 bins, 3 x 8   5.2 MB   680, 1027, 965   697, 998, 925
-//     80 x 128, 16 bins    2.6 MB   359, 565, 564   382, 530, 515      116 x 200, 16 bins         5.9 MB   487, 769, 721    474, 737, 675
-//     58 x 100, 64 bins    3.0 MB   367, 533, 565   384, 510, 520      16 channels, 64 bins       9.9 MB   488, 759, 691    454, 721, 640
-//     70 x 119, 64 bins    4.2 MB   403, 610, 605   408, 577, 554      64 bins                   11.8 MB   571, 869, 803    538, 839, 766
-//     so an eighth from 5.5 MB on (three sixteenths: 64 bins 578, 825, 752; 16 bins 515, 749, 680).  On a map that is in LDS whole 3 to 20 % slower.
-//   Bfloat16, rows from memory, 4000 queries, none / three sixteenths: 70 x 119, 112 bins 3.1 MB 190, 299, 263 -> 213, 282, 241 (an eighth 194, 290, 250); 116 x 200, 59 bins
-//     5.6 MB 231, 355, 327 -> 228, 335, 302; 64 bins 5.9 MB 250, 379, 351 -> 229, 341, 302: from 5 MB on.  The coarser levels in LDS, 10000 queries, 64 bins, a sixteenth /
-//     an eighth: 475, 795, 738 -> 482, 760, 684 / 486, 738, 663; 128 bins 498, 763, 697 -> 505, 748, 676 / 515, 733, 665: not, for the points around the query.
+//     58 x 100, 16 bins          1.5 MB   323, 499, 517   359, 478, 483
+//     80 x 128, 16 bins          2.6 MB   359, 565, 564   382, 530, 515
+//     58 x 100, 64 bins          3.0 MB   367, 533, 565   384, 510, 520
+//     70 x 119, 64 bins          4.2 MB   403, 610, 605   408, 577, 554
+//     80 x 128, 64 bins, 3 x 8   5.2 MB   680, 1027, 965   697, 998, 925
+//     116 x 200, 16 bins         5.9 MB   487, 769, 721   474, 737, 675   (three sixteenths 515, 749, 680)
+//     16 channels, 64 bins       9.9 MB   488, 759, 691   454, 721, 640
+//     64 bins                   11.8 MB   571, 869, 803   538, 839, 766   (three sixteenths 578, 825, 752)
+//   Bfloat16, rows from memory, 4000 queries, none / three sixteenths:
+//     70 x 119, 112 bins         3.1 MB   190, 299, 263   213, 282, 241   (an eighth 194, 290, 250)
+//     116 x 200, 59 bins         5.6 MB   231, 355, 327   228, 335, 302
+//     64 bins                    5.9 MB   250, 379, 351   229, 341, 302
+//   Bfloat16, the coarser levels in LDS, 10000 queries, none / a sixteenth / an eighth:
+//     64 bins   475, 795, 738   482, 760, 684   486, 738, 663     128 bins   498, 763, 697   505, 748, 676   515, 733, 665
 template <typename T> static int points_by_scalar(const FwdArgs &a, const LdsRows &lds) {
   const int LP = a.L * a.P;
   if (sizeof(T) > 4 || a.dist == nullptr || a.packed_dist != nullptr || a.D < 2 || LP < 3 || (lds.parts > 0 && lds.rows == a.S)) return 0;
@@ -704,21 +728,23 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
   const int par = std::min(upw & -upw, kWave / LPR);
   const long long map_bytes = (long long)a.S * a.C * (long long)sizeof(T);                  // a (batch, head)'s value rows
   const bool in_turn = kWave / LPR > par && map_bytes <= (2LL << 20) && !(fused && a.packed_dist != nullptr && sizeof(T) == 4);
-  // Plain attention, the first group's locations and weights before the level table: a wavefront of one group then waits once, not twice, but all of
-  // them gather rows the sooner together, which costs more where caches serve them.  Float32 units of four points with rows of whole lines on maps above
-  // 1.5 MB gain.  4 x 31250 queries around the query and anywhere, table first and early, us: 32 channels, 1.1 MB 110, 110 and 106, 107; 2.2 MB
-  // 136, 133 and 137, 139; 8.7 MB 206, 204 and 269, 268; two levels of 2 points, 2.7 MB 137, 134 and 155, 156; 64 channels, 2.1 MB 203, 196 and
-  // 189, 186; 4.4 MB 238, 229 and 269, 271.  16 channels, 4.4 MB 143, 145 and 220, 219; 20 channels, 5.4 MB 189, 202 and 308, 307; 2 points a unit,
-  // 2.2 MB 120, 122 and 127, 130.  Early over table first, 32 channels, four sizes of map: 8 to 64
-  // points 1.00 - 1.12 (20 points 0.96 - 1.01), bfloat16 0.99 - 1.07 (15 and 20 points 0.95 - 1.02), float64 up to 1.08.
-  // Depth taps, each wavefront reading the levels' sizes by scalar loads instead of the table: no faster with a barrier in the table's place and slower with a
-  // table for each wavefront, so it is not the barrier that makes the difference but when the first rows are asked for.  Gains where a packed float32
-  // distribution leaves the value rows of a map above 1.5 MB to the caches.  Table and own sizes, us, around the query and anywhere, 4 levels of 8 points,
-  // 4 x 9000 queries on 116 x 197, 112 bins 300, 284 and 424, 405; 4 x 3906 on 100 x 170 117, 114 and 169, 162; 64 channels 191, 188 and 258, 251;
-  // on 70 x 119 (1.4 MB) 96, 100 and 132, 129; 16 channels 80, 93 and 117, 113; 3 levels of 4 points 119, 122 and 150, 145, 16 channels 95, 113 and
-  // 129, 125.  Bfloat16, packed, 60 x 102, 3 levels of 4 points 62, 69 and 73, 74; 4 levels of 8, 16 channels 80, 96 and 102, 105; 116 x 197 244, 251 and 349,
-  // 351.  A distribution per head, 60 x 102, 4 levels of 8 points 111, 111 and 157, 162 (bfloat16 106, 107 and 160, 167); other shapes 0.98 - 1.06
-  // around the query and 0.99 - 1.02 anywhere, own over table.
+  // Early: plain attention asks for the first group's locations and weights before the level table, depth taps read the levels' sizes by
+  // scalar loads instead of the table.  Float32 on maps above 1.5 MB: units of four points with rows of whole lines, and a packed distribution.
+  // A wavefront of one group then waits once, not twice, but all of them gather rows the sooner together, which costs more where
+  // caches serve them (a barrier in the table's place changes nothing, a table for each wavefront is slower).
+  //   Plain attention, 4 x 31250 queries of 4 points, around the query and anywhere, us, table first and early:
+  //     32 channels  1.1 MB 110, 110 and 106, 107    2.2 MB 136, 133 and 137, 139    8.7 MB 206, 204 and 269, 268    2 x 2 points, 2.7 MB 137, 134
+  //       and 155, 156
+  //     64 channels  2.1 MB 203, 196 and 189, 186    4.4 MB 238, 229 and 269, 271    16 channels  4.4 MB 143, 145 and 220, 219
+  //     20 channels  5.4 MB 189, 202 and 308, 307    2 points a unit, 2.2 MB 120, 122 and 127, 130
+  //     early over table first, 32 channels, four sizes of map: 8 to 64 points 1.00 - 1.12 (20 points 0.96 - 1.01), bfloat16 0.99 - 1.07 (15 and 20 points
+  //     0.95 - 1.02), float64 up to 1.08
+  //   Packed distribution, around the query and anywhere, us, table and own sizes, 4 levels of 8 points:
+  //     4 x 9000 queries on 116 x 197, 112 bins 300, 284 and 424, 405    4 x 3906 on 100 x 170 117, 114 and 169, 162    64 channels 191, 188 and 258, 251
+  //     on 70 x 119 (1.4 MB) 96, 100 and 132, 129    16 channels 80, 93 and 117, 113    3 levels of 4 points 119, 122 and 150, 145, 16 channels
+  //       95, 113 and 129, 125
+  //     bfloat16, 60 x 102, 3 levels of 4 points 62, 69 and 73, 74    4 levels of 8, 16 channels 80, 96 and 102, 105    116 x 197 244, 251 and 349, 351
+  //   A distribution per head, 60 x 102, 111, 111 and 157, 162 (bfloat16 106, 107 and 160, 167); other shapes 0.98 - 1.06 and 0.99 - 1.02, own over table.
   const bool early = sizeof(T) == 4 && !in_turn && 2 * map_bytes > (3LL << 20) &&
                      (fused ? a.packed_dist != nullptr : a.score_in == nullptr && a.L * a.P == 4 && a.C >= 32);
   auto launch = [&](auto kernel, int threads, size_t bytes) -> hipError_t {

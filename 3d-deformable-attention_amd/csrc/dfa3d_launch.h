@@ -178,8 +178,8 @@ hipError_t launch_locations(const float *uv, const float *dz, const float *logit
 hipError_t launch_locations_grad(const float *grad_loc, const float *grad_attn, const float *attn, const int64_t *shapes3, float *grad_uv, float *grad_dz,
                                  float *grad_logits, long long rows, int M, int L, int P, hipStream_t stream);
 
-// Linear layers (dfa3d_linear.hip): y (N, O) = x (N, K) w (O, K)^T + bias + addend (N, O) (or nullptr), and y (N, K) = sum over the sets of rows (N, width) weight
-// (width, K); O, K and widths even, K (widths) a multiple of four in the first (second).
+// Linear layers (dfa3d_linear.hip): y (N, O) = x (N, K) w (O, K)^T + bias + addend (N, O) (or nullptr), and y (N, K) = sum over the sets of rows
+// (N, width) weight (width, K); O, K and widths even, K (widths) a multiple of four in the first (second).
 struct LinearSet { const float *weight, *rows; int width; };
 struct LinearSets { LinearSet set[DFA3D_MAX_LINEAR_SETS]; int n; };
 hipError_t launch_linear(const float *x, const float *w, const float *bias, const float *addend, float *y, long long N, int O, int K, hipStream_t stream);

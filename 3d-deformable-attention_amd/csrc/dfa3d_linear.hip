@@ -22,10 +22,10 @@
 //   * Rows beyond the end and columns beyond O or K read as zero (buffer range check).
 //
 // Library (forward and grad_x) or the float32 matrix instructions before (weight gradient), and now, us, between other kernels: 184950 rows of
-// 256 x 256 229, 177 (forward), 220, 171 (grad_x), 227, 147 (weight gradient); 58000 of 256 x 256 80, 56; 22500 45, 26; 5520 20, 12; 6600 of 256 x 64 19, 9.
-// Relative error against float64 (2-norm), the same: forward 2.0e-7, 1.7e-7 (5520 to 10^6 rows); grad_x 2.9e-7, 2.4e-7; weight gradient
-// 184950 rows 6.9e-7, 4.4e-7, 10^6 rows 1.6e-6, 9.6e-7, all positive 6.7e-8, 4.8e-8; grad_bias 2.1e-7, 2.1e-7.  Library's and these, forward
-// and grad_x alike, random signs (all positive): sums of 256 2.9e-7, 2.4e-7 (2.2e-7, 1.8e-7), 512 4.1e-7, 3.4e-7 (3.1e-7, 2.4e-7), 1024 5.7e-7, 4.9e-7
+// 256 x 256 229, 177 (forward), 220, 171 (grad_x), 227, 147 (weight gradient); 58000 of 256 x 256 80, 56; 22500 45, 26; 5520 20, 12; 6600 of 256 x
+// 64 19, 9.  Relative error against float64 (2-norm), the same: forward 2.0e-7, 1.7e-7 (5520 to 10^6 rows); grad_x 2.9e-7, 2.4e-7; weight gradient
+// 184950 rows 6.9e-7, 4.4e-7, 10^6 rows 1.6e-6, 9.6e-7, all positive 6.7e-8, 4.8e-8; grad_bias 2.1e-7, 2.1e-7.  Library's and these, forward and
+// grad_x alike, random signs (all positive): sums of 256 2.9e-7, 2.4e-7 (2.2e-7, 1.8e-7), 512 4.1e-7, 3.4e-7 (3.1e-7, 2.4e-7), 1024 5.7e-7, 4.9e-7
 // (4.3e-7, 2.9e-7), 2048 8.1e-7, 7.0e-7 (6.0e-7, 3.8e-7), 4096 1.2e-6, 1.0e-6 (8.5e-7, 5.3e-7).  Of few rows (linear_few_kernel): sums of 256
 // 2.9e-7, 1.2e-7 (2.4e-7, 0.6e-7), of 512, 256 and 256 terms of three layers 3.5e-7, 1.3e-7 (2.0e-7, 0.4e-7).
 #include <algorithm>
@@ -130,7 +130,8 @@ template <int MT, int NT> __device__ __forceinline__ void zero_sums(f32x16 (&x)[
 // acc += sum over depth contraction steps of A(m, k) B(n, k) for a TM x TN tile by four wavefronts, 2 x 2; `seen` is called with A's registers
 // once per kStep steps.  FLUSH: an instruction cuts off what lies about 2^-24 below the largest of its terms instead of rounding it (16 products of
 // 2^-27 on a sum of 1 leave 1, 16 of -2^-27 leave 1 - 2^-23; one of 3 2^-25 is rounded up), which a chain over thousands of rows of a weight
-// gradient feels; its sums start from zero every FLUSH steps and the vector unit adds them up.  Without, up to 4096 terms: see above.  `most`: the largest size among the operands that this thread brought.
+// gradient feels; its sums start from zero every FLUSH steps and the vector unit adds them up.  Without, up to 4096 terms: see above.  `most`: the
+// largest size among the operands that this thread brought.
 template <int TM, int TN, bool A_ACROSS, bool B_ACROSS, int FLUSH, typename Seen>
 __device__ __forceinline__ void split_product(unsigned char *lds, rsrc_t a_r, int lda, int a_row0, int a_rows, rsrc_t b_r, int ldb, int b_row0,
                                               int b_rows, int depth, f32x16 (&acc)[TM / 64][TN / 64], float &most, const Seen &seen) {
@@ -244,9 +245,9 @@ template <bool ACROSS> __device__ __forceinline__ void load_whole(rsrc_t r, int 
 }
 
 // acc += the wavefront's part of the tile by float32 matrix instructions, straight from memory: what split_product forms, for sums that
-// parts give no number for; row_a, row_b: this lane's first rows within the tile.  Gradients of a loss that is no number are all of that kind, and cost a few times the usual, not a walk
-// over the rows per element: weight gradient of 58000 rows of 256 x 256 56 us, all NaN 119 (by
-// one lane per element 10000); grad_x 59, 124 (3280); with one NaN row in a thousand 125 (6400) and 70 (173).
+// parts give no number for; row_a, row_b: this lane's first rows within the tile.  Gradients of a loss that is no number are all of that kind, and
+// cost a few times the usual, not a walk over the rows per element: weight gradient of 58000 rows of 256 x 256 56 us, all NaN 119 (by one lane per
+// element 10000); grad_x 59, 124 (3280); with one NaN row in a thousand 125 (6400) and 70 (173).
 template <int MT, int NT, bool A_ACROSS, bool B_ACROSS>
 __device__ __forceinline__ void whole_product(rsrc_t a_r, int lda, int a_row0, int a_rows, rsrc_t b_r, int ldb, int b_row0, int b_rows, int depth,
                                               int row_a, int row_b, f32x16 (&acc)[MT][NT]) {
@@ -275,8 +276,8 @@ __device__ __forceinline__ void whole_tile(rsrc_t a_r, int lda, int a_row0, int 
 }
 
 // c (TM x TN tile of `ms` x `ns` valid elements, row length ldc) = acc + bias, + addend (as c) where there is one, asked for
-// 16 elements at a time (one by one, each between two stores, 2500 rows of 256 x 256 14.5 us; product 8.5, product and sum 12.3, so 9.6; 22500 of 128 x 128 17.4; 11.0,
-// 19.3, 11.5; 40000 of 512 x 512 178; 134, 168, 143).
+// 16 elements at a time (one by one, each between two stores, 2500 rows of 256 x 256 14.5 us; product 8.5, product and sum 12.3, so 9.6; 22500 of
+// 128 x 128 17.4; 11.0, 19.3, 11.5; 40000 of 512 x 512 178; 134, 168, 143).
 template <int TM, int TN>
 __device__ __forceinline__ void store_product(const f32x16 (&acc)[TM / 64][TN / 64], float *__restrict__ c, int ldc, int ms, int ns,
                                               const float *__restrict__ bias, const float *__restrict__ addend = nullptr) {
@@ -385,10 +386,10 @@ template <bool ACROSS> __device__ __forceinline__ void load_eight(rsrc_t r, int 
   }
 }
 
-// The same products and sums where the tiles of the two kernels above are few: y (N, cols) = sum over the sets of rows (N, width) weight (cols, width)^T, or
-// (ACROSS) weight (width, cols), + bias + addend.  A workgroup forms 32 x 32, and its four wavefronts take every fourth 16 steps each, straight
-// from memory into registers, four of their steps at a time: a chain a sixteenth as long as those kernels', on up to four times as many workgroups.
-// Sums start from zero every four steps (split_product, FLUSH) and the vector unit adds them up; those of the wavefronts meet in LDS.
+// The same products and sums where the tiles of the two kernels above are few: y (N, cols) = sum over the sets of rows (N, width) weight (cols,
+// width)^T, or (ACROSS) weight (width, cols), + bias + addend.  A workgroup forms 32 x 32, and its four wavefronts take every fourth 16 steps each,
+// straight from memory into registers, four of their steps at a time: a chain a sixteenth as long as those kernels', on up to four times as many
+// workgroups. Sums start from zero every four steps (split_product, FLUSH) and the vector unit adds them up; those of the wavefronts meet in LDS.
 constexpr int kFewTile = 32, kFewSteps = 4;
 template <bool ACROSS>
 __global__ __launch_bounds__(256, 2) void linear_few_kernel(LinearSets sets, const float *__restrict__ bias, const float *__restrict__ addend,
@@ -571,9 +572,9 @@ template <int KS> __device__ __forceinline__ void load_columns(rsrc_t r, int col
   }
 }
 
-// ADD: `addend` (N, cols) is added to the result: its elements are asked for when the tile's last product is under way (there are no registers to hold them before),
-// and what their way takes per tile is less than a pass over the result: product, product and sum, and both in one, 22500 rows of 256 x 256 23.2, 37.6 and 29.6 us;
-// 40000 34.2, 56.5, 45.7; 80000 67, 101, 82.
+// ADD: `addend` (N, cols) is added to the result: its elements are asked for when the tile's last product is under way (there are no registers to
+// hold them before), and what their way takes per tile is less than a pass over the result: product, product and sum, and both in one, 22500 rows
+// of 256 x 256 23.2, 37.6 and 29.6 us; 40000 34.2, 56.5, 45.7; 80000 67, 101, 82.
 template <int KS, bool ACROSS, bool ADD>
 __global__ __launch_bounds__(kRowThreads, 2) void linear_rows_kernel(const float *__restrict__ x, const float *__restrict__ weight,
                                                                      const float *__restrict__ bias, const float *__restrict__ addend,
@@ -709,8 +710,8 @@ static LinearTiles linear_tiles(long long N, int O, int K) {
   return t;
 }
 
-// What the kernels are told of the layers: of layer i the workgroups from first[i] on in the first launch and from first_sum[i] on in the second.  Each layer's parts
-// and tiles are those that it would have alone, so its results are too, to the bit.
+// What the kernels are told of the layers: of layer i the workgroups from first[i] on in the first launch and from first_sum[i] on in the second.
+// Each layer's parts and tiles are those that it would have alone, so its results are too, to the bit.
 struct GradLayers {
   LinearGradSet set[DFA3D_MAX_LINEAR_SETS];
   LinearTiles tiles[DFA3D_MAX_LINEAR_SETS];
@@ -810,16 +811,17 @@ static hipError_t launch_linear_cfg(const float *x, const float *w, const float 
 
 // Where linear_rows_kernel takes a product.  A workgroup multiplies by 256 columns and 256 steps whether they are there or not and begins with 5 us of
 // weights, more where they lie along the depth; the other kernels' tiles end where a multiple of 64 columns does.  So the share of the products that the
-// others would form too, in sixteenths, has to be the larger the fewer row tiles a CU gets and the more blocks of columns there are.  Time over that of the
-// others, 4928 to 185000 rows, depths 196 to 256, 130 to 1024 columns, lowest and highest where this kernel is taken and where not:
+// others would form too, in sixteenths, has to be the larger the fewer row tiles a CU gets and the more blocks of columns there are.  Time over
+// that of the others, 4928 to 185000 rows, depths 196 to 256, 130 to 1024 columns, lowest and highest where this kernel is taken and where not:
 //   row tiles per CU        0.6 - 1                    1.5 - 2                    2 - 4                      4 - 8                      8 and more
 //   256 columns or fewer    x W^T from 15, g W 12      from 14                    from 10                    all                        all
 //     taken, not            0.77 - 1.01, 0.93 - 1.35   0.81 - 0.97, 0.89 - 1.19   0.83 - 1.02, 0.93 - 1.06   0.77 - 0.96                0.67 - 0.88
 //   more                    none                       none                       512 from 14 (more: below)  from 12                    from 9
 //     taken, not                                       0.95 - 1.54                0.87 - 1.05, 0.88 - 1.44   0.80 - 1.06, 0.89 - 1.23   0.72 - 0.93
-// More than 512 columns gain from three tiles per CU on if they are whole blocks (25000 rows, 768 columns 0.88, 1024 0.96; 16500 rows 1.02, 1.08).  In us, the
-// others and this one: 4928 rows of 256 x 256 10.7, 10.8 (x W^T), 13.0, 11.1 (g W); 12500 17.8, 15.2 and 18.5, 15.2; 12500 of 258 columns 22.5, 27.6 and 21.8, 29.5;
-// 25000 of 320 38.7, 42.5; 58000 of 320 77.5, 78.5; 58000 of 512 108, 89; of 128 columns 27850 21.1, 25.1.  (16-byte loads to LDS want their addresses whole.)
+// More than 512 columns gain from three tiles per CU on if they are whole blocks (25000 rows, 768 columns 0.88, 1024 0.96; 16500 rows 1.02, 1.08).
+// In us, the others and this one: 4928 rows of 256 x 256 10.7, 10.8 (x W^T), 13.0, 11.1 (g W); 12500 17.8, 15.2 and 18.5, 15.2; 12500 of 258
+// columns 22.5, 27.6 and 21.8, 29.5; 25000 of 320 38.7, 42.5; 58000 of 320 77.5, 78.5; 58000 of 512 108, 89; of 128 columns 27850 21.1, 25.1.
+// (16-byte loads to LDS want their addresses whole.)
 static bool rows_kernel_applies(const float *x, const float *weight, long long N, int cols, int depth, bool across) {
   if (cols <= 128 || depth <= 192 || depth > 256 || (depth & 3) != 0 || (((uintptr_t)x | (uintptr_t)weight) & 15) != 0) return false;
   const long long tiles = (N + kRowTile - 1) / kRowTile, cus = cu_count(), blocks = (cols + kRowCols - 1) / kRowCols;
@@ -843,12 +845,14 @@ static hipError_t launch_linear_rows(const float *x, const float *w, const float
   return hipGetLastError();
 }
 
-// Where linear_few_kernel takes a product: few 64 x 64 tiles for the depth of the sums, as its own 32 x 32 read operands twice as often.  On the device alone
-// (captured in a graph), the other kernels and this one, us:
-//   x W^T, 256 columns of 256 terms   100 rows 8.0, 5.9   625 (40 tiles) 8.1, 6.2   1500 (96) 8.3, 8.1   2500 (160) 8.7, 10.3     64 columns  6600 (104) 8.4, 8.2
+// Where linear_few_kernel takes a product: few 64 x 64 tiles for the depth of the sums, as its own 32 x 32 read operands twice as often.  On the
+// device alone (captured in a graph), the other kernels and this one, us:
+//   x W^T, 256 columns of 256 terms   100 rows 8.0, 5.9   625 (40 tiles) 8.1, 6.2   1500 (96) 8.3, 8.1   2500 (160) 8.7, 10.3
+//     64 columns                      6600 rows (104) 8.4, 8.2
 //     128 columns of 128 terms        625 (20) 5.9, 5.5   1500 (48) 5.9, 5.5   2500 (80) 6.0, 6.8     256 of 64 terms 100 (8) 4.7, 5.0
 //   sums of 512, 256 and 256 terms    16 rows 35.6, 9.1   1000 (64) 37.1, 12.0   4000 (252) 43.0, 27.8   5500 (344) 47.0, 36.8   8000 (500) 50.3, 52.2
-//     of 256, 128 and 128             1000 20.5, 8.3   4000 (252) 22.7, 20.9   5500 (344) 25.7, 26.8     of 128, 64 and 64  2000 (128) 13.2, 12.1   4000 13.9, 18.8
+//     of 256, 128 and 128             1000 20.5, 8.3   4000 (252) 22.7, 20.9   5500 (344) 25.7, 26.8
+//     of 128, 64 and 64               2000 (128) 13.2, 12.1   4000 13.9, 18.8
 //     of 64, 32 and 32                1000 (64) 9.0, 7.9   2000 (128) 9.2, 10.8
 static bool few_rows(long long N, int cols, int depth, bool across) {
   const long long tiles = (N + 63) / 64 * ((cols + 63) / 64);
@@ -898,8 +902,8 @@ size_t linear_grad_workspace_bytes(long long N, int O, int K) {
   return (size_t)linear_tiles(N, O, K).parts * ((size_t)O * K + O) * sizeof(float);
 }
 
-// Several layers in two launches, whose workgroups fill the device together where one layer has few parts: 512, 256 and 256 columns on rows of 256, three pairs of launches
-// and these, 1000 rows 45 us, 21; 7700 78, 42; 58000 231, 208; 256, 128 and 128 columns 7700 rows 70, 29.
+// Several layers in two launches, whose workgroups fill the device together where one layer has few parts: 512, 256 and 256 columns on rows of 256,
+// three pairs of launches and these, 1000 rows 45 us, 21; 7700 78, 42; 58000 231, 208; 256, 128 and 128 columns 7700 rows 70, 29.
 hipError_t launch_linear_grads(const float *x, const LinearGradSets &sets, float *workspace, long long N, int K, hipStream_t stream) {
   GradLayers layers{};
   layers.n = sets.n;

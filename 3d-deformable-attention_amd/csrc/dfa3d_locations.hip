@@ -3,13 +3,13 @@
 //
 //   loc[n, m, l, p] = (u / W_l, v / H_l, d / D_l) + ref[n, p % Z]
 //
-// with (u, v) = uv[n, m, l, p] and d = dz[n, m, l, p]; and the gradients of uv and dz.  With them, where a head's points are a power of two up to a wavefront's
-// lanes, the softmax over those of what the layer predicts as their weights, and its gradient.  Pure streaming, 24 bytes read or
-// written per point and direction (with the weights 32, back 36), where tensor operations took three passes each way (softmax: one, back two).  A thread keeps its
-// place in the row and walks down the block's rows, as many at once as 256 threads have room for, so that the place is decoded once and neighbouring lanes are
-// neighbouring points; a head's points are neighbouring lanes.  Locations and softmax by
-// themselves (with 16 rows a block, one at once) and in one kernel, us: 50000 rows of 8 heads, 32 points each 74 and 26, 77; back 55 and 46, 84; 27500 rows of 8 points each 12
-// and 5, 12; 9 and 10, 12; 3300 rows of 16 6 and 3, 5.6; 5 and 5, 4.9.
+// with (u, v) = uv[n, m, l, p] and d = dz[n, m, l, p]; and the gradients of uv and dz.  With them, where a head's points are a power of two up to a
+// wavefront's lanes, the softmax over those of what the layer predicts as their weights, and its gradient.  Pure streaming, 24 bytes read or
+// written per point and direction (with the weights 32, back 36), where tensor operations took three passes each way (softmax: one, back two).  A
+// thread keeps its place in the row and walks down the block's rows, as many at once as 256 threads have room for, so that the place is decoded
+// once and neighbouring lanes are neighbouring points; a head's points are neighbouring lanes.  Locations and softmax by themselves (with 16 rows a
+// block, one at once) and in one kernel, us: 50000 rows of 8 heads, 32 points each 74 and 26, 77; back 55 and 46, 84; 27500 rows of 8 points each
+// 12 and 5, 12; 9 and 10, 12; 3300 rows of 16 6 and 3, 5.6; 5 and 5, 4.9.
 #include <algorithm>
 #include <type_traits>
 
@@ -107,9 +107,9 @@ hipError_t launch_level_table(const int64_t *shapes, int64_t *shapes3, int L, in
   hipLaunchKernelGGL(level_table_kernel, dim3(1), dim3(64), 0, stream, shapes, shapes3, L, D);
   return hipGetLastError();
 }
-// Rows of a block: four times those that it takes at once, fewer where that leaves fewer than 1024 blocks.  50000 rows of 256 points, 4, 8 and 16 rows a block, there and
-// back 77 and 84, 79 and 87, 84 and 93 us; 27500 rows of 64, 6 and 13 rows (four at once) 15 and 13, 12 and 12; 3300 rows of 128, 2, 3 and 16 rows 5.8 and 5.0, 5.6 and
-// 4.9, 9.4 and 6.9.
+// Rows of a block: four times those that it takes at once, fewer where that leaves fewer than 1024 blocks.  50000 rows of 256 points, 4, 8 and 16
+// rows a block, there and back 77 and 84, 79 and 87, 84 and 93 us; 27500 rows of 64, 6 and 13 rows (four at once) 15 and 13, 12 and 12; 3300 rows
+// of 128, 2, 3 and 16 rows 5.8 and 5.0, 5.6 and 4.9, 9.4 and 6.9.
 static int rows_per_block(long long rows, int MLP) {
   const long long at_once = MLP < kLocThreads ? kLocThreads / MLP : 1, share = rows / 1024;
   return (int)std::max(at_once, std::min(share, 4 * at_once));

@@ -140,10 +140,10 @@ __global__ __launch_bounds__(kRebatchBlock) void rebatch_combine_kernel(
 }
 
 // The layer's gather in one launch: dst[j, i, k, :] = src[j, q, :] + plus[j, q, :] (`plus` may be null), zero in the padding, and
-// ref_dst[j, i, k, :] = ref[i, j, q, :], `ref_pad` in the padding, q = index[i, k].  One thread per VEC elements of a row of dst, then one per VEC_REF of a row of
-// ref_dst.  Bound by what is read and written; the queries alone are summed as they are read and the sum
-// not written out and read again: 22500 queries of 256 and their positions, a fifth in each of six cameras, 14.5 us for 10.9 (sum), 10.5 and 2.7 (gathers);
-// 40000 24.0 for 18.1, 16.7 and 3.0 (a copy of the result 9 and 15).
+// ref_dst[j, i, k, :] = ref[i, j, q, :], `ref_pad` in the padding, q = index[i, k].  One thread per VEC elements of a row of dst, then one per
+// VEC_REF of a row of ref_dst.  Bound by what is read and written; the queries alone are summed as they are read and the sum not written out and
+// read again: 22500 queries of 256 and their positions, a fifth in each of six cameras, 14.5 us for 10.9 (sum), 10.5 and 2.7 (gathers); 40000 24.0
+// for 18.1, 16.7 and 3.0 (a copy of the result 9 and 15).
 template <typename T, int VEC, int VEC_REF>
 __global__ __launch_bounds__(kRebatchBlock) void rebatch_queries_kernel(
     const T *__restrict__ src, const T *__restrict__ plus, const T *__restrict__ ref, const int *__restrict__ index, T *__restrict__ dst,
@@ -300,8 +300,8 @@ __global__ __launch_bounds__(256) void camera_hits_kernel(const uint8_t *__restr
 }
 
 // The same, and how many queries of each camera each workgroup hit: counts (cams, gridDim.x), which the host adds up.  A pass over `hit` by one
-// workgroup per camera and its launch are saved: 22500 queries, six cameras 4.3 us for 3.1 and 4.6, 40000 4.3 for 3.1 and 6.6; with lists, copy and host 36.7 for 40.1, 37.6
-// for 47.4.
+// workgroup per camera and its launch are saved: 22500 queries, six cameras 4.3 us for 3.1 and 4.6, 40000 4.3 for 3.1 and 6.6; with lists, copy and
+// host 36.7 for 40.1, 37.6 for 47.4.
 __global__ __launch_bounds__(kHitsBlock) void camera_hits_counted_kernel(const uint8_t *__restrict__ mask, uint8_t *__restrict__ hit, float *__restrict__ scale,
                                                                          int *__restrict__ counts, int cams, int bs, int Nq, int Z) {
   __shared__ int s_count[kHitsCams];
