@@ -5,8 +5,8 @@
 The library lands next to the python package (dfa3D/libdfa3d_hip.so) so that it travels with
 the source tree, as does the module that calls it with torch's tensors (dfa3D/_binding.*.so, host code).  That module fits
 one torch and one Python and is built again when either is another; where it cannot be built, calls go through ctypes.
-Two more libraries land beside bench.py, which is what uses them: the yardstick kernels (libdfa3d_measure.so) and, with --clocks, libdfa3d_hip_clocks.so: the same sources compiled with
--DDFA3D_TILE_TIMING, i.e. with the per-phase clocks of the backward's tile kernels (`bench.py --phase-costs`).
+Two more libraries land beside bench.py, which is what uses them: the yardstick kernels (libdfa3d_measure.so) and, with
+--clocks, libdfa3d_hip_clocks.so: the same sources compiled with -DDFA3D_TILE_TIMING, i.e. with the per-phase clocks of the backward's tile kernels (`bench.py --phase-costs`).
 """
 import os
 import subprocess

@@ -65,7 +65,8 @@ class _LocationsFunction(OperatorFunction):
 
 
 class _SamplingFunction(OperatorFunction):
-    """As ``_LocationsFunction``, and logits (bs, Q, M, L, P) to their softmax over a head's points: ``apply(uv, dz, logits, reference_points, shapes3)``."""
+    """As ``_LocationsFunction``, and logits (bs, Q, M, L, P) to their softmax over a head's points:
+    ``apply(uv, dz, logits, reference_points, shapes3)``."""
 
     own = True
 
@@ -84,7 +85,8 @@ class _SamplingFunction(OperatorFunction):
     @staticmethod
     def backward(ctx, grad_loc, grad_attn):
         shapes3, attn = ctx.saved_tensors
-        if not (plain_gradient(grad_loc) and plain_gradient(grad_attn) and as_plain(attn, grad_attn) and _readable(shapes3, attn)) or attn.numel() == 0:
+        if (not (plain_gradient(grad_loc) and plain_gradient(grad_attn) and as_plain(attn, grad_attn) and _readable(shapes3, attn))
+                or attn.numel() == 0):
             scaled = grad_loc / shapes3[:, [1, 0, 2]].to(grad_loc.device, grad_loc.dtype)[None, None, None, :, None, :]
             weighted = grad_attn * attn
             return scaled[..., :2], scaled[..., 2:], weighted - attn * weighted.sum((-1, -2), keepdim=True), None, None

@@ -28,12 +28,13 @@ def ordinary(*tensors, dtype=torch.float32):
 
 def _widths_apply(O, K):
     """Where the kernel takes the gradient of an O x K weight: even widths of up to 2048 whose product is at most 2^20.  The
-    library's product is slow where the result has few tiles, and has caught up at about 64 tiles of 128 x 128.  Times as
-    fast as the library's product and column sum, 4096 / 20000 / 100000 rows: 256 x 512 1.5 / 4.5 / 4.1, 256 x 2048 1.2 /
-    1.8 / 1.3, 512 x 1024 1.2 / 1.0 / 1.0, 1024 x 1024 1.05 / 0.95 / 1.1; beyond, 1024 x 2048 0.89 / 0.87 / 0.87, 2048 x 2048
-    0.84 / 0.87 / 0.85, 64 x 4096 1.1 / 0.9 / 0.8.  Fewer rows, library and kernels, us a call: 256 x 256 16 rows 25 / 13, 128 41 / 13,
-    1000 235 / 14, 2000 28 / 20; 512 x 256 24 / 13, 24 / 13, 28 / 15, 29 / 22 (on the device alone 6.6 / 10 at 16 rows, else as good or better).  The rule also bounds the workspace, 512 to 1024 tiles of 64 KB (2048 x
-    2048 would take 134 MB, 16384 x 16384 8.6 GB)."""
+    library's product is slow where the result has few tiles, and has caught up at about 64 tiles of 128 x 128.  The rule also bounds the
+    workspace, 512 to 1024 tiles of 64 KB (2048 x 2048 would take 134 MB, 16384 x 16384 8.6 GB).  Times as fast as the library's product and
+    column sum, 4096 / 20000 / 100000 rows: 256 x 512 1.5 / 4.5 / 4.1, 256 x 2048 1.2 / 1.8 / 1.3, 512 x 1024 1.2 / 1.0 / 1.0, 1024 x 1024
+    1.05 / 0.95 / 1.1; beyond, 1024 x 2048 0.89 / 0.87 / 0.87, 2048 x 2048 0.84 / 0.87 / 0.85, 64 x 4096 1.1 / 0.9 / 0.8.
+    Fewer rows, library and kernels, us a call (on the device alone): 256 x 256 16 rows 26 / 13 (14 / 10), 128 42 / 13 (41 / 10), 1000
+    235 / 16 (234 / 15), 2000 30 / 21 (28 / 21); 512 x 256 16 rows 26 / 13 (7 / 11), 128 26 / 13 (10 / 11), 1000 30 / 17 (20 / 16); 128 x 128
+    16 rows 26 / 13 (8 / 9), 300 30 / 13 (28 / 10)."""
     return O % 2 == 0 and K % 2 == 0 and max(O, K) <= 2048 and O * K <= 2 ** 20
 
 

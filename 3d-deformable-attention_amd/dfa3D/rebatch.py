@@ -36,8 +36,8 @@ def _on_their_way(counts):
     return counts, on_host, done
 
 
-# Workgroups that count, 1024 queries each at a time, and up to how many queries of all batch elements they count as they mark the hits; with more of them,
-# workgroups that mark alone are as many as there are queries for.
+# Workgroups that count, 1024 queries each at a time, and up to how many queries of all batch elements they count as they mark the
+# hits; with more of them, workgroups that mark alone are as many as there are queries for.
 _PARTS, _COUNTED_QUERIES = 64, 2 ** 18
 
 

@@ -26,14 +26,16 @@ class _Notes:
 
 
 class OperatorFunction(Function):
-    """A Function whose ``apply`` is its ``forward`` where gradients are off, and one call of the binding module, node and all, where that knows
-    the call (``kind``) and takes its operands: making a node in Python and wrapping what comes back is 4 of the 12 us that a forward of 2 x 100 queries
-    takes, and its backward holds the interpreter on the engine's thread.  Tracing, compilation, functorch transforms, forward mode, and profilers and
-    other observers, which see a call or refuse it, have the Python node made all the same, as do autocast, launch options, subclasses from elsewhere (and all calls where there is no
-    binding module to say who sees them; asked one by one from here they are 0.2 us of 9).  A class says with ``own = True`` in its own body that its ``forward`` asks no more of its context than ``_Notes``
-    has and returns none of its operands: ``Function`` hands out another tensor where a forward does, this the operand itself.  A native node
-    saves the operands as ``save_for_backward`` does; where its backward is not one call of the library (a gradient that is recorded itself, or operands
-    that saved-tensor hooks have made into something else) it runs the class's own ``backward``."""
+    """A Function whose ``apply`` is its ``forward`` where gradients are off, and one call of the binding module, node and all, where that
+    knows the call (``kind``) and takes its operands: making a node in Python and wrapping what comes back is 4 of the 12 us that a forward
+    of 2 x 100 queries takes, and its backward holds the interpreter on the engine's thread.  Tracing, compilation, functorch transforms,
+    forward mode, and profilers and other observers, which see a call or refuse it, have the Python node made all the same, as do autocast,
+    launch options, subclasses from elsewhere (and all calls where there is no binding module to say who sees them; asked one by one from
+    here they are 0.2 us of 9).  A class says with ``own = True`` in its own body that its ``forward`` asks no more of its context than
+    ``_Notes`` has and returns none of its operands: ``Function`` hands out another tensor where a forward does, this the operand itself.
+    A native node saves the operands as ``save_for_backward`` does and shows them, the step and the class's name as a node in Python does;
+    where its backward is not one call of the library (a gradient that is recorded itself, operands that saved-tensor hooks have made into
+    something else, an observer that has come since) it runs the class's own ``backward``."""
 
     own = False
     kind = None          # in a class's own body: the binding module knows the call as a whole

@@ -280,8 +280,8 @@ int dfa3d_locations(const float *uv, const float *dz, const float *ref, const in
 int dfa3d_locations_grad(const float *grad_loc, const int64_t *shapes3, float *grad_uv, float *grad_dz, long long rows, int M, int L,
                          int P, void *stream);
 
-/* The same with the attention weights attn (rows, M, L, P), the softmax of logits over the L * P points of a head (a power of two up to 64), and the gradient of the
- * logits from attn and grad_attn. */
+/* The same with the attention weights attn (rows, M, L, P), the softmax of logits over the L * P points of a head (a power of two
+ * up to 64), and the gradient of the logits from attn and grad_attn. */
 int dfa3d_sampling(const float *uv, const float *dz, const float *logits, const float *ref, const int64_t *shapes3, float *loc, float *attn,
                    long long rows, int M, int L, int P, int Z, void *stream);
 int dfa3d_sampling_grad(const float *grad_loc, const float *grad_attn, const float *attn, const int64_t *shapes3, float *grad_uv, float *grad_dz,
