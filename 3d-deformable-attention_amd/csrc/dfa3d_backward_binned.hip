@@ -1585,19 +1585,20 @@ size_t binned_backward_least_workspace_bytes(const BwdArgs &a, int kind, int dty
 // atomic per 64-byte piece of what a point adds to, 20 G of which the L2 executes a second where points are spread; adds to the same
 // few lines wait for one another, some 40 ns each.  So the direct kernels take calls
 //   * whose atomics, as of spread points, cost less than launches and tiles do: lines drawn where neither points all over the map, nor
-//     around the query, nor clustered (a normal distribution about the middle, 0.15 of the map) lose more than a few percent;
+//     around the query, nor clustered (a normal distribution about the middle, 0.15 of the map) lose more than some percent;
 //   * with at most 8000 (stage 1: 4000) points of a batch element, head and level, ten of a row, three of a line of a shared
 //     distribution: they may lie closer together;
 //   * with float sums of 80 MB at most, where those are formed for bfloat16 gradients alone: the tile kernels add bfloat16 in place (384
 //     points, 6 x 116 x 200, 66 us; 222 for the direct kernels, whatever the points.  For a shared distribution 240 us and more).
 // The call's kernels alone (captured in a graph), 8 heads of 32 channels, 64 bins, float32, at the line, thousands of points: tile kernels,
 // direct; all over, around the query, clustered | normal, 0.02 of the map | all in one cell:
-//   2 x 40 x 60 and 20 x 30       42: 45, 36   46, 36   45, 42 | 75, 89 | 84, 109      16 channels   62: 45, 35   45, 34   46, 39 | 65, 114 | 80, 158
-//                                                                                      64 channels   27: 56, 39   56, 38   53, 40 | 69, 62 | 85, 90
-//   2 x 80 x 120, 3 levels        87: 99, 71   99, 70   89, 76 | 83, 131 | 121, 221
-//   2 x 116 x 200, 128 bins       128: 192, 137   190, 133   155, 131 | 96, 158 | 147, 432
-//   2 x 116 x 200, 4 levels       173: 180, 143   181, 138   147, 147 | 123, 322 | 193, 371
-//   6 x 116 x 200, 4 levels       283: 435, 303   413, 300   318, 314 | 219, 421 | 327, 554
+//   1 x 20 x 30, 32 bins          33: 33, 28   34, 26   36, 41 | 69, 156 | 87, 192
+//   2 x 40 x 60 and 20 x 30       47: 46, 39   46, 38   46, 45 | 67, 94 | 91, 125
+//     16 channels, 64 channels    69: 44, 39   45, 37   47, 43 | 67, 111 | 93, 168             30: 57, 42   57, 41   55, 42 | 71, 68 | 90, 99
+//   2 x 80 x 120, 3 levels        97: 100, 76   100, 75   91, 84 | 83, 159 | 129, 268
+//   2 x 116 x 200, 128 bins       128: 192, 140   192, 136   158, 135 | 98, 155 | 150, 462
+//   2 x 116 x 200, 4 levels       193: 182, 156   183, 152   152, 164 | 133, 335 | 195, 448
+//   6 x 116 x 200, 4 levels       283: 434, 306   415, 301   318, 311 | 221, 416 | 336, 566
 //     (beyond the line              500: 451, 424   452, 413   352, 431 | 288, 712 | 491, 1057)
 //   one distribution for all heads, 2 x 40 x 60   53: 54, 42   54, 40   56, 49 | 73, 165 | 96, 268
 //     6 x 116 x 200, 4 levels     554: 536, 372   536, 359   443, 408 | 392, 881 | 624, 1182
@@ -1606,11 +1607,11 @@ size_t binned_backward_least_workspace_bytes(const BwdArgs &a, int kind, int dty
 //   stage 1 alone, 2 x 40 x 60    64: 48, 22   49, 20   53, 22 | 53, 36 | 66, 170
 //     (beyond the line            177: 59, 46   61, 41   55, 46 | 61, 91 | 86, 528)
 //     6 x 116 x 200, 4 levels     151: 159, 141   154, 122   158, 148 | 141, 137 | 156, 135
-//   bfloat16, 2 x 40 x 60         31: 42, 35   42, 34   44, 39 | 145, 75 | 275, 88
-//     2 x 80 x 120, 3 levels      42: 93, 60   89, 59   80, 63 | 143, 86 | 259, 129
+//   bfloat16, 2 x 40 x 60         36: 42, 39   42, 38   43, 44 | 137, 85 | 264, 93
+//     2 x 80 x 120, 3 levels      52: 93, 66   90, 66   81, 70 | 167, 100 | 312, 159
 //     sums of 95 MB               0.5: 41, 49   37: 101, 64   100, 63   81, 63 | 115, 111 | 329, 145
 //     of 189 MB                   25: 129, 99   108, 97   94, 97 | 69, 108 | 140, 122
-//     one distribution for all heads, 6 x 116 x 200, 4 levels   416: 533, 353   528, 345   420, 374 | 470, 705 | 745, 940
+//     one distribution for all heads, 6 x 116 x 200, 4 levels   207: 510, 236   488, 233   390, 247 | 363, 363 | 482, 486
 //   beyond ten of a row: plain, 15 x 21                            51: 38, 31   40, 31   48, 61 | 72, 255 | 96, 265
 //   beyond three of a line: 4 x 45 x 70, 4 levels, 16 bins         84: 78, 70   79, 63   74, 109
 bool few_points(const BwdArgs &a, int kind, int dtype) {
@@ -1628,7 +1629,7 @@ bool few_points(const BwdArgs &a, int kind, int dtype) {
     atomics_us += sums * 0.35e-6;
   }
   if (shared_dist(a)) return points < 3.0 * a.B * a.S * ((a.D * 4 + 63) / 64) && atomics_us < 22 + rows * 0.21e-3;
-  return atomics_us < std::min(17 + rows * (0.08e-3 + 0.001e-3 * (a.C + a.D)), 170.0);
+  return atomics_us < std::min(19 + rows * (0.10e-3 + 0.001e-3 * (a.C + a.D)), 170.0);
 }
 
 static size_t few_points_value_bytes(const BwdArgs &a) { return ((size_t)a.B * a.S * a.M * a.C * sizeof(float) + 255) & ~(size_t)255; }

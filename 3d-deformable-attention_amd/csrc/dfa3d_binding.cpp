@@ -440,9 +440,10 @@ PyObject *pack_dist(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 }
 
 // Calls of the Functions as a whole: forward, and the node of the graph where one is recorded, whose backward runs without the interpreter.  A
-// node of Python's needs the interpreter's lock on the engine's thread, which is handed over twice a backward, and costs its context and two wrappers:
-// 1 x 50 queries on 15 x 25 maps, a training pass in a row of them, 99 -> 68 us (backward 69 -> 54; with the engine on the caller's own thread the pass
-// 50 -> 42), the forward 11.7 -> 8.3 recorded and 9.4 -> 7.6 not.
+// node of Python's needs the interpreter's lock on the engine's thread, which is handed over twice a backward, and costs its context and two
+// wrappers: 1 x 50 queries on 15 x 25 maps, passes in a row, six measurements on one card, node in Python and native: a training pass 49 to 109
+// and 41 to 78 us (the hand-over to the engine's thread takes next to nothing or most of that, from run to run), the forward 11.9 to 12.7 and
+// 9.4 to 10.2 recorded, 10.1 and 8.0 not.
 enum Kind { kScore, kStage2, kPlain, kFused, kWeightUpdate };      // numbered as in recording.py
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;

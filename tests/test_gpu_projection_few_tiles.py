@@ -88,3 +88,20 @@ def test_both_sides_of_the_line(N, cols, depth, across):
         w = w.t()
     for y in (got, few):
         _within_roundings(y, [(x[part], w)])
+
+
+def test_replayed_in_a_graph():
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, w, b, r = _rand(g, 100, 256), _rand(g, 64, 256), _rand(g, 64), _rand(g, 100, 64)
+    pairs = [(_rand(g, 100, d), _rand(g, d, 64)) for d in (128, 68)]
+    call = lambda: (_product(x, w, b, r), _sum(pairs))
+    call()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for _ in range(3):
+        x.copy_(_rand(g, 100, 256))
+        pairs[0][0].copy_(_rand(g, 100, 128))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, e) for a, e in zip(out, call()))
